@@ -84,6 +84,14 @@ struct DwGeometry {
 bool dwconv_strip_fits(int KH, int KW, int dil_h, int dil_w, int stride_h, int stride_w, int in_c_stride, int ocp, uint32_t flags);
 void launch_dwconv(const ConvArgs& a, int KH, int KW, int dil_h, int dil_w, int variant, const DwGeometry& g, hipStream_t s);
 
+// the arguments of one launch as the single-launch program reads them (program.hip); false: nothing to compute
+struct ConvLaunch {
+    ConvArgs a;
+    bool depthwise;
+    int kh, kw, dil_h, dil_w;
+};
+bool conv_launch_arguments(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out, ConvLaunch& l);
+
 // frees the split-K workspace kept for this stream, if any (for the owner of a stream, before it destroys
 // the stream and after the stream's work has finished)
 void release_split_workspace(int device, hipStream_t s);

@@ -2493,3 +2493,10 @@ int hipie_conv_run_static(const hipie_conv* c, const hipie_tensor* in, const hip
 }
 
 }  // extern "C"
+
+bool hipie::conv_launch_arguments(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out, ConvLaunch& l) {
+    int32_t oh, ow;
+    l.depthwise = c->depthwise;
+    l.kh = c->d.kh; l.kw = c->d.kw; l.dil_h = c->d.dil_h; l.dil_w = c->d.dil_w;
+    return fill_conv_args(c, &in, residual, &out, l.a, oh, ow) != 0;
+}

@@ -70,6 +70,15 @@ struct hipie_fq;
 namespace hipie {
 // `fq` (null for an f32 result) must give integer levels (hipie_fq_create's q8 form); fq_gives_levels says whether it does
 bool fq_gives_levels(const hipie_fq* fq);
+// what a kernel that stores byte levels needs: stored byte = level index + off; false where hipie_fq_run_q8 would refuse
+struct FqLaunch {
+    const FqChannel* table;    // on the device
+    FqChannel first;           // channel 0 (per-tensor ranges)
+    int channels;
+    bool rcp;
+    float lm1, off;
+};
+bool fq_launch_arguments(const hipie_fq* fq, int out_dtype, FqLaunch& l);
 void run_eltwise(const hipie_fq* fq, const EltArgs& a, hipStream_t s);
 
 }  // namespace hipie

@@ -659,6 +659,13 @@ __global__ __launch_bounds__(kThreads) void eltwise_nhwc_kernel(const EltArgs a,
 
 bool hipie::fq_gives_levels(const hipie_fq* fq) { return fq && fq->q8_ok && fq->clamp_ok; }
 
+bool hipie::fq_launch_arguments(const hipie_fq* fq, int out_dtype, FqLaunch& l) {
+    if (!fq->table.ptr || !fq->q8_ok || !fq->clamp_ok || (out_dtype != HIPIE_U8B && out_dtype != HIPIE_I8)) return false;
+    if (out_dtype == HIPIE_U8B ? fq->q8_base < 0 : fq->q8_base + fq->lm1 > 127.0f) return false;
+    l = {fq->table.as<FqChannel>(), fq->host[0], static_cast<int>(fq->C), fq->rcp, fq->lm1, out_dtype == HIPIE_U8B ? fq->q8_base - 128.0f : fq->q8_base};
+    return true;
+}
+
 void hipie::run_eltwise(const hipie_fq* fq, const EltArgs& a, hipStream_t s) {
     const int64_t pixels = static_cast<int64_t>(a.N) * a.H * a.W;
     if (pixels == 0 || a.C == 0) return;

@@ -17,6 +17,7 @@
 #include "fq.h"
 #include "graph.h"
 #include "requant.h"
+#include "program.h"
 
 namespace hipie {
 namespace {
@@ -154,6 +155,9 @@ struct Step {
     virtual int launches() const { return 1; }   // kernels the step enqueues
     // vector instructions x lanes the step's f32 chain needs per inference (results x epilogue_valu_ops); 0: not counted
     virtual double valu_ops() const { return 0.0; }
+    // appends the step to the plan's single-launch form; false: that form does not take it.  Inputs and outputs are the
+    // builder's stand-ins (ProgBuilder::fake_arena, fake_io)
+    virtual bool program(ProgBuilder&, const std::vector<TensorInfo>&, void* const*, void* const*) const { return false; }
     virtual uint32_t epilogue_flags() const { return 0u; }   // the fused f32 chain of a convolution step as its flag word
 };
 
@@ -179,6 +183,9 @@ struct EntryStep : Step {
         check_status(u8_in ? hipie_fq_run_q8_tensor_u8(fq, static_cast<const uint8_t*>(inputs[param_index]), &d, s)
                            : hipie_fq_run_q8_tensor(fq, static_cast<const float*>(inputs[param_index]), &d, s),
                      name.c_str());
+    }
+    bool program(ProgBuilder& b, const std::vector<TensorInfo>& tensors, void* const* inputs, void* const*) const override {
+        return b.entry(fq, u8_in, inputs[param_index], tensors[out].desc(b.fake_arena()));
     }
 };
 
@@ -247,6 +254,18 @@ struct ConvStep : Step {
             else if (res_param >= 0) r = input_residual(o, inputs[res_param]);
         }
         check_status(hipie_conv_run(conv, &i, (fused || res >= 0 || res_param >= 0) ? &r : nullptr, &o, s), name.c_str());
+    }
+    bool program(ProgBuilder& b, const std::vector<TensorInfo>& tensors, void* const* inputs, void* const* outputs) const override {
+        const hipie_tensor i = tensors[in].desc(b.fake_arena()), o = tensors[out].desc(b.fake_arena());
+        hipie_tensor r{};
+        if (fused) {
+            r = tensors[shortcut->in].desc(b.fake_arena());
+        } else {
+            if (shortcut) return false;
+            if (res >= 0) r = tensors[res].desc(b.fake_arena());
+            else if (res_param >= 0) r = input_residual(o, inputs[res_param]);
+        }
+        return b.conv(conv, i, (fused || res >= 0 || res_param >= 0) ? &r : nullptr, o);
     }
     // a dense f32 [rows, channels] request input as the residual operand of output tensor `o`
     static hipie_tensor input_residual(const hipie_tensor& o, void* data) {
@@ -422,6 +441,9 @@ struct PairStep : Step {
         bytes = first->bytes + second->bytes - (fused ? 2 * mid_bytes : 0);
     }
     int launches() const override { return fused ? 1 : first->launches() + second->launches(); }
+    bool program(ProgBuilder& b, const std::vector<TensorInfo>& tensors, void* const* inputs, void* const* outputs) const override {
+        return first->program(b, tensors, inputs, outputs) && second->program(b, tensors, inputs, outputs);
+    }
     double valu_ops() const override { return first->valu_ops() + second->valu_ops(); }
     void run_fused(uint8_t* arena, const std::vector<TensorInfo>& tensors, hipStream_t s) const {
         const hipie_tensor i = tensors[first->in].desc(arena), o = tensors[second->out].desc(arena), r = tensors[second->res].desc(arena);
@@ -556,8 +578,7 @@ struct PoolStep : Step {
             a.fq_d = d_d.as<float>(); a.fq_r = d_r.as<float>();
         }
     }
-    void run(uint8_t* arena, const std::vector<TensorInfo>& tensors, void* const*, void* const*,
-             hipStream_t s) const override {
+    PoolArgs arguments(uint8_t* arena, const std::vector<TensorInfo>& tensors) const {
         const hipie_tensor i = tensors[in].desc(arena), o = tensors[out].desc(arena);
         PoolArgs b = a;
         b.in = i.data;
@@ -566,6 +587,14 @@ struct PoolStep : Step {
         b.in_sw = static_cast<int32_t>(i.stride_w);
         b.out_sn = static_cast<int32_t>(o.stride_n); b.out_sh = static_cast<int32_t>(o.stride_h);
         b.out_sw = static_cast<int32_t>(o.stride_w);
+        return b;
+    }
+    bool program(ProgBuilder& b, const std::vector<TensorInfo>& tensors, void* const*, void* const*) const override {
+        return b.pool(arguments(b.fake_arena(), tensors), avg, rcp);
+    }
+    void run(uint8_t* arena, const std::vector<TensorInfo>& tensors, void* const*, void* const*,
+             hipStream_t s) const override {
+        const PoolArgs b = arguments(arena, tensors);
         if (avg) launch_avg_pool(b, rcp, s);
         else launch_max_pool(b, s);
         HIPIE_CHECK_HIP(hipGetLastError());
@@ -684,8 +713,7 @@ struct ExitStep : Step {
         if (!sub.empty()) { const auto v = expand(sub); d_sub.upload(device, v.data(), v.size() * 4); }
         if (!mul.empty()) { const auto v = expand(mul); d_mul.upload(device, v.data(), v.size() * 4); }
     }
-    void run(uint8_t* arena, const std::vector<TensorInfo>& tensors, void* const*, void* const* outputs,
-             hipStream_t s) const override {
+    ExitArgs arguments(uint8_t* arena, const std::vector<TensorInfo>& tensors, void* const* outputs) const {
         const TensorInfo& t = tensors[in];
         const hipie_tensor i = t.desc(arena);
         ExitArgs a{};
@@ -698,7 +726,14 @@ struct ExitStep : Step {
         a.sub = sub.empty() ? nullptr : d_sub.as<float>();
         a.mul = mul.empty() ? nullptr : d_mul.as<float>();
         a.out_u8 = out_u8;
-        launch_exit(a, t.dtype, s);
+        return a;
+    }
+    bool program(ProgBuilder& b, const std::vector<TensorInfo>& tensors, void* const*, void* const* outputs) const override {
+        return b.exit(arguments(b.fake_arena(), tensors, outputs), tensors[in].dtype);
+    }
+    void run(uint8_t* arena, const std::vector<TensorInfo>& tensors, void* const*, void* const* outputs,
+             hipStream_t s) const override {
+        launch_exit(arguments(arena, tensors, outputs), tensors[in].dtype, s);
         HIPIE_CHECK_HIP(hipGetLastError());
     }
 };
@@ -848,6 +883,9 @@ struct MatFqStep : Step {
         check_status(hipie_fq_run_q8(fq, reinterpret_cast<const float*>(in.ptr(arena, tensors, inputs)),
                                      arena + tensors[out].offset, 1, n, static_cast<hipie_dtype>(out_dtype), HIPIE_NCHW, 0, s), name.c_str());
     }
+    bool program(ProgBuilder& b, const std::vector<TensorInfo>& tensors, void* const* inputs, void* const*) const override {
+        return b.fq_rows(fq, in.ptr(b.fake_arena(), tensors, inputs), b.fake_arena() + tensors[out].offset, out_dtype, n);
+    }
 };
 
 // Softmax / MVN (+ LayerNorm gamma, beta) / Gelu over the last axis of a dense f32 value
@@ -881,6 +919,12 @@ struct GlueStep : Step {
         else st = q ? hipie_mvn_q8(x, y, q, rows, axis, normalize_variance, eps, eps_inside_sqrt, gm, bt, r, s)
                     : hipie_mvn_f32(x, y, rows, axis, normalize_variance, eps, eps_inside_sqrt, gm, bt, s);
         check_status(st, name.c_str());
+    }
+    bool program(ProgBuilder& b, const std::vector<TensorInfo>& tensors, void* const* inputs, void* const*) const override {
+        if (kind == OP_SOFTMAX || kind == OP_GELU) return false;
+        auto at = [&](int t) { return t >= 0 ? b.fake_arena() + tensors[t].offset : nullptr; };
+        return b.mvn(in.ptr(b.fake_arena(), tensors, inputs), at(out), at(outq), rows, axis, normalize_variance, eps, eps_inside_sqrt,
+                     gamma.empty() ? nullptr : d_gamma.as<float>(), beta.empty() ? nullptr : d_beta.as<float>(), outq >= 0 ? &rq : nullptr);
     }
 };
 
@@ -962,6 +1006,12 @@ struct AttentionStep : Step {
                                          v.ptr(arena, tensors, inputs), ld[2], inner[2], outer[2], arena + tensors[out].offset,
                                          ldo, so, oo, batch, batch_outer, mk, 0, desc.seq, sc, pr, s), name.c_str());
     }
+    bool program(ProgBuilder& b, const std::vector<TensorInfo>& tensors, void* const* inputs, void* const*) const override {
+        if (scores >= 0 || probs >= 0 || (masked && mask_param < 0)) return false;
+        const void* const qkv[3] = {q.ptr(b.fake_arena(), tensors, inputs), k.ptr(b.fake_arena(), tensors, inputs), v.ptr(b.fake_arena(), tensors, inputs)};
+        return b.attention(att, qkv, ld, inner, outer, b.fake_arena() + tensors[out].offset, ldo, so, oo, batch, batch_outer,
+                           masked ? inputs[mask_param] : nullptr);
+    }
 };
 
 // Gather of a constant f32 table by the i32 token ids of a request input, with the embedding Adds
@@ -986,6 +1036,10 @@ struct EmbeddingStep : Step {
                                          add[0].empty() ? nullptr : d_add[0].as<float>(), per_position[0],
                                          add[1].empty() ? nullptr : d_add[1].as<float>(), per_position[1],
                                          reinterpret_cast<float*>(arena + tensors[out].offset), s), name.c_str());
+    }
+    bool program(ProgBuilder& b, const std::vector<TensorInfo>& tensors, void* const* inputs, void* const*) const override {
+        return b.embed(d_table.as<float>(), vocab, hidden, inputs[param], tokens, seq, add[0].empty() ? nullptr : d_add[0].as<float>(), per_position[0],
+                       add[1].empty() ? nullptr : d_add[1].as<float>(), per_position[1], b.fake_arena() + tensors[out].offset);
     }
 };
 
@@ -1021,6 +1075,9 @@ struct MatExitStep : Step {
         else
             HIPIE_CHECK_HIP(hipMemcpyAsync(outputs[result_index], in.ptr(arena, tensors, inputs), static_cast<size_t>(nbytes),
                                            hipMemcpyDeviceToDevice, s));
+    }
+    bool program(ProgBuilder& b, const std::vector<TensorInfo>& tensors, void* const* inputs, void* const* outputs) const override {
+        return !strided && b.copy(in.ptr(b.fake_arena(), tensors, inputs), outputs[result_index], nbytes);
     }
 };
 
@@ -1061,6 +1118,8 @@ struct PlanConfig {
     bool merge_linear = true;      // HIP_MERGE_LINEAR
     int fuse_convs = 1;            // HIP_FUSE_CONVOLUTIONS: a 3 x 3 convolution and the 1 x 1 behind it in one kernel - NO (0), AUTO
                                    // (1: where the load-time measurement says it is faster), YES (2: wherever the kernel takes the pair)
+    int single_launch = 1;         // HIP_SINGLE_LAUNCH: a request that is waited for runs as one kernel - NO (0), AUTO (1: a plan
+                                   // for one stream, where the load-time measurement says it is faster), YES (2: wherever there is such a form)
     int device_id = -1;            // DEVICE_ID (must agree with the device argument when given)
     std::string network_name = "hipie_network";
 
@@ -1077,6 +1136,7 @@ struct PlanConfig {
         c.fuse_attention = env_flag("HIPIE_FUSE_ATTENTION", true);
         c.merge_linear = env_flag("HIPIE_MERGE_LINEAR", true);
         if (const char* fc = std::getenv("HIPIE_FUSE_CONVS")) c.fuse_convs = std::max(0, std::min(2, std::atoi(fc)));
+        if (const char* sl = std::getenv("HIPIE_SINGLE_LAUNCH")) c.single_launch = std::max(0, std::min(2, std::atoi(sl)));
         return c;
     }
     static bool yes_no(const char* key, const char* v) {
@@ -1111,6 +1171,9 @@ struct PlanConfig {
         else if (k == "HIP_FUSE_CONVOLUTIONS") {
             if (!std::strcmp(value, "AUTO")) fuse_convs = 1;
             else fuse_convs = yes_no(key, value) ? 2 : 0;
+        } else if (k == "HIP_SINGLE_LAUNCH") {
+            if (!std::strcmp(value, "AUTO")) single_launch = 1;
+            else single_launch = yes_no(key, value) ? 2 : 0;
         }
         else if (k == "NETWORK_NAME") network_name = value;
         else fail(HIPIE_NOT_FOUND, "config key '%s' is not supported", key);
@@ -1125,12 +1188,13 @@ struct PlanConfig {
         else if (k == "HIP_KEEP_F32") v = yn(keep_f32);
         else if (k == "HIP_FUSE_ATTENTION") v = yn(fuse_attention);
         else if (k == "HIP_MERGE_LINEAR") v = yn(merge_linear);
+        else if (k == "HIP_SINGLE_LAUNCH") v = single_launch == 1 ? "AUTO" : yn(single_launch == 2);
         else if (k == "HIP_FUSE_CONVOLUTIONS") v = fuse_convs == 1 ? "AUTO" : yn(fuse_convs == 2);
         else return false;
         return true;
     }
 };
-constexpr const char* kConfigKeys = "PERF_COUNT DEVICE_ID HIP_THROUGHPUT_STREAMS HIP_TUNE HIP_TUNE_FILE HIP_KEEP_F32 HIP_FUSE_ATTENTION HIP_MERGE_LINEAR HIP_FUSE_CONVOLUTIONS";
+constexpr const char* kConfigKeys = "PERF_COUNT DEVICE_ID HIP_THROUGHPUT_STREAMS HIP_TUNE HIP_TUNE_FILE HIP_KEEP_F32 HIP_FUSE_ATTENTION HIP_MERGE_LINEAR HIP_FUSE_CONVOLUTIONS HIP_SINGLE_LAUNCH";
 
 // thrown by the planner for a node it cannot take: the status and text of any Error, plus the node
 struct UnsupportedNode : Error {
@@ -2875,6 +2939,8 @@ struct hipie_plan {
     // uploads the packed operands and takes the checks' verdicts instead of packing and checking again
     FqVerdicts verdicts;
     PackTape tape;
+    // the single-launch form, where the plan has one and runs it (requests that are waited for)
+    std::unique_ptr<Program> program;
 };
 
 struct hipie_request {
@@ -2887,11 +2953,21 @@ struct hipie_request {
     // written by the thread that starts and waits, and by whichever thread calls hipie_request_cancel meanwhile
     std::atomic<bool> started{false};
     std::atomic<bool> cancelled{false};      // hipie_request_cancel was called on the running inference
-    std::vector<void*> pending_out;          // host destinations of the running async infer
+    // the single-launch form: the request's slot (-1: none), its control block behind the arena, launches it counts, and
+    // what a run that the kernel gave up has to do again by steps
+    int slot = -1;
+    uint32_t* control = nullptr;
+    uint32_t launches = 0;
+    bool by_program = false;
+    std::vector<void*> run_in, run_out, host_out;
     ~hipie_request() {
         for (auto e : events) (void)hipEventDestroy(e);
         if (stream) {
             (void)hipStreamSynchronize(stream);
+            if (slot >= 0) {
+                program_done(*plan->program, stream);
+                plan->program->give_slot(slot);
+            }
             if (plan) release_split_workspace(plan->device, stream);
             (void)hipStreamDestroy(stream);
         }
@@ -2920,6 +2996,45 @@ void enqueue(hipie_request* r, void* const* in, void* const* out) {
         p.steps[i]->run(arena, p.tensors, in, out, r->stream);
     }
     if (r->perf) HIPIE_CHECK_HIP(hipEventRecord(r->events[p.steps.size()], r->stream));
+}
+
+// by the plan's single-launch form
+void enqueue_program(hipie_request* r, void* const* in, void* const* out) {
+    const hipie_plan& p = *r->plan;
+    void* io[kProgramIo] = {};
+    for (size_t i = 0; i < p.inputs.size(); ++i) io[i] = in[i];
+    for (size_t i = 0; i < p.outputs.size(); ++i) io[p.inputs.size() + i] = out[i];
+    launch_program(*p.program, r->arena.as<uint8_t>(), io, static_cast<int>(p.inputs.size() + p.outputs.size()), r->control, r->launches++, r->slot, r->stream);
+}
+
+// the stream has been waited for: where the single launch gave up (its workgroups did not come together), the inference
+// runs again by steps, outputs included
+void finish_program(hipie_request* r) {
+    if (!r->by_program) return;
+    r->by_program = false;
+    const hipie_plan& p = *r->plan;
+    program_done(*p.program, r->stream);
+    if (!program_failed(*p.program, r->slot, r->control, r->stream)) return;
+    r->launches = 0;
+    enqueue(r, r->run_in.data(), r->run_out.data());
+    for (size_t i = 0; i < r->host_out.size(); ++i)
+        HIPIE_CHECK_HIP(hipMemcpyAsync(r->host_out[i], r->run_out[i], static_cast<size_t>(p.outputs[i].bytes), hipMemcpyDeviceToHost, r->stream));
+    HIPIE_CHECK_HIP(hipStreamSynchronize(r->stream));
+}
+
+// the single-launch form of a plan whose every step has one, or null
+std::unique_ptr<Program> build_program(const hipie_plan& p, int workgroups) {
+    if (p.inputs.size() + p.outputs.size() > static_cast<size_t>(kProgramIo)) return nullptr;
+    ProgBuilder b;
+    b.device = p.device;
+    b.workgroups = workgroups;
+    std::vector<void*> in, out;
+    for (size_t i = 0; i < p.inputs.size(); ++i) in.push_back(b.fake_io(static_cast<int>(i)));
+    for (size_t i = 0; i < p.outputs.size(); ++i) out.push_back(b.fake_io(static_cast<int>(p.inputs.size() + i)));
+    DeviceGuard g(p.device);
+    for (const auto& s : p.steps)
+        if (!s->program(b, p.tensors, in.data(), out.data())) return nullptr;
+    return make_program(std::move(b));
 }
 
 // `preset`: kernel variants of an imported plan, one per step; used when they fit the steps planned
@@ -3253,6 +3368,39 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
                 }
             }
         }
+    }
+    if (device >= 0 && (cfg.single_launch == 2 || (cfg.single_launch == 1 && cfg.streams == 1 && cfg.tune))) {
+        // The single-launch form in its three sizes and the steps, as a caller sees them (start to wait): the fastest stays.
+        // Fewer workgroups have the cheaper barrier, more of them the shorter steps.
+        auto trial = [&] {
+            hipie_request* q = nullptr;
+            check_status(hipie_request_create(plan.get(), 0, &q), "hipie_compile: single-launch trial");
+            const std::unique_ptr<hipie_request, void (*)(hipie_request*)> hold(q, hipie_request_destroy);
+            std::vector<void*> in, out;
+            for (auto& b : q->in_dev) in.push_back(b.ptr);
+            for (auto& b : q->out_dev) out.push_back(b.ptr);
+            std::vector<double> t;
+            for (int turn = 0; turn < 15; ++turn) {
+                const auto t0 = std::chrono::steady_clock::now();
+                check_status(hipie_request_infer(q, in.data(), out.data(), 1), "hipie_compile: single-launch trial");
+                if (turn >= 4) t.push_back(std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
+            }
+            std::sort(t.begin(), t.end());
+            return t[t.size() / 2];
+        };
+        DeviceGuard dg(device);
+        double best = cfg.single_launch == 2 ? 1e30 : trial();
+        std::unique_ptr<Program> fastest;
+        for (int workgroups : {64, 128, 256}) {
+            plan->program = build_program(*plan, workgroups);
+            if (!plan->program) break;
+            const double t = trial();
+            if (t < best) {
+                best = t;
+                fastest = std::move(plan->program);
+            }
+        }
+        plan->program = std::move(fastest);
     }
     return plan;
 }
@@ -3626,10 +3774,13 @@ int hipie_request_create(const hipie_plan* p, int perf_count, hipie_request** ou
         r->perf = perf_count < 0 ? p->config.perf_count : perf_count != 0;   // < 0: the plan's PERF_COUNT
         DeviceGuard g(p->device);
         HIPIE_CHECK_HIP(hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking));
-        r->arena.alloc(p->device, static_cast<size_t>(p->arena_bytes));
+        const int64_t control_at = round_up(p->arena_bytes, 256);
+        r->arena.alloc(p->device, static_cast<size_t>(control_at) + kProgramControlBytes);
         // level 0 everywhere: halos and channel padding are never written again
         uint8_t* a = r->arena.as<uint8_t>();
-        HIPIE_CHECK_HIP(hipMemsetAsync(a, 0, static_cast<size_t>(p->arena_bytes), r->stream));
+        HIPIE_CHECK_HIP(hipMemsetAsync(a, 0, static_cast<size_t>(control_at) + kProgramControlBytes, r->stream));
+        r->control = reinterpret_cast<uint32_t*>(a + control_at);
+        if (p->program && !r->perf) r->slot = p->program->take_slot();
         for (const auto& t : p->tensors) {
             if (t.alias >= 0) continue;
             const int byte = t.dtype == HIPIE_U8B ? t.fill_level - 128 : (t.dtype == HIPIE_I8 ? t.fill_level : 0);
@@ -3700,7 +3851,16 @@ int hipie_request_start(hipie_request* r, const void* const* inputs, void* const
             HIPIE_REQUIRE(outputs[i], HIPIE_PARAMETER_MISMATCH, "hipie_request_start: output %zu is null", i);
             out[i] = device_memory ? outputs[i] : r->out_dev[i].ptr;
         }
-        enqueue(r, in.data(), out.data());
+        r->by_program = r->slot >= 0;
+        if (r->by_program) {
+            enqueue_program(r, in.data(), out.data());
+            r->run_in = in;
+            r->run_out = out;
+            r->host_out.clear();
+            if (!device_memory) r->host_out.assign(outputs, outputs + out.size());
+        } else {
+            enqueue(r, in.data(), out.data());
+        }
         if (!device_memory)
             for (size_t i = 0; i < out.size(); ++i)
                 HIPIE_CHECK_HIP(hipMemcpyAsync(outputs[i], out[i], static_cast<size_t>(p.outputs[i].bytes),
@@ -3727,6 +3887,7 @@ int hipie_request_wait_for(hipie_request* r, int64_t timeout_ms) {
             const hipError_t e = hipStreamSynchronize(r->stream);
             r->started = false;
             HIPIE_CHECK_HIP(e);
+            finish_program(r);
         } else {
             const auto deadline = std::chrono::steady_clock::now() + std::chrono::milliseconds(timeout_ms);
             for (;;) {
@@ -3737,6 +3898,7 @@ int hipie_request_wait_for(hipie_request* r, int64_t timeout_ms) {
                 std::this_thread::sleep_for(std::chrono::microseconds(50));
             }
             r->started = false;
+            finish_program(r);
         }
         if (r->cancelled.exchange(false)) fail(HIPIE_INFER_CANCELLED, "the inference was cancelled");
     });

@@ -1,0 +1,169 @@
+// A whole plan as ONE persistent kernel.
+//
+// What this is for: a request that somebody waits for.  As separate launches a batch-1 ResNet-50 is 54 dependent kernels
+// at about 9 us each: 2.4 us of launch, then a cold start (arguments, descriptors, tables, operands from the memory-side
+// cache - an XCD's L2 is written back and invalidated between kernels) in front of 1 - 2 us of work.  Here the workgroups
+// stay, and a step ends in a barrier among them: with the stores in front of it and the loads behind it 2.3 us for 64
+// workgroups, 2.9 for 128, 3.2 for 256 - and the cold start disappears behind it, because a workgroup that has arrived
+// prepares its next tile (descriptor, offsets, weights, constants) before it waits.
+//
+// Coherence: the eight XCDs' L2 caches are not coherent with each other.  Every result is stored write-through with device
+// scope (sc1), is awaited (s_waitcnt vmcnt(0)) in front of the barrier, and is loaded with device scope behind it; fences,
+// which write back or invalidate a whole L2 each, are not needed.  Weights, tables and the caller's inputs, which nothing
+// writes during the launch, are ordinary cached loads.
+//
+// Termination: a barrier needs every workgroup resident.  The roll call in front of the first step has a deadline: if the
+// launch is not complete in time (other work holds the compute units), it is cancelled by compare-and-swap before it has
+// written anything, the kernel drains, and the host runs the inference step by step.  Later waits are bounded as well (all
+// workgroups are resident by then, so they end; a bound that is hit ends the kernel and the host falls back the same way).
+// One program is in flight per device: launches on different streams are ordered by an event (ProgramGate).
+//
+// (Measured beside it: one XCD per batch element, whose barrier costs 0.95 us and whose results stay in its own L2.  Thirty-two
+// compute units on one L2 then do all of an image's work: 20 - 30 bytes a clock and unit of operands and the whole f32 chain
+// of 11 M values; ResNet-50 took 415 us that way and the encoder 831.)
+#pragma once
+#include <array>
+#include <memory>
+#include <mutex>
+
+#include "attention.h"
+#include "conv.h"
+#include "pool.h"
+#include "requant.h"
+
+namespace hipie {
+
+constexpr int kProgramThreads = 512;
+constexpr int kProgramIo = 6;            // graph inputs + outputs a program can address
+constexpr int kProgramStepWords = 128;
+
+enum ProgKind : int32_t { PK_CONV, PK_DW, PK_ENTRY, PK_MAXPOOL, PK_AVGPOOL, PK_EXIT, PK_EMBED, PK_MVN, PK_ATTENTION, PK_FQROWS, PK_COPY };
+
+// where an operand is: base 0 an arena offset, 1 + k an offset in the k-th input / output buffer of the call; < 0 absent
+struct ProgRef {
+    int32_t base;
+    uint32_t lo, hi;
+};
+struct ProgPtr { uint32_t lo, hi; };   // a load-time buffer
+
+// convolution, weight MatMul (1 x 1 over rows) and depthwise 3 x 3
+struct ProgConv {
+    int32_t kind, a, b, ks_shift;     // oc fragments, pixel fragments of a wave's tile; log2 of the waves that share a tile's K
+    int32_t p_tiles, tiles;           // pixel tiles; all tiles of the step
+    float inv_p_tiles;
+    ProgRef in, out, res, in2;         // `in` already moved to the first window's origin
+    ProgPtr wgt, koff, constants;      
+    ProgPtr wgt2, koff2, constants2;
+    ProgPtr pixels;                    // four words a pixel: byte offsets of its window in `in` and `in2`, of itself in `out` and `res`
+    int32_t nk, nk2, OCp, M;
+    int32_t out_limit, res_limit;     // channels the tensors hold
+    uint32_t flags;
+    float lm1, out_off, clamp_lo, clamp_hi;
+    // depthwise
+    int32_t stride, c4, quads, OH, OW, items;
+    int32_t in_sn, in_sh, in_sw, row_sh, out_sn, out_sh, out_sw, res_sn, res_sh, res_sw;
+    float inv_c4, inv_quads, inv_OH;
+};
+struct ProgEntry {
+    int32_t kind, u8_in, N, C, cs, HW, W;
+    float inv_W, lm1, off;
+    int64_t out_sn, out_sh;
+    ProgRef in, out;
+    ProgPtr tab;
+};
+struct ProgPool {
+    int32_t kind, k3, items;
+    ProgRef in, out;
+    PoolArgs a;
+};
+struct ProgExit {
+    int32_t kind, in_dtype;
+    ProgRef in, out;
+    ExitArgs a;
+};
+struct ProgEmbed {
+    int32_t kind, hidden, seq, pos0, pos1, tokens;
+    int64_t vocab;
+    ProgRef ids, out;
+    ProgPtr table, add0, add1;
+};
+struct ProgMvn {
+    int32_t kind, axis, rows, normalize, eps_inside;
+    float eps;
+    ProgRef in, out, outq;             // base < 0: absent
+    ProgPtr gamma, beta;
+    Requant fq;
+};
+struct ProgAttention {
+    int32_t kind, S, heads, units, waves, parts;   // waves of a workgroup that take 32 queries each, workgroups per (element, head)
+    ProgRef q, k, v, out, mask;
+    int32_t has_mask, pform;
+    AttentionArgs a;
+};
+struct ProgRows {
+    int32_t kind;
+    int64_t n;                        // elements (PK_FQROWS) or bytes (PK_COPY), a multiple of 16 bytes read
+    ProgRef in, out;
+    FqChannel p;
+    float lm1, off;
+};
+
+// Builds the step list while a plan is compiled.  Every method returns false when the single-launch form does not take
+// the step (the plan then has no program).
+struct ProgBuilder {
+    int device = 0;
+    int workgroups = 256;
+    std::vector<std::array<int32_t, kProgramStepWords>> steps;
+    std::vector<DeviceBuffer> owned;      // repacked weights, tables
+    ProgPtr keep(const void* host, size_t bytes);                              // a table of the program's own
+    ProgPtr gather(const std::vector<const void*>& rows, size_t pitch);
+    static uint8_t* fake_arena() { return reinterpret_cast<uint8_t*>(uintptr_t(1) << 32); }
+    static uint8_t* fake_io(int k) { return reinterpret_cast<uint8_t*>(uintptr_t(1) << 44) + (uintptr_t(k) << 40); }
+    static ProgRef ref(const void* p);     // of a pointer into one of the two
+    static ProgPtr ptr(const void* p) { return {static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p)), static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p) >> 32)}; }
+    template <typename T> void add(const T& s) {
+        static_assert(sizeof(T) <= kProgramStepWords * 4 && sizeof(T) % 4 == 0, "step descriptor");
+        std::array<int32_t, kProgramStepWords> w{};
+        std::memcpy(w.data(), &s, sizeof(T));
+        steps.push_back(w);
+    }
+    bool conv(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out);
+    bool entry(const hipie_fq* fq, bool u8_in, const void* in, const hipie_tensor& out);
+    bool pool(const PoolArgs& a, bool avg, bool rcp);
+    bool exit(const ExitArgs& a, int in_dtype);
+    bool embed(const float* table, int64_t vocab, int64_t hidden, const void* ids, int64_t tokens, int64_t seq, const float* add0, bool pos0,
+               const float* add1, bool pos1, void* out);
+    bool mvn(const void* in, void* out, void* outq, int64_t rows, int64_t axis, bool normalize, float eps, bool eps_inside, const float* gamma,
+             const float* beta, const hipie_requant* rq);
+    bool attention(const hipie_attention* att, const void* const (&qkv)[3], const int64_t (&ld)[3], const int64_t (&inner)[3],
+                   const int64_t (&outer)[3], void* out, int64_t ldo, int64_t so, int64_t oo, int batch, int batch_outer, const void* mask);
+    bool fq_rows(const hipie_fq* fq, const void* in, void* out, int out_dtype, int64_t n);
+    bool copy(const void* in, void* out, int64_t bytes);
+};
+
+// A plan's program: the step list on the device and the page-locked words the kernel reports failures in.
+struct Program {
+    int device = 0, workgroups = 0, n_steps = 0;
+    uint32_t roll_call_ticks = 0;
+    DeviceBuffer steps;
+    std::vector<DeviceBuffer> owned;
+    static constexpr int kSlots = 64;        // requests of one plan that can use the program
+    uint32_t* report = nullptr;              // page-locked, 16 dwords per slot
+    std::mutex lock;
+    uint64_t taken = 0;
+    ~Program();
+    int take_slot();                         // -1: none left
+    void give_slot(int slot);
+};
+std::unique_ptr<Program> make_program(ProgBuilder&& b);
+
+constexpr size_t kProgramControlBytes = 4096;    // barrier counters and the roll call's verdict: behind the arena, zero before the first launch
+// `launch`: how many launches used this control block before; io: the call's input and output buffers in order
+void launch_program(const Program& p, uint8_t* arena, void* const* io, int n_io, uint32_t* control, uint32_t launch, int slot, hipStream_t s);
+// after the stream has been waited for (or is about to be destroyed)
+void program_done(const Program& p, hipStream_t s);
+// what the last launch of a slot reported: 0 done; anything else: it did not run to its end, and `control` has been
+// cleared on the stream (the caller runs the inference by steps and counts its launches from zero again)
+bool program_failed(const Program& p, int slot, uint32_t* control, hipStream_t s);
+
+}  // namespace hipie

@@ -1,0 +1,1681 @@
+// The single-launch form of a plan (program.h says what it is for and why it is shaped like this).
+//
+// Convolution tiles use v_mfma_i32_16x16x64_i8 with the pixels as rows and the output channels as columns: a lane holds
+// four pixels of ONE channel per accumulator, so the epilogue's per-channel constants are one register each for the whole
+// tile.  (With channels as rows, as in the per-layer kernels, every lane needs four channels' constants per accumulator:
+// through LDS or as 16-byte loads they cost more than the arithmetic when a tile is this small.)  The A accumulators of a
+// tile hold neighbouring channels (the weights' packing sees to it), so a lane stores A bytes of a pixel at once, 16 lanes
+// its 16 A channels.  Both operands come from memory straight into operand registers: the weights of a tile are packed in
+// fragment order (1 KB per load), a pixel fragment is 64 contiguous bytes of 16 pixels.  Waves of a workgroup split a
+// tile's K (`ks`) where there are fewer tiles than waves: no byte is then loaded twice inside a workgroup, and the partial
+// sums meet in LDS.  Where a pixel's window starts and where its results go is a table (four words a pixel): decoding them
+// cost 200 instructions a tile, a sixth of a step.
+// Reference semantics: as conv_kernel.h, dwconv.hip, pool.hip, fq.hip, glue.hip and attention.hip - the arithmetic of every
+// step is the same sequence of f32 operations as in the per-step kernels, so the results are the same bits.
+#include "program.h"
+
+#include "div2.h"
+
+struct hipie_fq;
+
+namespace hipie {
+namespace {
+
+constexpr int kPartBytes = 128 * 1024;       // partial sums of eight waves x 16 fragments
+constexpr int kKoffBytes = 16 * 1024;        // K offsets of the step's convolutions
+constexpr int kMaxPieces = kKoffBytes / 4 / 2;
+constexpr int kLdsBytes = kPartBytes + kKoffBytes + 64;
+constexpr uint32_t kRollCallTicks = 3000000; // 30 ms of the 100 MHz clock
+constexpr uint64_t kBarrierTicks = 200000000;
+
+typedef __attribute__((address_space(3))) int8_t* lds_ptr;
+typedef __attribute__((address_space(3))) v4i* lds_v4i;
+typedef __attribute__((address_space(3))) int32_t* lds_i32;
+
+struct ProgArgs {
+    const int32_t* steps;
+    void* bases[1 + kProgramIo];             // the arena, the call's inputs and outputs (ProgRef::base)
+    uint32_t* control;
+    uint32_t* report;
+    int32_t n_steps, workgroups;
+    uint32_t launch, roll_call_ticks;
+};
+
+// control words: the root counter, the roll call's verdict, a counter per XCD (128 bytes apart)
+constexpr int kCtlRoot = 0, kCtlState = 32, kCtlXcd = 64;
+constexpr int kFlat = 128;                   // up to here every workgroup counts at the root (256 at one address: 4.8 us, by way of the XCDs 3.2)
+
+struct Ctx {
+    int rank, n_wg;                          // neighbouring ranks share an XCD
+    int tid, lane, wave;
+    uint32_t *root, *sub;                    // counters; sub null: flat
+    uint32_t root_target, sub_target;        // the values of the barrier that comes next
+    uint32_t* report;
+    bool dead;
+    lds_i32 flag;
+
+    // counts this workgroup (one lane); true when it completes the barrier
+    __device__ __forceinline__ bool count() {
+        if (sub) {
+            if (__hip_atomic_fetch_add(sub, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 != sub_target) return false;
+        }
+        return __hip_atomic_fetch_add(root, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == root_target;
+    }
+    __device__ __forceinline__ void next_targets() {
+        root_target += sub ? 8 : n_wg;
+        sub_target += n_wg / 8;
+    }
+    // The barrier between two steps comes in halves: every workgroup arrives with its stores acknowledged, then prepares the
+    // next step - descriptor, tile, weights, constants: nothing the step before it wrote - and only then waits.
+    __device__ __forceinline__ void arrive() {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        next_targets();
+        if (tid == 0) (void)count();
+    }
+    __device__ __forceinline__ void wait() {
+        if (tid == 0) {
+            int ok = 1;
+            if (static_cast<int32_t>(__hip_atomic_load(root, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - root_target) < 0) {
+                const uint64_t t0 = wall_clock64();
+                while (static_cast<int32_t>(__hip_atomic_load(root, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - root_target) < 0)
+                    if (wall_clock64() - t0 > kBarrierTicks) {
+                        ok = 0;
+                        break;
+                    }
+            }
+            if (!ok) __hip_atomic_store(report, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            flag[0] = ok;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        dead = __builtin_amdgcn_readfirstlane(flag[0]) == 0;
+    }
+};
+
+// A step's descriptor is read through the constant address space: scalar loads, at the place of use (a tile loop reads its
+// fields again from the scalar cache instead of keeping eighty of them in registers).
+#if defined(__HIP_DEVICE_COMPILE__)
+#define PROG_CONSTANT const __attribute__((address_space(4)))
+#else
+#define PROG_CONSTANT const
+#endif
+typedef PROG_CONSTANT int32_t* StepPtr;
+typedef PROG_CONSTANT ProgConv ConstConv;
+__device__ __forceinline__ StepPtr step_ptr(const int32_t* steps, int s) {
+    return (StepPtr)(reinterpret_cast<uintptr_t>(steps) + static_cast<uintptr_t>(s) * (kProgramStepWords * 4));
+}
+template <typename T>
+__device__ __forceinline__ T unpack(StepPtr p) {
+    constexpr int n = static_cast<int>(sizeof(T) / 4);
+    int32_t w[n];
+#pragma unroll
+    for (int i = 0; i < n; ++i) w[i] = p[i];
+    T t;
+    __builtin_memcpy(&t, w, sizeof(T));
+    return t;
+}
+// the same descriptor as a pointer the compiler knows nothing about: fields read through it are read here, not kept from before
+__device__ __forceinline__ ConstConv* again(ConstConv* c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(c));
+#endif
+    return c;
+}
+// (addresses made from integers are told to be global memory: as generic pointers their loads would be FLAT, which the
+// compiler waits for on the LDS counter as well)
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __attribute__((address_space(1))) uint8_t* GlobalBytes;
+#else
+typedef uint8_t* GlobalBytes;
+#endif
+// an operand's address: its base comes from the kernel's arguments by a scalar load
+__device__ __forceinline__ uint8_t* resolve(int32_t base, uint32_t lo, uint32_t hi) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef uint8_t* BasePtr;
+    typedef const __attribute__((address_space(4))) BasePtr* Bases;
+    Bases b = (Bases)((const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(ProgArgs, bases));
+    return (uint8_t*)(GlobalBytes)(reinterpret_cast<uintptr_t>(b[base]) + ((static_cast<uint64_t>(hi) << 32) | lo));
+#else
+    return nullptr;
+#endif
+}
+#define PROG_REF(x, r) resolve((r).base, (r).lo, (r).hi)
+#define PROG_TABLE(T, p) reinterpret_cast<const T*>((const uint8_t*)(GlobalBytes)((static_cast<uint64_t>((p).hi) << 32) | (p).lo))
+
+
+constexpr int kBeyond = 0x7ffffff0;          // a buffer offset no buffer reaches: loads give zero, stores nothing
+constexpr int kDeviceScope = 16;             // sc1: what another XCD wrote, or will read
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __amdgpu_buffer_rsrc_t Buffer;
+__device__ __forceinline__ Buffer make_buffer(const void* p) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, kBeyond, 0x00020000); }
+template <int AUX> __device__ __forceinline__ v4i load16(Buffer b, uint32_t o, int imm = 0) { return __builtin_amdgcn_raw_buffer_load_b128(b, static_cast<int>(o), imm, AUX); }
+__device__ __forceinline__ v4i shared16(Buffer b, uint32_t o) { return load16<kDeviceScope>(b, o); }
+__device__ __forceinline__ uint32_t shared4(Buffer b, uint32_t o) { return static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b32(b, static_cast<int>(o), 0, kDeviceScope)); }
+__device__ __forceinline__ uint32_t shared2(Buffer b, uint32_t o) { return static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(b, static_cast<int>(o), 0, kDeviceScope)); }
+__device__ __forceinline__ uint32_t shared1(Buffer b, uint32_t o) { return static_cast<uint8_t>(__builtin_amdgcn_raw_buffer_load_b8(b, static_cast<int>(o), 0, kDeviceScope)); }
+typedef int v2i __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ v2i shared8(Buffer b, uint32_t o) { return __builtin_amdgcn_raw_buffer_load_b64(b, static_cast<int>(o), 0, kDeviceScope); }
+__device__ __forceinline__ void publish16(Buffer b, uint32_t o, v4i v) { __builtin_amdgcn_raw_buffer_store_b128(v, b, static_cast<int>(o), 0, kDeviceScope); }
+__device__ __forceinline__ void publish8(Buffer b, uint32_t o, v2i v) { __builtin_amdgcn_raw_buffer_store_b64(v, b, static_cast<int>(o), 0, kDeviceScope); }
+__device__ __forceinline__ void publish4(Buffer b, uint32_t o, uint32_t v) { __builtin_amdgcn_raw_buffer_store_b32(static_cast<int>(v), b, static_cast<int>(o), 0, kDeviceScope); }
+__device__ __forceinline__ void publish2(Buffer b, uint32_t o, uint32_t v) { __builtin_amdgcn_raw_buffer_store_b16(static_cast<short>(v), b, static_cast<int>(o), 0, kDeviceScope); }
+__device__ __forceinline__ void publish1(Buffer b, uint32_t o, uint32_t v) { __builtin_amdgcn_raw_buffer_store_b8(static_cast<char>(v), b, static_cast<int>(o), 0, kDeviceScope); }
+#else
+typedef const void* Buffer;
+typedef int v2i __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ Buffer make_buffer(const void* p) { return p; }
+template <int AUX> __device__ __forceinline__ v4i load16(Buffer, uint32_t, int = 0) { return v4i{0, 0, 0, 0}; }
+__device__ __forceinline__ v4i shared16(Buffer, uint32_t) { return v4i{0, 0, 0, 0}; }
+__device__ __forceinline__ v2i shared8(Buffer, uint32_t) { return v2i{0, 0}; }
+__device__ __forceinline__ uint32_t shared4(Buffer, uint32_t) { return 0; }
+__device__ __forceinline__ uint32_t shared2(Buffer, uint32_t) { return 0; }
+__device__ __forceinline__ uint32_t shared1(Buffer, uint32_t) { return 0; }
+__device__ __forceinline__ void publish16(Buffer, uint32_t, v4i) {}
+__device__ __forceinline__ void publish8(Buffer, uint32_t, v2i) {}
+__device__ __forceinline__ void publish4(Buffer, uint32_t, uint32_t) {}
+__device__ __forceinline__ void publish2(Buffer, uint32_t, uint32_t) {}
+__device__ __forceinline__ void publish1(Buffer, uint32_t, uint32_t) {}
+#endif
+__device__ __forceinline__ float4 shared16f(Buffer b, uint32_t o) {
+    const v4i v = shared16(b, o);
+    return make_float4(__int_as_float(v.x), __int_as_float(v.y), __int_as_float(v.z), __int_as_float(v.w));
+}
+__device__ __forceinline__ void publish16f(Buffer b, uint32_t o, const float4& v) {
+    publish16(b, o, v4i{__float_as_int(v.x), __float_as_int(v.y), __float_as_int(v.z), __float_as_int(v.w)});
+}
+
+// ---- convolution --------------------------------------------------------------------------------------------------------
+
+// Operand registers of a tile: D K steps in flight.  The L2 is 600 - 1000 clocks away and a wave's share of K is a handful
+// of steps, so what counts is that all of them are requested at once, without a branch between two loads (behind a branch
+// the compiler waits for every load in flight): the ring is always filled, and a step behind the end is a buffer load out
+// of range (by its per-lane offset), which asks memory for nothing and adds zeros.
+template <int A, int B> constexpr int ring_depth() { return A * B >= 16 ? 2 : (A * B >= 8 ? 4 : 6); }
+template <int A, int B>
+struct Ring {
+    static constexpr int D = ring_depth<A, B>();
+    v4i w[D][A], p[D][B];
+};
+
+// where a wave's tile finds its K steps
+struct KSource {
+    Buffer w, in;
+    lds_i32 koff;
+    int kk, ks, nk;                          // the steps kk, kk + ks, .. of nk
+};
+
+template <int A, int B>
+__device__ __forceinline__ void load_weights(Ring<A, B>& g, const KSource& s, int d, int k, int lane) {
+    const uint32_t o = static_cast<uint32_t>(lane * 16) + static_cast<uint32_t>(k < s.nk ? k * (A * 1024) : kBeyond);
+#pragma unroll
+    for (int a = 0; a < A; ++a) g.w[d][a] = load16<0>(s.w, o, a * 1024);
+}
+template <int A, int B>
+__device__ __forceinline__ void load_pixels(Ring<A, B>& g, const KSource& s, const uint32_t (&off)[B], int d, int k, int lane) {
+    // (the K-offset table is read at the last step where k lies behind the end: what LDS holds there, added to kBeyond, could
+    // wrap round to an offset in range.  Contiguous K pieces come from a table too: a second form of the loop costs registers)
+    const uint32_t o = static_cast<uint32_t>(s.koff[4 * min(k, s.nk - 1) + (lane >> 4)]) + (k < s.nk ? 0u : static_cast<uint32_t>(kBeyond));
+#pragma unroll
+    for (int b = 0; b < B; ++b) g.p[d][b] = shared16(s.in, off[b] + o);
+}
+template <int A, int B>
+__device__ __forceinline__ void first_weights(Ring<A, B>& g, const KSource& s, int lane) {
+#pragma unroll
+    for (int d = 0; d < Ring<A, B>::D; ++d) load_weights<A, B>(g, s, d, s.kk + d * s.ks, lane);
+}
+
+// acc += the wave's K steps; the first D steps' weights are already on their way (first_weights)
+template <int A, int B>
+__device__ __forceinline__ void k_loop(Ring<A, B>& g, const KSource& s, const uint32_t (&off)[B], int lane, v4i (&acc)[A][B]) {
+    constexpr int D = Ring<A, B>::D;
+    auto multiply = [&](int d) {
+#pragma unroll
+        for (int a = 0; a < A; ++a)
+#pragma unroll
+            for (int b = 0; b < B; ++b) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(g.p[d][b], g.w[d][a], acc[a][b], 0, 0, 0);
+    };
+    int k = s.kk;
+#pragma unroll
+    for (int d = 0; d < D; ++d) load_pixels<A, B>(g, s, off, d, k + d * s.ks, lane);
+    while (k + D * s.ks < s.nk) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            multiply(d);
+            load_weights<A, B>(g, s, d, k + (d + D) * s.ks, lane);
+            load_pixels<A, B>(g, s, off, d, k + (d + D) * s.ks, lane);
+        }
+        k += D * s.ks;
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (d == 0 || k + d * s.ks < s.nk) multiply(d);
+}
+
+template <int A>
+struct ChannelConstants {
+    int32_t corr[A];
+    float bias[A], scale[A], rmul[A], il[A], ih[A], r[A];
+    float r2[A];                             // the second word of the two-operation division, else the divisor
+};
+
+template <int A, typename T>
+__device__ __forceinline__ void load_channels(const T* p, T (&v)[A]) {
+    if constexpr (A == 4) {
+        const uint4 t = *reinterpret_cast<const uint4*>(p);
+        v[0] = __builtin_bit_cast(T, t.x); v[1] = __builtin_bit_cast(T, t.y); v[2] = __builtin_bit_cast(T, t.z); v[3] = __builtin_bit_cast(T, t.w);
+    } else if constexpr (A == 2) {
+        const uint2 t = *reinterpret_cast<const uint2*>(p);
+        v[0] = __builtin_bit_cast(T, t.x); v[1] = __builtin_bit_cast(T, t.y);
+    } else v[0] = p[0];
+}
+
+// The tables a step uses, one row of OCp words each, behind one another in this order (ProgBuilder::constants)
+template <int A>
+__device__ __forceinline__ void load_constants(ConstConv& c, int oc, ChannelConstants<A>& k) {
+    const uint32_t fl = c.flags;
+    const uint8_t* row = PROG_TABLE(uint8_t, c.constants) + oc * 4;
+    const int pitch = c.OCp * 4;
+    auto next = [&](auto& v) {
+        typedef std::remove_reference_t<decltype(v[0])> T;
+        load_channels<A>(reinterpret_cast<const T*>(row), v);
+        row += pitch;
+    };
+    next(k.corr);
+    if (fl & CF_BIAS) next(k.bias);
+    if (fl & CF_SCALE) next(k.scale);
+    if (fl & CF_RES_MUL) next(k.rmul);
+    if (fl & CF_OUT_FQ) {
+        next(k.r);
+        next(k.r2);
+        if (!(fl & CF_FQ_SAT)) next(k.ih);
+        if (!(fl & CF_FQ_IL0)) next(k.il);
+    }
+}
+
+// four pixels of the output: byte offsets in the output and residual tensors (kBeyond: not there), and their residual values
+template <int A>
+struct PixelQuad {
+    uint32_t out[4], res[4];
+    static constexpr int kRaw = A == 4 ? 1 : A;
+    uint32_t raw[4][kRaw];                   // A bytes in raw[.][0], or A f32 values (A = 4: those are loaded where they are used)
+};
+template <int A>
+__device__ __forceinline__ void load_residual(ConstConv& c, Buffer res, int oc, PixelQuad<A>& q) {
+    const uint32_t fl = c.flags;
+    if (!(fl & CF_RES) || (fl & CF_RES_GEMM)) return;
+    const bool f32 = fl & CF_RES_F32;
+    const uint32_t o = oc < c.res_limit ? static_cast<uint32_t>(f32 ? 4 * oc : oc) : static_cast<uint32_t>(kBeyond);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if (f32) {
+            if constexpr (A == 2) {
+                const v2i v = shared8(res, q.res[r] + o);
+                q.raw[r][0] = v.x; q.raw[r][1] = v.y;
+            } else if constexpr (A == 1) q.raw[r][0] = shared4(res, q.res[r] + o);
+        } else {
+            if constexpr (A == 4) q.raw[r][0] = shared4(res, q.res[r] + o);
+            else if constexpr (A == 2) q.raw[r][0] = shared2(res, q.res[r] + o);
+            else q.raw[r][0] = shared1(res, q.res[r] + o);
+        }
+    }
+}
+
+// the fused f32 chain (conv_epilogue.h) on A neighbouring channels of four pixels, and their store
+template <int A, bool PAIR = false>
+__device__ __forceinline__ void finish(ConstConv& c, Buffer out, Buffer res, const ChannelConstants<A>& k, const v4i (&sum)[A], const float (&rgemm)[A][4],
+                                       const PixelQuad<A>& q, int oc) {
+    const uint32_t fl = c.flags;
+    float x[A][4];
+#define PROG_EACH for (int a = 0; a < A; ++a) for (int r = 0; r < 4; ++r)
+#pragma unroll
+    PROG_EACH x[a][r] = static_cast<float>(sum[a][r]);
+    if (fl & CF_BIAS) {
+#pragma unroll
+        PROG_EACH x[a][r] = x[a][r] + k.bias[a];
+    }
+    if (fl & CF_SCALE) {
+#pragma unroll
+        PROG_EACH x[a][r] = x[a][r] * k.scale[a];
+    }
+    if (fl & CF_RES) {
+        float rv[A][4];
+        if constexpr (PAIR) {
+#pragma unroll
+            PROG_EACH rv[a][r] = rgemm[a][r];
+        } else if (fl & CF_RES_F32) {
+            if constexpr (A == 4) {
+                const uint32_t o = oc < c.res_limit ? static_cast<uint32_t>(4 * oc) : static_cast<uint32_t>(kBeyond);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float4 v = shared16f(res, q.res[r] + o);
+                    rv[0][r] = v.x; rv[1][r] = v.y; rv[2][r] = v.z; rv[3][r] = v.w;
+                }
+            } else {
+#pragma unroll
+                PROG_EACH rv[a][r] = __uint_as_float(q.raw[r][a]);
+            }
+        } else if (fl & CF_RES_U8B) {
+#pragma unroll
+            PROG_EACH rv[a][r] = res_byte_to_float<true>(q.raw[r][0], a);
+        } else {
+#pragma unroll
+            PROG_EACH rv[a][r] = res_byte_to_float<false>(q.raw[r][0], a);
+        }
+        if (fl & CF_RES_MUL) {
+#pragma unroll
+            PROG_EACH rv[a][r] = rv[a][r] * k.rmul[a];
+        }
+#pragma unroll
+        PROG_EACH x[a][r] = x[a][r] + rv[a][r];
+    }
+    if (fl & CF_RELU) {
+#pragma unroll
+        PROG_EACH x[a][r] = x[a][r] > 0.0f ? x[a][r] : 0.0f;
+    }
+    if (fl & CF_CLAMP) {
+        if (fl & CF_OUT_FQ) {
+#pragma unroll
+            PROG_EACH x[a][r] = __builtin_amdgcn_fmed3f(x[a][r], c.clamp_lo, c.clamp_hi);
+        } else {
+#pragma unroll
+            PROG_EACH x[a][r] = x[a][r] < c.clamp_lo ? c.clamp_lo : (x[a][r] > c.clamp_hi ? c.clamp_hi : x[a][r]);
+        }
+    }
+    if constexpr (A != 1)                    // (choose_tile)
+        if (fl & CF_GELU) {
+#pragma unroll
+            PROG_EACH x[a][r] = gelu_one(x[a][r]);
+        }
+    if (!(fl & CF_OUT_FQ)) {
+        const uint32_t o = oc < c.out_limit ? static_cast<uint32_t>(4 * oc) : static_cast<uint32_t>(kBeyond);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if constexpr (A == 4) publish16f(out, q.out[r] + o, make_float4(x[0][r], x[1][r], x[2][r], x[3][r]));
+            else if constexpr (A == 2) publish8(out, q.out[r] + o, v2i{__float_as_int(x[0][r]), __float_as_int(x[1][r])});
+            else publish4(out, q.out[r] + o, __float_as_uint(x[0][r]));
+        }
+        return;
+    }
+    // level index: as fq_level_fast, operation by operation
+    const bool il0 = (fl & CF_FQ_IL0) != 0;
+    if (!(fl & CF_FQ_SAT)) {
+#pragma unroll
+        PROG_EACH x[a][r] = __builtin_amdgcn_fmed3f(x[a][r], il0 ? 0.f : k.il[a], k.ih[a]);
+    }
+    if (!il0) {
+#pragma unroll
+        PROG_EACH x[a][r] = x[a][r] - k.il[a];
+    }
+    if (fl & CF_FQ_DIV2) {
+#pragma unroll
+        PROG_EACH x[a][r] = fmaf(x[a][r], k.r[a], x[a][r] * k.r2[a]) * c.lm1;
+    } else {                                 // CF_FQ_RCP: the builder takes no layer whose ranges need the dividing form
+#pragma unroll
+        PROG_EACH {
+            const float n = x[a][r], d = k.r2[a];
+            const float q0 = n * k.r[a];
+            const float e0 = fmaf(-d, q0, n);
+            const float q1 = fmaf(e0, k.r[a], q0);
+            const float e1 = fmaf(-d, q1, n);
+            x[a][r] = fmaf(e1, k.r[a], q1) * c.lm1;
+        }
+    }
+    const uint32_t xmask = (fl & CF_OUT_XOR) ? 0x80808080u : 0u;
+    const uint32_t o = oc < c.out_limit ? static_cast<uint32_t>(oc) : static_cast<uint32_t>(kBeyond);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        uint32_t w = 0;
+#pragma unroll
+        for (int a = 0; a < A; ++a) w = __builtin_amdgcn_cvt_pk_u8_f32(x[a][r], a, w);
+        if (fl & CF_OUT_ADD) w = add_bytes(w, (static_cast<uint32_t>(static_cast<int>(c.out_off)) & 0xffu) * 0x01010101u);
+        w ^= xmask;
+        if constexpr (A == 4) publish4(out, q.out[r] + o, w);
+        else if constexpr (A == 2) publish2(out, q.out[r] + o, w);
+        else publish1(out, q.out[r] + o, w);
+    }
+#undef PROG_EACH
+}
+
+// A step's K offsets into LDS.  Every lane takes part in every round (those behind the end repeat the last entry): no lane
+// is masked off here.  The compiler's live-range splitting may put the copy of a register that merely lives through a masked
+// region in front of the instruction that ends the mask, which leaves the other lanes' values behind - seen with the
+// lane-derived addresses of a later attention step around a divergent form of this loop.
+__device__ __forceinline__ void stage_offsets(lds_i32 to, const int32_t* from, int n, int tid) {
+    for (int base = 0; base < n; base += kProgramThreads) {
+        const int i = min(base + tid, n - 1);
+        to[i] = from[i];
+    }
+}
+
+template <int A, int B, bool PAIR = false>     // PAIR: a projection shortcut as a second product (F <= 8: room for two sets of partial sums)
+__device__ __forceinline__ void conv_tiles(ConstConv* desc, Ctx& x, lds_ptr lds) {
+    constexpr int F = A * B;                  // fragments of a tile
+    lds_i32 koff = (lds_i32)(lds + kPartBytes);
+    KSource src, src2{};
+    int per, sub, t0, t1;
+    {
+        ConstConv& c = *again(desc);
+        const int32_t* ko = PROG_TABLE(int32_t, c.koff);
+        const int shift = c.ks_shift;
+        src.ks = 1 << shift;
+        per = 8 >> shift;                     // waves per tile, tiles a workgroup works on at once
+        sub = x.wave >> shift;
+        src.kk = x.wave & (src.ks - 1);
+        src.koff = koff;
+        src.nk = c.nk;
+        src.in = make_buffer(PROG_REF(x, c.in));
+        stage_offsets(koff, ko, 4 * c.nk, x.tid);
+        if constexpr (PAIR) {
+            const int32_t* ko2 = PROG_TABLE(int32_t, c.koff2);
+            stage_offsets(koff + kMaxPieces, ko2, 4 * c.nk2, x.tid);
+            src2 = src;
+            src2.koff = koff + kMaxPieces;
+            src2.nk = c.nk2;
+            src2.in = make_buffer(PROG_REF(x, c.in2));
+        }
+        t0 = static_cast<int>(static_cast<uint32_t>(x.rank) * static_cast<uint32_t>(c.tiles) / static_cast<uint32_t>(x.n_wg));
+        t1 = static_cast<int>(static_cast<uint32_t>(x.rank + 1) * static_cast<uint32_t>(c.tiles) / static_cast<uint32_t>(x.n_wg));
+    }
+    lds_v4i part = (lds_v4i)lds + x.wave * (F * 64) + x.lane;
+    lds_v4i part2 = (lds_v4i)(lds + kPartBytes / 2) + x.wave * (F * 64) + x.lane;
+    const lds_v4i mine = (lds_v4i)lds + sub * src.ks * (F * 64) + x.lane, mine2 = (lds_v4i)(lds + kPartBytes / 2) + sub * src.ks * (F * 64) + x.lane;
+    bool first = true;
+    int base = t0;
+    do {
+        const int tile = base + sub;
+        const bool on = tile < t1;
+        ChannelConstants<A> k;
+        ChannelConstants<A> k2;
+        Ring<A, B> ring;
+        uint32_t off[B], off2[B];
+        PixelQuad<A> q;
+        int mt, oc;
+        const int kk = src.kk, lane16 = x.lane & 15, quad = x.lane >> 4;
+        {
+            ConstConv& c = *again(desc);
+            int ot = 0, pt = 0;
+            if (on) fast_divmod(tile, c.p_tiles, c.inv_p_tiles, ot, pt);
+            ot = __builtin_amdgcn_readfirstlane(ot);
+            pt = __builtin_amdgcn_readfirstlane(pt);
+            mt = pt * (16 * B);
+            oc = ot * (16 * A) + A * lane16;
+            const uint32_t* pix = PROG_TABLE(uint32_t, c.pixels);
+            src.w = make_buffer(PROG_TABLE(int8_t, c.wgt) + static_cast<int64_t>(ot) * c.nk * (A * 1024));
+#pragma unroll
+            for (int b = 0; b < B; ++b) off[b] = pix[mt + 16 * b + lane16];
+            if constexpr (PAIR) {
+                src2.w = make_buffer(PROG_TABLE(int8_t, c.wgt2) + static_cast<int64_t>(ot) * c.nk2 * (A * 1024));
+#pragma unroll
+                for (int b = 0; b < B; ++b) off2[b] = pix[3 * c.M + mt + 16 * b + lane16];
+                first_weights<A, B>(ring, src2, x.lane);
+                const int32_t* t2 = PROG_TABLE(int32_t, c.constants2) + oc;
+                load_channels<A>(t2, k2.corr);
+                load_channels<A>(reinterpret_cast<const float*>(t2 + c.OCp), k2.bias);
+                load_channels<A>(reinterpret_cast<const float*>(t2 + 2 * c.OCp), k2.scale);
+            } else {
+                first_weights<A, B>(ring, src, x.lane);
+            }
+            load_constants<A>(c, oc, k);
+            // the first column this wave finishes
+            const uint4 po = *reinterpret_cast<const uint4*>(pix + c.M + mt + 16 * (kk & (B - 1)) + 4 * quad);
+            const uint4 pr = *reinterpret_cast<const uint4*>(pix + 2 * c.M + mt + 16 * (kk & (B - 1)) + 4 * quad);
+            q.out[0] = po.x; q.out[1] = po.y; q.out[2] = po.z; q.out[3] = po.w;
+            q.res[0] = pr.x; q.res[1] = pr.y; q.res[2] = pr.z; q.res[3] = pr.w;
+        }
+        if (first) {
+            x.wait();
+            first = false;
+            if (x.dead) return;
+        }
+        v4i acc[A][B];
+        auto start = [&](const int32_t (&corr)[A]) {      // the sum starts from the channel's integer correction, once per tile
+#pragma unroll
+            for (int a = 0; a < A; ++a) {
+                const int c0 = kk == 0 ? corr[a] : 0;
+#pragma unroll
+                for (int b = 0; b < B; ++b) acc[a][b] = v4i{c0, c0, c0, c0};
+            }
+        };
+        auto put = [&](lds_v4i to) {
+#pragma unroll
+            for (int a = 0; a < A; ++a)
+#pragma unroll
+                for (int b = 0; b < B; ++b) to[(b * A + a) * 64] = acc[a][b];
+        };
+        if (on) {
+            if constexpr (PAIR) {
+                start(k2.corr);
+                k_loop<A, B>(ring, src2, off2, x.lane, acc);
+                first_weights<A, B>(ring, src, x.lane);
+                put(part2);
+            }
+            start(k.corr);
+            if (kk < B) load_residual<A>(*desc, make_buffer(resolve(max(desc->res.base, 0), desc->res.lo, desc->res.hi)), oc, q);
+            k_loop<A, B>(ring, src, off, x.lane, acc);
+            put(part);
+        }
+        if (src.ks > 1) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        }
+        if (on && kk < B) {
+            ConstConv& c = *again(desc);
+            const Buffer out = make_buffer(PROG_REF(x, c.out)), res = make_buffer(resolve(max(c.res.base, 0), c.res.lo, c.res.hi));
+            for (int b = kk;;) {
+                v4i sum[A];
+                float rg[A][4] = {};
+#pragma unroll
+                for (int a = 0; a < A; ++a) sum[a] = mine[(b * A + a) * 64];
+                for (int s = 1; s < src.ks; ++s)
+#pragma unroll
+                    for (int a = 0; a < A; ++a) sum[a] += mine[s * (F * 64) + (b * A + a) * 64];
+                if constexpr (PAIR) {
+                    v4i s2[A];
+#pragma unroll
+                    for (int a = 0; a < A; ++a) s2[a] = mine2[(b * A + a) * 64];
+                    for (int s = 1; s < src.ks; ++s)
+#pragma unroll
+                        for (int a = 0; a < A; ++a) s2[a] += mine2[s * (F * 64) + (b * A + a) * 64];
+#pragma unroll
+                    for (int a = 0; a < A; ++a)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) rg[a][r] = (static_cast<float>(s2[a][r]) + k2.bias[a]) * k2.scale[a];
+                }
+                finish<A, PAIR>(c, out, res, k, sum, rg, q, oc);
+                b += src.ks;
+                if (b >= B) break;
+                const uint32_t* pix = PROG_TABLE(uint32_t, c.pixels);
+                const uint4 po = *reinterpret_cast<const uint4*>(pix + c.M + mt + 16 * b + 4 * quad);
+                const uint4 pr = *reinterpret_cast<const uint4*>(pix + 2 * c.M + mt + 16 * b + 4 * quad);
+                q.out[0] = po.x; q.out[1] = po.y; q.out[2] = po.z; q.out[3] = po.w;
+                q.res[0] = pr.x; q.res[1] = pr.y; q.res[2] = pr.z; q.res[3] = pr.w;
+                load_residual<A>(c, res, oc, q);
+            }
+        }
+        base += per;
+        if (src.ks > 1 && base < t1) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        }
+    } while (base < t1);
+}
+
+// ---- depthwise 3 x 3 ----------------------------------------------------------------------------------------------------
+// A lane owns four channels of four output pixels of a row: six (stride 1) or nine columns of three input rows, byte
+// transposes (v_perm) and v_dot4_i32_i8 as in dwconv.hip; consecutive lanes take consecutive channels.
+template <int STRIDE>
+__device__ __forceinline__ void dw_items(ConstConv& c, Ctx& x) {
+    constexpr int COLS = 3 + 3 * STRIDE;
+    const int OH = c.OH, items = c.items, stride = 8 * x.n_wg * 64;
+    const Buffer in = make_buffer(PROG_REF(x, c.in)), out = make_buffer(PROG_REF(x, c.out)), res = make_buffer(resolve(max(c.res.base, 0), c.res.lo, c.res.hi));
+    const int last_col = (c.OW - 1) * STRIDE + 2;
+    bool first = true;
+    int i0 = (x.wave * x.n_wg + x.rank) * 64;
+    do {
+        const int item = min(i0 + x.lane, items - 1);
+        const bool on = i0 + x.lane < items;
+        int q, c4, row, quad, n, oh;
+        fast_divmod(item, c.c4, c.inv_c4, q, c4);
+        fast_divmod(q, c.quads, c.inv_quads, row, quad);
+        fast_divmod(row, OH, c.inv_OH, n, oh);
+        const int oc = 4 * c4, ow0 = 4 * quad;
+        const uint32_t p = static_cast<uint32_t>(n * c.in_sn + oh * c.in_sh + oc);
+        uint32_t v[3][COLS];
+        uint4 wr[3];
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+            wr[r] = *reinterpret_cast<const uint4*>(PROG_TABLE(int8_t, c.wgt) + (static_cast<int64_t>(r) * c.OCp + oc) * 4);
+        ChannelConstants<4> k;
+        load_constants<4>(c, oc, k);
+        uint32_t col[COLS];
+#pragma unroll
+        for (int j = 0; j < COLS; ++j) col[j] = p + static_cast<uint32_t>(min(ow0 * STRIDE + j, last_col) * c.in_sw);
+        PixelQuad<4> pq;
+        {
+            const bool f32 = c.flags & CF_RES_F32, fo = !(c.flags & CF_OUT_FQ);
+            const uint32_t o = static_cast<uint32_t>(n * c.out_sn + oh * c.out_sh), s = static_cast<uint32_t>(n * c.res_sn + oh * c.res_sh);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int ow = min(ow0 + r, c.OW - 1);
+                pq.out[r] = on && ow0 + r < c.OW ? (o + ow * c.out_sw) << (fo ? 2 : 0) : static_cast<uint32_t>(kBeyond);
+                pq.res[r] = (s + ow * c.res_sw) << (f32 ? 2 : 0);
+            }
+        }
+        if (first) {
+            x.wait();
+            first = false;
+            if (x.dead) return;
+        }
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+#pragma unroll
+            for (int j = 0; j < COLS; ++j) v[r][j] = shared4(in, col[j] + static_cast<uint32_t>(r * c.row_sh));
+        load_residual<4>(c, res, oc, pq);
+        v4i acc[4];                           // [channel][pixel]
+#pragma unroll
+        for (int a = 0; a < 4; ++a) acc[a] = v4i{k.corr[a], k.corr[a], k.corr[a], k.corr[a]};
+        auto transpose4 = [&](uint32_t p0, uint32_t p1, uint32_t p2, uint32_t p3, uint32_t (&t)[4]) {
+            const uint32_t lo01 = __builtin_amdgcn_perm(p1, p0, 0x05010400u), hi01 = __builtin_amdgcn_perm(p1, p0, 0x07030602u);
+            const uint32_t lo23 = __builtin_amdgcn_perm(p3, p2, 0x05010400u), hi23 = __builtin_amdgcn_perm(p3, p2, 0x07030602u);
+            t[0] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+            t[1] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+            t[2] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+            t[3] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+        };
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            const uint32_t w[4] = {wr[r].x, wr[r].y, wr[r].z, wr[r].w};
+            if constexpr (STRIDE == 1) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    uint32_t t[4];
+                    transpose4(v[r][2 * h], v[r][2 * h + 1], v[r][2 * h + 2], v[r][2 * h + 3], t);
+#pragma unroll
+                    for (int a = 0; a < 4; ++a) {
+                        acc[a][2 * h] = __builtin_amdgcn_sdot4(static_cast<int>(t[a]), static_cast<int>(w[a]), acc[a][2 * h], false);
+                        acc[a][2 * h + 1] = __builtin_amdgcn_sdot4(static_cast<int>(t[a]), static_cast<int>(w[a] << 8), acc[a][2 * h + 1], false);
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int h = 0; h < 4; ++h) {
+                    uint32_t t[4];
+                    transpose4(v[r][2 * h], v[r][2 * h + 1], v[r][2 * h + 2], v[r][2 * h + 2], t);
+#pragma unroll
+                    for (int a = 0; a < 4; ++a) acc[a][h] = __builtin_amdgcn_sdot4(static_cast<int>(t[a]), static_cast<int>(w[a]), acc[a][h], false);
+                }
+            }
+        }
+        const float none[4][4] = {};
+        finish<4>(c, out, res, k, acc, none, pq, oc);
+        i0 += stride;
+    } while (i0 < items);
+}
+
+// ---- entry, pooling, exit ---------------------------------------------------------------------------------------------------
+__device__ __forceinline__ uint32_t level_bytes(const FqChannel& f, float lm1, float off, float v) {
+    return static_cast<uint32_t>(static_cast<int>(fq_level_clamped<true>(f, lm1, v) + off)) & 0xffu;
+}
+
+__device__ __forceinline__ void entry_items(const ProgEntry& e, const Ctx& x) {
+    const uint8_t* in = PROG_REF(x, e.in);
+    const Buffer out = make_buffer(PROG_REF(x, e.out));
+    const FqChannel* tab = PROG_TABLE(FqChannel, e.tab);
+    const int groups = e.cs / 4, waves_per_plane = (e.HW + 63) / 64;       // four channels of 64 pixels of one image
+    const int items = e.N * groups * waves_per_plane;
+    for (int i = x.wave * x.n_wg + x.rank; i < items; i += 8 * x.n_wg) {
+        const int pw = i % waves_per_plane, np = i / waves_per_plane, g = np % groups, n = np / groups;
+        const int p = pw * 64 + x.lane;
+        const bool on = p < e.HW;
+        int h, w;
+        fast_divmod(on ? p : 0, e.W, e.inv_W, h, w);
+        const int64_t src = (static_cast<int64_t>(n) * e.C + 4 * g) * e.HW + (on ? p : 0);
+        float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (4 * g + j < e.C) {
+                const int64_t o = src + static_cast<int64_t>(j) * e.HW;
+                v[j] = e.u8_in ? static_cast<float>(in[o]) : reinterpret_cast<const float*>(in)[o];
+            }
+        uint32_t dw = (static_cast<uint32_t>(static_cast<int>(e.off)) & 0xffu) * 0x01010101u;     // level 0 in the channels that do not exist
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (4 * g + j < e.C) dw = (dw & ~(0xffu << (8 * j))) | (level_bytes(tab[4 * g + j], e.lm1, e.off, v[j]) << (8 * j));
+        publish4(out, on ? static_cast<uint32_t>(n * e.out_sn + h * e.out_sh + static_cast<int64_t>(w) * e.cs + 4 * g) : static_cast<uint32_t>(kBeyond), dw);
+    }
+}
+
+// bytewise running maxima in the order-preserving unsigned domain, as pool.hip
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void max_take(uint32_t stored, uint32_t& even, uint32_t& odd) {
+    const uint32_t v = stored ^ 0x80808080u;
+    even = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, even), __builtin_bit_cast(u16x2, v & 0x00ff00ffu)));
+    odd = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, odd), __builtin_bit_cast(u16x2, v & 0xff00ff00u)));
+}
+
+__device__ __forceinline__ void max_pool_items(const ProgPool& s, const Ctx& x) {
+    const PoolArgs& a = s.a;
+    const int cg = a.cs / 4;
+    const Buffer in = make_buffer(PROG_REF(x, s.in)), out = make_buffer(PROG_REF(x, s.out));
+    for (int i0 = (x.wave * x.n_wg + x.rank) * 64; i0 < s.items; i0 += 8 * x.n_wg * 64) {
+        const int t = i0 + x.lane;
+        if (t >= s.items) continue;
+        const int m = t / cg, c = (t - m * cg) * 4;
+        const int n = m / a.OHOW, rem = m - n * a.OHOW, oh = rem / a.OW, ow = rem - oh * a.OW;
+        const int y0 = oh * a.sh - a.pt, x0 = ow * a.sw - a.pl;
+        const uint32_t base = static_cast<uint32_t>(n * a.in_sn + c);
+        uint32_t even = 0, odd = 0;
+        if (s.k3) {
+            uint32_t v[9];
+#pragma unroll
+            for (int j = 0; j < 9; ++j) {
+                const int yy = min(max(y0 + j / 3, 0), a.H - 1), xx = min(max(x0 + j % 3, 0), a.W - 1);
+                v[j] = shared4(in, base + static_cast<uint32_t>(yy * a.in_sh + xx * a.in_sw));
+            }
+#pragma unroll
+            for (int j = 0; j < 9; ++j) max_take(v[j], even, odd);
+        } else {
+            const int ya = max(y0, 0), xa = max(x0, 0);
+            const int yb = min(min(y0 + a.kh, a.H + a.pb), a.H), xb = min(min(x0 + a.kw, a.W + a.pr), a.W);
+            for (int yy = ya; yy < yb; ++yy)
+                for (int xx = xa; xx < xb; ++xx) max_take(shared4(in, base + static_cast<uint32_t>(yy * a.in_sh + xx * a.in_sw)), even, odd);
+        }
+        publish4(out, static_cast<uint32_t>(n * a.out_sn + oh * a.out_sh + ow * a.out_sw + c), (even | odd) ^ 0x80808080u);
+    }
+}
+
+// Average pool: sixteen lanes share a window (a lane sums every sixteenth cell of four channels), so that a global pool of
+// one image - a few hundred outputs of 49 cells - still has all of the group's waves loading.
+__device__ __forceinline__ void avg_pool_items(const ProgPool& s, const Ctx& x) {
+    const PoolArgs& a = s.a;
+    const int cg = a.cs / 4, items = s.items;
+    const Buffer in = make_buffer(PROG_REF(x, s.in)), out = make_buffer(PROG_REF(x, s.out));
+    const int share = x.lane >> 2;            // lanes 4 q + j of a wave: share q of item j
+    for (int i0 = (x.wave * x.n_wg + x.rank) * 4; i0 < items; i0 += 8 * x.n_wg * 4) {
+        const int t = min(i0 + (x.lane & 3), items - 1);
+        const int m = t / cg, c = (t - m * cg) * 4;
+        const int n = m / a.OHOW, rem = m - n * a.OHOW, oh = rem / a.OW, ow = rem - oh * a.OW;
+        const int y0 = oh * a.sh - a.pt, x0 = ow * a.sw - a.pl;
+        const int y1 = min(y0 + a.kh, a.H + a.pb), x1 = min(x0 + a.kw, a.W + a.pr);
+        const bool padding_present = a.pt || a.pl || a.pb || a.pr;
+        const int ya = max(y0, 0), yb = min(y1, a.H), xa = max(x0, 0), xb = min(x1, a.W);
+        const int wx = max(xb - xa, 0), cells = max(yb - ya, 0) * wx;
+        int count = padding_present ? cells : (y1 - y0) * (x1 - x0);
+        const uint32_t base = static_cast<uint32_t>(n * a.in_sn + c);
+        int sum[4] = {0, 0, 0, 0};
+        for (int j = share; j < cells; j += 64) {
+            uint32_t v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int jj = min(j + 16 * u, cells - 1), yy = jj / wx, xx = jj - yy * wx;
+                v[u] = shared4(in, base + static_cast<uint32_t>((ya + yy) * a.in_sh + (xa + xx) * a.in_sw));
+                if (j + 16 * u >= cells) v[u] = 0;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) sum[b] += static_cast<int8_t>(v[u] >> (8 * b));
+        }
+#pragma unroll
+        for (int o = 4; o < 64; o <<= 1)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) sum[b] += __shfl_xor(sum[b], o, 64);
+        if (share != 0 || i0 + (x.lane & 3) >= items) continue;
+        if (a.include_pad && padding_present) count = a.kh * a.kw;
+        const float nf = static_cast<float>(count);
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float t4 = static_cast<float>(sum[j] + a.in_bias * cells) / nf;
+            if (a.mul) t4 = t4 * a.mul[c + j];
+            v[j] = t4;
+        }
+        const uint32_t o = static_cast<uint32_t>(n * a.out_sn + oh * a.out_sh + ow * a.out_sw + c);
+        if (a.preserve) {
+            uint32_t packed = 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int total = sum[j] + a.in_bias * cells;
+                const int r = a.preserve == 1 ? (total & 0xff) : static_cast<int>(static_cast<int8_t>(total & 0xff));
+                const int level = static_cast<int>(__builtin_rintf(static_cast<float>(r) / nf));
+                packed |= (static_cast<uint32_t>(level - (a.preserve == 1 ? 128 : 0)) & 0xffu) << (8 * j);
+            }
+            publish4(out, o, packed);
+        } else if (a.fq_il) {
+            uint32_t packed = 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                FqChannel p;
+                p.il = a.fq_il[c + j]; p.ih = a.fq_ih[c + j]; p.d = a.fq_d[c + j]; p.r = a.fq_r[c + j];
+                packed |= level_bytes(p, a.lm1, a.out_off, v[j]) << (8 * j);
+            }
+            publish4(out, o, packed);
+        } else {
+            publish16f(out, 4 * o, make_float4(v[0], v[1], v[2], v[3]));
+        }
+    }
+}
+
+// (the caller's output buffer: nothing in the launch reads it)
+template <typename TIn>
+__device__ __forceinline__ void exit_items(const ProgExit& s, const Ctx& x) {
+    const ExitArgs& a = s.a;
+    const Buffer in = make_buffer(PROG_REF(x, s.in));
+    uint8_t* out = PROG_REF(x, s.out);
+    auto one = [&](const TIn raw, int n, int c, int p) {
+        float v = static_cast<float>(raw) + a.in_bias;
+        if (a.sub) v = v - a.sub[c];
+        if (a.mul) v = v * a.mul[c];
+        const int64_t o = (static_cast<int64_t>(n) * a.C + c) * a.HW + p;
+        if (a.out_u8) out[o] = static_cast<uint8_t>(static_cast<int>(v));
+        else reinterpret_cast<float*>(out)[o] = v;
+    };
+    if (a.HW >= 16) {                        // lanes along the pixels, four channels each (a pixel's channels are padded to four)
+        const int waves = (a.HW + 63) / 64, cg = (a.C + 3) / 4, items = a.N * cg * waves;
+        for (int i = x.wave * x.n_wg + x.rank; i < items; i += 8 * x.n_wg) {
+            const int pw = i % waves, ng = i / waves, g = ng % cg, n = ng / cg, p = pw * 64 + x.lane;
+            if (p >= a.HW) continue;
+            const int h = p / a.W, w = p - h * a.W;
+            const uint32_t q = static_cast<uint32_t>(n * a.in_sn + h * a.in_sh + w * a.in_sw + 4 * g) * sizeof(TIn);
+            TIn raw[4];
+            if constexpr (sizeof(TIn) == 4) {
+                const v4i t = shared16(in, q);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int32_t word = t[j];
+                    raw[j] = __builtin_bit_cast(TIn, word);
+                }
+            } else {
+                const uint32_t t = shared4(in, q);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) raw[j] = static_cast<TIn>(t >> (8 * j));
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (4 * g + j < a.C) one(raw[j], n, 4 * g + j, p);
+        }
+    } else {
+        const int items = a.N * a.HW * a.C;
+        for (int i0 = (x.wave * x.n_wg + x.rank) * 64; i0 < items; i0 += 8 * x.n_wg * 64) {
+            const int i = i0 + x.lane;
+            if (i >= items) continue;
+            const int np = i / a.C, c = i - np * a.C, n = np / a.HW, p = np - n * a.HW;
+            const int h = p / a.W, w = p - h * a.W;
+            const uint32_t q = static_cast<uint32_t>(n * a.in_sn + h * a.in_sh + w * a.in_sw + c);
+            TIn raw;
+            if constexpr (sizeof(TIn) == 4) {
+                const uint32_t word = shared4(in, 4 * q);
+                raw = __builtin_bit_cast(TIn, word);
+            } else raw = static_cast<TIn>(shared1(in, q));
+            one(raw, n, c, p);
+        }
+    }
+}
+
+// ---- rows of an encoder -----------------------------------------------------------------------------------------------------
+__device__ __forceinline__ float wave_total(float v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+
+__device__ __forceinline__ uint32_t levels4(const Requant& f, const float4& v) {
+    return level_bytes(f.p, f.lm1, f.p.ol, v.x) | (level_bytes(f.p, f.lm1, f.p.ol, v.y) << 8) | (level_bytes(f.p, f.lm1, f.p.ol, v.z) << 16) |
+           (level_bytes(f.p, f.lm1, f.p.ol, v.w) << 24);
+}
+
+__device__ __forceinline__ void embed_rows(const ProgEmbed& e, const Ctx& x) {
+    const int32_t* ids = reinterpret_cast<const int32_t*>(PROG_REF(x, e.ids));
+    const Buffer out = make_buffer(PROG_REF(x, e.out));
+    const float *tab = PROG_TABLE(float, e.table), *add0 = PROG_TABLE(float, e.add0), *add1 = PROG_TABLE(float, e.add1);
+    for (int t = x.wave * x.n_wg + x.rank; t < e.tokens; t += 8 * x.n_wg) {
+        int64_t idx = ids[t];
+        if (idx < 0) idx += e.vocab;
+        idx = idx < 0 ? 0 : (idx >= e.vocab ? e.vocab - 1 : idx);
+        const int64_t p = t % e.seq;
+        const float* src = tab + idx * e.hidden;
+        const float* a0 = add0 ? add0 + (e.pos0 ? p * e.hidden : 0) : nullptr;
+        const float* a1 = add1 ? add1 + (e.pos1 ? p * e.hidden : 0) : nullptr;
+        for (int i = 4 * x.lane; i < e.hidden; i += 256) {
+            float4 v = ld4f(src + i);
+            if (a0) { const float4 a = ld4f(a0 + i); v.x = v.x + a.x; v.y = v.y + a.y; v.z = v.z + a.z; v.w = v.w + a.w; }
+            if (a1) { const float4 a = ld4f(a1 + i); v.x = v.x + a.x; v.y = v.y + a.y; v.z = v.z + a.z; v.w = v.w + a.w; }
+            publish16f(out, 4u * static_cast<uint32_t>(t * e.hidden + i), v);
+        }
+    }
+}
+
+constexpr int kMvnChunks = 4;                 // rows of up to 1024 values
+__device__ __forceinline__ void mvn_rows(const ProgMvn& s, const Ctx& x) {
+    const Buffer in = make_buffer(PROG_REF(x, s.in)), yb = make_buffer(resolve(max(s.out.base, 0), s.out.lo, s.out.hi)),
+                 qb = make_buffer(resolve(max(s.outq.base, 0), s.outq.lo, s.outq.hi));
+    const bool y = s.out.base >= 0, q = s.outq.base >= 0;
+    const float *gamma = PROG_TABLE(float, s.gamma), *beta = PROG_TABLE(float, s.beta);
+    const int axis = s.axis;
+    for (int row = x.wave * x.n_wg + x.rank; row < s.rows; row += 8 * x.n_wg) {
+        const uint32_t p = static_cast<uint32_t>(row * axis);
+        float4 v[kMvnChunks];
+        float sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < kMvnChunks; ++j) {
+            const int i = 256 * j + 4 * x.lane;
+            v[j] = shared16f(in, i < axis ? 4u * (p + i) : static_cast<uint32_t>(kBeyond));
+            sum += (v[j].x + v[j].y) + (v[j].z + v[j].w);
+        }
+        const float mean = wave_total(sum) / static_cast<float>(axis);
+        float sq = 0.f;
+#pragma unroll
+        for (int j = 0; j < kMvnChunks; ++j) {
+            const int i = 256 * j + 4 * x.lane;
+            v[j].x -= mean; v[j].y -= mean; v[j].z -= mean; v[j].w -= mean;
+            if (i < axis) sq += (v[j].x * v[j].x + v[j].y * v[j].y) + (v[j].z * v[j].z + v[j].w * v[j].w);
+        }
+        float denom = 1.f;
+        if (s.normalize) {
+            const float var = wave_total(sq) / static_cast<float>(axis);
+            denom = s.eps_inside ? sqrtf(var + s.eps) : sqrtf(var) + s.eps;
+        }
+#pragma unroll
+        for (int j = 0; j < kMvnChunks; ++j) {
+            const int i = 256 * j + 4 * x.lane;
+            if (i >= axis) continue;
+            float4 o = v[j];
+            if (s.normalize) { o.x = o.x / denom; o.y = o.y / denom; o.z = o.z / denom; o.w = o.w / denom; }
+            if (gamma) { const float4 g = ld4f(gamma + i); o.x = o.x * g.x; o.y = o.y * g.y; o.z = o.z * g.z; o.w = o.w * g.w; }
+            if (beta) { const float4 b = ld4f(beta + i); o.x = o.x + b.x; o.y = o.y + b.y; o.z = o.z + b.z; o.w = o.w + b.w; }
+            if (y) publish16f(yb, 4u * (p + i), o);
+            if (q) publish4(qb, p + i, levels4(s.fq, o));
+        }
+    }
+}
+
+__device__ __forceinline__ void fq_items(const ProgRows& s, const Ctx& x) {
+    const Buffer in = make_buffer(PROG_REF(x, s.in)), out = make_buffer(PROG_REF(x, s.out));
+    for (int i = 4 * ((x.wave * x.n_wg + x.rank) * 64 + x.lane); i < s.n; i += 4 * 8 * x.n_wg * 64) {
+        const float4 v = shared16f(in, 4u * static_cast<uint32_t>(i));
+        const float t[4] = {v.x, v.y, v.z, v.w};
+        uint32_t w = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w |= level_bytes(s.p, s.lm1, s.off, t[j]) << (8 * j);
+        publish4(out, static_cast<uint32_t>(i), w);
+    }
+}
+
+__device__ __forceinline__ void copy_items(const ProgRows& s, const Ctx& x) {
+    const Buffer in = make_buffer(PROG_REF(x, s.in)), out = make_buffer(PROG_REF(x, s.out));
+    for (int i = 16 * ((x.wave * x.n_wg + x.rank) * 64 + x.lane); i < s.n; i += 16 * 8 * x.n_wg * 64)
+        publish16(out, static_cast<uint32_t>(i), shared16(in, static_cast<uint32_t>(i)));
+}
+
+// ---- attention --------------------------------------------------------------------------------------------------------------
+// The core of attention.hip with the sequence length at run time: K and V^T of one (element, head) in LDS, a wave takes
+// 32 queries.  The scores do not stay in registers (S / 2 of them would limit S to 384 and need an instance per length):
+// they are multiplied out three times, for the maximum, the sum and the probabilities - the matrix pipe is idle here anyway.
+template <bool DIV2, int PFORM>
+__device__ __forceinline__ void attention_queries(const ProgAttention& s, Buffer qb, uint32_t qbase, Buffer out, uint32_t obase, int q0,
+                                                  lds_ptr sK, lds_ptr sVT, lds_i32 sVsum, const __attribute__((address_space(3))) float* sMask, int lane) {
+    const AttentionArgs& a = s.a;
+    const int S = s.S, nt = S / 32, l32 = lane & 31, h = lane >> 5, vt_ld = S + 16;
+    const int q_row = q0 + l32;
+    const uint32_t qrow = qbase + static_cast<uint32_t>(q_row * a.ldq);
+    const v4i qf[2] = {shared16(qb, qrow + 16 * h), shared16(qb, qrow + 32 + 16 * h)};
+    const int slot[2] = {((0 + h) ^ ((l32 >> 2) & 3)) * 16, ((2 + h) ^ ((l32 >> 2) & 3)) * 16};
+    constexpr float kLog2e = 1.4426950408889634f;
+    auto scores = [&](int t, float (&v)[16]) {
+        v16i acc = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const v4i kf = *(lds_v4i)(sK + (32 * t + l32) * 64 + slot[ks]);
+            acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf, qf[ks], acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            typedef float v4f __attribute__((ext_vector_type(4)));
+            v4f mk = {0.f, 0.f, 0.f, 0.f};
+            if (s.has_mask) mk = *(const __attribute__((address_space(3))) v4f*)(sMask + 32 * t + 8 * g + 4 * h);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                float y = static_cast<float>(acc[4 * g + j]) * a.scale1;
+                if (s.has_mask) y = y + mk[j];
+                v[4 * g + j] = y;
+            }
+        }
+    };
+    float m = -INFINITY;
+    for (int t = 0; t < nt; ++t) {
+        float v[16];
+        scores(t, v);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) m = fmaxf(m, v[r]);
+    }
+    m = fmaxf(m, __shfl_xor(m, 32, 64));
+    const float mL = -m * kLog2e;
+    float sum = 0.f;
+    for (int t = 0; t < nt; ++t) {
+        float v[16];
+        scores(t, v);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum += __builtin_amdgcn_exp2f(fmaf(v[r], kLog2e, mL));
+    }
+    sum += __shfl_xor(sum, 32, 64);
+    const float inv = 1.0f / sum;
+    v16i ctx[2] = {{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}};
+    if (a.p_bias) {
+#pragma unroll
+        for (int db = 0; db < 2; ++db)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const v4i sv = *(lds_v4i)(sVsum + 32 * db + 8 * g + 4 * h);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) ctx[db][4 * g + j] = sv[j] * a.p_bias;
+            }
+    }
+    for (int t = 0; t < nt; ++t) {
+        float v[16];
+        scores(t, v);
+        v4i pf;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            float p[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(fmaf(v[4 * g + j], kLog2e, mL)) * inv;
+            pf[g] = static_cast<int>(prob_levels4<DIV2, PFORM>(a, p[0], p[1], p[2], p[3]));
+        }
+#pragma unroll
+        for (int db = 0; db < 2; ++db) {
+            const v4i vf = *(lds_v4i)(sVT + (32 * db + l32) * vt_ld + 32 * t + 16 * h);
+            ctx[db] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf, pf, ctx[db], 0, 0, 0);
+        }
+    }
+    const uint32_t orow = obase + static_cast<uint32_t>(q_row * a.ldo);
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int d = 32 * db + 8 * g + 4 * h;
+            const float4 o = make_float4(static_cast<float>(ctx[db][4 * g]) * a.scale2, static_cast<float>(ctx[db][4 * g + 1]) * a.scale2,
+                                         static_cast<float>(ctx[db][4 * g + 2]) * a.scale2, static_cast<float>(ctx[db][4 * g + 3]) * a.scale2);
+            if (a.fq_o.levels) publish4(out, orow + d, levels4(a.fq_o, o));
+            else publish16f(out, 4u * (orow + d), o);
+        }
+}
+
+__device__ __forceinline__ void attention_units(const ProgAttention& s, const Ctx& x, lds_ptr lds) {
+    const AttentionArgs& a = s.a;
+    const int S = s.S, vt_ld = S + 16;
+    lds_ptr sK = lds, sVT = lds + S * 64;
+    lds_i32 sVsum = (lds_i32)(sVT + 64 * vt_ld);
+    __attribute__((address_space(3))) float* sMask = (__attribute__((address_space(3))) float*)(sVsum + 64);
+    const Buffer qb = make_buffer(PROG_REF(x, s.q)), kb = make_buffer(PROG_REF(x, s.k)), vb = make_buffer(PROG_REF(x, s.v)), out = make_buffer(PROG_REF(x, s.out));
+    const float* mask = s.has_mask ? reinterpret_cast<const float*>(PROG_REF(x, s.mask)) : nullptr;
+    for (int u = x.rank; u < s.units; u += x.n_wg) {
+        const int eh = u / s.parts, part = u - eh * s.parts, n = eh / s.heads, hd = eh - n * s.heads;
+        const uint32_t kp = static_cast<uint32_t>(n * a.ok + hd * a.sk), vp = static_cast<uint32_t>(n * a.ov + hd * a.sv);
+        if (x.tid < 64) sVsum[x.tid] = 0;
+        __syncthreads();
+        for (int i = x.tid; i < S * 4; i += kProgramThreads) {          // S * 4 pieces of K; as many groups of 4 keys x 4 d of V
+            const int r = i >> 2, c = i & 3;
+            *(lds_v4i)(sK + r * 64 + ((c ^ ((r >> 2) & 3)) * 16)) = shared16(kb, kp + static_cast<uint32_t>(r * a.ldk + c * 16));
+        }
+        int32_t vsum[4] = {0, 0, 0, 0};
+        for (int i = x.tid; i < S * 4; i += kProgramThreads) {
+            const int d4 = i & 15, kq = i >> 4;
+            uint32_t w[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) w[q] = shared4(vb, vp + static_cast<uint32_t>((4 * kq + q) * a.ldv + 4 * d4));
+            const uint32_t lo01 = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u), hi01 = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u);
+            const uint32_t lo23 = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u), hi23 = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
+            const uint32_t t[4] = {__builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
+                                   __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u)};
+            const int key = 4 * kq, tile = key >> 5, in = key & 31;
+            const int col = tile * 32 + ((in >> 2) & 1) * 16 + (in >> 3) * 4;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                *(__attribute__((address_space(3))) uint32_t*)(sVT + (4 * d4 + q) * vt_ld + col) = t[q];
+                vsum[q] = __builtin_amdgcn_sdot4(static_cast<int>(t[q]), 0x01010101, vsum[q], false);
+            }
+        }
+        if (a.p_bias) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                __hip_atomic_fetch_add(sVsum + 4 * (x.tid & 15) + q, vsum[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        if (mask)
+            for (int i = x.tid; i < S; i += kProgramThreads) sMask[i] = mask[n * a.mask_outer + hd * a.mask_inner + i];
+        __syncthreads();
+        const int q0 = 32 * (part * s.waves + x.wave);
+        if (x.wave < s.waves && q0 < S) {
+            const uint32_t qbase = static_cast<uint32_t>(n * a.oq + hd * a.sq), obase = static_cast<uint32_t>(n * a.oo + hd * a.so);
+            if (s.pform == 2) attention_queries<true, 2>(s, qb, qbase, out, obase, q0, sK, sVT, sVsum, sMask, x.lane);
+            else attention_queries<true, 0>(s, qb, qbase, out, obase, q0, sK, sVT, sVsum, sMask, x.lane);
+        }
+        __syncthreads();
+    }
+}
+
+// ---- the program ------------------------------------------------------------------------------------------------------------
+__global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgArgs g) {
+    extern __shared__ __attribute__((aligned(16))) int8_t smem[];
+    lds_ptr lds = (lds_ptr)smem;
+    lds_i32 flag = (lds_i32)(lds + kPartBytes + kKoffBytes);
+    Ctx x;
+    x.tid = threadIdx.x;
+    x.lane = x.tid & 63;
+    x.wave = __builtin_amdgcn_readfirstlane(x.tid >> 6);
+    x.n_wg = g.workgroups;
+    x.rank = static_cast<int>(blockIdx.x % 8) * (x.n_wg / 8) + static_cast<int>(blockIdx.x / 8);
+    const bool tree = x.n_wg > kFlat;
+    x.root = g.control + kCtlRoot;
+    x.sub = tree ? g.control + kCtlXcd + 32 * (blockIdx.x % 8) : nullptr;
+    x.root_target = g.launch * static_cast<uint32_t>(g.n_steps * (tree ? 8 : x.n_wg));      // roll call + n_steps - 1 barriers a launch
+    x.sub_target = g.launch * static_cast<uint32_t>(g.n_steps * (x.n_wg / 8));
+    x.next_targets();
+    x.report = g.report;
+    x.dead = false;
+    x.flag = flag;
+    // roll call: everybody is resident, or nobody starts
+    if (x.tid == 0) {
+        uint32_t* state = g.control + kCtlState;
+        const uint32_t before = 2 * g.launch, go = before + 2, off = before + 3;
+        uint32_t s = __hip_atomic_load(state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (s == before) {
+            uint32_t expect = before;
+            if (x.count()) __hip_atomic_compare_exchange_strong(state, &expect, go, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint64_t t0 = wall_clock64();
+            for (;;) {
+                s = __hip_atomic_load(state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (s != before) break;
+                if (wall_clock64() - t0 > g.roll_call_ticks) {
+                    expect = before;
+                    if (__hip_atomic_compare_exchange_strong(state, &expect, off, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) expect = off;
+                    s = expect;
+                    break;
+                }
+            }
+        }
+        if (s != go) __hip_atomic_store(g.report, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        flag[0] = s == go ? 1 : 0;
+    }
+    __syncthreads();
+    if (flag[0] == 0) return;
+    for (int step = 0; step < g.n_steps; ++step) {
+        // the thread's place is derived again in every step: as loop invariants its many functions (row, piece, quad ... of every
+        // kind of step) would live in registers across all of them, and be moved out of the way and back around the large tiles
+        int tid = threadIdx.x;
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("" : "+v"(tid));
+#endif
+        x.tid = tid;
+        x.lane = tid & 63;
+        const StepPtr words = step_ptr(g.steps, step);
+        const int kind = words[0];
+        if (kind != PK_CONV && kind != PK_DW) {
+            x.wait();
+            if (x.dead) return;
+        }
+        switch (kind) {
+        case PK_CONV: {
+            ConstConv* c = (ConstConv*)words;
+            switch (c->a * 8 + c->b + (c->nk2 ? 64 : 0)) {
+            case 8 + 4: conv_tiles<1, 4>(c, x, lds); break;
+            case 16 + 1: conv_tiles<2, 1>(c, x, lds); break;
+            case 16 + 2: conv_tiles<2, 2>(c, x, lds); break;
+            case 16 + 4: conv_tiles<2, 4>(c, x, lds); break;
+            case 32 + 2: conv_tiles<4, 2>(c, x, lds); break;
+            case 64 + 16 + 2: conv_tiles<2, 2, true>(c, x, lds); break;
+            case 64 + 16 + 4: conv_tiles<2, 4, true>(c, x, lds); break;
+            default: conv_tiles<4, 4>(c, x, lds); break;
+            }
+            break;
+        }
+        case PK_DW: {
+            ConstConv& c = *(ConstConv*)words;
+            if (c.stride == 1) dw_items<1>(c, x);
+            else dw_items<2>(c, x);
+            break;
+        }
+        case PK_ENTRY: entry_items(unpack<ProgEntry>(words), x); break;
+        case PK_MAXPOOL: max_pool_items(unpack<ProgPool>(words), x); break;
+        case PK_AVGPOOL: avg_pool_items(unpack<ProgPool>(words), x); break;
+        case PK_EXIT: {
+            const ProgExit e = unpack<ProgExit>(words);
+            if (e.in_dtype == HIPIE_F32) exit_items<float>(e, x);
+            else if (e.in_dtype == HIPIE_I32) exit_items<int32_t>(e, x);
+            else exit_items<int8_t>(e, x);
+            break;
+        }
+        case PK_EMBED: embed_rows(unpack<ProgEmbed>(words), x); break;
+        case PK_MVN: mvn_rows(unpack<ProgMvn>(words), x); break;
+        case PK_ATTENTION: attention_units(unpack<ProgAttention>(words), x, lds); break;
+        case PK_FQROWS: fq_items(unpack<ProgRows>(words), x); break;
+        default: copy_items(unpack<ProgRows>(words), x); break;
+        }
+        if (x.dead) return;
+        if (step + 1 == g.n_steps) break;
+        {   // the next step's descriptor into the scalar cache
+            const StepPtr next = step_ptr(g.steps, step + 1);
+#pragma unroll
+            for (int i = 0; i < kProgramStepWords; i += 16) asm volatile("" ::"s"(next[i]));
+        }
+        x.arrive();
+    }
+}
+
+// constant weights [OCp][Kp] in the per-layer kernels' row order -> fragments of the tile kernel: for every tile of 16 A
+// channels and every K step of 64 bytes A fragments, lane l's 16 bytes = channel 16 A tile + A (l % 16) + a, K bytes 16 (l / 16) on
+__global__ __launch_bounds__(256) void pack_fragments_kernel(const int8_t* __restrict__ w, int8_t* __restrict__ f, int A, int OCp, int Kp, int64_t pieces) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= pieces) return;
+    const int l = static_cast<int>(i & 63), nk = Kp / 64;
+    const int64_t fr = i >> 6;
+    const int a = static_cast<int>(fr % A), k = static_cast<int>(fr / A % nk), ot = static_cast<int>(fr / A / nk);
+    const int oc = ot * 16 * A + A * (l & 15) + a;
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (oc < OCp) {
+        const int e = oc & 63;
+        const int row = (oc & ~63) + 32 * ((e >> 4) & 1) + 8 * ((e >> 2) & 3) + 4 * (e >> 5) + (e & 3);
+        v = *reinterpret_cast<const uint4*>(w + static_cast<int64_t>(row) * Kp + 64 * k + 16 * (l >> 4));
+    }
+    reinterpret_cast<uint4*>(f)[i] = v;
+}
+
+__global__ void clear_words(uint32_t* p, int n) {
+    for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
+}
+
+// Tile shape of a convolution step, by the clocks its busiest compute unit should take (measured on single steps: a round
+// trip behind the barrier is about 1500 clocks; a load of 1 KB occupies a unit's path for 20; a matrix instruction its pipe
+// for 16; the exact f32 chain is 12 vector instructions per value, one every 8 clocks for a wave that is alone on its SIMD,
+// one every 4 when another fills the gaps; meeting in LDS costs 500).  Rounds are tiles a wave takes one after another.
+struct TileChoice { int a, b, ks; };
+TileChoice choose_tile(int workgroups, int oc, int64_t pixels, int nk, int nk2, bool gelu) {
+    static constexpr int kShapes[6][2] = {{4, 4}, {4, 2}, {2, 4}, {2, 2}, {2, 1}, {1, 4}};
+    TileChoice best{4, 4, 1};
+    double best_t = 1e30;
+    for (const auto& shape : kShapes)
+        for (int ks : {1, 2, 4, 8}) {
+            const int a = shape[0], b = shape[1];
+            if ((nk2 && (a != 2 || b < 2)) || (gelu && a == 1)) continue;
+            const int depth = a * b >= 16 ? 2 : (a * b >= 8 ? 4 : 6);
+            const int64_t tiles = ceil_div(oc, 16 * a) * ceil_div(pixels, 16 * b), per_wg = ceil_div(tiles, workgroups);
+            const int64_t rounds = ceil_div(per_wg, 8 / ks);
+            const double waves = std::min<double>(8.0, static_cast<double>(per_wg) * ks / static_cast<double>(rounds));   // of a workgroup, busy
+            auto loop = [&](int steps) {
+                const double n = static_cast<double>(ceil_div(steps, ks));
+                const double rate = std::max(waves * (a + b) * 20.0, std::max(1.0, waves / 4.0) * a * b * 16.0 + 30.0);
+                return std::max(n * rate, std::ceil(n / depth) * 1500.0) + 300.0;
+            };
+            const double columns = std::ceil(static_cast<double>(b) / ks), writers = waves / ks * std::min(ks, b);
+            const double chain = (gelu ? 44.0 : 12.0) * 4 * a + 60.0;
+            const double epi = columns * chain * std::max(8.0, writers);          // writers / 4 waves per SIMD, 4 clocks each
+            const double t = static_cast<double>(rounds) * (loop(nk) + (nk2 ? loop(nk2) : 0.0) + epi + (ks > 1 ? 500.0 : 100.0) + 400.0);
+            if (t < best_t) {
+                best_t = t;
+                best = {a, b, ks};
+            }
+        }
+    return best;
+}
+
+struct ProgramGate {
+    std::mutex lock;
+    hipStream_t last = nullptr;      // stream of the program in flight, if any
+    hipEvent_t event = nullptr;
+};
+ProgramGate& gate(int device) {
+    static ProgramGate gates[64];
+    return gates[device & 63];
+}
+
+}  // namespace
+
+ProgRef ProgBuilder::ref(const void* p) {
+    const uint64_t v = reinterpret_cast<uintptr_t>(p), io = uint64_t(1) << 44, ar = uint64_t(1) << 32;
+    int32_t base = 0;
+    uint64_t off = v - ar;
+    if (v >= io - (uint64_t(1) << 39)) {
+        const uint64_t k = (v - io + (uint64_t(1) << 39)) >> 40;
+        base = 1 + static_cast<int32_t>(k);
+        off = v - io - (k << 40);
+    }
+    return {base, static_cast<uint32_t>(off), static_cast<uint32_t>(off >> 32)};
+}
+
+ProgPtr ProgBuilder::keep(const void* host, size_t bytes) {
+    owned.emplace_back();
+    owned.back().upload(device, host, bytes);
+    return ptr(owned.back().ptr);
+}
+
+bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out) {
+    ConvLaunch l;
+    if (!conv_launch_arguments(conv, in, residual, out, l)) return false;
+    const ConvArgs& a = l.a;
+    const int64_t M = a.M;
+    if (M > (1 << 20) || a.koff_tile || (a.flags & CF_OUT_I32) || ((a.flags & CF_OUT_FQ) && !(a.flags & CF_FQ_RCP)) || (a.flags & (CF_RES_SUB | CF_POST_SCALE)))
+        return false;
+    const bool f32_out = !(a.flags & CF_OUT_FQ), f32_res = (a.flags & CF_RES_F32) != 0;
+    for (int64_t bytes : {static_cast<int64_t>(out.n) * a.out_sn * (f32_out ? 4 : 1), static_cast<int64_t>(out.n) * a.res_sn * (f32_res ? 4 : 1)})
+        if (bytes >= kBeyond) return false;
+    ProgConv c{};
+    c.in = ref(a.in + a.in_origin);
+    c.out = ref(a.out);
+    c.res = a.res ? ref(a.res) : ProgRef{-2, 0, 0};
+    c.in2 = ProgRef{-2, 0, 0};
+    c.out_limit = a.out_sw;
+    c.res_limit = a.res_sw;
+    {   // the tables the flags ask for, in load_constants' order
+        const uint32_t fl = a.flags;
+        std::vector<const void*> rows{a.corr};
+        if (fl & CF_BIAS) rows.push_back(a.bias);
+        if (fl & CF_SCALE) rows.push_back(a.scale);
+        if (fl & CF_RES_MUL) rows.push_back(a.res_mul);
+        if (fl & CF_OUT_FQ) {
+            rows.push_back(a.fq_r);
+            rows.push_back((fl & CF_FQ_DIV2) ? a.fq_r2 : a.fq_d);
+            if (!(fl & CF_FQ_SAT)) rows.push_back(a.fq_ih);
+            if (!(fl & CF_FQ_IL0)) rows.push_back(a.fq_il);
+        }
+        c.constants = gather(rows, static_cast<size_t>(a.OCp) * 4);
+    }
+    c.flags = a.flags; c.lm1 = a.lm1; c.out_off = a.out_off; c.clamp_lo = a.clamp_lo; c.clamp_hi = a.clamp_hi;
+    c.OCp = a.OCp;
+    if (l.depthwise) {
+        c.OH = a.OHOW / a.OW;
+        c.OW = a.OW;
+        if (l.kh != 3 || l.kw != 3 || l.dil_h != 1 || l.dil_w != 1 || a.conv_sh != a.conv_sw || a.conv_sh > 2 || !a.wgt2 || a.in_sw < a.out_sw) return false;
+        c.kind = PK_DW;
+        c.stride = a.conv_sh;
+        c.wgt = ptr(a.wgt2);
+        c.in_sn = a.in_sn; c.in_sh = a.in_sh * a.conv_sh; c.in_sw = a.in_sw; c.row_sh = a.in_sh;
+        c.out_sn = a.out_sn; c.out_sh = a.out_sh; c.out_sw = a.out_sw;
+        c.res_sn = a.res_sn; c.res_sh = a.res_sh; c.res_sw = a.res_sw;
+        c.c4 = a.out_sw / 4;
+        c.quads = static_cast<int32_t>(ceil_div(a.OW, 4));
+        const int64_t items = static_cast<int64_t>(out.n) * c.OH * c.quads * c.c4;
+        if (items >= (1 << 24)) return false;
+        c.items = static_cast<int32_t>(items);
+        c.inv_c4 = 1.0f / static_cast<float>(c.c4);
+        c.inv_quads = 1.0f / static_cast<float>(c.quads);
+        c.inv_OH = 1.0f / static_cast<float>(c.OH);
+        add(c);
+        return true;
+    }
+    c.kind = PK_CONV;
+    c.nk = a.nk;
+    const bool pair = (a.flags & CF_RES_GEMM) != 0;
+    if (4 * a.nk > kMaxPieces || (pair && 4 * a.nk2 > kMaxPieces)) return false;
+    const TileChoice t = choose_tile(workgroups, a.OC, M, a.nk, pair ? a.nk2 : 0, (a.flags & CF_GELU) != 0);
+    c.a = t.a; c.b = t.b; c.ks_shift = __builtin_ctz(static_cast<unsigned>(t.ks));
+    // (the channels the tensor is padded with are written too)
+    const int o_tiles = static_cast<int>(ceil_div(std::min(a.out_sw, a.OCp), 16 * t.a));
+    c.p_tiles = static_cast<int32_t>(ceil_div(M, 16 * t.b));
+    c.inv_p_tiles = 1.0f / static_cast<float>(c.p_tiles);
+    const int64_t tiles = static_cast<int64_t>(c.p_tiles) * o_tiles;
+    if (tiles * workgroups >= (1ll << 31) || tiles >= (1 << 24) || static_cast<int64_t>(a.nk) * t.a * 1024 >= kBeyond) return false;
+    c.tiles = static_cast<int32_t>(tiles);
+    c.koff = ptr(a.koff);
+    auto repack = [&](const int8_t* w, int Kp) {
+        owned.emplace_back();
+        const int64_t pieces = static_cast<int64_t>(o_tiles) * t.a * Kp;        // 16 a x Kp bytes per tile, 16 bytes a piece
+        owned.back().alloc(device, static_cast<size_t>(pieces) * 16);
+        hipLaunchKernelGGL(pack_fragments_kernel, dim3(static_cast<uint32_t>(ceil_div(pieces, 256))), dim3(256), 0, nullptr, w, owned.back().as<int8_t>(), t.a,
+                           a.OCp, Kp, pieces);
+        HIPIE_CHECK_HIP(hipGetLastError());
+        return ptr(owned.back().ptr);
+    };
+    c.wgt = repack(a.wgt, a.Kp);
+    if (pair) {
+        c.in2 = ref(a.in2 + a.in2_origin);
+        c.wgt2 = repack(a.wgt2, a.Kp2);
+        c.koff2 = ptr(a.koff2);
+        c.nk2 = a.nk2;
+        c.constants2 = gather({a.corr2, a.bias2, a.scale2}, static_cast<size_t>(a.OCp) * 4);
+    }
+    // where every pixel's window and results are; pixels behind the last one read where it does and store nowhere
+    const int64_t pitch = static_cast<int64_t>(c.p_tiles) * 16 * t.b;
+    c.M = static_cast<int32_t>(pitch);
+    std::vector<uint32_t> pix(static_cast<size_t>(4 * pitch));
+    for (int64_t i = 0; i < pitch; ++i) {
+        const int64_t m = std::min(i, M - 1), n = m / a.OHOW, rem = m - n * a.OHOW, oh = rem / a.OW, ow = rem - oh * a.OW;
+        auto at = [&](int sn, int sh, int sw) { return static_cast<uint32_t>(n * sn + oh * sh + ow * sw); };
+        pix[static_cast<size_t>(i)] = at(a.in_sn, a.in_sh * a.conv_sh, a.in_sw * a.conv_sw);
+        pix[static_cast<size_t>(pitch + i)] = i < M ? at(a.out_sn, a.out_sh, a.out_sw) * (f32_out ? 4u : 1u) : static_cast<uint32_t>(kBeyond);
+        pix[static_cast<size_t>(2 * pitch + i)] = at(a.res_sn, a.res_sh, a.res_sw) * (f32_res ? 4u : 1u);
+        pix[static_cast<size_t>(3 * pitch + i)] = pair ? at(a.in2_sn, a.in2_sh * a.conv2_sh, a.in2_sw * a.conv2_sw) : 0u;
+    }
+    c.pixels = keep(pix.data(), pix.size() * 4);
+    add(c);
+    return true;
+}
+
+// tables of `pitch` bytes behind one another in a buffer of the program's own
+ProgPtr ProgBuilder::gather(const std::vector<const void*>& rows, size_t pitch) {
+    owned.emplace_back();
+    owned.back().alloc(device, rows.size() * pitch);
+    for (size_t i = 0; i < rows.size(); ++i)
+        HIPIE_CHECK_HIP(hipMemcpyAsync(owned.back().as<uint8_t>() + i * pitch, rows[i], pitch, hipMemcpyDeviceToDevice, nullptr));
+    return ptr(owned.back().ptr);
+}
+
+bool ProgBuilder::entry(const hipie_fq* fq, bool u8_in, const void* in, const hipie_tensor& out) {
+    FqLaunch f;
+    if (!fq_launch_arguments(fq, out.dtype, f) || !f.rcp || out.c != f.channels) return false;
+    const int64_t hw = static_cast<int64_t>(out.h) * out.w;
+    if (hw >= (1 << 24) || out.stride_w % 4 != 0 || (out.stride_w > 4 && out.stride_w % 16 != 0) || static_cast<int64_t>(out.n) * out.stride_n >= kBeyond || out.n * hw * out.stride_w >= (1ll << 30)) return false;
+    ProgEntry e{};
+    e.kind = PK_ENTRY;
+    e.N = out.n;
+    e.u8_in = u8_in;
+    e.C = out.c;
+    e.cs = static_cast<int32_t>(out.stride_w);
+    e.HW = static_cast<int32_t>(hw);
+    e.W = out.w;
+    e.inv_W = 1.0f / static_cast<float>(out.w);
+    e.lm1 = f.lm1;
+    e.off = f.off;
+    e.out_sn = out.stride_n;
+    e.out_sh = out.stride_h;
+    e.in = ref(in);
+    e.out = ref(out.data);
+    e.tab = ptr(f.table);
+    add(e);
+    return true;
+}
+
+bool ProgBuilder::pool(const PoolArgs& a, bool avg, bool rcp) {
+    const int64_t span = static_cast<int64_t>(a.M / a.OHOW) * std::max<int64_t>(a.in_sn, 4ll * a.out_sn);
+    if ((a.fq_il && !rcp) || static_cast<int64_t>(a.M) * a.cs >= (1ll << 30) || a.cs % 4 != 0 || span >= kBeyond) return false;
+    ProgPool p{};
+    p.kind = avg ? PK_AVGPOOL : PK_MAXPOOL;
+    p.items = a.M * (a.cs / 4);
+    const int OH = a.OHOW / a.OW;
+    p.k3 = a.kh == 3 && a.kw == 3 && (OH - 1) * a.sh - a.pt + 3 <= a.H + a.pb && (a.OW - 1) * a.sw - a.pl + 3 <= a.W + a.pr;
+    p.in = ref(a.in);
+    p.out = ref(a.out);
+    p.a = a;
+    add(p);
+    return true;
+}
+
+bool ProgBuilder::exit(const ExitArgs& a, int in_dtype) {
+    if (static_cast<int64_t>(a.N) * a.HW * a.C >= (1ll << 30) || static_cast<int64_t>(a.N) * a.in_sn * 4 >= kBeyond || a.in_sw % 4 != 0) return false;
+    ProgExit e{};
+    e.kind = PK_EXIT;
+    e.in_dtype = in_dtype;
+    e.in = ref(a.in);
+    e.out = ref(a.out);
+    e.a = a;
+    add(e);
+    return true;
+}
+
+bool ProgBuilder::embed(const float* table, int64_t vocab, int64_t hidden, const void* ids, int64_t tokens, int64_t seq, const float* add0, bool pos0,
+                       const float* add1, bool pos1, void* out) {
+    if (hidden % 4 != 0 || tokens * hidden * 4 >= kBeyond || seq >= (1 << 24)) return false;
+    ProgEmbed e{};
+    e.kind = PK_EMBED;
+    e.hidden = static_cast<int32_t>(hidden);
+    e.seq = static_cast<int32_t>(seq);
+    e.pos0 = pos0;
+    e.pos1 = pos1;
+    e.tokens = static_cast<int32_t>(tokens);
+    e.vocab = vocab;
+    e.ids = ref(ids);
+    e.out = ref(out);
+    e.table = ptr(table);
+    e.add0 = ptr(add0);
+    e.add1 = ptr(add1);
+    add(e);
+    return true;
+}
+
+bool ProgBuilder::mvn(const void* in, void* out, void* outq, int64_t rows, int64_t axis, bool normalize, float eps, bool eps_inside, const float* gamma,
+                     const float* beta, const hipie_requant* rq) {
+    if (rows * axis * 4 >= kBeyond || axis % 4 != 0 || axis > 256 * kMvnChunks) return false;
+    ProgMvn m{};
+    m.kind = PK_MVN;
+    m.axis = static_cast<int32_t>(axis);
+    m.rows = static_cast<int32_t>(rows);
+    m.normalize = normalize;
+    m.eps_inside = eps_inside;
+    m.eps = eps;
+    m.in = ref(in);
+    m.out = out ? ref(out) : ProgRef{-2, 0, 0};
+    m.outq = outq ? ref(outq) : ProgRef{-2, 0, 0};
+    m.gamma = ptr(gamma);
+    m.beta = ptr(beta);
+    if (outq) m.fq = make_requant(rq, "single-launch program");
+    if (outq && !m.fq.rcp) return false;
+    add(m);
+    return true;
+}
+
+bool ProgBuilder::attention(const hipie_attention* att, const void* const (&qkv)[3], const int64_t (&ld)[3], const int64_t (&inner)[3],
+                           const int64_t (&outer)[3], void* out, int64_t ldo, int64_t so, int64_t oo, int batch, int batch_outer, const void* mask) {
+    const AttentionArgs& proto = attention_prototype(att);
+    if (!proto.p_div2 || (proto.fq_o.levels && !proto.fq_o.rcp)) return false;
+    for (int i = 0; i < 3; ++i)
+        if (batch_outer * outer[i] + batch * inner[i] + proto.S * ld[i] >= kBeyond) return false;
+    if (4 * (batch_outer * oo + batch * so + proto.S * ldo) >= kBeyond) return false;
+    if (proto.S * 64 + 64 * (proto.S + 16) + 256 + 4 * proto.S > kPartBytes) return false;
+    ProgAttention s{};
+    s.kind = PK_ATTENTION;
+    s.S = proto.S;
+    s.heads = batch;
+    s.q = ref(qkv[0]); s.k = ref(qkv[1]); s.v = ref(qkv[2]);
+    s.out = ref(out);
+    s.has_mask = mask != nullptr;
+    s.mask = mask ? ref(mask) : ProgRef{-2, 0, 0};
+    s.pform = proto.p_sat ? 2 : 0;
+    s.a = proto;
+    s.a.ldq = ld[0]; s.a.sq = inner[0]; s.a.oq = outer[0];
+    s.a.ldk = ld[1]; s.a.sk = inner[1]; s.a.ok = outer[1];
+    s.a.ldv = ld[2]; s.a.sv = inner[2]; s.a.ov = outer[2];
+    s.a.ldo = ldo; s.a.so = so; s.a.oo = oo;
+    s.a.mask_inner = 0;
+    s.a.mask_outer = proto.S;
+    // queries per workgroup: rounds x (staging, about 4 clocks a key + a wave's 20 instructions per score, two waves to a
+    // SIMD from five on)
+    const int qt = proto.S / 32;
+    const int64_t elements = static_cast<int64_t>(batch_outer) * batch;
+    double best = 1e30;
+    for (int w = 1; w <= 8; ++w) {
+        const int64_t parts = ceil_div(qt, w), rounds = ceil_div(elements * parts, workgroups);
+        const double t = static_cast<double>(rounds) * (1500.0 + 4.0 * proto.S + (w > 4 ? 1.7 : 1.0) * qt * 16 * 20 * 4);
+        if (t < best) {
+            best = t;
+            s.waves = w;
+            s.parts = static_cast<int32_t>(parts);
+            s.units = static_cast<int32_t>(elements * parts);
+        }
+    }
+    add(s);
+    return true;
+}
+
+bool ProgBuilder::fq_rows(const hipie_fq* fq, const void* in, void* out, int out_dtype, int64_t n) {
+    FqLaunch f;
+    if (!fq_launch_arguments(fq, out_dtype, f) || !f.rcp || f.channels != 1 || n % 4 != 0 || 4 * n >= kBeyond / 2) return false;
+    ProgRows r{};
+    r.kind = PK_FQROWS;
+    r.n = n;
+    r.in = ref(in);
+    r.out = ref(out);
+    r.p = f.first;
+    r.lm1 = f.lm1;
+    r.off = f.off;
+    add(r);
+    return true;
+}
+
+bool ProgBuilder::copy(const void* in, void* out, int64_t bytes) {
+    if (bytes % 16 != 0 || bytes >= kBeyond / 2) return false;
+    ProgRows r{};
+    r.kind = PK_COPY;
+    r.n = bytes;
+    r.in = ref(in);
+    r.out = ref(out);
+    add(r);
+    return true;
+}
+
+Program::~Program() {
+    if (report) (void)hipHostFree(report);
+}
+
+int Program::take_slot() {
+    std::lock_guard<std::mutex> g(lock);
+    for (int i = 0; i < kSlots; ++i)
+        if (!((taken >> i) & 1)) {
+            taken |= uint64_t(1) << i;
+            report[16 * i] = 0;
+            return i;
+        }
+    return -1;
+}
+
+void Program::give_slot(int slot) {
+    std::lock_guard<std::mutex> g(lock);
+    taken &= ~(uint64_t(1) << slot);
+}
+
+std::unique_ptr<Program> make_program(ProgBuilder&& b) {
+    auto p = std::make_unique<Program>();
+    p->device = b.device;
+    p->workgroups = b.workgroups;
+    const char* ticks = std::getenv("HIPIE_ROLL_CALL_TICKS");      // (0: every launch is cancelled and runs again by steps)
+    p->roll_call_ticks = ticks ? static_cast<uint32_t>(std::strtoul(ticks, nullptr, 10)) : kRollCallTicks;
+    p->n_steps = static_cast<int>(b.steps.size());
+    p->steps.upload(b.device, b.steps.data(), b.steps.size() * kProgramStepWords * 4);
+    p->owned = std::move(b.owned);
+    DeviceGuard g(b.device);
+    HIPIE_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&p->report), Program::kSlots * 64, hipHostMallocDefault));
+    std::memset(p->report, 0, Program::kSlots * 64);
+    HIPIE_CHECK_HIP(hipStreamSynchronize(nullptr));      // the repacking kernels
+    HIPIE_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&program_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    return p;
+}
+
+void launch_program(const Program& p, uint8_t* arena, void* const* io, int n_io, uint32_t* control, uint32_t launch, int slot, hipStream_t s) {
+    ProgArgs a{};
+    a.steps = p.steps.as<int32_t>();
+    a.bases[0] = arena;
+    for (int i = 0; i < n_io; ++i) a.bases[1 + i] = io[i];
+    a.control = control;
+    a.report = p.report + 16 * slot;
+    a.n_steps = p.n_steps;
+    a.workgroups = p.workgroups;
+    a.launch = launch;
+    a.roll_call_ticks = p.roll_call_ticks;
+    p.report[16 * slot] = 0;
+    ProgramGate& g = gate(p.device);
+    std::lock_guard<std::mutex> hold(g.lock);
+    if (g.last && g.last != s) {
+        if (!g.event) HIPIE_CHECK_HIP(hipEventCreateWithFlags(&g.event, hipEventDisableTiming));
+        HIPIE_CHECK_HIP(hipEventRecord(g.event, g.last));
+        HIPIE_CHECK_HIP(hipStreamWaitEvent(s, g.event, 0));
+    }
+    hipLaunchKernelGGL(program_kernel, dim3(static_cast<uint32_t>(p.workgroups)), dim3(kProgramThreads), kLdsBytes, s, a);
+    HIPIE_CHECK_HIP(hipGetLastError());
+    g.last = s;
+}
+
+void program_done(const Program& p, hipStream_t s) {
+    ProgramGate& g = gate(p.device);
+    std::lock_guard<std::mutex> hold(g.lock);
+    if (g.last == s) g.last = nullptr;
+}
+
+bool program_failed(const Program& p, int slot, uint32_t* control, hipStream_t s) {
+    if (__atomic_load_n(p.report + 16 * slot, __ATOMIC_ACQUIRE) == 0) return false;
+    hipLaunchKernelGGL(clear_words, dim3(1), dim3(256), 0, s, control, static_cast<int>(kProgramControlBytes / 4));
+    HIPIE_CHECK_HIP(hipGetLastError());
+    return true;
+}
+
+}  // namespace hipie

@@ -481,9 +481,12 @@ int hipie_compile(const hipie_graph* graph, int device, hipie_plan** plan);
  * (YES | NO), HIP_FUSE_CONVOLUTIONS (a 3 x 3 convolution and the 1 x 1 convolution that alone reads its result as one
  * kernel, hipie_conv_run_pair: AUTO = where the load-time measurement finds it faster, YES = wherever the kernel takes
  * the pair, NO; the tensor between two layers run that way exists in LDS only and hipie_request_tensor gives
- * HIPIE_NOT_FOUND for it), NETWORK_NAME.  An unknown key gives HIPIE_NOT_FOUND, a value the key does not take
+ * HIPIE_NOT_FOUND for it), HIP_SINGLE_LAUNCH (a request that is started and waited for runs as one persistent kernel:
+ * AUTO = a plan for one stream, where the load-time measurement finds it faster, YES = wherever the plan has such a form,
+ * NO), NETWORK_NAME.  An unknown key gives HIPIE_NOT_FOUND, a value the key does not take
  * HIPIE_PARAMETER_MISMATCH.  The environment variables HIPIE_TUNE, HIPIE_TUNE_FILE, HIPIE_TUNE_STREAMS,
- * HIPIE_FUSE_ATTENTION, HIPIE_MERGE_LINEAR, HIPIE_KEEP_F32, HIPIE_FUSE_CONVS (0 | 1 | 2 = NO | AUTO | YES) are the
+ * HIPIE_FUSE_ATTENTION, HIPIE_MERGE_LINEAR, HIPIE_KEEP_F32, HIPIE_FUSE_CONVS and
+ * HIPIE_SINGLE_LAUNCH (0 | 1 | 2 = NO | AUTO | YES) are the
  * process-wide defaults of these keys. */
 int hipie_compile_opts(const hipie_graph* graph, int device, const char* const* keys, const char* const* values,
                        int n_opts, hipie_plan** plan);

@@ -1,0 +1,92 @@
+"""The single-launch form of a plan (csrc/program.hip) against its steps, bit for bit: tile remainders in pixels and channels,
+K of one step and of many, strides, residuals, shortcuts, depthwise, pools, encoder steps; the ordering of launches on
+several streams; and the way back to the steps when a launch is cancelled."""
+import numpy as np
+import pytest
+import torch
+
+from dldt_amd import builders
+
+pytestmark = pytest.mark.gpu
+
+GRAPHS = {
+    "block_1x3x7": lambda: builders.conv_block(n=1, c=3, hw=7, oc=8)[0],
+    "block_2x17x9": lambda: builders.conv_block(n=2, c=17, hw=9, oc=65)[0],
+    "block_1x64x56": lambda: builders.conv_block(n=1, c=64, hw=56, oc=64)[0],
+    "block_3x256x16": lambda: builders.conv_block(n=3, c=256, hw=16, oc=130)[0],
+    "resnet_1": lambda: builders.resnet50(batch=1, res=64, width=16, classes=10, seed=7)[0],
+    "resnet_3_u8": lambda: builders.resnet50(batch=3, res=96, u8_input=True)[0],
+    "mobilenet_2": lambda: builders.mobilenet_v2(batch=2, res=96)[0],
+    "encoder_1x32": lambda: builders.bert_encoder(layers=1, batch=1, seq=32, vocab=100, mask=True)[0],
+    "encoder_3x96": lambda: builders.bert_encoder(layers=1, batch=3, seq=96, vocab=0, mask=False)[0],
+    "encoder_2x384": lambda: builders.bert_encoder(layers=1, batch=2, seq=384, vocab=100, mask=True)[0],
+}
+
+
+def _fill(ins, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    for t in ins:
+        if t.dtype == torch.int32:
+            t.copy_(torch.randint(0, 100, t.shape, generator=gen, device="cuda", dtype=torch.int32))
+        elif t.dtype == torch.uint8:
+            t.copy_(torch.randint(0, 256, t.shape, generator=gen, device="cuda", dtype=torch.uint8))
+        elif t.dim() == 4 and t.shape[1] == t.shape[2] == 1:          # the attention mask
+            keep = torch.arange(t.shape[3], device="cuda") < t.shape[3] * 2 // 3
+            t.copy_(torch.where(keep, 0.0, -10000.0).expand(t.shape))
+        else:
+            t.copy_(torch.rand(t.shape, generator=gen, device="cuda") * 2)
+
+
+def _compile(g, mode):
+    return g.compile(0, config={"HIP_SINGLE_LAUNCH": mode, "HIP_TUNE": "NO", "HIP_THROUGHPUT_STREAMS": "1"})
+
+
+def _infer(req, seed):
+    ins, outs = req.device_buffers()
+    _fill(ins, seed)
+    for o in outs:
+        o.fill_(0 if o.dtype == torch.uint8 else float("nan"))
+    torch.cuda.synchronize()
+    req.infer_device(ins, outs)
+    return [o.cpu().numpy() for o in outs]
+
+
+@pytest.mark.parametrize("name", sorted(GRAPHS))
+def test_single_launch_equals_steps(name):
+    g = GRAPHS[name]()
+    steps, single = _compile(g, "NO"), _compile(g, "YES")
+    assert single.config("HIP_SINGLE_LAUNCH") == "YES"
+    a, b = steps.create_request(), single.create_request()
+    for seed in range(3):
+        for x, y in zip(_infer(a, seed), _infer(b, seed)):
+            assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
+
+
+def test_single_launch_requests_on_two_streams():
+    g = GRAPHS["resnet_1"]()
+    steps, single = _compile(g, "NO"), _compile(g, "YES")
+    want = [_infer(steps.create_request(), s) for s in range(2)]
+    reqs = [single.create_request() for _ in range(2)]
+    bufs = [r.host_buffers() for r in reqs]
+    for s, (ins, _) in enumerate(bufs):
+        dev = steps.create_request().device_buffers()[0]
+        _fill(dev, s)
+        ins[0].array[...] = dev[0].cpu().numpy()
+    for _ in range(20):
+        for r, (ins, outs) in zip(reqs, bufs):
+            r.start(ins, outs)
+        for r in reqs:
+            r.wait()
+        for (_, outs), w in zip(bufs, want):
+            assert np.array_equal(outs[0].array.view(np.uint8), w[0].view(np.uint8))
+
+
+def test_cancelled_launch_runs_by_steps(monkeypatch):
+    g = GRAPHS["resnet_1"]()
+    steps = _compile(g, "NO")
+    monkeypatch.setenv("HIPIE_ROLL_CALL_TICKS", "0")
+    single = _compile(g, "YES")
+    a, b = steps.create_request(), single.create_request()
+    for seed in range(3):
+        for x, y in zip(_infer(a, seed), _infer(b, seed)):
+            assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
