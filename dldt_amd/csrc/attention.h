@@ -50,6 +50,19 @@ __device__ __forceinline__ uint32_t prob_levels4(const AttentionArgs& a, float p
     return a.p_add ? add_bytes(w, a.p_add) : (w ^ a.p_xor);
 }
 
+// Rows longer than this have the Softmax of the stand-alone kernel bit for bit (softmax_rows_reg: exp(x - max), sums of
+// four keys, the chunks of 256 keys, then a tree over the groups of four), so that their levels do not depend on whether
+// the core is one kernel.  Up to it exp2 of one fused multiply-add, a serial sum and the reciprocal, within the same
+// tolerance: a third of the instructions.
+constexpr int kPlainSoftmax = 384;
+
+// e / sum rounded once, from inv = 1 / sum rounded once: quotient, exact residual, correction.  Equal to the IEEE
+// quotient for e in [2^-60, 1] and sum in [1, 1024) (8 x 10^9 pairs compared); below, the level is that of zero.
+__device__ __forceinline__ float quotient(float e, float sum, float inv) {
+    const float q = e * inv;
+    return fmaf(fmaf(-q, sum, e), inv, q);
+}
+
 }  // namespace hipie
 
 struct hipie_attention;

@@ -19,12 +19,17 @@
 namespace hipie {
 namespace {
 
-constexpr int kMaxSeq = 384;   // S / 2 accumulator registers per lane
+// A lane holds S / 2 scores in registers: up to 384 keys two waves share a SIMD, up to 512 (192 more registers than the
+// accumulators and operands take) one has it to itself.  An instance per length: in steps of 32 keys to 384, of 64 beyond.
+// 3 x 12 heads x 512 keys: 28 us, VALU-bound (exp and quotient of 9.4 million scores), where the two products, the Softmax
+// and the passes over 38 MB of scores between them took 85 us as kernels of their own.
+constexpr int kMaxSeq = 512;
 constexpr int kHeadDim = 64;
 
 template <int NT, bool DIV2, bool MASK, int PFORM>   // NT = S / 32 key tiles
-__global__ __launch_bounds__(256, 2) void attention_kernel(const AttentionArgs a) {
+__global__ __launch_bounds__(256, NT * 32 <= kPlainSoftmax ? 2 : 1) void attention_kernel(const AttentionArgs a) {
     constexpr int S = NT * 32;
+    constexpr bool kLong = S > kPlainSoftmax;
     constexpr int VT_LD = S + 16;                     // odd number of 16-byte groups per row: conflict-free
     __shared__ __attribute__((aligned(16))) int8_t sK[S * 64];       // [key][d], chunk c of row r in slot c ^ ((r >> 2) & 3)
     __shared__ __attribute__((aligned(16))) int8_t sVT[64 * VT_LD];  // [d][tile][half][j]: key 32 t + 8 (j / 4) + 4 half + j % 4
@@ -174,11 +179,12 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const AttentionArgs a
         }
     };
     // probabilities of a tile -> levels -> second product
-    auto finish_tile = [&](int t, const float (&e)[16], float inv) {
+    auto finish_tile = [&](int t, const float (&e)[16], float sum, float inv) {
         v4i pf;
+        auto prob = [&](int r) { return kLong ? quotient(e[r], sum, inv) : e[r] * inv; };
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const float4 p4 = make_float4(e[4 * g] * inv, e[4 * g + 1] * inv, e[4 * g + 2] * inv, e[4 * g + 3] * inv);
+            const float4 p4 = make_float4(prob(4 * g), prob(4 * g + 1), prob(4 * g + 2), prob(4 * g + 3));
             if (a.probs && q_ok)
                 *reinterpret_cast<float4*>(a.probs + dump_row + 32 * t + 8 * g + 4 * h) = p4;
             pf[g] = static_cast<int>(prob_levels4<DIV2, PFORM>(a, p4.x, p4.y, p4.z, p4.w));
@@ -208,21 +214,42 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const AttentionArgs a
     // exp(x - m) as 2^((x - m) log2 e) on the hardware's exp2, the division as a multiplication by the
     // reciprocal of the sum: within the tolerance the stand-alone kernel is held to.
     m = fmaxf(m, __shfl_xor(m, 32, 64));
-    const float mL = -m * kLog2e;
     float s = 0.f;
+    if constexpr (kLong) {
+        // four keys, then the chunks of 8 tiles, then halves of the groups (tile bits 2, 1, 0, g bits 1, 0, h)
+        float part[8][4];
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+        for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            x[t][r] = __builtin_amdgcn_exp2f(fmaf(x[t][r], kLog2e, mL));
-            s += x[t][r];
-        }
+            for (int g = 0; g < 4; ++g) {
+#pragma unroll
+                for (int r = 4 * g; r < 4 * g + 4; ++r) x[t][r] = expf(x[t][r] - m);
+                const float e4 = (x[t][4 * g] + x[t][4 * g + 1]) + (x[t][4 * g + 2] + x[t][4 * g + 3]);
+                part[t % 8][g] = t < 8 ? e4 : part[t % 8][g] + e4;
+            }
+#pragma unroll
+        for (int o = 4; o > 0; o >>= 1)
+#pragma unroll
+            for (int t = 0; t < o; ++t)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) part[t][g] += part[t + o][g];
+        s = (part[0][0] + part[0][2]) + (part[0][1] + part[0][3]);
+    } else {
+        const float mL = -m * kLog2e;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                x[t][r] = __builtin_amdgcn_exp2f(fmaf(x[t][r], kLog2e, mL));
+                s += x[t][r];
+            }
+    }
     s += __shfl_xor(s, 32, 64);
     const float inv = 1.0f / s;
     // probabilities -> i8 levels -> second product, one 32-key tile at a time
     init_ctx();
 #pragma unroll
-    for (int t = 0; t < NT; ++t) finish_tile(t, x[t], inv);
+    for (int t = 0; t < NT; ++t) finish_tile(t, x[t], s, inv);
 
     ATT_STAMP(5);
     // ---- context of query q_row: d = 32 db + 8 (r / 4) + 4 h + r % 4 --------------------------------
@@ -284,15 +311,15 @@ const AttentionArgs& hipie::attention_prototype(const hipie_attention* att) { re
 extern "C" {
 
 int hipie_attention_supported(int32_t seq, int32_t head_dim) {
-    return seq > 0 && seq % 32 == 0 && seq <= kMaxSeq && head_dim == kHeadDim;
+    return seq > 0 && seq % (seq <= kPlainSoftmax ? 32 : 64) == 0 && seq <= kMaxSeq && head_dim == kHeadDim;
 }
 
 int hipie_attention_create(int device, const hipie_attention_desc* desc, hipie_attention** out) {
     return guarded([&] {
         HIPIE_REQUIRE(desc && out, HIPIE_PARAMETER_MISMATCH, "hipie_attention_create: null argument");
         HIPIE_REQUIRE(hipie_attention_supported(desc->seq, desc->head_dim), HIPIE_NOT_IMPLEMENTED,
-                      "hipie_attention_create: sequence length %d (multiple of 32 up to %d) / head dimension %d (%d)", desc->seq,
-                      kMaxSeq, desc->head_dim, kHeadDim);
+                      "hipie_attention_create: sequence length %d (multiple of 32 up to %d, of 64 up to %d) / head dimension %d (%d)", desc->seq,
+                      kPlainSoftmax, kMaxSeq, desc->head_dim, kHeadDim);
         HIPIE_REQUIRE(desc->out_dtype == HIPIE_I8 || desc->out_dtype == HIPIE_F32, HIPIE_PARAMETER_MISMATCH,
                       "hipie_attention_create: output type %d", desc->out_dtype);
         HIPIE_REQUIRE(desc->prob_dtype == 0 || desc->prob_dtype == HIPIE_I8 || desc->prob_dtype == HIPIE_U8B, HIPIE_PARAMETER_MISMATCH,
@@ -375,7 +402,9 @@ int hipie_attention_run(const hipie_attention* att, const void* q, int64_t ldq, 
         case 9: launch<9>(a, batches, s); break;
         case 10: launch<10>(a, batches, s); break;
         case 11: launch<11>(a, batches, s); break;
-        default: launch<12>(a, batches, s); break;
+        case 12: launch<12>(a, batches, s); break;
+        case 14: launch<14>(a, batches, s); break;
+        default: launch<16>(a, batches, s); break;
         }
         HIPIE_CHECK_HIP(hipGetLastError());
     });

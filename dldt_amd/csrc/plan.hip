@@ -1934,6 +1934,9 @@ struct Planner {
         const size_t r = qv.rank();
         const int64_t S = qv.shape[r - 2], D = qv.shape[r - 1];
         if (kv.shape[r - 2] != S || !hipie_attention_supported(static_cast<int32_t>(S), static_cast<int32_t>(D))) return false;
+        // a plan that keeps its f32 tensors writes scores and probabilities out anyway: the long rows, where the fused
+        // kernel has one wave per SIMD to hide those stores, are left to the separate kernels
+        if (keep_f32 && S > 384) return false;
         if (qv.stride[r - 1] != 1 || kv.stride[r - 1] != 1) return false;
         if (!single_user(id)) return false;
         const int mul = n.users[0];

@@ -146,8 +146,8 @@ __device__ __forceinline__ uint8_t* resolve(int32_t base, uint32_t lo, uint32_t 
 
 
 constexpr int kBeyond = 0x7ffffff0;          // a buffer offset no buffer reaches: loads give zero, stores nothing
-constexpr int kDeviceScope = 16;             // sc1: what another XCD wrote, or will read
 #if defined(__HIP_DEVICE_COMPILE__)
+constexpr int kDeviceScope = 16;             // sc1: what another XCD wrote, or will read
 typedef __amdgpu_buffer_rsrc_t Buffer;
 __device__ __forceinline__ Buffer make_buffer(const void* p) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, kBeyond, 0x00020000); }
 template <int AUX> __device__ __forceinline__ v4i load16(Buffer b, uint32_t o, int imm = 0) { return __builtin_amdgcn_raw_buffer_load_b128(b, static_cast<int>(o), imm, AUX); }
@@ -995,7 +995,8 @@ __device__ __forceinline__ void copy_items(const ProgRows& s, const Ctx& x) {
 // The core of attention.hip with the sequence length at run time: K and V^T of one (element, head) in LDS, a wave takes
 // 32 queries.  The scores do not stay in registers (S / 2 of them would limit S to 384 and need an instance per length):
 // they are multiplied out three times, for the maximum, the sum and the probabilities - the matrix pipe is idle here anyway.
-template <bool DIV2, int PFORM>
+// LONG: the Softmax of rows longer than kPlainSoftmax.
+template <bool LONG, int PFORM>
 __device__ __forceinline__ void attention_queries(const ProgAttention& s, Buffer qb, uint32_t qbase, Buffer out, uint32_t obase, int q0,
                                                   lds_ptr sK, lds_ptr sVT, lds_i32 sVsum, const __attribute__((address_space(3))) float* sMask, int lane) {
     const AttentionArgs& a = s.a;
@@ -1035,11 +1036,34 @@ __device__ __forceinline__ void attention_queries(const ProgAttention& s, Buffer
     m = fmaxf(m, __shfl_xor(m, 32, 64));
     const float mL = -m * kLog2e;
     float sum = 0.f;
-    for (int t = 0; t < nt; ++t) {
-        float v[16];
-        scores(t, v);
+    if constexpr (LONG) {
+        // the order of the stand-alone Softmax: four keys, the tiles t and t + 8, then tile bits 2, 1, 0 and g bits 1, 0
+        float b0[4] = {}, b1[4] = {}, b2[4] = {}, tile[4] = {};
+        for (int i = 0; i < 16; ++i) {                       // i = (bit 0, bit 1, bit 2, chunk) of the tile
+            const int t = (i >> 3) + 2 * ((i >> 2) & 1) + 4 * ((i >> 1) & 1) + 8 * (i & 1);
+            if (t < nt) {
+                float v[16];
+                scores(t, v);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) sum += __builtin_amdgcn_exp2f(fmaf(v[r], kLog2e, mL));
+                for (int g = 0; g < 4; ++g)
+                    tile[g] += (expf(v[4 * g] - m) + expf(v[4 * g + 1] - m)) + (expf(v[4 * g + 2] - m) + expf(v[4 * g + 3] - m));
+            }
+            auto carry = [](float (&from)[4], float (&to)[4]) {
+#pragma unroll
+                for (int g = 0; g < 4; ++g) { to[g] += from[g]; from[g] = 0.f; }
+            };
+            if ((i & 1) == 1) carry(tile, b2);
+            if ((i & 3) == 3) carry(b2, b1);
+            if ((i & 7) == 7) carry(b1, b0);
+        }
+        sum = (b0[0] + b0[2]) + (b0[1] + b0[3]);
+    } else {
+        for (int t = 0; t < nt; ++t) {
+            float v[16];
+            scores(t, v);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sum += __builtin_amdgcn_exp2f(fmaf(v[r], kLog2e, mL));
+        }
     }
     sum += __shfl_xor(sum, 32, 64);
     const float inv = 1.0f / sum;
@@ -1062,8 +1086,8 @@ __device__ __forceinline__ void attention_queries(const ProgAttention& s, Buffer
         for (int g = 0; g < 4; ++g) {
             float p[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(fmaf(v[4 * g + j], kLog2e, mL)) * inv;
-            pf[g] = static_cast<int>(prob_levels4<DIV2, PFORM>(a, p[0], p[1], p[2], p[3]));
+            for (int j = 0; j < 4; ++j) p[j] = LONG ? quotient(expf(v[4 * g + j] - m), sum, inv) : __builtin_amdgcn_exp2f(fmaf(v[4 * g + j], kLog2e, mL)) * inv;
+            pf[g] = static_cast<int>(prob_levels4<true, PFORM>(a, p[0], p[1], p[2], p[3]));
         }
 #pragma unroll
         for (int db = 0; db < 2; ++db) {
@@ -1130,8 +1154,9 @@ __device__ __forceinline__ void attention_units(const ProgAttention& s, const Ct
         const int q0 = 32 * (part * s.waves + x.wave);
         if (x.wave < s.waves && q0 < S) {
             const uint32_t qbase = static_cast<uint32_t>(n * a.oq + hd * a.sq), obase = static_cast<uint32_t>(n * a.oo + hd * a.so);
-            if (s.pform == 2) attention_queries<true, 2>(s, qb, qbase, out, obase, q0, sK, sVT, sVsum, sMask, x.lane);
-            else attention_queries<true, 0>(s, qb, qbase, out, obase, q0, sK, sVT, sVsum, sMask, x.lane);
+            if (S > kPlainSoftmax) attention_queries<true, 0>(s, qb, qbase, out, obase, q0, sK, sVT, sVsum, sMask, x.lane);
+            else if (s.pform == 2) attention_queries<false, 2>(s, qb, qbase, out, obase, q0, sK, sVT, sVsum, sMask, x.lane);
+            else attention_queries<false, 0>(s, qb, qbase, out, obase, q0, sK, sVT, sVsum, sMask, x.lane);
         }
         __syncthreads();
     }

@@ -361,7 +361,7 @@ int hipie_embedding_f32(const float* table, int64_t vocabulary, int64_t hidden, 
  * batch element (strides in elements; 0 shares a row between the heads of a sequence), added to the
  * scaled scores of every query (reference::add with numpy broadcast).  scores / probs, when not NULL, receive the f32 values in front of and
  * behind the Softmax as dense [batch_outer * batch][seq][seq] arrays (inspection; the kernel is
- * otherwise the same).  Sequence lengths: multiples of 32 up to 384; head_dim 64
+ * otherwise the same).  Sequence lengths: multiples of 32 up to 384, of 64 up to 512; head_dim 64
  * (hipie_attention_supported). */
 typedef struct hipie_attention_desc {
     int32_t seq, head_dim;

@@ -321,6 +321,12 @@ def test_fused_attention(orc, B, NH, S):
     assert len(np.unique(want_q)) > 40
 
 
+@pytest.mark.parametrize("B,NH,S", [(1, 3, 448), (2, 1, 512), (2, 8, 512)])
+def test_fused_attention_of_long_rows(orc, B, NH, S):
+    """beyond 384 keys: rows of queries that do not fill the last workgroup (448), the longest, and the grouped grid"""
+    test_fused_attention(orc, B, NH, S)
+
+
 def test_fused_attention_rejects_unsupported_shapes():
     import torch
     from dldt_amd import HipieError, attention

@@ -19,6 +19,7 @@ GRAPHS = {
     "mobilenet_2": lambda: builders.mobilenet_v2(batch=2, res=96)[0],
     "encoder_1x32": lambda: builders.bert_encoder(layers=1, batch=1, seq=32, vocab=100, mask=True)[0],
     "encoder_3x96": lambda: builders.bert_encoder(layers=1, batch=3, seq=96, vocab=0, mask=False)[0],
+    "encoder_1x512": lambda: builders.bert_encoder(layers=1, batch=1, seq=512, vocab=100, mask=True)[0],
     "encoder_2x384": lambda: builders.bert_encoder(layers=1, batch=2, seq=384, vocab=100, mask=True)[0],
 }
 
