@@ -1119,7 +1119,8 @@ struct PlanConfig {
     int fuse_convs = 1;            // HIP_FUSE_CONVOLUTIONS: a 3 x 3 convolution and the 1 x 1 behind it in one kernel - NO (0), AUTO
                                    // (1: where the load-time measurement says it is faster), YES (2: wherever the kernel takes the pair)
     int single_launch = 1;         // HIP_SINGLE_LAUNCH: a request that is waited for runs as one kernel - NO (0), AUTO (1: a plan
-                                   // for one stream, where the load-time measurement says it is faster), YES (2: wherever there is such a form)
+                                   // for one stream, where the load-time measurement says it is faster), YES (2: wherever there
+                                   // is such a form, in the fastest of its sizes), 64 / 128 / 256: that many workgroups
     int device_id = -1;            // DEVICE_ID (must agree with the device argument when given)
     std::string network_name = "hipie_network";
 
@@ -1173,6 +1174,7 @@ struct PlanConfig {
             else fuse_convs = yes_no(key, value) ? 2 : 0;
         } else if (k == "HIP_SINGLE_LAUNCH") {
             if (!std::strcmp(value, "AUTO")) single_launch = 1;
+            else if (!std::strcmp(value, "64") || !std::strcmp(value, "128") || !std::strcmp(value, "256")) single_launch = std::atoi(value);
             else single_launch = yes_no(key, value) ? 2 : 0;
         }
         else if (k == "NETWORK_NAME") network_name = value;
@@ -1188,7 +1190,7 @@ struct PlanConfig {
         else if (k == "HIP_KEEP_F32") v = yn(keep_f32);
         else if (k == "HIP_FUSE_ATTENTION") v = yn(fuse_attention);
         else if (k == "HIP_MERGE_LINEAR") v = yn(merge_linear);
-        else if (k == "HIP_SINGLE_LAUNCH") v = single_launch == 1 ? "AUTO" : yn(single_launch == 2);
+        else if (k == "HIP_SINGLE_LAUNCH") v = single_launch == 1 ? "AUTO" : (single_launch > 2 ? std::to_string(single_launch) : yn(single_launch == 2));
         else if (k == "HIP_FUSE_CONVOLUTIONS") v = fuse_convs == 1 ? "AUTO" : yn(fuse_convs == 2);
         else return false;
         return true;
@@ -2942,8 +2944,10 @@ struct hipie_plan {
     // uploads the packed operands and takes the checks' verdicts instead of packing and checking again
     FqVerdicts verdicts;
     PackTape tape;
-    // the single-launch form, where the plan has one and runs it (requests that are waited for)
+    // the single-launch form, where the plan has one and runs it (requests that are waited for), and where it has none
+    // although it was asked for, the step that no single launch takes
     std::unique_ptr<Program> program;
+    std::string single_launch_refused;
 };
 
 struct hipie_request {
@@ -3017,7 +3021,9 @@ void finish_program(hipie_request* r) {
     r->by_program = false;
     const hipie_plan& p = *r->plan;
     program_done(*p.program, r->stream);
-    if (!program_failed(*p.program, r->slot, r->control, r->stream)) return;
+    const bool failed = program_failed(*p.program, r->slot, r->control, r->stream);
+    p.program->count(!failed);
+    if (!failed) return;
     r->launches = 0;
     enqueue(r, r->run_in.data(), r->run_out.data());
     for (size_t i = 0; i < r->host_out.size(); ++i)
@@ -3025,9 +3031,12 @@ void finish_program(hipie_request* r) {
     HIPIE_CHECK_HIP(hipStreamSynchronize(r->stream));
 }
 
-// the single-launch form of a plan whose every step has one, or null
-std::unique_ptr<Program> build_program(const hipie_plan& p, int workgroups) {
-    if (p.inputs.size() + p.outputs.size() > static_cast<size_t>(kProgramIo)) return nullptr;
+// the single-launch form of a plan whose every step has one, or null and what it has no room for
+std::unique_ptr<Program> build_program(const hipie_plan& p, int workgroups, std::string& refused) {
+    if (p.inputs.size() + p.outputs.size() > static_cast<size_t>(kProgramIo)) {
+        refused = "inputs and outputs";
+        return nullptr;
+    }
     ProgBuilder b;
     b.device = p.device;
     b.workgroups = workgroups;
@@ -3036,7 +3045,10 @@ std::unique_ptr<Program> build_program(const hipie_plan& p, int workgroups) {
     for (size_t i = 0; i < p.outputs.size(); ++i) out.push_back(b.fake_io(static_cast<int>(p.inputs.size() + i)));
     DeviceGuard g(p.device);
     for (const auto& s : p.steps)
-        if (!s->program(b, p.tensors, in.data(), out.data())) return nullptr;
+        if (!s->program(b, p.tensors, in.data(), out.data())) {
+            refused = s->name;
+            return nullptr;
+        }
     return make_program(std::move(b));
 }
 
@@ -3372,9 +3384,9 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
             }
         }
     }
-    if (device >= 0 && (cfg.single_launch == 2 || (cfg.single_launch == 1 && cfg.streams == 1 && cfg.tune))) {
+    if (device >= 0 && (cfg.single_launch >= 2 || (cfg.single_launch == 1 && cfg.streams == 1 && cfg.tune))) {
         // The single-launch form in its three sizes and the steps, as a caller sees them (start to wait): the fastest stays.
-        // Fewer workgroups have the cheaper barrier, more of them the shorter steps.
+        // Fewer workgroups have the cheaper barrier, more of them the shorter steps.  A size that was asked for is not measured.
         auto trial = [&] {
             hipie_request* q = nullptr;
             check_status(hipie_request_create(plan.get(), 0, &q), "hipie_compile: single-launch trial");
@@ -3392,18 +3404,21 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
             return t[t.size() / 2];
         };
         DeviceGuard dg(device);
-        double best = cfg.single_launch == 2 ? 1e30 : trial();
+        const bool fixed = cfg.single_launch > 2;
+        double best = cfg.single_launch >= 2 ? 1e30 : trial();
         std::unique_ptr<Program> fastest;
         for (int workgroups : {64, 128, 256}) {
-            plan->program = build_program(*plan, workgroups);
+            if (fixed && workgroups != cfg.single_launch) continue;
+            plan->program = build_program(*plan, workgroups, plan->single_launch_refused);
             if (!plan->program) break;
-            const double t = trial();
+            const double t = fixed ? 0.0 : trial();
             if (t < best) {
                 best = t;
                 fastest = std::move(plan->program);
             }
         }
         plan->program = std::move(fastest);
+        if (plan->program) plan->program->reset_counts();
     }
     return plan;
 }
@@ -3540,10 +3555,15 @@ int hipie_plan_get_metric(const hipie_plan* p, const char* name, char* buf, size
         HIPIE_REQUIRE(p && name, HIPIE_PARAMETER_MISMATCH, "hipie_plan_get_metric: null argument");
         const std::string k = name;
         std::string v;
-        if (k == "SUPPORTED_METRICS") v = "NETWORK_NAME SUPPORTED_METRICS SUPPORTED_CONFIG_KEYS OPTIMAL_NUMBER_OF_INFER_REQUESTS";
+        if (k == "SUPPORTED_METRICS")
+            v = "NETWORK_NAME SUPPORTED_METRICS SUPPORTED_CONFIG_KEYS OPTIMAL_NUMBER_OF_INFER_REQUESTS SINGLE_LAUNCH_WORKGROUPS "
+                "SINGLE_LAUNCH_COUNTS SINGLE_LAUNCH_REFUSED";
         else if (k == "SUPPORTED_CONFIG_KEYS") v = kConfigKeys;
         else if (k == "NETWORK_NAME") v = p->config.network_name;
         else if (k == "OPTIMAL_NUMBER_OF_INFER_REQUESTS") v = std::to_string(p->config.streams);
+        else if (k == "SINGLE_LAUNCH_WORKGROUPS") v = std::to_string(p->program ? p->program->workgroups : 0);
+        else if (k == "SINGLE_LAUNCH_COUNTS") v = p->program ? p->program->counts() : "0 0";
+        else if (k == "SINGLE_LAUNCH_REFUSED") v = p->single_launch_refused;
         else fail(HIPIE_NOT_FOUND, "metric '%s' is not supported", name);
         copy_text(v, buf, cap, "hipie_plan_get_metric");
     });

@@ -25,6 +25,7 @@
 #include <array>
 #include <memory>
 #include <mutex>
+#include <string>
 
 #include "attention.h"
 #include "conv.h"
@@ -151,9 +152,13 @@ struct Program {
     uint32_t* report = nullptr;              // page-locked, 16 dwords per slot
     std::mutex lock;
     uint64_t taken = 0;
+    uint64_t done = 0, cancelled = 0;        // launches that ran to their end, launches that were given up
     ~Program();
     int take_slot();                         // -1: none left
     void give_slot(int slot);
+    void count(bool ran);
+    void reset_counts();
+    std::string counts();                    // "done cancelled"
 };
 std::unique_ptr<Program> make_program(ProgBuilder&& b);
 

@@ -1649,6 +1649,21 @@ void Program::give_slot(int slot) {
     taken &= ~(uint64_t(1) << slot);
 }
 
+void Program::count(bool ran) {
+    std::lock_guard<std::mutex> g(lock);
+    ++(ran ? done : cancelled);
+}
+
+void Program::reset_counts() {
+    std::lock_guard<std::mutex> g(lock);
+    done = cancelled = 0;
+}
+
+std::string Program::counts() {
+    std::lock_guard<std::mutex> g(lock);
+    return std::to_string(done) + " " + std::to_string(cancelled);
+}
+
 std::unique_ptr<Program> make_program(ProgBuilder&& b) {
     auto p = std::make_unique<Program>();
     p->device = b.device;

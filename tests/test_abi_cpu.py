@@ -186,6 +186,19 @@ def test_device_metrics():
     assert metric("SUPPORTED_METRICS", cap=8)[0] == -6                          # buffer too small: OUT_OF_BOUNDS
 
 
+def test_single_launch_key_and_metrics():
+    g, _ = _tiny_graph()
+    for value in ("NO", "AUTO", "YES", "64", "128", "256"):
+        assert g.compile(-1, config={"HIP_SINGLE_LAUNCH": value}).config("HIP_SINGLE_LAUNCH") == value
+    for value in ("32", "512", "064", "64 ", ""):
+        with pytest.raises(HipieError) as e:
+            g.compile(-1, config={"HIP_SINGLE_LAUNCH": value})
+        assert e.value.status == -4
+    plan = g.compile(-1, config={"HIP_SINGLE_LAUNCH": "64"})                   # a dry run has no launches of any form
+    assert [plan.metric("SINGLE_LAUNCH_" + k) for k in ("WORKGROUPS", "COUNTS", "REFUSED")] == ["0", "0 0", ""]
+    assert "SINGLE_LAUNCH_WORKGROUPS" in plan.metric("SUPPORTED_METRICS").split()
+
+
 def test_query_reports_every_unsupported_node():
     g, ids = _tiny_graph(extra_relu=True)
     with pytest.raises(HipieError) as e:                                       # compiling stops at the first one ...

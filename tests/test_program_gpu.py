@@ -14,6 +14,8 @@ GRAPHS = {
     "block_2x17x9": lambda: builders.conv_block(n=2, c=17, hw=9, oc=65)[0],
     "block_1x64x56": lambda: builders.conv_block(n=1, c=64, hw=56, oc=64)[0],
     "block_3x256x16": lambda: builders.conv_block(n=3, c=256, hw=16, oc=130)[0],
+    "block_3x64x14": lambda: builders.conv_block(n=3, c=64, hw=14, oc=512)[0],
+    "block_7x64x32": lambda: builders.conv_block(n=7, c=64, hw=32, oc=130)[0],
     "resnet_1": lambda: builders.resnet50(batch=1, res=64, width=16, classes=10, seed=7)[0],
     "resnet_3_u8": lambda: builders.resnet50(batch=3, res=96, u8_input=True)[0],
     "mobilenet_2": lambda: builders.mobilenet_v2(batch=2, res=96)[0],
@@ -61,6 +63,34 @@ def test_single_launch_equals_steps(name):
     for seed in range(3):
         for x, y in zip(_infer(a, seed), _infer(b, seed)):
             assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
+
+
+# 256 workgroups meet through the XCDs, the others at one counter.  Together these choose every tile instance of the kernel:
+# 4 x 2 in the blocks of 3x64x14 (64 workgroups) and 7x64x32 (256), the others in the networks at every size
+@pytest.mark.parametrize("workgroups", [64, 128, 256])
+@pytest.mark.parametrize("name", sorted(GRAPHS))
+def test_every_size_runs_and_equals_steps(name, workgroups):
+    g = GRAPHS[name]()
+    steps, single = _compile(g, "NO"), _compile(g, str(workgroups))
+    assert single.config("HIP_SINGLE_LAUNCH") == single.metric("SINGLE_LAUNCH_WORKGROUPS") == str(workgroups)
+    assert steps.metric("SINGLE_LAUNCH_WORKGROUPS") == "0" and single.metric("SINGLE_LAUNCH_REFUSED") == ""
+    a, b = steps.create_request(), single.create_request()
+    for seed in range(3):
+        for x, y in zip(_infer(a, seed), _infer(b, seed)):
+            assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
+    assert single.metric("SINGLE_LAUNCH_COUNTS") == "3 0"       # the launches were the results compared
+
+
+def test_a_step_without_a_single_launch_form_is_named():
+    g = builders.bert_encoder(layers=1, batch=1, seq=64, vocab=100, mask=True)[0]
+    unfused = {"HIP_FUSE_ATTENTION": "NO", "HIP_TUNE": "NO", "HIP_THROUGHPUT_STREAMS": "1"}      # products and a Softmax of their own
+    plan = g.compile(0, config=dict(unfused, HIP_SINGLE_LAUNCH="YES"))
+    assert plan.metric("SINGLE_LAUNCH_WORKGROUPS") == "0" and plan.metric("SINGLE_LAUNCH_REFUSED") != ""
+    req = plan.create_request()
+    steps = g.compile(0, config=dict(unfused, HIP_SINGLE_LAUNCH="NO")).create_request()
+    for x, y in zip(_infer(steps, 0), _infer(req, 0)):
+        assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
+    assert plan.metric("SINGLE_LAUNCH_COUNTS") == "0 0"
 
 
 def test_single_launch_requests_on_two_streams():
