@@ -2966,6 +2966,7 @@ struct hipie_request {
     uint32_t* control = nullptr;
     uint32_t launches = 0;
     bool by_program = false;
+    bool stream_taken = false;               // hipie_request_stream gave the stream out: its work is complete in stream order
     std::vector<void*> run_in, run_out, host_out;
     ~hipie_request() {
         for (auto e : events) (void)hipEventDestroy(e);
@@ -3014,21 +3015,22 @@ void enqueue_program(hipie_request* r, void* const* in, void* const* out) {
     launch_program(*p.program, r->arena.as<uint8_t>(), io, static_cast<int>(p.inputs.size() + p.outputs.size()), r->control, r->launches++, r->slot, r->stream);
 }
 
-// the stream has been waited for: where the single launch gave up (its workgroups did not come together), the inference
-// runs again by steps, outputs included
-void finish_program(hipie_request* r) {
-    if (!r->by_program) return;
+// The stream has drained.  Where a single launch gave up (its workgroups did not come together) the inference is queued
+// again by steps, outputs included, and true says that there is something to wait for once more.
+bool run_again(hipie_request* r) {
+    if (!r->by_program) return false;
     r->by_program = false;
     const hipie_plan& p = *r->plan;
     program_done(*p.program, r->stream);
     const bool failed = program_failed(*p.program, r->slot, r->control, r->stream);
     p.program->count(!failed);
-    if (!failed) return;
+    if (!failed) return false;
     r->launches = 0;
+    if (r->cancelled) return false;          // (nobody reads its outputs)
     enqueue(r, r->run_in.data(), r->run_out.data());
     for (size_t i = 0; i < r->host_out.size(); ++i)
         HIPIE_CHECK_HIP(hipMemcpyAsync(r->host_out[i], r->run_out[i], static_cast<size_t>(p.outputs[i].bytes), hipMemcpyDeviceToHost, r->stream));
-    HIPIE_CHECK_HIP(hipStreamSynchronize(r->stream));
+    return true;
 }
 
 // the single-launch form of a plan whose every step has one, or null and what it has no room for
@@ -3843,10 +3845,16 @@ int hipie_request_stream(hipie_request* r, void** stream) {
     return guarded([&] {
         HIPIE_REQUIRE(r && stream, HIPIE_PARAMETER_MISMATCH, "hipie_request_stream: null argument");
         *stream = r->stream;
+        r->stream_taken = true;
     });
 }
 
-int hipie_request_start(hipie_request* r, const void* const* inputs, void* const* outputs, int device_memory) {
+// Which form an inference takes.  A single launch that does not come together is made up for by the host when it waits,
+// so it is taken only where nobody can see the outputs, or write the inputs, before that: inside hipie_request_infer, and
+// from host memory (the inputs are copied, the outputs are the caller's when the wait returns) while the caller does not
+// hold the stream.  Device buffers between start and wait may be read and written by work the caller orders behind the
+// stream, a synchronization of the device included: those inferences run by steps.
+static int start_request(hipie_request* r, const void* const* inputs, void* const* outputs, int device_memory, bool awaited) {
     return guarded([&] {
         HIPIE_REQUIRE(r && inputs && outputs, HIPIE_PARAMETER_MISMATCH, "hipie_request_start: null argument");
         HIPIE_REQUIRE(!r->started, HIPIE_REQUEST_BUSY, "hipie_request_start: request is busy");
@@ -3855,10 +3863,15 @@ int hipie_request_start(hipie_request* r, const void* const* inputs, void* const
         // a failure half-way leaves copies or kernels queued that read the caller's buffers: the stream is drained
         // before the error is reported, so that the caller may free or reuse them
         struct Drain {
-            hipStream_t s;
+            hipie_request* r;
             bool armed = true;
-            ~Drain() { if (armed) (void)hipStreamSynchronize(s); }
-        } drain{r->stream};
+            ~Drain() {
+                if (!armed) return;
+                (void)hipStreamSynchronize(r->stream);
+                if (r->by_program) program_done(*r->plan->program, r->stream);
+                r->by_program = false;
+            }
+        } drain{r};
         std::vector<void*> in(p.inputs.size()), out(p.outputs.size());
         for (size_t i = 0; i < in.size(); ++i) {
             HIPIE_REQUIRE(inputs[i], HIPIE_PARAMETER_MISMATCH, "hipie_request_start: input %zu is null", i);
@@ -3874,8 +3887,8 @@ int hipie_request_start(hipie_request* r, const void* const* inputs, void* const
             HIPIE_REQUIRE(outputs[i], HIPIE_PARAMETER_MISMATCH, "hipie_request_start: output %zu is null", i);
             out[i] = device_memory ? outputs[i] : r->out_dev[i].ptr;
         }
-        r->by_program = r->slot >= 0;
-        if (r->by_program) {
+        if (r->slot >= 0 && (awaited || (!device_memory && !r->stream_taken))) {
+            r->by_program = true;
             enqueue_program(r, in.data(), out.data());
             r->run_in = in;
             r->run_out = out;
@@ -3894,6 +3907,10 @@ int hipie_request_start(hipie_request* r, const void* const* inputs, void* const
     });
 }
 
+int hipie_request_start(hipie_request* r, const void* const* inputs, void* const* outputs, int device_memory) {
+    return start_request(r, inputs, outputs, device_memory, false);
+}
+
 /* Wait(millis_timeout) of AsyncInferRequestThreadSafeDefault (ie_infer_async_request_thread_safe_default.hpp:167-204):
  * -1 (RESULT_READY) blocks until the result is there, 0 (STATUS_ONLY) only asks, a positive value waits that many
  * milliseconds at most; HIPIE_RESULT_NOT_READY leaves the request busy.  A request that was cancelled while it
@@ -3905,24 +3922,31 @@ int hipie_request_wait_for(hipie_request* r, int64_t timeout_ms) {
                       "hipie_request_wait_for: timeout %lld (RESULT_READY = -1, STATUS_ONLY = 0, or milliseconds)", (long long)timeout_ms);
         HIPIE_REQUIRE(r->started, HIPIE_INFER_NOT_STARTED, "hipie_request_wait: nothing was started");
         DeviceGuard g(r->plan->device);
-        if (timeout_ms < 0) {
-            // (the request stays busy while this blocks: a Cancel from another thread in the meantime is seen below)
-            const hipError_t e = hipStreamSynchronize(r->stream);
-            r->started = false;
-            HIPIE_CHECK_HIP(e);
-            finish_program(r);
-        } else {
-            const auto deadline = std::chrono::steady_clock::now() + std::chrono::milliseconds(timeout_ms);
+        const auto deadline = std::chrono::steady_clock::now() + std::chrono::milliseconds(std::max<int64_t>(timeout_ms, 0));
+        // (the request stays busy while this blocks: a Cancel from another thread in the meantime is seen below; it is idle
+        // afterwards, also where the wait reports an error)
+        struct Idle {
+            hipie_request* r;
+            ~Idle() { if (r) r->started = r->by_program = false; }
+        } idle{r};
+        do {
+            if (timeout_ms < 0) {
+                HIPIE_CHECK_HIP(hipStreamSynchronize(r->stream));
+                continue;
+            }
             for (;;) {
                 const hipError_t q = hipStreamQuery(r->stream);
                 if (q == hipSuccess) break;
                 if (q != hipErrorNotReady) HIPIE_CHECK_HIP(q);
-                if (std::chrono::steady_clock::now() >= deadline) fail(HIPIE_RESULT_NOT_READY, "the inference is still running");
+                if (std::chrono::steady_clock::now() >= deadline) {
+                    idle.r = nullptr;
+                    fail(HIPIE_RESULT_NOT_READY, "the inference is still running");
+                }
                 std::this_thread::sleep_for(std::chrono::microseconds(50));
             }
-            r->started = false;
-            finish_program(r);
-        }
+        } while (run_again(r));
+        r->started = false;
+        idle.r = nullptr;
         if (r->cancelled.exchange(false)) fail(HIPIE_INFER_CANCELLED, "the inference was cancelled");
     });
 }
@@ -3941,7 +3965,7 @@ int hipie_request_cancel(hipie_request* r) {
 }
 
 int hipie_request_infer(hipie_request* r, const void* const* inputs, void* const* outputs, int device_memory) {
-    const int st = hipie_request_start(r, inputs, outputs, device_memory);
+    const int st = start_request(r, inputs, outputs, device_memory, true);
     return st != HIPIE_OK ? st : hipie_request_wait(r);
 }
 

@@ -16,6 +16,8 @@
 // launch is not complete in time (other work holds the compute units), it is cancelled by compare-and-swap before it has
 // written anything, the kernel drains, and the host runs the inference step by step.  Later waits are bounded as well (all
 // workgroups are resident by then, so they end; a bound that is hit ends the kernel and the host falls back the same way).
+// So the outputs are there when the host has waited, not before: the form is for inferences whose outputs nothing on the
+// device reads earlier (plan.hip, start_request).
 // One program is in flight per device: launches on different streams are ordered by an event (ProgramGate).
 //
 // (Measured beside it: one XCD per batch element, whose barrier costs 0.95 us and whose results stay in its own L2.  Thirty-two

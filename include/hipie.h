@@ -557,7 +557,11 @@ void hipie_request_destroy(hipie_request* request);
  * stream) or device memory (device_memory = 1: kernels only). */
 int hipie_request_infer(hipie_request* request, const void* const* inputs, void* const* outputs,
                         int device_memory);
-/* StartAsync / Wait(RESULT_READY) (ie_infer_async_request_thread_safe_default.hpp:167-214) */
+/* StartAsync / Wait(RESULT_READY) (ie_infer_async_request_thread_safe_default.hpp:167-214).  Device buffers are read and
+ * written in the order of the request's stream.  Host outputs are complete when the wait returns; where the caller took the
+ * request's stream (hipie_request_stream) they are complete in that stream's order as well.  A plan's single-launch form
+ * (HIP_SINGLE_LAUNCH) is used by hipie_request_infer, and by hipie_request_start on host memory of a request whose stream
+ * was not taken: a launch that does not come together is made up for by steps inside the wait. */
 int hipie_request_start(hipie_request* request, const void* const* inputs, void* const* outputs,
                         int device_memory);
 int hipie_request_wait(hipie_request* request);

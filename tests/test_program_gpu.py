@@ -5,7 +5,8 @@ import numpy as np
 import pytest
 import torch
 
-from dldt_amd import builders
+from dldt_amd import HipieError, builders
+from dldt_amd._lib import check, lib
 
 pytestmark = pytest.mark.gpu
 
@@ -110,6 +111,74 @@ def test_single_launch_requests_on_two_streams():
             r.wait()
         for (_, outs), w in zip(bufs, want):
             assert np.array_equal(outs[0].array.view(np.uint8), w[0].view(np.uint8))
+
+
+def _start_device(req, ins, outs):
+    check(lib().hipie_request_start(req._h, *req._ptrs(ins, outs), 1))
+
+
+@pytest.mark.parametrize("memory", ["device", "host"])
+def test_outputs_are_complete_in_the_order_of_a_stream_the_caller_holds(monkeypatch, memory):
+    """a copy that the caller queues behind the start sees the outputs, whatever becomes of a single launch"""
+    g = GRAPHS["resnet_1"]()
+    want = _infer(_compile(g, "NO").create_request(), 0)[0]
+    monkeypatch.setenv("HIPIE_ROLL_CALL_TICKS", "0")             # every launch is given up
+    req = _compile(g, "64").create_request()
+    ins, outs = req.device_buffers()
+    _fill(ins, 0)
+    stream = torch.cuda.ExternalStream(req.stream)
+    outs[0].fill_(float("nan"))
+    torch.cuda.synchronize()
+    if memory == "device":
+        _start_device(req, ins, outs)
+        with torch.cuda.stream(stream):
+            seen = outs[0].clone()
+            ins[0].zero_()                                       # the inference has read its input by then
+        stream.synchronize()
+    else:
+        hin, hout = req.host_buffers()
+        hin[0].array[...] = ins[0].cpu().numpy()
+        hout[0].array[...] = np.nan
+        req.start(hin, hout)
+        stream.synchronize()
+        seen = torch.from_numpy(hout[0].array.copy())
+    req.wait()
+    assert np.array_equal(seen.cpu().numpy().view(np.uint8), want.view(np.uint8))
+
+
+@pytest.mark.parametrize("timeout", [-1, 0, 5, 10000])
+def test_cancelled_launch_of_host_buffers_is_made_up_for_in_the_wait(monkeypatch, timeout):
+    g = GRAPHS["resnet_1"]()
+    steps = _compile(g, "NO").create_request()
+    monkeypatch.setenv("HIPIE_ROLL_CALL_TICKS", "0")
+    plan = _compile(g, "128")
+    req = plan.create_request()
+    hin, hout = req.host_buffers()
+    for seed in range(2):
+        want = _infer(steps, seed)[0]
+        dev = steps.device_buffers()[0]
+        _fill(dev, seed)
+        hin[0].array[...] = dev[0].cpu().numpy()
+        hout[0].array[...] = np.nan
+        req.start(hin, hout)
+        for _ in range(100000):
+            try:
+                req.wait_for(timeout)
+                break
+            except HipieError as e:
+                assert e.status == -9 and timeout != -1          # still running, busy
+        assert np.array_equal(hout[0].array.view(np.uint8), want.view(np.uint8))
+        with pytest.raises(HipieError):                          # idle again
+            req.wait()
+    # a caller that revoked the inference gets no outputs of it, and the next one is whole
+    req.start(hin, hout)
+    req.cancel()
+    with pytest.raises(HipieError) as e:
+        req.wait()
+    assert e.value.status == -13
+    req.start(hin, hout)
+    req.wait()
+    assert np.array_equal(hout[0].array.view(np.uint8), want.view(np.uint8))
 
 
 def test_cancelled_launch_runs_by_steps(monkeypatch):
