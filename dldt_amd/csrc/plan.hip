@@ -2946,12 +2946,16 @@ struct hipie_plan {
     PackTape tape;
     // the single-launch form, where the plan has one and runs it (requests that are waited for), and where it has none
     // although it was asked for, the step that no single launch takes
-    std::unique_ptr<Program> program;
+    std::shared_ptr<Program> program;
     std::string single_launch_refused;
 };
 
 struct hipie_request {
+    // (what the destructor needs is held here: a plan may be destroyed before its requests, e.g. by a garbage collector that
+    // finds both in one cycle)
     const hipie_plan* plan = nullptr;
+    int device = 0;
+    std::shared_ptr<Program> program;
     DeviceBuffer arena;
     std::vector<DeviceBuffer> in_dev, out_dev;
     hipStream_t stream = nullptr;
@@ -2973,10 +2977,10 @@ struct hipie_request {
         if (stream) {
             (void)hipStreamSynchronize(stream);
             if (slot >= 0) {
-                program_done(*plan->program, stream);
-                plan->program->give_slot(slot);
+                program_done(*program, stream);
+                program->give_slot(slot);
             }
-            if (plan) release_split_workspace(plan->device, stream);
+            release_split_workspace(device, stream);
             (void)hipStreamDestroy(stream);
         }
     }
@@ -3012,7 +3016,7 @@ void enqueue_program(hipie_request* r, void* const* in, void* const* out) {
     void* io[kProgramIo] = {};
     for (size_t i = 0; i < p.inputs.size(); ++i) io[i] = in[i];
     for (size_t i = 0; i < p.outputs.size(); ++i) io[p.inputs.size() + i] = out[i];
-    launch_program(*p.program, r->arena.as<uint8_t>(), io, static_cast<int>(p.inputs.size() + p.outputs.size()), r->control, r->launches++, r->slot, r->stream);
+    launch_program(*r->program, r->arena.as<uint8_t>(), io, static_cast<int>(p.inputs.size() + p.outputs.size()), r->control, r->launches++, r->slot, r->stream);
 }
 
 // The stream has drained.  Where a single launch gave up (its workgroups did not come together) the inference is queued
@@ -3021,9 +3025,9 @@ bool run_again(hipie_request* r) {
     if (!r->by_program) return false;
     r->by_program = false;
     const hipie_plan& p = *r->plan;
-    program_done(*p.program, r->stream);
-    const bool failed = program_failed(*p.program, r->slot, r->control, r->stream);
-    p.program->count(!failed);
+    program_done(*r->program, r->stream);
+    const bool failed = program_failed(*r->program, r->slot, r->control, r->stream);
+    r->program->count(!failed);
     if (!failed) return false;
     r->launches = 0;
     if (r->cancelled) return false;          // (nobody reads its outputs)
@@ -3408,7 +3412,7 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
         DeviceGuard dg(device);
         const bool fixed = cfg.single_launch > 2;
         double best = cfg.single_launch >= 2 ? 1e30 : trial();
-        std::unique_ptr<Program> fastest;
+        std::shared_ptr<Program> fastest;
         for (int workgroups : {64, 128, 256}) {
             if (fixed && workgroups != cfg.single_launch) continue;
             plan->program = build_program(*plan, workgroups, plan->single_launch_refused);
@@ -3796,6 +3800,7 @@ int hipie_request_create(const hipie_plan* p, int perf_count, hipie_request** ou
                       "hipie_request_create: the plan was compiled without a device (dry run)");
         auto r = std::make_unique<hipie_request>();
         r->plan = p;
+        r->device = p->device;
         r->perf = perf_count < 0 ? p->config.perf_count : perf_count != 0;   // < 0: the plan's PERF_COUNT
         DeviceGuard g(p->device);
         HIPIE_CHECK_HIP(hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking));
@@ -3805,7 +3810,10 @@ int hipie_request_create(const hipie_plan* p, int perf_count, hipie_request** ou
         uint8_t* a = r->arena.as<uint8_t>();
         HIPIE_CHECK_HIP(hipMemsetAsync(a, 0, static_cast<size_t>(control_at) + kProgramControlBytes, r->stream));
         r->control = reinterpret_cast<uint32_t*>(a + control_at);
-        if (p->program && !r->perf) r->slot = p->program->take_slot();
+        if (p->program && !r->perf) {
+            r->program = p->program;
+            r->slot = r->program->take_slot();
+        }
         for (const auto& t : p->tensors) {
             if (t.alias >= 0) continue;
             const int byte = t.dtype == HIPIE_U8B ? t.fill_level - 128 : (t.dtype == HIPIE_I8 ? t.fill_level : 0);
@@ -3868,7 +3876,7 @@ static int start_request(hipie_request* r, const void* const* inputs, void* cons
             ~Drain() {
                 if (!armed) return;
                 (void)hipStreamSynchronize(r->stream);
-                if (r->by_program) program_done(*r->plan->program, r->stream);
+                if (r->by_program) program_done(*r->program, r->stream);
                 r->by_program = false;
             }
         } drain{r};

@@ -551,6 +551,7 @@ int hipie_plan_step_sources(const hipie_plan* plan, int index, int* sources, int
 /* IExecutableNetworkInternal::CreateInferRequestImpl: own stream + own activation arena; weights
  * stay shared in the plan.  perf_count mirrors the PERF_COUNT config key (ie_plugin_config.hpp:277). */
 int hipie_request_create(const hipie_plan* plan, int perf_count /* 1, 0, or -1 = the plan's PERF_COUNT */, hipie_request** request);
+/* (also after its plan was destroyed; nothing else can be done with a request then) */
 void hipie_request_destroy(hipie_request* request);
 /* IInferRequestInternal::InferImpl (ie_iinfer_request_internal.hpp:57).  inputs / outputs are dense
  * NCHW buffers in plan order: host memory (device_memory = 0: H2D, kernels, D2H on the request's

@@ -181,6 +181,22 @@ def test_cancelled_launch_of_host_buffers_is_made_up_for_in_the_wait(monkeypatch
     assert np.array_equal(hout[0].array.view(np.uint8), want.view(np.uint8))
 
 
+def test_a_request_outlives_its_plan():
+    """the order in which a garbage collector finalizes a cycle that holds both"""
+    g = GRAPHS["resnet_1"]()
+    plan = _compile(g, "64")
+    reqs = [plan.create_request() for _ in range(3)]
+    for r in reqs:
+        _infer(r, 0)
+    lib().hipie_plan_destroy(plan._h)
+    plan._h = None
+    junk = [_compile(GRAPHS["block_1x3x7"](), "NO") for _ in range(3)]      # takes the freed memory
+    for r in reqs:
+        lib().hipie_request_destroy(r._h)
+        r._h = None
+    del junk
+
+
 def test_cancelled_launch_runs_by_steps(monkeypatch):
     g = GRAPHS["resnet_1"]()
     steps = _compile(g, "NO")
