@@ -3862,6 +3862,21 @@ int hipie_request_stream(hipie_request* r, void** stream) {
 // from host memory (the inputs are copied, the outputs are the caller's when the wait returns) while the caller does not
 // hold the stream.  Device buffers between start and wait may be read and written by work the caller orders behind the
 // stream, a synchronization of the device included: those inferences run by steps.
+//
+// The steps look at the caller's pointers each time they run (alignment: some take the general path, some refuse); the
+// single launch was checked with stand-ins, on a 16-byte boundary and apart from each other.  Other buffers go by steps.
+static bool buffers_fit_program(const hipie_plan& p, void* const* in, void* const* out) {
+    const size_t n_in = p.inputs.size(), n = n_in + p.outputs.size();
+    auto at = [&](size_t k) { return reinterpret_cast<uintptr_t>(k < n_in ? in[k] : out[k - n_in]); };
+    auto bytes = [&](size_t k) { return static_cast<uintptr_t>(k < n_in ? p.inputs[k].bytes : p.outputs[k - n_in].bytes); };
+    for (size_t k = 0; k < n; ++k) {
+        if (at(k) % 16 != 0) return false;
+        for (size_t j = n_in; k >= n_in ? j < k : j < n; ++j)        // (inputs may lie on each other: they are only read)
+            if (at(k) < at(j) + bytes(j) && at(j) < at(k) + bytes(k)) return false;
+    }
+    return true;
+}
+
 static int start_request(hipie_request* r, const void* const* inputs, void* const* outputs, int device_memory, bool awaited) {
     return guarded([&] {
         HIPIE_REQUIRE(r && inputs && outputs, HIPIE_PARAMETER_MISMATCH, "hipie_request_start: null argument");
@@ -3895,7 +3910,7 @@ static int start_request(hipie_request* r, const void* const* inputs, void* cons
             HIPIE_REQUIRE(outputs[i], HIPIE_PARAMETER_MISMATCH, "hipie_request_start: output %zu is null", i);
             out[i] = device_memory ? outputs[i] : r->out_dev[i].ptr;
         }
-        if (r->slot >= 0 && (awaited || (!device_memory && !r->stream_taken))) {
+        if (r->slot >= 0 && (awaited || (!device_memory && !r->stream_taken)) && buffers_fit_program(p, in.data(), out.data())) {
             r->by_program = true;
             enqueue_program(r, in.data(), out.data());
             r->run_in = in;

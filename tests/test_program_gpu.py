@@ -181,6 +181,54 @@ def test_cancelled_launch_of_host_buffers_is_made_up_for_in_the_wait(monkeypatch
     assert np.array_equal(hout[0].array.view(np.uint8), want.view(np.uint8))
 
 
+def _at(t, offset):
+    """the tensor's values `offset` elements behind a 256-byte boundary"""
+    room = torch.zeros(t.numel() + 64, dtype=t.dtype, device="cuda")
+    view = room[offset:offset + t.numel()].view(t.shape)
+    view.copy_(t)
+    return view
+
+
+@pytest.mark.parametrize("offset", [0, 1, 2, 4])
+@pytest.mark.parametrize("name", ["block_1x64x56", "encoder_3x96"])
+def test_buffers_off_the_boundary_are_left_to_the_steps(name, offset):
+    """what the steps refuse (an f32 residual that is a graph input) stays refused, what they take stays right"""
+    g = GRAPHS[name]()
+    steps, single = _compile(g, "NO"), _compile(g, "64")
+    a, b = steps.create_request(), single.create_request()
+    ins, _ = a.device_buffers()
+    _fill(ins, 0)
+    want = _infer(a, 0)
+    shifted = [_at(t, offset) for t in ins]
+    outs = [_at(torch.zeros_like(o), offset) for o in a.device_buffers()[1]]
+    status = []
+    for r in (a, b):
+        for o in outs:
+            o.fill_(float("nan"))
+        torch.cuda.synchronize()
+        try:
+            r.infer_device(shifted, outs)
+            status.append(0)
+            assert np.array_equal(outs[0].cpu().numpy().view(np.uint8), want[0].view(np.uint8))
+        except HipieError as e:
+            status.append(e.status)
+    assert status[0] == status[1]
+    assert status[0] == (-4 if name.startswith("encoder") and offset % 4 else 0)
+    assert single.metric("SINGLE_LAUNCH_COUNTS") == ("0 0" if offset % 4 else "1 0")
+
+
+def test_an_output_on_its_input_is_left_to_the_steps():
+    g = builders.conv_block(n=1, c=64, hw=14, oc=64)[0]
+    plan = _compile(g, "64")
+    req = plan.create_request()
+    want = _infer(req, 0)[0]
+    ins, outs = req.device_buffers()
+    _fill(ins, 0)
+    req.infer_device(ins, ins)
+    assert np.array_equal(ins[0].cpu().numpy().view(np.uint8), want.view(np.uint8))
+    assert plan.metric("SINGLE_LAUNCH_COUNTS") == "1 0"
+
+
 def test_a_request_outlives_its_plan():
     """the order in which a garbage collector finalizes a cycle that holds both"""
     g = GRAPHS["resnet_1"]()
