@@ -3418,6 +3418,7 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
             plan->program = build_program(*plan, workgroups, plan->single_launch_refused);
             if (!plan->program) break;
             const double t = fixed ? 0.0 : trial();
+            if (cfg.single_launch == 1 && plan->program->cancelled) continue;      // (something else holds the device: not this form's time)
             if (t < best) {
                 best = t;
                 fastest = std::move(plan->program);
@@ -3910,7 +3911,8 @@ static int start_request(hipie_request* r, const void* const* inputs, void* cons
             HIPIE_REQUIRE(outputs[i], HIPIE_PARAMETER_MISMATCH, "hipie_request_start: output %zu is null", i);
             out[i] = device_memory ? outputs[i] : r->out_dev[i].ptr;
         }
-        if (r->slot >= 0 && (awaited || (!device_memory && !r->stream_taken)) && buffers_fit_program(p, in.data(), out.data())) {
+        if (r->slot >= 0 && (awaited || (!device_memory && !r->stream_taken)) && buffers_fit_program(p, in.data(), out.data()) &&
+            r->program->admit()) {
             r->by_program = true;
             enqueue_program(r, in.data(), out.data());
             r->run_in = in;

@@ -14,7 +14,8 @@
 //
 // Termination: a barrier needs every workgroup resident.  The roll call in front of the first step has a deadline: if the
 // launch is not complete in time (other work holds the compute units), it is cancelled by compare-and-swap before it has
-// written anything, the kernel drains, and the host runs the inference step by step.  Later waits are bounded as well (all
+// written anything, the kernel drains, and the host runs the inference step by step, as it does with a growing number of the
+// requests behind it (Program::count).  Later waits are bounded as well (all
 // workgroups are resident by then, so they end; a bound that is hit ends the kernel and the host falls back the same way).
 // So the outputs are there when the host has waited, not before: the form is for inferences whose outputs nothing on the
 // device reads earlier (plan.hip, start_request).
@@ -155,9 +156,14 @@ struct Program {
     std::mutex lock;
     uint64_t taken = 0;
     uint64_t done = 0, cancelled = 0;        // launches that ran to their end, launches that were given up
+    // A launch that was given up cost its wait, and what held the compute units is likely still there: the next requests run
+    // by steps, 4 of them, 20, 84 .. as launches go on failing; every launch that completes halves the number.
+    static constexpr uint32_t kMostSkipped = 1024;
+    uint32_t skip = 0, penalty = 0;
     ~Program();
     int take_slot();                         // -1: none left
     void give_slot(int slot);
+    bool admit();                            // whether the next request is to be launched as one
     void count(bool ran);
     void reset_counts();
     std::string counts();                    // "done cancelled"

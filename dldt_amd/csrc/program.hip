@@ -25,7 +25,10 @@ constexpr int kPartBytes = 128 * 1024;       // partial sums of eight waves x 16
 constexpr int kKoffBytes = 16 * 1024;        // K offsets of the step's convolutions
 constexpr int kMaxPieces = kKoffBytes / 4 / 2;
 constexpr int kLdsBytes = kPartBytes + kKoffBytes + 64;
-constexpr uint32_t kRollCallTicks = 3000000; // 30 ms of the 100 MHz clock
+// How long a launch waits for its last workgroup: 1 ms of the 100 MHz clock.  Alone it is complete in a few microseconds, behind
+// the kernels of another request in the time these take; what holds compute units longer (another process's launch that
+// waits for the same units) does not let go, and the steps need less than that beside it.
+constexpr uint32_t kRollCallTicks = 100000, kMaxRollCallTicks = 10000000;
 constexpr uint64_t kBarrierTicks = 200000000;
 
 typedef __attribute__((address_space(3))) int8_t* lds_ptr;
@@ -1649,14 +1652,29 @@ void Program::give_slot(int slot) {
     taken &= ~(uint64_t(1) << slot);
 }
 
+bool Program::admit() {
+    std::lock_guard<std::mutex> g(lock);
+    if (skip == 0) return true;
+    --skip;
+    return false;
+}
+
 void Program::count(bool ran) {
     std::lock_guard<std::mutex> g(lock);
-    ++(ran ? done : cancelled);
+    if (ran) {
+        ++done;
+        penalty /= 2;
+    } else {
+        ++cancelled;
+        penalty = std::min(4 * penalty + 4, kMostSkipped);
+        skip = penalty;
+    }
 }
 
 void Program::reset_counts() {
     std::lock_guard<std::mutex> g(lock);
     done = cancelled = 0;
+    skip = penalty = 0;
 }
 
 std::string Program::counts() {
@@ -1668,8 +1686,12 @@ std::unique_ptr<Program> make_program(ProgBuilder&& b) {
     auto p = std::make_unique<Program>();
     p->device = b.device;
     p->workgroups = b.workgroups;
-    const char* ticks = std::getenv("HIPIE_ROLL_CALL_TICKS");      // (0: every launch is cancelled and runs again by steps)
-    p->roll_call_ticks = ticks ? static_cast<uint32_t>(std::strtoul(ticks, nullptr, 10)) : kRollCallTicks;
+    p->roll_call_ticks = kRollCallTicks;
+    if (const char* ticks = std::getenv("HIPIE_ROLL_CALL_TICKS")) {      // (0: every launch is given up and runs again by steps)
+        char* end = nullptr;
+        const unsigned long n = std::strtoul(ticks, &end, 10);
+        if (end != ticks && *end == 0) p->roll_call_ticks = static_cast<uint32_t>(std::min<unsigned long>(n, kMaxRollCallTicks));
+    }
     p->n_steps = static_cast<int>(b.steps.size());
     p->steps.upload(b.device, b.steps.data(), b.steps.size() * kProgramStepWords * 4);
     p->owned = std::move(b.owned);

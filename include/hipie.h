@@ -487,7 +487,8 @@ int hipie_compile(const hipie_graph* graph, int device, hipie_plan** plan);
  * HIPIE_PARAMETER_MISMATCH.  The environment variables HIPIE_TUNE, HIPIE_TUNE_FILE, HIPIE_TUNE_STREAMS,
  * HIPIE_FUSE_ATTENTION, HIPIE_MERGE_LINEAR, HIPIE_KEEP_F32, HIPIE_FUSE_CONVS and
  * HIPIE_SINGLE_LAUNCH (0 | 1 | 2 = NO | AUTO | YES) are the
- * process-wide defaults of these keys. */
+ * process-wide defaults of these keys.  HIPIE_ROLL_CALL_TICKS (0 .. 10000000, in units of 10 ns, default 100000 = 1 ms; read
+ * when a plan is compiled) is how long a single launch waits until all of its workgroups run before it is given up. */
 int hipie_compile_opts(const hipie_graph* graph, int device, const char* const* keys, const char* const* values,
                        int n_opts, hipie_plan** plan);
 void hipie_plan_destroy(hipie_plan* plan);

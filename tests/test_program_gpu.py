@@ -181,6 +181,29 @@ def test_cancelled_launch_of_host_buffers_is_made_up_for_in_the_wait(monkeypatch
     assert np.array_equal(hout[0].array.view(np.uint8), want.view(np.uint8))
 
 
+def test_launches_that_fail_are_tried_less_and_less(monkeypatch):
+    g = GRAPHS["block_2x17x9"]()
+    want = _infer(_compile(g, "NO").create_request(), 0)[0]
+    monkeypatch.setenv("HIPIE_ROLL_CALL_TICKS", "0")
+    plan = _compile(g, "64")
+    req = plan.create_request()
+    given_up = []
+    for i in range(1 + 4 + 1 + 20 + 1 + 84 + 1):
+        before = plan.metric("SINGLE_LAUNCH_COUNTS")
+        assert np.array_equal(_infer(req, 0)[0].view(np.uint8), want.view(np.uint8))
+        if plan.metric("SINGLE_LAUNCH_COUNTS") != before:
+            given_up.append(i)
+    assert given_up == [0, 5, 26, 111] and plan.metric("SINGLE_LAUNCH_COUNTS") == "0 4"
+
+
+@pytest.mark.parametrize("ticks,counts", [("", "1 0"), ("soon", "1 0"), ("-1", "1 0"), ("99999999999999999999", "1 0"), ("0", "0 1")])
+def test_roll_call_deadline_is_a_number_within_its_range(monkeypatch, ticks, counts):
+    monkeypatch.setenv("HIPIE_ROLL_CALL_TICKS", ticks)
+    plan = _compile(GRAPHS["block_2x17x9"](), "64")
+    _infer(plan.create_request(), 0)
+    assert plan.metric("SINGLE_LAUNCH_COUNTS") == counts
+
+
 def _at(t, offset):
     """the tensor's values `offset` elements behind a 256-byte boundary"""
     room = torch.zeros(t.numel() + 64, dtype=t.dtype, device="cuda")
