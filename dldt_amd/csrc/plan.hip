@@ -2964,22 +2964,31 @@ struct hipie_request {
     // written by the thread that starts and waits, and by whichever thread calls hipie_request_cancel meanwhile
     std::atomic<bool> started{false};
     std::atomic<bool> cancelled{false};      // hipie_request_cancel was called on the running inference
-    // the single-launch form: the request's slot (-1: none), its control block behind the arena, launches it counts, and
-    // what a run that the kernel gave up has to do again by steps
+    // the single-launch form: the request's slot (-1: none), its control blocks behind the arena (of the lone and the shared
+    // form) and the launches they count, the form that is running, and what a run that the kernel gave up has to do again by steps
     int slot = -1;
     uint32_t* control = nullptr;
-    uint32_t launches = 0;
-    bool by_program = false;
+    uint32_t launches[kProgramControlBlocks] = {};
+    const ProgramForm* form = nullptr;
+    bool entered = false;                    // counted among the device's requests in flight
     bool stream_taken = false;               // hipie_request_stream gave the stream out: its work is complete in stream order
     std::vector<void*> run_in, run_out, host_out;
+    // the stream has drained
+    void leave_form() {
+        if (form) program->leave(form);
+        form = nullptr;
+    }
+    void leave() {
+        leave_form();
+        if (entered) request_leaves(device);
+        entered = false;
+    }
     ~hipie_request() {
         for (auto e : events) (void)hipEventDestroy(e);
         if (stream) {
             (void)hipStreamSynchronize(stream);
-            if (slot >= 0) {
-                program_done(*program, stream);
-                program->give_slot(slot);
-            }
+            leave();
+            if (slot >= 0) program->give_slot(slot);
             release_split_workspace(device, stream);
             (void)hipStreamDestroy(stream);
         }
@@ -3016,20 +3025,22 @@ void enqueue_program(hipie_request* r, void* const* in, void* const* out) {
     void* io[kProgramIo] = {};
     for (size_t i = 0; i < p.inputs.size(); ++i) io[i] = in[i];
     for (size_t i = 0; i < p.outputs.size(); ++i) io[p.inputs.size() + i] = out[i];
-    launch_program(*r->program, r->arena.as<uint8_t>(), io, static_cast<int>(p.inputs.size() + p.outputs.size()), r->control, r->launches++, r->slot, r->stream);
+    const int block = r->form == r->program->lone.get() ? 0 : 1;
+    launch_program(*r->program, *r->form, r->arena.as<uint8_t>(), io, static_cast<int>(p.inputs.size() + p.outputs.size()),
+                   r->control + block * (kProgramControlBytes / 4), r->launches[block]++, r->slot, r->stream);
 }
 
 // The stream has drained.  Where a single launch gave up (its workgroups did not come together) the inference is queued
 // again by steps, outputs included, and true says that there is something to wait for once more.
 bool run_again(hipie_request* r) {
-    if (!r->by_program) return false;
-    r->by_program = false;
+    if (!r->form) return false;
     const hipie_plan& p = *r->plan;
-    program_done(*r->program, r->stream);
-    const bool failed = program_failed(*r->program, r->slot, r->control, r->stream);
+    const int block = r->form == r->program->lone.get() ? 0 : 1;
+    r->leave_form();
+    const bool failed = program_failed(*r->program, r->slot, r->control + block * (kProgramControlBytes / 4), r->stream);
     r->program->count(!failed);
     if (!failed) return false;
-    r->launches = 0;
+    r->launches[block] = 0;
     if (r->cancelled) return false;          // (nobody reads its outputs)
     enqueue(r, r->run_in.data(), r->run_out.data());
     for (size_t i = 0; i < r->host_out.size(); ++i)
@@ -3038,7 +3049,7 @@ bool run_again(hipie_request* r) {
 }
 
 // the single-launch form of a plan whose every step has one, or null and what it has no room for
-std::unique_ptr<Program> build_program(const hipie_plan& p, int workgroups, std::string& refused) {
+std::shared_ptr<ProgramForm> build_program(const hipie_plan& p, int workgroups, std::string& refused) {
     if (p.inputs.size() + p.outputs.size() > static_cast<size_t>(kProgramIo)) {
         refused = "inputs and outputs";
         return nullptr;
@@ -3055,7 +3066,7 @@ std::unique_ptr<Program> build_program(const hipie_plan& p, int workgroups, std:
             refused = s->name;
             return nullptr;
         }
-    return make_program(std::move(b));
+    return make_program_form(std::move(b));
 }
 
 // `preset`: kernel variants of an imported plan, one per step; used when they fit the steps planned
@@ -3391,8 +3402,11 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
         }
     }
     if (device >= 0 && (cfg.single_launch >= 2 || (cfg.single_launch == 1 && cfg.streams == 1 && cfg.tune))) {
-        // The single-launch form in its three sizes and the steps, as a caller sees them (start to wait): the fastest stays.
-        // Fewer workgroups have the cheaper barrier, more of them the shorter steps.  A size that was asked for is not measured.
+        // The single-launch form in its three sizes and the steps, as a caller sees them (start to wait): the fastest is what a
+        // lone request takes.  Fewer workgroups have the cheaper barrier, more of them the shorter steps.  Beside other requests
+        // the smallest form that is no slower than the steps is taken: two or four of them side by side are faster than the
+        // steps of as many requests, which at best share the device without loss.  A size that was asked for is not measured.
+        constexpr int kTrialTurns = 15;
         auto trial = [&] {
             hipie_request* q = nullptr;
             check_status(hipie_request_create(plan.get(), 0, &q), "hipie_compile: single-launch trial");
@@ -3401,7 +3415,7 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
             for (auto& b : q->in_dev) in.push_back(b.ptr);
             for (auto& b : q->out_dev) out.push_back(b.ptr);
             std::vector<double> t;
-            for (int turn = 0; turn < 15; ++turn) {
+            for (int turn = 0; turn < kTrialTurns; ++turn) {
                 const auto t0 = std::chrono::steady_clock::now();
                 check_status(hipie_request_infer(q, in.data(), out.data(), 1), "hipie_compile: single-launch trial");
                 if (turn >= 4) t.push_back(std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
@@ -3411,21 +3425,38 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
         };
         DeviceGuard dg(device);
         const bool fixed = cfg.single_launch > 2;
-        double best = cfg.single_launch >= 2 ? 1e30 : trial();
-        std::shared_ptr<Program> fastest;
+        const double steps_time = fixed ? 0.0 : trial();
+        double best = cfg.single_launch >= 2 ? 1e30 : steps_time;
+        auto program = make_program(device);
+        std::shared_ptr<ProgramForm> lone, shared;
         for (int workgroups : {64, 128, 256}) {
-            if (fixed && workgroups != cfg.single_launch) continue;
-            plan->program = build_program(*plan, workgroups, plan->single_launch_refused);
-            if (!plan->program) break;
-            const double t = fixed ? 0.0 : trial();
-            if (cfg.single_launch == 1 && plan->program->cancelled) continue;      // (something else holds the device: not this form's time)
+            if ((fixed && workgroups != cfg.single_launch) || workgroups > program->units) continue;
+            const auto form = build_program(*plan, workgroups, plan->single_launch_refused);
+            if (!form) break;
+            if (fixed) {
+                lone = shared = form;
+                break;
+            }
+            plan->program = program;
+            program->lone = program->shared = form;
+            program->reset_counts();
+            const double t = trial();
+            plan->program = nullptr;
+            // (other work held the device and some of these requests ran by steps: not this form's time)
+            const bool own_time = program->done >= kTrialTurns;
+            if (cfg.single_launch == 1 && !own_time) continue;
+            if (own_time && t <= steps_time && workgroups < 256 && !shared) shared = form;
             if (t < best) {
                 best = t;
-                fastest = std::move(plan->program);
+                lone = form;
             }
         }
-        plan->program = std::move(fastest);
-        if (plan->program) plan->program->reset_counts();
+        if (lone) {
+            program->lone = lone;
+            program->shared = shared;
+            program->reset_counts();
+            plan->program = program;
+        }
     }
     return plan;
 }
@@ -3564,11 +3595,12 @@ int hipie_plan_get_metric(const hipie_plan* p, const char* name, char* buf, size
         std::string v;
         if (k == "SUPPORTED_METRICS")
             v = "NETWORK_NAME SUPPORTED_METRICS SUPPORTED_CONFIG_KEYS OPTIMAL_NUMBER_OF_INFER_REQUESTS SINGLE_LAUNCH_WORKGROUPS "
-                "SINGLE_LAUNCH_COUNTS SINGLE_LAUNCH_REFUSED";
+                "SINGLE_LAUNCH_SHARED_WORKGROUPS SINGLE_LAUNCH_COUNTS SINGLE_LAUNCH_REFUSED";
         else if (k == "SUPPORTED_CONFIG_KEYS") v = kConfigKeys;
         else if (k == "NETWORK_NAME") v = p->config.network_name;
         else if (k == "OPTIMAL_NUMBER_OF_INFER_REQUESTS") v = std::to_string(p->config.streams);
-        else if (k == "SINGLE_LAUNCH_WORKGROUPS") v = std::to_string(p->program ? p->program->workgroups : 0);
+        else if (k == "SINGLE_LAUNCH_WORKGROUPS") v = std::to_string(p->program ? p->program->lone->workgroups : 0);
+        else if (k == "SINGLE_LAUNCH_SHARED_WORKGROUPS") v = std::to_string(p->program && p->program->shared ? p->program->shared->workgroups : 0);
         else if (k == "SINGLE_LAUNCH_COUNTS") v = p->program ? p->program->counts() : "0 0";
         else if (k == "SINGLE_LAUNCH_REFUSED") v = p->single_launch_refused;
         else fail(HIPIE_NOT_FOUND, "metric '%s' is not supported", name);
@@ -3806,10 +3838,11 @@ int hipie_request_create(const hipie_plan* p, int perf_count, hipie_request** ou
         DeviceGuard g(p->device);
         HIPIE_CHECK_HIP(hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking));
         const int64_t control_at = round_up(p->arena_bytes, 256);
-        r->arena.alloc(p->device, static_cast<size_t>(control_at) + kProgramControlBytes);
+        const size_t control_bytes = kProgramControlBytes * kProgramControlBlocks;
+        r->arena.alloc(p->device, static_cast<size_t>(control_at) + control_bytes);
         // level 0 everywhere: halos and channel padding are never written again
         uint8_t* a = r->arena.as<uint8_t>();
-        HIPIE_CHECK_HIP(hipMemsetAsync(a, 0, static_cast<size_t>(control_at) + kProgramControlBytes, r->stream));
+        HIPIE_CHECK_HIP(hipMemsetAsync(a, 0, static_cast<size_t>(control_at) + control_bytes, r->stream));
         r->control = reinterpret_cast<uint32_t*>(a + control_at);
         if (p->program && !r->perf) {
             r->program = p->program;
@@ -3892,8 +3925,7 @@ static int start_request(hipie_request* r, const void* const* inputs, void* cons
             ~Drain() {
                 if (!armed) return;
                 (void)hipStreamSynchronize(r->stream);
-                if (r->by_program) program_done(*r->program, r->stream);
-                r->by_program = false;
+                r->leave();
             }
         } drain{r};
         std::vector<void*> in(p.inputs.size()), out(p.outputs.size());
@@ -3911,9 +3943,11 @@ static int start_request(hipie_request* r, const void* const* inputs, void* cons
             HIPIE_REQUIRE(outputs[i], HIPIE_PARAMETER_MISMATCH, "hipie_request_start: output %zu is null", i);
             out[i] = device_memory ? outputs[i] : r->out_dev[i].ptr;
         }
-        if (r->slot >= 0 && (awaited || (!device_memory && !r->stream_taken)) && buffers_fit_program(p, in.data(), out.data()) &&
-            r->program->admit()) {
-            r->by_program = true;
+        r->entered = true;
+        const int together = request_enters(p.device);
+        if (r->slot >= 0 && (awaited || (!device_memory && !r->stream_taken)) && buffers_fit_program(p, in.data(), out.data()))
+            r->form = r->program->choose(together);
+        if (r->form) {
             enqueue_program(r, in.data(), out.data());
             r->run_in = in;
             r->run_out = out;
@@ -3950,28 +3984,32 @@ int hipie_request_wait_for(hipie_request* r, int64_t timeout_ms) {
         const auto deadline = std::chrono::steady_clock::now() + std::chrono::milliseconds(std::max<int64_t>(timeout_ms, 0));
         // (the request stays busy while this blocks: a Cancel from another thread in the meantime is seen below; it is idle
         // afterwards, also where the wait reports an error)
-        struct Idle {
-            hipie_request* r;
-            ~Idle() { if (r) r->started = r->by_program = false; }
-        } idle{r};
-        do {
-            if (timeout_ms < 0) {
-                HIPIE_CHECK_HIP(hipStreamSynchronize(r->stream));
-                continue;
-            }
-            for (;;) {
-                const hipError_t q = hipStreamQuery(r->stream);
-                if (q == hipSuccess) break;
-                if (q != hipErrorNotReady) HIPIE_CHECK_HIP(q);
-                if (std::chrono::steady_clock::now() >= deadline) {
-                    idle.r = nullptr;
-                    fail(HIPIE_RESULT_NOT_READY, "the inference is still running");
+        {
+            struct Idle {
+                hipie_request* r;
+                ~Idle() {
+                    if (!r) return;
+                    r->leave();
+                    r->started = false;
                 }
-                std::this_thread::sleep_for(std::chrono::microseconds(50));
-            }
-        } while (run_again(r));
-        r->started = false;
-        idle.r = nullptr;
+            } idle{r};
+            do {
+                if (timeout_ms < 0) {
+                    HIPIE_CHECK_HIP(hipStreamSynchronize(r->stream));
+                    continue;
+                }
+                for (;;) {
+                    const hipError_t q = hipStreamQuery(r->stream);
+                    if (q == hipSuccess) break;
+                    if (q != hipErrorNotReady) HIPIE_CHECK_HIP(q);
+                    if (std::chrono::steady_clock::now() >= deadline) {
+                        idle.r = nullptr;
+                        fail(HIPIE_RESULT_NOT_READY, "the inference is still running");
+                    }
+                    std::this_thread::sleep_for(std::chrono::microseconds(50));
+                }
+            } while (run_again(r));
+        }
         if (r->cancelled.exchange(false)) fail(HIPIE_INFER_CANCELLED, "the inference was cancelled");
     });
 }

@@ -19,7 +19,7 @@
 // workgroups are resident by then, so they end; a bound that is hit ends the kernel and the host falls back the same way).
 // So the outputs are there when the host has waited, not before: the form is for inferences whose outputs nothing on the
 // device reads earlier (plan.hip, start_request).
-// One program is in flight per device: launches on different streams are ordered by an event (ProgramGate).
+// Programs in flight together never ask for more compute units than there are (Program::choose).
 //
 // (Measured beside it: one XCD per batch element, whose barrier costs 0.95 us and whose results stay in its own L2.  Thirty-two
 // compute units on one L2 then do all of an image's work: 20 - 30 bytes a clock and unit of operands and the whole f32 chain
@@ -145,12 +145,20 @@ struct ProgBuilder {
     bool copy(const void* in, void* out, int64_t bytes);
 };
 
-// A plan's program: the step list on the device and the page-locked words the kernel reports failures in.
-struct Program {
-    int device = 0, workgroups = 0, n_steps = 0;
-    uint32_t roll_call_ticks = 0;
+// The step list of one size on the device, with its own packing of the weights (the tile shapes depend on the size)
+struct ProgramForm {
+    int workgroups = 0, n_steps = 0;
     DeviceBuffer steps;
     std::vector<DeviceBuffer> owned;
+};
+std::shared_ptr<ProgramForm> make_program_form(ProgBuilder&& b);
+
+// A plan's program: its forms and the page-locked words the kernel reports failures in.
+struct Program {
+    int device = 0, units = 0;               // compute units the device has
+    uint32_t roll_call_ticks = 0;
+    std::shared_ptr<ProgramForm> lone;       // for a request that has the device to itself
+    std::shared_ptr<ProgramForm> shared;     // beside other requests (may be the same one; null: those run by steps)
     static constexpr int kSlots = 64;        // requests of one plan that can use the program
     uint32_t* report = nullptr;              // page-locked, 16 dwords per slot
     std::mutex lock;
@@ -163,18 +171,23 @@ struct Program {
     ~Program();
     int take_slot();                         // -1: none left
     void give_slot(int slot);
-    bool admit();                            // whether the next request is to be launched as one
+    const ProgramForm* choose(int together); // the form that the next request takes, its compute units held; null: the steps
+    void leave(const ProgramForm* f);        // gives them back: the stream has been waited for
     void count(bool ran);
     void reset_counts();
     std::string counts();                    // "done cancelled"
 };
-std::unique_ptr<Program> make_program(ProgBuilder&& b);
+std::shared_ptr<Program> make_program(int device);
+// A request is started / has been waited for, by whatever form; the former gives how many were in flight together lately
+int request_enters(int device);
+void request_leaves(int device);
 
-constexpr size_t kProgramControlBytes = 4096;    // barrier counters and the roll call's verdict: behind the arena, zero before the first launch
+// barrier counters and the roll call's verdict: behind the arena, zero before the first launch.  A block counts the launches
+// of one form, whose number of workgroups it adds up.
+constexpr size_t kProgramControlBytes = 2048, kProgramControlBlocks = 2;
 // `launch`: how many launches used this control block before; io: the call's input and output buffers in order
-void launch_program(const Program& p, uint8_t* arena, void* const* io, int n_io, uint32_t* control, uint32_t launch, int slot, hipStream_t s);
-// after the stream has been waited for (or is about to be destroyed)
-void program_done(const Program& p, hipStream_t s);
+void launch_program(const Program& p, const ProgramForm& f, uint8_t* arena, void* const* io, int n_io, uint32_t* control, uint32_t launch, int slot,
+                    hipStream_t s);
 // what the last launch of a slot reported: 0 done; anything else: it did not run to its end, and `control` has been
 // cleared on the stream (the caller runs the inference by steps and counts its launches from zero again)
 bool program_failed(const Program& p, int slot, uint32_t* control, hipStream_t s);

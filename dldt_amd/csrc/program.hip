@@ -1329,14 +1329,17 @@ TileChoice choose_tile(int workgroups, int oc, int64_t pixels, int nk, int nk2, 
     return best;
 }
 
-struct ProgramGate {
+// What is in flight on a device, of all plans: how many requests were started and not yet waited for, and how many compute
+// units their programs hold.
+struct DeviceLoad {
     std::mutex lock;
-    hipStream_t last = nullptr;      // stream of the program in flight, if any
-    hipEvent_t event = nullptr;
+    int requests = 0, units = 0;
+    int together = 0, hold = 0;      // the most requests in flight when one of the last kHold was started
+    static constexpr int kHold = 16;
 };
-ProgramGate& gate(int device) {
-    static ProgramGate gates[64];
-    return gates[device & 63];
+DeviceLoad& device_load(int device) {
+    static DeviceLoad loads[64];
+    return loads[device & 63];
 }
 
 }  // namespace
@@ -1652,13 +1655,6 @@ void Program::give_slot(int slot) {
     taken &= ~(uint64_t(1) << slot);
 }
 
-bool Program::admit() {
-    std::lock_guard<std::mutex> g(lock);
-    if (skip == 0) return true;
-    --skip;
-    return false;
-}
-
 void Program::count(bool ran) {
     std::lock_guard<std::mutex> g(lock);
     if (ran) {
@@ -1682,55 +1678,93 @@ std::string Program::counts() {
     return std::to_string(done) + " " + std::to_string(cancelled);
 }
 
-std::unique_ptr<Program> make_program(ProgBuilder&& b) {
-    auto p = std::make_unique<Program>();
-    p->device = b.device;
-    p->workgroups = b.workgroups;
+std::shared_ptr<ProgramForm> make_program_form(ProgBuilder&& b) {
+    auto f = std::make_shared<ProgramForm>();
+    f->workgroups = b.workgroups;
+    f->n_steps = static_cast<int>(b.steps.size());
+    f->steps.upload(b.device, b.steps.data(), b.steps.size() * kProgramStepWords * 4);
+    f->owned = std::move(b.owned);
+    DeviceGuard g(b.device);
+    HIPIE_CHECK_HIP(hipStreamSynchronize(nullptr));      // the repacking kernels
+    return f;
+}
+
+std::shared_ptr<Program> make_program(int device) {
+    auto p = std::make_shared<Program>();
+    p->device = device;
     p->roll_call_ticks = kRollCallTicks;
     if (const char* ticks = std::getenv("HIPIE_ROLL_CALL_TICKS")) {      // (0: every launch is given up and runs again by steps)
         char* end = nullptr;
         const unsigned long n = std::strtoul(ticks, &end, 10);
         if (end != ticks && *end == 0) p->roll_call_ticks = static_cast<uint32_t>(std::min<unsigned long>(n, kMaxRollCallTicks));
     }
-    p->n_steps = static_cast<int>(b.steps.size());
-    p->steps.upload(b.device, b.steps.data(), b.steps.size() * kProgramStepWords * 4);
-    p->owned = std::move(b.owned);
-    DeviceGuard g(b.device);
+    HIPIE_CHECK_HIP(hipDeviceGetAttribute(&p->units, hipDeviceAttributeMultiprocessorCount, device));
+    DeviceGuard g(device);
     HIPIE_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&p->report), Program::kSlots * 64, hipHostMallocDefault));
     std::memset(p->report, 0, Program::kSlots * 64);
-    HIPIE_CHECK_HIP(hipStreamSynchronize(nullptr));      // the repacking kernels
     HIPIE_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&program_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     return p;
 }
 
-void launch_program(const Program& p, uint8_t* arena, void* const* io, int n_io, uint32_t* control, uint32_t launch, int slot, hipStream_t s) {
+int request_enters(int device) {
+    DeviceLoad& d = device_load(device);
+    std::lock_guard<std::mutex> g(d.lock);
+    ++d.requests;
+    if (d.requests >= d.together || --d.hold <= 0) {
+        d.together = d.requests;
+        d.hold = DeviceLoad::kHold;
+    }
+    return d.together;
+}
+
+void request_leaves(int device) {
+    DeviceLoad& d = device_load(device);
+    std::lock_guard<std::mutex> g(d.lock);
+    --d.requests;
+}
+
+// A lone request takes the form that was fastest alone.  Beside others it takes the smaller one, if units are left for it
+// (never more workgroups than compute units, so that all of them find a place), and else the steps, whose kernels share the
+// device.  ResNet-50, batch 1, us a request with 2 and 4 in flight: 256 workgroups one behind the other 322 and 321, steps 252
+// and 245, 64 workgroups side by side 186 and 177 (alone: 294, 488, 352).  With more than twice as many requests as find a
+// place the ones by steps wait for the others: batch 3 with 128 workgroups, 4 in flight: 244, steps 261; 6 in flight: 207, steps
+// 179 (batch 1 with 64 workgroups, 6 in flight: 135, steps 166).
+const ProgramForm* Program::choose(int together) {
+    const ProgramForm* f = together > 1 ? shared.get() : lone.get();
+    if (!f || (lone != shared && together > 1 && together * f->workgroups > 2 * units)) return nullptr;
+    std::lock_guard<std::mutex> g(lock);
+    if (skip > 0) {
+        --skip;
+        return nullptr;
+    }
+    DeviceLoad& d = device_load(device);
+    std::lock_guard<std::mutex> hold(d.lock);
+    if (d.units + f->workgroups > units) return nullptr;
+    d.units += f->workgroups;
+    return f;
+}
+
+void Program::leave(const ProgramForm* f) {
+    DeviceLoad& d = device_load(device);
+    std::lock_guard<std::mutex> g(d.lock);
+    d.units -= f->workgroups;
+}
+
+void launch_program(const Program& p, const ProgramForm& f, uint8_t* arena, void* const* io, int n_io, uint32_t* control, uint32_t launch, int slot,
+                    hipStream_t s) {
     ProgArgs a{};
-    a.steps = p.steps.as<int32_t>();
+    a.steps = f.steps.as<int32_t>();
     a.bases[0] = arena;
     for (int i = 0; i < n_io; ++i) a.bases[1 + i] = io[i];
     a.control = control;
     a.report = p.report + 16 * slot;
-    a.n_steps = p.n_steps;
-    a.workgroups = p.workgroups;
+    a.n_steps = f.n_steps;
+    a.workgroups = f.workgroups;
     a.launch = launch;
     a.roll_call_ticks = p.roll_call_ticks;
     p.report[16 * slot] = 0;
-    ProgramGate& g = gate(p.device);
-    std::lock_guard<std::mutex> hold(g.lock);
-    if (g.last && g.last != s) {
-        if (!g.event) HIPIE_CHECK_HIP(hipEventCreateWithFlags(&g.event, hipEventDisableTiming));
-        HIPIE_CHECK_HIP(hipEventRecord(g.event, g.last));
-        HIPIE_CHECK_HIP(hipStreamWaitEvent(s, g.event, 0));
-    }
-    hipLaunchKernelGGL(program_kernel, dim3(static_cast<uint32_t>(p.workgroups)), dim3(kProgramThreads), kLdsBytes, s, a);
+    hipLaunchKernelGGL(program_kernel, dim3(static_cast<uint32_t>(f.workgroups)), dim3(kProgramThreads), kLdsBytes, s, a);
     HIPIE_CHECK_HIP(hipGetLastError());
-    g.last = s;
-}
-
-void program_done(const Program& p, hipStream_t s) {
-    ProgramGate& g = gate(p.device);
-    std::lock_guard<std::mutex> hold(g.lock);
-    if (g.last == s) g.last = nullptr;
 }
 
 bool program_failed(const Program& p, int slot, uint32_t* control, hipStream_t s) {

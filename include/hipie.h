@@ -483,7 +483,9 @@ int hipie_compile(const hipie_graph* graph, int device, hipie_plan** plan);
  * the pair, NO; the tensor between two layers run that way exists in LDS only and hipie_request_tensor gives
  * HIPIE_NOT_FOUND for it), HIP_SINGLE_LAUNCH (a request that is started and waited for runs as one persistent kernel:
  * AUTO = a plan for one stream, where the load-time measurement finds it faster, YES = wherever the plan has such a form,
- * in the fastest of its sizes, 64 / 128 / 256 = with that many workgroups, NO), NETWORK_NAME.  An unknown key gives HIPIE_NOT_FOUND, a value the key does not take
+ * in the fastest of its sizes, 64 / 128 / 256 = with that many workgroups, NO; beside other requests in flight the smallest
+ * form that was no slower than the steps is used, as many at a time as the device has compute units for, and the steps
+ * otherwise), NETWORK_NAME.  An unknown key gives HIPIE_NOT_FOUND, a value the key does not take
  * HIPIE_PARAMETER_MISMATCH.  The environment variables HIPIE_TUNE, HIPIE_TUNE_FILE, HIPIE_TUNE_STREAMS,
  * HIPIE_FUSE_ATTENTION, HIPIE_MERGE_LINEAR, HIPIE_KEEP_F32, HIPIE_FUSE_CONVS and
  * HIPIE_SINGLE_LAUNCH (0 | 1 | 2 = NO | AUTO | YES) are the
@@ -505,7 +507,8 @@ int hipie_get_metric(int device, const char* name, char* buf, size_t buf_len);
 /* IExecutableNetworkInternal::GetMetric / GetConfig (template_executable_network.cpp:154-176): NETWORK_NAME,
  * SUPPORTED_METRICS, SUPPORTED_CONFIG_KEYS, OPTIMAL_NUMBER_OF_INFER_REQUESTS (what benchmark_app asks for,
  * samples/benchmark_app/main.cpp:456-472); the config keys of hipie_compile_opts with the values the plan was compiled with.
- * Beside the reference's metrics, of the plan's single-launch form: SINGLE_LAUNCH_WORKGROUPS (0: the plan runs by steps),
+ * Beside the reference's metrics, of the plan's single-launch form: SINGLE_LAUNCH_WORKGROUPS of a lone request (0: the plan
+ * runs by steps) and SINGLE_LAUNCH_SHARED_WORKGROUPS of one beside others (0: those run by steps),
  * SINGLE_LAUNCH_COUNTS ("completed given-up": requests that ran as one launch, launches that did not come together and ran
  * again by steps), SINGLE_LAUNCH_REFUSED (the step that has no such form where one was wanted, else empty) */
 int hipie_plan_get_metric(const hipie_plan* plan, const char* name, char* buf, size_t buf_len);

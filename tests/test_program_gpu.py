@@ -1,6 +1,8 @@
 """The single-launch form of a plan (csrc/program.hip) against its steps, bit for bit: tile remainders in pixels and channels,
 K of one step and of many, strides, residuals, shortcuts, depthwise, pools, encoder steps; the ordering of launches on
 several streams; and the way back to the steps when a launch is cancelled."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -179,6 +181,103 @@ def test_cancelled_launch_of_host_buffers_is_made_up_for_in_the_wait(monkeypatch
     req.start(hin, hout)
     req.wait()
     assert np.array_equal(hout[0].array.view(np.uint8), want.view(np.uint8))
+
+
+def _host_request(plan, feed):
+    """(request, its host blobs) with the values of the device tensors `feed` in the inputs"""
+    req = plan.create_request()
+    ins, outs = req.host_buffers()
+    for a, t in zip(ins, feed):
+        a.array[...] = t.cpu().numpy()
+    return req, ins, outs
+
+
+def _feed_and_result(g, seed):
+    req = _compile(g, "NO").create_request()
+    out = _infer(req, seed)
+    ins, _ = req.device_buffers()
+    _fill(ins, seed)
+    return ins, out
+
+
+def _same(outs, want):
+    return all(np.array_equal(o.array.view(np.uint8), w.view(np.uint8)) for o, w in zip(outs, want))
+
+
+@pytest.mark.parametrize("workgroups,together", [(64, 4), (128, 2), (256, 1)])
+def test_programs_in_flight_fit_the_device(workgroups, together):
+    """five requests of one plan started one behind the other: as many run as programs as there are compute units for"""
+    g = GRAPHS["resnet_1"]()
+    plan = _compile(g, str(workgroups))
+    work = [_feed_and_result(g, s) for s in range(5)]
+    reqs = [_host_request(plan, feed) for feed, _ in work]
+    for turn in range(1, 4):
+        for r, ins, outs in reqs:
+            outs[0].array[...] = np.nan
+            r.start(ins, outs)
+        for r, _, _ in reqs:
+            r.wait()
+        assert all(_same(outs, want) for (_, _, outs), (_, want) in zip(reqs, work))
+        assert plan.metric("SINGLE_LAUNCH_COUNTS") == "%d 0" % (turn * together)
+
+
+def test_programs_of_two_plans_and_steps_of_a_third_side_by_side():
+    graphs = [GRAPHS[n]() for n in ("encoder_3x96", "mobilenet_2", "resnet_3_u8")]
+    plans = [_compile(g, m) for g, m in zip(graphs, ("64", "128", "NO"))]
+    work = [_feed_and_result(g, 1) for g in graphs]
+    reqs = [_host_request(p, feed) for p, (feed, _) in zip(plans, work)]
+    for _ in range(20):
+        for r, ins, outs in reqs:
+            outs[0].array[...] = np.nan
+            r.start(ins, outs)
+        for r, _, _ in reversed(reqs):
+            r.wait()
+        assert all(_same(outs, want) for (_, _, outs), (_, want) in zip(reqs, work))
+    assert [p.metric("SINGLE_LAUNCH_COUNTS") for p in plans] == ["20 0", "20 0", "0 0"]
+
+
+@pytest.mark.parametrize("mode", ["64", "256", "YES"])
+def test_requests_of_several_threads(mode):
+    """three threads that infer one request each, of two plans; every result, whichever form it took"""
+    graphs = [GRAPHS["resnet_1"](), GRAPHS["encoder_1x32"]()]
+    plans = [_compile(g, mode) for g in graphs]
+    failed = []
+
+    def loop(which, seed):
+        try:
+            torch.cuda.set_device(0)
+            feed, want = work[seed]
+            req = plans[which].create_request()
+            _, outs = req.device_buffers()
+            for _ in range(50):
+                req.infer_device(feed, outs)
+                if not np.array_equal(outs[0].cpu().numpy().view(np.uint8), want[0].view(np.uint8)):
+                    failed.append(seed)
+        except Exception as e:                                   # noqa: BLE001 (reported below)
+            failed.append(e)
+
+    work = [_feed_and_result(graphs[which], seed) for seed, which in enumerate((0, 1, 0))]
+    threads = [threading.Thread(target=loop, args=(which, seed)) for seed, which in enumerate((0, 1, 0))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed
+    assert all(p.metric("SINGLE_LAUNCH_COUNTS") != "0 0" for p in plans)
+
+
+def test_more_requests_than_a_plan_has_slots():
+    g = GRAPHS["block_1x3x7"]()
+    plan = _compile(g, "64")
+    want = _infer(_compile(g, "NO").create_request(), 0)[0]
+    reqs = [plan.create_request() for _ in range(66)]            # 64 slots; the others run by steps
+    for r in reqs:
+        assert np.array_equal(_infer(r, 0)[0].view(np.uint8), want.view(np.uint8))
+    assert plan.metric("SINGLE_LAUNCH_COUNTS") == "64 0"
+    del reqs[10]                                                 # (r is the last one)
+    again = plan.create_request()
+    assert np.array_equal(_infer(again, 0)[0].view(np.uint8), want.view(np.uint8))
+    assert plan.metric("SINGLE_LAUNCH_COUNTS") == "65 0"
 
 
 def test_launches_that_fail_are_tried_less_and_less(monkeypatch):
