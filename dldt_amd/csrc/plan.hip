@@ -2927,6 +2927,14 @@ struct Planner {
 
 using namespace hipie;
 
+// The sizes of the single-launch form that a measurement chose (0: the steps), from an exported plan or a tuning file
+struct FormChoice {
+    bool known = false, imported = false;
+    int lone = 0, shared = 0;
+    static bool size(int v) { return v == 0 || v == 64 || v == 128 || v == 256; }
+    bool valid() const { return size(lone) && size(shared) && (lone != 0 || shared == 0); }
+};
+
 struct hipie_plan {
     int device = 0;
     hipie_graph graph;                       // the description the plan was compiled from (what an export writes)
@@ -2948,6 +2956,7 @@ struct hipie_plan {
     // although it was asked for, the step that no single launch takes
     std::shared_ptr<Program> program;
     std::string single_launch_refused;
+    FormChoice forms;                        // what was measured of it, for an export
 };
 
 struct hipie_request {
@@ -3162,7 +3171,8 @@ bool to_two_spatial_dimensions(const hipie_graph& g, hipie_graph& out) {
 }
 
 std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const std::vector<int>* preset,
-                                         const PlanConfig& cfg = PlanConfig::from_environment(), PlanPrepared* prepared = nullptr) {
+                                         const PlanConfig& cfg = PlanConfig::from_environment(), PlanPrepared* prepared = nullptr,
+                                         FormChoice forms = FormChoice()) {
     HIPIE_REQUIRE(!g->results.empty(), HIPIE_PARAMETER_MISMATCH, "hipie_compile: graph has no Result");
     HIPIE_REQUIRE(cfg.device_id < 0 || device < 0 || cfg.device_id == device, HIPIE_PARAMETER_MISMATCH,
                   "hipie_compile: DEVICE_ID %d against device %d", cfg.device_id, device);
@@ -3338,7 +3348,8 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
         plan->outputs.push_back({n.name, dt, n.shape, n.numel() * (dt == HIPIE_F32 ? 4 : 1)});
     }
     // Kernel selection by measurement on a scratch request (HIPIE_TUNE=0 keeps the shape-based
-    // defaults).  HIPIE_TUNE_FILE names a cache of the choices, one "step variant" pair a line:
+    // defaults).  HIPIE_TUNE_FILE names a cache of the choices, one "step variant" pair a line, and behind them the workgroups
+    // of the single-launch form as "-1 lone" and "-2 shared" where that was measured:
     // read when it matches this plan, written after tuning otherwise (the reference's GPU plugin
     // keeps its tuning results in a file the same way, inference-engine/include/cldnn/cldnn_config.hpp:125 KEY_TUNING_FILE).
     bool preset_used = false;
@@ -3350,16 +3361,29 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
             preset_used = true;
         }
     }
+    const char* cache = nullptr;
+    auto write_cache = [&] {
+        FILE* f = cache ? std::fopen(cache, "w") : nullptr;
+        if (!f) return;
+        for (size_t i = 0; i < plan->steps.size(); ++i) std::fprintf(f, "%zu %d\n", i, plan->steps[i]->variant());
+        if (forms.known) std::fprintf(f, "-1 %d\n-2 %d\n", forms.lone, forms.shared);
+        std::fclose(f);
+    };
     if (device >= 0 && !preset_used && cfg.tune) {
-        const char* cache = cfg.tune_file.empty() ? nullptr : cfg.tune_file.c_str();
+        cache = cfg.tune_file.empty() ? nullptr : cfg.tune_file.c_str();
         bool loaded = false;
         if (cache) {
             if (FILE* f = std::fopen(cache, "r")) {
                 std::vector<int> v(plan->steps.size(), -2);
                 size_t n = 0;
                 int idx = 0, var = 0;
+                FormChoice stored;
+                int found = 0;
                 while (std::fscanf(f, "%d %d", &idx, &var) == 2)
-                    if (idx >= 0 && static_cast<size_t>(idx) < v.size() && v[idx] == -2) {
+                    if (idx == -1 || idx == -2) {
+                        (idx == -1 ? stored.lone : stored.shared) = var;
+                        found |= -idx;
+                    } else if (idx >= 0 && static_cast<size_t>(idx) < v.size() && v[idx] == -2) {
                         v[idx] = var;
                         ++n;
                     }
@@ -3370,6 +3394,8 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
                 if (match) {
                     for (size_t i = 0; i < v.size(); ++i) plan->steps[i]->set_variant(v[i]);
                     loaded = true;
+                    stored.known = found == 3;
+                    if (stored.known && stored.valid()) forms = stored;
                 }
             }
         }
@@ -3392,16 +3418,12 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
             }
             DeviceGuard dg(device);
             for (auto& s : plan->steps) s->tune(lanes, plan->tensors);
-            if (cache) {
-                if (FILE* f = std::fopen(cache, "w")) {
-                    for (size_t i = 0; i < plan->steps.size(); ++i)
-                        std::fprintf(f, "%zu %d\n", i, plan->steps[i]->variant());
-                    std::fclose(f);
-                }
-            }
+            write_cache();
         }
     }
-    if (device >= 0 && (cfg.single_launch >= 2 || (cfg.single_launch == 1 && cfg.streams == 1 && cfg.tune))) {
+    // (a plan that was exported with its kernels chosen and no form measured had none)
+    const bool measured = forms.known || (forms.imported && preset_used);
+    if (device >= 0 && (cfg.single_launch >= 2 || (cfg.single_launch == 1 && cfg.streams == 1 && (measured ? forms.known : cfg.tune)))) {
         // The single-launch form in its three sizes and the steps, as a caller sees them (start to wait): the fastest is what a
         // lone request takes.  Fewer workgroups have the cheaper barrier, more of them the shorter steps.  Beside other requests
         // the smallest form that is no slower than the steps is taken: two or four of them side by side are faster than the
@@ -3424,40 +3446,47 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
             return t[t.size() / 2];
         };
         DeviceGuard dg(device);
-        const bool fixed = cfg.single_launch > 2;
-        const double steps_time = fixed ? 0.0 : trial();
-        double best = cfg.single_launch >= 2 ? 1e30 : steps_time;
         auto program = make_program(device);
-        std::shared_ptr<ProgramForm> lone, shared;
-        for (int workgroups : {64, 128, 256}) {
-            if ((fixed && workgroups != cfg.single_launch) || workgroups > program->units) continue;
-            const auto form = build_program(*plan, workgroups, plan->single_launch_refused);
-            if (!form) break;
-            if (fixed) {
-                lone = shared = form;
-                break;
+        auto build = [&](int workgroups) {
+            return workgroups == 0 || workgroups > program->units ? nullptr : build_program(*plan, workgroups, plan->single_launch_refused);
+        };
+        if (cfg.single_launch > 2) {
+            program->lone = program->shared = build(cfg.single_launch);
+        } else if (forms.known && (forms.lone != 0 || cfg.single_launch == 1)) {
+            program->lone = build(forms.lone);
+            if (program->lone) program->shared = forms.shared == forms.lone ? program->lone : build(forms.shared);
+        } else {
+            const double steps_time = trial();
+            double best = cfg.single_launch == 2 ? 1e30 : steps_time;
+            std::shared_ptr<ProgramForm> lone, shared;
+            for (int workgroups : {64, 128, 256}) {
+                const auto form = build(workgroups);
+                if (!form) break;
+                plan->program = program;
+                program->lone = program->shared = form;
+                program->reset_counts();
+                const double t = trial();
+                plan->program = nullptr;
+                // (other work held the device and some of these requests ran by steps: not this form's time)
+                const bool own_time = program->done >= kTrialTurns;
+                if (cfg.single_launch == 1 && !own_time) continue;
+                if (own_time && t <= steps_time && workgroups < 256 && !shared) shared = form;
+                if (t < best) {
+                    best = t;
+                    lone = form;
+                }
             }
-            plan->program = program;
-            program->lone = program->shared = form;
-            program->reset_counts();
-            const double t = trial();
-            plan->program = nullptr;
-            // (other work held the device and some of these requests ran by steps: not this form's time)
-            const bool own_time = program->done >= kTrialTurns;
-            if (cfg.single_launch == 1 && !own_time) continue;
-            if (own_time && t <= steps_time && workgroups < 256 && !shared) shared = form;
-            if (t < best) {
-                best = t;
-                lone = form;
-            }
-        }
-        if (lone) {
             program->lone = lone;
-            program->shared = shared;
+            program->shared = lone ? shared : nullptr;
+            forms = FormChoice{true, false, lone ? lone->workgroups : 0, program->shared ? program->shared->workgroups : 0};
+            write_cache();
+        }
+        if (program->lone) {
             program->reset_counts();
             plan->program = program;
         }
     }
+    plan->forms = forms;
     return plan;
 }
 
@@ -3617,7 +3646,27 @@ int hipie_plan_get_config(const hipie_plan* p, const char* key, char* buf, size_
     });
 }
 
-/* stream layout: magic[8], format u32, step count u32, one i32 kernel variant per step, graph bytes u64 + the graph
+/* The configuration an exported plan keeps, in 16 bits behind the format number: HIP_THROUGHPUT_STREAMS (4 bits),
+ * HIP_SINGLE_LAUNCH (3: NO, AUTO, YES, 64, 128, 256), and of the single-launch form whether its sizes were measured (1) and
+ * which were chosen, lone and shared (2 each: none, 64, 128, 256).  0: a stream that keeps none of it. */
+static uint16_t pack_options(const hipie_plan& p) {
+    auto code = [](int workgroups) { return workgroups == 0 ? 0 : (workgroups == 64 ? 1 : (workgroups == 128 ? 2 : 3)); };
+    const int mode = p.config.single_launch <= 2 ? p.config.single_launch : 2 + code(p.config.single_launch);
+    return static_cast<uint16_t>(p.config.streams | mode << 4 | (p.forms.known ? 1 : 0) << 7 | code(p.forms.lone) << 8 | code(p.forms.shared) << 10);
+}
+// (a variable of the environment is the caller's own word about a key: it holds for imported plans too)
+static void unpack_options(uint16_t o, PlanConfig& cfg, FormChoice& forms) {
+    if (o == 0) return;
+    constexpr int sizes[4] = {0, 64, 128, 256};
+    const int streams = o & 15, mode = (o >> 4) & 7;
+    forms = FormChoice{((o >> 7) & 1) != 0, true, sizes[(o >> 8) & 3], sizes[(o >> 10) & 3]};
+    HIPIE_REQUIRE(streams >= 1 && streams <= 8 && mode <= 5 && (o >> 12) == 0 && forms.valid() && (forms.known || forms.lone == 0),
+                  HIPIE_NETWORK_NOT_READ, "hipie_plan_import: options %#x", static_cast<unsigned>(o));
+    if (!std::getenv("HIPIE_TUNE_STREAMS")) cfg.streams = streams;
+    if (!std::getenv("HIPIE_SINGLE_LAUNCH")) cfg.single_launch = mode <= 2 ? mode : sizes[mode - 2];
+}
+
+/* stream layout: magic[8], format u16, options u16 (above), step count u32, one i32 kernel variant per step, graph bytes u64 + the graph
  * description, the load-time checks' verdicts (count u64 + 6 u32 each: il, ih, d, r, levels - 1, exact; count u64 +
  * 4 u32 each: d, zh, zl, verified), the packed operands (count u64, then byte count u64 + bytes each), FNV-1a of
  * everything before it u64 */
@@ -3633,7 +3682,7 @@ int hipie_plan_export(const hipie_plan* p, void* buffer, size_t capacity, size_t
         HIPIE_REQUIRE(capacity >= *size, HIPIE_OUT_OF_BOUNDS, "hipie_plan_export: %zu bytes needed, %zu given", *size, capacity);
         uint8_t* b = static_cast<uint8_t*>(buffer);
         std::memcpy(b, kPlanMagic, 8);
-        const uint32_t fmt = kPlanFormat, ns = static_cast<uint32_t>(p->steps.size());
+        const uint32_t fmt = kPlanFormat | static_cast<uint32_t>(pack_options(*p)) << 16, ns = static_cast<uint32_t>(p->steps.size());
         std::memcpy(b + 8, &fmt, 4);
         std::memcpy(b + 12, &ns, 4);
         for (size_t i = 0; i < p->steps.size(); ++i) {
@@ -3680,7 +3729,8 @@ int hipie_plan_import(const void* blob, size_t size, int device, hipie_plan** ou
         uint32_t fmt, ns;
         std::memcpy(&fmt, b + 8, 4);
         std::memcpy(&ns, b + 12, 4);
-        HIPIE_REQUIRE(fmt == kPlanFormat, HIPIE_NETWORK_NOT_READ, "hipie_plan_import: stream format %u, this library reads %u", fmt, kPlanFormat);
+        HIPIE_REQUIRE((fmt & 0xffff) == kPlanFormat, HIPIE_NETWORK_NOT_READ, "hipie_plan_import: stream format %u, this library reads %u", fmt & 0xffff,
+                      kPlanFormat);
         uint64_t stored;
         std::memcpy(&stored, b + size - 8, 8);
         HIPIE_REQUIRE(stored == fnv1a(b, size - 8), HIPIE_NETWORK_NOT_READ, "hipie_plan_import: checksum mismatch (damaged stream)");
@@ -3744,7 +3794,10 @@ int hipie_plan_import(const void* blob, size_t size, int device, hipie_plan** ou
             r += n;
         }
         HIPIE_REQUIRE(r == end, HIPIE_NETWORK_NOT_READ, "hipie_plan_import: %zu bytes behind the packed operands", static_cast<size_t>(end - r));
-        *out = compile_plan(g.get(), device, &variants, PlanConfig::from_environment(), &prepared).release();
+        PlanConfig cfg = PlanConfig::from_environment();
+        FormChoice forms;
+        unpack_options(static_cast<uint16_t>(fmt >> 16), cfg, forms);
+        *out = compile_plan(g.get(), device, &variants, cfg, &prepared, forms).release();
     });
 }
 

@@ -518,9 +518,12 @@ int hipie_plan_get_config(const hipie_plan* plan, const char* key, char* buf, si
  * IInferencePlugin::ImportNetwork(std::istream&, config) (ie_iplugin_internal.hpp:213-222), as the
  * template plugin implements them (template_executable_network.cpp:179-201 writes the model,
  * :43-75 reads it back and compiles it again).  The stream holds the graph description with its
- * constants and the kernel variant chosen for every step, so an imported plan skips the timing runs
+ * constants and the kernel variant chosen for every step, the values of HIP_THROUGHPUT_STREAMS and HIP_SINGLE_LAUNCH and
+ * the sizes of the single-launch form that were chosen, so an imported plan skips the timing runs
  * of hipie_compile and runs the same kernels as the exported one; everything else (fusion, arena
- * layout, constant packing) is redone, through the same validation as a newly described graph.
+ * layout, constant packing) is redone, through the same validation as a newly described graph.  HIPIE_TUNE_STREAMS and
+ * HIPIE_SINGLE_LAUNCH, where the environment sets them, hold for imported plans too.  Streams written before these values
+ * were kept are read as well.
  * hipie_plan_export with buffer == NULL only reports the size.  A stream that is truncated, damaged
  * (checksum), of another format version or not a plan gives HIPIE_NETWORK_NOT_READ. */
 int hipie_plan_export(const hipie_plan* plan, void* buffer, size_t capacity, size_t* size);

@@ -68,6 +68,33 @@ def test_round_trip(net):
     assert back.export() == blob                       # the description survives unchanged, constants included
 
 
+def test_streams_and_single_launch_travel(monkeypatch):
+    g = builders.conv_block()[0]
+    for key in ("HIPIE_TUNE_STREAMS", "HIPIE_SINGLE_LAUNCH"):
+        monkeypatch.delenv(key, raising=False)
+    for streams in ("1", "3", "8"):
+        for mode in ("NO", "AUTO", "YES", "64", "128", "256"):
+            plan = g.compile(-1, config={"HIP_THROUGHPUT_STREAMS": streams, "HIP_SINGLE_LAUNCH": mode})
+            blob = plan.export()
+            back = Plan.load(blob, -1)
+            assert (back.config("HIP_THROUGHPUT_STREAMS"), back.config("HIP_SINGLE_LAUNCH")) == (streams, mode)
+            assert back.metric("OPTIMAL_NUMBER_OF_INFER_REQUESTS") == streams and back.export() == blob
+    monkeypatch.setenv("HIPIE_TUNE_STREAMS", "2")                # the importer's own word
+    monkeypatch.setenv("HIPIE_SINGLE_LAUNCH", "0")
+    back = Plan.load(blob, -1)
+    assert (back.config("HIP_THROUGHPUT_STREAMS"), back.config("HIP_SINGLE_LAUNCH")) == ("2", "NO")
+    monkeypatch.delenv("HIPIE_TUNE_STREAMS")
+    monkeypatch.delenv("HIPIE_SINGLE_LAUNCH")
+    # a stream without them is one that was written before they were kept
+    old = Plan.load(_reseal(blob[:10] + b"\0\0" + blob[12:-8]), -1)
+    assert (old.config("HIP_THROUGHPUT_STREAMS"), old.config("HIP_SINGLE_LAUNCH")) == ("3", "AUTO")
+    # streams 0 or 9, a mode there is none of, a shared form beside no lone one, sizes that were not measured, a stray bit
+    for options in (0x10, 0x19, 0x61, 0x71, 0x491, 0x111, 0x1011, 0x8011):
+        with pytest.raises(HipieError) as e:
+            Plan.load(_reseal(blob[:10] + struct.pack("<H", options) + blob[12:-8]), -1)
+        assert e.value.status == -12, hex(options)
+
+
 def test_refused_streams():
     blob = builders.conv_block()[0].compile(-1).export()
     cases = {

@@ -9,6 +9,7 @@ import torch
 
 from dldt_amd import HipieError, builders
 from dldt_amd._lib import check, lib
+from dldt_amd.graph import Plan
 
 pytestmark = pytest.mark.gpu
 
@@ -264,6 +265,39 @@ def test_requests_of_several_threads(mode):
         t.join()
     assert not failed
     assert all(p.metric("SINGLE_LAUNCH_COUNTS") != "0 0" for p in plans)
+
+
+def _forms(plan):
+    return plan.metric("SINGLE_LAUNCH_WORKGROUPS"), plan.metric("SINGLE_LAUNCH_SHARED_WORKGROUPS")
+
+
+@pytest.mark.parametrize("config", [{"HIP_SINGLE_LAUNCH": "AUTO"}, {"HIP_SINGLE_LAUNCH": "YES", "HIP_TUNE": "NO"},
+                                    {"HIP_SINGLE_LAUNCH": "128", "HIP_TUNE": "NO"}, {"HIP_TUNE": "NO"}])
+def test_an_exported_plan_keeps_its_form(config):
+    g = GRAPHS["resnet_1"]()
+    plan = g.compile(0, config=dict(config, HIP_THROUGHPUT_STREAMS="1"))
+    back = Plan.load(plan.export())
+    assert _forms(back) == _forms(plan) and back.config("HIP_THROUGHPUT_STREAMS") == "1"
+    assert back.export() == plan.export()
+    for x, y in zip(_infer(plan.create_request(), 0), _infer(back.create_request(), 0)):
+        assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
+
+
+def test_the_tuning_file_keeps_the_form(tmp_path):
+    g = GRAPHS["resnet_1"]()
+    path = tmp_path / "choices"
+    config = {"HIP_THROUGHPUT_STREAMS": "1", "HIP_TUNE_FILE": str(path)}
+    first = _forms(g.compile(0, config=config))
+    text = path.read_text()
+    assert text.endswith("-1 %s\n-2 %s\n" % first)
+    steps = text[:text.index("-1 ")]
+    for lone, shared in ((64, 64), (256, 128), (128, 0), (0, 0)):
+        path.write_text(steps + "-1 %d\n-2 %d\n" % (lone, shared))
+        assert _forms(g.compile(0, config=config)) == (str(lone), str(shared))       # taken as it is, not measured
+    for damaged in ("", "-1 64\n", "-1 32\n-2 0\n", "-1 0\n-2 64\n"):
+        path.write_text(steps + damaged)
+        g.compile(0, config=config)                                                  # measured, and written again
+        assert path.read_text().startswith(steps + "-1 ") and path.read_text().count("\n") == text.count("\n")
 
 
 def test_more_requests_than_a_plan_has_slots():
