@@ -442,9 +442,10 @@ __device__ __forceinline__ void finish(ConstConv& c, Buffer out, Buffer res, con
 }
 
 // A step's K offsets into LDS.  Every lane takes part in every round (those behind the end repeat the last entry): no lane
-// is masked off here.  The compiler's live-range splitting may put the copy of a register that merely lives through a masked
-// region in front of the instruction that ends the mask, which leaves the other lanes' values behind - seen with the
-// lane-derived addresses of a later attention step around a divergent form of this loop.
+// is masked off here, in the loop that every convolution step begins with.  (An earlier compilation with a divergent form of
+// it had the copy of a register that merely lives through the masked region in front of the instruction that ends the mask,
+// which left the other lanes' values behind in a later attention step.  The other loops of this kernel do mask lanes off;
+// tests/test_program_cpu.py reads the assembly of the whole kernel for such a copy.)
 __device__ __forceinline__ void stage_offsets(lds_i32 to, const int32_t* from, int n, int tid) {
     for (int base = 0; base < n; base += kProgramThreads) {
         const int i = min(base + tid, n - 1);
