@@ -57,7 +57,8 @@ __device__ __forceinline__ uint32_t prob_levels4(const AttentionArgs& a, float p
 constexpr int kPlainSoftmax = 384;
 
 // e / sum rounded once, from inv = 1 / sum rounded once: quotient, exact residual, correction.  Equal to the IEEE
-// quotient for e in [2^-60, 1] and sum in [1, 1024) (8 x 10^9 pairs compared); below, the level is that of zero.
+// quotient for e in [2^-60, 1] and sum in [1, 1024): tests/test_quotient_cpu.py derives which pairs of significands could round
+// the other way and compares all of them.  Below that range of e the level is that of zero.
 __device__ __forceinline__ float quotient(float e, float sum, float inv) {
     const float q = e * inv;
     return fmaf(fmaf(-q, sum, e), inv, q);

@@ -534,7 +534,10 @@ int hipie_plan_io_desc(const hipie_plan* plan, int is_output, int index, char* n
                        int* dtype, int64_t* dims /* [8]: ranks up to 8 */, int* rank);
 int64_t hipie_plan_arena_bytes(const hipie_plan* plan);
 /* executed (fused) steps, in order: the exec-graph / perf-counter view
- * (exec_graph_info.hpp:34-76, ie_common.h InferenceEngineProfileInfo) */
+ * (exec_graph_info.hpp:34-76, ie_common.h InferenceEngineProfileInfo).  The view is of an inference by steps: what
+ * hipie_request_enqueue and requests with counters always run.  A plan with a single-launch form (the metric
+ * SINGLE_LAUNCH_WORKGROUPS) computes the same steps in the same order inside one kernel, with tiles of its own: there the
+ * attributes "kernels" and "primitiveType" and the counters say nothing about how long a step takes. */
 int hipie_plan_num_steps(const hipie_plan* plan);
 int hipie_plan_step_info(const hipie_plan* plan, int index, char* name, size_t name_len, char* type,
                          size_t type_len, int64_t* macs, int64_t* bytes);
@@ -585,7 +588,7 @@ int hipie_request_cancel(hipie_request* request);
 /* enqueue the kernels only, on the request's stream, without copies or synchronisation */
 int hipie_request_enqueue(hipie_request* request, const void* const* inputs, void* const* outputs);
 int hipie_request_stream(hipie_request* request, void** stream);
-/* milliseconds of step `index` in the last inference (GetPerformanceCounts) */
+/* milliseconds of step `index` in the last inference (GetPerformanceCounts); a request with counters runs by steps */
 int hipie_request_perf(hipie_request* request, int index, float* ms);
 /* the arena tensor holding the value of graph node `node_id` (inspection, parity tests) */
 int hipie_request_tensor(const hipie_request* request, int node_id, hipie_tensor* tensor);

@@ -300,6 +300,16 @@ def test_the_tuning_file_keeps_the_form(tmp_path):
         assert path.read_text().startswith(steps + "-1 ") and path.read_text().count("\n") == text.count("\n")
 
 
+def test_a_request_with_counters_runs_by_steps():
+    g = GRAPHS["resnet_1"]()
+    plan = _compile(g, "64")
+    timed = plan.create_request(perf_count=True)
+    want = _infer(plan.create_request(), 0)[0]
+    assert np.array_equal(_infer(timed, 0)[0].view(np.uint8), want.view(np.uint8))
+    assert plan.metric("SINGLE_LAUNCH_COUNTS") == "1 0"
+    assert all(st["ms"] > 0 for st in timed.perf())
+
+
 def test_more_requests_than_a_plan_has_slots():
     g = GRAPHS["block_1x3x7"]()
     plan = _compile(g, "64")
