@@ -1296,10 +1296,15 @@ __global__ void clear_words(uint32_t* p, int n) {
     for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
 }
 
-// Tile shape of a convolution step, by the clocks its busiest compute unit should take (measured on single steps: a round
-// trip behind the barrier is about 1500 clocks; a load of 1 KB occupies a unit's path for 20; a matrix instruction its pipe
-// for 16; the exact f32 chain is 12 vector instructions per value, one every 8 clocks for a wave that is alone on its SIMD,
-// one every 4 when another fills the gaps; meeting in LDS costs 500).  Rounds are tiles a wave takes one after another.
+// Tile shape of a convolution step, by the clocks its busiest compute unit takes.  The constants are fitted, not derived: to
+// the time of whole networks with one class of layers at a time in each of the 24 shapes (188 classes of ResNet-50,
+// MobileNetV2, encoders and the convolution block, at 64, 128 and 256 workgroups), so that the choice loses as little as
+// possible against the best shape of every class.  Summed over a network's classes that is 0.1 - 6 % of its time (MobileNetV2,
+// whose 20 classes hardly tell the shapes apart from the runs' scatter of a microsecond, at 256 workgroups 16 %), where the
+// constants before lost 1 - 18 %: ResNet-50 at batch 1 took 290 us with those and 277 with these.
+// What the terms stand for: a load of 1 KB on a unit's path, a matrix instruction, a round trip to memory per filled ring, the
+// f32 chain per value, a store instruction, the partial sums of the waves that share a K in LDS.  Rounds are tiles a wave takes
+// one after another.
 struct TileChoice { int a, b, ks; };
 TileChoice choose_tile(int workgroups, int oc, int64_t pixels, int nk, int nk2, bool gelu) {
     static constexpr int kShapes[6][2] = {{4, 4}, {4, 2}, {2, 4}, {2, 2}, {2, 1}, {1, 4}};
@@ -1315,13 +1320,14 @@ TileChoice choose_tile(int workgroups, int oc, int64_t pixels, int nk, int nk2, 
             const double waves = std::min<double>(8.0, static_cast<double>(per_wg) * ks / static_cast<double>(rounds));   // of a workgroup, busy
             auto loop = [&](int steps) {
                 const double n = static_cast<double>(ceil_div(steps, ks));
-                const double rate = std::max(waves * (a + b) * 20.0, std::max(1.0, waves / 4.0) * a * b * 16.0 + 30.0);
-                return std::max(n * rate, std::ceil(n / depth) * 1500.0) + 300.0;
+                const double rate = std::max(waves * (a + b) * 13.0, std::max(1.0, waves / 4.0) * a * b * 19.0 + 7.0);
+                return std::max(n * rate, std::ceil(n / depth) * 600.0) + 1485.0;
             };
             const double columns = std::ceil(static_cast<double>(b) / ks), writers = waves / ks * std::min(ks, b);
-            const double chain = (gelu ? 44.0 : 12.0) * 4 * a + 60.0;
-            const double epi = columns * chain * std::max(8.0, writers);          // writers / 4 waves per SIMD, 4 clocks each
-            const double t = static_cast<double>(rounds) * (loop(nk) + (nk2 ? loop(nk2) : 0.0) + epi + (ks > 1 ? 500.0 : 100.0) + 400.0);
+            const double chain = (gelu ? 20.0 : 2.9) * 4 * a + 90.0;
+            const double epi = columns * (chain * std::max(8.0, writers) + 4 * 44.0 * writers);
+            const double meet = ks > 1 ? 195.0 + 112.0 * ks * a * columns : 0.0;
+            const double t = static_cast<double>(rounds) * (loop(nk) + (nk2 ? loop(nk2) : 0.0) + epi + meet + 1240.0);
             if (t < best_t) {
                 best_t = t;
                 best = {a, b, ks};

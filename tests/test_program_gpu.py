@@ -20,8 +20,11 @@ GRAPHS = {
     "block_3x256x16": lambda: builders.conv_block(n=3, c=256, hw=16, oc=130)[0],
     "block_3x64x14": lambda: builders.conv_block(n=3, c=64, hw=14, oc=512)[0],
     "block_7x64x32": lambda: builders.conv_block(n=7, c=64, hw=32, oc=130)[0],
+    "block_2x256x14": lambda: builders.conv_block(n=2, c=256, hw=14, oc=144)[0],
+    "block_7x128x14": lambda: builders.conv_block(n=7, c=128, hw=14, oc=72)[0],
     "resnet_1": lambda: builders.resnet50(batch=1, res=64, width=16, classes=10, seed=7)[0],
     "resnet_3_u8": lambda: builders.resnet50(batch=3, res=96, u8_input=True)[0],
+    "resnet_7_u8": lambda: builders.resnet50(batch=7, res=96, u8_input=True)[0],
     "mobilenet_2": lambda: builders.mobilenet_v2(batch=2, res=96)[0],
     "encoder_1x32": lambda: builders.bert_encoder(layers=1, batch=1, seq=32, vocab=100, mask=True)[0],
     "encoder_3x96": lambda: builders.bert_encoder(layers=1, batch=3, seq=96, vocab=0, mask=False)[0],
@@ -70,7 +73,8 @@ def test_single_launch_equals_steps(name):
 
 
 # 256 workgroups meet through the XCDs, the others at one counter.  Together these choose every tile instance of the kernel:
-# 4 x 2 in the blocks of 3x64x14 (64 workgroups) and 7x64x32 (256), the others in the networks at every size
+# 1 x 4 in the blocks of 2x256x14 (64 workgroups) and 7x128x14 (128), 2 x 4 in resnet_7_u8 (64, as the pair with a projection
+# shortcut too), 2 x 1, 2 x 2, 4 x 2, 4 x 4 and the 2 x 2 pair in the networks
 @pytest.mark.parametrize("workgroups", [64, 128, 256])
 @pytest.mark.parametrize("name", sorted(GRAPHS))
 def test_every_size_runs_and_equals_steps(name, workgroups):
