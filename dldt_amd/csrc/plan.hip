@@ -3624,12 +3624,13 @@ int hipie_plan_get_metric(const hipie_plan* p, const char* name, char* buf, size
         std::string v;
         if (k == "SUPPORTED_METRICS")
             v = "NETWORK_NAME SUPPORTED_METRICS SUPPORTED_CONFIG_KEYS OPTIMAL_NUMBER_OF_INFER_REQUESTS SINGLE_LAUNCH_WORKGROUPS "
-                "SINGLE_LAUNCH_SHARED_WORKGROUPS SINGLE_LAUNCH_COUNTS SINGLE_LAUNCH_REFUSED";
+                "SINGLE_LAUNCH_SHARED_WORKGROUPS SINGLE_LAUNCH_COUNTS SINGLE_LAUNCH_REFUSED SINGLE_LAUNCH_BYTES";
         else if (k == "SUPPORTED_CONFIG_KEYS") v = kConfigKeys;
         else if (k == "NETWORK_NAME") v = p->config.network_name;
         else if (k == "OPTIMAL_NUMBER_OF_INFER_REQUESTS") v = std::to_string(p->config.streams);
         else if (k == "SINGLE_LAUNCH_WORKGROUPS") v = std::to_string(p->program ? p->program->lone->workgroups : 0);
         else if (k == "SINGLE_LAUNCH_SHARED_WORKGROUPS") v = std::to_string(p->program && p->program->shared ? p->program->shared->workgroups : 0);
+        else if (k == "SINGLE_LAUNCH_BYTES") v = std::to_string(p->program ? p->program->device_bytes() : size_t(0));
         else if (k == "SINGLE_LAUNCH_COUNTS") v = p->program ? p->program->counts() : "0 0";
         else if (k == "SINGLE_LAUNCH_REFUSED") v = p->single_launch_refused;
         else fail(HIPIE_NOT_FOUND, "metric '%s' is not supported", name);

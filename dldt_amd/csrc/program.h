@@ -3,9 +3,9 @@
 // What this is for: a request that somebody waits for.  As separate launches a batch-1 ResNet-50 is 54 dependent kernels
 // at about 9 us each: 2.4 us of launch, then a cold start (arguments, descriptors, tables, operands from the memory-side
 // cache - an XCD's L2 is written back and invalidated between kernels) in front of 1 - 2 us of work.  Here the workgroups
-// stay, and a step ends in a barrier among them: with the stores in front of it and the loads behind it 2.3 us for 64
-// workgroups, 2.9 for 128, 3.2 for 256 - and the cold start disappears behind it, because a workgroup that has arrived
-// prepares its next tile (descriptor, offsets, weights, constants) before it waits.
+// stay, and a step ends in a barrier among them: a step without work takes 2.2 us with 64 workgroups, 2.9 with 128 and 3.0
+// with 256 - and the cold start disappears behind it, because a workgroup that has arrived prepares its next tile (descriptor,
+// offsets, weights, constants) before it waits.
 //
 // Coherence: the eight XCDs' L2 caches are not coherent with each other.  Every result is stored write-through with device
 // scope (sc1), is awaited (s_waitcnt vmcnt(0)) in front of the barrier, and is loaded with device scope behind it; fences,
@@ -15,15 +15,10 @@
 // Termination: a barrier needs every workgroup resident.  The roll call in front of the first step has a deadline: if the
 // launch is not complete in time (other work holds the compute units), it is cancelled by compare-and-swap before it has
 // written anything, the kernel drains, and the host runs the inference step by step, as it does with a growing number of the
-// requests behind it (Program::count).  Later waits are bounded as well (all
-// workgroups are resident by then, so they end; a bound that is hit ends the kernel and the host falls back the same way).
-// So the outputs are there when the host has waited, not before: the form is for inferences whose outputs nothing on the
-// device reads earlier (plan.hip, start_request).
+// requests behind it (Program::count).  Later waits are bounded as well (all workgroups are resident by then, so they end; a
+// bound that is hit ends the kernel and the host falls back the same way).  So the outputs are there when the host has waited,
+// not before: the form is for inferences whose outputs nothing on the device reads earlier (plan.hip, start_request).
 // Programs in flight together never ask for more compute units than there are (Program::choose).
-//
-// (Measured beside it: one XCD per batch element, whose barrier costs 0.95 us and whose results stay in its own L2.  Thirty-two
-// compute units on one L2 then do all of an image's work: 20 - 30 bytes a clock and unit of operands and the whole f32 chain
-// of 11 M values; ResNet-50 took 415 us that way and the encoder 831.)
 #pragma once
 #include <array>
 #include <memory>
@@ -145,7 +140,9 @@ struct ProgBuilder {
     bool copy(const void* in, void* out, int64_t bytes);
 };
 
-// The step list of one size on the device, with its own packing of the weights (the tile shapes depend on the size)
+// The step list of one size on the device, with its own packing of the dense layers' weights (the tile shapes depend on the
+// size) and four words per output pixel of each: a second copy of the weights for the lone form, a third one where the shared
+// form is another, and at load, while the sizes are measured, one more.
 struct ProgramForm {
     int workgroups = 0, n_steps = 0;
     DeviceBuffer steps;
@@ -176,6 +173,7 @@ struct Program {
     void count(bool ran);
     void reset_counts();
     std::string counts();                    // "done cancelled"
+    size_t device_bytes() const;             // of its forms
 };
 std::shared_ptr<Program> make_program(int device);
 // A request is started / has been waited for, by whatever form; the former gives how many were in flight together lately

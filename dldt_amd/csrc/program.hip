@@ -46,7 +46,7 @@ struct ProgArgs {
 
 // control words: the root counter, the roll call's verdict, a counter per XCD (128 bytes apart)
 constexpr int kCtlRoot = 0, kCtlState = 32, kCtlXcd = 64;
-constexpr int kFlat = 128;                   // up to here every workgroup counts at the root (256 at one address: 4.8 us, by way of the XCDs 3.2)
+constexpr int kFlat = 128;                   // up to here every workgroup counts at the root (256 at one address: 4.7 us a step without work, by way of the XCDs 3.0)
 
 struct Ctx {
     int rank, n_wg;                          // neighbouring ranks share an XCD
@@ -1683,6 +1683,16 @@ void Program::reset_counts() {
 std::string Program::counts() {
     std::lock_guard<std::mutex> g(lock);
     return std::to_string(done) + " " + std::to_string(cancelled);
+}
+
+size_t Program::device_bytes() const {
+    size_t n = 0;
+    for (const ProgramForm* f : {lone.get(), shared == lone ? nullptr : shared.get()})
+        if (f) {
+            n += f->steps.bytes;
+            for (const auto& b : f->owned) n += b.bytes;
+        }
+    return n;
 }
 
 std::shared_ptr<ProgramForm> make_program_form(ProgBuilder&& b) {

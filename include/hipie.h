@@ -510,7 +510,9 @@ int hipie_get_metric(int device, const char* name, char* buf, size_t buf_len);
  * Beside the reference's metrics, of the plan's single-launch form: SINGLE_LAUNCH_WORKGROUPS of a lone request (0: the plan
  * runs by steps) and SINGLE_LAUNCH_SHARED_WORKGROUPS of one beside others (0: those run by steps),
  * SINGLE_LAUNCH_COUNTS ("completed given-up": requests that ran as one launch, launches that did not come together and ran
- * again by steps), SINGLE_LAUNCH_REFUSED (the step that has no such form where one was wanted, else empty) */
+ * again by steps), SINGLE_LAUNCH_REFUSED (the step that has no such form where one was wanted, else empty),
+ * SINGLE_LAUNCH_BYTES (device memory of the form: the weights of the dense layers once more, and a third time where the
+ * shared form is not the lone one; while hipie_compile measures the sizes there is one copy more) */
 int hipie_plan_get_metric(const hipie_plan* plan, const char* name, char* buf, size_t buf_len);
 int hipie_plan_get_config(const hipie_plan* plan, const char* key, char* buf, size_t buf_len);
 

@@ -195,7 +195,7 @@ def test_single_launch_key_and_metrics():
             g.compile(-1, config={"HIP_SINGLE_LAUNCH": value})
         assert e.value.status == -4
     plan = g.compile(-1, config={"HIP_SINGLE_LAUNCH": "64"})                   # a dry run has no launches of any form
-    assert [plan.metric("SINGLE_LAUNCH_" + k) for k in ("WORKGROUPS", "COUNTS", "REFUSED")] == ["0", "0 0", ""]
+    assert [plan.metric("SINGLE_LAUNCH_" + k) for k in ("WORKGROUPS", "SHARED_WORKGROUPS", "COUNTS", "REFUSED", "BYTES")] == ["0", "0", "0 0", "", "0"]
     assert "SINGLE_LAUNCH_WORKGROUPS" in plan.metric("SUPPORTED_METRICS").split()
 
 

@@ -304,6 +304,18 @@ def test_the_tuning_file_keeps_the_form(tmp_path):
         assert path.read_text().startswith(steps + "-1 ") and path.read_text().count("\n") == text.count("\n")
 
 
+def test_the_memory_of_the_form_is_reported():
+    """ResNet-50: 25.5 million weights, and four words per output pixel of a layer; one copy when both forms are the same"""
+    g = builders.resnet50(batch=1, res=64)[0]
+    assert _compile(g, "NO").metric("SINGLE_LAUNCH_BYTES") == "0"
+    one = int(_compile(g, "64").metric("SINGLE_LAUNCH_BYTES"))
+    assert 25.4e6 < one < 29e6
+    free = torch.cuda.mem_get_info()[0]
+    plan = _compile(g, "64")
+    assert free - torch.cuda.mem_get_info()[0] > one
+    del plan
+
+
 def test_a_request_with_counters_runs_by_steps():
     g = GRAPHS["resnet_1"]()
     plan = _compile(g, "64")
