@@ -1167,6 +1167,9 @@ __device__ __forceinline__ void attention_units(const ProgAttention& s, const Ct
 }
 
 // ---- the program ------------------------------------------------------------------------------------------------------------
+// 246 vector registers, which the 4 x 4 tiles ask for, and none spilled to memory; 230 scalar registers of the many step kinds
+// are kept in lanes of a vector register.  A new step kind adds to these for all steps: it belongs into a kernel of its own
+// where it needs more than they have.
 __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgArgs g) {
     extern __shared__ __attribute__((aligned(16))) int8_t smem[];
     lds_ptr lds = (lds_ptr)smem;
@@ -1598,7 +1601,8 @@ bool ProgBuilder::attention(const hipie_attention* att, const void* const (&qkv)
     s.a.mask_inner = 0;
     s.a.mask_outer = proto.S;
     // queries per workgroup: rounds x (staging, about 4 clocks a key + a wave's 20 instructions per score, two waves to a
-    // SIMD from five on)
+    // SIMD from five on).  Against the best of 1 .. 8 waves the choice costs an encoder of two layers 0 - 4 % of its time
+    // (1 to 4 sequences of 32 to 512 keys, 64 and 256 workgroups).
     const int qt = proto.S / 32;
     const int64_t elements = static_cast<int64_t>(batch_outer) * batch;
     double best = 1e30;
