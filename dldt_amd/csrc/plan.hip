@@ -3459,6 +3459,7 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
             const double steps_time = trial();
             double best = cfg.single_launch == 2 ? 1e30 : steps_time;
             std::shared_ptr<ProgramForm> lone, shared;
+            bool all_measured = true;
             for (int workgroups : {64, 128, 256}) {
                 const auto form = build(workgroups);
                 if (!form) break;
@@ -3469,6 +3470,7 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
                 plan->program = nullptr;
                 // (other work held the device and some of these requests ran by steps: not this form's time)
                 const bool own_time = program->done >= kTrialTurns;
+                all_measured = all_measured && own_time;
                 if (cfg.single_launch == 1 && !own_time) continue;
                 if (own_time && t <= steps_time && workgroups < 256 && !shared) shared = form;
                 if (t < best) {
@@ -3478,8 +3480,10 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
             }
             program->lone = lone;
             program->shared = lone ? shared : nullptr;
-            forms = FormChoice{true, false, lone ? lone->workgroups : 0, program->shared ? program->shared->workgroups : 0};
-            write_cache();
+            if (all_measured) {                  // (a choice made beside other work is not one to keep in files)
+                forms = FormChoice{true, false, lone ? lone->workgroups : 0, program->shared ? program->shared->workgroups : 0};
+                write_cache();
+            }
         }
         if (program->lone) {
             program->reset_counts();

@@ -188,6 +188,18 @@ def test_cancelled_launch_of_host_buffers_is_made_up_for_in_the_wait(monkeypatch
     assert np.array_equal(hout[0].array.view(np.uint8), want.view(np.uint8))
 
 
+@pytest.mark.parametrize("mode", ["AUTO", "YES"])
+def test_a_choice_made_on_a_busy_device_is_not_kept(monkeypatch, tmp_path, mode):
+    """launches that are given up while the sizes are measured: AUTO runs by steps, and neither file nor stream says why"""
+    g = GRAPHS["block_2x17x9"]()
+    path = tmp_path / "choices"
+    monkeypatch.setenv("HIPIE_ROLL_CALL_TICKS", "0")
+    plan = g.compile(0, config={"HIP_THROUGHPUT_STREAMS": "1", "HIP_SINGLE_LAUNCH": mode, "HIP_TUNE_FILE": str(path)})
+    assert (plan.metric("SINGLE_LAUNCH_WORKGROUPS") == "0") == (mode == "AUTO")
+    assert plan.metric("SINGLE_LAUNCH_SHARED_WORKGROUPS") == "0"
+    assert "\n-" not in path.read_text() and not plan.export()[10] & 0x80
+
+
 def _host_request(plan, feed):
     """(request, its host blobs) with the values of the device tensors `feed` in the inputs"""
     req = plan.create_request()
