@@ -3075,6 +3075,10 @@ std::shared_ptr<ProgramForm> build_program(const hipie_plan& p, int workgroups, 
             refused = s->name;
             return nullptr;
         }
+    if (b.map_kinds && b.rows_kinds) {       // (a kernel with the steps of both has no registers left for either's)
+        refused = "feature maps and rows";
+        return nullptr;
+    }
     return make_program_form(std::move(b));
 }
 

@@ -3,9 +3,9 @@
 // What this is for: a request that somebody waits for.  As separate launches a batch-1 ResNet-50 is 54 dependent kernels
 // at about 9 us each: 2.4 us of launch, then a cold start (arguments, descriptors, tables, operands from the memory-side
 // cache - an XCD's L2 is written back and invalidated between kernels) in front of 1 - 2 us of work.  Here the workgroups
-// stay, and a step ends in a barrier among them: a step without work takes 2.2 us with 64 workgroups, 2.9 with 128 and 3.0
-// with 256 - and the cold start disappears behind it, because a workgroup that has arrived prepares its next tile (descriptor,
-// offsets, weights, constants) before it waits.
+// stay, and a step ends in a barrier among them (Ctx::arrive; with the wait for a store in front of it 1.3 us with 64
+// workgroups, 1.5 with 128, 1.6 with 256).  The cold start disappears behind it, because a workgroup that has arrived prepares
+// its next tile (offsets, weights, constants) before it waits, and the descriptor of the next step comes beside the stores.
 //
 // Coherence: the eight XCDs' L2 caches are not coherent with each other.  Every result is stored write-through with device
 // scope (sc1), is awaited (s_waitcnt vmcnt(0)) in front of the barrier, and is loaded with device scope behind it; fences,
@@ -57,9 +57,11 @@ struct ProgConv {
     int32_t nk, nk2, OCp, M;
     int32_t out_limit, res_limit;     // channels the tensors hold
     uint32_t flags;
-    float lm1, out_off, clamp_lo, clamp_hi;
+    float lm1;
+    uint32_t off_bytes;                // the level offset in every byte
+    float clamp_lo, clamp_hi;
     // depthwise
-    int32_t stride, c4, quads, OH, OW, items;
+    int32_t stride, group, c4, quads, OH, OW, items;
     int32_t in_sn, in_sh, in_sw, row_sh, out_sn, out_sh, out_sw, res_sn, res_sh, res_sw;
     float inv_c4, inv_quads, inv_OH;
 };
@@ -114,6 +116,7 @@ struct ProgBuilder {
     int workgroups = 256;
     std::vector<std::array<int32_t, kProgramStepWords>> steps;
     std::vector<DeviceBuffer> owned;      // repacked weights, tables
+    bool map_kinds = false, rows_kinds = false;      // steps of a network over feature maps, of an encoder: a kernel for each
     ProgPtr keep(const void* host, size_t bytes);                              // a table of the program's own
     ProgPtr gather(const std::vector<const void*>& rows, size_t pitch);
     static uint8_t* fake_arena() { return reinterpret_cast<uint8_t*>(uintptr_t(1) << 32); }
@@ -145,6 +148,7 @@ struct ProgBuilder {
 // form is another, and at load, while the sizes are measured, one more.
 struct ProgramForm {
     int workgroups = 0, n_steps = 0;
+    bool encoder = false;                    // which of the two kernels
     DeviceBuffer steps;
     std::vector<DeviceBuffer> owned;
 };

@@ -24,7 +24,8 @@ namespace {
 constexpr int kPartBytes = 128 * 1024;       // partial sums of eight waves x 16 fragments
 constexpr int kKoffBytes = 16 * 1024;        // K offsets of the step's convolutions
 constexpr int kMaxPieces = kKoffBytes / 4 / 2;
-constexpr int kLdsBytes = kPartBytes + kKoffBytes + 64;
+constexpr int kPlainAt = kPartBytes + kKoffBytes + 64;        // 16 i at entry i: the K offsets of a step whose K pieces lie one behind the other
+constexpr int kLdsBytes = kPlainAt + kMaxPieces * 4;
 // How long a launch waits for its last workgroup: 1 ms of the 100 MHz clock.  Alone it is complete in a few microseconds, behind
 // the kernels of another request in the time these take; what holds compute units longer (another process's launch that
 // waits for the same units) does not let go, and the steps need less than that beside it.
@@ -44,68 +45,116 @@ struct ProgArgs {
     uint32_t launch, roll_call_ticks;
 };
 
-// control words: the root counter, the roll call's verdict, a counter per XCD (128 bytes apart)
-constexpr int kCtlRoot = 0, kCtlState = 32, kCtlXcd = 64;
-constexpr int kFlat = 128;                   // up to here every workgroup counts at the root (256 at one address: 4.7 us a step without work, by way of the XCDs 3.0)
+// (addresses made from integers are told to be global memory: as generic pointers their loads would be FLAT, which the
+// compiler waits for on the LDS counter as well)
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __attribute__((address_space(1))) uint8_t* GlobalBytes;
+#else
+typedef uint8_t* GlobalBytes;
+#endif
+
+// control words: a counter per XCD, 128 bytes apart
+constexpr int kXcdWords = 32;
+constexpr uint32_t kGivenUp = 1u << 26;      // added to a counter that was not complete when the roll call's time was up (a launch counts far less)
 
 struct Ctx {
-    int rank, n_wg;                          // neighbouring ranks share an XCD
+    int rank, n_wg, wg_shift;                // neighbouring ranks share an XCD; n_wg = 1 << wg_shift
     int tid, lane, wave;
-    uint32_t *root, *sub;                    // counters; sub null: flat
-    uint32_t root_target, sub_target;        // the values of the barrier that comes next
+    const int32_t* steps;
+    uint32_t words;                          // lane i: word i of the descriptor of the step that is run or prepared
+    uint32_t bases;                          // lanes 2 b, 2 b + 1: where operands of base b are (ProgArgs::bases)
+    uint32_t *xcds, *own;                    // the eight counters, the one this workgroup counts at
+    uint32_t target;                         // what each of them holds when the barrier that comes next is complete
     uint32_t* report;
-    bool dead;
+    bool started, dead;                      // between the roll call and the first step's wait; after a wait that was given up
     lds_i32 flag;
 
-    // counts this workgroup (one lane); true when it completes the barrier
-    __device__ __forceinline__ bool count() {
-        if (sub) {
-            if (__hip_atomic_fetch_add(sub, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 != sub_target) return false;
-        }
-        return __hip_atomic_fetch_add(root, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == root_target;
-    }
-    __device__ __forceinline__ void next_targets() {
-        root_target += sub ? 8 : n_wg;
-        sub_target += n_wg / 8;
+    __device__ __forceinline__ uint32_t load_words(int step) const { return static_cast<uint32_t>(steps[step * kProgramStepWords + lane]); }
+    // an operand's address (of an absent one: the arena's, which nothing uses)
+    __device__ __forceinline__ uint8_t* place(ProgRef r) const {
+        const int b = 2 * max(r.base, 0);
+        const uint64_t base = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(bases), b)) |
+                              (static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(bases), b + 1))) << 32);
+        return (uint8_t*)(GlobalBytes)(base + ((static_cast<uint64_t>(r.hi) << 32) | r.lo));
     }
     // The barrier between two steps comes in halves: every workgroup arrives with its stores acknowledged, then prepares the
     // next step - descriptor, tile, weights, constants: nothing the step before it wrote - and only then waits.
-    __device__ __forceinline__ void arrive() {
+    // A workgroup counts at its XCD's counter and reads all eight: 32 additions to one address is what 256 workgroups take
+    // (an address serves one every 10 ns: at a single one they took 4.1 us, at four a XCD the readers' traffic cost more than
+    // it gave), and no second addition stands between the last arrival and its readers.  An empty barrier with the wait for a
+    // store in front, us with 64 / 128 / 256 workgroups: 1.3 / 1.5 / 1.6; by way of a root counter that the last of an XCD
+    // adds to 2.1 / 2.3 / 2.6, all at one counter 1.5 / 2.3 / 4.1, a flag per workgroup that everybody reads 1.4 / 1.6 / 1.8.
+    // (One way between two workgroups, store to sight, takes 0.5 - 0.6 us, the wait for a store 0.36.)
+    __device__ __forceinline__ void arrive(int next_step) {
+        words = load_words(next_step);
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
-        next_targets();
-        if (tid == 0) (void)count();
+        target += n_wg / 8;
+        if (tid == 0) (void)__hip_atomic_fetch_add(own, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        dead = __builtin_amdgcn_readfirstlane(flag[0]) == 0;      // (of the wait before: its verdict is not waited for)
     }
     __device__ __forceinline__ void wait() {
-        if (tid == 0) {
-            int ok = 1;
-            if (static_cast<int32_t>(__hip_atomic_load(root, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - root_target) < 0) {
-                const uint64_t t0 = wall_clock64();
-                while (static_cast<int32_t>(__hip_atomic_load(root, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - root_target) < 0)
-                    if (wall_clock64() - t0 > kBarrierTicks) {
-                        ok = 0;
-                        break;
+        if (wave == 0 && !started) {
+            const uint32_t* c = xcds + kXcdWords * (lane & 7);
+            uint64_t t0 = 0;
+            for (uint32_t n = 1;; ++n) {
+                const uint32_t v = __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (__builtin_amdgcn_ballot_w64(static_cast<int32_t>(v - target) < 0) == 0) break;
+                if ((n & 255) != 0) continue;
+                if (t0 == 0) t0 = wall_clock64();
+                if (wall_clock64() - t0 > kBarrierTicks) {
+                    if (lane == 0) {
+                        __hip_atomic_store(report, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                        flag[0] = 0;
                     }
+                    break;
+                }
             }
-            if (!ok) __hip_atomic_store(report, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            flag[0] = ok;
         }
+        started = false;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        dead = __builtin_amdgcn_readfirstlane(flag[0]) == 0;
+    }
+    // Everybody is resident, or nobody starts.  A workgroup whose time is up adds kGivenUp to a counter that it has seen short
+    // and that has not moved since: from then on that counter never holds what completes the roll call.  So "all eight have
+    // been complete" and "one was given up" exclude each other, neither is ever taken back, and all workgroups find the same.
+    __device__ __forceinline__ bool roll_call(uint32_t ticks) {
+        if (wave == 0) {
+            uint32_t* c = xcds + kXcdWords * (lane & 7);
+            // (no time at all: given up before it can be complete)
+            if (lane == 0) (void)__hip_atomic_fetch_add(own, ticks == 0 && rank == 0 ? 1u + kGivenUp : 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint64_t t0 = wall_clock64();
+            bool all = false;
+            for (;;) {
+                const uint32_t v = __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const int32_t beyond = static_cast<int32_t>(v - target);
+                if (__builtin_amdgcn_ballot_w64(beyond >= static_cast<int32_t>(kGivenUp / 2)) != 0) break;
+                const uint64_t missing = __builtin_amdgcn_ballot_w64(beyond < 0);
+                all = missing == 0;
+                if (all) break;
+                if (wall_clock64() - t0 > ticks && lane == __builtin_ctzll(missing)) {
+                    uint32_t expect = v;
+                    (void)__hip_atomic_compare_exchange_strong(c, &expect, v + kGivenUp, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+            if (lane == 0) {
+                if (!all) __hip_atomic_store(report, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                flag[0] = all ? 1 : 0;
+            }
+        }
+        __syncthreads();
+        return flag[0] != 0;
     }
 };
 
-// A step's descriptor is read through the constant address space: scalar loads, at the place of use (a tile loop reads its
-// fields again from the scalar cache instead of keeping eighty of them in registers).
+// The steps that are not convolutions read their descriptor through the constant address space: scalar loads.
 #if defined(__HIP_DEVICE_COMPILE__)
 #define PROG_CONSTANT const __attribute__((address_space(4)))
 #else
 #define PROG_CONSTANT const
 #endif
 typedef PROG_CONSTANT int32_t* StepPtr;
-typedef PROG_CONSTANT ProgConv ConstConv;
 __device__ __forceinline__ StepPtr step_ptr(const int32_t* steps, int s) {
     return (StepPtr)(reinterpret_cast<uintptr_t>(steps) + static_cast<uintptr_t>(s) * (kProgramStepWords * 4));
 }
@@ -119,20 +168,6 @@ __device__ __forceinline__ T unpack(StepPtr p) {
     __builtin_memcpy(&t, w, sizeof(T));
     return t;
 }
-// the same descriptor as a pointer the compiler knows nothing about: fields read through it are read here, not kept from before
-__device__ __forceinline__ ConstConv* again(ConstConv* c) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" : "+s"(c));
-#endif
-    return c;
-}
-// (addresses made from integers are told to be global memory: as generic pointers their loads would be FLAT, which the
-// compiler waits for on the LDS counter as well)
-#if defined(__HIP_DEVICE_COMPILE__)
-typedef __attribute__((address_space(1))) uint8_t* GlobalBytes;
-#else
-typedef uint8_t* GlobalBytes;
-#endif
 // an operand's address: its base comes from the kernel's arguments by a scalar load
 __device__ __forceinline__ uint8_t* resolve(int32_t base, uint32_t lo, uint32_t hi) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -256,6 +291,26 @@ __device__ __forceinline__ void k_loop(Ring<A, B>& g, const KSource& s, const ui
         if (d == 0 || k + d * s.ks < s.nk) multiply(d);
 }
 
+// ---- a step's descriptor in a vector register: lane i holds word i (ProgConv has fewer than 64) -----------------------------
+// Scalar loads cost 90 ns each where they stand one behind the other, hits included, and a step's preparation was a chain of
+// fourteen of them; a word of this register costs an instruction.  It is loaded beside the wait for the step's stores.
+__device__ __forceinline__ uint32_t word_of(uint32_t words, int i) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(words), i)); }
+template <typename T>
+__device__ __forceinline__ T words_of(uint32_t words, int i) {
+    static_assert(sizeof(T) % 4 == 0, "words");
+    uint32_t w[sizeof(T) / 4];
+#pragma unroll
+    for (int k = 0; k < static_cast<int>(sizeof(T) / 4); ++k) w[k] = word_of(words, i + k);
+    T t;
+    __builtin_memcpy(&t, w, sizeof(T));
+    return t;
+}
+static_assert(sizeof(ProgConv) <= 64 * 4, "a lane per word");
+#define PROG_FIELD(words, f) words_of<decltype(ProgConv::f)>(words, static_cast<int>(offsetof(ProgConv, f) / 4))
+#define PROG_PLACE(x, f) (x).place(PROG_FIELD((x).words, f))
+#define PROG_TABLE_OF(T, words, f) table_at<T>(PROG_FIELD(words, f))
+template <typename T> __device__ __forceinline__ const T* table_at(ProgPtr p) { return PROG_TABLE(T, p); }
+
 template <int A>
 struct ChannelConstants {
     int32_t corr[A];
@@ -276,10 +331,8 @@ __device__ __forceinline__ void load_channels(const T* p, T (&v)[A]) {
 
 // The tables a step uses, one row of OCp words each, behind one another in this order (ProgBuilder::constants)
 template <int A>
-__device__ __forceinline__ void load_constants(ConstConv& c, int oc, ChannelConstants<A>& k) {
-    const uint32_t fl = c.flags;
-    const uint8_t* row = PROG_TABLE(uint8_t, c.constants) + oc * 4;
-    const int pitch = c.OCp * 4;
+__device__ __forceinline__ void load_constants(uint32_t fl, const uint8_t* table, int pitch, int oc, ChannelConstants<A>& k) {
+    const uint8_t* row = table + oc * 4;
     auto next = [&](auto& v) {
         typedef std::remove_reference_t<decltype(v[0])> T;
         load_channels<A>(reinterpret_cast<const T*>(row), v);
@@ -297,41 +350,61 @@ __device__ __forceinline__ void load_constants(ConstConv& c, int oc, ChannelCons
     }
 }
 
-// four pixels of the output: byte offsets in the output and residual tensors (kBeyond: not there), and their residual values
+// what the chain behind a sum needs besides the channels' constants: the step's, the same for all lanes
+struct StepConstants {
+    uint32_t flags;
+    Buffer out, res;
+    float lm1, clamp_lo, clamp_hi;
+    uint32_t off_bytes;                      // the level offset, four times
+    int out_limit, res_limit;
+};
+__device__ __forceinline__ StepConstants step_constants(const Ctx& x) {
+    StepConstants s;
+    s.flags = PROG_FIELD(x.words, flags);
+    s.out = make_buffer(PROG_PLACE(x, out));
+    s.res = make_buffer(PROG_PLACE(x, res));
+    s.lm1 = PROG_FIELD(x.words, lm1);
+    s.clamp_lo = PROG_FIELD(x.words, clamp_lo);
+    s.clamp_hi = PROG_FIELD(x.words, clamp_hi);
+    s.off_bytes = PROG_FIELD(x.words, off_bytes);
+    s.out_limit = PROG_FIELD(x.words, out_limit);
+    s.res_limit = PROG_FIELD(x.words, res_limit);
+    return s;
+}
+
+// up to four pixels of the output: byte offsets in the output and residual tensors (kBeyond: not there), and their residual values
 template <int A>
-struct PixelQuad {
+struct Pixels {
     uint32_t out[4], res[4];
     static constexpr int kRaw = A == 4 ? 1 : A;
     uint32_t raw[4][kRaw];                   // A bytes in raw[.][0], or A f32 values (A = 4: those are loaded where they are used)
 };
-template <int A>
-__device__ __forceinline__ void load_residual(ConstConv& c, Buffer res, int oc, PixelQuad<A>& q) {
-    const uint32_t fl = c.flags;
-    if (!(fl & CF_RES) || (fl & CF_RES_GEMM)) return;
-    const bool f32 = fl & CF_RES_F32;
-    const uint32_t o = oc < c.res_limit ? static_cast<uint32_t>(f32 ? 4 * oc : oc) : static_cast<uint32_t>(kBeyond);
+template <int A, int R>
+__device__ __forceinline__ void load_residual(const StepConstants& s, int oc, Pixels<A>& q) {
+    if (!(s.flags & CF_RES) || (s.flags & CF_RES_GEMM)) return;
+    const bool f32 = s.flags & CF_RES_F32;
+    const uint32_t o = oc < s.res_limit ? static_cast<uint32_t>(f32 ? 4 * oc : oc) : static_cast<uint32_t>(kBeyond);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
+    for (int r = 0; r < R; ++r) {
         if (f32) {
             if constexpr (A == 2) {
-                const v2i v = shared8(res, q.res[r] + o);
+                const v2i v = shared8(s.res, q.res[r] + o);
                 q.raw[r][0] = v.x; q.raw[r][1] = v.y;
-            } else if constexpr (A == 1) q.raw[r][0] = shared4(res, q.res[r] + o);
+            } else if constexpr (A == 1) q.raw[r][0] = shared4(s.res, q.res[r] + o);
         } else {
-            if constexpr (A == 4) q.raw[r][0] = shared4(res, q.res[r] + o);
-            else if constexpr (A == 2) q.raw[r][0] = shared2(res, q.res[r] + o);
-            else q.raw[r][0] = shared1(res, q.res[r] + o);
+            if constexpr (A == 4) q.raw[r][0] = shared4(s.res, q.res[r] + o);
+            else if constexpr (A == 2) q.raw[r][0] = shared2(s.res, q.res[r] + o);
+            else q.raw[r][0] = shared1(s.res, q.res[r] + o);
         }
     }
 }
 
-// the fused f32 chain (conv_epilogue.h) on A neighbouring channels of four pixels, and their store
-template <int A, bool PAIR = false>
-__device__ __forceinline__ void finish(ConstConv& c, Buffer out, Buffer res, const ChannelConstants<A>& k, const v4i (&sum)[A], const float (&rgemm)[A][4],
-                                       const PixelQuad<A>& q, int oc) {
+// the fused f32 chain (conv_epilogue.h) on A neighbouring channels of R pixels, and their store
+template <bool GELU, int A, int R, bool PAIR = false>
+__device__ __forceinline__ void finish(const StepConstants& c, const ChannelConstants<A>& k, const int32_t (&sum)[A][R], const float (&rgemm)[A][R], const Pixels<A>& q, int oc) {
     const uint32_t fl = c.flags;
-    float x[A][4];
-#define PROG_EACH for (int a = 0; a < A; ++a) for (int r = 0; r < 4; ++r)
+    float x[A][R];
+#define PROG_EACH for (int a = 0; a < A; ++a) for (int r = 0; r < R; ++r)
 #pragma unroll
     PROG_EACH x[a][r] = static_cast<float>(sum[a][r]);
     if (fl & CF_BIAS) {
@@ -343,7 +416,7 @@ __device__ __forceinline__ void finish(ConstConv& c, Buffer out, Buffer res, con
         PROG_EACH x[a][r] = x[a][r] * k.scale[a];
     }
     if (fl & CF_RES) {
-        float rv[A][4];
+        float rv[A][R];
         if constexpr (PAIR) {
 #pragma unroll
             PROG_EACH rv[a][r] = rgemm[a][r];
@@ -351,8 +424,8 @@ __device__ __forceinline__ void finish(ConstConv& c, Buffer out, Buffer res, con
             if constexpr (A == 4) {
                 const uint32_t o = oc < c.res_limit ? static_cast<uint32_t>(4 * oc) : static_cast<uint32_t>(kBeyond);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float4 v = shared16f(res, q.res[r] + o);
+                for (int r = 0; r < R; ++r) {
+                    const float4 v = shared16f(c.res, q.res[r] + o);
                     rv[0][r] = v.x; rv[1][r] = v.y; rv[2][r] = v.z; rv[3][r] = v.w;
                 }
             } else {
@@ -386,7 +459,7 @@ __device__ __forceinline__ void finish(ConstConv& c, Buffer out, Buffer res, con
             PROG_EACH x[a][r] = x[a][r] < c.clamp_lo ? c.clamp_lo : (x[a][r] > c.clamp_hi ? c.clamp_hi : x[a][r]);
         }
     }
-    if constexpr (A != 1)                    // (choose_tile)
+    if constexpr (GELU && A != 1)            // (choose_tile)
         if (fl & CF_GELU) {
 #pragma unroll
             PROG_EACH x[a][r] = gelu_one(x[a][r]);
@@ -394,10 +467,10 @@ __device__ __forceinline__ void finish(ConstConv& c, Buffer out, Buffer res, con
     if (!(fl & CF_OUT_FQ)) {
         const uint32_t o = oc < c.out_limit ? static_cast<uint32_t>(4 * oc) : static_cast<uint32_t>(kBeyond);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if constexpr (A == 4) publish16f(out, q.out[r] + o, make_float4(x[0][r], x[1][r], x[2][r], x[3][r]));
-            else if constexpr (A == 2) publish8(out, q.out[r] + o, v2i{__float_as_int(x[0][r]), __float_as_int(x[1][r])});
-            else publish4(out, q.out[r] + o, __float_as_uint(x[0][r]));
+        for (int r = 0; r < R; ++r) {
+            if constexpr (A == 4) publish16f(c.out, q.out[r] + o, make_float4(x[0][r], x[1][r], x[2][r], x[3][r]));
+            else if constexpr (A == 2) publish8(c.out, q.out[r] + o, v2i{__float_as_int(x[0][r]), __float_as_int(x[1][r])});
+            else publish4(c.out, q.out[r] + o, __float_as_uint(x[0][r]));
         }
         return;
     }
@@ -428,63 +501,117 @@ __device__ __forceinline__ void finish(ConstConv& c, Buffer out, Buffer res, con
     const uint32_t xmask = (fl & CF_OUT_XOR) ? 0x80808080u : 0u;
     const uint32_t o = oc < c.out_limit ? static_cast<uint32_t>(oc) : static_cast<uint32_t>(kBeyond);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
+    for (int r = 0; r < R; ++r) {
         uint32_t w = 0;
 #pragma unroll
         for (int a = 0; a < A; ++a) w = __builtin_amdgcn_cvt_pk_u8_f32(x[a][r], a, w);
-        if (fl & CF_OUT_ADD) w = add_bytes(w, (static_cast<uint32_t>(static_cast<int>(c.out_off)) & 0xffu) * 0x01010101u);
+        if (fl & CF_OUT_ADD) w = add_bytes(w, c.off_bytes);
         w ^= xmask;
-        if constexpr (A == 4) publish4(out, q.out[r] + o, w);
-        else if constexpr (A == 2) publish2(out, q.out[r] + o, w);
-        else publish1(out, q.out[r] + o, w);
+        if constexpr (A == 4) publish4(c.out, q.out[r] + o, w);
+        else if constexpr (A == 2) publish2(c.out, q.out[r] + o, w);
+        else publish1(c.out, q.out[r] + o, w);
     }
 #undef PROG_EACH
 }
 
-// A step's K offsets into LDS.  Every lane takes part in every round (those behind the end repeat the last entry): no lane
-// is masked off here, in the loop that every convolution step begins with.  (An earlier compilation with a divergent form of
-// it had the copy of a register that merely lives through the masked region in front of the instruction that ends the mask,
-// which left the other lanes' values behind in a later attention step.  The other loops of this kernel do mask lanes off;
-// tests/test_program_cpu.py reads the assembly of the whole kernel for such a copy.)
-__device__ __forceinline__ void stage_offsets(lds_i32 to, const int32_t* from, int n, int tid) {
-    for (int base = 0; base < n; base += kProgramThreads) {
+// A step's K offsets into LDS.  A thread's first entry is requested here and stored by the caller, behind the tile's other
+// requests (`first`); only a K of more than 512 pieces is waited for.  Every lane takes part in every round (those behind the
+// end repeat the last entry): no lane is masked off here.
+__device__ __forceinline__ int32_t request_offsets(lds_i32 to, const int32_t* from, int n, int tid) {
+    for (int base = kProgramThreads; base < n; base += kProgramThreads) {
         const int i = min(base + tid, n - 1);
         to[i] = from[i];
     }
+    return from[min(tid, n - 1)];
 }
 
-template <int A, int B, bool PAIR = false>     // PAIR: a projection shortcut as a second product (F <= 8: room for two sets of partial sums)
-__device__ __forceinline__ void conv_tiles(ConstConv* desc, Ctx& x, lds_ptr lds) {
-    constexpr int F = A * B;                  // fragments of a tile
-    lds_i32 koff = (lds_i32)(lds + kPartBytes);
-    KSource src, src2{};
-    int per, sub, t0, t1;
-    {
-        ConstConv& c = *again(desc);
-        const int32_t* ko = PROG_TABLE(int32_t, c.koff);
-        const int shift = c.ks_shift;
-        src.ks = 1 << shift;
-        per = 8 >> shift;                     // waves per tile, tiles a workgroup works on at once
-        sub = x.wave >> shift;
-        src.kk = x.wave & (src.ks - 1);
-        src.koff = koff;
-        src.nk = c.nk;
-        src.in = make_buffer(PROG_REF(x, c.in));
-        stage_offsets(koff, ko, 4 * c.nk, x.tid);
-        if constexpr (PAIR) {
-            const int32_t* ko2 = PROG_TABLE(int32_t, c.koff2);
-            stage_offsets(koff + kMaxPieces, ko2, 4 * c.nk2, x.tid);
-            src2 = src;
-            src2.koff = koff + kMaxPieces;
-            src2.nk = c.nk2;
-            src2.in = make_buffer(PROG_REF(x, c.in2));
-        }
-        t0 = static_cast<int>(static_cast<uint32_t>(x.rank) * static_cast<uint32_t>(c.tiles) / static_cast<uint32_t>(x.n_wg));
-        t1 = static_cast<int>(static_cast<uint32_t>(x.rank + 1) * static_cast<uint32_t>(c.tiles) / static_cast<uint32_t>(x.n_wg));
+typedef uint32_t words4 __attribute__((ext_vector_type(4), aligned(4)));
+
+// four consecutive entries of a pixel table, from any of them (the table has room behind its last row)
+typedef uint32_t Words4 __attribute__((ext_vector_type(4), aligned(4)));
+template <int A>
+__device__ __forceinline__ void place_pixels(const uint32_t* pix, int M, int at, Pixels<A>& q) {
+    const Words4 po = *reinterpret_cast<const Words4*>(pix + M + at), pr = *reinterpret_cast<const Words4*>(pix + 2 * M + at);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        q.out[r] = po[r];
+        q.res[r] = pr[r];
     }
-    lds_v4i part = (lds_v4i)lds + x.wave * (F * 64) + x.lane;
-    lds_v4i part2 = (lds_v4i)(lds + kPartBytes / 2) + x.wave * (F * 64) + x.lane;
+}
+
+typedef __attribute__((address_space(3))) int32_t* lds_words;
+// pixels r0 .. r0 + R - 1 of the quads of one column: the partial sums of the ks waves that share the tile, and the chain
+template <bool GELU, int A, int B, int R, bool PAIR>
+__device__ __forceinline__ void finish_column(const StepConstants& sc, const ChannelConstants<A>& k, const ChannelConstants<A>& k2, lds_v4i mine, lds_v4i mine2, int ks,
+                                              int b, int r0, const Pixels<A>& q, int oc) {
+    auto total = [&](lds_v4i from, int32_t (&sum)[A][R]) {
+        const lds_words w = (lds_words)(from + b * A * 64) + r0;
+        for (int s = 0; s < ks; ++s)
+#pragma unroll
+            for (int a = 0; a < A; ++a) {
+                const lds_words v = w + (s * (A * B) + a) * 256;
+                if constexpr (R == 4) {
+                    const v4i t = *(lds_v4i)v;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sum[a][r] = s == 0 ? t[r] : sum[a][r] + t[r];
+                } else {
+#pragma unroll
+                    for (int r = 0; r < R; ++r) sum[a][r] = s == 0 ? v[r] : sum[a][r] + v[r];
+                }
+            }
+    };
+    int32_t sum[A][R];
+    float rg[A][R] = {};
+    total(mine, sum);
+    if constexpr (PAIR) {
+        int32_t s2[A][R];
+        total(mine2, s2);
+#pragma unroll
+        for (int a = 0; a < A; ++a)
+#pragma unroll
+            for (int r = 0; r < R; ++r) rg[a][r] = (static_cast<float>(s2[a][r]) + k2.bias[a]) * k2.scale[a];
+    }
+    finish<GELU, A, R, PAIR>(sc, k, sum, rg, q, oc);
+}
+
+template <bool GELU, int A, int B, bool PAIR = false>     // PAIR: a projection shortcut as a second product (F <= 8: room for two sets of partial sums)
+__device__ __forceinline__ void conv_tiles(Ctx& x, lds_ptr lds) {
+    constexpr int F = A * B;                  // fragments of a tile
+    constexpr bool kLate = F >= 16;           // the largest tile has no registers for the channels' constants before its sums are done
+    KSource src, src2{};
+    const int shift = PROG_FIELD(x.words, ks_shift);
+    src.ks = 1 << shift;
+    const int per = 8 >> shift, sub = x.wave >> shift;       // tiles a workgroup works on at once; the wave's
+    src.kk = x.wave & (src.ks - 1);
+    src.nk = PROG_FIELD(x.words, nk);
+    src.in = make_buffer(PROG_PLACE(x, in));
+    const bool plain = PROG_FIELD(x.words, koff).hi == 0;
+    const lds_i32 koff = (lds_i32)(lds + kPartBytes);
+    src.koff = plain ? (lds_i32)(lds + kPlainAt) : koff;
+    int32_t staged = 0, staged2 = 0;
+    if (!plain) staged = request_offsets(koff, PROG_TABLE_OF(int32_t, x.words, koff), 4 * src.nk, x.tid);
+    if constexpr (PAIR) {
+        src2 = src;
+        src2.nk = PROG_FIELD(x.words, nk2);
+        src2.in = make_buffer(PROG_PLACE(x, in2));
+        if (!plain) {
+            src2.koff = koff + kMaxPieces;
+            staged2 = request_offsets(koff + kMaxPieces, PROG_TABLE_OF(int32_t, x.words, koff2), 4 * src2.nk, x.tid);
+        }
+    }
+    const uint32_t tiles = static_cast<uint32_t>(PROG_FIELD(x.words, tiles));
+    const int t0 = static_cast<int>((static_cast<uint32_t>(x.rank) * tiles) >> x.wg_shift), t1 = static_cast<int>((static_cast<uint32_t>(x.rank + 1) * tiles) >> x.wg_shift);
+    const StepConstants sc = step_constants(x);
+    const int M = PROG_FIELD(x.words, M);
+    const uint32_t* pix = PROG_TABLE_OF(uint32_t, x.words, pixels);
+    const lds_v4i part = (lds_v4i)lds + x.wave * (F * 64) + x.lane;
+    const lds_v4i part2 = (lds_v4i)(lds + kPartBytes / 2) + x.wave * (F * 64) + x.lane;
     const lds_v4i mine = (lds_v4i)lds + sub * src.ks * (F * 64) + x.lane, mine2 = (lds_v4i)(lds + kPartBytes / 2) + sub * src.ks * (F * 64) + x.lane;
+    // The waves that share a tile's K share its chain as well: whole columns of pixels, or two of a quad's four pixels, or one.
+    // (The chain on one wave's eight values is 0.3 us of a step; the others of its tile would only wait for it.)
+    const int kk = src.kk, rows = B == 4 ? 4 : (4 * B) >> shift;      // (four columns and eight waves to a tile: choose_tile does not)
+    const int col0 = rows >= 4 ? kk & (B - 1) : (rows == 2 ? kk >> 1 : min(kk >> 2, B - 1)), r0 = rows >= 4 ? 0 : (rows == 2 ? 2 * (kk & 1) : kk & 3);
+    const bool finishes = rows >= 4 ? kk < B : kk < 4 * B;
     bool first = true;
     int base = t0;
     do {
@@ -494,44 +621,41 @@ __device__ __forceinline__ void conv_tiles(ConstConv* desc, Ctx& x, lds_ptr lds)
         ChannelConstants<A> k2;
         Ring<A, B> ring;
         uint32_t off[B], off2[B];
-        PixelQuad<A> q;
-        int mt, oc;
-        const int kk = src.kk, lane16 = x.lane & 15, quad = x.lane >> 4;
-        {
-            ConstConv& c = *again(desc);
-            int ot = 0, pt = 0;
-            if (on) fast_divmod(tile, c.p_tiles, c.inv_p_tiles, ot, pt);
-            ot = __builtin_amdgcn_readfirstlane(ot);
-            pt = __builtin_amdgcn_readfirstlane(pt);
-            mt = pt * (16 * B);
-            oc = ot * (16 * A) + A * lane16;
-            const uint32_t* pix = PROG_TABLE(uint32_t, c.pixels);
-            src.w = make_buffer(PROG_TABLE(int8_t, c.wgt) + static_cast<int64_t>(ot) * c.nk * (A * 1024));
+        Pixels<A> q;
+        const int lane16 = x.lane & 15, quad = x.lane >> 4;
+        int ot, pt;
+        fast_divmod(on ? tile : 0, PROG_FIELD(x.words, p_tiles), PROG_FIELD(x.words, inv_p_tiles), ot, pt);
+        ot = __builtin_amdgcn_readfirstlane(ot);
+        pt = __builtin_amdgcn_readfirstlane(pt);
+        const int mt = pt * (16 * B), oc = ot * (16 * A) + A * lane16;
+        src.w = make_buffer(PROG_TABLE_OF(int8_t, x.words, wgt) + static_cast<int64_t>(ot) * src.nk * (A * 1024));
+        if constexpr (PAIR) src2.w = make_buffer(PROG_TABLE_OF(int8_t, x.words, wgt2) + static_cast<int64_t>(ot) * src2.nk * (A * 1024));
+        if (on) {
 #pragma unroll
             for (int b = 0; b < B; ++b) off[b] = pix[mt + 16 * b + lane16];
+            const int pitch = PROG_FIELD(x.words, OCp) * 4;
             if constexpr (PAIR) {
-                src2.w = make_buffer(PROG_TABLE(int8_t, c.wgt2) + static_cast<int64_t>(ot) * c.nk2 * (A * 1024));
 #pragma unroll
-                for (int b = 0; b < B; ++b) off2[b] = pix[3 * c.M + mt + 16 * b + lane16];
+                for (int b = 0; b < B; ++b) off2[b] = pix[3 * M + mt + 16 * b + lane16];
                 first_weights<A, B>(ring, src2, x.lane);
-                const int32_t* t2 = PROG_TABLE(int32_t, c.constants2) + oc;
-                load_channels<A>(t2, k2.corr);
-                load_channels<A>(reinterpret_cast<const float*>(t2 + c.OCp), k2.bias);
-                load_channels<A>(reinterpret_cast<const float*>(t2 + 2 * c.OCp), k2.scale);
+                const uint8_t* t2 = PROG_TABLE_OF(uint8_t, x.words, constants2) + oc * 4;
+                load_channels<A>(reinterpret_cast<const int32_t*>(t2), k2.corr);
+                load_channels<A>(reinterpret_cast<const float*>(t2 + pitch), k2.bias);
+                load_channels<A>(reinterpret_cast<const float*>(t2 + 2 * pitch), k2.scale);
             } else {
                 first_weights<A, B>(ring, src, x.lane);
             }
-            load_constants<A>(c, oc, k);
-            // the first column this wave finishes
-            const uint4 po = *reinterpret_cast<const uint4*>(pix + c.M + mt + 16 * (kk & (B - 1)) + 4 * quad);
-            const uint4 pr = *reinterpret_cast<const uint4*>(pix + 2 * c.M + mt + 16 * (kk & (B - 1)) + 4 * quad);
-            q.out[0] = po.x; q.out[1] = po.y; q.out[2] = po.z; q.out[3] = po.w;
-            q.res[0] = pr.x; q.res[1] = pr.y; q.res[2] = pr.z; q.res[3] = pr.w;
+            if constexpr (kLate) load_channels<A>(reinterpret_cast<const int32_t*>(PROG_TABLE_OF(uint8_t, x.words, constants) + oc * 4), k.corr);
+            else load_constants<A>(sc.flags, PROG_TABLE_OF(uint8_t, x.words, constants), pitch, oc, k);
+            place_pixels<A>(pix, M, mt + 16 * col0 + 4 * quad + r0, q);      // the first column this wave finishes
         }
         if (first) {
+            if (!plain) {
+                koff[min(x.tid, 4 * src.nk - 1)] = staged;
+                if constexpr (PAIR) koff[kMaxPieces + min(x.tid, 4 * src2.nk - 1)] = staged2;
+            }
             x.wait();
             first = false;
-            if (x.dead) return;
         }
         v4i acc[A][B];
         auto start = [&](const int32_t (&corr)[A]) {      // the sum starts from the channel's integer correction, once per tile
@@ -556,8 +680,13 @@ __device__ __forceinline__ void conv_tiles(ConstConv* desc, Ctx& x, lds_ptr lds)
                 put(part2);
             }
             start(k.corr);
-            if (kk < B) load_residual<A>(*desc, make_buffer(resolve(max(desc->res.base, 0), desc->res.lo, desc->res.hi)), oc, q);
+            if (finishes) {
+                if (rows >= 4) load_residual<A, 4>(sc, oc, q);
+                else if (rows == 2) load_residual<A, 2>(sc, oc, q);
+                else load_residual<A, 1>(sc, oc, q);
+            }
             k_loop<A, B>(ring, src, off, x.lane, acc);
+            if constexpr (kLate) load_constants<A>(sc.flags, PROG_TABLE_OF(uint8_t, x.words, constants), PROG_FIELD(x.words, OCp) * 4, oc, k);
             put(part);
         }
         if (src.ks > 1) {
@@ -565,38 +694,18 @@ __device__ __forceinline__ void conv_tiles(ConstConv* desc, Ctx& x, lds_ptr lds)
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
         }
-        if (on && kk < B) {
-            ConstConv& c = *again(desc);
-            const Buffer out = make_buffer(PROG_REF(x, c.out)), res = make_buffer(resolve(max(c.res.base, 0), c.res.lo, c.res.hi));
-            for (int b = kk;;) {
-                v4i sum[A];
-                float rg[A][4] = {};
-#pragma unroll
-                for (int a = 0; a < A; ++a) sum[a] = mine[(b * A + a) * 64];
-                for (int s = 1; s < src.ks; ++s)
-#pragma unroll
-                    for (int a = 0; a < A; ++a) sum[a] += mine[s * (F * 64) + (b * A + a) * 64];
-                if constexpr (PAIR) {
-                    v4i s2[A];
-#pragma unroll
-                    for (int a = 0; a < A; ++a) s2[a] = mine2[(b * A + a) * 64];
-                    for (int s = 1; s < src.ks; ++s)
-#pragma unroll
-                        for (int a = 0; a < A; ++a) s2[a] += mine2[s * (F * 64) + (b * A + a) * 64];
-#pragma unroll
-                    for (int a = 0; a < A; ++a)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) rg[a][r] = (static_cast<float>(s2[a][r]) + k2.bias[a]) * k2.scale[a];
+        if (on && finishes) {
+            if (B == 4 || rows >= 4) {
+                for (int b = kk;;) {
+                    finish_column<GELU, A, B, 4, PAIR>(sc, k, k2, mine, mine2, src.ks, b, 0, q, oc);
+                    b += src.ks;
+                    if (b >= B) break;
+                    place_pixels<A>(pix, M, mt + 16 * b + 4 * quad, q);
+                    load_residual<A, 4>(sc, oc, q);
                 }
-                finish<A, PAIR>(c, out, res, k, sum, rg, q, oc);
-                b += src.ks;
-                if (b >= B) break;
-                const uint32_t* pix = PROG_TABLE(uint32_t, c.pixels);
-                const uint4 po = *reinterpret_cast<const uint4*>(pix + c.M + mt + 16 * b + 4 * quad);
-                const uint4 pr = *reinterpret_cast<const uint4*>(pix + 2 * c.M + mt + 16 * b + 4 * quad);
-                q.out[0] = po.x; q.out[1] = po.y; q.out[2] = po.z; q.out[3] = po.w;
-                q.res[0] = pr.x; q.res[1] = pr.y; q.res[2] = pr.z; q.res[3] = pr.w;
-                load_residual<A>(c, res, oc, q);
+            } else if constexpr (B < 4) {
+                if (rows == 2) finish_column<GELU, A, B, 2, PAIR>(sc, k, k2, mine, mine2, src.ks, col0, r0, q, oc);
+                else finish_column<GELU, A, B, 1, PAIR>(sc, k, k2, mine, mine2, src.ks, col0, r0, q, oc);
             }
         }
         base += per;
@@ -609,59 +718,69 @@ __device__ __forceinline__ void conv_tiles(ConstConv* desc, Ctx& x, lds_ptr lds)
 }
 
 // ---- depthwise 3 x 3 ----------------------------------------------------------------------------------------------------
-// A lane owns four channels of four output pixels of a row: six (stride 1) or nine columns of three input rows, byte
-// transposes (v_perm) and v_dot4_i32_i8 as in dwconv.hip; consecutive lanes take consecutive channels.
-template <int STRIDE>
-__device__ __forceinline__ void dw_items(ConstConv& c, Ctx& x) {
-    constexpr int COLS = 3 + 3 * STRIDE;
-    const int OH = c.OH, items = c.items, stride = 8 * x.n_wg * 64;
-    const Buffer in = make_buffer(PROG_REF(x, c.in)), out = make_buffer(PROG_REF(x, c.out)), res = make_buffer(resolve(max(c.res.base, 0), c.res.lo, c.res.hi));
-    const int last_col = (c.OW - 1) * STRIDE + 2;
+// A lane owns four channels of G output pixels of a row: its columns of three input rows, byte transposes (v_perm) and
+// v_dot4_i32_i8 as in dwconv.hip; consecutive lanes take consecutive channels.  G = 4 does the fewest operations per value,
+// G = 1 a quarter of the work per lane: where a step's values are no more than the launch's lanes at one pixel each, what a
+// lane does is what the step takes (ProgBuilder::conv).
+template <int STRIDE, int G>
+__device__ __forceinline__ void dw_items(Ctx& x) {
+    constexpr int COLS = G == 1 ? 3 : 3 + 3 * STRIDE;
+    const int OH = PROG_FIELD(x.words, OH), OW = PROG_FIELD(x.words, OW), items = PROG_FIELD(x.words, items), stride = 8 * x.n_wg * 64;
+    const int c4s = PROG_FIELD(x.words, c4), quads = PROG_FIELD(x.words, quads), OCp = PROG_FIELD(x.words, OCp);
+    const int in_sn = PROG_FIELD(x.words, in_sn), in_sh = PROG_FIELD(x.words, in_sh), in_sw = PROG_FIELD(x.words, in_sw), row_sh = PROG_FIELD(x.words, row_sh);
+    const int out_sn = PROG_FIELD(x.words, out_sn), out_sh = PROG_FIELD(x.words, out_sh), out_sw = PROG_FIELD(x.words, out_sw);
+    const int res_sn = PROG_FIELD(x.words, res_sn), res_sh = PROG_FIELD(x.words, res_sh), res_sw = PROG_FIELD(x.words, res_sw);
+    const float inv_c4 = PROG_FIELD(x.words, inv_c4), inv_quads = PROG_FIELD(x.words, inv_quads), inv_OH = PROG_FIELD(x.words, inv_OH);
+    const Buffer in = make_buffer(PROG_PLACE(x, in));
+    const StepConstants sc = step_constants(x);
+    const int8_t* wgt = PROG_TABLE_OF(int8_t, x.words, wgt);
+    const uint8_t* constants = PROG_TABLE_OF(uint8_t, x.words, constants);
+    const bool f32 = sc.flags & CF_RES_F32, fo = !(sc.flags & CF_OUT_FQ);
+    const int last_col = (OW - 1) * STRIDE + 2;
     bool first = true;
     int i0 = (x.wave * x.n_wg + x.rank) * 64;
     do {
         const int item = min(i0 + x.lane, items - 1);
         const bool on = i0 + x.lane < items;
         int q, c4, row, quad, n, oh;
-        fast_divmod(item, c.c4, c.inv_c4, q, c4);
-        fast_divmod(q, c.quads, c.inv_quads, row, quad);
-        fast_divmod(row, OH, c.inv_OH, n, oh);
-        const int oc = 4 * c4, ow0 = 4 * quad;
-        const uint32_t p = static_cast<uint32_t>(n * c.in_sn + oh * c.in_sh + oc);
+        fast_divmod(item, c4s, inv_c4, q, c4);
+        fast_divmod(q, quads, inv_quads, row, quad);
+        fast_divmod(row, OH, inv_OH, n, oh);
+        const int oc = 4 * c4, ow0 = G * quad;
+        const uint32_t p = static_cast<uint32_t>(n * in_sn + oh * in_sh + oc);
         uint32_t v[3][COLS];
         uint4 wr[3];
 #pragma unroll
-        for (int r = 0; r < 3; ++r)
-            wr[r] = *reinterpret_cast<const uint4*>(PROG_TABLE(int8_t, c.wgt) + (static_cast<int64_t>(r) * c.OCp + oc) * 4);
+        for (int r = 0; r < 3; ++r) wr[r] = *reinterpret_cast<const uint4*>(wgt + (static_cast<int64_t>(r) * OCp + oc) * 4);
         ChannelConstants<4> k;
-        load_constants<4>(c, oc, k);
+        load_constants<4>(sc.flags, constants, OCp * 4, oc, k);
         uint32_t col[COLS];
 #pragma unroll
-        for (int j = 0; j < COLS; ++j) col[j] = p + static_cast<uint32_t>(min(ow0 * STRIDE + j, last_col) * c.in_sw);
-        PixelQuad<4> pq;
+        for (int j = 0; j < COLS; ++j) col[j] = p + static_cast<uint32_t>((G == 1 ? ow0 * STRIDE + j : min(ow0 * STRIDE + j, last_col)) * in_sw);
+        Pixels<4> pq;
         {
-            const bool f32 = c.flags & CF_RES_F32, fo = !(c.flags & CF_OUT_FQ);
-            const uint32_t o = static_cast<uint32_t>(n * c.out_sn + oh * c.out_sh), s = static_cast<uint32_t>(n * c.res_sn + oh * c.res_sh);
+            const uint32_t o = static_cast<uint32_t>(n * out_sn + oh * out_sh), s = static_cast<uint32_t>(n * res_sn + oh * res_sh);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int ow = min(ow0 + r, c.OW - 1);
-                pq.out[r] = on && ow0 + r < c.OW ? (o + ow * c.out_sw) << (fo ? 2 : 0) : static_cast<uint32_t>(kBeyond);
-                pq.res[r] = (s + ow * c.res_sw) << (f32 ? 2 : 0);
+            for (int r = 0; r < G; ++r) {
+                const int ow = min(ow0 + r, OW - 1);
+                pq.out[r] = on && ow0 + r < OW ? (o + ow * out_sw) << (fo ? 2 : 0) : static_cast<uint32_t>(kBeyond);
+                pq.res[r] = (s + ow * res_sw) << (f32 ? 2 : 0);
             }
         }
         if (first) {
             x.wait();
             first = false;
-            if (x.dead) return;
         }
 #pragma unroll
         for (int r = 0; r < 3; ++r)
 #pragma unroll
-            for (int j = 0; j < COLS; ++j) v[r][j] = shared4(in, col[j] + static_cast<uint32_t>(r * c.row_sh));
-        load_residual<4>(c, res, oc, pq);
-        v4i acc[4];                           // [channel][pixel]
+            for (int j = 0; j < COLS; ++j) v[r][j] = shared4(in, col[j] + static_cast<uint32_t>(r * row_sh));
+        load_residual<4, G>(sc, oc, pq);
+        int32_t acc[4][G];                    // [channel][pixel]
 #pragma unroll
-        for (int a = 0; a < 4; ++a) acc[a] = v4i{k.corr[a], k.corr[a], k.corr[a], k.corr[a]};
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int r = 0; r < G; ++r) acc[a][r] = k.corr[a];
         auto transpose4 = [&](uint32_t p0, uint32_t p1, uint32_t p2, uint32_t p3, uint32_t (&t)[4]) {
             const uint32_t lo01 = __builtin_amdgcn_perm(p1, p0, 0x05010400u), hi01 = __builtin_amdgcn_perm(p1, p0, 0x07030602u);
             const uint32_t lo23 = __builtin_amdgcn_perm(p3, p2, 0x05010400u), hi23 = __builtin_amdgcn_perm(p3, p2, 0x07030602u);
@@ -673,7 +792,7 @@ __device__ __forceinline__ void dw_items(ConstConv& c, Ctx& x) {
 #pragma unroll
         for (int r = 0; r < 3; ++r) {
             const uint32_t w[4] = {wr[r].x, wr[r].y, wr[r].z, wr[r].w};
-            if constexpr (STRIDE == 1) {
+            if constexpr (STRIDE == 1 && G == 4) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     uint32_t t[4];
@@ -686,7 +805,7 @@ __device__ __forceinline__ void dw_items(ConstConv& c, Ctx& x) {
                 }
             } else {
 #pragma unroll
-                for (int h = 0; h < 4; ++h) {
+                for (int h = 0; h < G; ++h) {
                     uint32_t t[4];
                     transpose4(v[r][2 * h], v[r][2 * h + 1], v[r][2 * h + 2], v[r][2 * h + 2], t);
 #pragma unroll
@@ -694,8 +813,8 @@ __device__ __forceinline__ void dw_items(ConstConv& c, Ctx& x) {
                 }
             }
         }
-        const float none[4][4] = {};
-        finish<4>(c, out, res, k, acc, none, pq, oc);
+        const float none[4][G] = {};
+        finish<false, 4, G>(sc, k, acc, none, pq, oc);
         i0 += stride;
     } while (i0 < items);
 }
@@ -901,9 +1020,21 @@ __device__ __forceinline__ void exit_items(const ProgExit& s, const Ctx& x) {
 }
 
 // ---- rows of an encoder -----------------------------------------------------------------------------------------------------
+// v summed over the wave as a butterfly, lanes 32 apart first: the pairs and the order of __shfl_xor by 32, 16 .. 1.  Lanes 32 and
+// 16 apart come together by a swap of rows, and behind those the value repeats every 16, 8, 4 lanes, so that a rotation by
+// 8 and by 4 of a row's lanes and two permutations of its quads find the same partners: an instruction each, where a shuffle
+// by way of LDS takes 0.05 us (twelve of them were 0.7 us of a LayerNorm step).
 __device__ __forceinline__ float wave_total(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+#if defined(__HIP_DEVICE_COMPILE__)
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+    const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true));      // row_ror:8
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, true));      // row_ror:4
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4e, 0xf, 0xf, true));       // quad_perm 2 3 0 1
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xb1, 0xf, 0xf, true));       // quad_perm 1 0 3 2
+#endif
     return v;
 }
 
@@ -934,13 +1065,22 @@ __device__ __forceinline__ void embed_rows(const ProgEmbed& e, const Ctx& x) {
 }
 
 constexpr int kMvnChunks = 4;                 // rows of up to 1024 values
-__device__ __forceinline__ void mvn_rows(const ProgMvn& s, const Ctx& x) {
-    const Buffer in = make_buffer(PROG_REF(x, s.in)), yb = make_buffer(resolve(max(s.out.base, 0), s.out.lo, s.out.hi)),
-                 qb = make_buffer(resolve(max(s.outq.base, 0), s.outq.lo, s.outq.hi));
+__device__ __forceinline__ void mvn_rows(const ProgMvn& s, Ctx& x) {
+    const Buffer in = make_buffer(x.place(s.in)), yb = make_buffer(x.place(s.out)), qb = make_buffer(x.place(s.outq));
     const bool y = s.out.base >= 0, q = s.outq.base >= 0;
     const float *gamma = PROG_TABLE(float, s.gamma), *beta = PROG_TABLE(float, s.beta);
     const int axis = s.axis;
-    for (int row = x.wave * x.n_wg + x.rank; row < s.rows; row += 8 * x.n_wg) {
+    int row = x.wave * x.n_wg + x.rank;
+    // the affine part of a lane's columns, the same for all its rows, while the step before comes to its end
+    float4 g[kMvnChunks], b[kMvnChunks];
+#pragma unroll
+    for (int j = 0; j < kMvnChunks; ++j) {
+        const int i = min(256 * j + 4 * x.lane, axis - 4);
+        if (gamma) g[j] = ld4f(gamma + i);
+        if (beta) b[j] = ld4f(beta + i);
+    }
+    x.wait();
+    for (; row < s.rows; row += 8 * x.n_wg) {
         const uint32_t p = static_cast<uint32_t>(row * axis);
         float4 v[kMvnChunks];
         float sum = 0.f;
@@ -948,8 +1088,9 @@ __device__ __forceinline__ void mvn_rows(const ProgMvn& s, const Ctx& x) {
         for (int j = 0; j < kMvnChunks; ++j) {
             const int i = 256 * j + 4 * x.lane;
             v[j] = shared16f(in, i < axis ? 4u * (p + i) : static_cast<uint32_t>(kBeyond));
-            sum += (v[j].x + v[j].y) + (v[j].z + v[j].w);
         }
+#pragma unroll
+        for (int j = 0; j < kMvnChunks; ++j) sum += (v[j].x + v[j].y) + (v[j].z + v[j].w);
         const float mean = wave_total(sum) / static_cast<float>(axis);
         float sq = 0.f;
 #pragma unroll
@@ -969,8 +1110,8 @@ __device__ __forceinline__ void mvn_rows(const ProgMvn& s, const Ctx& x) {
             if (i >= axis) continue;
             float4 o = v[j];
             if (s.normalize) { o.x = o.x / denom; o.y = o.y / denom; o.z = o.z / denom; o.w = o.w / denom; }
-            if (gamma) { const float4 g = ld4f(gamma + i); o.x = o.x * g.x; o.y = o.y * g.y; o.z = o.z * g.z; o.w = o.w * g.w; }
-            if (beta) { const float4 b = ld4f(beta + i); o.x = o.x + b.x; o.y = o.y + b.y; o.z = o.z + b.z; o.w = o.w + b.w; }
+            if (gamma) { o.x = o.x * g[j].x; o.y = o.y * g[j].y; o.z = o.z * g[j].z; o.w = o.w * g[j].w; }
+            if (beta) { o.x = o.x + b[j].x; o.y = o.y + b[j].y; o.z = o.z + b[j].z; o.w = o.w + b[j].w; }
             if (y) publish16f(yb, 4u * (p + i), o);
             if (q) publish4(qb, p + i, levels4(s.fq, o));
         }
@@ -1166,10 +1307,14 @@ __device__ __forceinline__ void attention_units(const ProgAttention& s, const Ct
     }
 }
 
+__device__ __forceinline__ int lane_index() { return static_cast<int>(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u))); }
+
 // ---- the program ------------------------------------------------------------------------------------------------------------
-// 246 vector registers, which the 4 x 4 tiles ask for, and none spilled to memory; 230 scalar registers of the many step kinds
-// are kept in lanes of a vector register.  A new step kind adds to these for all steps: it belongs into a kernel of its own
-// where it needs more than they have.
+// Two kernels, for networks over feature maps and for encoders: every kind of step adds to the registers of all others (all in
+// one spill).  The 4 x 4 tiles ask for 250 and more vector registers, none is spilled to memory; 300 - 400 scalar registers of
+// the many step kinds are kept in lanes of vector registers.  A new step kind belongs into a kernel of its own where it needs
+// more than they have.
+template <bool ENCODER>
 __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgArgs g) {
     extern __shared__ __attribute__((aligned(16))) int8_t smem[];
     lds_ptr lds = (lds_ptr)smem;
@@ -1179,80 +1324,51 @@ __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgA
     x.lane = x.tid & 63;
     x.wave = __builtin_amdgcn_readfirstlane(x.tid >> 6);
     x.n_wg = g.workgroups;
+    x.wg_shift = __builtin_ctz(x.n_wg);
+    x.steps = g.steps;
+    x.words = x.load_words(0);
+    x.bases = reinterpret_cast<const uint32_t*>(g.bases)[min(x.lane, 2 * (1 + kProgramIo) - 1)];
+    for (int i = x.tid; i < kMaxPieces; i += kProgramThreads) ((lds_i32)(lds + kPlainAt))[i] = 16 * i;
     x.rank = static_cast<int>(blockIdx.x % 8) * (x.n_wg / 8) + static_cast<int>(blockIdx.x / 8);
-    const bool tree = x.n_wg > kFlat;
-    x.root = g.control + kCtlRoot;
-    x.sub = tree ? g.control + kCtlXcd + 32 * (blockIdx.x % 8) : nullptr;
-    x.root_target = g.launch * static_cast<uint32_t>(g.n_steps * (tree ? 8 : x.n_wg));      // roll call + n_steps - 1 barriers a launch
-    x.sub_target = g.launch * static_cast<uint32_t>(g.n_steps * (x.n_wg / 8));
-    x.next_targets();
+    x.xcds = g.control;
+    x.own = x.xcds + kXcdWords * (blockIdx.x % 8);
+    x.target = (g.launch * static_cast<uint32_t>(g.n_steps) + 1) * static_cast<uint32_t>(x.n_wg / 8);      // a launch: the roll call and n_steps - 1 barriers
     x.report = g.report;
+    x.started = true;
     x.dead = false;
     x.flag = flag;
-    // roll call: everybody is resident, or nobody starts
-    if (x.tid == 0) {
-        uint32_t* state = g.control + kCtlState;
-        const uint32_t before = 2 * g.launch, go = before + 2, off = before + 3;
-        uint32_t s = __hip_atomic_load(state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (s == before) {
-            uint32_t expect = before;
-            if (x.count()) __hip_atomic_compare_exchange_strong(state, &expect, go, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const uint64_t t0 = wall_clock64();
-            for (;;) {
-                s = __hip_atomic_load(state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (s != before) break;
-                if (wall_clock64() - t0 > g.roll_call_ticks) {
-                    expect = before;
-                    if (__hip_atomic_compare_exchange_strong(state, &expect, off, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) expect = off;
-                    s = expect;
-                    break;
-                }
-            }
-        }
-        if (s != go) __hip_atomic_store(g.report, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        flag[0] = s == go ? 1 : 0;
-    }
-    __syncthreads();
-    if (flag[0] == 0) return;
+    if (!x.roll_call(g.roll_call_ticks)) return;
     for (int step = 0; step < g.n_steps; ++step) {
         // the thread's place is derived again in every step: as loop invariants its many functions (row, piece, quad ... of every
         // kind of step) would live in registers across all of them, and be moved out of the way and back around the large tiles
-        int tid = threadIdx.x;
+        int lane = lane_index();
 #if defined(__HIP_DEVICE_COMPILE__)
-        asm volatile("" : "+v"(tid));
+        asm volatile("" : "+v"(lane));
 #endif
-        x.tid = tid;
-        x.lane = tid & 63;
+        x.lane = lane;
+        x.tid = 64 * x.wave + lane;
         const StepPtr words = step_ptr(g.steps, step);
-        const int kind = words[0];
-        if (kind != PK_CONV && kind != PK_DW) {
-            x.wait();
-            if (x.dead) return;
-        }
+        const int kind = static_cast<int>(word_of(x.words, 0));
+        if (kind != PK_CONV && kind != PK_DW && kind != PK_MVN) x.wait();
         switch (kind) {
         case PK_CONV: {
-            ConstConv* c = (ConstConv*)words;
-            switch (c->a * 8 + c->b + (c->nk2 ? 64 : 0)) {
-            case 8 + 4: conv_tiles<1, 4>(c, x, lds); break;
-            case 16 + 1: conv_tiles<2, 1>(c, x, lds); break;
-            case 16 + 2: conv_tiles<2, 2>(c, x, lds); break;
-            case 16 + 4: conv_tiles<2, 4>(c, x, lds); break;
-            case 32 + 2: conv_tiles<4, 2>(c, x, lds); break;
-            case 64 + 16 + 2: conv_tiles<2, 2, true>(c, x, lds); break;
-            case 64 + 16 + 4: conv_tiles<2, 4, true>(c, x, lds); break;
-            default: conv_tiles<4, 4>(c, x, lds); break;
+            switch (PROG_FIELD(x.words, a) * 8 + PROG_FIELD(x.words, b) + (PROG_FIELD(x.words, nk2) ? 64 : 0)) {
+            case 8 + 4: conv_tiles<ENCODER, 1, 4>(x, lds); break;
+            case 16 + 1: conv_tiles<ENCODER, 2, 1>(x, lds); break;
+            case 16 + 2: conv_tiles<ENCODER, 2, 2>(x, lds); break;
+            case 16 + 4: conv_tiles<ENCODER, 2, 4>(x, lds); break;
+            case 32 + 2: conv_tiles<ENCODER, 4, 2>(x, lds); break;
+            case 64 + 16 + 2:
+                if constexpr (!ENCODER) conv_tiles<ENCODER, 2, 2, true>(x, lds);
+                break;
+            case 64 + 16 + 4:
+                if constexpr (!ENCODER) conv_tiles<ENCODER, 2, 4, true>(x, lds);
+                break;
+            default: conv_tiles<ENCODER, 4, 4>(x, lds); break;
             }
             break;
         }
-        case PK_DW: {
-            ConstConv& c = *(ConstConv*)words;
-            if (c.stride == 1) dw_items<1>(c, x);
-            else dw_items<2>(c, x);
-            break;
-        }
         case PK_ENTRY: entry_items(unpack<ProgEntry>(words), x); break;
-        case PK_MAXPOOL: max_pool_items(unpack<ProgPool>(words), x); break;
-        case PK_AVGPOOL: avg_pool_items(unpack<ProgPool>(words), x); break;
         case PK_EXIT: {
             const ProgExit e = unpack<ProgExit>(words);
             if (e.in_dtype == HIPIE_F32) exit_items<float>(e, x);
@@ -1260,20 +1376,32 @@ __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgA
             else exit_items<int8_t>(e, x);
             break;
         }
-        case PK_EMBED: embed_rows(unpack<ProgEmbed>(words), x); break;
-        case PK_MVN: mvn_rows(unpack<ProgMvn>(words), x); break;
-        case PK_ATTENTION: attention_units(unpack<ProgAttention>(words), x, lds); break;
         case PK_FQROWS: fq_items(unpack<ProgRows>(words), x); break;
-        default: copy_items(unpack<ProgRows>(words), x); break;
+        case PK_COPY: copy_items(unpack<ProgRows>(words), x); break;
+        default:
+            if constexpr (ENCODER) {
+                if (kind == PK_EMBED) embed_rows(unpack<ProgEmbed>(words), x);
+                else if (kind == PK_MVN) mvn_rows(unpack<ProgMvn>(words), x);
+                else attention_units(unpack<ProgAttention>(words), x, lds);
+            } else if (kind == PK_DW) {
+                switch (PROG_FIELD(x.words, stride) * 8 + PROG_FIELD(x.words, group)) {
+                case 8 + 1: dw_items<1, 1>(x); break;
+                case 8 + 4: dw_items<1, 4>(x); break;
+                case 16 + 1: dw_items<2, 1>(x); break;
+                default: dw_items<2, 4>(x); break;
+                }
+            } else if (kind == PK_MAXPOOL) max_pool_items(unpack<ProgPool>(words), x);
+            else avg_pool_items(unpack<ProgPool>(words), x);
         }
-        if (x.dead) return;
         if (step + 1 == g.n_steps) break;
-        {   // the next step's descriptor into the scalar cache
-            const StepPtr next = step_ptr(g.steps, step + 1);
-#pragma unroll
-            for (int i = 0; i < kProgramStepWords; i += 16) asm volatile("" ::"s"(next[i]));
+        {   // the next step's descriptor into the scalar cache: its eight lines asked for together, beside the stores' way to memory
+            // (one behind the other they took 0.7 us of every step)
+            const StepPtr n = step_ptr(g.steps, step + 1);
+            static_assert(kProgramStepWords == 128, "eight lines of 64 bytes");
+            asm volatile("" ::"s"(n[0]), "s"(n[16]), "s"(n[32]), "s"(n[48]), "s"(n[64]), "s"(n[80]), "s"(n[96]), "s"(n[112]));
         }
-        x.arrive();
+        x.arrive(step + 1);
+        if (x.dead) return;
     }
 }
 
@@ -1316,7 +1444,7 @@ TileChoice choose_tile(int workgroups, int oc, int64_t pixels, int nk, int nk2, 
     for (const auto& shape : kShapes)
         for (int ks : {1, 2, 4, 8}) {
             const int a = shape[0], b = shape[1];
-            if ((nk2 && (a != 2 || b < 2)) || (gelu && a == 1)) continue;
+            if ((nk2 && (a != 2 || b < 2)) || (gelu && a == 1) || (b == 4 && ks == 8)) continue;
             const int depth = a * b >= 16 ? 2 : (a * b >= 8 ? 4 : 6);
             const int64_t tiles = ceil_div(oc, 16 * a) * ceil_div(pixels, 16 * b), per_wg = ceil_div(tiles, workgroups);
             const int64_t rounds = ceil_div(per_wg, 8 / ks);
@@ -1403,20 +1531,23 @@ bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hip
         }
         c.constants = gather(rows, static_cast<size_t>(a.OCp) * 4);
     }
-    c.flags = a.flags; c.lm1 = a.lm1; c.out_off = a.out_off; c.clamp_lo = a.clamp_lo; c.clamp_hi = a.clamp_hi;
+    c.flags = a.flags; c.lm1 = a.lm1; c.off_bytes = (static_cast<uint32_t>(static_cast<int>(a.out_off)) & 0xffu) * 0x01010101u; c.clamp_lo = a.clamp_lo; c.clamp_hi = a.clamp_hi;
     c.OCp = a.OCp;
     if (l.depthwise) {
         c.OH = a.OHOW / a.OW;
         c.OW = a.OW;
         if (l.kh != 3 || l.kw != 3 || l.dil_h != 1 || l.dil_w != 1 || a.conv_sh != a.conv_sw || a.conv_sh > 2 || !a.wgt2 || a.in_sw < a.out_sw) return false;
         c.kind = PK_DW;
+        map_kinds = true;
         c.stride = a.conv_sh;
         c.wgt = ptr(a.wgt2);
         c.in_sn = a.in_sn; c.in_sh = a.in_sh * a.conv_sh; c.in_sw = a.in_sw; c.row_sh = a.in_sh;
         c.out_sn = a.out_sn; c.out_sh = a.out_sh; c.out_sw = a.out_sw;
         c.res_sn = a.res_sn; c.res_sh = a.res_sh; c.res_sw = a.res_sw;
         c.c4 = a.out_sw / 4;
-        c.quads = static_cast<int32_t>(ceil_div(a.OW, 4));
+        // four pixels a lane where a step has more values than that leaves lanes idle
+        c.group = static_cast<int64_t>(out.n) * c.OH * a.OW * c.c4 <= static_cast<int64_t>(workgroups) * kProgramThreads ? 1 : 4;
+        c.quads = static_cast<int32_t>(ceil_div(a.OW, c.group));
         const int64_t items = static_cast<int64_t>(out.n) * c.OH * c.quads * c.c4;
         if (items >= (1 << 24)) return false;
         c.items = static_cast<int32_t>(items);
@@ -1429,6 +1560,8 @@ bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hip
     c.kind = PK_CONV;
     c.nk = a.nk;
     const bool pair = (a.flags & CF_RES_GEMM) != 0;
+    if (a.flags & CF_GELU) rows_kinds = true;
+    if (pair) map_kinds = true;
     if (4 * a.nk > kMaxPieces || (pair && 4 * a.nk2 > kMaxPieces)) return false;
     const TileChoice t = choose_tile(workgroups, a.OC, M, a.nk, pair ? a.nk2 : 0, (a.flags & CF_GELU) != 0);
     c.a = t.a; c.b = t.b; c.ks_shift = __builtin_ctz(static_cast<unsigned>(t.ks));
@@ -1439,7 +1572,7 @@ bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hip
     const int64_t tiles = static_cast<int64_t>(c.p_tiles) * o_tiles;
     if (tiles * workgroups >= (1ll << 31) || tiles >= (1 << 24) || static_cast<int64_t>(a.nk) * t.a * 1024 >= kBeyond) return false;
     c.tiles = static_cast<int32_t>(tiles);
-    c.koff = ptr(a.koff);
+    if (!(a.k_linear && (!pair || a.k_linear2))) c.koff = ptr(a.koff);       // (0: the kernel's own table, 16 i)
     auto repack = [&](const int8_t* w, int Kp) {
         owned.emplace_back();
         const int64_t pieces = static_cast<int64_t>(o_tiles) * t.a * Kp;        // 16 a x Kp bytes per tile, 16 bytes a piece
@@ -1460,7 +1593,7 @@ bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hip
     // where every pixel's window and results are; pixels behind the last one read where it does and store nowhere
     const int64_t pitch = static_cast<int64_t>(c.p_tiles) * 16 * t.b;
     c.M = static_cast<int32_t>(pitch);
-    std::vector<uint32_t> pix(static_cast<size_t>(4 * pitch));
+    std::vector<uint32_t> pix(static_cast<size_t>(4 * pitch + 4));       // (a wave reads four entries from any of them)
     for (int64_t i = 0; i < pitch; ++i) {
         const int64_t m = std::min(i, M - 1), n = m / a.OHOW, rem = m - n * a.OHOW, oh = rem / a.OW, ow = rem - oh * a.OW;
         auto at = [&](int sn, int sh, int sw) { return static_cast<uint32_t>(n * sn + oh * sh + ow * sw); };
@@ -1513,6 +1646,7 @@ bool ProgBuilder::pool(const PoolArgs& a, bool avg, bool rcp) {
     if ((a.fq_il && !rcp) || static_cast<int64_t>(a.M) * a.cs >= (1ll << 30) || a.cs % 4 != 0 || span >= kBeyond) return false;
     ProgPool p{};
     p.kind = avg ? PK_AVGPOOL : PK_MAXPOOL;
+    map_kinds = true;
     p.items = a.M * (a.cs / 4);
     const int OH = a.OHOW / a.OW;
     p.k3 = a.kh == 3 && a.kw == 3 && (OH - 1) * a.sh - a.pt + 3 <= a.H + a.pb && (a.OW - 1) * a.sw - a.pl + 3 <= a.W + a.pr;
@@ -1540,6 +1674,7 @@ bool ProgBuilder::embed(const float* table, int64_t vocab, int64_t hidden, const
     if (hidden % 4 != 0 || tokens * hidden * 4 >= kBeyond || seq >= (1 << 24)) return false;
     ProgEmbed e{};
     e.kind = PK_EMBED;
+    rows_kinds = true;
     e.hidden = static_cast<int32_t>(hidden);
     e.seq = static_cast<int32_t>(seq);
     e.pos0 = pos0;
@@ -1560,6 +1695,7 @@ bool ProgBuilder::mvn(const void* in, void* out, void* outq, int64_t rows, int64
     if (rows * axis * 4 >= kBeyond || axis % 4 != 0 || axis > 256 * kMvnChunks) return false;
     ProgMvn m{};
     m.kind = PK_MVN;
+    rows_kinds = true;
     m.axis = static_cast<int32_t>(axis);
     m.rows = static_cast<int32_t>(rows);
     m.normalize = normalize;
@@ -1586,6 +1722,7 @@ bool ProgBuilder::attention(const hipie_attention* att, const void* const (&qkv)
     if (proto.S * 64 + 64 * (proto.S + 16) + 256 + 4 * proto.S > kPartBytes) return false;
     ProgAttention s{};
     s.kind = PK_ATTENTION;
+    rows_kinds = true;
     s.S = proto.S;
     s.heads = batch;
     s.q = ref(qkv[0]); s.k = ref(qkv[1]); s.v = ref(qkv[2]);
@@ -1703,6 +1840,7 @@ std::shared_ptr<ProgramForm> make_program_form(ProgBuilder&& b) {
     auto f = std::make_shared<ProgramForm>();
     f->workgroups = b.workgroups;
     f->n_steps = static_cast<int>(b.steps.size());
+    f->encoder = b.rows_kinds;
     f->steps.upload(b.device, b.steps.data(), b.steps.size() * kProgramStepWords * 4);
     f->owned = std::move(b.owned);
     DeviceGuard g(b.device);
@@ -1723,7 +1861,8 @@ std::shared_ptr<Program> make_program(int device) {
     DeviceGuard g(device);
     HIPIE_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&p->report), Program::kSlots * 64, hipHostMallocDefault));
     std::memset(p->report, 0, Program::kSlots * 64);
-    HIPIE_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&program_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    for (auto kernel : {&program_kernel<false>, &program_kernel<true>})
+        HIPIE_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     return p;
 }
 
@@ -1784,7 +1923,7 @@ void launch_program(const Program& p, const ProgramForm& f, uint8_t* arena, void
     a.launch = launch;
     a.roll_call_ticks = p.roll_call_ticks;
     p.report[16 * slot] = 0;
-    hipLaunchKernelGGL(program_kernel, dim3(static_cast<uint32_t>(f.workgroups)), dim3(kProgramThreads), kLdsBytes, s, a);
+    hipLaunchKernelGGL(f.encoder ? program_kernel<true> : program_kernel<false>, dim3(static_cast<uint32_t>(f.workgroups)), dim3(kProgramThreads), kLdsBytes, s, a);
     HIPIE_CHECK_HIP(hipGetLastError());
 }
 

@@ -68,10 +68,13 @@ def test_no_register_is_copied_where_a_mask_of_the_persistent_kernel_ends(tmp_pa
     subprocess.run([build.HIPCC] + build.FLAGS + ["-x", "hip", "--offload-device-only", "-S", os.path.join(build.CSRC, "program.hip"), "-o", str(out)],
                    check=True, capture_output=True)
     text = out.read_text()
-    kernel = text[re.search(r"^_ZN\S*program_kernel\S*:", text, re.M).start():]
-    kernel = kernel[:kernel.index(".end_amdhsa_kernel")]
-    lines = kernel.splitlines()
-    assert sum("exec, exec" in line for line in lines) > 40     # the masks are there to be read
-    assert masked_writes(lines) == []
-    assert re.search(r"\.amdhsa_private_segment_fixed_size 0\b", kernel)
+    found = [m.start() for m in re.finditer(r"^_ZN\S*program_kernel\S*:", text, re.M)]
+    assert len(found) == 2                                          # feature maps, encoders
+    for start in found:
+        kernel = text[start:]
+        kernel = kernel[:kernel.index(".end_amdhsa_kernel")]
+        lines = kernel.splitlines()
+        assert sum("exec, exec" in line for line in lines) > 40     # the masks are there to be read
+        assert masked_writes(lines) == []
+        assert re.search(r"\.amdhsa_private_segment_fixed_size 0\b", kernel)
     assert set(re.findall(r"\.vgpr_spill_count: *(\d+)", text)) == {"0"}
