@@ -96,7 +96,7 @@ struct ProgMvn {
     Requant fq;
 };
 struct ProgAttention {
-    int32_t kind, S, heads, units, waves, parts;   // waves of a workgroup that take 32 queries each, workgroups per (element, head)
+    int32_t kind, S, heads, units, split_shift, parts;   // log2 of the waves that share 32 queries, workgroups per (element, head)
     ProgRef q, k, v, out, mask;
     int32_t has_mask, pform;
     AttentionArgs a;

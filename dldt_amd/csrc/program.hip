@@ -1137,174 +1137,228 @@ __device__ __forceinline__ void copy_items(const ProgRows& s, const Ctx& x) {
 }
 
 // ---- attention --------------------------------------------------------------------------------------------------------------
-// The core of attention.hip with the sequence length at run time: K and V^T of one (element, head) in LDS, a wave takes
-// 32 queries.  The scores do not stay in registers (S / 2 of them would limit S to 384 and need an instance per length):
-// they are multiplied out three times, for the maximum, the sum and the probabilities - the matrix pipe is idle here anyway.
+// The core of attention.hip with the sequence length at run time: K and V^T of one (element, head) in LDS.  32 queries are the
+// work of `split` waves: each takes every split-th tile of 32 keys - its scores stay in registers, up to kMostTiles of them -
+// and the waves meet for the maximum, for the sum and for the integer sums of the context.  What bounds a step is the chain of
+// exponentials and levels of one wave (1 us for a tile of 32 x 32), so the fewer tiles a wave has the better while there are
+// compute units: one sequence of 128 tokens, 12 heads, took 10.9 us with a wave for 32 queries, 48 waves in all, that
+// multiplied the scores out three times, and takes 4.8 with four.  The sum keeps its order - a lane's keys one behind the
+// other - so one wave adds the exponentials of all.  They take K's place in LDS, and the context's partial sums theirs.
+constexpr int kMostTiles = 4;                 // of a wave
+constexpr int kMostSplit = 8;
+// LDS: V^T; K, then exponentials, then partial sums of the context; the mask, the maxima and the sums of the waves' rows
+__host__ __device__ constexpr int attention_exchange(int S, int split) {
+    const int k = S * 64, ctx = 64 * 1024, e = split > 1 ? kMostSplit / split * (S / 32) * 4096 : 0;
+    return k > ctx ? (k > e ? k : e) : (ctx > e ? ctx : e);
+}
+__host__ __device__ constexpr int attention_lds(int S, int split) { return 64 * (S + 16) + attention_exchange(S, split) + 4 * S + 8 * 32 * 4 + 8 * 64 * 4; }
 // LONG: the Softmax of rows longer than kPlainSoftmax.
 template <bool LONG, int PFORM>
-__device__ __forceinline__ void attention_queries(const ProgAttention& s, Buffer qb, uint32_t qbase, Buffer out, uint32_t obase, int q0,
-                                                  lds_ptr sK, lds_ptr sVT, lds_i32 sVsum, const __attribute__((address_space(3))) float* sMask, int lane) {
+__device__ __forceinline__ void attention_units(const ProgAttention& s, Ctx& x, lds_ptr lds) {
+    typedef __attribute__((address_space(3))) float* lds_f32;
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) v4f* lds_v4f;
     const AttentionArgs& a = s.a;
-    const int S = s.S, nt = S / 32, l32 = lane & 31, h = lane >> 5, vt_ld = S + 16;
-    const int q_row = q0 + l32;
-    const uint32_t qrow = qbase + static_cast<uint32_t>(q_row * a.ldq);
-    const v4i qf[2] = {shared16(qb, qrow + 16 * h), shared16(qb, qrow + 32 + 16 * h)};
-    const int slot[2] = {((0 + h) ^ ((l32 >> 2) & 3)) * 16, ((2 + h) ^ ((l32 >> 2) & 3)) * 16};
+    const int S = s.S, nt = S / 32, vt_ld = S + 16, split = 1 << s.split_shift, w = x.wave & (split - 1), block = x.wave >> s.split_shift, blocks = kMostSplit >> s.split_shift;
+    const int l32 = x.lane & 31, h = x.lane >> 5;
+    const lds_ptr sVT = lds, sK = lds + 64 * vt_ld;
+    const lds_v4i sCtx = (lds_v4i)sK;                                   // [wave][8 groups of 4 registers][64]
+    const lds_f32 sMask = (lds_f32)(sK + attention_exchange(S, split)), sMax = sMask + S, sSum = sMax + 8 * 32 + block * 64 + x.lane;
+    const Buffer qb = make_buffer(x.place(s.q)), kb = make_buffer(x.place(s.k)), vb = make_buffer(x.place(s.v)), out = make_buffer(x.place(s.out));
+    const float* mask = s.has_mask ? reinterpret_cast<const float*>(x.place(s.mask)) : nullptr;
     constexpr float kLog2e = 1.4426950408889634f;
-    auto scores = [&](int t, float (&v)[16]) {
-        v16i acc = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const v4i kf = *(lds_v4i)(sK + (32 * t + l32) * 64 + slot[ks]);
-            acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf, qf[ks], acc, 0, 0, 0);
-        }
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            typedef float v4f __attribute__((ext_vector_type(4)));
-            v4f mk = {0.f, 0.f, 0.f, 0.f};
-            if (s.has_mask) mk = *(const __attribute__((address_space(3))) v4f*)(sMask + 32 * t + 8 * g + 4 * h);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                float y = static_cast<float>(acc[4 * g + j]) * a.scale1;
-                if (s.has_mask) y = y + mk[j];
-                v[4 * g + j] = y;
-            }
-        }
+    auto meet = [] {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
     };
-    float m = -INFINITY;
-    for (int t = 0; t < nt; ++t) {
-        float v[16];
-        scores(t, v);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) m = fmaxf(m, v[r]);
-    }
-    m = fmaxf(m, __shfl_xor(m, 32, 64));
-    const float mL = -m * kLog2e;
-    float sum = 0.f;
-    if constexpr (LONG) {
-        // the order of the stand-alone Softmax: four keys, the tiles t and t + 8, then tile bits 2, 1, 0 and g bits 1, 0
-        float b0[4] = {}, b1[4] = {}, b2[4] = {}, tile[4] = {};
-        for (int i = 0; i < 16; ++i) {                       // i = (bit 0, bit 1, bit 2, chunk) of the tile
-            const int t = (i >> 3) + 2 * ((i >> 2) & 1) + 4 * ((i >> 1) & 1) + 8 * (i & 1);
-            if (t < nt) {
-                float v[16];
-                scores(t, v);
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    tile[g] += (expf(v[4 * g] - m) + expf(v[4 * g + 1] - m)) + (expf(v[4 * g + 2] - m) + expf(v[4 * g + 3] - m));
-            }
-            auto carry = [](float (&from)[4], float (&to)[4]) {
-#pragma unroll
-                for (int g = 0; g < 4; ++g) { to[g] += from[g]; from[g] = 0.f; }
-            };
-            if ((i & 1) == 1) carry(tile, b2);
-            if ((i & 3) == 3) carry(b2, b1);
-            if ((i & 7) == 7) carry(b1, b0);
-        }
-        sum = (b0[0] + b0[2]) + (b0[1] + b0[3]);
-    } else {
-        for (int t = 0; t < nt; ++t) {
-            float v[16];
-            scores(t, v);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) sum += __builtin_amdgcn_exp2f(fmaf(v[r], kLog2e, mL));
-        }
-    }
-    sum += __shfl_xor(sum, 32, 64);
-    const float inv = 1.0f / sum;
-    v16i ctx[2] = {{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}};
-    if (a.p_bias) {
-#pragma unroll
-        for (int db = 0; db < 2; ++db)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const v4i sv = *(lds_v4i)(sVsum + 32 * db + 8 * g + 4 * h);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) ctx[db][4 * g + j] = sv[j] * a.p_bias;
-            }
-    }
-    for (int t = 0; t < nt; ++t) {
-        float v[16];
-        scores(t, v);
-        v4i pf;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            float p[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) p[j] = LONG ? quotient(expf(v[4 * g + j] - m), sum, inv) : __builtin_amdgcn_exp2f(fmaf(v[4 * g + j], kLog2e, mL)) * inv;
-            pf[g] = static_cast<int>(prob_levels4<true, PFORM>(a, p[0], p[1], p[2], p[3]));
-        }
-#pragma unroll
-        for (int db = 0; db < 2; ++db) {
-            const v4i vf = *(lds_v4i)(sVT + (32 * db + l32) * vt_ld + 32 * t + 16 * h);
-            ctx[db] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf, pf, ctx[db], 0, 0, 0);
-        }
-    }
-    const uint32_t orow = obase + static_cast<uint32_t>(q_row * a.ldo);
-#pragma unroll
-    for (int db = 0; db < 2; ++db)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int d = 32 * db + 8 * g + 4 * h;
-            const float4 o = make_float4(static_cast<float>(ctx[db][4 * g]) * a.scale2, static_cast<float>(ctx[db][4 * g + 1]) * a.scale2,
-                                         static_cast<float>(ctx[db][4 * g + 2]) * a.scale2, static_cast<float>(ctx[db][4 * g + 3]) * a.scale2);
-            if (a.fq_o.levels) publish4(out, orow + d, levels4(a.fq_o, o));
-            else publish16f(out, 4u * (orow + d), o);
-        }
-}
-
-__device__ __forceinline__ void attention_units(const ProgAttention& s, const Ctx& x, lds_ptr lds) {
-    const AttentionArgs& a = s.a;
-    const int S = s.S, vt_ld = S + 16;
-    lds_ptr sK = lds, sVT = lds + S * 64;
-    lds_i32 sVsum = (lds_i32)(sVT + 64 * vt_ld);
-    __attribute__((address_space(3))) float* sMask = (__attribute__((address_space(3))) float*)(sVsum + 64);
-    const Buffer qb = make_buffer(PROG_REF(x, s.q)), kb = make_buffer(PROG_REF(x, s.k)), vb = make_buffer(PROG_REF(x, s.v)), out = make_buffer(PROG_REF(x, s.out));
-    const float* mask = s.has_mask ? reinterpret_cast<const float*>(PROG_REF(x, s.mask)) : nullptr;
-    for (int u = x.rank; u < s.units; u += x.n_wg) {
-        const int eh = u / s.parts, part = u - eh * s.parts, n = eh / s.heads, hd = eh - n * s.heads;
+    bool first = true;
+    int u = x.rank;
+    do {
+        const int eh = min(u, s.units - 1) / s.parts, part = u - eh * s.parts, n = eh / s.heads, hd = eh - n * s.heads;
         const uint32_t kp = static_cast<uint32_t>(n * a.ok + hd * a.sk), vp = static_cast<uint32_t>(n * a.ov + hd * a.sv);
-        if (x.tid < 64) sVsum[x.tid] = 0;
-        __syncthreads();
-        for (int i = x.tid; i < S * 4; i += kProgramThreads) {          // S * 4 pieces of K; as many groups of 4 keys x 4 d of V
-            const int r = i >> 2, c = i & 3;
-            *(lds_v4i)(sK + r * 64 + ((c ^ ((r >> 2) & 3)) * 16)) = shared16(kb, kp + static_cast<uint32_t>(r * a.ldk + c * 16));
-        }
-        int32_t vsum[4] = {0, 0, 0, 0};
-        for (int i = x.tid; i < S * 4; i += kProgramThreads) {
-            const int d4 = i & 15, kq = i >> 4;
-            uint32_t w[4];
+        const int q0 = 32 * (part * blocks + block);
+        const bool on = q0 < S && block < blocks;
+        const uint32_t qbase = static_cast<uint32_t>(n * a.oq + hd * a.sq), obase = static_cast<uint32_t>(n * a.oo + hd * a.so);
+        const int q_row = min(q0, S - 32) + l32;
+        const float mk1 = mask ? mask[n * a.mask_outer + hd * a.mask_inner + min(x.tid, S - 1)] : 0.f;
+        if (first) x.wait();
+        first = false;
+        if (u >= s.units) return;
+        // K into LDS, V transposed into LDS: everything is requested before any of it is used
+        constexpr int kRounds = 4;              // S * 4 pieces of K, as many groups of 4 keys x 4 d of V, by 512 threads
+        v4i kx[kRounds];
+        uint32_t vw[kRounds][4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) w[q] = shared4(vb, vp + static_cast<uint32_t>((4 * kq + q) * a.ldv + 4 * d4));
-            const uint32_t lo01 = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u), hi01 = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u);
-            const uint32_t lo23 = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u), hi23 = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
+        for (int j = 0; j < kRounds; ++j) {
+            if (j * kProgramThreads >= S * 4) continue;
+            const int i = min(x.tid + j * kProgramThreads, S * 4 - 1), r = i >> 2, c = i & 3;      // (threads behind the end repeat the last piece)
+            kx[j] = shared16(kb, kp + static_cast<uint32_t>(r * a.ldk + c * 16));
+        }
+#pragma unroll
+        for (int j = 0; j < kRounds; ++j) {
+            if (j * kProgramThreads >= S * 4) continue;
+            const int i = min(x.tid + j * kProgramThreads, S * 4 - 1), d4 = i & 15, kq = i >> 4;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) vw[j][q] = shared4(vb, vp + static_cast<uint32_t>((4 * kq + q) * a.ldv + 4 * d4));
+        }
+        const uint32_t qrow = qbase + static_cast<uint32_t>(q_row * a.ldq);
+        const v4i qf[2] = {shared16(qb, qrow + 16 * h), shared16(qb, qrow + 32 + 16 * h)};
+        if (mask) sMask[min(x.tid, S - 1)] = mk1;
+#pragma unroll
+        for (int j = 0; j < kRounds; ++j) {
+            if (j * kProgramThreads >= S * 4) continue;
+            const int i = min(x.tid + j * kProgramThreads, S * 4 - 1), r = i >> 2, c = i & 3;
+            *(lds_v4i)(sK + r * 64 + ((c ^ ((r >> 2) & 3)) * 16)) = kx[j];
+        }
+#pragma unroll
+        for (int j = 0; j < kRounds; ++j) {
+            if (j * kProgramThreads >= S * 4) continue;
+            const int i = min(x.tid + j * kProgramThreads, S * 4 - 1), d4 = i & 15, kq = i >> 4;
+            const uint32_t* v = vw[j];
+            const uint32_t lo01 = __builtin_amdgcn_perm(v[1], v[0], 0x05010400u), hi01 = __builtin_amdgcn_perm(v[1], v[0], 0x07030602u);
+            const uint32_t lo23 = __builtin_amdgcn_perm(v[3], v[2], 0x05010400u), hi23 = __builtin_amdgcn_perm(v[3], v[2], 0x07030602u);
             const uint32_t t[4] = {__builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
                                    __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u)};
             const int key = 4 * kq, tile = key >> 5, in = key & 31;
             const int col = tile * 32 + ((in >> 2) & 1) * 16 + (in >> 3) * 4;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                *(__attribute__((address_space(3))) uint32_t*)(sVT + (4 * d4 + q) * vt_ld + col) = t[q];
-                vsum[q] = __builtin_amdgcn_sdot4(static_cast<int>(t[q]), 0x01010101, vsum[q], false);
+            for (int q = 0; q < 4; ++q) *(__attribute__((address_space(3))) uint32_t*)(sVT + (4 * d4 + q) * vt_ld + col) = t[q];
+        }
+        meet();
+        // the scores of this wave's tiles and their maximum
+        float v[kMostTiles][16];
+        float m = -INFINITY;
+        const int slot[2] = {((0 + h) ^ ((l32 >> 2) & 3)) * 16, ((2 + h) ^ ((l32 >> 2) & 3)) * 16};
+#pragma unroll
+        for (int j = 0; j < kMostTiles; ++j) {
+            const int t = w + (j << s.split_shift);
+            if (!on || t >= nt) continue;
+            v16i acc = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(*(lds_v4i)(sK + (32 * t + l32) * 64 + slot[ks]), qf[ks], acc, 0, 0, 0);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                v4f mk = {0.f, 0.f, 0.f, 0.f};
+                if (s.has_mask) mk = *(lds_v4f)(sMask + 32 * t + 8 * g + 4 * h);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float y = static_cast<float>(acc[4 * g + r]) * a.scale1;
+                    if (s.has_mask) y = y + mk[r];
+                    v[j][4 * g + r] = y;
+                    m = fmaxf(m, y);
+                }
             }
         }
-        if (a.p_bias) {
+        m = fmaxf(m, __shfl_xor(m, 32, 64));
+        if (split > 1) {
+            sMax[x.wave * 32 + l32] = m;            // (the same in both halves of the wave)
+            meet();
+            for (int k = 0; k < split; ++k) m = fmaxf(m, sMax[(block * split + k) * 32 + l32]);
+        }
+        // exponentials, and their sum: a lane's one behind the other (LONG: sums of four, and the tree over them of the stand-alone
+        // Softmax)
+        const float mL = -m * kLog2e;
+        const lds_v4f sE = (lds_v4f)sK + block * nt * 4 * 64 + x.lane;   // [tile][group of four][64]
+        const lds_f32 sE4 = (lds_f32)sK + block * nt * 4 * 64 + x.lane;
+        float sum = 0.f;
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                __hip_atomic_fetch_add(sVsum + 4 * (x.tid & 15) + q, vsum[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        for (int j = 0; j < kMostTiles; ++j) {
+            const int t = w + (j << s.split_shift);
+            if (!on || t >= nt) continue;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+#pragma unroll
+                for (int r = 4 * g; r < 4 * g + 4; ++r) {
+                    v[j][r] = LONG ? expf(v[j][r] - m) : __builtin_amdgcn_exp2f(fmaf(v[j][r], kLog2e, mL));
+                    if (!LONG) sum += v[j][r];
+                }
+                if constexpr (LONG) sE4[(4 * t + g) * 64] = (v[j][4 * g] + v[j][4 * g + 1]) + (v[j][4 * g + 2] + v[j][4 * g + 3]);
+                else if (split > 1) sE[(4 * t + g) * 64] = v4f{v[j][4 * g], v[j][4 * g + 1], v[j][4 * g + 2], v[j][4 * g + 3]};
+            }
         }
-        if (mask)
-            for (int i = x.tid; i < S; i += kProgramThreads) sMask[i] = mask[n * a.mask_outer + hd * a.mask_inner + i];
-        __syncthreads();
-        const int q0 = 32 * (part * s.waves + x.wave);
-        if (x.wave < s.waves && q0 < S) {
-            const uint32_t qbase = static_cast<uint32_t>(n * a.oq + hd * a.sq), obase = static_cast<uint32_t>(n * a.oo + hd * a.so);
-            if (S > kPlainSoftmax) attention_queries<true, 0>(s, qb, qbase, out, obase, q0, sK, sVT, sVsum, sMask, x.lane);
-            else if (s.pform == 2) attention_queries<false, 2>(s, qb, qbase, out, obase, q0, sK, sVT, sVsum, sMask, x.lane);
-            else attention_queries<false, 0>(s, qb, qbase, out, obase, q0, sK, sVT, sVsum, sMask, x.lane);
+        if (split > 1) {
+            meet();
+            if (on && w == 0) {
+                if constexpr (LONG) {
+                    float p[8][4];
+#pragma unroll
+                    for (int t = 0; t < 8; ++t)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            p[t][g] = sE4[(4 * t + g) * 64];
+                            if (t + 8 < nt) p[t][g] += sE4[(4 * (t + 8) + g) * 64];
+                        }
+#pragma unroll
+                    for (int o = 4; o > 0; o >>= 1)
+#pragma unroll
+                        for (int t = 0; t < o; ++t)
+#pragma unroll
+                            for (int g = 0; g < 4; ++g) p[t][g] += p[t + o][g];
+                    sum = (p[0][0] + p[0][2]) + (p[0][1] + p[0][3]);
+                } else {
+                    sum = 0.f;
+                    for (int t = 0; t < nt; ++t)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            const v4f e = sE[(4 * t + g) * 64];
+                            sum += e.x; sum += e.y; sum += e.z; sum += e.w;
+                        }
+                }
+                sSum[0] = sum;
+            }
+            meet();
+            sum = sSum[0];
+        } else meet();                          // (K's last readers are through)
+        sum += __shfl_xor(sum, 32, 64);
+        const float inv = 1.0f / sum;
+        // probabilities -> levels -> this wave's part of the second product
+        v16i ctx[2] = {{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}};
+#pragma unroll
+        for (int j = 0; j < kMostTiles; ++j) {
+            const int t = w + (j << s.split_shift);
+            if (!on || t >= nt) continue;
+            v4i pf = {0, 0, 0, 0};
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                float p[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) p[r] = LONG ? quotient(v[j][4 * g + r], sum, inv) : v[j][4 * g + r] * inv;
+                pf[g] = static_cast<int>(prob_levels4<true, PFORM>(a, p[0], p[1], p[2], p[3]));
+            }
+            // u8 probabilities q are stored as q - 128: the 128 that is missing from each, as twice 64
+            const int n64 = a.p_bias ? 0x40404040 : 0;
+            const v4i bias = {n64, n64, n64, n64};
+#pragma unroll
+            for (int db = 0; db < 2; ++db) {
+                const v4i vf = *(lds_v4i)(sVT + (32 * db + l32) * vt_ld + 32 * t + 16 * h);
+                ctx[db] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf, pf, ctx[db], 0, 0, 0);
+                if (a.p_bias) {
+                    ctx[db] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf, bias, ctx[db], 0, 0, 0);
+                    ctx[db] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf, bias, ctx[db], 0, 0, 0);
+                }
+            }
         }
-        __syncthreads();
-    }
+        // the waves' integer sums meet; each finishes 8 / split groups of four registers
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            sCtx[(x.wave * 8 + i) * 64 + x.lane] = v4i{ctx[i >> 2][4 * (i & 3)], ctx[i >> 2][4 * (i & 3) + 1], ctx[i >> 2][4 * (i & 3) + 2], ctx[i >> 2][4 * (i & 3) + 3]};
+        meet();
+        if (on) {
+            const uint32_t orow = obase + static_cast<uint32_t>(q_row * a.ldo);
+            for (int i = w; i < 8; i += split) {
+                v4i c = {0, 0, 0, 0};
+                for (int k = 0; k < split; ++k) c += sCtx[((block * split + k) * 8 + i) * 64 + x.lane];
+                const int d = 32 * (i >> 2) + 8 * (i & 3) + 4 * h;
+                const float4 o = make_float4(static_cast<float>(c.x) * a.scale2, static_cast<float>(c.y) * a.scale2, static_cast<float>(c.z) * a.scale2,
+                                             static_cast<float>(c.w) * a.scale2);
+                if (a.fq_o.levels) publish4(out, orow + d, levels4(a.fq_o, o));
+                else publish16f(out, 4u * (orow + d), o);
+            }
+        }
+        u += x.n_wg;
+        if (u < s.units) meet();
+    } while (u < s.units);
 }
 
 __device__ __forceinline__ int lane_index() { return static_cast<int>(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u))); }
@@ -1349,7 +1403,7 @@ __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgA
         x.tid = 64 * x.wave + lane;
         const StepPtr words = step_ptr(g.steps, step);
         const int kind = static_cast<int>(word_of(x.words, 0));
-        if (kind != PK_CONV && kind != PK_DW && kind != PK_MVN) x.wait();
+        if (kind != PK_CONV && kind != PK_DW && kind != PK_MVN && kind != PK_ATTENTION) x.wait();      // (those wait when they have prepared)
         switch (kind) {
         case PK_CONV: {
             switch (PROG_FIELD(x.words, a) * 8 + PROG_FIELD(x.words, b) + (PROG_FIELD(x.words, nk2) ? 64 : 0)) {
@@ -1382,7 +1436,12 @@ __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgA
             if constexpr (ENCODER) {
                 if (kind == PK_EMBED) embed_rows(unpack<ProgEmbed>(words), x);
                 else if (kind == PK_MVN) mvn_rows(unpack<ProgMvn>(words), x);
-                else attention_units(unpack<ProgAttention>(words), x, lds);
+                else {
+                    const ProgAttention t = unpack<ProgAttention>(words);
+                    if (t.S > kPlainSoftmax) attention_units<true, 0>(t, x, lds);
+                    else if (t.pform == 2) attention_units<false, 2>(t, x, lds);
+                    else attention_units<false, 0>(t, x, lds);
+                }
             } else if (kind == PK_DW) {
                 switch (PROG_FIELD(x.words, stride) * 8 + PROG_FIELD(x.words, group)) {
                 case 8 + 1: dw_items<1, 1>(x); break;
@@ -1719,7 +1778,7 @@ bool ProgBuilder::attention(const hipie_attention* att, const void* const (&qkv)
     for (int i = 0; i < 3; ++i)
         if (batch_outer * outer[i] + batch * inner[i] + proto.S * ld[i] >= kBeyond) return false;
     if (4 * (batch_outer * oo + batch * so + proto.S * ldo) >= kBeyond) return false;
-    if (proto.S * 64 + 64 * (proto.S + 16) + 256 + 4 * proto.S > kPartBytes) return false;
+    if (proto.S > 512 || proto.S % 32 != 0 || proto.S < 32) return false;
     ProgAttention s{};
     s.kind = PK_ATTENTION;
     rows_kinds = true;
@@ -1737,22 +1796,26 @@ bool ProgBuilder::attention(const hipie_attention* att, const void* const (&qkv)
     s.a.ldo = ldo; s.a.so = so; s.a.oo = oo;
     s.a.mask_inner = 0;
     s.a.mask_outer = proto.S;
-    // queries per workgroup: rounds x (staging, about 4 clocks a key + a wave's 20 instructions per score, two waves to a
-    // SIMD from five on).  Against the best of 1 .. 8 waves the choice costs an encoder of two layers 0 - 4 % of its time
-    // (1 to 4 sequences of 32 to 512 keys, 64 and 256 workgroups).
+    // Waves per 32 queries, by the clocks of a workgroup's round: staging, and the chain of a wave's tiles (from five waves on two
+    // share a SIMD).  Against the best of the four splits the choice costs an encoder of two layers 0 - 1 % of its time (1 to 4
+    // sequences of 32 to 512 keys, 64 and 256 workgroups).
     const int qt = proto.S / 32;
     const int64_t elements = static_cast<int64_t>(batch_outer) * batch;
     double best = 1e30;
-    for (int w = 1; w <= 8; ++w) {
-        const int64_t parts = ceil_div(qt, w), rounds = ceil_div(elements * parts, workgroups);
-        const double t = static_cast<double>(rounds) * (1500.0 + 4.0 * proto.S + (w > 4 ? 1.7 : 1.0) * qt * 16 * 20 * 4);
+    for (int shift = 0; (1 << shift) <= kMostSplit; ++shift) {
+        const int split = 1 << shift, blocks = std::min(kMostSplit / split, qt);
+        const int64_t tiles = ceil_div(qt, split), parts = ceil_div(qt, kMostSplit / split), rounds = ceil_div(elements * parts, workgroups);
+        if (tiles > kMostTiles || attention_lds(proto.S, split) > kPlainAt) continue;
+        const double waves = static_cast<double>(blocks * std::min(split, qt));
+        const double t = static_cast<double>(rounds) * (5000.0 + 4.0 * proto.S + std::max(1.0, waves / 5.0) * static_cast<double>(tiles) * 2400.0);
         if (t < best) {
             best = t;
-            s.waves = w;
+            s.split_shift = shift;
             s.parts = static_cast<int32_t>(parts);
             s.units = static_cast<int32_t>(elements * parts);
         }
     }
+    if (best >= 1e30) return false;
     add(s);
     return true;
 }

@@ -29,6 +29,9 @@ GRAPHS = {
     "encoder_1x32": lambda: builders.bert_encoder(layers=1, batch=1, seq=32, vocab=100, mask=True)[0],
     "encoder_3x96": lambda: builders.bert_encoder(layers=1, batch=3, seq=96, vocab=0, mask=False)[0],
     "encoder_1x512": lambda: builders.bert_encoder(layers=1, batch=1, seq=512, vocab=100, mask=True)[0],
+    "encoder_1x160": lambda: builders.bert_encoder(layers=1, batch=1, seq=160, vocab=100, mask=True)[0],       # five tiles of keys for eight waves
+    "encoder_4x128": lambda: builders.bert_encoder(layers=1, batch=4, seq=128, vocab=100, mask=True)[0],       # two waves for 32 queries (64 workgroups)
+    "encoder_1x448": lambda: builders.bert_encoder(layers=1, batch=1, seq=448, vocab=100, mask=True)[0],
     "encoder_2x384": lambda: builders.bert_encoder(layers=1, batch=2, seq=384, vocab=100, mask=True)[0],
 }
 
