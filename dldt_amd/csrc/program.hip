@@ -1407,10 +1407,9 @@ __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgA
         switch (kind) {
         case PK_CONV: {
             switch (PROG_FIELD(x.words, a) * 8 + PROG_FIELD(x.words, b) + (PROG_FIELD(x.words, nk2) ? 64 : 0)) {
-            case 8 + 4: conv_tiles<ENCODER, 1, 4>(x, lds); break;
+            case 8 + 1: conv_tiles<ENCODER, 1, 1>(x, lds); break;
             case 16 + 1: conv_tiles<ENCODER, 2, 1>(x, lds); break;
             case 16 + 2: conv_tiles<ENCODER, 2, 2>(x, lds); break;
-            case 16 + 4: conv_tiles<ENCODER, 2, 4>(x, lds); break;
             case 32 + 2: conv_tiles<ENCODER, 4, 2>(x, lds); break;
             case 64 + 16 + 2:
                 if constexpr (!ENCODER) conv_tiles<ENCODER, 2, 2, true>(x, lds);
@@ -1487,37 +1486,39 @@ __global__ void clear_words(uint32_t* p, int n) {
 }
 
 // Tile shape of a convolution step, by the clocks its busiest compute unit takes.  The constants are fitted, not derived: to
-// the time of whole networks with one class of layers at a time in each of the 24 shapes (188 classes of ResNet-50,
-// MobileNetV2, encoders and the convolution block, at 64, 128 and 256 workgroups), so that the choice loses as little as
-// possible against the best shape of every class.  Summed over a network's classes that is 0.1 - 6 % of its time (MobileNetV2,
-// whose 20 classes hardly tell the shapes apart from the runs' scatter of a microsecond, at 256 workgroups 16 %), where the
-// constants before lost 1 - 18 %: ResNet-50 at batch 1 took 290 us with those and 277 with these.
+// the time of whole networks with one class of layers at a time in each of the shapes (184 classes of ResNet-50 at batch 1, 3 and
+// 7, MobileNetV2 at 1 and 4, encoders and the convolution block, at 64, 128 and 256 workgroups), so that the choice loses as
+// little as possible against the best shape of every class: summed over a network's classes 1 - 10 % of its time, of which 1 -
+// 8 % is what the best of thirty noisy times lies too low, where the constants before lost 3 - 14 %.  Of the other shapes that were
+// measured (1 x 2, 1 x 4, 2 x 4 of fragments) none is the best of a class by more than the runs differ.
 // What the terms stand for: a load of 1 KB on a unit's path, a matrix instruction, a round trip to memory per filled ring, the
 // f32 chain per value, a store instruction, the partial sums of the waves that share a K in LDS.  Rounds are tiles a wave takes
 // one after another.
 struct TileChoice { int a, b, ks; };
 TileChoice choose_tile(int workgroups, int oc, int64_t pixels, int nk, int nk2, bool gelu) {
-    static constexpr int kShapes[6][2] = {{4, 4}, {4, 2}, {2, 4}, {2, 2}, {2, 1}, {1, 4}};
+    static constexpr int kShapes[6][2] = {{4, 4}, {4, 2}, {2, 2}, {2, 1}, {1, 1}, {2, 4}};
     TileChoice best{4, 4, 1};
     double best_t = 1e30;
     for (const auto& shape : kShapes)
         for (int ks : {1, 2, 4, 8}) {
             const int a = shape[0], b = shape[1];
-            if ((nk2 && (a != 2 || b < 2)) || (gelu && a == 1) || (b == 4 && ks == 8)) continue;
+            if ((nk2 && (a != 2 || b < 2)) || (gelu && a == 1) || (b == 4 && (ks == 8 || (a == 2 && !nk2)))) continue;
             const int depth = a * b >= 16 ? 2 : (a * b >= 8 ? 4 : 6);
             const int64_t tiles = ceil_div(oc, 16 * a) * ceil_div(pixels, 16 * b), per_wg = ceil_div(tiles, workgroups);
             const int64_t rounds = ceil_div(per_wg, 8 / ks);
             const double waves = std::min<double>(8.0, static_cast<double>(per_wg) * ks / static_cast<double>(rounds));   // of a workgroup, busy
             auto loop = [&](int steps) {
                 const double n = static_cast<double>(ceil_div(steps, ks));
-                const double rate = std::max(waves * (a + b) * 13.0, std::max(1.0, waves / 4.0) * a * b * 19.0 + 7.0);
-                return std::max(n * rate, std::ceil(n / depth) * 600.0) + 1485.0;
+                const double rate = std::max(waves * (a + b) * 11.4, std::max(1.0, waves / 4.0) * a * b * 14.6 + 2.7);
+                return std::max(n * rate, std::ceil(n / depth) * 431.0) + 1368.0;
             };
-            const double columns = std::ceil(static_cast<double>(b) / ks), writers = waves / ks * std::min(ks, b);
-            const double chain = (gelu ? 20.0 : 2.9) * 4 * a + 90.0;
-            const double epi = columns * (chain * std::max(8.0, writers) + 4 * 44.0 * writers);
-            const double meet = ks > 1 ? 195.0 + 112.0 * ks * a * columns : 0.0;
-            const double t = static_cast<double>(rounds) * (loop(nk) + (nk2 ? loop(nk2) : 0.0) + epi + meet + 1240.0);
+            // a wave finishes whole columns of four pixels a lane, or part of one
+            const double rows = b == 4 ? 4.0 : std::min(4.0, std::max(1.0, 4.0 * b / ks)), columns = std::max(1.0, std::ceil(static_cast<double>(b) / ks));
+            const double writers = waves / ks * std::min(ks, b == 4 ? 4 : 4 * b);
+            const double chain = (gelu ? 74.3 : 2.6) * rows * a + 376.0;
+            const double epi = columns * (chain * std::max(5.8, writers) + rows * 10.6 * writers);
+            const double meet = ks > 1 ? 354.0 + 67.6 * (waves * a * b / 8.0 + ks * a * columns * rows / 4.0) : 0.0;
+            const double t = static_cast<double>(rounds) * (loop(nk) + (nk2 ? loop(nk2) : 0.0) + epi + meet + 1224.0) + 248.0 * static_cast<double>(rounds - 1);
             if (t < best_t) {
                 best_t = t;
                 best = {a, b, ks};

@@ -75,9 +75,8 @@ def test_single_launch_equals_steps(name):
             assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
 
 
-# 256 workgroups meet through the XCDs, the others at one counter.  Together these choose every tile instance of the kernel:
-# 1 x 4 in the blocks of 2x256x14 (64 workgroups) and 7x128x14 (128), 2 x 4 in resnet_7_u8 (64, as the pair with a projection
-# shortcut too), 2 x 1, 2 x 2, 4 x 2, 4 x 4 and the 2 x 2 pair in the networks
+# Together these choose every tile instance of the kernels (fragments of 16 channels x fragments of 16 pixels) and every way a
+# tile's waves share its chain
 @pytest.mark.parametrize("workgroups", [64, 128, 256])
 @pytest.mark.parametrize("name", sorted(GRAPHS))
 def test_every_size_runs_and_equals_steps(name, workgroups):
