@@ -2264,12 +2264,13 @@ static int64_t fill_conv_args(const hipie_conv* c, const hipie_tensor* in, const
 }
 
 static int conv_run(const hipie_conv* c, const hipie_tensor* in, const hipie_tensor* residual,
-                    const hipie_tensor* out, void* stream, bool static_scratch_only) {
+                    const hipie_tensor* out, void* stream, bool static_scratch_only, void* planes = nullptr) {
     return guarded([&] {
         ConvArgs a;
         int32_t oh, ow;
         const int64_t M = fill_conv_args(c, in, residual, out, a, oh, ow);
         if (M == 0) return;
+        if (planes) planes_arguments(a, planes);
         const hipie_conv_desc& d = c->d;
         if (c->depthwise) {
             HIPIE_REQUIRE(in->stride_w >= d.ic && in->stride_w % 16 == 0, HIPIE_PARAMETER_MISMATCH,
@@ -2493,6 +2494,23 @@ int hipie_conv_run_static(const hipie_conv* c, const hipie_tensor* in, const hip
 }
 
 }  // extern "C"
+
+void hipie::planes_arguments(ConvArgs& a, void* planes) {
+    a.out = planes;
+    a.out_plane = a.OHOW;
+    a.out_sn = a.OC * a.OHOW;
+    a.out_sh = a.OW;
+    a.out_sw = 1;
+    a.flat_out = a.OC == 1 || a.M == a.OHOW;      // (one image, or one channel: pixel m sits at m)
+}
+
+bool hipie::conv_takes_planes(const hipie_conv* c, int64_t n, int64_t oh, int64_t ow) {
+    return !c->depthwise && !c->fused && c->epi.out_dtype == HIPIE_F32 && !(c->epi.flags & CF_RES) && n * c->d.oc * oh * ow < (1ll << 31);
+}
+
+int hipie::conv_run_planes(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor& out, void* planes, hipStream_t s) {
+    return conv_run(c, &in, nullptr, &out, s, false, planes);
+}
 
 bool hipie::conv_launch_arguments(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out, ConvLaunch& l) {
     int32_t oh, ow;

@@ -107,6 +107,7 @@ struct ConvArgs {
     int32_t conv_sh, conv_sw;        // convolution strides
     int32_t in_origin;               // -(pad_top * in_sh + pad_left * in_sw)
     int32_t out_sn, out_sh, out_sw;  // output strides in elements
+    int32_t out_plane;               // f32 results stored channel by channel (NCHW, out_sw = 1): elements from one plane to the next; 0: channels innermost
     int32_t res_sn, res_sh, res_sw;  // residual strides in elements
     int32_t OC, OCp;
     int32_t nk;                      // Kp / 64

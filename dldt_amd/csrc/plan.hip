@@ -204,6 +204,11 @@ struct ConvStep : Step {
     // run inside this step's kernel when the fused form applies, else right before it
     std::unique_ptr<ConvStep> shortcut;
     bool fused = false;
+    // the graph's result that this step's f32 output is, and nothing else reads: it goes straight into the caller's buffer (-1: none)
+    int result = -1;
+    // ... which the layer's kernels can write; the values of single pixels ([N, C]) are a row each either way, their copy is no
+    // transposition and goes away in the single launch only
+    bool writes_result = false, direct = false;
     float tuned_us = 0.f;          // per launch with every tuning lane busy, of the variant the tuner kept (0: not tuned)
     ~ConvStep() override { hipie_conv_destroy(conv); }
     void fill_desc(const std::vector<TensorInfo>& tensors) {
@@ -241,11 +246,18 @@ struct ConvStep : Step {
         }
         weights.clear();
         weights.shrink_to_fit();
+        const TensorInfo& t = tensors[out];
+        writes_result = result >= 0 && !shortcut && res < 0 && res_param < 0 && conv_takes_planes(conv, t.n, t.h, t.w);
+        direct = writes_result && t.h * t.w > 1;
     }
     void run(uint8_t* arena, const std::vector<TensorInfo>& tensors, void* const* inputs, void* const* outputs,
              hipStream_t s) const override {
         const hipie_tensor i = tensors[in].desc(arena), o = tensors[out].desc(arena);
         hipie_tensor r{};
+        if (direct) {
+            check_status(conv_run_planes(conv, i, o, outputs[result], s), name.c_str());
+            return;
+        }
         if (fused) {
             r = tensors[shortcut->in].desc(arena);
         } else {
@@ -258,6 +270,7 @@ struct ConvStep : Step {
     bool program(ProgBuilder& b, const std::vector<TensorInfo>& tensors, void* const* inputs, void* const* outputs) const override {
         const hipie_tensor i = tensors[in].desc(b.fake_arena()), o = tensors[out].desc(b.fake_arena());
         hipie_tensor r{};
+        if (writes_result) return b.conv(conv, i, nullptr, o, outputs[result]);
         if (fused) {
             r = tensors[shortcut->in].desc(b.fake_arena());
         } else {
@@ -322,8 +335,9 @@ struct ConvStep : Step {
         const bool has_res = fused || res >= 0 || res_param >= 0;
         auto launch_all = [&](int times) {
             for (int w = 0; w < times; ++w)
-                for (size_t l = 0; l < nl; ++l)
-                    check_status(hipie_conv_run(conv, &ti[l], has_res ? &tr[l] : nullptr, &to[l], lanes[l].stream), name.c_str());
+                for (size_t l = 0; l < nl; ++l)      // (a direct result lands in the tensor's own place, which nothing else uses)
+                    check_status(direct ? conv_run_planes(conv, ti[l], to[l], to[l].data, lanes[l].stream)
+                                        : hipie_conv_run(conv, &ti[l], has_res ? &tr[l] : nullptr, &to[l], lanes[l].stream), name.c_str());
         };
         std::vector<hipEvent_t> e0(nl), e1(nl);
         for (size_t l = 0; l < nl; ++l) {
@@ -701,6 +715,9 @@ struct EltwiseStep : Step {
 struct ExitStep : Step {
     int in = -1, result_index = 0, C = 0;
     bool out_u8 = false;
+    const ConvStep* writer = nullptr;      // the step that writes the result itself where it can (ConvStep::direct)
+    bool done() const { return writer && writer->direct; }
+    int launches() const override { return done() ? 0 : 1; }
     std::vector<float> sub, mul;
     DeviceBuffer d_sub, d_mul;
     void create(int device, const std::vector<TensorInfo>&) override {
@@ -729,10 +746,11 @@ struct ExitStep : Step {
         return a;
     }
     bool program(ProgBuilder& b, const std::vector<TensorInfo>& tensors, void* const*, void* const* outputs) const override {
-        return b.exit(arguments(b.fake_arena(), tensors, outputs), tensors[in].dtype);
+        return (writer && writer->writes_result) || b.exit(arguments(b.fake_arena(), tensors, outputs), tensors[in].dtype);
     }
     void run(uint8_t* arena, const std::vector<TensorInfo>& tensors, void* const*, void* const* outputs,
              hipStream_t s) const override {
+        if (done()) return;
         launch_exit(arguments(arena, tensors, outputs), tensors[in].dtype, s);
         HIPIE_CHECK_HIP(hipGetLastError());
     }
@@ -2914,6 +2932,14 @@ struct Planner {
         st->out_u8 = x.kind == VK_TENSOR && tensors[x.tensor].esize() == 1;
         for (size_t i = 0; i < g.results.size(); ++i)
             if (g.results[i] == id) st->result_index = static_cast<int>(i);
+        // an f32 result that only the caller reads: its producer stores it there, in the caller's layout (HIPIE_KEEP_F32 keeps
+        // it where hipie_request_tensor finds it, and copies)
+        if (x.kind == VK_TENSOR && tensors[x.tensor].dtype == HIPIE_F32 && N(n.in[0]).users.size() == 1 && !keep_f32)
+            for (auto& step : steps)
+                if (auto* conv = dynamic_cast<ConvStep*>(step.get()); conv && conv->out == x.tensor && conv->out_node == n.in[0]) {
+                    conv->result = st->result_index;
+                    st->writer = conv;
+                }
         st->name = n.name;
         st->type = "Result";
         st->bytes = n.numel() * 5;
@@ -4141,6 +4167,10 @@ int hipie_request_tensor(const hipie_request* r, int node_id, hipie_tensor* t) {
             if (auto* pair = dynamic_cast<const PairStep*>(st.get()))
                 HIPIE_REQUIRE(!(pair->fused && pair->first->out == it->second), HIPIE_NOT_FOUND,
                               "hipie_request_tensor: node %d lives in LDS only (two convolutions run as one kernel)", node_id);
+        for (const auto& st : r->plan->steps)
+            if (auto* conv = dynamic_cast<const ConvStep*>(st.get()))
+                HIPIE_REQUIRE(!(conv->direct && conv->out == it->second), HIPIE_NOT_FOUND, "hipie_request_tensor: node %d is a result, stored in the caller's buffer only",
+                              node_id);
         *t = r->plan->tensors[it->second].desc(r->arena.as<uint8_t>());
     });
 }

@@ -62,7 +62,7 @@ struct ProgConv {
     float clamp_lo, clamp_hi;
     // depthwise
     int32_t stride, group, c4, quads, OH, OW, items;
-    int32_t in_sn, in_sh, in_sw, row_sh, out_sn, out_sh, out_sw, res_sn, res_sh, res_sw;
+    int32_t in_sn, in_sh, in_sw, row_sh, out_sn, out_sh, out_sw, res_sn, res_sh, res_sw;      // (dense: out_sn = bytes between the planes of f32 results, 0: channels innermost)
     float inv_c4, inv_quads, inv_OH;
 };
 struct ProgEntry {
@@ -129,7 +129,8 @@ struct ProgBuilder {
         std::memcpy(w.data(), &s, sizeof(T));
         steps.push_back(w);
     }
-    bool conv(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out);
+    // planes: the f32 results channel by channel at this address instead (conv_run_planes)
+    bool conv(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out, void* planes = nullptr);
     bool entry(const hipie_fq* fq, bool u8_in, const void* in, const hipie_tensor& out);
     bool pool(const PoolArgs& a, bool avg, bool rcp);
     bool exit(const ExitArgs& a, int in_dtype);

@@ -357,7 +357,9 @@ struct StepConstants {
     float lm1, clamp_lo, clamp_hi;
     uint32_t off_bytes;                      // the level offset, four times
     int out_limit, res_limit;
+    uint32_t plane;                          // bytes between the planes of f32 results; 0: channels innermost
 };
+template <bool DENSE>
 __device__ __forceinline__ StepConstants step_constants(const Ctx& x) {
     StepConstants s;
     s.flags = PROG_FIELD(x.words, flags);
@@ -369,6 +371,7 @@ __device__ __forceinline__ StepConstants step_constants(const Ctx& x) {
     s.off_bytes = PROG_FIELD(x.words, off_bytes);
     s.out_limit = PROG_FIELD(x.words, out_limit);
     s.res_limit = PROG_FIELD(x.words, res_limit);
+    s.plane = DENSE ? static_cast<uint32_t>(PROG_FIELD(x.words, out_sn)) : 0u;
     return s;
 }
 
@@ -464,6 +467,15 @@ __device__ __forceinline__ void finish(const StepConstants& c, const ChannelCons
 #pragma unroll
             PROG_EACH x[a][r] = gelu_one(x[a][r]);
         }
+    if (!(fl & CF_OUT_FQ) && c.plane != 0) {
+#pragma unroll
+        for (int a = 0; a < A; ++a) {
+            const uint32_t o = oc + a < c.out_limit ? static_cast<uint32_t>(oc + a) * c.plane : static_cast<uint32_t>(kBeyond);
+#pragma unroll
+            for (int r = 0; r < R; ++r) publish4(c.out, q.out[r] + o, __float_as_uint(x[a][r] + 0.f));
+        }
+        return;
+    }
     if (!(fl & CF_OUT_FQ)) {
         const uint32_t o = oc < c.out_limit ? static_cast<uint32_t>(4 * oc) : static_cast<uint32_t>(kBeyond);
 #pragma unroll
@@ -601,7 +613,7 @@ __device__ __forceinline__ void conv_tiles(Ctx& x, lds_ptr lds) {
     }
     const uint32_t tiles = static_cast<uint32_t>(PROG_FIELD(x.words, tiles));
     const int t0 = static_cast<int>((static_cast<uint32_t>(x.rank) * tiles) >> x.wg_shift), t1 = static_cast<int>((static_cast<uint32_t>(x.rank + 1) * tiles) >> x.wg_shift);
-    const StepConstants sc = step_constants(x);
+    const StepConstants sc = step_constants<true>(x);
     const int M = PROG_FIELD(x.words, M);
     const uint32_t* pix = PROG_TABLE_OF(uint32_t, x.words, pixels);
     const lds_v4i part = (lds_v4i)lds + x.wave * (F * 64) + x.lane;
@@ -732,7 +744,7 @@ __device__ __forceinline__ void dw_items(Ctx& x) {
     const int res_sn = PROG_FIELD(x.words, res_sn), res_sh = PROG_FIELD(x.words, res_sh), res_sw = PROG_FIELD(x.words, res_sw);
     const float inv_c4 = PROG_FIELD(x.words, inv_c4), inv_quads = PROG_FIELD(x.words, inv_quads), inv_OH = PROG_FIELD(x.words, inv_OH);
     const Buffer in = make_buffer(PROG_PLACE(x, in));
-    const StepConstants sc = step_constants(x);
+    const StepConstants sc = step_constants<false>(x);
     const int8_t* wgt = PROG_TABLE_OF(int8_t, x.words, wgt);
     const uint8_t* constants = PROG_TABLE_OF(uint8_t, x.words, constants);
     const bool f32 = sc.flags & CF_RES_F32, fo = !(sc.flags & CF_OUT_FQ);
@@ -1560,9 +1572,10 @@ ProgPtr ProgBuilder::keep(const void* host, size_t bytes) {
     return ptr(owned.back().ptr);
 }
 
-bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out) {
+bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out, void* planes) {
     ConvLaunch l;
     if (!conv_launch_arguments(conv, in, residual, out, l)) return false;
+    if (planes) planes_arguments(l.a, planes);
     const ConvArgs& a = l.a;
     const int64_t M = a.M;
     if (M > (1 << 20) || a.koff_tile || (a.flags & CF_OUT_I32) || ((a.flags & CF_OUT_FQ) && !(a.flags & CF_FQ_RCP)) || (a.flags & (CF_RES_SUB | CF_POST_SCALE)))
@@ -1575,7 +1588,8 @@ bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hip
     c.out = ref(a.out);
     c.res = a.res ? ref(a.res) : ProgRef{-2, 0, 0};
     c.in2 = ProgRef{-2, 0, 0};
-    c.out_limit = a.out_sw;
+    const int channels = planes ? a.OC : a.out_sw;       // that the output holds
+    c.out_limit = channels;
     c.res_limit = a.res_sw;
     {   // the tables the flags ask for, in load_constants' order
         const uint32_t fl = a.flags;
@@ -1618,6 +1632,7 @@ bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hip
         return true;
     }
     c.kind = PK_CONV;
+    if (planes) c.out_sn = 4 * a.out_plane;
     c.nk = a.nk;
     const bool pair = (a.flags & CF_RES_GEMM) != 0;
     if (a.flags & CF_GELU) rows_kinds = true;
@@ -1626,7 +1641,7 @@ bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hip
     const TileChoice t = choose_tile(workgroups, a.OC, M, a.nk, pair ? a.nk2 : 0, (a.flags & CF_GELU) != 0);
     c.a = t.a; c.b = t.b; c.ks_shift = __builtin_ctz(static_cast<unsigned>(t.ks));
     // (the channels the tensor is padded with are written too)
-    const int o_tiles = static_cast<int>(ceil_div(std::min(a.out_sw, a.OCp), 16 * t.a));
+    const int o_tiles = static_cast<int>(ceil_div(std::min(channels, a.OCp), 16 * t.a));
     c.p_tiles = static_cast<int32_t>(ceil_div(M, 16 * t.b));
     c.inv_p_tiles = 1.0f / static_cast<float>(c.p_tiles);
     const int64_t tiles = static_cast<int64_t>(c.p_tiles) * o_tiles;

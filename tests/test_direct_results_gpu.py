@@ -1,0 +1,76 @@
+"""A convolution whose f32 values are the graph's result stores them into the caller's [N, C, H, W] buffer itself: every kernel
+variant the layer has and the single launch, against the copy kernel behind the same convolution (HIP_KEEP_F32), bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from dldt_amd import HipieError, builders
+
+pytestmark = pytest.mark.gpu
+VARIANTS = [*range(24), 24 + 32]
+
+
+def _graph(relu, results):
+    """a convolution whose f32 value is `results` results"""
+    rng = np.random.default_rng(3)
+    q = builders.QuantizedNet()
+    x = q.input("data", (2, 20, 11, 11), 2.55)
+    y = q.conv_f32(x, rng.standard_normal((37, 20, 3, 3), dtype=np.float32) * np.float32(0.05), rng.standard_normal(37, dtype=np.float32), pads=(1, 1), relu=relu)
+    for k in range(results):
+        q.g.result(y, "out%d" % k)
+    return q.g
+
+
+def _run(plan, x, offset=0):
+    req = plan.create_request()
+    ins, outs = req.device_buffers()
+    ins[0].copy_(x)
+    place = [torch.full((o.numel() + 8,), float("nan"), device="cuda")[offset:offset + o.numel()].view(o.shape) for o in outs]
+    torch.cuda.synchronize()
+    req.enqueue(ins, place)
+    torch.cuda.synchronize()
+    return [p.cpu().numpy().view(np.uint32) for p in place]
+
+
+@pytest.mark.parametrize("n,c,hw,oc", [(1, 3, 7, 8), (2, 17, 9, 65), (3, 64, 14, 70), (1, 64, 33, 129), (5, 128, 8, 3), (2, 32, 1, 1)])
+def test_every_variant_stores_the_planes_that_the_copy_stores(tmp_path, n, c, hw, oc):
+    g = builders.conv_block(n=n, c=c, hw=hw, oc=oc)[0]
+    x = torch.rand((n, c, hw, hw), generator=torch.Generator(device="cuda").manual_seed(1), device="cuda") * 2.55
+    kept = g.compile(0, config={"HIP_KEEP_F32": "YES", "HIP_TUNE": "NO"})
+    want = _run(kept, x)
+    plan = g.compile(0, config={"HIP_TUNE": "NO"})
+    types = [s["type"] for s in plan.steps]
+    assert int(plan.step_rt_info(len(types) - 1, "kernels")) == (0 if hw > 1 else 1)
+    ran = 0
+    for v in VARIANTS:
+        path = tmp_path / str(v)
+        path.write_text("".join("%d %d\n" % (i, v if t.startswith("Convolution") else -1) for i, t in enumerate(types)))
+        try:
+            plan = g.compile(0, config={"HIP_TUNE_FILE": str(path), "HIP_SINGLE_LAUNCH": "NO"})
+        except HipieError:
+            continue                                          # a variant this layer does not have
+        for offset in (0, 1):                                 # (a buffer on a 4-byte boundary only)
+            got = _run(plan, x, offset)
+            assert np.array_equal(got[0], want[0]), (v, offset)
+        ran += 1
+    assert ran >= 3
+    single = g.compile(0, config={"HIP_TUNE": "NO", "HIP_THROUGHPUT_STREAMS": "1", "HIP_SINGLE_LAUNCH": "256"})
+    req = single.create_request()
+    ins, outs = req.device_buffers()
+    ins[0].copy_(x)
+    torch.cuda.synchronize()
+    req.infer_device(ins, outs)
+    assert np.array_equal(outs[0].cpu().numpy().view(np.uint32), want[0])
+
+
+@pytest.mark.parametrize("relu", [False, True])
+@pytest.mark.parametrize("results", [1, 2])
+def test_values_without_an_activation_and_with_two_results(relu, results):
+    x = torch.rand((2, 20, 11, 11), generator=torch.Generator(device="cuda").manual_seed(2), device="cuda") * 2.55
+    g = _graph(relu, results)
+    want = _run(g.compile(0, config={"HIP_KEEP_F32": "YES", "HIP_TUNE": "NO"}), x)
+    plan = g.compile(0, config={"HIP_TUNE": "NO"})
+    got = _run(plan, x)
+    assert len(got) == results and all(np.array_equal(a, b) for a, b in zip(got, want))
+    # two readers: the value stays in a tensor and is copied twice
+    assert [int(plan.step_rt_info(i, "kernels")) for i, s in enumerate(plan.steps) if s["type"] == "Result"] == ([0] if results == 1 else [1, 1])
