@@ -13,9 +13,17 @@ namespace hipie {
 // hardware exp2 instead of the library erfc's three dozen instructions, which made the kernel
 // compute-bound (double-precision erf: 63 us for [6144, 3072]; library erfcf: 29 us; this: 25 us, the
 // HBM time of its 151 MB).
+// The quotient 1 / d (gelu_reciprocal) is the hardware's approximation with one Newton step in fused multiply-adds: the IEEE quotient for every
+// d in [1, 2^63) (all significands compared: tests/test_matmul_glue_gpu.py), at three instructions instead of eleven.  z ends
+// at 2^60, where erfc has long been zero, so that d is in that range for an infinite or undefined x as well.
+__device__ __forceinline__ float gelu_reciprocal(float d) {
+    const float t = __builtin_amdgcn_rcpf(d);
+    return fmaf(fmaf(-d, t, 1.0f), t, t);
+}
+
 __device__ __forceinline__ float gelu_one(float x) {
-    const float z = fabsf(x) * 0.70710678118654752f;
-    const float t = 1.0f / (1.0f + 0.5f * z);
+    const float z = fminf(fabsf(x) * 0.70710678118654752f, 0x1p60f);
+    const float t = gelu_reciprocal(fmaf(0.5f, z, 1.0f));                  // (half of z is exact)
     float p = 0.17087277f;
     p = fmaf(p, t, -0.82215223f);
     p = fmaf(p, t, 1.48851587f);

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include "common.h"
+#include "gelu.h"
 #include "hipie_diag.h"
 
 namespace hipie {
@@ -144,6 +145,29 @@ extern "C" int hipie_probe_lds_rate(int device, int iterations, int waves_per_si
         const double per_second = total / (ms * 1e-3);
         *bytes_per_clock_per_cu = core_hz > 0 ? per_second / prop.multiProcessorCount / core_hz : 0.0;
         if (gigabytes_per_second) *gigabytes_per_second = per_second / 1e9;
+    });
+}
+
+namespace hipie {
+namespace {
+__global__ __launch_bounds__(256) void reciprocal_check(int exponent, unsigned long long* wrong) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;                   // 2^15 blocks: every significand
+    const float d = __uint_as_float((static_cast<uint32_t>(127 + exponent) << 23) | i);
+    if (__float_as_uint(gelu_reciprocal(d)) != __float_as_uint(1.0f / d)) atomicAdd(wrong, 1ull);
+}
+}  // namespace
+}  // namespace hipie
+
+extern "C" int hipie_probe_reciprocal(int device, int exponent, int64_t* wrong) {
+    return guarded([&] {
+        HIPIE_REQUIRE(wrong && exponent >= -126 && exponent <= 127, HIPIE_PARAMETER_MISMATCH, "hipie_probe_reciprocal: exponent %d", exponent);
+        DeviceGuard g(device);
+        DeviceBuffer count;
+        const unsigned long long zero = 0;
+        count.upload(device, &zero, sizeof zero);
+        hipLaunchKernelGGL(reciprocal_check, dim3(1u << 15), dim3(256), 0, nullptr, exponent, count.as<unsigned long long>());
+        HIPIE_CHECK_HIP(hipGetLastError());
+        HIPIE_CHECK_HIP(hipMemcpy(wrong, count.ptr, sizeof zero, hipMemcpyDeviceToHost));
     });
 }
 

@@ -75,6 +75,10 @@ int hipie_probe_mfma_rate(int device, int iterations, int waves_per_simd, double
 int hipie_probe_lds_rate(int device, int iterations, int waves_per_simd, int with_mfma, double* bytes_per_clock_per_cu,
                          double* gigabytes_per_second);
 
+/* How many d of [2^exponent, 2^(exponent + 1)), all 2^23 significands, the quotient 1 / d of the Gelu kernels (hardware
+ * approximation and one correction) rounds otherwise than IEEE division: 0 for 0 <= exponent < 63, all they meet. */
+int hipie_probe_reciprocal(int device, int exponent, int64_t* wrong);
+
 #ifdef __cplusplus
 }
 #endif

@@ -424,3 +424,26 @@ def test_nested_batches_inside_a_packed_tensor():
     transpose_bytes(base + 2 * H, 3 * H, D, vt.data_ptr(), S, D * S, S, D, NH, batch_outer=B,
                     outer_src=S * 3 * H, outer_dst=NH * D * S)
     np.testing.assert_array_equal(vt.cpu().numpy(), qkv.reshape(B, S, 3, NH, D)[:, :, 2].transpose(0, 2, 3, 1))
+
+
+def test_the_quotient_of_gelu_is_the_ieee_quotient():
+    """1 / (1 + z / 2) by the hardware's approximation and one correction: every significand of every binade that it meets"""
+    import ctypes
+
+    from dldt_amd._lib import check, lib
+    wrong = ctypes.c_int64(-1)
+    for exponent in range(63):
+        check(lib().hipie_probe_reciprocal(0, exponent, ctypes.byref(wrong)))
+        assert wrong.value == 0, exponent
+
+
+def test_gelu_of_the_extremes():
+    import torch
+
+    from dldt_amd import gelu
+    x = torch.tensor([float("inf"), float("-inf"), float("nan"), 0.0, -0.0, 3e38, -3e38, 1e-40, -1e-40, 2.0 ** 61, -2.0 ** 61, 12.0], device="cuda")
+    y = gelu(x).cpu().numpy()
+    # x Phi(x): infinity stays, -inf * 0 and NaN are NaN, large values are themselves or zero
+    assert y[0] == np.inf and np.isnan(y[1]) and np.isnan(y[2]) and y[3] == 0 and y[4] == 0
+    assert y[5] == np.float32(3e38) and y[6] == 0 and y[9] == np.float32(2.0 ** 61) and y[10] == 0 and y[11] == 12
+    assert np.all(np.abs(y[7:9]) <= 1e-40)
