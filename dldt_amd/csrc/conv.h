@@ -88,7 +88,7 @@ void launch_dwconv(const ConvArgs& a, int KH, int KW, int dil_h, int dil_w, int 
 struct ConvLaunch {
     ConvArgs a;
     bool depthwise;
-    int kh, kw, dil_h, dil_w;
+    int kh, kw, dil_h, dil_w, pad_top, pad_left;
 };
 bool conv_launch_arguments(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out, ConvLaunch& l);
 // the same with the f32 results channel by channel, [N, C, H, W] dense at `planes`; `out` says their shape.  Layers that take it:

@@ -2516,5 +2516,6 @@ bool hipie::conv_launch_arguments(const hipie_conv* c, const hipie_tensor& in, c
     int32_t oh, ow;
     l.depthwise = c->depthwise;
     l.kh = c->d.kh; l.kw = c->d.kw; l.dil_h = c->d.dil_h; l.dil_w = c->d.dil_w;
+    l.pad_top = c->d.pad_top; l.pad_left = c->d.pad_left;
     return fill_conv_args(c, &in, residual, &out, l.a, oh, ow) != 0;
 }

@@ -280,6 +280,15 @@ struct ConvStep : Step {
         }
         return b.conv(conv, i, (fused || res >= 0 || res_param >= 0) ? &r : nullptr, o);
     }
+    // this layer and the depthwise layer that alone reads it as one step of the single launch; false: they are two
+    bool joins(const ConvStep& next, ProgBuilder& b, const std::vector<TensorInfo>& tensors) const {
+        const TensorInfo& mid = tensors[out];
+        if (next.in != out || shortcut || res >= 0 || res_param >= 0 || writes_result || next.shortcut || next.res >= 0 || next.res_param >= 0 || next.writes_result ||
+            mid.alias >= 0 || !mid.fill_levels.empty() || (mid.dtype != HIPIE_U8B && mid.dtype != HIPIE_I8))
+            return false;
+        return b.expand_depthwise(conv, tensors[in].desc(b.fake_arena()), mid.desc(b.fake_arena()), next.conv, tensors[next.out].desc(b.fake_arena()),
+                                  mid.dtype == HIPIE_U8B ? mid.fill_level - 128 : mid.fill_level);
+    }
     // a dense f32 [rows, channels] request input as the residual operand of output tensor `o`
     static hipie_tensor input_residual(const hipie_tensor& o, void* data) {
         hipie_tensor r = o;
@@ -3005,6 +3014,7 @@ struct hipie_request {
     uint32_t* control = nullptr;
     uint32_t launches[kProgramControlBlocks] = {};
     const ProgramForm* form = nullptr;
+    const ProgramForm* ran = nullptr;        // the form of the last inference, if it was one (hipie_request_tensor)
     bool entered = false;                    // counted among the device's requests in flight
     bool stream_taken = false;               // hipie_request_stream gave the stream out: its work is complete in stream order
     std::vector<void*> run_in, run_out, host_out;
@@ -3076,6 +3086,7 @@ bool run_again(hipie_request* r) {
     r->program->count(!failed);
     if (!failed) return false;
     r->launches[block] = 0;
+    r->ran = nullptr;
     if (r->cancelled) return false;          // (nobody reads its outputs)
     enqueue(r, r->run_in.data(), r->run_out.data());
     for (size_t i = 0; i < r->host_out.size(); ++i)
@@ -3084,7 +3095,7 @@ bool run_again(hipie_request* r) {
 }
 
 // the single-launch form of a plan whose every step has one, or null and what it has no room for
-std::shared_ptr<ProgramForm> build_program(const hipie_plan& p, int workgroups, std::string& refused) {
+std::shared_ptr<ProgramForm> build_program(const hipie_plan& p, int workgroups, bool keep_values, std::string& refused) {
     if (p.inputs.size() + p.outputs.size() > static_cast<size_t>(kProgramIo)) {
         refused = "inputs and outputs";
         return nullptr;
@@ -3096,16 +3107,38 @@ std::shared_ptr<ProgramForm> build_program(const hipie_plan& p, int workgroups, 
     for (size_t i = 0; i < p.inputs.size(); ++i) in.push_back(b.fake_io(static_cast<int>(i)));
     for (size_t i = 0; i < p.outputs.size(); ++i) out.push_back(b.fake_io(static_cast<int>(p.inputs.size() + i)));
     DeviceGuard g(p.device);
-    for (const auto& s : p.steps)
+    // a step's readers: a layer whose only one is a depthwise layer can be one step with it
+    std::vector<int> readers(p.steps.size(), 0), reader(p.steps.size(), -1);
+    for (size_t i = 0; i < p.steps.size(); ++i)
+        for (int from : p.steps[i]->sources)
+            if (from >= 0) {
+                ++readers[static_cast<size_t>(from)];
+                reader[static_cast<size_t>(from)] = static_cast<int>(i);
+            }
+    std::vector<int> inside;
+    for (size_t i = 0; i < p.steps.size(); ++i) {
+        const Step* s = p.steps[i].get();
+        if (!keep_values && i + 1 < p.steps.size() && readers[i] == 1 && reader[i] == static_cast<int>(i) + 1) {
+            const auto* first = dynamic_cast<const ConvStep*>(s);
+            const auto* second = dynamic_cast<const ConvStep*>(p.steps[i + 1].get());
+            if (first && second && first->joins(*second, b, p.tensors)) {
+                inside.push_back(first->out);
+                ++i;
+                continue;
+            }
+        }
         if (!s->program(b, p.tensors, in.data(), out.data())) {
             refused = s->name;
             return nullptr;
         }
+    }
     if (b.map_kinds && b.rows_kinds) {       // (a kernel with the steps of both has no registers left for either's)
         refused = "feature maps and rows";
         return nullptr;
     }
-    return make_program_form(std::move(b));
+    auto form = make_program_form(std::move(b));
+    form->inside = std::move(inside);
+    return form;
 }
 
 // `preset`: kernel variants of an imported plan, one per step; used when they fit the steps planned
@@ -3478,7 +3511,7 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
         DeviceGuard dg(device);
         auto program = make_program(device);
         auto build = [&](int workgroups) {
-            return workgroups == 0 || workgroups > program->units ? nullptr : build_program(*plan, workgroups, plan->single_launch_refused);
+            return workgroups == 0 || workgroups > program->units ? nullptr : build_program(*plan, workgroups, cfg.keep_f32, plan->single_launch_refused);
         };
         if (cfg.single_launch > 2) {
             program->lone = program->shared = build(cfg.single_launch);
@@ -4032,11 +4065,13 @@ static int start_request(hipie_request* r, const void* const* inputs, void* cons
             out[i] = device_memory ? outputs[i] : r->out_dev[i].ptr;
         }
         r->entered = true;
+        r->ran = nullptr;
         const int together = request_enters(p.device);
         if (r->slot >= 0 && (awaited || (!device_memory && !r->stream_taken)) && buffers_fit_program(p, in.data(), out.data()))
             r->form = r->program->choose(together);
         if (r->form) {
             enqueue_program(r, in.data(), out.data());
+            r->ran = r->form;
             r->run_in = in;
             r->run_out = out;
             r->host_out.clear();
@@ -4128,6 +4163,7 @@ int hipie_request_enqueue(hipie_request* r, const void* const* inputs, void* con
         DeviceGuard g(r->plan->device);
         std::vector<void*> in(r->plan->inputs.size());
         for (size_t i = 0; i < in.size(); ++i) in[i] = const_cast<void*>(inputs[i]);
+        r->ran = nullptr;
         enqueue(r, in.data(), outputs);
     });
 }
@@ -4171,6 +4207,9 @@ int hipie_request_tensor(const hipie_request* r, int node_id, hipie_tensor* t) {
             if (auto* conv = dynamic_cast<const ConvStep*>(st.get()))
                 HIPIE_REQUIRE(!(conv->direct && conv->out == it->second), HIPIE_NOT_FOUND, "hipie_request_tensor: node %d is a result, stored in the caller's buffer only",
                               node_id);
+        if (r->ran)
+            for (int tensor : r->ran->inside)
+                HIPIE_REQUIRE(tensor != it->second, HIPIE_NOT_FOUND, "hipie_request_tensor: node %d lives in LDS only (two layers are one step of the single launch)", node_id);
         *t = r->plan->tensors[it->second].desc(r->arena.as<uint8_t>());
     });
 }

@@ -36,7 +36,7 @@ constexpr int kProgramThreads = 512;
 constexpr int kProgramIo = 6;            // graph inputs + outputs a program can address
 constexpr int kProgramStepWords = 128;
 
-enum ProgKind : int32_t { PK_CONV, PK_DW, PK_ENTRY, PK_MAXPOOL, PK_AVGPOOL, PK_EXIT, PK_EMBED, PK_MVN, PK_ATTENTION, PK_FQROWS, PK_COPY };
+enum ProgKind : int32_t { PK_CONV, PK_DW, PK_ENTRY, PK_MAXPOOL, PK_AVGPOOL, PK_EXIT, PK_EMBED, PK_MVN, PK_ATTENTION, PK_FQROWS, PK_COPY, PK_EXPAND_DW };
 
 // where an operand is: base 0 an arena offset, 1 + k an offset in the k-th input / output buffer of the call; < 0 absent
 struct ProgRef {
@@ -131,6 +131,12 @@ struct ProgBuilder {
     }
     // planes: the f32 results channel by channel at this address instead (conv_run_planes)
     bool conv(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out, void* planes = nullptr);
+    // a dense layer and the depthwise 3 x 3 layer that is its only reader; `fill`: the stored byte of the padding between them
+    bool expand_depthwise(const hipie_conv* first, const hipie_tensor& in, const hipie_tensor& mid, const hipie_conv* second, const hipie_tensor& out, int fill);
+    ProgPtr constants(const ConvArgs& a);
+    ProgPtr fragments(const int8_t* w, int o_tiles, int A, int OCp, int Kp);
+    bool layer(const ConvArgs& a, const hipie_tensor& out, ProgConv& c);
+    bool depthwise(const ConvLaunch& l, ProgConv& c);
     bool entry(const hipie_fq* fq, bool u8_in, const void* in, const hipie_tensor& out);
     bool pool(const PoolArgs& a, bool avg, bool rcp);
     bool exit(const ExitArgs& a, int in_dtype);
@@ -149,6 +155,7 @@ struct ProgBuilder {
 // form is another, and at load, while the sizes are measured, one more.
 struct ProgramForm {
     int workgroups = 0, n_steps = 0;
+    std::vector<int> inside;              // the plan's tensors that live inside a step
     bool encoder = false;                    // which of the two kernels
     DeviceBuffer steps;
     std::vector<DeviceBuffer> owned;

@@ -62,6 +62,7 @@ struct Ctx {
     int tid, lane, wave;
     const int32_t* steps;
     uint32_t words;                          // lane i: word i of the descriptor of the step that is run or prepared
+    uint32_t words2;                         // ... word 64 + i
     uint32_t bases;                          // lanes 2 b, 2 b + 1: where operands of base b are (ProgArgs::bases)
     uint32_t *xcds, *own;                    // the eight counters, the one this workgroup counts at
     uint32_t target;                         // what each of them holds when the barrier that comes next is complete
@@ -69,7 +70,7 @@ struct Ctx {
     bool started, dead;                      // between the roll call and the first step's wait; after a wait that was given up
     lds_i32 flag;
 
-    __device__ __forceinline__ uint32_t load_words(int step) const { return static_cast<uint32_t>(steps[step * kProgramStepWords + lane]); }
+    __device__ __forceinline__ uint32_t load_words(int step, int half) const { return static_cast<uint32_t>(steps[step * kProgramStepWords + half * (kProgramStepWords / 2) + lane]); }
     // an operand's address (of an absent one: the arena's, which nothing uses)
     __device__ __forceinline__ uint8_t* place(ProgRef r) const {
         const int b = 2 * max(r.base, 0);
@@ -86,7 +87,8 @@ struct Ctx {
     // adds to 2.1 / 2.3 / 2.6, all at one counter 1.5 / 2.3 / 4.1, a flag per workgroup that everybody reads 1.4 / 1.6 / 1.8.
     // (One way between two workgroups, store to sight, takes 0.5 - 0.6 us, the wait for a store 0.36.)
     __device__ __forceinline__ void arrive(int next_step) {
-        words = load_words(next_step);
+        words = load_words(next_step, 0);
+        words2 = load_words(next_step, 1);
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         target += n_wg / 8;
@@ -360,18 +362,18 @@ struct StepConstants {
     uint32_t plane;                          // bytes between the planes of f32 results; 0: channels innermost
 };
 template <bool DENSE>
-__device__ __forceinline__ StepConstants step_constants(const Ctx& x) {
+__device__ __forceinline__ StepConstants step_constants(const Ctx& x, uint32_t words) {
     StepConstants s;
-    s.flags = PROG_FIELD(x.words, flags);
-    s.out = make_buffer(PROG_PLACE(x, out));
-    s.res = make_buffer(PROG_PLACE(x, res));
-    s.lm1 = PROG_FIELD(x.words, lm1);
-    s.clamp_lo = PROG_FIELD(x.words, clamp_lo);
-    s.clamp_hi = PROG_FIELD(x.words, clamp_hi);
-    s.off_bytes = PROG_FIELD(x.words, off_bytes);
-    s.out_limit = PROG_FIELD(x.words, out_limit);
-    s.res_limit = PROG_FIELD(x.words, res_limit);
-    s.plane = DENSE ? static_cast<uint32_t>(PROG_FIELD(x.words, out_sn)) : 0u;
+    s.flags = PROG_FIELD(words, flags);
+    s.out = make_buffer(x.place(PROG_FIELD(words, out)));
+    s.res = make_buffer(x.place(PROG_FIELD(words, res)));
+    s.lm1 = PROG_FIELD(words, lm1);
+    s.clamp_lo = PROG_FIELD(words, clamp_lo);
+    s.clamp_hi = PROG_FIELD(words, clamp_hi);
+    s.off_bytes = PROG_FIELD(words, off_bytes);
+    s.out_limit = PROG_FIELD(words, out_limit);
+    s.res_limit = PROG_FIELD(words, res_limit);
+    s.plane = DENSE ? static_cast<uint32_t>(PROG_FIELD(words, out_sn)) : 0u;
     return s;
 }
 
@@ -402,11 +404,11 @@ __device__ __forceinline__ void load_residual(const StepConstants& s, int oc, Pi
     }
 }
 
-// the fused f32 chain (conv_epilogue.h) on A neighbouring channels of R pixels, and their store
+// the fused f32 chain (conv_epilogue.h) on A neighbouring channels of R pixels, up to the FakeQuantize
 template <bool GELU, int A, int R, bool PAIR = false>
-__device__ __forceinline__ void finish(const StepConstants& c, const ChannelConstants<A>& k, const int32_t (&sum)[A][R], const float (&rgemm)[A][R], const Pixels<A>& q, int oc) {
+__device__ __forceinline__ void chain(const StepConstants& c, const ChannelConstants<A>& k, const int32_t (&sum)[A][R], const float (&rgemm)[A][R], const Pixels<A>& q, int oc,
+                                      float (&x)[A][R]) {
     const uint32_t fl = c.flags;
-    float x[A][R];
 #define PROG_EACH for (int a = 0; a < A; ++a) for (int r = 0; r < R; ++r)
 #pragma unroll
     PROG_EACH x[a][r] = static_cast<float>(sum[a][r]);
@@ -467,25 +469,12 @@ __device__ __forceinline__ void finish(const StepConstants& c, const ChannelCons
 #pragma unroll
             PROG_EACH x[a][r] = gelu_one(x[a][r]);
         }
-    if (!(fl & CF_OUT_FQ) && c.plane != 0) {
-#pragma unroll
-        for (int a = 0; a < A; ++a) {
-            const uint32_t o = oc + a < c.out_limit ? static_cast<uint32_t>(oc + a) * c.plane : static_cast<uint32_t>(kBeyond);
-#pragma unroll
-            for (int r = 0; r < R; ++r) publish4(c.out, q.out[r] + o, __float_as_uint(x[a][r] + 0.f));
-        }
-        return;
-    }
-    if (!(fl & CF_OUT_FQ)) {
-        const uint32_t o = oc < c.out_limit ? static_cast<uint32_t>(4 * oc) : static_cast<uint32_t>(kBeyond);
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if constexpr (A == 4) publish16f(c.out, q.out[r] + o, make_float4(x[0][r], x[1][r], x[2][r], x[3][r]));
-            else if constexpr (A == 2) publish8(c.out, q.out[r] + o, v2i{__float_as_int(x[0][r]), __float_as_int(x[1][r])});
-            else publish4(c.out, q.out[r] + o, __float_as_uint(x[0][r]));
-        }
-        return;
-    }
+}
+
+// the stored bytes of A neighbouring channels of R pixels; x is used up
+template <int A, int R>
+__device__ __forceinline__ void levels(const StepConstants& c, const ChannelConstants<A>& k, float (&x)[A][R], uint32_t (&bytes)[R]) {
+    const uint32_t fl = c.flags;
     // level index: as fq_level_fast, operation by operation
     const bool il0 = (fl & CF_FQ_IL0) != 0;
     if (!(fl & CF_FQ_SAT)) {
@@ -511,17 +500,49 @@ __device__ __forceinline__ void finish(const StepConstants& c, const ChannelCons
         }
     }
     const uint32_t xmask = (fl & CF_OUT_XOR) ? 0x80808080u : 0u;
-    const uint32_t o = oc < c.out_limit ? static_cast<uint32_t>(oc) : static_cast<uint32_t>(kBeyond);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         uint32_t w = 0;
 #pragma unroll
         for (int a = 0; a < A; ++a) w = __builtin_amdgcn_cvt_pk_u8_f32(x[a][r], a, w);
         if (fl & CF_OUT_ADD) w = add_bytes(w, c.off_bytes);
-        w ^= xmask;
-        if constexpr (A == 4) publish4(c.out, q.out[r] + o, w);
-        else if constexpr (A == 2) publish2(c.out, q.out[r] + o, w);
-        else publish1(c.out, q.out[r] + o, w);
+        bytes[r] = w ^ xmask;
+    }
+}
+
+// the chain and the store of its values
+template <bool GELU, int A, int R, bool PAIR = false>
+__device__ __forceinline__ void finish(const StepConstants& c, const ChannelConstants<A>& k, const int32_t (&sum)[A][R], const float (&rgemm)[A][R], const Pixels<A>& q, int oc) {
+    const uint32_t fl = c.flags;
+    float x[A][R];
+    chain<GELU, A, R, PAIR>(c, k, sum, rgemm, q, oc, x);
+    if (!(fl & CF_OUT_FQ) && c.plane != 0) {
+#pragma unroll
+        for (int a = 0; a < A; ++a) {
+            const uint32_t o = oc + a < c.out_limit ? static_cast<uint32_t>(oc + a) * c.plane : static_cast<uint32_t>(kBeyond);
+#pragma unroll
+            for (int r = 0; r < R; ++r) publish4(c.out, q.out[r] + o, __float_as_uint(x[a][r] + 0.f));
+        }
+        return;
+    }
+    if (!(fl & CF_OUT_FQ)) {
+        const uint32_t o = oc < c.out_limit ? static_cast<uint32_t>(4 * oc) : static_cast<uint32_t>(kBeyond);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if constexpr (A == 4) publish16f(c.out, q.out[r] + o, make_float4(x[0][r], x[1][r], x[2][r], x[3][r]));
+            else if constexpr (A == 2) publish8(c.out, q.out[r] + o, v2i{__float_as_int(x[0][r]), __float_as_int(x[1][r])});
+            else publish4(c.out, q.out[r] + o, __float_as_uint(x[0][r]));
+        }
+        return;
+    }
+    uint32_t w[R];
+    levels<A, R>(c, k, x, w);
+    const uint32_t o = oc < c.out_limit ? static_cast<uint32_t>(oc) : static_cast<uint32_t>(kBeyond);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if constexpr (A == 4) publish4(c.out, q.out[r] + o, w[r]);
+        else if constexpr (A == 2) publish2(c.out, q.out[r] + o, w[r]);
+        else publish1(c.out, q.out[r] + o, w[r]);
     }
 #undef PROG_EACH
 }
@@ -613,7 +634,7 @@ __device__ __forceinline__ void conv_tiles(Ctx& x, lds_ptr lds) {
     }
     const uint32_t tiles = static_cast<uint32_t>(PROG_FIELD(x.words, tiles));
     const int t0 = static_cast<int>((static_cast<uint32_t>(x.rank) * tiles) >> x.wg_shift), t1 = static_cast<int>((static_cast<uint32_t>(x.rank + 1) * tiles) >> x.wg_shift);
-    const StepConstants sc = step_constants<true>(x);
+    const StepConstants sc = step_constants<true>(x, x.words);
     const int M = PROG_FIELD(x.words, M);
     const uint32_t* pix = PROG_TABLE_OF(uint32_t, x.words, pixels);
     const lds_v4i part = (lds_v4i)lds + x.wave * (F * 64) + x.lane;
@@ -734,6 +755,16 @@ __device__ __forceinline__ void conv_tiles(Ctx& x, lds_ptr lds) {
 // v_dot4_i32_i8 as in dwconv.hip; consecutive lanes take consecutive channels.  G = 4 does the fewest operations per value,
 // G = 1 a quarter of the work per lane: where a step's values are no more than the launch's lanes at one pixel each, what a
 // lane does is what the step takes (ProgBuilder::conv).
+// 4 x 4 byte transpose: t[e] = bytes e of p0 .. p3
+__device__ __forceinline__ void transpose_bytes(uint32_t p0, uint32_t p1, uint32_t p2, uint32_t p3, uint32_t (&t)[4]) {
+    const uint32_t lo01 = __builtin_amdgcn_perm(p1, p0, 0x05010400u), hi01 = __builtin_amdgcn_perm(p1, p0, 0x07030602u);
+    const uint32_t lo23 = __builtin_amdgcn_perm(p3, p2, 0x05010400u), hi23 = __builtin_amdgcn_perm(p3, p2, 0x07030602u);
+    t[0] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+    t[1] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+    t[2] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+    t[3] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+}
+
 template <int STRIDE, int G>
 __device__ __forceinline__ void dw_items(Ctx& x) {
     constexpr int COLS = G == 1 ? 3 : 3 + 3 * STRIDE;
@@ -744,7 +775,7 @@ __device__ __forceinline__ void dw_items(Ctx& x) {
     const int res_sn = PROG_FIELD(x.words, res_sn), res_sh = PROG_FIELD(x.words, res_sh), res_sw = PROG_FIELD(x.words, res_sw);
     const float inv_c4 = PROG_FIELD(x.words, inv_c4), inv_quads = PROG_FIELD(x.words, inv_quads), inv_OH = PROG_FIELD(x.words, inv_OH);
     const Buffer in = make_buffer(PROG_PLACE(x, in));
-    const StepConstants sc = step_constants<false>(x);
+    const StepConstants sc = step_constants<false>(x, x.words);
     const int8_t* wgt = PROG_TABLE_OF(int8_t, x.words, wgt);
     const uint8_t* constants = PROG_TABLE_OF(uint8_t, x.words, constants);
     const bool f32 = sc.flags & CF_RES_F32, fo = !(sc.flags & CF_OUT_FQ);
@@ -793,14 +824,6 @@ __device__ __forceinline__ void dw_items(Ctx& x) {
         for (int a = 0; a < 4; ++a)
 #pragma unroll
             for (int r = 0; r < G; ++r) acc[a][r] = k.corr[a];
-        auto transpose4 = [&](uint32_t p0, uint32_t p1, uint32_t p2, uint32_t p3, uint32_t (&t)[4]) {
-            const uint32_t lo01 = __builtin_amdgcn_perm(p1, p0, 0x05010400u), hi01 = __builtin_amdgcn_perm(p1, p0, 0x07030602u);
-            const uint32_t lo23 = __builtin_amdgcn_perm(p3, p2, 0x05010400u), hi23 = __builtin_amdgcn_perm(p3, p2, 0x07030602u);
-            t[0] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
-            t[1] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
-            t[2] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
-            t[3] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
-        };
 #pragma unroll
         for (int r = 0; r < 3; ++r) {
             const uint32_t w[4] = {wr[r].x, wr[r].y, wr[r].z, wr[r].w};
@@ -808,7 +831,7 @@ __device__ __forceinline__ void dw_items(Ctx& x) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     uint32_t t[4];
-                    transpose4(v[r][2 * h], v[r][2 * h + 1], v[r][2 * h + 2], v[r][2 * h + 3], t);
+                    transpose_bytes(v[r][2 * h], v[r][2 * h + 1], v[r][2 * h + 2], v[r][2 * h + 3], t);
 #pragma unroll
                     for (int a = 0; a < 4; ++a) {
                         acc[a][2 * h] = __builtin_amdgcn_sdot4(static_cast<int>(t[a]), static_cast<int>(w[a]), acc[a][2 * h], false);
@@ -819,7 +842,7 @@ __device__ __forceinline__ void dw_items(Ctx& x) {
 #pragma unroll
                 for (int h = 0; h < G; ++h) {
                     uint32_t t[4];
-                    transpose4(v[r][2 * h], v[r][2 * h + 1], v[r][2 * h + 2], v[r][2 * h + 2], t);
+                    transpose_bytes(v[r][2 * h], v[r][2 * h + 1], v[r][2 * h + 2], v[r][2 * h + 2], t);
 #pragma unroll
                     for (int a = 0; a < 4; ++a) acc[a][h] = __builtin_amdgcn_sdot4(static_cast<int>(t[a]), static_cast<int>(w[a]), acc[a][h], false);
                 }
@@ -829,6 +852,163 @@ __device__ __forceinline__ void dw_items(Ctx& x) {
         finish<false, 4, G>(sc, k, acc, none, pq, oc);
         i0 += stride;
     } while (i0 < items);
+}
+
+// ---- expansion and depthwise 3 x 3 in one step ------------------------------------------------------------------------------
+// A convolution whose only reader is the depthwise layer behind it (the first two layers of an inverted residual block): a
+// workgroup computes 16 A channels of the input rows under a band of R output rows, requantised, into a patch in LDS - the rows
+// between two bands by both - and the depthwise layer from there.  The tensor between the layers does not exist, and the block
+// is two steps instead of three: a step of a network at batch 1 takes 3 - 4 us whatever it does (barrier, preparation, first
+// operands, stores), a row computed twice a matrix instruction and a chain on four values a lane.  MobileNetV2 at batch 1, us:
+// 197 with the layers apart, 182 with this, 170 with a fragment's pixels requested while the one before is multiplied, 168 with
+// the second layer's constants requested behind the wait instead of in front of it (the preparation, 2.2 us, was longer than
+// the barrier; 1.6 now).  What is left of such a step: 1.5 preparation and barrier, 1.2 - 2.3 first layer, 0.6 - 1.0 second.
+// The descriptor's first half is the convolution, with the geometry in the fields that only depthwise layers have
+// (ProgBuilder::expand_depthwise), its second half the depthwise layer.
+constexpr int kExpandSteps = 4;               // K steps of the convolution, held in registers
+
+template <int A>
+__device__ __forceinline__ void expand_depthwise(Ctx& x, lds_ptr lds) {
+    // (what only the layers' ends need is read and requested behind the wait, while the first pixels are on their way: before it,
+    // it stands between this step and the one before)
+    const int nk = PROG_FIELD(x.words, nk), S = PROG_FIELD(x.words, stride), R = PROG_FIELD(x.words, group), W = PROG_FIELD(x.words, quads), H = PROG_FIELD(x.words, OW);
+    const int bands = PROG_FIELD(x.words, OH), all_bands = PROG_FIELD(x.words, res_sw), PW = PROG_FIELD(x.words, in_sn), pad_t = PROG_FIELD(x.words, in_sh);
+    const int OH = PROG_FIELD(x.words, row_sh);
+    const bool plain = PROG_FIELD(x.words, koff).hi == 0;
+    const lds_i32 staged_to = (lds_i32)(lds + kPartBytes), koff = plain ? (lds_i32)(lds + kPlainAt) : staged_to;
+    int32_t staged = 0;
+    if (!plain) staged = request_offsets(staged_to, PROG_TABLE_OF(int32_t, x.words, koff), 4 * nk, x.tid);
+    const uint32_t units = static_cast<uint32_t>(PROG_FIELD(x.words, tiles));
+    const int t0 = static_cast<int>((static_cast<uint32_t>(x.rank) * units) >> x.wg_shift), t1 = static_cast<int>((static_cast<uint32_t>(x.rank + 1) * units) >> x.wg_shift);
+    if (t0 >= t1) {
+        x.wait();
+        return;
+    }
+    const uint32_t* pix = PROG_TABLE_OF(uint32_t, x.words, pixels);
+    const int lane16 = x.lane & 15, quad = x.lane >> 4, c4 = x.tid & (4 * A - 1);
+    auto meet = [] {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    int unit = t0;
+    do {
+        int ct, nb, n, band;
+        fast_divmod(unit, all_bands, PROG_FIELD(x.words, inv_c4), ct, nb);
+        ct = __builtin_amdgcn_readfirstlane(ct);
+        nb = __builtin_amdgcn_readfirstlane(nb);
+        fast_divmod(nb, bands, PROG_FIELD(x.words, inv_OH), n, band);
+        n = __builtin_amdgcn_readfirstlane(n);
+        band = __builtin_amdgcn_readfirstlane(band);
+        const int oy0 = band * R, rows = min(R, OH - oy0), iy0 = oy0 * S - pad_t, patch_rows = (rows - 1) * S + 3;
+        const int y0 = max(iy0, 0), y1 = min(iy0 + patch_rows, H), count = (y1 - y0) * W, m0 = (n * H + y0) * W;
+        const int oc = ct * (16 * A) + A * lane16, oc4 = ct * (16 * A) + 4 * c4;
+        const Buffer wb = make_buffer(PROG_TABLE_OF(int8_t, x.words, wgt) + static_cast<int64_t>(ct) * nk * (A * 1024));
+        v4i wt[kExpandSteps][A];
+#pragma unroll
+        for (int k = 0; k < kExpandSteps; ++k)
+#pragma unroll
+            for (int a = 0; a < A; ++a) wt[k][a] = load16<0>(wb, static_cast<uint32_t>(x.lane * 16) + static_cast<uint32_t>(k < nk ? k * (A * 1024) : kBeyond), a * 1024);
+        ChannelConstants<A> k1;
+        load_constants<A>(PROG_FIELD(x.words, flags), PROG_TABLE_OF(uint8_t, x.words, constants), PROG_FIELD(x.words, OCp) * 4, oc, k1);
+        int f = x.wave;
+        uint32_t off = pix[m0 + min(16 * f + lane16, count - 1)];
+        // the patch at the level of the padding (every lane takes part, those behind the end repeat the last piece)
+        const int pieces = patch_rows * PW * A, fill = PROG_FIELD(x.words, res_sh);
+        for (int base = 0; base < pieces; base += kProgramThreads) ((lds_v4i)lds)[min(base + x.tid, pieces - 1)] = v4i{fill, fill, fill, fill};
+        if (unit == t0) {
+            if (!plain) staged_to[min(x.tid, 4 * nk - 1)] = staged;
+            x.wait();
+        } else meet();
+        // the convolution: a wave's fragments of 16 pixels, eight apart
+        const Buffer in = make_buffer(PROG_PLACE(x, in));
+        const int frags = (count + 15) / 16;
+        v4i p[kExpandSteps], next[kExpandSteps];
+        auto request = [&](v4i (&to)[kExpandSteps]) {
+#pragma unroll
+            for (int k = 0; k < kExpandSteps; ++k)
+                to[k] = shared16(in, off + static_cast<uint32_t>(koff[4 * min(k, nk - 1) + quad]) + (k < nk ? 0u : static_cast<uint32_t>(kBeyond)));
+        };
+        request(p);
+        off = pix[m0 + min(16 * f + 128 + lane16, count - 1)];
+        const StepConstants c1 = step_constants<false>(x, x.words), c2 = step_constants<false>(x, x.words2);
+        const int OCp2 = PROG_FIELD(x.words2, OCp), pad_l = PROG_FIELD(x.words, in_sw);
+        const float inv_W = PROG_FIELD(x.words, inv_quads);
+        uint4 wr[3];
+#pragma unroll
+        for (int r = 0; r < 3; ++r) wr[r] = *reinterpret_cast<const uint4*>(PROG_TABLE_OF(int8_t, x.words2, wgt) + (static_cast<int64_t>(r) * OCp2 + oc4) * 4);
+        ChannelConstants<4> k2;
+        load_constants<4>(c2.flags, PROG_TABLE_OF(uint8_t, x.words2, constants), OCp2 * 4, oc4, k2);
+        while (f < frags) {
+            const int j0 = 16 * f + 4 * quad;
+            f += 8;
+            request(next);                       // (those behind the last one read its pixels)
+            off = pix[m0 + min(16 * f + 128 + lane16, count - 1)];
+            v4i acc[A];
+#pragma unroll
+            for (int a = 0; a < A; ++a) acc[a] = v4i{k1.corr[a], k1.corr[a], k1.corr[a], k1.corr[a]};
+#pragma unroll
+            for (int k = 0; k < kExpandSteps; ++k)
+                if (k == 0 || k < nk)
+#pragma unroll
+                    for (int a = 0; a < A; ++a) acc[a] = __builtin_amdgcn_mfma_i32_16x16x64_i8(p[k], wt[k][a], acc[a], 0, 0, 0);
+            int32_t sum[A][4];
+            const float none[A][4] = {};
+            float v[A][4];
+            uint32_t bytes[4];
+#pragma unroll
+            for (int a = 0; a < A; ++a)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sum[a][r] = acc[a][r];
+            const Pixels<A> nowhere{};
+            chain<false, A, 4>(c1, k1, sum, none, nowhere, oc, v);
+            levels<A, 4>(c1, k1, v, bytes);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                int row, col;
+                fast_divmod(min(j0 + r, count - 1), W, inv_W, row, col);        // (pixels behind the last one hold its values)
+                const lds_ptr at = lds + ((y0 - iy0 + row) * PW + col + pad_l) * (16 * A) + A * lane16;
+                if constexpr (A == 1) *at = static_cast<int8_t>(bytes[r]);
+                else *(__attribute__((address_space(3))) uint16_t*)at = static_cast<uint16_t>(bytes[r]);
+            }
+#pragma unroll
+            for (int k = 0; k < kExpandSteps; ++k) p[k] = next[k];
+        }
+        meet();
+        // the depthwise layer: four channels of a pixel per lane
+        const int OW = PROG_FIELD(x.words, res_sn), items = rows * OW * (4 * A);
+        const int out_sn = PROG_FIELD(x.words2, out_sn), out_sh = PROG_FIELD(x.words2, out_sh), out_sw = PROG_FIELD(x.words2, out_sw);
+        const float inv_OW = PROG_FIELD(x.words, inv_p_tiles);
+        for (int base = 0; base < items; base += kProgramThreads) {
+            const bool on = base + x.tid < items;
+            int oy, ox;
+            fast_divmod(min(base + x.tid, items - 1) / (4 * A), OW, inv_OW, oy, ox);
+            const lds_ptr at = lds + (oy * S * PW + ox * S) * (16 * A) + 4 * c4;
+            int32_t acc[4][1];
+#pragma unroll
+            for (int a = 0; a < 4; ++a) acc[a][0] = k2.corr[a];
+            uint32_t v[3][3];
+#pragma unroll
+            for (int r = 0; r < 3; ++r)
+#pragma unroll
+                for (int j = 0; j < 3; ++j) v[r][j] = *(const __attribute__((address_space(3))) uint32_t*)(at + (r * PW + j) * (16 * A));
+#pragma unroll
+            for (int r = 0; r < 3; ++r) {
+                const uint32_t w[4] = {wr[r].x, wr[r].y, wr[r].z, wr[r].w};
+                uint32_t t[4];
+                transpose_bytes(v[r][0], v[r][1], v[r][2], v[r][2], t);
+#pragma unroll
+                for (int a = 0; a < 4; ++a) acc[a][0] = __builtin_amdgcn_sdot4(static_cast<int>(t[a]), static_cast<int>(w[a]), acc[a][0], false);
+            }
+            Pixels<4> q;
+            q.out[0] = on ? static_cast<uint32_t>(n * out_sn + (oy0 + oy) * out_sh + ox * out_sw) : static_cast<uint32_t>(kBeyond);
+            q.res[0] = 0;
+            const float none[4][1] = {};
+            finish<false, 4, 1>(c2, k2, acc, none, q, oc4);
+        }
+        ++unit;
+        if (unit < t1) meet();
+    } while (unit < t1);
 }
 
 // ---- entry, pooling, exit ---------------------------------------------------------------------------------------------------
@@ -1392,7 +1572,8 @@ __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgA
     x.n_wg = g.workgroups;
     x.wg_shift = __builtin_ctz(x.n_wg);
     x.steps = g.steps;
-    x.words = x.load_words(0);
+    x.words = x.load_words(0, 0);
+    x.words2 = x.load_words(0, 1);
     x.bases = reinterpret_cast<const uint32_t*>(g.bases)[min(x.lane, 2 * (1 + kProgramIo) - 1)];
     for (int i = x.tid; i < kMaxPieces; i += kProgramThreads) ((lds_i32)(lds + kPlainAt))[i] = 16 * i;
     x.rank = static_cast<int>(blockIdx.x % 8) * (x.n_wg / 8) + static_cast<int>(blockIdx.x / 8);
@@ -1415,7 +1596,7 @@ __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgA
         x.tid = 64 * x.wave + lane;
         const StepPtr words = step_ptr(g.steps, step);
         const int kind = static_cast<int>(word_of(x.words, 0));
-        if (kind != PK_CONV && kind != PK_DW && kind != PK_MVN && kind != PK_ATTENTION) x.wait();      // (those wait when they have prepared)
+        if (kind != PK_CONV && kind != PK_DW && kind != PK_EXPAND_DW && kind != PK_MVN && kind != PK_ATTENTION) x.wait();      // (those wait when they have prepared)
         switch (kind) {
         case PK_CONV: {
             switch (PROG_FIELD(x.words, a) * 8 + PROG_FIELD(x.words, b) + (PROG_FIELD(x.words, nk2) ? 64 : 0)) {
@@ -1460,6 +1641,9 @@ __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgA
                 case 16 + 1: dw_items<2, 1>(x); break;
                 default: dw_items<2, 4>(x); break;
                 }
+            } else if (kind == PK_EXPAND_DW) {
+                if (PROG_FIELD(x.words, a) == 1) expand_depthwise<1>(x, lds);
+                else expand_depthwise<2>(x, lds);
             } else if (kind == PK_MAXPOOL) max_pool_items(unpack<ProgPool>(words), x);
             else avg_pool_items(unpack<ProgPool>(words), x);
         }
@@ -1572,53 +1756,138 @@ ProgPtr ProgBuilder::keep(const void* host, size_t bytes) {
     return ptr(owned.back().ptr);
 }
 
+// the channel tables that a layer's flags ask for, in load_constants' order
+ProgPtr ProgBuilder::constants(const ConvArgs& a) {
+    const uint32_t fl = a.flags;
+    std::vector<const void*> rows{a.corr};
+    if (fl & CF_BIAS) rows.push_back(a.bias);
+    if (fl & CF_SCALE) rows.push_back(a.scale);
+    if (fl & CF_RES_MUL) rows.push_back(a.res_mul);
+    if (fl & CF_OUT_FQ) {
+        rows.push_back(a.fq_r);
+        rows.push_back((fl & CF_FQ_DIV2) ? a.fq_r2 : a.fq_d);
+        if (!(fl & CF_FQ_SAT)) rows.push_back(a.fq_ih);
+        if (!(fl & CF_FQ_IL0)) rows.push_back(a.fq_il);
+    }
+    return gather(rows, static_cast<size_t>(a.OCp) * 4);
+}
+
+ProgPtr ProgBuilder::fragments(const int8_t* w, int o_tiles, int A, int OCp, int Kp) {
+    owned.emplace_back();
+    const int64_t pieces = static_cast<int64_t>(o_tiles) * A * Kp;        // 16 A x Kp bytes per tile, 16 bytes a piece
+    owned.back().alloc(device, static_cast<size_t>(pieces) * 16);
+    hipLaunchKernelGGL(pack_fragments_kernel, dim3(static_cast<uint32_t>(ceil_div(pieces, 256))), dim3(256), 0, nullptr, w, owned.back().as<int8_t>(), A, OCp, Kp, pieces);
+    HIPIE_CHECK_HIP(hipGetLastError());
+    return ptr(owned.back().ptr);
+}
+
+// a depthwise layer's own fields; false: not a 3 x 3 layer that the kernel takes
+bool ProgBuilder::depthwise(const ConvLaunch& l, ProgConv& c) {
+    const ConvArgs& a = l.a;
+    c.OH = a.OHOW / a.OW;
+    c.OW = a.OW;
+    if (l.kh != 3 || l.kw != 3 || l.dil_h != 1 || l.dil_w != 1 || a.conv_sh != a.conv_sw || a.conv_sh > 2 || !a.wgt2 || a.in_sw < a.out_sw) return false;
+    c.kind = PK_DW;
+    map_kinds = true;
+    c.stride = a.conv_sh;
+    c.wgt = ptr(a.wgt2);
+    c.in_sn = a.in_sn; c.in_sh = a.in_sh * a.conv_sh; c.in_sw = a.in_sw; c.row_sh = a.in_sh;
+    c.out_sn = a.out_sn; c.out_sh = a.out_sh; c.out_sw = a.out_sw;
+    c.res_sn = a.res_sn; c.res_sh = a.res_sh; c.res_sw = a.res_sw;
+    c.c4 = a.out_sw / 4;
+    return true;
+}
+
+// what convolutions and depthwise layers have in common; false: the kernel does not take the layer
+bool ProgBuilder::layer(const ConvArgs& a, const hipie_tensor& out, ProgConv& c) {
+    if (a.M > (1 << 20) || a.koff_tile || (a.flags & CF_OUT_I32) || ((a.flags & CF_OUT_FQ) && !(a.flags & CF_FQ_RCP)) || (a.flags & (CF_RES_SUB | CF_POST_SCALE)))
+        return false;
+    const bool f32_out = !(a.flags & CF_OUT_FQ), f32_res = (a.flags & CF_RES_F32) != 0;
+    for (int64_t bytes : {static_cast<int64_t>(out.n) * a.out_sn * (f32_out ? 4 : 1), static_cast<int64_t>(out.n) * a.res_sn * (f32_res ? 4 : 1)})
+        if (bytes >= kBeyond) return false;
+    c.in = ref(a.in + a.in_origin);
+    c.out = ref(a.out);
+    c.res = a.res ? ref(a.res) : ProgRef{-2, 0, 0};
+    c.in2 = ProgRef{-2, 0, 0};
+    c.out_limit = a.out_plane ? a.OC : a.out_sw;       // channels that the output holds
+    c.res_limit = a.res_sw;
+    c.constants = constants(a);
+    c.flags = a.flags; c.lm1 = a.lm1; c.off_bytes = (static_cast<uint32_t>(static_cast<int>(a.out_off)) & 0xffu) * 0x01010101u; c.clamp_lo = a.clamp_lo; c.clamp_hi = a.clamp_hi;
+    c.OCp = a.OCp;
+    return true;
+}
+
+// Two layers as one step (expand_depthwise in this file), or false: they are two.  Where the kernel takes both layers one step is
+// always the faster form (MobileNetV2 at batch 1, 2 and 4: 199, 207 and 221 us by two steps, 171, 183 and 204 by one).
+// Channels per tile and rows per band are what gives a workgroup the fewest clocks; the times above move by less than 1 us where
+// any of these constants is doubled or halved, as long as the units fit the workgroups in one round.
+bool ProgBuilder::expand_depthwise(const hipie_conv* first, const hipie_tensor& in, const hipie_tensor& mid, const hipie_conv* second, const hipie_tensor& out, int fill) {
+    ConvLaunch l1, l2;
+    if (!conv_launch_arguments(first, in, nullptr, mid, l1) || !conv_launch_arguments(second, mid, nullptr, out, l2)) return false;
+    const ConvArgs &a1 = l1.a, &a2 = l2.a;
+    if (l1.depthwise || !l2.depthwise || a1.nk > kExpandSteps || !(a1.flags & CF_OUT_FQ) || !(a2.flags & CF_OUT_FQ) || ((a1.flags | a2.flags) & (CF_RES | CF_GELU))) return false;
+    const int N = mid.n, H = mid.h, W = mid.w, OH = a2.OHOW / a2.OW, OW = a2.OW, S = a2.conv_sh;
+    const int pw = std::max((OW - 1) * S + 3, W + l2.pad_left), channels = std::min(a1.out_sw, a2.out_sw);
+    if (l2.pad_top > 2 || (OH - 1) * S - l2.pad_top >= H || channels % 16 != 0) return false;      // (every band has an input row)
+    int best_a = 0, best_r = 0;
+    double best = 1e30;
+    for (int A : {1, 2})
+        for (int R = 1; R <= OH; ++R) {
+            const int64_t rows = (R - 1) * S + 3;
+            if (rows * pw * 16 * A > kPartBytes) break;
+            const int64_t units = ceil_div(channels, 16 * A) * N * ceil_div(OH, R), rounds = ceil_div(units, workgroups);
+            const double frags = static_cast<double>(ceil_div(ceil_div(std::min<int64_t>(rows, H) * W, 16), 8)), items = static_cast<double>(ceil_div(R * OW * 4 * A, kProgramThreads));
+            const double t = static_cast<double>(rounds) * (2500.0 + frags * (500.0 + 100.0 * A + 60.0 * A * a1.nk) + items * 1200.0);
+            if (t < best) {
+                best = t;
+                best_a = A;
+                best_r = R;
+            }
+        }
+    if (!best_a) return false;
+    ProgConv c{}, d{};
+    if (!layer(a1, mid, c) || !layer(a2, out, d) || !depthwise(l2, d)) return false;
+    const int64_t bands = ceil_div(OH, best_r), cts = ceil_div(channels, 16 * best_a), units = cts * N * bands;
+    if (units * workgroups >= (1ll << 31) || units >= (1 << 24)) return false;
+    c.kind = PK_EXPAND_DW;
+    c.a = best_a;
+    c.b = 1;
+    c.tiles = static_cast<int32_t>(units);
+    c.nk = a1.nk;
+    if (!a1.k_linear) c.koff = ptr(a1.koff);
+    c.wgt = fragments(a1.wgt, static_cast<int>(cts), best_a, a1.OCp, a1.Kp);
+    std::vector<uint32_t> pix(static_cast<size_t>(a1.M));
+    for (int64_t m = 0; m < a1.M; ++m) {
+        const int64_t n = m / a1.OHOW, rem = m - n * a1.OHOW, y = rem / a1.OW, xx = rem - y * a1.OW;
+        pix[static_cast<size_t>(m)] = static_cast<uint32_t>(n * a1.in_sn + y * a1.in_sh * a1.conv_sh + xx * a1.in_sw * a1.conv_sw);
+    }
+    c.pixels = keep(pix.data(), pix.size() * 4);
+    c.stride = S; c.group = best_r; c.quads = W; c.OW = H; c.OH = static_cast<int32_t>(bands); c.res_sw = static_cast<int32_t>(N * bands);
+    c.in_sn = pw; c.in_sh = l2.pad_top; c.in_sw = l2.pad_left; c.row_sh = OH; c.res_sn = OW;
+    c.res_sh = static_cast<int32_t>((static_cast<uint32_t>(fill) & 0xffu) * 0x01010101u);
+    c.inv_c4 = 1.0f / static_cast<float>(N * bands);
+    c.inv_quads = 1.0f / static_cast<float>(W);
+    c.inv_OH = 1.0f / static_cast<float>(bands);
+    c.inv_p_tiles = 1.0f / static_cast<float>(OW);
+    c.out_sn = 0;
+    std::array<int32_t, kProgramStepWords> w{};
+    std::memcpy(w.data(), &c, sizeof c);
+    std::memcpy(w.data() + kProgramStepWords / 2, &d, sizeof d);
+    steps.push_back(w);
+    return true;
+}
+
 bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out, void* planes) {
     ConvLaunch l;
     if (!conv_launch_arguments(conv, in, residual, out, l)) return false;
     if (planes) planes_arguments(l.a, planes);
     const ConvArgs& a = l.a;
     const int64_t M = a.M;
-    if (M > (1 << 20) || a.koff_tile || (a.flags & CF_OUT_I32) || ((a.flags & CF_OUT_FQ) && !(a.flags & CF_FQ_RCP)) || (a.flags & (CF_RES_SUB | CF_POST_SCALE)))
-        return false;
     const bool f32_out = !(a.flags & CF_OUT_FQ), f32_res = (a.flags & CF_RES_F32) != 0;
-    for (int64_t bytes : {static_cast<int64_t>(out.n) * a.out_sn * (f32_out ? 4 : 1), static_cast<int64_t>(out.n) * a.res_sn * (f32_res ? 4 : 1)})
-        if (bytes >= kBeyond) return false;
     ProgConv c{};
-    c.in = ref(a.in + a.in_origin);
-    c.out = ref(a.out);
-    c.res = a.res ? ref(a.res) : ProgRef{-2, 0, 0};
-    c.in2 = ProgRef{-2, 0, 0};
-    const int channels = planes ? a.OC : a.out_sw;       // that the output holds
-    c.out_limit = channels;
-    c.res_limit = a.res_sw;
-    {   // the tables the flags ask for, in load_constants' order
-        const uint32_t fl = a.flags;
-        std::vector<const void*> rows{a.corr};
-        if (fl & CF_BIAS) rows.push_back(a.bias);
-        if (fl & CF_SCALE) rows.push_back(a.scale);
-        if (fl & CF_RES_MUL) rows.push_back(a.res_mul);
-        if (fl & CF_OUT_FQ) {
-            rows.push_back(a.fq_r);
-            rows.push_back((fl & CF_FQ_DIV2) ? a.fq_r2 : a.fq_d);
-            if (!(fl & CF_FQ_SAT)) rows.push_back(a.fq_ih);
-            if (!(fl & CF_FQ_IL0)) rows.push_back(a.fq_il);
-        }
-        c.constants = gather(rows, static_cast<size_t>(a.OCp) * 4);
-    }
-    c.flags = a.flags; c.lm1 = a.lm1; c.off_bytes = (static_cast<uint32_t>(static_cast<int>(a.out_off)) & 0xffu) * 0x01010101u; c.clamp_lo = a.clamp_lo; c.clamp_hi = a.clamp_hi;
-    c.OCp = a.OCp;
+    if (!layer(a, out, c)) return false;
     if (l.depthwise) {
-        c.OH = a.OHOW / a.OW;
-        c.OW = a.OW;
-        if (l.kh != 3 || l.kw != 3 || l.dil_h != 1 || l.dil_w != 1 || a.conv_sh != a.conv_sw || a.conv_sh > 2 || !a.wgt2 || a.in_sw < a.out_sw) return false;
-        c.kind = PK_DW;
-        map_kinds = true;
-        c.stride = a.conv_sh;
-        c.wgt = ptr(a.wgt2);
-        c.in_sn = a.in_sn; c.in_sh = a.in_sh * a.conv_sh; c.in_sw = a.in_sw; c.row_sh = a.in_sh;
-        c.out_sn = a.out_sn; c.out_sh = a.out_sh; c.out_sw = a.out_sw;
-        c.res_sn = a.res_sn; c.res_sh = a.res_sh; c.res_sw = a.res_sw;
-        c.c4 = a.out_sw / 4;
+        if (!depthwise(l, c)) return false;
         // four pixels a lane where a step has more values than that leaves lanes idle
         c.group = static_cast<int64_t>(out.n) * c.OH * a.OW * c.c4 <= static_cast<int64_t>(workgroups) * kProgramThreads ? 1 : 4;
         c.quads = static_cast<int32_t>(ceil_div(a.OW, c.group));
@@ -1641,26 +1910,17 @@ bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hip
     const TileChoice t = choose_tile(workgroups, a.OC, M, a.nk, pair ? a.nk2 : 0, (a.flags & CF_GELU) != 0);
     c.a = t.a; c.b = t.b; c.ks_shift = __builtin_ctz(static_cast<unsigned>(t.ks));
     // (the channels the tensor is padded with are written too)
-    const int o_tiles = static_cast<int>(ceil_div(std::min(channels, a.OCp), 16 * t.a));
+    const int o_tiles = static_cast<int>(ceil_div(std::min(c.out_limit, a.OCp), 16 * t.a));
     c.p_tiles = static_cast<int32_t>(ceil_div(M, 16 * t.b));
     c.inv_p_tiles = 1.0f / static_cast<float>(c.p_tiles);
     const int64_t tiles = static_cast<int64_t>(c.p_tiles) * o_tiles;
     if (tiles * workgroups >= (1ll << 31) || tiles >= (1 << 24) || static_cast<int64_t>(a.nk) * t.a * 1024 >= kBeyond) return false;
     c.tiles = static_cast<int32_t>(tiles);
     if (!(a.k_linear && (!pair || a.k_linear2))) c.koff = ptr(a.koff);       // (0: the kernel's own table, 16 i)
-    auto repack = [&](const int8_t* w, int Kp) {
-        owned.emplace_back();
-        const int64_t pieces = static_cast<int64_t>(o_tiles) * t.a * Kp;        // 16 a x Kp bytes per tile, 16 bytes a piece
-        owned.back().alloc(device, static_cast<size_t>(pieces) * 16);
-        hipLaunchKernelGGL(pack_fragments_kernel, dim3(static_cast<uint32_t>(ceil_div(pieces, 256))), dim3(256), 0, nullptr, w, owned.back().as<int8_t>(), t.a,
-                           a.OCp, Kp, pieces);
-        HIPIE_CHECK_HIP(hipGetLastError());
-        return ptr(owned.back().ptr);
-    };
-    c.wgt = repack(a.wgt, a.Kp);
+    c.wgt = fragments(a.wgt, o_tiles, t.a, a.OCp, a.Kp);
     if (pair) {
         c.in2 = ref(a.in2 + a.in2_origin);
-        c.wgt2 = repack(a.wgt2, a.Kp2);
+        c.wgt2 = fragments(a.wgt2, o_tiles, t.a, a.OCp, a.Kp2);
         c.koff2 = ptr(a.koff2);
         c.nk2 = a.nk2;
         c.constants2 = gather({a.corr2, a.bias2, a.scale2}, static_cast<size_t>(a.OCp) * 4);

@@ -26,6 +26,8 @@ GRAPHS = {
     "resnet_3_u8": lambda: builders.resnet50(batch=3, res=96, u8_input=True)[0],
     "resnet_7_u8": lambda: builders.resnet50(batch=7, res=96, u8_input=True)[0],
     "mobilenet_2": lambda: builders.mobilenet_v2(batch=2, res=96)[0],
+    "mobilenet_1x160": lambda: builders.mobilenet_v2(batch=1, res=160)[0],                  # maps of 80, 40, 20, 10 and 5
+    "mobilenet_3x64": lambda: builders.mobilenet_v2(batch=3, res=64)[0],                    # ... of 32, 16, 8, 4 and 2
     "encoder_1x32": lambda: builders.bert_encoder(layers=1, batch=1, seq=32, vocab=100, mask=True)[0],
     "encoder_3x96": lambda: builders.bert_encoder(layers=1, batch=3, seq=96, vocab=0, mask=False)[0],
     "encoder_1x512": lambda: builders.bert_encoder(layers=1, batch=1, seq=512, vocab=100, mask=True)[0],
