@@ -97,6 +97,22 @@ bool conv_takes_planes(const hipie_conv* c, int64_t n, int64_t oh, int64_t ow);
 int conv_run_planes(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor& out, void* planes, hipStream_t s);
 void planes_arguments(ConvArgs& a, void* planes);
 
+// a 1 x 1 convolution and the depthwise 3 x 3 layer that alone reads it in one launch (expand_dw.hip); form 0: 32 channels a
+// workgroup, 1: the same in bands of half the height, 2: 48 channels, 3: 32 channels of several small images.
+// expand_dw_geometry: ok = false where the kernel does not take the layers
+constexpr int kExpandForms = 4;
+struct ExpandGeometry {
+    bool ok;
+    int tiles, quads, patch_w, slabs, rows, bands, images;
+    size_t lds;
+};
+bool expand_dw_epilogues_fit(uint32_t flags1, uint32_t flags2);
+ExpandGeometry expand_dw_geometry(int channels, int images, int h, int w, int oh, int ow, int stride, int pad_top, int pad_left, int form);
+void launch_expand_dw(const ConvLaunch& first, const ConvLaunch& second, int images, int h, int w, int fill, int form, hipStream_t s);
+// ... of two layers' objects: whether the form takes them (`mid`: the tensor between them, whose bytes nobody touches)
+bool conv_expand_fits(const hipie_conv* first, const hipie_conv* second, const hipie_tensor& mid, const hipie_tensor& out, int form);
+void conv_run_expand(const hipie_conv* first, const hipie_conv* second, const hipie_tensor& in, const hipie_tensor& mid, const hipie_tensor& out, int fill, int form, hipStream_t s);
+
 // frees the split-K workspace kept for this stream, if any (for the owner of a stream, before it destroys
 // the stream and after the stream's work has finished)
 void release_split_workspace(int device, hipStream_t s);

@@ -2519,3 +2519,23 @@ bool hipie::conv_launch_arguments(const hipie_conv* c, const hipie_tensor& in, c
     l.pad_top = c->d.pad_top; l.pad_left = c->d.pad_left;
     return fill_conv_args(c, &in, residual, &out, l.a, oh, ow) != 0;
 }
+
+bool hipie::conv_expand_fits(const hipie_conv* first, const hipie_conv* second, const hipie_tensor& mid, const hipie_tensor& out, int form) {
+    const hipie_conv_desc &a = first->d, &b = second->d;
+    if (first->depthwise || first->fused || first->koff_tile || !second->depthwise || first->device != second->device) return false;
+    if (a.kh != 1 || a.kw != 1 || a.groups != 1 || a.stride_h != 1 || a.stride_w != 1 || a.pad_top || a.pad_left || a.pad_bottom || a.pad_right || a.in_c_stride % 16 != 0 ||
+        first->Kp > 3 * 64)
+        return false;
+    if (b.kh != 3 || b.kw != 3 || b.dil_h != 1 || b.dil_w != 1 || b.stride_h != b.stride_w || b.stride_h > 2 || b.ic != a.oc || b.oc != a.oc || b.in_dtype != first->epi.out_dtype)
+        return false;
+    if (!expand_dw_epilogues_fit(first->epi.flags, second->epi.flags)) return false;
+    return expand_dw_geometry(static_cast<int>(std::min(mid.stride_w, out.stride_w)), mid.n, mid.h, mid.w, out.h, out.w, b.stride_h, b.pad_top, b.pad_left, form).ok;
+}
+
+void hipie::conv_run_expand(const hipie_conv* first, const hipie_conv* second, const hipie_tensor& in, const hipie_tensor& mid, const hipie_tensor& out, int fill, int form, hipStream_t s) {
+    ConvLaunch l1, l2;
+    if (!conv_launch_arguments(first, in, nullptr, mid, l1) || !conv_launch_arguments(second, mid, nullptr, out, l2)) return;
+    DeviceGuard g(first->device);
+    launch_expand_dw(l1, l2, mid.n, mid.h, mid.w, fill, form, s);
+    HIPIE_CHECK_HIP(hipGetLastError());
+}

@@ -426,14 +426,16 @@ struct ConvStep : Step {
 
 // A 3 x 3 convolution and the 1 x 1 convolution that is its only reader (the tail of a bottleneck block), planned as
 // two layers and run either one after the other or - where hipie_conv_pair_fits takes them and it is faster - as one
-// kernel that keeps the tensor between them in LDS (hipie_conv_run_pair).  Same bits either way.
+// kernel that keeps the tensor between them in LDS (hipie_conv_run_pair).  Same bits either way.  With `expands`: a 1 x 1
+// convolution and the depthwise layer that is its only reader (conv_run_expand).
 struct PairStep : Step {
+    bool expands = false;
     std::unique_ptr<ConvStep> first, second;
     int mode = 1;                  // PlanConfig::fuse_convs
-    bool fits = false, fused = false, fits_groups = false;
+    bool fits = false, fused = false;
     // form of the fused kernel: 0 three steps of weights in flight, 1 nine steps (one workgroup per compute unit),
-    // 2 eight waves in two groups (where fits_groups)
-    int form = 0;
+    // 2 eight waves in two groups; with `expands` those of expand_dw.hip.  forms: bit f where form f takes the layers
+    int form = 0, forms = 0;
     static int stages_of(int form) { return form == 1 ? 8 : (form == 2 ? 7 : 0); }
     void create(int, const std::vector<TensorInfo>& tensors) override {   // (the layers exist already)
         name = second->name;
@@ -446,21 +448,33 @@ struct PairStep : Step {
         runtime_precision = first->runtime_precision;
         output_precision = second->output_precision;
         output_layout = second->output_layout;
-        const TensorInfo& ti = tensors[first->in];
-        int f = 0;
-        check_status(hipie_conv_pair_fits(first->conv, second->conv, ti.h, ti.w, &f), name.c_str());
-        fits = f != 0 && ti.halo >= 1 && second->res >= 0 && second->res_param < 0;
-        fits_groups = fits && (f & 2) != 0;
-        const TensorInfo& tm = tensors[first->out];
+        const TensorInfo &ti = tensors[first->in], &tm = tensors[first->out];
+        if (expands) {
+            for (int f = kExpandForms - 1; f >= 0; --f)
+                if (takes(f, tensors)) {
+                    fits = true;
+                    forms |= 1 << f;
+                    form = f;
+                }
+        } else {
+            int f = 0;
+            check_status(hipie_conv_pair_fits(first->conv, second->conv, ti.h, ti.w, &f), name.c_str());
+            fits = f != 0 && ti.halo >= 1 && second->res >= 0 && second->res_param < 0;
+            forms = fits ? ((f & 2) != 0 ? 7 : 3) : 0;
+        }
         mid_bytes = static_cast<int64_t>(tm.n) * tm.h * tm.w * tm.c;
         choose(fits && mode == 2);
+    }
+    // whether form f takes a dense layer and the depthwise layer behind it
+    bool takes(int f, const std::vector<TensorInfo>& tensors) const {
+        return conv_expand_fits(first->conv, second->conv, tensors[first->out].desc(nullptr), tensors[second->out].desc(nullptr), f);
     }
     int64_t mid_bytes = 0;         // the tensor between the layers: written and read when they run apart
     void choose(bool one_kernel) {
         fused = one_kernel;
         // the depth is a setting of the first layer's object: the pair's when they run as one kernel, else its own
-        if (first->conv) check_status(hipie_conv_set_stages(first->conv, fused ? stages_of(form) : (first->deep ? 8 : 0)), name.c_str());
-        type = fused ? "Convolution+Convolution" : "Convolution,Convolution";
+        if (first->conv) check_status(hipie_conv_set_stages(first->conv, fused && !expands ? stages_of(form) : (first->deep ? 8 : 0)), name.c_str());
+        type = std::string(fused ? "Convolution+" : "Convolution,") + (expands ? "GroupConvolution" : "Convolution");
         bytes = first->bytes + second->bytes - (fused ? 2 * mid_bytes : 0);
     }
     int launches() const override { return fused ? 1 : first->launches() + second->launches(); }
@@ -469,7 +483,13 @@ struct PairStep : Step {
     }
     double valu_ops() const override { return first->valu_ops() + second->valu_ops(); }
     void run_fused(uint8_t* arena, const std::vector<TensorInfo>& tensors, hipStream_t s) const {
-        const hipie_tensor i = tensors[first->in].desc(arena), o = tensors[second->out].desc(arena), r = tensors[second->res].desc(arena);
+        const hipie_tensor i = tensors[first->in].desc(arena), o = tensors[second->out].desc(arena);
+        if (expands) {
+            const TensorInfo& mid = tensors[first->out];
+            conv_run_expand(first->conv, second->conv, i, mid.desc(arena), o, mid.dtype == HIPIE_U8B ? mid.fill_level - 128 : mid.fill_level, form, s);
+            return;
+        }
+        const hipie_tensor r = tensors[second->res].desc(arena);
         check_status(hipie_conv_run_pair(first->conv, second->conv, &i, &r, &o, s), name.c_str());
     }
     void run(uint8_t* arena, const std::vector<TensorInfo>& tensors, void* const* inputs, void* const* outputs,
@@ -496,8 +516,11 @@ struct PairStep : Step {
                 for (size_t l = 0; l < nl; ++l) run_fused(lanes[l].arena, tensors, lanes[l].stream);
         };
         float best_fused = 0.f;
-        for (int d = 0; d < (fits_groups ? 3 : 2); ++d) {
-        check_status(hipie_conv_set_stages(first->conv, stages_of(d)), name.c_str());
+        int best_form = -1;
+        for (int d = 0; d < 4; ++d) {
+        if (!(forms >> d & 1)) continue;
+        form = d;
+        if (!expands) check_status(hipie_conv_set_stages(first->conv, stages_of(d)), name.c_str());
         launch_all(2);
         float ms = 0.f;   // the same protocol as the layers' own variants: fastest of three rounds of five launches per lane
         for (int round = 0; round < 3; ++round) {
@@ -515,11 +538,12 @@ struct PairStep : Step {
                 }
             ms = round == 0 ? span : std::min(ms, span);
         }
-        if (d == 0 || ms < 0.97f * best_fused) {
+        if (best_form < 0 || ms < 0.97f * best_fused) {
             best_fused = ms;
-            form = d;
+            best_form = d;
         }
         }
+        form = best_form;
         for (size_t l = 0; l < nl; ++l) {
             (void)hipEventDestroy(e0[l]);
             (void)hipEventDestroy(e1[l]);
@@ -528,7 +552,7 @@ struct PairStep : Step {
         choose(mode == 2 || (apart_us > 0.f && fused_us < 0.97f * apart_us));
         if (std::getenv("HIPIE_TUNE_LOG"))
             std::fprintf(stderr, "hipie tune: %-28s one kernel %.1f us (%s), two %.1f us per launch with %zu in flight: %s\n", name.c_str(),
-                         fused_us, form == 2 ? "two wave groups" : (form == 1 ? "nine steps in flight" : "three steps in flight"), apart_us, nl,
+                         fused_us, expands ? (form == 3 ? "several images" : form == 2 ? "48 channels" : form == 1 ? "32 channels, low bands" : "32 channels") : form == 2 ? "two wave groups" : (form == 1 ? "nine steps in flight" : "three steps in flight"), apart_us, nl,
                          fused ? "fused" : "apart");
     }
     // the layers' variants and the choice between one kernel and two, in one integer
@@ -538,7 +562,7 @@ struct PairStep : Step {
         first->set_variant(v & 63);
         second->set_variant((v >> 6) & 63);
         form = (v >> 13) & 3;
-        if (form == 3 || (form == 2 && !fits_groups)) form = 0;
+        if (!(forms >> form & 1)) form = forms ? __builtin_ctz(static_cast<unsigned>(forms)) : 0;
         choose(fits && (v & 4096) != 0 && mode != 0);
     }
 };
@@ -3127,6 +3151,10 @@ std::shared_ptr<ProgramForm> build_program(const hipie_plan& p, int workgroups, 
                 continue;
             }
         }
+        if (const auto* pair = dynamic_cast<const PairStep*>(s); pair && pair->expands && !keep_values && pair->first->joins(*pair->second, b, p.tensors)) {
+            inside.push_back(pair->first->out);
+            continue;
+        }
         if (!s->program(b, p.tensors, in.data(), out.data())) {
             refused = s->name;
             return nullptr;
@@ -3354,6 +3382,31 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
             plan->steps[j] = std::move(pair);
             plan->steps.erase(plan->steps.begin() + static_cast<std::ptrdiff_t>(i));
             --i;
+        }
+    // A 1 x 1 convolution whose result only the next depthwise layer reads: one step, and one launch where that is faster
+    // (values that are kept stay two steps, and so do layers that nothing measures: choices of a plan that had them apart,
+    // plans without a device, plans that are not tuned)
+    const bool measured_pairs = device >= 0 && (preset ? preset->size() != plan->steps.size() : cfg.tune);
+    if (!cfg.keep_f32 && (cfg.fuse_convs == 2 || (cfg.fuse_convs == 1 && measured_pairs)))
+        for (size_t i = 0; i + 1 < plan->steps.size(); ++i) {
+            auto* a = dynamic_cast<ConvStep*>(plan->steps[i].get());
+            auto* b = dynamic_cast<ConvStep*>(plan->steps[i + 1].get());
+            if (!a || !b || !a->conv || !b->conv || b->in != a->out || a->out_node < 0 || g->nodes[a->out_node].users.size() != 1) continue;
+            const TensorInfo& mid = plan->tensors[a->out];
+            if (a->shortcut || a->res >= 0 || a->res_param >= 0 || a->writes_result || b->shortcut || b->res >= 0 || b->res_param >= 0 || b->writes_result ||
+                mid.alias >= 0 || !mid.fill_levels.empty())
+                continue;
+            auto pair = std::make_unique<PairStep>();
+            pair->expands = true;
+            pair->mode = cfg.fuse_convs;
+            bool fits = false;
+            for (int f = 0; f < kExpandForms && !fits; ++f) fits = conv_expand_fits(a->conv, b->conv, mid.desc(nullptr), plan->tensors[b->out].desc(nullptr), f);
+            if (!fits) continue;
+            pair->first.reset(static_cast<ConvStep*>(plan->steps[i].release()));
+            pair->second.reset(static_cast<ConvStep*>(plan->steps[i + 1].release()));
+            pair->create(device, plan->tensors);
+            plan->steps[i] = std::move(pair);
+            plan->steps.erase(plan->steps.begin() + static_cast<std::ptrdiff_t>(i) + 1);
         }
     {
         // the edges of the executed graph (what GetExecGraphInfo draws): an operand of a step is a node outside its set -

@@ -1,0 +1,68 @@
+"""A 1 x 1 convolution and the depthwise 3 x 3 layer that alone reads it in one launch (csrc/expand_dw.hip), in every form it
+has, against the two layers' own kernels bit for bit: bands and columns with remainders, strides, padding, one K step and three,
+channels that fill a workgroup's and that do not, fewer units than compute units and more, the three epilogues."""
+import numpy as np
+import pytest
+import torch
+
+from dldt_amd import HipieError
+from dldt_amd.builders import QuantizedNet
+
+pytestmark = pytest.mark.gpu
+
+#        n, c, h, w, channels, stride and padding of the depthwise layer, top of the range (above 6: the Clamp stays), ReLU6 or not
+CASES = {
+    "columns_17": (1, 16, 13, 17, 48, 1, 1, 3.0, True),
+    "stride_2_odd": (3, 24, 15, 9, 80, 2, 1, 3.0, True),
+    "stride_2_unpadded": (2, 16, 12, 20, 32, 2, 0, 8.0, True),
+    "unpadded": (1, 64, 7, 5, 16, 1, 0, 3.0, True),
+    "padded_by_2": (1, 65, 6, 6, 16, 1, 2, 8.0, True),
+    "three_k_steps": (2, 160, 9, 7, 104, 1, 1, 3.0, True),
+    "one_pixel": (5, 32, 1, 1, 16, 1, 1, 3.0, True),
+    "wide_rows": (2, 16, 30, 111, 96, 2, 1, 3.0, True),
+    "many_units": (9, 24, 40, 24, 144, 1, 1, 3.0, True),
+    "small_images": (65, 16, 7, 7, 368, 1, 1, 3.0, True),
+    "small_images_stride_2": (70, 24, 7, 9, 368, 2, 1, 3.0, True),
+    "no_scale": (3, 48, 21, 19, 70, 1, 1, 3.0, False),
+    "no_scale_stride_2": (3, 48, 21, 19, 70, 2, 1, 3.0, False),
+}
+
+
+def _graph(n, c, h, w, oc, stride, pads, high, relu6):
+    rng = np.random.default_rng(oc * h)
+    net = QuantizedNet()
+    a = net.input("data", (n, c, h, w), 2.0)
+    conv = net.conv_relu6 if relu6 else net.conv
+    mid = conv(a, rng.normal(0, 1 / np.sqrt(c), (oc, c, 1, 1)).astype(np.float32), rng.normal(0, 0.2, oc).astype(np.float32), high)
+    b = conv(mid, rng.normal(0, 0.4, (oc, 1, 3, 3)).astype(np.float32), rng.normal(0, 0.2, oc).astype(np.float32), high, strides=(stride, stride), pads=(pads, pads), grouped=True)
+    net.g.result(net.conv_f32(b, rng.normal(0, 0.2, (24, oc, 1, 1)).astype(np.float32), None), "out")
+    return net.g, mid["node"]
+
+
+@pytest.mark.parametrize("name,form", [(n, f) for n in sorted(CASES) for f in range(4) if f < 3 or n.startswith("small")])
+def test_one_launch_equals_two(name, form, tmp_path):
+    g, mid = _graph(*CASES[name])
+    base = {"HIP_THROUGHPUT_STREAMS": "1", "HIP_SINGLE_LAUNCH": "NO"}
+    apart = g.compile(0, config=dict(base, HIP_TUNE="NO", HIP_FUSE_CONVOLUTIONS="NO"))
+    default = g.compile(0, config=dict(base, HIP_TUNE="NO", HIP_FUSE_CONVOLUTIONS="YES"))
+    pair = [i for i, s in enumerate(default.steps) if s["type"] == "Convolution+GroupConvolution"]
+    assert len(pair) == 1
+    choices = tmp_path / "choices"
+    choices.write_text("".join(f"{i} {s['variant'] % 8192 + 8192 * form if i in pair else s['variant']}\n" for i, s in enumerate(default.steps)))
+    fused = g.compile(0, config=dict(base, HIP_TUNE="YES", HIP_TUNE_FILE=str(choices), HIP_FUSE_CONVOLUTIONS="YES"))
+    assert fused.steps[pair[0]]["variant"] >> 13 == form
+    results = []
+    x = torch.rand(CASES[name][:4], generator=torch.Generator(device="cuda").manual_seed(form), device="cuda") * 2
+    reqs = [p.create_request() for p in (apart, fused)]
+    for r in reqs:
+        ins, outs = r.device_buffers()
+        ins[0].copy_(x)
+        outs[0].fill_(float("nan"))
+        torch.cuda.synchronize()
+        r.infer_device(ins, outs)
+        results.append(outs[0].cpu().numpy())
+    assert not np.isnan(results[0]).any() and np.abs(results[0]).max() > 0
+    assert np.array_equal(results[0].view(np.uint32), results[1].view(np.uint32))
+    assert reqs[0].tensor(mid) is not None
+    with pytest.raises(HipieError, match="LDS only"):
+        reqs[1].tensor(mid)
