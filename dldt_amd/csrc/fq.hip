@@ -25,25 +25,82 @@ __device__ __forceinline__ uint32_t pack_levels(float k0, float k1, float k2, fl
     return b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
 }
 
-// [N, C, HW] f32 -> same layout, one byte per element.  hw4 = HW / 4 (HW % 4 == 0).
-template <bool RCP>
-__global__ __launch_bounds__(kThreads) void fq_nchw_q8_vec4(const float4* __restrict__ x,
-                                                             uint32_t* __restrict__ y,
-                                                             const FqChannel* __restrict__ tab,
-                                                             float lm1, float off, int64_t n4,
-                                                             uint32_t hw4, uint32_t C) {
-    const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < n4; i += stride) {
-        const uint32_t plane = static_cast<uint32_t>(i / hw4);
-        const FqChannel p = tab[plane % C];
-        const float4 v = x[i];
-        y[i] = pack_levels(fq_level_clamped<RCP>(p, lm1, v.x), fq_level_clamped<RCP>(p, lm1, v.y),
-                           fq_level_clamped<RCP>(p, lm1, v.z), fq_level_clamped<RCP>(p, lm1, v.w),
-                           off);
+int grid_for(int64_t work_items) {
+    // enough blocks to fill 256 CUs several times over, capped so the grid-stride loop amortises
+    const int64_t blocks = ceil_div(work_items, kThreads);
+    return static_cast<int>(std::min<int64_t>(blocks, 256 * 16));
+}
+
+// x / d for every 32-bit x: a product with floor(2^32 / d) is the quotient or one less (d = 1: with 2^32 - 1)
+struct Divider {
+    uint32_t d, m;
+    explicit Divider(uint32_t by) : d(by), m(by == 1 ? 0xffffffffu : static_cast<uint32_t>((1ull << 32) / by)) {}
+    __device__ __forceinline__ uint32_t operator()(uint32_t x, uint32_t& rest) const {
+        uint32_t q = __umulhi(x, m);
+        rest = x - q * d;
+        if (rest >= d) { ++q; rest -= d; }
+        return q;
+    }
+};
+
+// [N, C, HW] f32 -> the same layout, bytes (LEVELS) or f32: four consecutive elements a thread whatever HW is, in whole
+// 16-byte loads and stores; where a plane ends among the four, the ones behind it are quantised with the next channel's
+// ranges (WHOLE: HW % 4 == 0, no plane does, and `hw` divides by HW / 4).  Bound by memory, below some 10^6 elements by the
+// launch: [32, 256, 55, 57] -> f32 33.5 us = 6.1 TB/s (an element a thread with 64-bit divisions: 59.2), -> u8 21.3 (36.7).
+template <bool RCP, bool LEVELS, bool WHOLE>
+__global__ __launch_bounds__(kThreads) void fq_nchw_flat(const float* __restrict__ x, void* __restrict__ y, const FqChannel* __restrict__ tab,
+                                                         float lm1, float off, uint32_t total, Divider hw, Divider C) {
+    const uint32_t stride = gridDim.x * kThreads, groups = total / 4 + (total % 4 != 0);
+    for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < groups; i += stride) {
+        const bool whole = WHOLE || 4 * i + 4 <= total;
+        float v[4], k[4];
+        if (whole) {
+            const float4 q = reinterpret_cast<const float4*>(x)[i];
+            v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+        } else {
+            for (uint32_t j = 0; j < 4; ++j) v[j] = x[min(4 * i + j, total - 1)];
+        }
+        uint32_t at, c;
+        C(hw(WHOLE ? i : 4 * i, at), c);
+        const FqChannel p = tab[c];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) k[j] = LEVELS ? fq_level_clamped<RCP>(p, lm1, v[j]) : fq_value<RCP>(p, lm1, v[j]);
+        const uint32_t left = hw.d - at;                // elements of the plane from this one on
+        if (!WHOLE && left < 4) {
+            const FqChannel n = tab[c + 1 == C.d ? 0 : c + 1];
+#pragma unroll
+            for (uint32_t j = 1; j < 4; ++j)
+                if (j >= left) k[j] = LEVELS ? fq_level_clamped<RCP>(n, lm1, v[j]) : fq_value<RCP>(n, lm1, v[j]);
+        }
+        if (LEVELS) {
+            const uint32_t b = pack_levels(k[0], k[1], k[2], k[3], off);
+            if (whole) static_cast<uint32_t*>(y)[i] = b;
+            else
+                for (uint32_t j = 0; 4 * i + j < total; ++j) static_cast<uint8_t*>(y)[4 * i + j] = static_cast<uint8_t>(b >> (8 * j));
+        } else {
+            if (whole) static_cast<float4*>(y)[i] = make_float4(k[0], k[1], k[2], k[3]);
+            else
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j)
+                    if (4 * i + j < total) static_cast<float*>(y)[4 * i + j] = k[j];
+        }
     }
 }
 
-// any HW: one element per thread-iteration
+template <bool LEVELS>
+void launch_flat(bool rcp, const float* x, void* y, const FqChannel* tab, float lm1, float off, int64_t total, int64_t hw, uint32_t C, hipStream_t s) {
+    const dim3 grid(grid_for(ceil_div(total, 4))), block(kThreads);
+    const uint32_t n = static_cast<uint32_t>(total);
+    if (hw % 4 == 0) {
+        auto k = rcp ? fq_nchw_flat<true, LEVELS, true> : fq_nchw_flat<false, LEVELS, true>;
+        hipLaunchKernelGGL(k, grid, block, 0, s, x, y, tab, lm1, off, n, Divider(static_cast<uint32_t>(hw / 4)), Divider(C));
+    } else {
+        auto k = rcp ? fq_nchw_flat<true, LEVELS, false> : fq_nchw_flat<false, LEVELS, false>;
+        hipLaunchKernelGGL(k, grid, block, 0, s, x, y, tab, lm1, off, n, Divider(static_cast<uint32_t>(hw)), Divider(C));
+    }
+}
+
+// planes of fewer than three elements, buffers off the 16-byte boundary, 2^32 elements and more: one element per thread and iteration
 template <bool RCP>
 __global__ __launch_bounds__(kThreads) void fq_nchw_q8_scalar(const float* __restrict__ x,
                                                                uint8_t* __restrict__ y,
@@ -71,25 +128,6 @@ __global__ __launch_bounds__(kThreads) void fq_nchw_f32(const float* __restrict_
     }
 }
 
-template <bool RCP>
-__global__ __launch_bounds__(kThreads) void fq_nchw_f32_vec4(const float4* __restrict__ x,
-                                                              float4* __restrict__ y,
-                                                              const FqChannel* __restrict__ tab,
-                                                              float lm1, int64_t n4, uint32_t hw4,
-                                                              uint32_t C) {
-    const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < n4; i += stride) {
-        const FqChannel p = tab[static_cast<uint32_t>(i / hw4) % C];
-        const float4 v = x[i];
-        float4 o;
-        o.x = fq_value<RCP>(p, lm1, v.x);
-        o.y = fq_value<RCP>(p, lm1, v.y);
-        o.z = fq_value<RCP>(p, lm1, v.z);
-        o.w = fq_value<RCP>(p, lm1, v.w);
-        y[i] = o;
-    }
-}
-
 // [N, C, HW] f32 -> [N, HW, c_stride] bytes.  A block transposes 64 pixels x 64 channels
 // through LDS so that both the f32 reads (256 B per channel row) and the byte writes (16 B per
 // thread, whole pixels contiguous) are coalesced.  grid = (N * ceil(HW/64), ceil(c_stride/64)).
@@ -102,24 +140,27 @@ __global__ __launch_bounds__(kThreads) void fq_nchw_to_nhwc_q8(const TIn* __rest
                                                                 uint32_t tiles_per_image, uint32_t W,
                                                                 int64_t out_sn, int64_t out_sh) {
     __shared__ uint32_t tile[64][17];  // [pixel][16 dwords = 64 channel bytes] + 1 pad
+    __shared__ __attribute__((aligned(16))) FqChannel chan[64];
     const uint32_t n = blockIdx.x / tiles_per_image;
     const uint32_t p0 = (blockIdx.x % tiles_per_image) * 64;
     const uint32_t c0 = blockIdx.y * 64;
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t pix = p0 + lane;
-    // each wave quantises 16 channels of the 64; a lane owns one pixel and packs 4 channels/dword
+    // each wave quantises 16 channels of the 64, all requested before the first is used; a lane owns one pixel and packs 4
+    // channels a dword
+    if (threadIdx.x < 64) chan[threadIdx.x] = tab[min(c0 + threadIdx.x, C - 1)];
+    float v[16];
+#pragma unroll
+    for (uint32_t j = 0; j < 16; ++j) {
+        const uint32_t c = c0 + wave * 16 + j;
+        v[j] = c < C && pix < hw ? static_cast<float>(x[(static_cast<int64_t>(n) * C + c) * hw + pix]) : 0.0f;
+    }
+    __syncthreads();
+#pragma unroll
     for (uint32_t cc = 0; cc < 16; cc += 4) {
         float k[4];
 #pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
-            const uint32_t c = c0 + wave * 16 + cc + j;
-            if (c < C && pix < hw) {
-                const FqChannel p = tab[c];
-                k[j] = fq_level_clamped<RCP>(p, lm1, static_cast<float>(x[(static_cast<int64_t>(n) * C + c) * hw + pix]));
-            } else {
-                k[j] = 0.0f;
-            }
-        }
+        for (uint32_t j = 0; j < 4; ++j) k[j] = c0 + wave * 16 + cc + j < C && pix < hw ? fq_level_clamped<RCP>(chan[wave * 16 + cc + j], lm1, v[cc + j]) : 0.0f;
         tile[lane][wave * 4 + cc / 4] = pack_levels(k[0], k[1], k[2], k[3], off);
     }
     __syncthreads();
@@ -144,14 +185,22 @@ __global__ __launch_bounds__(kThreads) void fq_nchw_to_nhwc_q8(const TIn* __rest
     }
 }
 
-__device__ __forceinline__ float4 load4_as_float(const float* p) { return *reinterpret_cast<const float4*>(p); }
-__device__ __forceinline__ float4 load4_as_float(const uint8_t* p) {   // convert<uint8_t, float>: exact
-    const uint32_t w = *reinterpret_cast<const uint32_t*>(p);
+// four consecutive elements of a plane that has `left` from here on, at any element's address (what is behind the plane is 0)
+typedef float unaligned_float4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t unaligned_uint32 __attribute__((aligned(1)));
+__device__ __forceinline__ float4 load4_as_float(const float* p, uint32_t left) {
+    if (left < 4) return make_float4(p[0], left > 1 ? p[1] : 0.f, left > 2 ? p[2] : 0.f, 0.f);
+    const unaligned_float4 v = *reinterpret_cast<const unaligned_float4*>(p);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ float4 load4_as_float(const uint8_t* p, uint32_t left) {   // convert<uint8_t, float>: exact
+    if (left < 4) return make_float4(static_cast<float>(p[0]), left > 1 ? static_cast<float>(p[1]) : 0.f, left > 2 ? static_cast<float>(p[2]) : 0.f, 0.f);
+    const uint32_t w = *reinterpret_cast<const unaligned_uint32*>(p);
     return make_float4(static_cast<float>(w & 0xffu), static_cast<float>((w >> 8) & 0xffu),
                        static_cast<float>((w >> 16) & 0xffu), static_cast<float>(w >> 24));
 }
 
-// The same transposition for HW % 4 == 0, 256 pixels x 64 channels per workgroup.  A lane reads float4s (four
+// The same transposition for planes below 2^24 pixels, 256 pixels x 64 channels per workgroup.  A lane reads float4s (four
 // consecutive pixels of one channel; a wave's load instruction is 1 KB contiguous) of four consecutive channels at a
 // time, sixteen loads in flight per lane, and packs each pixel's four channels into one dword.  LDS holds the tile as
 // [16 channel dwords][256 pixels + 4]: the four dwords a lane produces per step are one conflict-free 16-byte write, and
@@ -171,7 +220,7 @@ __global__ __launch_bounds__(kThreads) void fq_nchw_to_nhwc_q8_wide(const TIn* _
     const uint32_t c0 = blockIdx.y * 64;
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t pix = p0 + 4 * lane;
-    const bool pix_on = pix < hw;                      // HW % 4 == 0: a group of four is inside or outside as a whole
+    const bool pix_on = pix < hw;
     if (threadIdx.x < 64) chan[threadIdx.x] = tab[min(c0 + threadIdx.x, C - 1)];
     float4 v[4][4];                                    // [step][channel of the quad]
 #pragma unroll
@@ -180,7 +229,7 @@ __global__ __launch_bounds__(kThreads) void fq_nchw_to_nhwc_q8_wide(const TIn* _
         for (uint32_t j = 0; j < 4; ++j) {
             const uint32_t c = c0 + 4 * (wave + 4 * it) + j;
             v[it][j] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (pix_on && c < C) v[it][j] = load4_as_float(x + (static_cast<int64_t>(n) * C + c) * hw + pix);
+            if (pix_on && c < C) v[it][j] = load4_as_float(x + (static_cast<int64_t>(n) * C + c) * hw + pix, hw - pix);
         }
     __syncthreads();
 #pragma unroll
@@ -258,7 +307,7 @@ __global__ __launch_bounds__(kThreads) void fq_nchw_to_nhwc_q8_lines(const TIn* 
     const uint32_t c0 = blockIdx.y * 256;
     const uint32_t pg = threadIdx.x & 7, cq_lo = threadIdx.x >> 3;
     const uint32_t pix = p0 + 4 * pg;
-    const bool pix_on = pix < hw;                      // HW % 4 == 0: a group of four is inside or outside as a whole
+    const bool pix_on = pix < hw;
     chan[threadIdx.x] = tab[min(c0 + threadIdx.x, C - 1)];
     float4 v[2][4];                                    // [step][channel of the quad]
 #pragma unroll
@@ -267,7 +316,7 @@ __global__ __launch_bounds__(kThreads) void fq_nchw_to_nhwc_q8_lines(const TIn* 
         for (uint32_t j = 0; j < 4; ++j) {
             const uint32_t c = c0 + 4 * (cq_lo + 32 * it) + j;
             v[it][j] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (pix_on && c < C) v[it][j] = load4_as_float(x + (static_cast<int64_t>(n) * C + c) * hw + pix);
+            if (pix_on && c < C) v[it][j] = load4_as_float(x + (static_cast<int64_t>(n) * C + c) * hw + pix, hw - pix);
         }
     __syncthreads();
 #pragma unroll
@@ -353,7 +402,7 @@ __global__ __launch_bounds__(kThreads) void fq_nchw_to_nhwc4_q8(const TIn* __res
         }
 #pragma unroll
         for (uint32_t c = 0; c < 4; ++c)
-            if (c < C) v[t][c] = load4_as_float(x + ((static_cast<int64_t>(n) * C + c) * H + h[t]) * W + wq[t] * 4);
+            if (c < C) v[t][c] = load4_as_float(x + ((static_cast<int64_t>(n) * C + c) * H + h[t]) * W + wq[t] * 4, 4);
     }
 #pragma unroll
     for (uint32_t t = 0; t < kItems; ++t) {
@@ -378,12 +427,6 @@ __global__ __launch_bounds__(kThreads) void fq_nchw_to_nhwc4_q8(const TIn* __res
 #pragma unroll
         for (uint32_t p = 0; p < 4; ++p) dst[p] = pack_levels(k[p][0], k[p][1], k[p][2], k[p][3], off);
     }
-}
-
-int grid_for(int64_t work_items) {
-    // enough blocks to fill 256 CUs several times over, capped so the grid-stride loop amortises
-    const int64_t blocks = ceil_div(work_items, kThreads);
-    return static_cast<int>(std::min<int64_t>(blocks, 256 * 16));
 }
 
 // r = correctly rounded 1/d: pick among the neighbours of (float)(1.0/d) the one whose exact
@@ -507,6 +550,15 @@ struct hipie_fq {
     DeviceBuffer table;
 };
 
+// whether a transposition runs in tiles of 32 pixels x 256 channels or 256 x 64 (four pixels a lane) instead of 64 x 64 (one).
+// The former take every tensor whose channels make whole lines ([32, 256, 55, 57] 34.9 us, 40.0 in small tiles); the latter need
+// a workgroup for every compute unit, two of them where their loads are not aligned: small tiles / 256 x 64 in us,
+// [12, 72, 44, 44] (192 workgroups) 5.1 / 6.2, [64, 64, 28, 28] (256) 7.2 / 6.6, [64, 64, 31, 31] (256) 7.4 / 8.3,
+// [32, 96, 111, 111] (3136) 59.7 / 36.4.  The reciprocal decode ends at 2^24 pixels.
+bool wide_tiles(int64_t n, int64_t hw, int64_t cs) {
+    return hw < (1 << 24) && (cs >= 128 || n * ceil_div(hw, 256) * ceil_div(cs, 64) >= (hw % 4 == 0 ? 256 : 512));
+}
+
 template <typename TIn>
 void run_q8_tensor(const hipie_fq* fq, const TIn* x, const hipie_tensor* out, void* stream) {
     {
@@ -543,7 +595,7 @@ void run_q8_tensor(const hipie_fq* fq, const TIn* x, const hipie_tensor* out, vo
             HIPIE_CHECK_HIP(hipGetLastError());
             return;
         }
-        if (hw % 4 == 0 && hw < (1 << 24) && cs >= 128) {   // whole float4s per lane, whole cache lines per pixel
+        if (wide_tiles(out->n, hw, cs) && cs >= 128) {   // whole cache lines per pixel
             const uint32_t tiles = static_cast<uint32_t>(ceil_div(hw, 32));
             HIPIE_REQUIRE(static_cast<int64_t>(out->n) * tiles < (1ll << 31), HIPIE_OUT_OF_BOUNDS, "hipie_fq_run_q8_tensor: grid too large");
             auto kl = fq->rcp ? fq_nchw_to_nhwc_q8_lines<true, TIn> : fq_nchw_to_nhwc_q8_lines<false, TIn>;
@@ -555,7 +607,7 @@ void run_q8_tensor(const hipie_fq* fq, const TIn* x, const hipie_tensor* out, vo
             HIPIE_CHECK_HIP(hipGetLastError());
             return;
         }
-        if (hw % 4 == 0 && hw < (1 << 24)) {   // whole float4s per lane
+        if (wide_tiles(out->n, hw, cs)) {
             const uint32_t tiles = static_cast<uint32_t>(ceil_div(hw, 256));
             auto kw = fq->rcp ? fq_nchw_to_nhwc_q8_wide<true, TIn> : fq_nchw_to_nhwc_q8_wide<false, TIn>;
             hipLaunchKernelGGL(kw, dim3(static_cast<uint32_t>(out->n * tiles), static_cast<uint32_t>(ceil_div(cs, 64))),
@@ -771,15 +823,10 @@ int hipie_fq_run_f32(const hipie_fq* fq, const float* x, float* y, int64_t n, in
         DeviceGuard g(fq->device);
         const FqChannel* tab = fq->table.as<FqChannel>();
         const uint32_t C = static_cast<uint32_t>(fq->C);
-        const bool vec = hw % 4 == 0 && (reinterpret_cast<uintptr_t>(x) % 16 == 0) &&
-                         (reinterpret_cast<uintptr_t>(y) % 16 == 0);
         hipStream_t s = as_stream(stream);
-        if (vec) {
-            const int64_t n4 = total / 4;
-            auto k = fq->rcp ? fq_nchw_f32_vec4<true> : fq_nchw_f32_vec4<false>;
-            hipLaunchKernelGGL(k, dim3(grid_for(n4)), dim3(kThreads), 0, s,
-                               reinterpret_cast<const float4*>(x), reinterpret_cast<float4*>(y),
-                               tab, fq->lm1, n4, static_cast<uint32_t>(hw / 4), C);
+        // (a plane of three elements and more ends at most once among four)
+        if (hw >= 3 && total < (1ll << 32) - 4 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0) {
+            launch_flat<false>(fq->rcp, x, y, tab, fq->lm1, 0.0f, total, hw, C, s);
         } else {
             auto k = fq->rcp ? fq_nchw_f32<true> : fq_nchw_f32<false>;
             hipLaunchKernelGGL(k, dim3(grid_for(total)), dim3(kThreads), 0, s, x, y, tab, fq->lm1,
@@ -830,15 +877,8 @@ int hipie_fq_run_q8(const hipie_fq* fq, const float* x, void* y, int64_t n, int6
         const uint32_t C = static_cast<uint32_t>(fq->C);
         hipStream_t s = as_stream(stream);
         if (out_layout == HIPIE_NCHW) {
-            const bool vec = hw % 4 == 0 && (reinterpret_cast<uintptr_t>(x) % 16 == 0) &&
-                             (reinterpret_cast<uintptr_t>(y) % 4 == 0);
-            if (vec) {
-                const int64_t n4 = total / 4;
-                auto k = fq->rcp ? fq_nchw_q8_vec4<true> : fq_nchw_q8_vec4<false>;
-                hipLaunchKernelGGL(k, dim3(grid_for(n4)), dim3(kThreads), 0, s,
-                                   reinterpret_cast<const float4*>(x),
-                                   static_cast<uint32_t*>(y), tab, fq->lm1, off, n4,
-                                   static_cast<uint32_t>(hw / 4), C);
+            if (hw >= 3 && total < (1ll << 32) - 4 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 4 == 0) {
+                launch_flat<true>(fq->rcp, x, y, tab, fq->lm1, off, total, hw, C, s);
             } else {
                 auto k = fq->rcp ? fq_nchw_q8_scalar<true> : fq_nchw_q8_scalar<false>;
                 hipLaunchKernelGGL(k, dim3(grid_for(total)), dim3(kThreads), 0, s, x,
@@ -851,7 +891,7 @@ int hipie_fq_run_q8(const hipie_fq* fq, const float* x, void* y, int64_t n, int6
                           (long long)c_stride, (long long)fq->C);
             HIPIE_REQUIRE(reinterpret_cast<uintptr_t>(y) % 16 == 0 || c_stride % 16 != 0,
                           HIPIE_PARAMETER_MISMATCH, "hipie_fq_run_q8: output must be 16 B aligned");
-            if (hw % 4 == 0 && hw < (1 << 24) && reinterpret_cast<uintptr_t>(x) % 16 == 0 && c_stride >= 128) {
+            if (wide_tiles(n, hw, c_stride) && reinterpret_cast<uintptr_t>(x) % 4 == 0 && c_stride >= 128) {
                 const uint32_t tiles = static_cast<uint32_t>(ceil_div(hw, 32));
                 const int64_t gx = n * tiles;
                 HIPIE_REQUIRE(gx < (1ll << 31), HIPIE_OUT_OF_BOUNDS, "hipie_fq_run_q8: grid too large");
@@ -864,7 +904,7 @@ int hipie_fq_run_q8(const hipie_fq* fq, const float* x, void* y, int64_t n, int6
                 HIPIE_CHECK_HIP(hipGetLastError());
                 return;
             }
-            if (hw % 4 == 0 && hw < (1 << 24) && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
+            if (wide_tiles(n, hw, c_stride) && reinterpret_cast<uintptr_t>(x) % 4 == 0) {
                 const uint32_t tiles = static_cast<uint32_t>(ceil_div(hw, 256));
                 const int64_t gx = n * tiles;
                 HIPIE_REQUIRE(gx < (1ll << 31), HIPIE_OUT_OF_BOUNDS, "hipie_fq_run_q8: grid too large");

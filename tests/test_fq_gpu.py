@@ -150,3 +150,30 @@ def test_two_operation_division_reports_unmatched_divisor():
     check(lib().hipie_fq_div2_constants(0, d.ctypes.data_as(fp), ctypes.c_int64(1), zh.ctypes.data_as(fp),
                                         zl.ctypes.data_as(fp), ctypes.byref(ok)))
     assert ok.value == 0
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("shape", [(3, 2, 1, 1), (5, 3, 1, 2), (3, 7, 1, 3), (2, 1, 3, 3), (5, 7, 1, 5), (3, 130, 7, 9), (9, 33, 15, 17), (8, 40, 131, 127), (2, 66, 128, 2)])
+def test_fq_planes_that_end_inside_a_group_of_four(orc, shape, shift):
+    # every element position of a plane's end, tensors that are no whole groups, buffers one element off their boundary, and
+    # the transposition's tiles with a remainder in pixels and channels: the same bits as the operator
+    import torch
+    from dldt_amd import FakeQuantize
+    rng = np.random.default_rng(shape[1] * 1000 + shift)
+    x = rng.uniform(-4, 4, shape).astype(np.float32)
+    x.reshape(-1)[:2] = np.inf, -np.inf
+    C = shape[1]
+    mean = rng.uniform(-0.5, 0.5, C).astype(np.float32)
+    il, ih = mean - 3, mean + 3
+    want = orc.fake_quantize(x, il.reshape(1, C, 1, 1), ih.reshape(1, C, 1, 1), np.float32(0), np.float32(255), 256)
+    fq = FakeQuantize(C, 256, il, ih, 0.0, 255.0)
+    xd = torch.empty(x.size + shift, device="cuda")[shift:].view(shape)
+    xd.copy_(torch.from_numpy(x))
+    np.testing.assert_array_equal(fq.run_f32(xd).cpu().numpy().view(np.uint32), want.view(np.uint32))
+    out = torch.full((x.size + 8,), 77, dtype=torch.uint8, device="cuda")
+    np.testing.assert_array_equal(fq.run_q8(xd, "u8", "nchw", out=out[:x.size].view(shape)).cpu().numpy(), want.astype(np.uint8))
+    assert (out[x.size:] == 77).all()
+    cs = -(-C // 16) * 16
+    lv = (fq.run_q8(xd, "u8b", "nhwc", cs).cpu().numpy().astype(np.int16) + 128).astype(np.uint8)
+    np.testing.assert_array_equal(lv[..., :C], want.astype(np.uint8).transpose(0, 2, 3, 1))
+    assert np.all(lv[..., C:] == 0)
