@@ -97,7 +97,7 @@ bool conv_takes_planes(const hipie_conv* c, int64_t n, int64_t oh, int64_t ow);
 int conv_run_planes(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor& out, void* planes, hipStream_t s);
 void planes_arguments(ConvArgs& a, void* planes);
 
-// a 1 x 1 convolution and the depthwise 3 x 3 layer that alone reads it in one launch (expand_dw.hip); form 0: 32 channels a
+// a convolution of a short K and the depthwise 3 x 3 layer that alone reads it in one launch (expand_dw.hip); form 0: 32 channels a
 // workgroup, 1: the same in bands of half the height, 2: 48 channels, 3: 32 channels of several small images.
 // expand_dw_geometry: ok = false where the kernel does not take the layers
 constexpr int kExpandForms = 4;

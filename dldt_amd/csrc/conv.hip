@@ -2523,9 +2523,7 @@ bool hipie::conv_launch_arguments(const hipie_conv* c, const hipie_tensor& in, c
 bool hipie::conv_expand_fits(const hipie_conv* first, const hipie_conv* second, const hipie_tensor& mid, const hipie_tensor& out, int form) {
     const hipie_conv_desc &a = first->d, &b = second->d;
     if (first->depthwise || first->fused || first->koff_tile || !second->depthwise || first->device != second->device) return false;
-    if (a.kh != 1 || a.kw != 1 || a.groups != 1 || a.stride_h != 1 || a.stride_w != 1 || a.pad_top || a.pad_left || a.pad_bottom || a.pad_right || a.in_c_stride % 16 != 0 ||
-        first->Kp > 3 * 64)
-        return false;
+    if (a.groups != 1 || first->Kp > 3 * 64) return false;
     if (b.kh != 3 || b.kw != 3 || b.dil_h != 1 || b.dil_w != 1 || b.stride_h != b.stride_w || b.stride_h > 2 || b.ic != a.oc || b.oc != a.oc || b.in_dtype != first->epi.out_dtype)
         return false;
     if (!expand_dw_epilogues_fit(first->epi.flags, second->epi.flags)) return false;

@@ -1,5 +1,5 @@
-// A 1 x 1 convolution and the depthwise 3 x 3 convolution that alone reads it (the first two layers of an inverted residual
-// block) in one launch: the expanded tensor lives in LDS only.
+// A convolution of at most 192 K bytes a pixel (1 x 1, or the few channels of an image) and the depthwise 3 x 3 convolution that
+// alone reads it, the first two layers of an inverted residual block, in one launch: the expanded tensor lives in LDS only.
 //
 // Reference semantics: reference::convolution / group_convolution on widened inputs
 // (ngraph/core/reference/.../convolution.hpp:63-146) and the elementwise chain behind each, as the layers' own kernels evaluate
@@ -28,6 +28,7 @@ namespace hipie {
 namespace {
 
 typedef int32_t v4i __attribute__((ext_vector_type(4)));
+typedef int32_t unaligned_v4i __attribute__((ext_vector_type(4), aligned(4)));      // (an image's pixels are 4 bytes)
 typedef __attribute__((address_space(3))) int8_t* lds_bytes;
 typedef __attribute__((address_space(3))) uint32_t* lds_dwords;
 typedef __attribute__((address_space(3))) v4i* lds_quads;
@@ -118,7 +119,7 @@ __global__ __launch_bounds__(256) void expand_dw_kernel(const ExpandArgs e) {
         fast_divmod(j, e.W, e.inv_W, row, col);
         const int8_t* const p = image + (m * e.in_sn + row * e.in_sh + col * e.in_sw);
 #pragma unroll
-        for (int k = 0; k < NK; ++k) to[k] = *reinterpret_cast<const v4i*>(p + ko[k]);
+        for (int k = 0; k < NK; ++k) to[k] = *reinterpret_cast<const unaligned_v4i*>(p + ko[k]);
         at = patch + m * e.image_bytes + ((y0 - iy0 + row) * e.PW + col + e.pad_l) * PS + 4 * quad;
     };
     v4i p0[NK], p1[NK];
@@ -313,7 +314,7 @@ void launch_expand_dw(const ConvLaunch& first, const ConvLaunch& second, int ima
     const ConvArgs &a = first.a, &b = second.a;
     const int OH = b.OHOW / b.OW, S = b.conv_sh, channels = std::min(a.out_sw, b.out_sw);
     const ExpandGeometry g = expand_dw_geometry(channels, images, h, w, OH, b.OW, S, second.pad_top, second.pad_left, form);
-    HIPIE_REQUIRE(g.ok && a.nk >= 1 && a.nk <= 3 && a.conv_sh == 1 && a.conv_sw == 1 && b.wgt2 && S == b.conv_sw && (S == 1 || S == 2), HIPIE_GENERAL_ERROR,
+    HIPIE_REQUIRE(g.ok && a.nk >= 1 && a.nk <= 3 && b.wgt2 && S == b.conv_sw && (S == 1 || S == 2), HIPIE_GENERAL_ERROR,
                   "expansion and depthwise layer in one launch: %d x %d, %d K steps", h, w, a.nk);
     ExpandArgs e{};
     e.l1 = expand_layer(a);
@@ -323,7 +324,7 @@ void launch_expand_dw(const ConvLaunch& first, const ConvLaunch& second, int ima
     e.wgt2 = b.wgt2;
     e.koff = a.koff;
     e.out = static_cast<int8_t*>(b.out);
-    e.in_sn = a.in_sn; e.in_sh = a.in_sh; e.in_sw = a.in_sw; e.Kp = a.Kp;
+    e.in_sn = a.in_sn; e.in_sh = a.in_sh * a.conv_sh; e.in_sw = a.in_sw * a.conv_sw; e.Kp = a.Kp;
     e.out_sn = b.out_sn; e.out_sh = b.out_sh; e.out_sw = b.out_sw;
     e.W = w; e.H = h; e.OW = b.OW; e.OH = OH; e.pad_t = second.pad_top; e.pad_l = second.pad_left;
     e.R = g.rows; e.PW = g.patch_w; e.slabs = g.slabs; e.bands = g.bands; e.units = static_cast<int32_t>(g.slabs * g.bands * ceil_div(images, g.images));

@@ -426,7 +426,7 @@ struct ConvStep : Step {
 
 // A 3 x 3 convolution and the 1 x 1 convolution that is its only reader (the tail of a bottleneck block), planned as
 // two layers and run either one after the other or - where hipie_conv_pair_fits takes them and it is faster - as one
-// kernel that keeps the tensor between them in LDS (hipie_conv_run_pair).  Same bits either way.  With `expands`: a 1 x 1
+// kernel that keeps the tensor between them in LDS (hipie_conv_run_pair).  Same bits either way.  With `expands`: a
 // convolution and the depthwise layer that is its only reader (conv_run_expand).
 struct PairStep : Step {
     bool expands = false;
@@ -3383,7 +3383,7 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
             plan->steps.erase(plan->steps.begin() + static_cast<std::ptrdiff_t>(i));
             --i;
         }
-    // A 1 x 1 convolution whose result only the next depthwise layer reads: one step, and one launch where that is faster
+    // A convolution whose result only the next depthwise layer reads: one step, and one launch where that is faster
     // (values that are kept stay two steps, and so do layers that nothing measures: choices of a plan that had them apart,
     // plans without a device, plans that are not tuned)
     const bool measured_pairs = device >= 0 && (preset ? preset->size() != plan->steps.size() : cfg.tune);

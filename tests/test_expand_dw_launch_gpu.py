@@ -1,4 +1,4 @@
-"""A 1 x 1 convolution and the depthwise 3 x 3 layer that alone reads it in one launch (csrc/expand_dw.hip), in every form it
+"""A convolution and the depthwise 3 x 3 layer that alone reads it in one launch (csrc/expand_dw.hip), in every form it
 has, against the two layers' own kernels bit for bit: bands and columns with remainders, strides, padding, one K step and three,
 channels that fill a workgroup's and that do not, fewer units than compute units and more, the three epilogues."""
 import numpy as np
@@ -10,7 +10,7 @@ from dldt_amd.builders import QuantizedNet
 
 pytestmark = pytest.mark.gpu
 
-#        n, c, h, w, channels, stride and padding of the depthwise layer, top of the range (above 6: the Clamp stays), ReLU6 or not
+#        n, c, h, w, channels (images of 3: a 3 x 3 convolution of stride 2), stride and padding of the depthwise layer, top of the range (above 6: the Clamp stays), ReLU6 or not
 CASES = {
     "columns_17": (1, 16, 13, 17, 48, 1, 1, 3.0, True),
     "stride_2_odd": (3, 24, 15, 9, 80, 2, 1, 3.0, True),
@@ -23,6 +23,8 @@ CASES = {
     "many_units": (9, 24, 40, 24, 144, 1, 1, 3.0, True),
     "small_images": (65, 16, 7, 7, 368, 1, 1, 3.0, True),
     "small_images_stride_2": (70, 24, 7, 9, 368, 2, 1, 3.0, True),
+    "image": (2, 3, 33, 31, 32, 1, 1, 3.0, True),
+    "image_stride_2": (3, 3, 57, 40, 40, 2, 1, 8.0, True),
     "no_scale": (3, 48, 21, 19, 70, 1, 1, 3.0, False),
     "no_scale_stride_2": (3, 48, 21, 19, 70, 2, 1, 3.0, False),
 }
@@ -33,7 +35,8 @@ def _graph(n, c, h, w, oc, stride, pads, high, relu6):
     net = QuantizedNet()
     a = net.input("data", (n, c, h, w), 2.0)
     conv = net.conv_relu6 if relu6 else net.conv
-    mid = conv(a, rng.normal(0, 1 / np.sqrt(c), (oc, c, 1, 1)).astype(np.float32), rng.normal(0, 0.2, oc).astype(np.float32), high)
+    k = 3 if c == 3 else 1
+    mid = conv(a, rng.normal(0, 1 / np.sqrt(c), (oc, c, k, k)).astype(np.float32), rng.normal(0, 0.2, oc).astype(np.float32), high, strides=(1 + k // 2,) * 2, pads=(k // 2,) * 2)
     b = conv(mid, rng.normal(0, 0.4, (oc, 1, 3, 3)).astype(np.float32), rng.normal(0, 0.2, oc).astype(np.float32), high, strides=(stride, stride), pads=(pads, pads), grouped=True)
     net.g.result(net.conv_f32(b, rng.normal(0, 0.2, (24, oc, 1, 1)).astype(np.float32), None), "out")
     return net.g, mid["node"]
