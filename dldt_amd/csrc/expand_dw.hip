@@ -13,11 +13,13 @@
 //                are requested two fragments ahead.  A patch pixel is 16 T + 4 bytes: both halves' dword accesses then meet
 //                the minimum of two lanes a bank.
 //   second half: the window in registers, v_dot4 on transposed dwords as dwconv3x3_lds_kernel.
-// What bounds it: the vector pipe (the exact chain, 8 + 15 instructions a value) on large maps, the launch on small ones.
+// What bounds it: the vector pipe on large maps (the exact chain and a lane's way to its next pixel, 10 + 15 instructions a value:
+// 16 -> 96 channels at 112 x 112, stride 2, batch 64 took 42 us alone with 39 of vector issue when the way was two divisions and
+// the sums came through accumulation registers, 34.2 -> 30.0 us a launch in flight without), the launch on small ones.
 // Small images share a workgroup: a 7 x 7 image alone gives the second half 64 of 256 lanes something to do.
 // Measured per launch with three requests in flight, the two layers' own kernels / this one: 16 -> 96 channels at 112 x 112,
-// stride 2, batch 64: 55.4 / 34.2 us; 24 -> 144 at 56 x 56 28.9 / 20.2; 64 -> 384 at 14 x 14 7.0 / 6.2; 160 -> 960 at 7 x 7
-// 7.3 / 9.7 with one image a workgroup, 4.6 with several.  At batch 8 all of them 5.5 - 8 / 2.8 - 5.3.
+// stride 2, batch 64: 55.8 / 30.0 us; 24 -> 144 at 56 x 56 29.1 / 19.5; 64 -> 384 at 14 x 14 7.1 / 6.4; 160 -> 960 at 7 x 7
+// 7.2 / 9.7 with one image a workgroup, 4.5 with several.  At batch 8 all of them 5.5 - 8 / 2.7 - 4.7.
 #include "conv_dispatch.h"
 #include "conv.h"
 
@@ -53,6 +55,9 @@ struct ExpandArgs {
     int32_t images, N;                     // images a workgroup takes one behind the other (1 where an image has several bands)
     int32_t image_pixels, image_bytes, image_items;   // where it takes several: of one image's patch
     float inv_image_pixels, inv_image_items;
+    // 64 pixels on: columns, and what that adds to the offsets in the input and in the patch; into the next row and the next image
+    int32_t step_col, step_row, image_rows, nowhere;
+    uint32_t step_in, step_lds, row_in, row_lds, image_in, image_lds;
     int32_t quads, channel_groups;         // groups of four output pixels in a row, of four channels that the output holds
     int32_t patch_pieces;                  // 16-byte pieces of the patch
     uint32_t fill;
@@ -95,14 +100,14 @@ __device__ __forceinline__ uint32_t level_into(const ExpandLayer& l, const Expan
 constexpr int kRows = 2;       // output rows a lane of the depthwise half computes at a time
 
 template <uint32_t F, int S, int NK, int T>
-__global__ __launch_bounds__(256) void expand_dw_kernel(const ExpandArgs e) {
+__global__ __launch_bounds__(256, T == 2 ? 4 : 3) void expand_dw_kernel(const ExpandArgs e) {
     extern __shared__ __attribute__((aligned(16))) int8_t patch_memory[];
     const lds_bytes patch = (lds_bytes)patch_memory;
     constexpr int PS = 16 * T + 4, G = 4 * T, SLOTS = 256 / G;
     const int unit = e.per_xcd > 0 ? static_cast<int>(blockIdx.x & 7) * e.per_xcd + static_cast<int>(blockIdx.x >> 3) : static_cast<int>(blockIdx.x);
     if (unit >= e.units) return;                      // whole workgroup, before the barriers
     const int slab = unit % e.slabs, nb = unit / e.slabs, band = nb % e.bands, n = nb / e.bands * e.images, images = min(e.images, e.N - n);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lane16 = lane & 15, quad = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane16 = lane & 15, quad = lane >> 4;
     const int oy0 = band * e.R, rows = min(e.R, e.OH - oy0), iy0 = oy0 * S - e.pad_t;
     const int y0 = max(iy0, 0), y1 = min(iy0 + (rows - 1) * S + 3, e.H), count = (y1 - y0) * e.W * images, frags = (count + 15) >> 4;
     const int c0 = slab * (16 * T);
@@ -113,19 +118,42 @@ __global__ __launch_bounds__(256) void expand_dw_kernel(const ExpandArgs e) {
 #pragma unroll
     for (int k = 0; k < NK; ++k) ko[k] = e.koff[4 * k + quad];
     const int8_t* const image = e.in + static_cast<int64_t>(n) * e.in_sn + static_cast<int64_t>(y0) * e.in_sh;
-    auto request = [&](int f, v4i (&to)[NK], lds_bytes& at) {       // (fragments behind the last one repeat its last pixel)
-        int row, col, m = 0, j = min(16 * f + lane16, count - 1);
-        if (images > 1) fast_divmod(j, e.image_pixels, e.inv_image_pixels, m, j);
+    // the lane's pixel of the next fragment to request, 64 pixels behind the one before: in mixed radix (image, row, column), as
+    // two divisions and their products a fragment cost as much as half of the chain on its values
+    int j = 16 * wave + lane16, col, row = 0, m = 0;
+    if (images > 1) {
+        fast_divmod(j, e.image_pixels, e.inv_image_pixels, m, row);
+        fast_divmod(row, e.W, e.inv_W, row, col);
+    } else {
         fast_divmod(j, e.W, e.inv_W, row, col);
-        const int8_t* const p = image + (m * e.in_sn + row * e.in_sh + col * e.in_sw);
+    }
+    uint32_t from = static_cast<uint32_t>(m * e.in_sn + row * e.in_sh + col * e.in_sw);
+    uint32_t to_lds = static_cast<uint32_t>(m * e.image_bytes + ((y0 - iy0 + row) * e.PW + col + e.pad_l) * PS + 4 * quad);
+    auto request = [&](v4i (&to)[NK], lds_bytes& at) {       // (pixels behind the last one: the first one's bytes, to where nobody reads)
+        const bool on = j < count;
+        const uint32_t off = on ? from : 0u;
 #pragma unroll
-        for (int k = 0; k < NK; ++k) to[k] = *reinterpret_cast<const unaligned_v4i*>(p + ko[k]);
-        at = patch + m * e.image_bytes + ((y0 - iy0 + row) * e.PW + col + e.pad_l) * PS + 4 * quad;
+        for (int k = 0; k < NK; ++k) to[k] = *reinterpret_cast<const unaligned_v4i*>(image + (off + static_cast<uint32_t>(ko[k])));
+        at = patch + (on ? to_lds : static_cast<uint32_t>(e.nowhere));
+        j += 64;
+        col += e.step_col;
+        from += e.step_in;
+        to_lds += e.step_lds;
+        const bool next_row = col >= e.W;
+        col -= next_row ? e.W : 0;
+        from += next_row ? e.row_in : 0u;
+        to_lds += next_row ? e.row_lds : 0u;
+        if (images > 1) {
+            row += e.step_row + (next_row ? 1 : 0);
+            const bool next_image = row >= e.image_rows;
+            row -= next_image ? e.image_rows : 0;
+            from += next_image ? e.image_in : 0u;
+            to_lds += next_image ? e.image_lds : 0u;
+        }
     };
     v4i p0[NK], p1[NK];
     lds_bytes at0, at1;
-    int f = wave;
-    request(f, p0, at0);
+    request(p0, at0);
 #pragma unroll
     for (int t = 0; t < T; ++t) {
         // row of the packed weights that holds the channel (conv_kernel.h)
@@ -137,7 +165,7 @@ __global__ __launch_bounds__(256) void expand_dw_kernel(const ExpandArgs e) {
     ExpandConstants<F, 4 * T> k1;
 #pragma unroll
     for (int t = 0; t < T; ++t) load_constants(e.l1, c0 + 16 * t + 4 * quad, 4 * t, k1);
-    request(f + 4, p1, at1);
+    request(p1, at1);
     for (int i = tid; i < e.patch_pieces; i += 256) {
         const int b = static_cast<int>(e.fill);
         ((lds_quads)patch)[i] = v4i{b, b, b, b};
@@ -155,11 +183,11 @@ __global__ __launch_bounds__(256) void expand_dw_kernel(const ExpandArgs e) {
             *(lds_dwords)(at + 16 * t) = packed ^ e.l1.xmask;
         }
     };
-    for (; f < frags; f += 8) {
+    for (int f = wave; f < frags; f += 8) {
         fragment(p0, at0);
-        request(f + 8, p0, at0);
+        request(p0, at0);
         if (f + 4 < frags) fragment(p1, at1);
-        request(f + 12, p1, at1);
+        request(p1, at1);
     }
 
     // ---- second half
@@ -304,7 +332,7 @@ ExpandGeometry expand_dw_geometry(int channels, int images, int h, int w, int oh
         while (g.images > 1 && g.slabs * ceil_div(images, g.images) < 256) --g.images;
         if (g.images < 2) return g;
     }
-    g.lds = static_cast<size_t>(round_up(patch * g.images, 16));
+    g.lds = static_cast<size_t>(round_up(patch * g.images, 16) + round_up(16 * g.tiles + 4, 16));      // (and a pixel nobody reads)
     const int64_t units = static_cast<int64_t>(g.slabs) * g.bands * ceil_div(images, g.images);
     g.ok = units < (1 << 24) && static_cast<int64_t>(h) * w < (1 << 24);
     return g;
@@ -330,9 +358,20 @@ void launch_expand_dw(const ConvLaunch& first, const ConvLaunch& second, int ima
     e.R = g.rows; e.PW = g.patch_w; e.slabs = g.slabs; e.bands = g.bands; e.units = static_cast<int32_t>(g.slabs * g.bands * ceil_div(images, g.images));
     e.images = g.images; e.N = images;
     // (an image in one band: its patch holds all of the rows that it reads)
-    e.image_pixels = std::min((OH - 1) * S + 3 - second.pad_top, h) * w;
+    e.image_rows = std::min((OH - 1) * S + 3 - second.pad_top, h);
+    e.image_pixels = e.image_rows * w;
     e.image_bytes = ((g.rows - 1) * S + 3) * g.patch_w * (16 * g.tiles + 4);
     e.image_items = (OH + kRows - 1) / kRows * g.quads;
+    const int PS = 16 * g.tiles + 4, per_image = g.images > 1 ? e.image_pixels : 1 << 30, step_images = 64 / per_image, rest = 64 % per_image;
+    e.step_row = rest / w;
+    e.step_col = rest % w;
+    e.step_in = static_cast<uint32_t>(step_images * e.in_sn + e.step_row * e.in_sh + e.step_col * e.in_sw);
+    e.step_lds = static_cast<uint32_t>(step_images * e.image_bytes + (e.step_row * g.patch_w + e.step_col) * PS);
+    e.row_in = static_cast<uint32_t>(e.in_sh - w * e.in_sw);
+    e.row_lds = static_cast<uint32_t>((g.patch_w - w) * PS);
+    e.image_in = static_cast<uint32_t>(e.in_sn - e.image_rows * e.in_sh);
+    e.image_lds = static_cast<uint32_t>(e.image_bytes - e.image_rows * g.patch_w * PS);
+    e.nowhere = static_cast<int32_t>(g.lds - round_up(PS, 16));
     e.inv_image_pixels = 1.0f / static_cast<float>(e.image_pixels);
     e.inv_image_items = 1.0f / static_cast<float>(e.image_items);
     e.quads = g.quads;
