@@ -253,13 +253,15 @@ void launch_requant_flat(const float* x, int8_t* q, int64_t n, const Requant& fq
     hipLaunchKernelGGL(requant_flat, dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0, s, x, q, n, fq);
 }
 
-void run_softmax(const float* x, float* y, int8_t* q, int64_t rows, int64_t axis, const hipie_requant* r, void* stream,
+}  // namespace
+}  // namespace hipie
+
+void hipie::run_softmax(const float* x, float* y, int8_t* q, int64_t rows, int64_t axis, const Requant* r, hipStream_t s,
                  const char* what) {
     if (rows == 0 || axis == 0) return;
     HIPIE_REQUIRE(x && (y || q) && rows > 0 && axis > 0 && axis < (1ll << 31), HIPIE_PARAMETER_MISMATCH, "%s: bad argument", what);
     HIPIE_REQUIRE(!q || r, HIPIE_PARAMETER_MISMATCH, "%s: quantized output without a requantisation", what);
-    const Requant fq = q ? make_requant(r, what) : Requant{};
-    hipStream_t s = as_stream(stream);
+    const Requant fq = q ? *r : Requant{};
     const bool aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0 &&
                          reinterpret_cast<uintptr_t>(q) % 4 == 0;
     if (!(aligned && dispatch_chunks<LaunchSoftmax>(static_cast<int>(axis), x, y, q, rows, static_cast<int>(axis), fq, s))) {
@@ -271,14 +273,13 @@ void run_softmax(const float* x, float* y, int8_t* q, int64_t rows, int64_t axis
     HIPIE_CHECK_HIP(hipGetLastError());
 }
 
-void run_mvn(const float* x, float* y, int8_t* q, int64_t rows, int64_t axis, int normalize_variance, float eps,
-             int eps_inside_sqrt, const float* gamma, const float* beta, const hipie_requant* r, void* stream,
+void hipie::run_mvn(const float* x, float* y, int8_t* q, int64_t rows, int64_t axis, int normalize_variance, float eps,
+             int eps_inside_sqrt, const float* gamma, const float* beta, const Requant* r, hipStream_t s,
              const char* what) {
     if (rows == 0 || axis == 0) return;
     HIPIE_REQUIRE(x && (y || q) && rows > 0 && axis > 0 && axis < (1ll << 31), HIPIE_PARAMETER_MISMATCH, "%s: bad argument", what);
     HIPIE_REQUIRE(!q || r, HIPIE_PARAMETER_MISMATCH, "%s: quantized output without a requantisation", what);
-    const Requant fq = q ? make_requant(r, what) : Requant{};
-    hipStream_t s = as_stream(stream);
+    const Requant fq = q ? *r : Requant{};
     const bool aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0 &&
                          reinterpret_cast<uintptr_t>(q) % 4 == 0 && reinterpret_cast<uintptr_t>(gamma) % 16 == 0 &&
                          reinterpret_cast<uintptr_t>(beta) % 16 == 0;
@@ -292,17 +293,20 @@ void run_mvn(const float* x, float* y, int8_t* q, int64_t rows, int64_t axis, in
     HIPIE_CHECK_HIP(hipGetLastError());
 }
 
-void run_gelu(const float* x, float* y, int8_t* q, int64_t n, const hipie_requant* r, void* stream, const char* what) {
+void hipie::run_gelu(const float* x, float* y, int8_t* q, int64_t n, const Requant* r, hipStream_t s, const char* what) {
     if (n == 0) return;
     HIPIE_REQUIRE(x && (y || q) && n > 0, HIPIE_PARAMETER_MISMATCH, "%s: bad argument", what);
     HIPIE_REQUIRE(!q || r, HIPIE_PARAMETER_MISMATCH, "%s: quantized output without a requantisation", what);
     HIPIE_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0 &&
                       reinterpret_cast<uintptr_t>(q) % 4 == 0, HIPIE_PARAMETER_MISMATCH, "%s: buffers must be 16-byte aligned", what);
-    const Requant fq = q ? make_requant(r, what) : Requant{};
+    const Requant fq = q ? *r : Requant{};
     const int64_t blocks = std::min<int64_t>(ceil_div(ceil_div(n, 4), kThreads), 256 * 32);
-    hipLaunchKernelGGL(gelu_erf, dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0, as_stream(stream), x, y, q, n, fq);
+    hipLaunchKernelGGL(gelu_erf, dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0, s, x, y, q, n, fq);
     HIPIE_CHECK_HIP(hipGetLastError());
 }
+
+namespace hipie {
+namespace {
 
 // Embedding lookup: one wavefront per token copies its table row (float4 per lane and step) and adds
 // up to two addends in the graph's order.
@@ -370,18 +374,18 @@ using namespace hipie;
 extern "C" {
 
 int hipie_softmax_f32(const float* x, float* y, int64_t rows, int64_t axis, void* stream) {
-    return guarded([&] { run_softmax(x, y, nullptr, rows, axis, nullptr, stream, "hipie_softmax_f32"); });
+    return guarded([&] { run_softmax(x, y, nullptr, rows, axis, nullptr, as_stream(stream), "hipie_softmax_f32"); });
 }
 
 int hipie_mvn_f32(const float* x, float* y, int64_t rows, int64_t axis, int normalize_variance, float eps,
                   int eps_inside_sqrt, const float* gamma, const float* beta, void* stream) {
     return guarded([&] {
-        run_mvn(x, y, nullptr, rows, axis, normalize_variance, eps, eps_inside_sqrt, gamma, beta, nullptr, stream, "hipie_mvn_f32");
+        run_mvn(x, y, nullptr, rows, axis, normalize_variance, eps, eps_inside_sqrt, gamma, beta, nullptr, as_stream(stream), "hipie_mvn_f32");
     });
 }
 
 int hipie_gelu_f32(const float* x, float* y, int64_t n, void* stream) {
-    return guarded([&] { run_gelu(x, y, nullptr, n, nullptr, stream, "hipie_gelu_f32"); });
+    return guarded([&] { run_gelu(x, y, nullptr, n, nullptr, as_stream(stream), "hipie_gelu_f32"); });
 }
 
 int hipie_add_broadcast_f32(const float* x, const int64_t* dims, const float* addend, const int64_t* addend_dims, int rank,
@@ -441,18 +445,25 @@ int hipie_copy_strided(const void* src, const int64_t* dims, const int64_t* stri
 
 int hipie_softmax_q8(const float* x, float* y, int8_t* q, int64_t rows, int64_t axis, const hipie_requant* requant,
                      void* stream) {
-    return guarded([&] { run_softmax(x, y, q, rows, axis, requant, stream, "hipie_softmax_q8"); });
+    return guarded([&] {
+        const Requant fq = rows && axis && q && requant ? make_requant(requant, "hipie_softmax_q8") : Requant{};
+        run_softmax(x, y, q, rows, axis, requant ? &fq : nullptr, as_stream(stream), "hipie_softmax_q8");
+    });
 }
 
 int hipie_mvn_q8(const float* x, float* y, int8_t* q, int64_t rows, int64_t axis, int normalize_variance, float eps,
                  int eps_inside_sqrt, const float* gamma, const float* beta, const hipie_requant* requant, void* stream) {
     return guarded([&] {
-        run_mvn(x, y, q, rows, axis, normalize_variance, eps, eps_inside_sqrt, gamma, beta, requant, stream, "hipie_mvn_q8");
+        const Requant fq = rows && axis && q && requant ? make_requant(requant, "hipie_mvn_q8") : Requant{};
+        run_mvn(x, y, q, rows, axis, normalize_variance, eps, eps_inside_sqrt, gamma, beta, requant ? &fq : nullptr, as_stream(stream), "hipie_mvn_q8");
     });
 }
 
 int hipie_gelu_q8(const float* x, float* y, int8_t* q, int64_t n, const hipie_requant* requant, void* stream) {
-    return guarded([&] { run_gelu(x, y, q, n, requant, stream, "hipie_gelu_q8"); });
+    return guarded([&] {
+        const Requant fq = n && q && requant ? make_requant(requant, "hipie_gelu_q8") : Requant{};
+        run_gelu(x, y, q, n, requant ? &fq : nullptr, as_stream(stream), "hipie_gelu_q8");
+    });
 }
 
 int hipie_embedding_f32(const float* table, int64_t vocabulary, int64_t hidden, const int32_t* ids, int64_t tokens,

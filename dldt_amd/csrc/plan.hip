@@ -951,7 +951,16 @@ struct GlueStep : Step {
     float eps = 0;
     std::vector<float> gamma, beta;
     DeviceBuffer d_gamma, d_beta;
+    Requant fq{};                  // of rq, where there is one (a range that has none is refused by every run)
+    bool fq_known = false;
     void create(int device, const std::vector<TensorInfo>&) override {
+        if (outq >= 0) {
+            try {
+                fq = make_requant(&rq, name.c_str());
+                fq_known = true;
+            } catch (const std::exception&) {
+            }
+        }
         if (device < 0) return;
         if (!gamma.empty()) d_gamma.upload(device, gamma.data(), gamma.size() * 4);
         if (!beta.empty()) d_beta.upload(device, beta.data(), beta.size() * 4);
@@ -961,15 +970,11 @@ struct GlueStep : Step {
         const float* x = reinterpret_cast<const float*>(in.ptr(arena, tensors, inputs));
         float* y = out >= 0 ? reinterpret_cast<float*>(arena + tensors[out].offset) : nullptr;
         int8_t* q = outq >= 0 ? reinterpret_cast<int8_t*>(arena + tensors[outq].offset) : nullptr;
-        const hipie_requant* r = outq >= 0 ? &rq : nullptr;
-        const float* gm = gamma.empty() ? nullptr : d_gamma.as<float>();
-        const float* bt = beta.empty() ? nullptr : d_beta.as<float>();
-        int st = HIPIE_OK;
-        if (kind == OP_SOFTMAX) st = q ? hipie_softmax_q8(x, y, q, rows, axis, r, s) : hipie_softmax_f32(x, y, rows, axis, s);
-        else if (kind == OP_GELU) st = q ? hipie_gelu_q8(x, y, q, rows * axis, r, s) : hipie_gelu_f32(x, y, rows * axis, s);
-        else st = q ? hipie_mvn_q8(x, y, q, rows, axis, normalize_variance, eps, eps_inside_sqrt, gm, bt, r, s)
-                    : hipie_mvn_f32(x, y, rows, axis, normalize_variance, eps, eps_inside_sqrt, gm, bt, s);
-        check_status(st, name.c_str());
+        const Requant refused = outq >= 0 && !fq_known ? make_requant(&rq, name.c_str()) : Requant{};
+        const Requant* r = outq < 0 ? nullptr : fq_known ? &fq : &refused;
+        if (kind == OP_SOFTMAX) run_softmax(x, y, q, rows, axis, r, s, name.c_str());
+        else if (kind == OP_GELU) run_gelu(x, y, q, rows * axis, r, s, name.c_str());
+        else run_mvn(x, y, q, rows, axis, normalize_variance, eps, eps_inside_sqrt, gamma.empty() ? nullptr : d_gamma.as<float>(), beta.empty() ? nullptr : d_beta.as<float>(), r, s, name.c_str());
     }
     bool program(ProgBuilder& b, const std::vector<TensorInfo>& tensors, void* const* inputs, void* const*) const override {
         if (kind == OP_SOFTMAX || kind == OP_GELU) return false;
