@@ -92,12 +92,13 @@ __global__ __launch_bounds__(kThreads) void mvn_rows_reg(const float* __restrict
         const float var = wave_sum(sq) / static_cast<float>(axis);
         denom = eps_inside ? sqrtf(var + eps) : sqrtf(var) + eps;
     }
+    const RowDivisor by(denom);
 #pragma unroll
     for (int j = 0; j < NCH; ++j) {
         const int i = 256 * j + 4 * lane;
         if (i >= axis) continue;
         float4 o = v[j];
-        if (normalize_variance) { o.x = o.x / denom; o.y = o.y / denom; o.z = o.z / denom; o.w = o.w / denom; }
+        if (normalize_variance) o = by(o);
         if (gamma) {
             const float4 gm = *reinterpret_cast<const float4*>(gamma + i);
             o.x = o.x * gm.x; o.y = o.y * gm.y; o.z = o.z * gm.z; o.w = o.w * gm.w;

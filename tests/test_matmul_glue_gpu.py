@@ -447,3 +447,16 @@ def test_gelu_of_the_extremes():
     assert y[0] == np.inf and np.isnan(y[1]) and np.isnan(y[2]) and y[3] == 0 and y[4] == 0
     assert y[5] == np.float32(3e38) and y[6] == 0 and y[9] == np.float32(2.0 ** 61) and y[10] == 0 and y[11] == 12
     assert np.all(np.abs(y[7:9]) <= 1e-40)
+
+
+@pytest.mark.parametrize("eps", [1234.567, 7.7e9, 1.3 * 2.0 ** 59, 1.1 * 2.0 ** 61])
+@pytest.mark.parametrize("axis", [4, 260, 768])
+def test_a_row_of_mvn_is_divided_as_by_the_ieee_division(axis, eps):
+    # pairs t, -t: the mean is 0; the deviation vanishes in eps, so that the divisor is eps itself (the last one takes the division)
+    import torch
+    from dldt_amd import mvn
+    t = np.random.default_rng(axis).uniform(1e-6, 1e-5, (257, axis // 2)).astype(np.float32)
+    x = np.stack([t, -t], axis=-1).reshape(257, axis)
+    want = x / np.float32(eps)
+    got = mvn(torch.from_numpy(x).cuda(), True, eps, False).cpu().numpy()
+    np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
