@@ -474,7 +474,8 @@ struct PairStep : Step {
         fused = one_kernel;
         // the depth is a setting of the first layer's object: the pair's when they run as one kernel, else its own
         if (first->conv) check_status(hipie_conv_set_stages(first->conv, fused && !expands ? stages_of(form) : (first->deep ? 8 : 0)), name.c_str());
-        type = std::string(fused ? "Convolution+" : "Convolution,") + (expands ? "GroupConvolution" : "Convolution");
+        // (an expansion goes under the name and type of the depthwise layer it feeds: one step, of one kernel or two)
+        type = expands ? "GroupConvolution" : fused ? "Convolution+Convolution" : "Convolution,Convolution";
         bytes = first->bytes + second->bytes - (fused ? 2 * mid_bytes : 0);
     }
     int launches() const override { return fused ? 1 : first->launches() + second->launches(); }
