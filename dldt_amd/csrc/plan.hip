@@ -518,7 +518,9 @@ struct PairStep : Step {
         };
         float best_fused = 0.f;
         int best_form = -1;
-        for (int d = 0; d < 4; ++d) {
+        // (several small images a workgroup first: where launches arrive more slowly than they run all forms take the same time, and
+        // the first one stays)
+        for (int d : {3, 0, 1, 2}) {
         if (!(forms >> d & 1)) continue;
         form = d;
         if (!expands) check_status(hipie_conv_set_stages(first->conv, stages_of(d)), name.c_str());
