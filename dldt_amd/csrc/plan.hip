@@ -1270,7 +1270,7 @@ struct Planner {
     std::vector<std::unique_ptr<Step>> steps;
     std::vector<char> visiting;
     // HIPIE_KEEP_F32=1: store the f32 result of Softmax / MVN / Gelu even when only a fused
-    // FakeQuantize reads it (inspection of the values behind the tolerance-only operations)
+    // FakeQuantize reads it (inspection of the values behind the tolerance-only operations), and an f32 result in its tensor
     bool keep_f32 = false;
     // HIPIE_FUSE_ATTENTION=0: plan the attention core as separate MatMul / Softmax kernels
     bool fuse_attention = true;
@@ -4266,8 +4266,8 @@ int hipie_request_tensor(const hipie_request* r, int node_id, hipie_tensor* t) {
                               "hipie_request_tensor: node %d lives in LDS only (two convolutions run as one kernel)", node_id);
         for (const auto& st : r->plan->steps)
             if (auto* conv = dynamic_cast<const ConvStep*>(st.get()))
-                HIPIE_REQUIRE(!(conv->direct && conv->out == it->second), HIPIE_NOT_FOUND, "hipie_request_tensor: node %d is a result, stored in the caller's buffer only",
-                              node_id);
+                HIPIE_REQUIRE(!((r->ran ? conv->writes_result : conv->direct) && conv->out == it->second), HIPIE_NOT_FOUND,
+                              "hipie_request_tensor: node %d is a result, stored in the caller's buffer only", node_id);
         if (r->ran)
             for (int tensor : r->ran->inside)
                 HIPIE_REQUIRE(tensor != it->second, HIPIE_NOT_FOUND, "hipie_request_tensor: node %d lives in LDS only (two layers are one step of the single launch)", node_id);

@@ -478,8 +478,8 @@ int hipie_compile(const hipie_graph* graph, int device, hipie_plan** plan);
  * flight together; the kernel variants are timed that way and OPTIMAL_NUMBER_OF_INFER_REQUESTS reports it),
  * HIP_TUNE (YES | NO: time the kernel variants at load, else shape-based defaults), HIP_TUNE_FILE (cache of the
  * choices, like the reference GPU plugin's KEY_TUNING_FILE), HIP_FUSE_ATTENTION, HIP_MERGE_LINEAR, HIP_KEEP_F32
- * (YES | NO), HIP_FUSE_CONVOLUTIONS (a 3 x 3 convolution and the 1 x 1 convolution that alone reads its result as one
- * kernel, hipie_conv_run_pair: AUTO = where the load-time measurement finds it faster, YES = wherever the kernel takes
+ * (YES | NO; HIP_KEEP_F32 keeps values that hipie_request_tensor does not find otherwise), HIP_FUSE_CONVOLUTIONS (a 3 x 3
+ * convolution and the 1 x 1 convolution that alone reads its result as one kernel, hipie_conv_run_pair: AUTO = where the load-time measurement finds it faster, YES = wherever the kernel takes
  * the pair, NO; the same for a convolution and the depthwise 3 x 3 layer that alone reads its result, in plans that are
  * tuned and without HIP_KEEP_F32; the tensor between two layers run that way exists in LDS only and hipie_request_tensor gives
  * HIPIE_NOT_FOUND for it), HIP_SINGLE_LAUNCH (a request that is started and waited for runs as one persistent kernel:
@@ -593,7 +593,10 @@ int hipie_request_enqueue(hipie_request* request, const void* const* inputs, voi
 int hipie_request_stream(hipie_request* request, void** stream);
 /* milliseconds of step `index` in the last inference (GetPerformanceCounts); a request with counters runs by steps */
 int hipie_request_perf(hipie_request* request, int index, float* ms);
-/* the arena tensor holding the value of graph node `node_id` (inspection, parity tests) */
+/* the arena tensor holding the value of graph node `node_id` (inspection, parity tests).  HIPIE_NOT_FOUND where the last
+ * inference left it in no tensor: a node fused into its reader, a value between two layers that ran as one kernel or as one step
+ * of a single launch, and an f32 result that nothing else reads and its convolution stored in the caller's buffer (of a feature
+ * map always, of [N, C] values in a single launch).  With HIP_KEEP_F32 results and values in front of a depthwise layer are there */
 int hipie_request_tensor(const hipie_request* request, int node_id, hipie_tensor* tensor);
 
 /* ======================================================================================
