@@ -3127,7 +3127,7 @@ bool run_again(hipie_request* r) {
 }
 
 // the single-launch form of a plan whose every step has one, or null and what it has no room for
-std::shared_ptr<ProgramForm> build_program(const hipie_plan& p, int workgroups, bool keep_values, std::string& refused) {
+std::shared_ptr<ProgramForm> build_program(const hipie_plan& p, int workgroups, std::string& refused) {
     if (p.inputs.size() + p.outputs.size() > static_cast<size_t>(kProgramIo)) {
         refused = "inputs and outputs";
         return nullptr;
@@ -3139,7 +3139,9 @@ std::shared_ptr<ProgramForm> build_program(const hipie_plan& p, int workgroups, 
     for (size_t i = 0; i < p.inputs.size(); ++i) in.push_back(b.fake_io(static_cast<int>(i)));
     for (size_t i = 0; i < p.outputs.size(); ++i) out.push_back(b.fake_io(static_cast<int>(p.inputs.size() + i)));
     DeviceGuard g(p.device);
-    // a step's readers: a layer whose only one is a depthwise layer can be one step with it
+    // a step's readers: a layer whose only one is a depthwise layer can be one step with it, unless the value between them is
+    // asked for (HIP_KEEP_F32) or no two convolutions are to be one (HIP_FUSE_CONVOLUTIONS)
+    const bool join = !p.config.keep_f32 && p.config.fuse_convs != 0;
     std::vector<int> readers(p.steps.size(), 0), reader(p.steps.size(), -1);
     for (size_t i = 0; i < p.steps.size(); ++i)
         for (int from : p.steps[i]->sources)
@@ -3150,7 +3152,7 @@ std::shared_ptr<ProgramForm> build_program(const hipie_plan& p, int workgroups, 
     std::vector<int> inside;
     for (size_t i = 0; i < p.steps.size(); ++i) {
         const Step* s = p.steps[i].get();
-        if (!keep_values && i + 1 < p.steps.size() && readers[i] == 1 && reader[i] == static_cast<int>(i) + 1) {
+        if (join && i + 1 < p.steps.size() && readers[i] == 1 && reader[i] == static_cast<int>(i) + 1) {
             const auto* first = dynamic_cast<const ConvStep*>(s);
             const auto* second = dynamic_cast<const ConvStep*>(p.steps[i + 1].get());
             if (first && second && first->joins(*second, b, p.tensors)) {
@@ -3159,7 +3161,7 @@ std::shared_ptr<ProgramForm> build_program(const hipie_plan& p, int workgroups, 
                 continue;
             }
         }
-        if (const auto* pair = dynamic_cast<const PairStep*>(s); pair && pair->expands && !keep_values && pair->first->joins(*pair->second, b, p.tensors)) {
+        if (const auto* pair = dynamic_cast<const PairStep*>(s); pair && pair->expands && join && pair->first->joins(*pair->second, b, p.tensors)) {
             inside.push_back(pair->first->out);
             continue;
         }
@@ -3572,7 +3574,7 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
         DeviceGuard dg(device);
         auto program = make_program(device);
         auto build = [&](int workgroups) {
-            return workgroups == 0 || workgroups > program->units ? nullptr : build_program(*plan, workgroups, cfg.keep_f32, plan->single_launch_refused);
+            return workgroups == 0 || workgroups > program->units ? nullptr : build_program(*plan, workgroups, plan->single_launch_refused);
         };
         if (cfg.single_launch > 2) {
             program->lone = program->shared = build(cfg.single_launch);

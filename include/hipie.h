@@ -479,9 +479,10 @@ int hipie_compile(const hipie_graph* graph, int device, hipie_plan** plan);
  * HIP_TUNE (YES | NO: time the kernel variants at load, else shape-based defaults), HIP_TUNE_FILE (cache of the
  * choices, like the reference GPU plugin's KEY_TUNING_FILE), HIP_FUSE_ATTENTION, HIP_MERGE_LINEAR, HIP_KEEP_F32
  * (YES | NO; HIP_KEEP_F32 keeps values that hipie_request_tensor does not find otherwise), HIP_FUSE_CONVOLUTIONS (a 3 x 3
- * convolution and the 1 x 1 convolution that alone reads its result as one kernel, hipie_conv_run_pair: AUTO = where the load-time measurement finds it faster, YES = wherever the kernel takes
- * the pair, NO; the same for a convolution and the depthwise 3 x 3 layer that alone reads its result, in plans that are
- * tuned and without HIP_KEEP_F32; the tensor between two layers run that way exists in LDS only and hipie_request_tensor gives
+ * convolution and the 1 x 1 convolution that alone reads its result as one kernel, hipie_conv_run_pair: AUTO = where the
+ * load-time measurement finds it faster, YES = wherever the kernel takes the pair, NO; the same for a convolution and the
+ * depthwise 3 x 3 layer that alone reads its result, without HIP_KEEP_F32, in plans that are tuned and, measured or not, in a
+ * single launch; the tensor between two layers run that way exists in LDS only and hipie_request_tensor gives
  * HIPIE_NOT_FOUND for it), HIP_SINGLE_LAUNCH (a request that is started and waited for runs as one persistent kernel:
  * AUTO = a plan for one stream, where the load-time measurement finds it faster, YES = wherever the plan has such a form,
  * in the fastest of its sizes, 64 / 128 / 256 = with that many workgroups, NO; beside other requests in flight the smallest

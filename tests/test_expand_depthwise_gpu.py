@@ -63,11 +63,14 @@ def test_one_step_equals_two(name, workgroups):
         reqs[1].tensor(mid)
 
 
-def test_values_that_are_kept_are_two_steps():
+@pytest.mark.parametrize("switch", [{"HIP_KEEP_F32": "YES"}, {"HIP_FUSE_CONVOLUTIONS": "NO"}])
+def test_values_that_are_kept_are_two_steps(switch):
     g, mid = _graph(*CASES["stride_2_odd"])
-    r = g.compile(0, config={"HIP_TUNE": "NO", "HIP_THROUGHPUT_STREAMS": "1", "HIP_SINGLE_LAUNCH": "256", "HIP_KEEP_F32": "YES"}).create_request()
+    plan = g.compile(0, config=dict(switch, HIP_TUNE="NO", HIP_THROUGHPUT_STREAMS="1", HIP_SINGLE_LAUNCH="256"))
+    r = plan.create_request()
     ins, outs = r.device_buffers()
     ins[0].fill_(1.0)
     torch.cuda.synchronize()
     r.infer_device(ins, outs)
+    assert plan.metric("SINGLE_LAUNCH_COUNTS") == "1 0"
     assert r.tensor(mid).max() > 0
