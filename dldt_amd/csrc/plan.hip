@@ -127,7 +127,7 @@ struct EpilogueSpec {
 struct TuneLane {
     uint8_t* arena;
     hipStream_t stream;
-    std::vector<void*> inputs;   // the scratch request's input buffers
+    std::vector<void*> inputs, outputs;   // the scratch request's buffers
 };
 
 struct Step {
@@ -204,7 +204,8 @@ struct ConvStep : Step {
     // run inside this step's kernel when the fused form applies, else right before it
     std::unique_ptr<ConvStep> shortcut;
     bool fused = false;
-    // the graph's result that this step's f32 output is, and nothing else reads: it goes straight into the caller's buffer (-1: none)
+    // the graph's result that this step's f32 output is, and nothing else reads: it goes into the caller's buffer as well as into
+    // its tensor, where hipie_request_tensor finds it (-1: none)
     int result = -1;
     // ... which the layer's kernels can write; the values of single pixels ([N, C]) are a row each either way, their copy is no
     // transposition and goes away in the single launch only
@@ -344,8 +345,8 @@ struct ConvStep : Step {
         const bool has_res = fused || res >= 0 || res_param >= 0;
         auto launch_all = [&](int times) {
             for (int w = 0; w < times; ++w)
-                for (size_t l = 0; l < nl; ++l)      // (a direct result lands in the tensor's own place, which nothing else uses)
-                    check_status(direct ? conv_run_planes(conv, ti[l], to[l], to[l].data, lanes[l].stream)
+                for (size_t l = 0; l < nl; ++l)
+                    check_status(direct ? conv_run_planes(conv, ti[l], to[l], lanes[l].outputs[result], lanes[l].stream)
                                         : hipie_conv_run(conv, &ti[l], has_res ? &tr[l] : nullptr, &to[l], lanes[l].stream), name.c_str());
         };
         std::vector<hipEvent_t> e0(nl), e1(nl);
@@ -1270,7 +1271,7 @@ struct Planner {
     std::vector<std::unique_ptr<Step>> steps;
     std::vector<char> visiting;
     // HIPIE_KEEP_F32=1: store the f32 result of Softmax / MVN / Gelu even when only a fused
-    // FakeQuantize reads it (inspection of the values behind the tolerance-only operations), and an f32 result in its tensor
+    // FakeQuantize reads it (inspection of the values behind the tolerance-only operations)
     bool keep_f32 = false;
     // HIPIE_FUSE_ATTENTION=0: plan the attention core as separate MatMul / Softmax kernels
     bool fuse_attention = true;
@@ -2973,8 +2974,8 @@ struct Planner {
         st->out_u8 = x.kind == VK_TENSOR && tensors[x.tensor].esize() == 1;
         for (size_t i = 0; i < g.results.size(); ++i)
             if (g.results[i] == id) st->result_index = static_cast<int>(i);
-        // an f32 result that only the caller reads: its producer stores it there, in the caller's layout (HIPIE_KEEP_F32 keeps
-        // it where hipie_request_tensor finds it, and copies)
+        // an f32 result that only the caller reads: its producer stores it there, in the caller's layout, beside its own tensor
+        // (with HIPIE_KEEP_F32 the tensor is copied)
         if (x.kind == VK_TENSOR && tensors[x.tensor].dtype == HIPIE_F32 && N(n.in[0]).users.size() == 1 && !keep_f32)
             for (auto& step : steps)
                 if (auto* conv = dynamic_cast<ConvStep*>(step.get()); conv && conv->out == x.tensor && conv->out_node == n.in[0]) {
@@ -3538,8 +3539,9 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
                 hipie_request* q = nullptr;
                 check_status(hipie_request_create(plan.get(), 0, &q), "hipie_compile: tuning request");
                 scratch.r.push_back(q);
-                TuneLane lane{q->arena.as<uint8_t>(), q->stream, {}};
+                TuneLane lane{q->arena.as<uint8_t>(), q->stream, {}, {}};
                 for (auto& b : q->in_dev) lane.inputs.push_back(b.ptr);
+                for (auto& b : q->out_dev) lane.outputs.push_back(b.ptr);
                 lanes.push_back(std::move(lane));
             }
             DeviceGuard dg(device);
@@ -4266,10 +4268,6 @@ int hipie_request_tensor(const hipie_request* r, int node_id, hipie_tensor* t) {
             if (auto* pair = dynamic_cast<const PairStep*>(st.get()))
                 HIPIE_REQUIRE(!(pair->fused && pair->first->out == it->second), HIPIE_NOT_FOUND,
                               "hipie_request_tensor: node %d lives in LDS only (two convolutions run as one kernel)", node_id);
-        for (const auto& st : r->plan->steps)
-            if (auto* conv = dynamic_cast<const ConvStep*>(st.get()))
-                HIPIE_REQUIRE(!((r->ran ? conv->writes_result : conv->direct) && conv->out == it->second), HIPIE_NOT_FOUND,
-                              "hipie_request_tensor: node %d is a result, stored in the caller's buffer only", node_id);
         if (r->ran)
             for (int tensor : r->ran->inside)
                 HIPIE_REQUIRE(tensor != it->second, HIPIE_NOT_FOUND, "hipie_request_tensor: node %d lives in LDS only (two layers are one step of the single launch)", node_id);

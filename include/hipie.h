@@ -595,9 +595,8 @@ int hipie_request_stream(hipie_request* request, void** stream);
 /* milliseconds of step `index` in the last inference (GetPerformanceCounts); a request with counters runs by steps */
 int hipie_request_perf(hipie_request* request, int index, float* ms);
 /* the arena tensor holding the value of graph node `node_id` (inspection, parity tests).  HIPIE_NOT_FOUND where the last
- * inference left it in no tensor: a node fused into its reader, a value between two layers that ran as one kernel or as one step
- * of a single launch, and an f32 result that nothing else reads and its convolution stored in the caller's buffer (of a feature
- * map always, of [N, C] values in a single launch).  With HIP_KEEP_F32 results and values in front of a depthwise layer are there */
+ * inference left it in no tensor: a node fused into its reader, and a value between two layers that ran as one kernel or as one
+ * step of a single launch.  With HIP_KEEP_F32 values in front of a depthwise layer are there */
 int hipie_request_tensor(const hipie_request* request, int node_id, hipie_tensor* tensor);
 
 /* ======================================================================================

@@ -77,28 +77,24 @@ def test_values_without_an_activation_and_with_two_results(relu, results):
 
 
 @pytest.mark.parametrize("hw", [1, 5])
-def test_a_result_that_no_tensor_holds_is_refused(hw):
-    """what the last inference stored in the caller's buffer only is not found, never an older value of its tensor"""
+@pytest.mark.parametrize("keep", ["NO", "YES"])
+def test_a_result_is_in_its_tensor_as_well(hw, keep):
+    """hipie_request_tensor gives a result's values of the last inference, queued or by the single launch, never older ones"""
     rng = np.random.default_rng(hw)
     q = builders.QuantizedNet()
     x = q.input("data", (2, 32, hw, hw), 2.55)
     node = q.conv_f32(x, rng.standard_normal((37, 32, 1, 1), dtype=np.float32) * np.float32(0.2), rng.standard_normal(37, dtype=np.float32))
     q.g.result(node, "out")
-    config = {"HIP_TUNE": "NO", "HIP_THROUGHPUT_STREAMS": "1", "HIP_SINGLE_LAUNCH": "256"}
-    for keep in (False, True):
-        plan = q.g.compile(0, config=dict(config, HIP_KEEP_F32="YES" if keep else "NO"))
-        req = plan.create_request()
-        ins, outs = req.device_buffers()
-        for turn, run in enumerate((req.enqueue, req.infer_device, req.enqueue)):
-            ins[0].uniform_(0, 2.55, generator=torch.Generator(device="cuda").manual_seed(turn))
-            torch.cuda.synchronize()
-            run(ins, outs)
-            torch.cuda.synchronize()
-            # by steps the values of single pixels come by way of the tensor, those of maps only where they are kept
-            if keep or (hw == 1 and run != req.infer_device):
-                assert np.array_equal(req.tensor(node).reshape(-1).view(np.uint32), outs[0].cpu().numpy().reshape(-1).view(np.uint32))
-            else:
-                with pytest.raises(HipieError, match="caller's buffer only") as e:
-                    req.tensor(node)
-                assert e.value.status == -5
-        assert plan.metric("SINGLE_LAUNCH_COUNTS") == "1 0"
+    plan = q.g.compile(0, config={"HIP_TUNE": "NO", "HIP_THROUGHPUT_STREAMS": "1", "HIP_SINGLE_LAUNCH": "256", "HIP_KEEP_F32": keep})
+    req = plan.create_request()
+    ins, outs = req.device_buffers()
+    seen = []
+    for turn, run in enumerate((req.enqueue, req.infer_device, req.enqueue, req.infer_device)):
+        ins[0].uniform_(0, 2.55, generator=torch.Generator(device="cuda").manual_seed(turn))
+        torch.cuda.synchronize()
+        run(ins, outs)
+        torch.cuda.synchronize()
+        seen.append(outs[0].cpu().numpy().reshape(-1))
+        assert np.array_equal(req.tensor(node).reshape(-1).view(np.uint32), seen[-1].view(np.uint32))
+    assert plan.metric("SINGLE_LAUNCH_COUNTS") == "2 0"
+    assert all(not np.array_equal(a, b) for a, b in zip(seen, seen[1:]))
