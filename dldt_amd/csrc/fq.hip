@@ -87,20 +87,41 @@ __global__ __launch_bounds__(kThreads) void fq_nchw_flat(const float* __restrict
     }
 }
 
+// elements that the kernel counts in 32 bits
+constexpr int64_t kFlatMost = (1ll << 32) - 8;
+
+// A plane of three elements and more ends at most once among four.  A tensor of more elements than the kernel counts goes in parts
+// (launch_flat), which have to begin on a 16-byte boundary: whole planes of HW % 4 == 0 do.  3 x 5 planes of 286331156,
+// 4.3e9 elements: -> u8 4.65 ms (an element a thread 7.47), 6 of 4 x 178956972 -> f32 7.69 (13.6).
+bool takes_flat(int64_t total, int64_t hw, const void* x, const void* y, int y_alignment) {
+    return hw >= 3 && (total <= kFlatMost || hw % 4 == 0) && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % y_alignment == 0;
+}
+
 template <bool LEVELS>
-void launch_flat(bool rcp, const float* x, void* y, const FqChannel* tab, float lm1, float off, int64_t total, int64_t hw, uint32_t C, hipStream_t s) {
+void launch_flat(bool rcp, const float* x, void* y, const FqChannel* tab, float lm1, float off, int64_t images, int64_t hw, int64_t C, hipStream_t s) {
+    const int64_t total = images * C * hw;
+    if (total > kFlatMost) {
+        // as many whole images as fit, or of one image channels
+        const int64_t plane = images > 1 ? C * hw : hw, planes = images > 1 ? images : C, most = std::max<int64_t>(1, kFlatMost / plane);
+        for (int64_t i = 0; i < planes; i += most) {
+            const int64_t count = std::min(most, planes - i);
+            launch_flat<LEVELS>(rcp, x + i * plane, static_cast<uint8_t*>(y) + i * plane * (LEVELS ? 1 : 4), images > 1 ? tab : tab + i, lm1, off,
+                                images > 1 ? count : 1, hw, images > 1 ? C : count, s);
+        }
+        return;
+    }
     const dim3 grid(grid_for(ceil_div(total, 4))), block(kThreads);
     const uint32_t n = static_cast<uint32_t>(total);
     if (hw % 4 == 0) {
         auto k = rcp ? fq_nchw_flat<true, LEVELS, true> : fq_nchw_flat<false, LEVELS, true>;
-        hipLaunchKernelGGL(k, grid, block, 0, s, x, y, tab, lm1, off, n, Divider(static_cast<uint32_t>(hw / 4)), Divider(C));
+        hipLaunchKernelGGL(k, grid, block, 0, s, x, y, tab, lm1, off, n, Divider(static_cast<uint32_t>(hw / 4)), Divider(static_cast<uint32_t>(C)));
     } else {
         auto k = rcp ? fq_nchw_flat<true, LEVELS, false> : fq_nchw_flat<false, LEVELS, false>;
-        hipLaunchKernelGGL(k, grid, block, 0, s, x, y, tab, lm1, off, n, Divider(static_cast<uint32_t>(hw)), Divider(C));
+        hipLaunchKernelGGL(k, grid, block, 0, s, x, y, tab, lm1, off, n, Divider(static_cast<uint32_t>(hw)), Divider(static_cast<uint32_t>(C)));
     }
 }
 
-// planes of fewer than three elements, buffers off the 16-byte boundary, 2^32 elements and more: one element per thread and iteration
+// what takes_flat refuses: one element per thread and iteration
 template <bool RCP>
 __global__ __launch_bounds__(kThreads) void fq_nchw_q8_scalar(const float* __restrict__ x,
                                                                uint8_t* __restrict__ y,
@@ -824,9 +845,8 @@ int hipie_fq_run_f32(const hipie_fq* fq, const float* x, float* y, int64_t n, in
         const FqChannel* tab = fq->table.as<FqChannel>();
         const uint32_t C = static_cast<uint32_t>(fq->C);
         hipStream_t s = as_stream(stream);
-        // (a plane of three elements and more ends at most once among four)
-        if (hw >= 3 && total < (1ll << 32) - 4 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0) {
-            launch_flat<false>(fq->rcp, x, y, tab, fq->lm1, 0.0f, total, hw, C, s);
+        if (takes_flat(total, hw, x, y, 16)) {
+            launch_flat<false>(fq->rcp, x, y, tab, fq->lm1, 0.0f, n, hw, fq->C, s);
         } else {
             auto k = fq->rcp ? fq_nchw_f32<true> : fq_nchw_f32<false>;
             hipLaunchKernelGGL(k, dim3(grid_for(total)), dim3(kThreads), 0, s, x, y, tab, fq->lm1,
@@ -877,8 +897,8 @@ int hipie_fq_run_q8(const hipie_fq* fq, const float* x, void* y, int64_t n, int6
         const uint32_t C = static_cast<uint32_t>(fq->C);
         hipStream_t s = as_stream(stream);
         if (out_layout == HIPIE_NCHW) {
-            if (hw >= 3 && total < (1ll << 32) - 4 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 4 == 0) {
-                launch_flat<true>(fq->rcp, x, y, tab, fq->lm1, off, total, hw, C, s);
+            if (takes_flat(total, hw, x, y, 4)) {
+                launch_flat<true>(fq->rcp, x, y, tab, fq->lm1, off, n, hw, fq->C, s);
             } else {
                 auto k = fq->rcp ? fq_nchw_q8_scalar<true> : fq_nchw_q8_scalar<false>;
                 hipLaunchKernelGGL(k, dim3(grid_for(total)), dim3(kThreads), 0, s, x,

@@ -177,3 +177,47 @@ def test_fq_planes_that_end_inside_a_group_of_four(orc, shape, shift):
     lv = (fq.run_q8(xd, "u8b", "nhwc", cs).cpu().numpy().astype(np.int16) + 128).astype(np.uint8)
     np.testing.assert_array_equal(lv[..., :C], want.astype(np.uint8).transpose(0, 2, 3, 1))
     assert np.all(lv[..., C:] == 0)
+
+
+@pytest.mark.parametrize("form,shape", [("u8", (3, 5, 1, 286331156)), ("u8", (1, 7, 1, 613566760)), ("f32", (2, 3, 4, 178956972)), ("u8", (2, 2, 1, 1073741826))])
+def test_more_than_32_bits_of_elements(form, shape):
+    """tensors that are split into launches of less than 2^32 elements, by images and by channels, against the operator image by
+    image and channel by channel; and in the time of these (a plane of HW % 4 != 0, the last shape, is not split)"""
+    import torch
+    from dldt_amd import FakeQuantize
+    n, c, h, w = shape
+    assert n * c * h * w >= 2 ** 32
+    x = torch.empty(shape, device="cuda")
+    for i in range(n):
+        for j in range(c):
+            x[i, j].normal_(0.1 * j, generator=torch.Generator(device="cuda").manual_seed(c * i + j))
+    low, high = np.linspace(-3, -2, c).astype(np.float32), np.linspace(2, 3, c).astype(np.float32)
+    fq = FakeQuantize(c, 256, low, high, 0.0, 255.0)
+    one = [FakeQuantize(1, 256, low[j], high[j], 0.0, 255.0) for j in range(c)]
+
+    def run(f, v, out):
+        return f.run_f32(v, out=out) if form == "f32" else f.run_q8(v, "u8", "nchw", out=out)
+
+    def micros(call):
+        t = []
+        for _ in range(4):
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            e[0].record()
+            call()
+            e[1].record()
+            torch.cuda.synchronize()
+            t.append(e[0].elapsed_time(e[1]) * 1e3)
+        return min(t)
+
+    dtype = torch.float32 if form == "f32" else torch.uint8
+    y, part = torch.empty(shape, dtype=dtype, device="cuda"), torch.empty((1, 1, h, w), dtype=dtype, device="cuda")
+    whole = micros(lambda: run(fq, x, y))
+    parts = 0.0
+    for i in range(n):
+        for j in range(c):
+            v = x[i:i + 1, j:j + 1]
+            parts += micros(lambda: run(one[j], v, part))
+            assert torch.equal(y[i, j], part[0, 0]), (i, j)
+    print("%s %s: %.0f us whole, %.0f in parts" % (form, shape, whole, parts))
+    if h * w % 4 == 0:
+        assert whole < 1.3 * parts
