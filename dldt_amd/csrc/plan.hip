@@ -3128,7 +3128,7 @@ bool run_again(hipie_request* r) {
 }
 
 // the single-launch form of a plan whose every step has one, or null and what it has no room for
-std::shared_ptr<ProgramForm> build_program(const hipie_plan& p, int workgroups, std::string& refused) {
+std::shared_ptr<ProgramForm> build_program(const hipie_plan& p, int workgroups, std::string& refused, bool mixed = false) {
     if (p.inputs.size() + p.outputs.size() > static_cast<size_t>(kProgramIo)) {
         refused = "inputs and outputs";
         return nullptr;
@@ -3136,6 +3136,7 @@ std::shared_ptr<ProgramForm> build_program(const hipie_plan& p, int workgroups, 
     ProgBuilder b;
     b.device = p.device;
     b.workgroups = workgroups;
+    b.mixed = mixed;
     std::vector<void*> in, out;
     for (size_t i = 0; i < p.inputs.size(); ++i) in.push_back(b.fake_io(static_cast<int>(i)));
     for (size_t i = 0; i < p.outputs.size(); ++i) out.push_back(b.fake_io(static_cast<int>(p.inputs.size() + i)));
@@ -3171,10 +3172,7 @@ std::shared_ptr<ProgramForm> build_program(const hipie_plan& p, int workgroups, 
             return nullptr;
         }
     }
-    if (b.map_kinds && b.rows_kinds) {       // (a kernel with the steps of both has no registers left for either's)
-        refused = "feature maps and rows";
-        return nullptr;
-    }
+    if (b.map_kinds && b.rows_kinds && !mixed) return build_program(p, workgroups, refused, true);       // (its tiles are chosen for its kernel)
     auto form = make_program_form(std::move(b));
     form->inside = std::move(inside);
     return form;

@@ -116,7 +116,8 @@ struct ProgBuilder {
     int workgroups = 256;
     std::vector<std::array<int32_t, kProgramStepWords>> steps;
     std::vector<DeviceBuffer> owned;      // repacked weights, tables
-    bool map_kinds = false, rows_kinds = false;      // steps of a network over feature maps, of an encoder: a kernel for each
+    bool map_kinds = false, rows_kinds = false;      // steps of a network over feature maps, of an encoder: a kernel for each, and one for both
+    bool mixed = false;                              // built for the latter
     ProgPtr keep(const void* host, size_t bytes);                              // a table of the program's own
     ProgPtr gather(const std::vector<const void*>& rows, size_t pitch);
     static uint8_t* fake_arena() { return reinterpret_cast<uint8_t*>(uintptr_t(1) << 32); }
@@ -156,7 +157,7 @@ struct ProgBuilder {
 struct ProgramForm {
     int workgroups = 0, n_steps = 0;
     std::vector<int> inside;              // the plan's tensors that live inside a step
-    bool encoder = false;                    // which of the two kernels
+    bool maps = false, rows = false;         // which of the kernels
     DeviceBuffer steps;
     std::vector<DeviceBuffer> owned;
 };

@@ -1555,11 +1555,13 @@ __device__ __forceinline__ void attention_units(const ProgAttention& s, Ctx& x, 
 __device__ __forceinline__ int lane_index() { return static_cast<int>(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u))); }
 
 // ---- the program ------------------------------------------------------------------------------------------------------------
-// Two kernels, for networks over feature maps and for encoders: every kind of step adds to the registers of all others (all in
-// one spill).  The 4 x 4 tiles ask for 250 and more vector registers, none is spilled to memory; 300 - 400 scalar registers of
-// the many step kinds are kept in lanes of vector registers.  A new step kind belongs into a kernel of its own where it needs
-// more than they have.
-template <bool ENCODER>
+// Three kernels, for networks over feature maps, for encoders, and for graphs with steps of both: every kind of step adds to the
+// registers of all others.  The 4 x 4 tiles ask for 250 and more vector registers, none is spilled to memory; 460 - 510 scalar
+// registers of the many step kinds are kept in lanes of vector registers.  The kernel with all kinds has no registers left for
+// 4 x 4 tiles (with them it spills); its convolutions take smaller ones (an encoder layer of 96 tokens beside a ResNet-50 of width
+// 16 at 64 x 64: 244 us, 467 by steps; beside a MobileNetV2 of 2 x 96 x 96 208 and 512).  A new step kind belongs into a kernel of its own where it
+// needs more than they have.
+template <bool MAPS, bool ROWS>
 __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgArgs g) {
     extern __shared__ __attribute__((aligned(16))) int8_t smem[];
     lds_ptr lds = (lds_ptr)smem;
@@ -1599,17 +1601,19 @@ __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgA
         switch (kind) {
         case PK_CONV: {
             switch (PROG_FIELD(x.words, a) * 8 + PROG_FIELD(x.words, b) + (PROG_FIELD(x.words, nk2) ? 64 : 0)) {
-            case 8 + 1: conv_tiles<ENCODER, 1, 1>(x, lds); break;
-            case 16 + 1: conv_tiles<ENCODER, 2, 1>(x, lds); break;
-            case 16 + 2: conv_tiles<ENCODER, 2, 2>(x, lds); break;
-            case 32 + 2: conv_tiles<ENCODER, 4, 2>(x, lds); break;
+            case 8 + 1: conv_tiles<ROWS, 1, 1>(x, lds); break;
+            case 16 + 1: conv_tiles<ROWS, 2, 1>(x, lds); break;
+            case 16 + 2: conv_tiles<ROWS, 2, 2>(x, lds); break;
+            case 32 + 2: conv_tiles<ROWS, 4, 2>(x, lds); break;
             case 64 + 16 + 2:
-                if constexpr (!ENCODER) conv_tiles<ENCODER, 2, 2, true>(x, lds);
+                if constexpr (MAPS) conv_tiles<ROWS, 2, 2, true>(x, lds);
                 break;
             case 64 + 16 + 4:
-                if constexpr (!ENCODER) conv_tiles<ENCODER, 2, 4, true>(x, lds);
+                if constexpr (MAPS) conv_tiles<ROWS, 2, 4, true>(x, lds);
                 break;
-            default: conv_tiles<ENCODER, 4, 4>(x, lds); break;
+            default:
+                if constexpr (!(MAPS && ROWS)) conv_tiles<ROWS, 4, 4>(x, lds);      // (choose_tile)
+                break;
             }
             break;
         }
@@ -1624,16 +1628,18 @@ __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgA
         case PK_FQROWS: fq_items(unpack<ProgRows>(words), x); break;
         case PK_COPY: copy_items(unpack<ProgRows>(words), x); break;
         default:
-            if constexpr (ENCODER) {
+            if constexpr (ROWS) {
                 if (kind == PK_EMBED) embed_rows(unpack<ProgEmbed>(words), x);
                 else if (kind == PK_MVN) mvn_rows(unpack<ProgMvn>(words), x);
-                else {
+                else if (!MAPS || kind == PK_ATTENTION) {
                     const ProgAttention t = unpack<ProgAttention>(words);
                     if (t.S > kPlainSoftmax) attention_units<true, 0>(t, x, lds);
                     else if (t.pform == 2) attention_units<false, 2>(t, x, lds);
                     else attention_units<false, 0>(t, x, lds);
                 }
-            } else if (kind == PK_DW) {
+            }
+            if constexpr (!MAPS) break;
+            else if (kind == PK_DW) {
                 switch (PROG_FIELD(x.words, stride) * 8 + PROG_FIELD(x.words, group)) {
                 case 8 + 1: dw_items<1, 1>(x); break;
                 case 8 + 4: dw_items<1, 4>(x); break;
@@ -1644,7 +1650,7 @@ __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgA
                 if (PROG_FIELD(x.words, a) == 1) expand_depthwise<1>(x, lds);
                 else expand_depthwise<2>(x, lds);
             } else if (kind == PK_MAXPOOL) max_pool_items(unpack<ProgPool>(words), x);
-            else avg_pool_items(unpack<ProgPool>(words), x);
+            else if (!ROWS || kind == PK_AVGPOOL) avg_pool_items(unpack<ProgPool>(words), x);
         }
         if (step + 1 == g.n_steps) break;
         {   // the next step's descriptor into the scalar cache: its eight lines asked for together, beside the stores' way to memory
@@ -1690,14 +1696,14 @@ __global__ void clear_words(uint32_t* p, int n) {
 // f32 chain per value, a store instruction, the partial sums of the waves that share a K in LDS.  Rounds are tiles a wave takes
 // one after another.
 struct TileChoice { int a, b, ks; };
-TileChoice choose_tile(int workgroups, int oc, int64_t pixels, int nk, int nk2, bool gelu) {
+TileChoice choose_tile(int workgroups, int oc, int64_t pixels, int nk, int nk2, bool gelu, bool mixed) {
     static constexpr int kShapes[6][2] = {{4, 4}, {4, 2}, {2, 2}, {2, 1}, {1, 1}, {2, 4}};
-    TileChoice best{4, 4, 1};
+    TileChoice best{4, 2, 1};
     double best_t = 1e30;
     for (const auto& shape : kShapes)
         for (int ks : {1, 2, 4, 8}) {
             const int a = shape[0], b = shape[1];
-            if ((nk2 && (a != 2 || b < 2)) || (gelu && a == 1) || (b == 4 && (ks == 8 || (a == 2 && !nk2)))) continue;
+            if ((nk2 && (a != 2 || b < 2)) || (gelu && a == 1) || (b == 4 && (ks == 8 || (a == 2 && !nk2) || (a == 4 && mixed)))) continue;
             const int depth = a * b >= 16 ? 2 : (a * b >= 8 ? 4 : 6);
             const int64_t tiles = ceil_div(oc, 16 * a) * ceil_div(pixels, 16 * b), per_wg = ceil_div(tiles, workgroups);
             const int64_t rounds = ceil_div(per_wg, 8 / ks);
@@ -1906,7 +1912,7 @@ bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hip
     if (a.flags & CF_GELU) rows_kinds = true;
     if (pair) map_kinds = true;
     if (4 * a.nk > kMaxPieces || (pair && 4 * a.nk2 > kMaxPieces)) return false;
-    const TileChoice t = choose_tile(workgroups, a.OC, M, a.nk, pair ? a.nk2 : 0, (a.flags & CF_GELU) != 0);
+    const TileChoice t = choose_tile(workgroups, a.OC, M, a.nk, pair ? a.nk2 : 0, (a.flags & CF_GELU) != 0, mixed);
     c.a = t.a; c.b = t.b; c.ks_shift = __builtin_ctz(static_cast<unsigned>(t.ks));
     // (the channels the tensor is padded with are written too)
     const int o_tiles = static_cast<int>(ceil_div(std::min(c.out_limit, a.OCp), 16 * t.a));
@@ -2178,7 +2184,8 @@ std::shared_ptr<ProgramForm> make_program_form(ProgBuilder&& b) {
     auto f = std::make_shared<ProgramForm>();
     f->workgroups = b.workgroups;
     f->n_steps = static_cast<int>(b.steps.size());
-    f->encoder = b.rows_kinds;
+    f->maps = b.map_kinds;
+    f->rows = b.rows_kinds;
     f->steps.upload(b.device, b.steps.data(), b.steps.size() * kProgramStepWords * 4);
     f->owned = std::move(b.owned);
     DeviceGuard g(b.device);
@@ -2199,7 +2206,7 @@ std::shared_ptr<Program> make_program(int device) {
     DeviceGuard g(device);
     HIPIE_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&p->report), Program::kSlots * 64, hipHostMallocDefault));
     std::memset(p->report, 0, Program::kSlots * 64);
-    for (auto kernel : {&program_kernel<false>, &program_kernel<true>})
+    for (auto kernel : {&program_kernel<true, false>, &program_kernel<false, true>, &program_kernel<true, true>})
         HIPIE_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     return p;
 }
@@ -2261,7 +2268,9 @@ void launch_program(const Program& p, const ProgramForm& f, uint8_t* arena, void
     a.launch = launch;
     a.roll_call_ticks = p.roll_call_ticks;
     p.report[16 * slot] = 0;
-    hipLaunchKernelGGL(f.encoder ? program_kernel<true> : program_kernel<false>, dim3(static_cast<uint32_t>(f.workgroups)), dim3(kProgramThreads), kLdsBytes, s, a);
+    auto kernel = &program_kernel<true, false>;
+    if (f.rows) kernel = f.maps ? &program_kernel<true, true> : &program_kernel<false, true>;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(f.workgroups)), dim3(kProgramThreads), kLdsBytes, s, a);
     HIPIE_CHECK_HIP(hipGetLastError());
 }
 

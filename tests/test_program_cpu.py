@@ -69,7 +69,7 @@ def test_no_register_is_copied_where_a_mask_of_the_persistent_kernel_ends(tmp_pa
                    check=True, capture_output=True)
     text = out.read_text()
     found = [m.start() for m in re.finditer(r"^_ZN\S*program_kernel\S*:", text, re.M)]
-    assert len(found) == 2                                          # feature maps, encoders
+    assert len(found) == 3                                          # feature maps, encoders, both
     for start in found:
         kernel = text[start:]
         kernel = kernel[:kernel.index(".end_amdhsa_kernel")]

@@ -2,6 +2,7 @@
 K of one step and of many, strides, residuals, shortcuts, depthwise, pools, encoder steps; the ordering of launches on
 several streams; and the way back to the steps when a launch is cancelled."""
 import threading
+from unittest import mock
 
 import numpy as np
 import pytest
@@ -12,6 +13,22 @@ from dldt_amd._lib import check, lib
 from dldt_amd.graph import Plan
 
 pytestmark = pytest.mark.gpu
+
+
+
+def _beside_an_encoder(build, **kw):
+    """an encoder and a network over feature maps as one graph of two branches"""
+    g = builders.bert_encoder(layers=1, batch=1, seq=96, vocab=100, mask=True)[0]
+
+    class Beside(builders.QuantizedNet):
+        def __init__(self):
+            super().__init__()
+            self.g = g
+
+    with mock.patch.object(builders, "QuantizedNet", Beside):
+        assert build(**kw)[0] is g
+    return g
+
 
 GRAPHS = {
     "block_1x3x7": lambda: builders.conv_block(n=1, c=3, hw=7, oc=8)[0],
@@ -34,6 +51,8 @@ GRAPHS = {
     "encoder_1x160": lambda: builders.bert_encoder(layers=1, batch=1, seq=160, vocab=100, mask=True)[0],       # five tiles of keys for eight waves
     "encoder_4x128": lambda: builders.bert_encoder(layers=1, batch=4, seq=128, vocab=100, mask=True)[0],       # two waves for 32 queries (64 workgroups)
     "encoder_1x448": lambda: builders.bert_encoder(layers=1, batch=1, seq=448, vocab=100, mask=True)[0],
+    "encoder_and_resnet": lambda: _beside_an_encoder(builders.resnet50, batch=1, res=64, width=16, classes=10, seed=7),
+    "encoder_and_mobilenet": lambda: _beside_an_encoder(builders.mobilenet_v2, batch=2, res=96),
     "encoder_2x384": lambda: builders.bert_encoder(layers=1, batch=2, seq=384, vocab=100, mask=True)[0],
 }
 
