@@ -3008,6 +3008,7 @@ struct hipie_plan {
     hipie_graph graph;                       // the description the plan was compiled from (what an export writes)
     std::vector<TensorInfo> tensors;
     std::vector<std::unique_ptr<Step>> steps;
+    std::vector<int> choices;                // kernel variants by step as planned, pairs as one, for an export
     std::map<int, int> node_tensor;          // graph node -> tensor holding its value
     struct Slice { int tensor; int64_t offset, rows, cols, pitch; };
     std::map<int, Slice> node_slice;         // graph node -> rows x cols window of a tensor (row-major views)
@@ -3417,38 +3418,6 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
             plan->steps[i] = std::move(pair);
             plan->steps.erase(plan->steps.begin() + static_cast<std::ptrdiff_t>(i) + 1);
         }
-    {
-        // the edges of the executed graph (what GetExecGraphInfo draws): an operand of a step is a node outside its set -
-        // computed by another step, held by a tensor another step produced (a symbolic dequantization in between belongs
-        // to nobody), or a graph input
-        std::map<int, int> step_of_node, param_index;
-        for (size_t i = 0; i < plan->steps.size(); ++i)
-            for (int v : plan->steps[i]->nodes) step_of_node[v] = static_cast<int>(i);
-        for (size_t k = 0; k < g->params.size(); ++k) param_index[g->params[k]] = static_cast<int>(k);
-        for (size_t i = 0; i < plan->steps.size(); ++i) {
-            Step& st = *plan->steps[i];
-            std::vector<int> src;
-            for (int v : st.nodes) {
-                std::vector<int> pending(g->nodes[v].in.begin(), g->nodes[v].in.end());
-                while (!pending.empty()) {
-                    const int in = pending.back();
-                    pending.pop_back();
-                    if (in < 0 || g->nodes[in].op == OP_CONSTANT || std::binary_search(st.nodes.begin(), st.nodes.end(), in)) continue;
-                    int from = 0;
-                    bool known = true;
-                    const auto own = step_of_node.find(in);
-                    if (own != step_of_node.end() && own->second != static_cast<int>(i)) from = own->second;
-                    else if (param_index.count(in)) from = -(1 + param_index[in]);
-                    else if (own == step_of_node.end()) {   // a node no step owns (Convert / Subtract / Multiply over bytes, Reshape): look through it
-                        for (int up : g->nodes[in].in) pending.push_back(up);
-                        known = false;
-                    } else known = false;
-                    if (known && std::find(src.begin(), src.end(), from) == src.end()) src.push_back(from);
-                }
-            }
-            st.sources = src;
-        }
-    }
     for (size_t i = 0; i < pl.values.size(); ++i)
         if (pl.values[i].kind == VK_TENSOR) {
             plan->node_tensor[static_cast<int>(i)] = pl.values[i].tensor;
@@ -3487,10 +3456,14 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
         }
     }
     const char* cache = nullptr;
+    auto keep_choices = [&] {
+        plan->choices.clear();
+        for (const auto& st : plan->steps) plan->choices.push_back(st->variant());
+    };
     auto write_cache = [&] {
         FILE* f = cache ? std::fopen(cache, "w") : nullptr;
         if (!f) return;
-        for (size_t i = 0; i < plan->steps.size(); ++i) std::fprintf(f, "%zu %d\n", i, plan->steps[i]->variant());
+        for (size_t i = 0; i < plan->choices.size(); ++i) std::fprintf(f, "%zu %d\n", i, plan->choices[i]);
         if (forms.known) std::fprintf(f, "-1 %d\n-2 %d\n", forms.lone, forms.shared);
         std::fclose(f);
     };
@@ -3544,7 +3517,50 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
             }
             DeviceGuard dg(device);
             for (auto& s : plan->steps) s->tune(lanes, plan->tensors);
+            keep_choices();
             write_cache();
+        }
+    }
+    keep_choices();
+    // an expansion that runs apart from its depthwise layer is a step of its own again (its counters, its node of the executed graph)
+    for (size_t i = 0; i < plan->steps.size(); ++i) {
+        auto* pair = dynamic_cast<PairStep*>(plan->steps[i].get());
+        if (!pair || !pair->expands || pair->fused) continue;
+        std::unique_ptr<Step> first = std::move(pair->first), second = std::move(pair->second);
+        plan->steps[i] = std::move(second);
+        plan->steps.insert(plan->steps.begin() + static_cast<std::ptrdiff_t>(i), std::move(first));
+        ++i;
+    }
+    {
+        // the edges of the executed graph (what GetExecGraphInfo draws): an operand of a step is a node outside its set -
+        // computed by another step, held by a tensor another step produced (a symbolic dequantization in between belongs
+        // to nobody), or a graph input
+        std::map<int, int> step_of_node, param_index;
+        for (size_t i = 0; i < plan->steps.size(); ++i)
+            for (int v : plan->steps[i]->nodes) step_of_node[v] = static_cast<int>(i);
+        for (size_t k = 0; k < g->params.size(); ++k) param_index[g->params[k]] = static_cast<int>(k);
+        for (size_t i = 0; i < plan->steps.size(); ++i) {
+            Step& st = *plan->steps[i];
+            std::vector<int> src;
+            for (int v : st.nodes) {
+                std::vector<int> pending(g->nodes[v].in.begin(), g->nodes[v].in.end());
+                while (!pending.empty()) {
+                    const int in = pending.back();
+                    pending.pop_back();
+                    if (in < 0 || g->nodes[in].op == OP_CONSTANT || std::binary_search(st.nodes.begin(), st.nodes.end(), in)) continue;
+                    int from = 0;
+                    bool known = true;
+                    const auto own = step_of_node.find(in);
+                    if (own != step_of_node.end() && own->second != static_cast<int>(i)) from = own->second;
+                    else if (param_index.count(in)) from = -(1 + param_index[in]);
+                    else if (own == step_of_node.end()) {   // a node no step owns (Convert / Subtract / Multiply over bytes, Reshape): look through it
+                        for (int up : g->nodes[in].in) pending.push_back(up);
+                        known = false;
+                    } else known = false;
+                    if (known && std::find(src.begin(), src.end(), from) == src.end()) src.push_back(from);
+                }
+            }
+            st.sources = src;
         }
     }
     // (a plan that was exported with its kernels chosen and no form measured had none)
@@ -3804,7 +3820,7 @@ static void unpack_options(uint16_t o, PlanConfig& cfg, FormChoice& forms) {
 int hipie_plan_export(const hipie_plan* p, void* buffer, size_t capacity, size_t* size) {
     return guarded([&] {
         HIPIE_REQUIRE(p && size, HIPIE_PARAMETER_MISMATCH, "hipie_plan_export: null argument");
-        const size_t head = 16 + 4 * p->steps.size();
+        const size_t head = 16 + 4 * p->choices.size();
         const size_t graph_bytes = serialize_graph(p->graph, nullptr);
         size_t prepared = 8 + 24 * p->verdicts.rcp.size() + 8 + 16 * p->verdicts.div2.size() + 8;
         for (const auto& blob : p->tape.blobs) prepared += 8 + blob.size();
@@ -3813,11 +3829,11 @@ int hipie_plan_export(const hipie_plan* p, void* buffer, size_t capacity, size_t
         HIPIE_REQUIRE(capacity >= *size, HIPIE_OUT_OF_BOUNDS, "hipie_plan_export: %zu bytes needed, %zu given", *size, capacity);
         uint8_t* b = static_cast<uint8_t*>(buffer);
         std::memcpy(b, kPlanMagic, 8);
-        const uint32_t fmt = kPlanFormat | static_cast<uint32_t>(pack_options(*p)) << 16, ns = static_cast<uint32_t>(p->steps.size());
+        const uint32_t fmt = kPlanFormat | static_cast<uint32_t>(pack_options(*p)) << 16, ns = static_cast<uint32_t>(p->choices.size());
         std::memcpy(b + 8, &fmt, 4);
         std::memcpy(b + 12, &ns, 4);
-        for (size_t i = 0; i < p->steps.size(); ++i) {
-            const int32_t v = p->steps[i]->variant();
+        for (size_t i = 0; i < p->choices.size(); ++i) {
+            const int32_t v = p->choices[i];
             std::memcpy(b + 16 + 4 * i, &v, 4);
         }
         const uint64_t gb = graph_bytes;

@@ -7,6 +7,7 @@ import torch
 
 from dldt_amd import HipieError
 from dldt_amd.builders import QuantizedNet
+from dldt_amd.graph import Plan
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +70,63 @@ def test_one_launch_equals_two(name, form, tmp_path):
     assert reqs[0].tensor(mid) is not None
     with pytest.raises(HipieError, match="LDS only"):
         reqs[1].tensor(mid)
+
+
+def _two_blocks():
+    rng = np.random.default_rng(8)
+    net = QuantizedNet()
+    a, mids = net.input("data", (2, 16, 12, 12), 2.0), []
+    for c, oc in ((16, 48), (24, 64)):
+        mid = net.conv_relu6(a, rng.normal(0, 1 / np.sqrt(c), (oc, c, 1, 1)).astype(np.float32), rng.normal(0, 0.2, oc).astype(np.float32), 3.0)
+        b = net.conv_relu6(mid, rng.normal(0, 0.4, (oc, 1, 3, 3)).astype(np.float32), rng.normal(0, 0.2, oc).astype(np.float32), 3.0, pads=(1, 1), grouped=True)
+        mids.append(mid["node"])
+        a = net.conv(b, rng.normal(0, 0.2, (24, oc, 1, 1)).astype(np.float32), None, 3.0)
+    net.g.result(net.dequantize(a), "out")
+    return net.g, mids
+
+
+@pytest.mark.parametrize("single", ["NO", "256"])
+@pytest.mark.parametrize("apart", [(), (0,), (1,), (0, 1)])
+def test_layers_that_run_apart_are_two_steps(apart, single, tmp_path):
+    """each has its line in the counters and its node of the executed graph; the choices survive a file and an export"""
+    g, mids = _two_blocks()
+    config = {"HIP_THROUGHPUT_STREAMS": "1", "HIP_SINGLE_LAUNCH": single}
+    both = g.compile(0, config=dict(config, HIP_TUNE="NO", HIP_FUSE_CONVOLUTIONS="YES"))
+    two = g.compile(0, config=dict(config, HIP_TUNE="NO", HIP_FUSE_CONVOLUTIONS="NO"))
+    pairs = [i for i, s in enumerate(both.steps) if s["type"] == "GroupConvolution"]
+    assert len(pairs) == 2 and len(both.steps) == len(two.steps) - 2
+    text = "".join("%d %d\n" % (i, s["variant"] & ~4096 if i in [pairs[k] for k in apart] else s["variant"]) for i, s in enumerate(both.steps))
+    (tmp_path / "choices").write_text(text)
+    plan = g.compile(0, config=dict(config, HIP_TUNE="YES", HIP_TUNE_FILE=str(tmp_path / "choices")))
+    assert (tmp_path / "choices").read_text() == text                     # it was taken as it is
+    assert len(plan.steps) == len(both.steps) + len(apart)
+    at = pairs[0]                                                         # the first block's step, or the first of its two
+    for k in range(2):
+        types = [s["type"] for s in plan.steps[at:at + 2]]
+        if k in apart:
+            assert types == ["Convolution", "GroupConvolution"] and plan.step_sources(at + 1) == [at] and plan.step_sources(at + 2) == [at + 1]
+        else:
+            assert types[0] == "GroupConvolution" and plan.step_sources(at + 1) == [at]
+        at += 3 if k in apart else 2                                      # (behind them the projection)
+    again = Plan.load(plan.export())
+    assert [(s["type"], s["name"], s["variant"]) for s in again.steps] == [(s["type"], s["name"], s["variant"]) for s in plan.steps]
+    x = torch.rand((2, 16, 12, 12), generator=torch.Generator(device="cuda").manual_seed(1), device="cuda") * 2
+    results = []
+    for p in (two, plan, again):
+        r = p.create_request(perf_count=p is plan and single == "NO")
+        ins, outs = r.device_buffers()
+        ins[0].copy_(x)
+        torch.cuda.synchronize()
+        r.infer_device(ins, outs)
+        results.append(outs[0].cpu().numpy())
+        if p is plan and single == "NO":
+            counters = {s["name"]: s["ms"] for s in r.perf()}
+            assert len(counters) == len(plan.steps) and all(ms > 0 for n, ms in counters.items() if n != "out")
+            for k in range(2):
+                if k in apart:
+                    assert r.tensor(mids[k]).max() > 0
+                else:
+                    with pytest.raises(HipieError, match="LDS only"):
+                        r.tensor(mids[k])
+    assert np.abs(results[0]).max() > 0
+    assert all(np.array_equal(results[0].view(np.uint8), v.view(np.uint8)) for v in results[1:])
