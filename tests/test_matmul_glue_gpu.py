@@ -460,3 +460,23 @@ def test_a_row_of_mvn_is_divided_as_by_the_ieee_division(axis, eps):
     want = x / np.float32(eps)
     got = mvn(torch.from_numpy(x).cuda(), True, eps, False).cpu().numpy()
     np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("eps", [1.0, 0.7, 3.1, 1.3 * 2.0 ** -20, 1.1 * 2.0 ** -59, 1.1 * 2.0 ** -61, 1.7 * 2.0 ** 59])
+@pytest.mark.parametrize("axis", [4, 260, 768])
+def test_a_row_of_mvn_keeps_the_ieee_quotient_of_small_values_and_zeros(axis, eps):
+    """pairs t, -t as above, with t from eps 2^-27 down to the least subnormal number, and zeros of both signs"""
+    import torch
+    from dldt_amd import mvn
+    rng = np.random.default_rng(axis)
+    rows, top = 600, np.floor(np.log2(eps)) - 27
+    least = np.linspace(-149.0, top, rows)[:, None]                       # a row's own range: eight binades from here on
+    t = np.exp2(np.minimum(least + rng.uniform(0, 8, (rows, axis // 2)), top)).astype(np.float32)
+    t[rng.random(t.shape) < 0.05] = 0
+    t *= rng.choice(np.float32([-1, 1]), t.shape)
+    x = np.stack([t, -t], axis=-1).reshape(rows, axis)
+    want = x / np.float32(eps)
+    assert np.signbit(x[x == 0]).any() and (np.abs(x[x != 0]).min() < 2.0 ** -126)
+    got = mvn(torch.from_numpy(x).cuda(), True, eps, False).cpu().numpy()
+    # a pair's sum is +0 whatever the signs of its zeros, and so is the mean
+    np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
