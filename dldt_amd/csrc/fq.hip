@@ -572,12 +572,20 @@ struct hipie_fq {
 };
 
 // whether a transposition runs in tiles of 32 pixels x 256 channels or 256 x 64 (four pixels a lane) instead of 64 x 64 (one).
-// The former take every tensor whose channels make whole lines ([32, 256, 55, 57] 34.9 us, 40.0 in small tiles); the latter need
-// a workgroup for every compute unit, two of them where their loads are not aligned: small tiles / 256 x 64 in us,
-// [12, 72, 44, 44] (192 workgroups) 5.1 / 6.2, [64, 64, 28, 28] (256) 7.2 / 6.6, [64, 64, 31, 31] (256) 7.4 / 8.3,
-// [32, 96, 111, 111] (3136) 59.7 / 36.4.  The reciprocal decode ends at 2^24 pixels.
+// The former take every tensor whose channels make whole lines ([32, 256, 55, 57] 34.9 us, 40.0 in small tiles); the latter, where
+// their loads are aligned, need a workgroup for every compute unit: small tiles / 256 x 64 in us, [12, 72, 44, 44] (192
+// workgroups) 5.1 / 6.2, [64, 64, 28, 28] (256) 7.2 / 6.6.  Where they are not, they pay once the small tiles no longer run
+// all at once (eight to a compute unit), for planes of three small tiles or more, of two where a workgroup's channels are half
+// empty: [512, 64, 13, 13] (1536 small tiles) 9.8 / 12.3, [128, 64, 31, 31] (2048) 12.6 / 12.7, [768, 64, 13, 13] (2304) 16.8 /
+// 14.7, [32, 96, 111, 111] 59.7 / 36.4; [1536, 64, 11, 11] (3072) 18.5 / 19.0, [1536, 32, 11, 11] 15.3 / 11.4; [2048, 32, 7, 7]
+// 6.7 / 14.2.
+// The reciprocal decode ends at 2^24 pixels.
 bool wide_tiles(int64_t n, int64_t hw, int64_t cs) {
-    return hw < (1 << 24) && (cs >= 128 || n * ceil_div(hw, 256) * ceil_div(cs, 64) >= (hw % 4 == 0 ? 256 : 512));
+    if (hw >= (1 << 24)) return false;
+    if (cs >= 128) return true;
+    const int64_t slabs = ceil_div(cs, 64);
+    if (hw % 4 == 0) return n * ceil_div(hw, 256) * slabs >= 256;
+    return hw > (cs <= 32 ? 64 : 128) && n * ceil_div(hw, 64) * slabs > 2048;
 }
 
 template <typename TIn>

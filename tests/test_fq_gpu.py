@@ -221,3 +221,34 @@ def test_more_than_32_bits_of_elements(form, shape):
     print("%s %s: %.0f us whole, %.0f in parts" % (form, shape, whole, parts))
     if h * w % 4 == 0:
         assert whole < 1.3 * parts
+
+
+@pytest.mark.parametrize("shape", [(2048, 32, 7, 7), (1024, 100, 7, 7)])
+def test_many_small_images_are_not_slower_than_their_pixels_in_one_row(shape):
+    """the transposition of planes of HW % 4 != 0 against that of one image of as many pixels a channel, which moves as many bytes
+    and whose tiles have no remainders: measured 1.0 times as long; in tiles of 256 pixels, which a plane fills to a fifth, 1.6 and 2.2"""
+    import torch
+    from dldt_amd import FakeQuantize
+    n, c, h, w = shape
+    cs = -(-c // 16) * 16
+    fq = FakeQuantize(c, 256, -3.0, 3.0, 0.0, 255.0)
+    x = torch.randn(shape, device="cuda")
+    out = torch.empty((n, h, w, cs), dtype=torch.int8, device="cuda")
+    row, row_out = x.view(1, c, 1, n * h * w), out.view(1, 1, n * h * w, cs)
+
+    def micros(call):
+        call()
+        t = []
+        for _ in range(9):
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            e[0].record()
+            for _ in range(50):
+                call()
+            e[1].record()
+            torch.cuda.synchronize()
+            t.append(e[0].elapsed_time(e[1]) * 20)
+        return min(t)
+
+    many, one = micros(lambda: fq.run_q8(x, "u8b", "nhwc", cs, out=out)), micros(lambda: fq.run_q8(row, "u8b", "nhwc", cs, out=row_out))
+    print("%s: %.1f us, one row %.1f" % (shape, many, one))
+    assert many < 1.35 * one
