@@ -1,5 +1,6 @@
-"""A convolution whose f32 values are the graph's result stores them into the caller's [N, C, H, W] buffer itself: every kernel
-variant the layer has and the single launch, against the copy kernel behind the same convolution (HIP_KEEP_F32), bit for bit."""
+"""A convolution whose f32 values are the graph's result stores them into the caller's [N, C, H, W] buffer itself, beside its own
+tensor: every kernel variant the layer has and the single launch, against the copy kernel behind the same convolution
+(HIP_KEEP_F32), bit for bit."""
 import numpy as np
 import pytest
 import torch
@@ -8,6 +9,7 @@ from dldt_amd import HipieError, builders
 
 pytestmark = pytest.mark.gpu
 VARIANTS = [*range(24), 24 + 32]
+ANY, LINES = [*range(6), 10, 11], [12, 14, 15, 22]        # those every layer has, those of 64 input channels and more
 
 
 def _graph(relu, results):
@@ -32,8 +34,9 @@ def _run(plan, x, offset=0):
     return [p.cpu().numpy().view(np.uint32) for p in place]
 
 
-@pytest.mark.parametrize("n,c,hw,oc", [(1, 3, 7, 8), (2, 17, 9, 65), (3, 64, 14, 70), (1, 64, 33, 129), (5, 128, 8, 3), (2, 32, 1, 1)])
-def test_every_variant_stores_the_planes_that_the_copy_stores(tmp_path, n, c, hw, oc):
+@pytest.mark.parametrize("n,c,hw,oc,more", [(1, 3, 7, 8, []), (2, 17, 9, 65, [14]), (3, 64, 14, 70, LINES), (1, 64, 33, 129, LINES),
+                                            (5, 128, 8, 3, [6, 7, 16, 18, 19, 20, 21] + LINES), (2, 32, 1, 1, [14])])
+def test_every_variant_stores_the_planes_that_the_copy_stores(tmp_path, n, c, hw, oc, more):
     g = builders.conv_block(n=n, c=c, hw=hw, oc=oc)[0]
     x = torch.rand((n, c, hw, hw), generator=torch.Generator(device="cuda").manual_seed(1), device="cuda") * 2.55
     kept = g.compile(0, config={"HIP_KEEP_F32": "YES", "HIP_TUNE": "NO"})
@@ -41,19 +44,21 @@ def test_every_variant_stores_the_planes_that_the_copy_stores(tmp_path, n, c, hw
     plan = g.compile(0, config={"HIP_TUNE": "NO"})
     types = [s["type"] for s in plan.steps]
     assert int(plan.step_rt_info(len(types) - 1, "kernels")) == (0 if hw > 1 else 1)
-    ran = 0
+    ran = []
     for v in VARIANTS:
         path = tmp_path / str(v)
-        path.write_text("".join("%d %d\n" % (i, v if t.startswith("Convolution") else -1) for i, t in enumerate(types)))
+        text = "".join("%d %d\n" % (i, v if t.startswith("Convolution") else -1) for i, t in enumerate(types))
+        path.write_text(text)
         try:
             plan = g.compile(0, config={"HIP_TUNE_FILE": str(path), "HIP_SINGLE_LAUNCH": "NO"})
         except HipieError:
             continue                                          # a variant this layer does not have
+        assert path.read_text() == text and [s["variant"] for s in plan.steps if s["type"].startswith("Convolution")] == [v]
         for offset in (0, 1):                                 # (a buffer on a 4-byte boundary only)
             got = _run(plan, x, offset)
             assert np.array_equal(got[0], want[0]), (v, offset)
-        ran += 1
-    assert ran >= 3
+        ran.append(v)
+    assert ran == sorted(ANY + more)
     single = g.compile(0, config={"HIP_TUNE": "NO", "HIP_THROUGHPUT_STREAMS": "1", "HIP_SINGLE_LAUNCH": "256"})
     req = single.create_request()
     ins, outs = req.device_buffers()
@@ -61,6 +66,7 @@ def test_every_variant_stores_the_planes_that_the_copy_stores(tmp_path, n, c, hw
     torch.cuda.synchronize()
     req.infer_device(ins, outs)
     assert np.array_equal(outs[0].cpu().numpy().view(np.uint32), want[0])
+    assert single.metric("SINGLE_LAUNCH_COUNTS") == "1 0"
 
 
 @pytest.mark.parametrize("relu", [False, True])
