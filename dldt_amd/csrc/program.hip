@@ -557,8 +557,6 @@ __device__ __forceinline__ int32_t request_offsets(lds_i32 to, const int32_t* fr
     return from[min(tid, n - 1)];
 }
 
-typedef uint32_t words4 __attribute__((ext_vector_type(4), aligned(4)));
-
 // four consecutive entries of a pixel table, from any of them (the table has room behind its last row)
 typedef uint32_t Words4 __attribute__((ext_vector_type(4), aligned(4)));
 template <int A>
@@ -571,17 +569,16 @@ __device__ __forceinline__ void place_pixels(const uint32_t* pix, int M, int at,
     }
 }
 
-typedef __attribute__((address_space(3))) int32_t* lds_words;
 // pixels r0 .. r0 + R - 1 of the quads of one column: the partial sums of the ks waves that share the tile, and the chain
 template <bool GELU, int A, int B, int R, bool PAIR>
 __device__ __forceinline__ void finish_column(const StepConstants& sc, const ChannelConstants<A>& k, const ChannelConstants<A>& k2, lds_v4i mine, lds_v4i mine2, int ks,
                                               int b, int r0, const Pixels<A>& q, int oc) {
     auto total = [&](lds_v4i from, int32_t (&sum)[A][R]) {
-        const lds_words w = (lds_words)(from + b * A * 64) + r0;
+        const lds_i32 w = (lds_i32)(from + b * A * 64) + r0;
         for (int s = 0; s < ks; ++s)
 #pragma unroll
             for (int a = 0; a < A; ++a) {
-                const lds_words v = w + (s * (A * B) + a) * 256;
+                const lds_i32 v = w + (s * (A * B) + a) * 256;
                 if constexpr (R == 4) {
                     const v4i t = *(lds_v4i)v;
 #pragma unroll
