@@ -45,6 +45,14 @@ struct ProgRef {
 };
 struct ProgPtr { uint32_t lo, hi; };   // a load-time buffer
 
+// a convolution and the depthwise layer behind it: the map between them and the bands it is computed in
+struct ProgExpand {
+    int32_t stride, pad_top, pad_left;        // of the depthwise layer
+    int32_t H, W, OH, OW;                     // of the map between the layers, of the result
+    int32_t rows, bands, all_bands;           // result rows of a band, bands of an image, of all images
+    int32_t patch_w, fill;                    // pixels of a patch row; four bytes of the padding's level
+    float inv_W, inv_OW, inv_bands, inv_all_bands;
+};
 // convolution, weight MatMul (1 x 1 over rows) and depthwise 3 x 3
 struct ProgConv {
     int32_t kind, a, b, ks_shift;     // oc fragments, pixel fragments of a wave's tile; log2 of the waves that share a tile's K
@@ -60,10 +68,14 @@ struct ProgConv {
     float lm1;
     uint32_t off_bytes;                // the level offset in every byte
     float clamp_lo, clamp_hi;
-    // depthwise
-    int32_t stride, group, c4, quads, OH, OW, items;
-    int32_t in_sn, in_sh, in_sw, row_sh, out_sn, out_sh, out_sw, res_sn, res_sh, res_sw;      // (dense: out_sn = bytes between the planes of f32 results that are stored at `res` as well, 0: none)
-    float inv_c4, inv_quads, inv_OH;
+    union {
+        struct {                       // depthwise
+            int32_t stride, group, c4, quads, OH, OW, items;
+            int32_t in_sn, in_sh, in_sw, row_sh, out_sn, out_sh, out_sw, res_sn, res_sh, res_sw;      // (dense: out_sn = bytes between the planes of f32 results that are stored at `res` as well, 0: none)
+            float inv_c4, inv_quads, inv_OH;
+        };
+        ProgExpand expand;             // PK_EXPAND_DW, whose depthwise layer is a descriptor of its own behind this one
+    };
 };
 struct ProgEntry {
     int32_t kind, u8_in, N, C, cs, HW, W;

@@ -859,17 +859,16 @@ __device__ __forceinline__ void dw_items(Ctx& x) {
 // 197 with the layers apart, 182 with this, 170 with a fragment's pixels requested while the one before is multiplied, 168 with
 // the second layer's constants requested behind the wait instead of in front of it (the preparation, 2.2 us, was longer than
 // the barrier; 1.6 now).  What is left of such a step: 1.5 preparation and barrier, 1.2 - 2.3 first layer, 0.6 - 1.0 second.
-// The descriptor's first half is the convolution, with the geometry in the fields that only depthwise layers have
-// (ProgBuilder::expand_depthwise), its second half the depthwise layer.
+// The descriptor's first half is the convolution with the geometry of both (ProgExpand), its second half the depthwise layer.
 constexpr int kExpandSteps = 4;               // K steps of the convolution, held in registers
 
 template <int A>
 __device__ __forceinline__ void expand_depthwise(Ctx& x, lds_ptr lds) {
     // (what only the layers' ends need is read and requested behind the wait, while the first pixels are on their way: before it,
     // it stands between this step and the one before)
-    const int nk = PROG_FIELD(x.words, nk), S = PROG_FIELD(x.words, stride), R = PROG_FIELD(x.words, group), W = PROG_FIELD(x.words, quads), H = PROG_FIELD(x.words, OW);
-    const int bands = PROG_FIELD(x.words, OH), all_bands = PROG_FIELD(x.words, res_sw), PW = PROG_FIELD(x.words, in_sn), pad_t = PROG_FIELD(x.words, in_sh);
-    const int OH = PROG_FIELD(x.words, row_sh);
+    const int nk = PROG_FIELD(x.words, nk), S = PROG_FIELD(x.words, expand.stride), R = PROG_FIELD(x.words, expand.rows), W = PROG_FIELD(x.words, expand.W);
+    const int H = PROG_FIELD(x.words, expand.H), bands = PROG_FIELD(x.words, expand.bands), all_bands = PROG_FIELD(x.words, expand.all_bands);
+    const int PW = PROG_FIELD(x.words, expand.patch_w), pad_t = PROG_FIELD(x.words, expand.pad_top), OH = PROG_FIELD(x.words, expand.OH);
     const bool plain = PROG_FIELD(x.words, koff).hi == 0;
     const lds_i32 staged_to = (lds_i32)(lds + kPartBytes), koff = plain ? (lds_i32)(lds + kPlainAt) : staged_to;
     int32_t staged = 0;
@@ -890,10 +889,10 @@ __device__ __forceinline__ void expand_depthwise(Ctx& x, lds_ptr lds) {
     int unit = t0;
     do {
         int ct, nb, n, band;
-        fast_divmod(unit, all_bands, PROG_FIELD(x.words, inv_c4), ct, nb);
+        fast_divmod(unit, all_bands, PROG_FIELD(x.words, expand.inv_all_bands), ct, nb);
         ct = __builtin_amdgcn_readfirstlane(ct);
         nb = __builtin_amdgcn_readfirstlane(nb);
-        fast_divmod(nb, bands, PROG_FIELD(x.words, inv_OH), n, band);
+        fast_divmod(nb, bands, PROG_FIELD(x.words, expand.inv_bands), n, band);
         n = __builtin_amdgcn_readfirstlane(n);
         band = __builtin_amdgcn_readfirstlane(band);
         const int oy0 = band * R, rows = min(R, OH - oy0), iy0 = oy0 * S - pad_t, patch_rows = (rows - 1) * S + 3;
@@ -910,7 +909,7 @@ __device__ __forceinline__ void expand_depthwise(Ctx& x, lds_ptr lds) {
         int f = x.wave;
         uint32_t off = pix[m0 + min(16 * f + lane16, count - 1)];
         // the patch at the level of the padding (every lane takes part, those behind the end repeat the last piece)
-        const int pieces = patch_rows * PW * A, fill = PROG_FIELD(x.words, res_sh);
+        const int pieces = patch_rows * PW * A, fill = PROG_FIELD(x.words, expand.fill);
         for (int base = 0; base < pieces; base += kProgramThreads) ((lds_v4i)lds)[min(base + x.tid, pieces - 1)] = v4i{fill, fill, fill, fill};
         if (unit == t0) {
             if (!plain) staged_to[min(x.tid, 4 * nk - 1)] = staged;
@@ -928,8 +927,8 @@ __device__ __forceinline__ void expand_depthwise(Ctx& x, lds_ptr lds) {
         request(p);
         off = pix[m0 + min(16 * f + 128 + lane16, count - 1)];
         const StepConstants c1 = step_constants<false>(x, x.words), c2 = step_constants<false>(x, x.words2);
-        const int OCp2 = PROG_FIELD(x.words2, OCp), pad_l = PROG_FIELD(x.words, in_sw);
-        const float inv_W = PROG_FIELD(x.words, inv_quads);
+        const int OCp2 = PROG_FIELD(x.words2, OCp), pad_l = PROG_FIELD(x.words, expand.pad_left);
+        const float inv_W = PROG_FIELD(x.words, expand.inv_W);
         uint4 wr[3];
 #pragma unroll
         for (int r = 0; r < 3; ++r) wr[r] = *reinterpret_cast<const uint4*>(PROG_TABLE_OF(int8_t, x.words2, wgt) + (static_cast<int64_t>(r) * OCp2 + oc4) * 4);
@@ -972,9 +971,9 @@ __device__ __forceinline__ void expand_depthwise(Ctx& x, lds_ptr lds) {
         }
         meet();
         // the depthwise layer: four channels of a pixel per lane
-        const int OW = PROG_FIELD(x.words, res_sn), items = rows * OW * (4 * A);
+        const int OW = PROG_FIELD(x.words, expand.OW), items = rows * OW * (4 * A);
         const int out_sn = PROG_FIELD(x.words2, out_sn), out_sh = PROG_FIELD(x.words2, out_sh), out_sw = PROG_FIELD(x.words2, out_sw);
-        const float inv_OW = PROG_FIELD(x.words, inv_p_tiles);
+        const float inv_OW = PROG_FIELD(x.words, expand.inv_OW);
         for (int base = 0; base < items; base += kProgramThreads) {
             const bool on = base + x.tid < items;
             int oy, ox;
@@ -1864,14 +1863,16 @@ bool ProgBuilder::expand_depthwise(const hipie_conv* first, const hipie_tensor& 
         pix[static_cast<size_t>(m)] = static_cast<uint32_t>(n * a1.in_sn + y * a1.in_sh * a1.conv_sh + xx * a1.in_sw * a1.conv_sw);
     }
     c.pixels = keep(pix.data(), pix.size() * 4);
-    c.stride = S; c.group = best_r; c.quads = W; c.OW = H; c.OH = static_cast<int32_t>(bands); c.res_sw = static_cast<int32_t>(N * bands);
-    c.in_sn = pw; c.in_sh = l2.pad_top; c.in_sw = l2.pad_left; c.row_sh = OH; c.res_sn = OW;
-    c.res_sh = static_cast<int32_t>((static_cast<uint32_t>(fill) & 0xffu) * 0x01010101u);
-    c.inv_c4 = 1.0f / static_cast<float>(N * bands);
-    c.inv_quads = 1.0f / static_cast<float>(W);
-    c.inv_OH = 1.0f / static_cast<float>(bands);
-    c.inv_p_tiles = 1.0f / static_cast<float>(OW);
-    c.out_sn = 0;
+    ProgExpand& e = c.expand;
+    e.stride = S; e.pad_top = l2.pad_top; e.pad_left = l2.pad_left;
+    e.H = H; e.W = W; e.OH = OH; e.OW = OW;
+    e.rows = best_r; e.bands = static_cast<int32_t>(bands); e.all_bands = static_cast<int32_t>(N * bands);
+    e.patch_w = pw;
+    e.fill = static_cast<int32_t>((static_cast<uint32_t>(fill) & 0xffu) * 0x01010101u);
+    e.inv_W = 1.0f / static_cast<float>(W);
+    e.inv_OW = 1.0f / static_cast<float>(OW);
+    e.inv_bands = 1.0f / static_cast<float>(bands);
+    e.inv_all_bands = 1.0f / static_cast<float>(N * bands);
     std::array<int32_t, kProgramStepWords> w{};
     std::memcpy(w.data(), &c, sizeof c);
     std::memcpy(w.data() + kProgramStepWords / 2, &d, sizeof d);
