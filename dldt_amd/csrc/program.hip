@@ -85,7 +85,8 @@ struct Ctx {
     // it gave), and no second addition stands between the last arrival and its readers.  An empty barrier with the wait for a
     // store in front, us with 64 / 128 / 256 workgroups: 1.3 / 1.5 / 1.6; by way of a root counter that the last of an XCD
     // adds to 2.1 / 2.3 / 2.6, all at one counter 1.5 / 2.3 / 4.1, a flag per workgroup that everybody reads 1.4 / 1.6 / 1.8.
-    // (One way between two workgroups, store to sight, takes 0.5 - 0.6 us, the wait for a store 0.36.)
+    // (One way between two workgroups, store to sight, takes 0.5 - 0.6 us, the wait for a store 0.36.)  In the program a step without
+    // work, a copy of no bytes, takes 1.6 / 1.7 / 1.9 us; with the root counter and descriptors by scalar loads 3.6 / 4.1 / 4.2.
     __device__ __forceinline__ void arrive(int next_step) {
         words = load_words(next_step, 0);
         words2 = load_words(next_step, 1);
@@ -1328,8 +1329,8 @@ __device__ __forceinline__ void copy_items(const ProgRows& s, const Ctx& x) {
 // work of `split` waves: each takes every split-th tile of 32 keys - its scores stay in registers, up to kMostTiles of them -
 // and the waves meet for the maximum, for the sum and for the integer sums of the context.  What bounds a step is the chain of
 // exponentials and levels of one wave (1 us for a tile of 32 x 32), so the fewer tiles a wave has the better while there are
-// compute units: one sequence of 128 tokens, 12 heads, took 10.9 us with a wave for 32 queries, 48 waves in all, that
-// multiplied the scores out three times, and takes 4.8 with four.  The sum keeps its order - a lane's keys one behind the
+// compute units: the step of one sequence of 128 tokens, 12 heads, barrier included, took 11.2 us with a wave for 32 queries, 48
+// waves in all, that multiplied the scores out three times, and takes 7.5 with four.  The sum keeps its order - a lane's keys one behind the
 // other - so one wave adds the exponentials of all.  They take K's place in LDS, and the context's partial sums theirs.
 constexpr int kMostTiles = 4;                 // of a wave
 constexpr int kMostSplit = 8;
@@ -1683,11 +1684,11 @@ __global__ void clear_words(uint32_t* p, int n) {
 }
 
 // Tile shape of a convolution step, by the clocks its busiest compute unit takes.  The constants are fitted, not derived: to
-// the time of whole networks with one class of layers at a time in each of the shapes (184 classes of ResNet-50 at batch 1, 3 and
-// 7, MobileNetV2 at 1 and 4, encoders and the convolution block, at 64, 128 and 256 workgroups), so that the choice loses as
-// little as possible against the best shape of every class: summed over a network's classes 1 - 10 % of its time, of which 1 -
-// 8 % is what the best of thirty noisy times lies too low, where the constants before lost 3 - 14 %.  Of the other shapes that were
-// measured (1 x 2, 1 x 4, 2 x 4 of fragments) none is the best of a class by more than the runs differ.
+// the time of whole networks with one class of layers at a time in each of the shapes (ResNet-50, MobileNetV2, encoders and the
+// convolution block, at 64, 128 and 256 workgroups), so that the choice loses as little as possible against the best shape of
+// every class: summed over a network's classes, 167 in all, 0 - 8 % of its time, most of which is what the best of many noisy
+// medians lies too low.  Of the other shapes that were measured (1 x 2, 1 x 4, 2 x 4 of fragments) none is the best of a class by
+// more than the runs differ.
 // What the terms stand for: a load of 1 KB on a unit's path, a matrix instruction, a round trip to memory per filled ring, the
 // f32 chain per value, a store instruction, the partial sums of the waves that share a K in LDS.  Rounds are tiles a wave takes
 // one after another.
@@ -2076,8 +2077,8 @@ bool ProgBuilder::attention(const hipie_attention* att, const void* const (&qkv)
     s.a.mask_inner = 0;
     s.a.mask_outer = proto.S;
     // Waves per 32 queries, by the clocks of a workgroup's round: staging, and the chain of a wave's tiles (from five waves on two
-    // share a SIMD).  Against the best of the four splits the choice costs an encoder of two layers 0 - 1 % of its time (1 to 4
-    // sequences of 32 to 512 keys, 64 and 256 workgroups).
+    // share a SIMD).  Against the best of the four splits the choice costs an encoder of two layers 0 - 2 % of its time (1 to 4
+    // sequences of 32 to 512 keys, 64 and 256 workgroups; 6 % for 32 keys and 256, where one tile leaves nothing to share).
     const int qt = proto.S / 32;
     const int64_t elements = static_cast<int64_t>(batch_outer) * batch;
     double best = 1e30;
@@ -2228,10 +2229,10 @@ void request_leaves(int device) {
 
 // A lone request takes the form that was fastest alone.  Beside others it takes the smaller one, if units are left for it
 // (never more workgroups than compute units, so that all of them find a place), and else the steps, whose kernels share the
-// device.  ResNet-50, batch 1, us a request with 2 and 4 in flight: 256 workgroups one behind the other 322 and 321, steps 252
-// and 245, 64 workgroups side by side 186 and 177 (alone: 294, 488, 352).  With more than twice as many requests as find a
-// place the ones by steps wait for the others: batch 3 with 128 workgroups, 4 in flight: 244, steps 261; 6 in flight: 207, steps
-// 179 (batch 1 with 64 workgroups, 6 in flight: 135, steps 166).
+// device.  ResNet-50, batch 1, us a request with 2 and 4 in flight: steps 251 and 167, 64 workgroups side by side 148 and 96
+// (alone: steps 492, 64 workgroups 284, 256 238).  With more than twice as many requests as find a place the ones by steps wait
+// for the others: batch 3 with 128 workgroups, 4 in flight: 182, steps 182; 6 in flight: 221, steps 173 (batch 1 with 64
+// workgroups, 6 in flight: 113, steps 163).
 const ProgramForm* Program::choose(int together) {
     const ProgramForm* f = together > 1 ? shared.get() : lone.get();
     if (!f || (lone != shared && together > 1 && together * f->workgroups > 2 * units)) return nullptr;
