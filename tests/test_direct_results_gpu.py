@@ -23,7 +23,8 @@ def _graph(relu, results):
     return q.g
 
 
-def _run(plan, x, offset=0):
+def _run(plan, x, offset=0, value=None):
+    """the outputs' bits; `value`: a node whose tensor holds the first one's values as well"""
     req = plan.create_request()
     ins, outs = req.device_buffers()
     ins[0].copy_(x)
@@ -31,6 +32,8 @@ def _run(plan, x, offset=0):
     torch.cuda.synchronize()
     req.enqueue(ins, place)
     torch.cuda.synchronize()
+    if value is not None:
+        assert np.array_equal(req.tensor(value).reshape(-1) + np.float32(0), place[0].cpu().numpy().reshape(-1))
     return [p.cpu().numpy().view(np.uint32) for p in place]
 
 
@@ -55,7 +58,7 @@ def test_every_variant_stores_the_planes_that_the_copy_stores(tmp_path, n, c, hw
             continue                                          # a variant this layer does not have
         assert path.read_text() == text and [s["variant"] for s in plan.steps if s["type"].startswith("Convolution")] == [v]
         for offset in (0, 1):                                 # (a buffer on a 4-byte boundary only)
-            got = _run(plan, x, offset)
+            got = _run(plan, x, offset, g.nodes[-1]["inputs"][0])
             assert np.array_equal(got[0], want[0]), (v, offset)
         ran.append(v)
     assert ran == sorted(ANY + more)
