@@ -3271,6 +3271,28 @@ bool to_two_spatial_dimensions(const hipie_graph& g, hipie_graph& out) {
     return true;
 }
 
+// what a tuning file holds: the variant of every step, and the sizes of the single-launch form where these were measured
+struct StoredChoices {
+    std::map<int, int> variants;
+    FormChoice forms;
+};
+StoredChoices read_choices(const std::string& file) {
+    StoredChoices c;
+    FILE* f = file.empty() ? nullptr : std::fopen(file.c_str(), "r");
+    if (!f) return c;
+    int idx = 0, var = 0, found = 0;
+    while (std::fscanf(f, "%d %d", &idx, &var) == 2)
+        if (idx == -1 || idx == -2) {
+            (idx == -1 ? c.forms.lone : c.forms.shared) = var;
+            found |= -idx;
+        } else if (idx >= 0) {
+            c.variants.emplace(idx, var);
+        }
+    std::fclose(f);
+    c.forms.known = found == 3;
+    return c;
+}
+
 std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const std::vector<int>* preset,
                                          const PlanConfig& cfg = PlanConfig::from_environment(), PlanPrepared* prepared = nullptr,
                                          FormChoice forms = FormChoice()) {
@@ -3394,9 +3416,10 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
             --i;
         }
     // A convolution whose result only the next depthwise layer reads: one step, and one launch where that is faster
-    // (values that are kept stay two steps, and so do layers that nothing measures: choices of a plan that had them apart,
-    // plans without a device, plans that are not tuned)
-    const bool measured_pairs = device >= 0 && (preset ? preset->size() != plan->steps.size() : cfg.tune);
+    // (values that are kept stay two steps, and so do layers that nothing measures: choices, of an exported plan or in a file, of
+    // a plan that had them apart, plans without a device, plans that are not tuned)
+    const StoredChoices stored = device >= 0 && cfg.tune ? read_choices(cfg.tune_file) : StoredChoices{};
+    const bool measured_pairs = device >= 0 && (preset ? preset->size() != plan->steps.size() : cfg.tune && stored.variants.size() != plan->steps.size());
     if (!cfg.keep_f32 && (cfg.fuse_convs == 2 || (cfg.fuse_convs == 1 && measured_pairs)))
         for (size_t i = 0; i + 1 < plan->steps.size(); ++i) {
             auto* a = dynamic_cast<ConvStep*>(plan->steps[i].get());
@@ -3471,30 +3494,17 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
         cache = cfg.tune_file.empty() ? nullptr : cfg.tune_file.c_str();
         bool loaded = false;
         if (cache) {
-            if (FILE* f = std::fopen(cache, "r")) {
-                std::vector<int> v(plan->steps.size(), -2);
-                size_t n = 0;
-                int idx = 0, var = 0;
-                FormChoice stored;
-                int found = 0;
-                while (std::fscanf(f, "%d %d", &idx, &var) == 2)
-                    if (idx == -1 || idx == -2) {
-                        (idx == -1 ? stored.lone : stored.shared) = var;
-                        found |= -idx;
-                    } else if (idx >= 0 && static_cast<size_t>(idx) < v.size() && v[idx] == -2) {
-                        v[idx] = var;
-                        ++n;
-                    }
-                std::fclose(f);
-                bool match = n == v.size();
-                for (size_t i = 0; match && i < v.size(); ++i)
-                    match = (v[i] < 0) == (plan->steps[i]->variant() < 0);
-                if (match) {
-                    for (size_t i = 0; i < v.size(); ++i) plan->steps[i]->set_variant(v[i]);
-                    loaded = true;
-                    stored.known = found == 3;
-                    if (stored.known && stored.valid()) forms = stored;
-                }
+            bool match = stored.variants.size() == plan->steps.size();      // (a file of a plan with other steps is of no use)
+            std::vector<int> v(plan->steps.size());
+            for (size_t i = 0; match && i < v.size(); ++i) {
+                const auto at = stored.variants.find(static_cast<int>(i));
+                match = at != stored.variants.end() && (at->second < 0) == (plan->steps[i]->variant() < 0);
+                if (match) v[i] = at->second;
+            }
+            if (match) {
+                for (size_t i = 0; i < v.size(); ++i) plan->steps[i]->set_variant(v[i]);
+                loaded = true;
+                if (stored.forms.known && stored.forms.valid()) forms = stored.forms;
             }
         }
         if (!loaded) {

@@ -130,3 +130,19 @@ def test_layers_that_run_apart_are_two_steps(apart, single, tmp_path):
                         r.tensor(mids[k])
     assert np.abs(results[0]).max() > 0
     assert all(np.array_equal(results[0].view(np.uint8), v.view(np.uint8)) for v in results[1:])
+
+
+def test_a_file_of_choices_apart_is_taken_as_it_is(tmp_path):
+    """a tuning file from before the two layers were ever one step, as those of HIP_FUSE_CONVOLUTIONS=NO are: not measured anew"""
+    g, mids = _two_blocks()
+    path = tmp_path / "choices"
+    config = {"HIP_THROUGHPUT_STREAMS": "1", "HIP_SINGLE_LAUNCH": "NO", "HIP_TUNE": "YES", "HIP_TUNE_FILE": str(path)}
+    apart = g.compile(0, config=dict(config, HIP_FUSE_CONVOLUTIONS="NO"))
+    text = path.read_text()
+    assert len(text.splitlines()) == len(apart.steps)
+    plan = g.compile(0, config=config)
+    assert path.read_text() == text and [s["variant"] for s in plan.steps] == [s["variant"] for s in apart.steps]
+    # a file with the choices of other steps is not
+    path.write_text(text + "%d 0\n" % len(apart.steps))
+    g.compile(0, config=config)
+    assert path.read_text() != text + "%d 0\n" % len(apart.steps)
