@@ -211,8 +211,11 @@ constexpr size_t kProgramControlBytes = 2048, kProgramControlBlocks = 2;
 // `launch`: how many launches used this control block before; io: the call's input and output buffers in order
 void launch_program(const Program& p, const ProgramForm& f, uint8_t* arena, void* const* io, int n_io, uint32_t* control, uint32_t launch, int slot,
                     hipStream_t s);
-// what the last launch of a slot reported: 0 done; anything else: it did not run to its end, and `control` has been
-// cleared on the stream (the caller runs the inference by steps and counts its launches from zero again)
+// looks at the slot's word until its launch is complete: true, and every result is in memory (its stream may still be draining).
+// false: it was given up, or takes long; the stream is to be waited for
+bool report_done(const Program& p, int slot);
+// the stream of a slot's last launch has drained, or report_done was true: true if it did not run to its end, and `control` has
+// been cleared on the stream (the caller runs the inference by steps and counts its launches from zero again)
 bool program_failed(const Program& p, int slot, uint32_t* control, hipStream_t s);
 
 }  // namespace hipie

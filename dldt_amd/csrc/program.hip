@@ -14,6 +14,8 @@
 // step is the same sequence of f32 operations as in the per-step kernels, so the results are the same bits.
 #include "program.h"
 
+#include <chrono>
+
 #include "div2.h"
 
 struct hipie_fq;
@@ -31,6 +33,8 @@ constexpr int kLdsBytes = kPlainAt + kMaxPieces * 4;
 // waits for the same units) does not let go, and the steps need less than that beside it.
 constexpr uint32_t kRollCallTicks = 100000, kMaxRollCallTicks = 10000000;
 constexpr uint64_t kBarrierTicks = 200000000;
+// what a launch tells the host in its slot's word, 0 before it
+constexpr uint32_t kReportCancelled = 1, kReportLost = 2, kReportDone = 3;
 
 typedef __attribute__((address_space(3))) int8_t* lds_ptr;
 typedef __attribute__((address_space(3))) v4i* lds_v4i;
@@ -57,6 +61,8 @@ typedef uint8_t* GlobalBytes;
 constexpr int kXcdWords = 32;
 constexpr uint32_t kGivenUp = 1u << 26;      // added to a counter that was not complete when the roll call's time was up (a launch counts far less)
 
+__device__ __forceinline__ int lane_index() { return static_cast<int>(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u))); }
+
 struct Ctx {
     int rank, n_wg, wg_shift;                // neighbouring ranks share an XCD; n_wg = 1 << wg_shift
     int tid, lane, wave;
@@ -66,7 +72,6 @@ struct Ctx {
     uint32_t bases;                          // lanes 2 b, 2 b + 1: where operands of base b are (ProgArgs::bases)
     uint32_t *xcds, *own;                    // the eight counters, the one this workgroup counts at
     uint32_t target;                         // what each of them holds when the barrier that comes next is complete
-    uint32_t* report;
     bool started, dead;                      // between the roll call and the first step's wait; after a wait that was given up
     lds_i32 flag;
 
@@ -107,7 +112,7 @@ struct Ctx {
                 if (t0 == 0) t0 = wall_clock64();
                 if (wall_clock64() - t0 > kBarrierTicks) {
                     if (lane == 0) {
-                        __hip_atomic_store(report, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                        tell(kReportLost);
                         flag[0] = 0;
                     }
                     break;
@@ -118,6 +123,21 @@ struct Ctx {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
+    }
+    // Every workgroup has arrived behind the last step: the first one tells the host in the page-locked word that it looks at
+    // (report_done).  All results were stored with device scope and acknowledged, so they are in memory.
+    __device__ __forceinline__ void finish() {
+        if (rank != 0) return;
+        lane = lane_index();
+        wait();
+        if (wave == 0 && lane == 0 && flag[0] != 0) tell(kReportDone);
+    }
+    __device__ __forceinline__ void tell(uint32_t what) const {
+#if defined(__HIP_DEVICE_COMPILE__)
+        typedef uint32_t* Word;
+        const Word w = *(const __attribute__((address_space(4))) Word*)((const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(ProgArgs, report));
+        __hip_atomic_store(w, what, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+#endif
     }
     // Everybody is resident, or nobody starts.  A workgroup whose time is up adds kGivenUp to a counter that it has seen short
     // and that has not moved since: from then on that counter never holds what completes the roll call.  So "all eight have
@@ -142,7 +162,7 @@ struct Ctx {
                 }
             }
             if (lane == 0) {
-                if (!all) __hip_atomic_store(report, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                if (!all) tell(kReportCancelled);
                 flag[0] = all ? 1 : 0;
             }
         }
@@ -1151,7 +1171,7 @@ __device__ __forceinline__ void avg_pool_items(const ProgPool& s, const Ctx& x) 
     }
 }
 
-// (the caller's output buffer: nothing in the launch reads it)
+// (the caller's output buffer, which can be larger than a buffer descriptor reaches: nothing in the launch reads it, the host does)
 template <typename TIn>
 __device__ __forceinline__ void exit_items(const ProgExit& s, const Ctx& x) {
     const ExitArgs& a = s.a;
@@ -1162,8 +1182,8 @@ __device__ __forceinline__ void exit_items(const ProgExit& s, const Ctx& x) {
         if (a.sub) v = v - a.sub[c];
         if (a.mul) v = v * a.mul[c];
         const int64_t o = (static_cast<int64_t>(n) * a.C + c) * a.HW + p;
-        if (a.out_u8) out[o] = static_cast<uint8_t>(static_cast<int>(v));
-        else reinterpret_cast<float*>(out)[o] = v;
+        if (a.out_u8) __hip_atomic_store(out + o, static_cast<uint8_t>(static_cast<int>(v)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else __hip_atomic_store(reinterpret_cast<float*>(out) + o, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
     if (a.HW >= 16) {                        // lanes along the pixels, four channels each (a pixel's channels are padded to four)
         const int waves = (a.HW + 63) / 64, cg = (a.C + 3) / 4, items = a.N * cg * waves;
@@ -1549,12 +1569,10 @@ __device__ __forceinline__ void attention_units(const ProgAttention& s, Ctx& x, 
     } while (u < s.units);
 }
 
-__device__ __forceinline__ int lane_index() { return static_cast<int>(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u))); }
-
 // ---- the program ------------------------------------------------------------------------------------------------------------
 // Three kernels, for networks over feature maps, for encoders, and for graphs with steps of both: every kind of step adds to the
-// registers of all others.  The 4 x 4 tiles ask for 250 and more vector registers, none is spilled to memory; 460 - 510 scalar
-// registers of the many step kinds are kept in lanes of vector registers.  The kernel with all kinds has no registers left for
+// registers of all others.  The 4 x 4 tiles ask for 250 and more vector registers, none is spilled to memory; 437, 422 and 696
+// scalar registers of the many step kinds are kept in lanes of vector registers.  The kernel with all kinds has no registers left for
 // 4 x 4 tiles (with them it spills); its convolutions take smaller ones (an encoder layer of 96 tokens beside a ResNet-50 of width
 // 16 at 64 x 64: 244 us, 467 by steps; beside a MobileNetV2 of 2 x 96 x 96 208 and 512).  A new step kind belongs into a kernel of its own where it
 // needs more than they have.
@@ -1577,8 +1595,7 @@ __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgA
     x.rank = static_cast<int>(blockIdx.x % 8) * (x.n_wg / 8) + static_cast<int>(blockIdx.x / 8);
     x.xcds = g.control;
     x.own = x.xcds + kXcdWords * (blockIdx.x % 8);
-    x.target = (g.launch * static_cast<uint32_t>(g.n_steps) + 1) * static_cast<uint32_t>(x.n_wg / 8);      // a launch: the roll call and n_steps - 1 barriers
-    x.report = g.report;
+    x.target = (g.launch * static_cast<uint32_t>(g.n_steps + 1) + 1) * static_cast<uint32_t>(x.n_wg / 8);      // a launch: the roll call and n_steps arrivals
     x.started = true;
     x.dead = false;
     x.flag = flag;
@@ -1649,16 +1666,17 @@ __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgA
             } else if (kind == PK_MAXPOOL) max_pool_items(unpack<ProgPool>(words), x);
             else if (!ROWS || kind == PK_AVGPOOL) avg_pool_items(unpack<ProgPool>(words), x);
         }
-        if (step + 1 == g.n_steps) break;
+        const int next = min(step + 1, g.n_steps - 1);       // (behind the last step nothing is prepared)
         {   // the next step's descriptor into the scalar cache: its eight lines asked for together, beside the stores' way to memory
             // (one behind the other they took 0.7 us of every step)
-            const StepPtr n = step_ptr(g.steps, step + 1);
+            const StepPtr n = step_ptr(g.steps, next);
             static_assert(kProgramStepWords == 128, "eight lines of 64 bytes");
             asm volatile("" ::"s"(n[0]), "s"(n[16]), "s"(n[32]), "s"(n[48]), "s"(n[64]), "s"(n[80]), "s"(n[96]), "s"(n[112]));
         }
-        x.arrive(step + 1);
+        x.arrive(next);
         if (x.dead) return;
     }
+    x.finish();
 }
 
 // constant weights [OCp][Kp] in the per-layer kernels' row order -> fragments of the tile kernel: for every tile of 16 A
@@ -2273,8 +2291,24 @@ void launch_program(const Program& p, const ProgramForm& f, uint8_t* arena, void
     HIPIE_CHECK_HIP(hipGetLastError());
 }
 
+// The word is there 4.4 us before hipStreamSynchronize returns (a kernel of 64 workgroups that takes 10 us, launch to answer: 17.4 and
+// 21.8 us), which waits for the kernel's end, its caches' write-back and a signal.  A launch that takes longer than kMostPolled is
+// left to the runtime: the core has better things to do, and errors of the device are found there.
+bool report_done(const Program& p, int slot) {
+    constexpr auto kMostPolled = std::chrono::milliseconds(5);
+    const uint32_t* word = p.report + 16 * slot;
+    const auto t0 = std::chrono::steady_clock::now();
+    for (uint32_t n = 1;; ++n) {
+        const uint32_t v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+        if (v != 0) return v == kReportDone;
+        if (n % 256 == 0 && std::chrono::steady_clock::now() - t0 > kMostPolled) return false;
+        __builtin_ia32_pause();
+    }
+}
+
 bool program_failed(const Program& p, int slot, uint32_t* control, hipStream_t s) {
-    if (__atomic_load_n(p.report + 16 * slot, __ATOMIC_ACQUIRE) == 0) return false;
+    const uint32_t v = __atomic_load_n(p.report + 16 * slot, __ATOMIC_ACQUIRE);
+    if (v == 0 || v == kReportDone) return false;
     hipLaunchKernelGGL(clear_words, dim3(1), dim3(256), 0, s, control, static_cast<int>(kProgramControlBytes / 4));
     HIPIE_CHECK_HIP(hipGetLastError());
     return true;

@@ -96,6 +96,38 @@ def test_single_launch_equals_steps(name):
             assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
 
 
+@pytest.mark.parametrize("name", ["block_1x3x7", "block_3x64x14", "resnet_3_u8", "mobilenet_1x160", "encoder_3x96", "encoder_and_resnet"])
+def test_results_are_there_when_the_call_returns(name):
+    """The call returns by the launch's own word, before its stream has drained: results are read on another stream at once, by a
+    kernel and by a copy to the host, and the request is destroyed or its next inference follows."""
+    g = GRAPHS[name]()
+    steps, single = _compile(g, "NO"), _compile(g, "64")
+    want = [_infer(steps.create_request(), seed) for seed in range(4)]
+    other = torch.cuda.Stream()
+    b = single.create_request()
+    buffers = []
+    for seed in range(4):
+        ins, outs = b.device_buffers()
+        _fill(ins, seed)
+        buffers.append((ins, outs))
+    torch.cuda.synchronize()
+    for turn in range(60):
+        ins, outs = buffers[turn % 4]
+        for o in outs:
+            o.fill_(0 if o.dtype == torch.uint8 else float("nan"))
+        torch.cuda.synchronize()
+        b.infer_device(ins, outs)
+        with torch.cuda.stream(other):
+            seen = [o.clone() if turn % 2 else o.cpu() for o in outs]
+        if turn % 5 == 4:
+            del b
+            b = single.create_request()
+        other.synchronize()
+        for x, y in zip(want[turn % 4], seen):
+            assert np.array_equal(x.view(np.uint8), y.cpu().numpy().view(np.uint8)), turn
+    assert single.metric("SINGLE_LAUNCH_COUNTS") == "60 0"
+
+
 # Together these choose every tile instance of the kernels (fragments of 16 channels x fragments of 16 pixels) and every way a
 # tile's waves share its chain
 @pytest.mark.parametrize("workgroups", [64, 128, 256])
