@@ -91,7 +91,7 @@ struct ConvLaunch {
     int kh, kw, dil_h, dil_w, pad_top, pad_left;
 };
 bool conv_launch_arguments(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out, ConvLaunch& l);
-// the same with the f32 results stored at `planes` as well, channel by channel, [N, C, H, W] dense.  Layers that take it:
+// the same with the f32 results channel by channel, [N, C, H, W] dense at `planes`; `out` says their shape.  Layers that take it:
 // dense convolutions without a residual
 bool conv_takes_planes(const hipie_conv* c, int64_t n, int64_t oh, int64_t ow);
 int conv_run_planes(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor& out, void* planes, hipStream_t s);

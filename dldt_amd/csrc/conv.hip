@@ -2496,11 +2496,12 @@ int hipie_conv_run_static(const hipie_conv* c, const hipie_tensor* in, const hip
 }  // extern "C"
 
 void hipie::planes_arguments(ConvArgs& a, void* planes) {
-    a.planes = static_cast<float*>(planes);
-    a.res_sn = a.OC * a.OHOW;
-    a.res_sh = a.OW;
-    a.res_sw = 1;
-    a.flat_out = a.flat_out && (a.OC == 1 || a.M == a.OHOW);      // (one image, or one channel: pixel m sits at m)
+    a.out = planes;
+    a.out_plane = a.OHOW;
+    a.out_sn = a.OC * a.OHOW;
+    a.out_sh = a.OW;
+    a.out_sw = 1;
+    a.flat_out = a.OC == 1 || a.M == a.OHOW;      // (one image, or one channel: pixel m sits at m)
 }
 
 bool hipie::conv_takes_planes(const hipie_conv* c, int64_t n, int64_t oh, int64_t ow) {

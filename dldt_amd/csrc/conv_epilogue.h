@@ -481,20 +481,6 @@ __device__ __forceinline__ void epilogue(const ConvArgs& a, const v16i (&acc)[2]
                 v[pb][j] = x;
             }
         }
-        if (kPlanes && a.planes) {
-            // a graph's result goes into the caller's layout as well: the 32 lanes of a half-wave hold a channel's values of 32
-            // neighbouring pixels, so every store is 128 contiguous bytes.  (+ 0: as a result that is copied out, never a negative zero)
-            // A convolution of 12 x 72 x 45 x 45 to 100 channels behind its FakeQuantize, queued: 14.3 us with a kernel that copies the
-            // result, 11.4 with these stores.
-#pragma unroll
-            for (int pb = 0; pb < 2; ++pb) {
-                if (staged_out && pb != pass) continue;
-                float* const o = a.planes + res_off[pb] - oc_lane;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (valid[pb] && oc_lane + 4 * e4 + j < a.OC) o[static_cast<int64_t>(oc_lane + 4 * e4 + j) * a.OHOW] = v[pb][j] + 0.f;
-            }
-        }
         if (fl & CF_OUT_FQ) {
             // the eight values of a group advance together, operation by operation, and the two dwords are packed in
             // turn: a wave that runs alone on its SIMD has nothing but its own independent instructions to put
@@ -549,6 +535,19 @@ __device__ __forceinline__ void epilogue(const ConvArgs& a, const v16i (&acc)[2]
             asm volatile("" : "+v"(packed[0]), "+v"(packed[1]) : : "memory");
             out_dw[0][e4] = packed[0];
             out_dw[1][e4] = packed[1];
+        } else if (kPlanes && a.out_plane) {
+            // a graph's result in the caller's layout: the 32 lanes of a half-wave hold a channel's values of 32 neighbouring
+            // pixels, so every store is 128 contiguous bytes.  (+ 0: as a result that is copied out, never a negative zero)
+            // A convolution of 12 x 72 x 45 x 45 to 100 channels behind its FakeQuantize, queued: 14.3 us with a kernel that copies the
+            // result, 11.4 with these stores beside those of its tensor, 8.6 with these alone.
+#pragma unroll
+            for (int pb = 0; pb < 2; ++pb) {
+                if (staged_out && pb != pass) continue;
+                float* const o = static_cast<float*>(a.out) + out_off[pb] - oc_lane;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (valid[pb] && oc_lane + 4 * e4 + j < a.OC) o[static_cast<int64_t>(oc_lane + 4 * e4 + j) * a.out_plane] = v[pb][j] + 0.f;
+            }
         } else if (staged_out) {
             typedef float v4f __attribute__((ext_vector_type(4)));
             const int row = lane_id & 31, c = ((lane_id >> 5) * 8 + e4) ^ (row & 15);
@@ -566,7 +565,7 @@ __device__ __forceinline__ void epilogue(const ConvArgs& a, const v16i (&acc)[2]
         }
         cur = nxt;
     }
-    if (staged_out) {
+    if (staged_out && !(kPlanes && a.out_plane)) {
         // LDS operations of one wave complete in order; the waits only keep the compiler from moving
         // accesses across the two phases
         typedef float v4f __attribute__((ext_vector_type(4)));

@@ -87,7 +87,6 @@ struct ConvArgs {
     const int8_t* wgt;    // packed [OCp][Kp]
     void* out;            // element (0,0,0,0) of the output tensor
     const void* res;      // residual tensor or nullptr
-    float* planes;        // f32 results are stored here as well, [N, C, H, W] dense; the residual strides are this buffer's (or nullptr)
     const int32_t* koff;  // [Kp/16] byte offset of every 16-byte K piece relative to the window origin
     // per-channel tables, each [OCp]
     const int32_t* corr;  // 128 * sum_k w[oc][k] for U8B inputs (0 for I8)
@@ -108,6 +107,7 @@ struct ConvArgs {
     int32_t conv_sh, conv_sw;        // convolution strides
     int32_t in_origin;               // -(pad_top * in_sh + pad_left * in_sw)
     int32_t out_sn, out_sh, out_sw;  // output strides in elements
+    int32_t out_plane;               // f32 results stored channel by channel (NCHW, out_sw = 1): elements from one plane to the next; 0: channels innermost
     int32_t res_sn, res_sh, res_sw;  // residual strides in elements
     int32_t OC, OCp;
     int32_t nk;                      // Kp / 64

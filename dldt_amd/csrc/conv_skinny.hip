@@ -75,7 +75,7 @@ __global__ __launch_bounds__(256) void conv_skinny_kernel(const ConvArgs a) {
     for (int q = 0; q < P / 4; ++q) {
         const int p = wave + 4 * q, m = m0 + p;
         const int sum = part[0][p][lane] + part[1][p][lane] + part[2][p][lane] + part[3][p][lane] + a.corr[oc];
-        if (m >= a.M || oc >= a.out_sw) continue;      // (out_sw: the output pixel's stride = its padded channels)
+        if (m >= a.M || oc >= (a.out_plane ? a.OC : a.out_sw)) continue;      // (out_sw: the output pixel's stride = its padded channels)
         const PixelCoord c = decode_pixel(a, m);
         const int64_t off = static_cast<int64_t>(c.n) * a.out_sn + c.oh * a.out_sh + c.ow * a.out_sw + oc;
         if (fl & CF_OUT_I32) {
@@ -86,8 +86,8 @@ __global__ __launch_bounds__(256) void conv_skinny_kernel(const ConvArgs a) {
         if (fl & CF_BIAS) v = v + a.bias[oc];
         if (fl & CF_SCALE) v = v * a.scale[oc];
         if (fl & CF_RELU) v = v > 0.f ? v : 0.f;
-        static_cast<float*>(a.out)[off] = v;
-        if (a.planes && oc < a.OC) a.planes[static_cast<int64_t>(c.n) * a.res_sn + c.oh * a.res_sh + c.ow + static_cast<int64_t>(oc) * a.OHOW] = v + 0.f;
+        if (a.out_plane) static_cast<float*>(a.out)[off + static_cast<int64_t>(oc) * (a.out_plane - 1)] = v + 0.f;
+        else static_cast<float*>(a.out)[off] = v;
     }
 }
 

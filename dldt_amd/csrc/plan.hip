@@ -204,8 +204,8 @@ struct ConvStep : Step {
     // run inside this step's kernel when the fused form applies, else right before it
     std::unique_ptr<ConvStep> shortcut;
     bool fused = false;
-    // the graph's result that this step's f32 output is, and nothing else reads: it goes into the caller's buffer as well as into
-    // its tensor, where hipie_request_tensor finds it (-1: none)
+    // the graph's result that this step's f32 output is, and nothing else reads: it goes straight into the caller's buffer, and into
+    // its tensor where somebody looks at that (`fill`; -1: none)
     int result = -1;
     // ... which the layer's kernels can write; the values of single pixels ([N, C]) are a row each either way, their copy is no
     // transposition and goes away in the single launch only
@@ -267,6 +267,11 @@ struct ConvStep : Step {
             else if (res_param >= 0) r = input_residual(o, inputs[res_param]);
         }
         check_status(hipie_conv_run(conv, &i, (fused || res >= 0 || res_param >= 0) ? &r : nullptr, &o, s), name.c_str());
+    }
+    // the tensor of a result that the last inference stored in the caller's buffer only: the layer once more, over the same operand
+    void fill(uint8_t* arena, const std::vector<TensorInfo>& tensors, hipStream_t s) const {
+        const hipie_tensor i = tensors[in].desc(arena), o = tensors[out].desc(arena);
+        check_status(hipie_conv_run(conv, &i, nullptr, &o, s), name.c_str());
     }
     bool program(ProgBuilder& b, const std::vector<TensorInfo>& tensors, void* const* inputs, void* const* outputs) const override {
         const hipie_tensor i = tensors[in].desc(b.fake_arena()), o = tensors[out].desc(b.fake_arena());
@@ -2974,8 +2979,8 @@ struct Planner {
         st->out_u8 = x.kind == VK_TENSOR && tensors[x.tensor].esize() == 1;
         for (size_t i = 0; i < g.results.size(); ++i)
             if (g.results[i] == id) st->result_index = static_cast<int>(i);
-        // an f32 result that only the caller reads: its producer stores it there, in the caller's layout, beside its own tensor
-        // (with HIPIE_KEEP_F32 the tensor is copied)
+        // an f32 result that only the caller reads: its producer stores it there, in the caller's layout (with HIPIE_KEEP_F32 it
+        // stores its tensor, which is copied)
         if (x.kind == VK_TENSOR && tensors[x.tensor].dtype == HIPIE_F32 && N(n.in[0]).users.size() == 1 && !keep_f32)
             for (auto& step : steps)
                 if (auto* conv = dynamic_cast<ConvStep*>(step.get()); conv && conv->out == x.tensor && conv->out_node == n.in[0]) {
@@ -3026,6 +3031,7 @@ struct hipie_plan {
     std::shared_ptr<Program> program;
     std::string single_launch_refused;
     FormChoice forms;                        // what was measured of it, for an export
+    std::vector<const ConvStep*> result_writers;      // steps that store a result in the caller's buffer and not in its tensor
 };
 
 struct hipie_request {
@@ -3056,6 +3062,15 @@ struct hipie_request {
     bool entered = false;                    // counted among the device's requests in flight
     bool stream_taken = false;               // hipie_request_stream gave the stream out: its work is complete in stream order
     std::vector<void*> run_in, run_out, host_out;
+    // Results whose tensors were looked at (hipie_request_tensor): from then on every inference fills these, so that a tensor
+    // that is held goes on showing the last one's values
+    mutable std::mutex looked_lock;
+    mutable std::vector<const ConvStep*> looked;
+    bool inferred = false;
+    bool looked_at() const {
+        std::lock_guard<std::mutex> g(looked_lock);
+        return !looked.empty();
+    }
     // the stream has drained
     void leave_form() {
         if (form) program->leave(form);
@@ -3093,6 +3108,23 @@ __global__ void fill_bytes(uint8_t* p, int64_t n, uint8_t v) {
     for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = v;
 }
 
+bool is_capturing(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    HIPIE_CHECK_HIP(hipStreamIsCapturing(s, &status));
+    return status != hipStreamCaptureStatusNone;
+}
+
+// The tensors of results that were looked at, behind the inference that was queued.  A captured inference runs again where the
+// host does not see it: it fills all of them.
+void fill_results(const hipie_request* r, bool single_launch) {
+    const hipie_plan& p = *r->plan;
+    if (p.result_writers.empty()) return;
+    const bool all = !single_launch && is_capturing(r->stream);
+    std::lock_guard<std::mutex> g(r->looked_lock);
+    for (const ConvStep* w : all ? p.result_writers : r->looked)
+        if (single_launch ? w->writes_result : w->direct) w->fill(r->arena.as<uint8_t>(), p.tensors, r->stream);
+}
+
 void enqueue(hipie_request* r, void* const* in, void* const* out) {
     const hipie_plan& p = *r->plan;
     uint8_t* arena = r->arena.as<uint8_t>();
@@ -3101,6 +3133,8 @@ void enqueue(hipie_request* r, void* const* in, void* const* out) {
         p.steps[i]->run(arena, p.tensors, in, out, r->stream);
     }
     if (r->perf) HIPIE_CHECK_HIP(hipEventRecord(r->events[p.steps.size()], r->stream));
+    fill_results(r, false);
+    r->inferred = true;
 }
 
 // by the plan's single-launch form
@@ -3112,6 +3146,8 @@ void enqueue_program(hipie_request* r, void* const* in, void* const* out) {
     const int block = r->form == r->program->lone.get() ? 0 : 1;
     launch_program(*r->program, *r->form, r->arena.as<uint8_t>(), io, static_cast<int>(p.inputs.size() + p.outputs.size()),
                    r->control + block * (kProgramControlBytes / 4), r->launches[block]++, r->slot, r->stream);
+    fill_results(r, true);
+    r->inferred = true;
 }
 
 // The stream has drained.  Where a single launch gave up (its workgroups did not come together) the inference is queued
@@ -3578,6 +3614,8 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
             st.sources = src;
         }
     }
+    for (const auto& st : plan->steps)
+        if (const auto* c = dynamic_cast<const ConvStep*>(st.get()); c && c->writes_result) plan->result_writers.push_back(c);
     // (a plan that was exported with its kernels chosen and no form measured had none)
     const bool measured = forms.known || (forms.imported && preset_used);
     if (device >= 0 && (cfg.single_launch >= 2 || (cfg.single_launch == 1 && cfg.streams == 1 && (measured ? forms.known : cfg.tune)))) {
@@ -4215,7 +4253,7 @@ int hipie_request_wait_for(hipie_request* r, int64_t timeout_ms) {
             do {
                 if (timeout_ms < 0) {
                     // (a single launch into the caller's device buffers says itself when they are written: nothing follows it)
-                    if (!r->form || !r->host_out.empty() || !report_done(*r->program, r->slot)) HIPIE_CHECK_HIP(hipStreamSynchronize(r->stream));
+                    if (!r->form || !r->host_out.empty() || r->looked_at() || !report_done(*r->program, r->slot)) HIPIE_CHECK_HIP(hipStreamSynchronize(r->stream));
                     continue;
                 }
                 for (;;) {
@@ -4303,6 +4341,18 @@ int hipie_request_tensor(const hipie_request* r, int node_id, hipie_tensor* t) {
         if (r->ran)
             for (int tensor : r->ran->inside)
                 HIPIE_REQUIRE(tensor != it->second, HIPIE_NOT_FOUND, "hipie_request_tensor: node %d lives in LDS only (two layers are one step of the single launch)", node_id);
+        for (const ConvStep* w : r->plan->result_writers) {
+            if (w->out != it->second) continue;
+            {
+                std::lock_guard<std::mutex> g(r->looked_lock);
+                if (std::find(r->looked.begin(), r->looked.end(), w) == r->looked.end()) r->looked.push_back(w);
+            }
+            if (!r->inferred || !(r->ran ? w->writes_result : w->direct)) continue;
+            DeviceGuard g(r->device);
+            if (is_capturing(r->stream)) continue;       // (what is captured fills it)
+            w->fill(r->arena.as<uint8_t>(), r->plan->tensors, r->stream);
+            if (!r->started) HIPIE_CHECK_HIP(hipStreamSynchronize(r->stream));      // (else the wait does)
+        }
         *t = r->plan->tensors[it->second].desc(r->arena.as<uint8_t>());
     });
 }

@@ -71,7 +71,7 @@ struct ProgConv {
     union {
         struct {                       // depthwise
             int32_t stride, group, c4, quads, OH, OW, items;
-            int32_t in_sn, in_sh, in_sw, row_sh, out_sn, out_sh, out_sw, res_sn, res_sh, res_sw;      // (dense: out_sn = bytes between the planes of f32 results that are stored at `res` as well, 0: none)
+            int32_t in_sn, in_sh, in_sw, row_sh, out_sn, out_sh, out_sw, res_sn, res_sh, res_sw;      // (dense: out_sn = bytes between the planes of f32 results, 0: channels innermost)
             float inv_c4, inv_quads, inv_OH;
         };
         ProgExpand expand;             // PK_EXPAND_DW, whose depthwise layer is a descriptor of its own behind this one
@@ -142,7 +142,7 @@ struct ProgBuilder {
         std::memcpy(w.data(), &s, sizeof(T));
         steps.push_back(w);
     }
-    // planes: the f32 results at this address as well, channel by channel (conv_run_planes)
+    // planes: the f32 results channel by channel at this address instead (conv_run_planes)
     bool conv(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out, void* planes = nullptr);
     // a dense layer and the depthwise 3 x 3 layer that is its only reader; `fill`: the stored byte of the padding between them
     bool expand_depthwise(const hipie_conv* first, const hipie_tensor& in, const hipie_tensor& mid, const hipie_conv* second, const hipie_tensor& out, int fill);

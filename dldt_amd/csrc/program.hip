@@ -380,7 +380,7 @@ struct StepConstants {
     float lm1, clamp_lo, clamp_hi;
     uint32_t off_bytes;                      // the level offset, four times
     int out_limit, res_limit;
-    uint32_t plane;                          // bytes between the planes of f32 results that are stored at `res` as well; 0: none
+    uint32_t plane;                          // bytes between the planes of f32 results; 0: channels innermost
 };
 template <bool DENSE>
 __device__ __forceinline__ StepConstants step_constants(const Ctx& x, uint32_t words) {
@@ -540,10 +540,11 @@ __device__ __forceinline__ void finish(const StepConstants& c, const ChannelCons
     if (!(fl & CF_OUT_FQ) && c.plane != 0) {
 #pragma unroll
         for (int a = 0; a < A; ++a) {
-            const uint32_t o = oc + a < c.res_limit ? static_cast<uint32_t>(oc + a) * c.plane : static_cast<uint32_t>(kBeyond);
+            const uint32_t o = oc + a < c.out_limit ? static_cast<uint32_t>(oc + a) * c.plane : static_cast<uint32_t>(kBeyond);
 #pragma unroll
-            for (int r = 0; r < R; ++r) publish4(c.res, q.res[r] + o, __float_as_uint(x[a][r] + 0.f));
+            for (int r = 0; r < R; ++r) publish4(c.out, q.out[r] + o, __float_as_uint(x[a][r] + 0.f));
         }
+        return;
     }
     if (!(fl & CF_OUT_FQ)) {
         const uint32_t o = oc < c.out_limit ? static_cast<uint32_t>(4 * oc) : static_cast<uint32_t>(kBeyond);
@@ -1822,15 +1823,15 @@ bool ProgBuilder::depthwise(const ConvLaunch& l, ProgConv& c) {
 bool ProgBuilder::layer(const ConvArgs& a, const hipie_tensor& out, ProgConv& c) {
     if (a.M > (1 << 20) || a.koff_tile || (a.flags & CF_OUT_I32) || ((a.flags & CF_OUT_FQ) && !(a.flags & CF_FQ_RCP)) || (a.flags & (CF_RES_SUB | CF_POST_SCALE)))
         return false;
-    const bool f32_out = !(a.flags & CF_OUT_FQ), f32_res = (a.flags & CF_RES_F32) != 0 || a.planes;
+    const bool f32_out = !(a.flags & CF_OUT_FQ), f32_res = (a.flags & CF_RES_F32) != 0;
     for (int64_t bytes : {static_cast<int64_t>(out.n) * a.out_sn * (f32_out ? 4 : 1), static_cast<int64_t>(out.n) * a.res_sn * (f32_res ? 4 : 1)})
         if (bytes >= kBeyond) return false;
     c.in = ref(a.in + a.in_origin);
     c.out = ref(a.out);
-    c.res = a.planes ? ref(a.planes) : a.res ? ref(a.res) : ProgRef{-2, 0, 0};
+    c.res = a.res ? ref(a.res) : ProgRef{-2, 0, 0};
     c.in2 = ProgRef{-2, 0, 0};
-    c.out_limit = a.out_sw;                            // channels that the output holds
-    c.res_limit = a.planes ? a.OC : a.res_sw;
+    c.out_limit = a.out_plane ? a.OC : a.out_sw;       // channels that the output holds
+    c.res_limit = a.res_sw;
     c.constants = constants(a);
     c.flags = a.flags; c.lm1 = a.lm1; c.off_bytes = (static_cast<uint32_t>(static_cast<int>(a.out_off)) & 0xffu) * 0x01010101u; c.clamp_lo = a.clamp_lo; c.clamp_hi = a.clamp_hi;
     c.OCp = a.OCp;
@@ -1905,7 +1906,7 @@ bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hip
     if (planes) planes_arguments(l.a, planes);
     const ConvArgs& a = l.a;
     const int64_t M = a.M;
-    const bool f32_out = !(a.flags & CF_OUT_FQ), f32_res = (a.flags & CF_RES_F32) != 0 || planes;
+    const bool f32_out = !(a.flags & CF_OUT_FQ), f32_res = (a.flags & CF_RES_F32) != 0;
     ProgConv c{};
     if (!layer(a, out, c)) return false;
     if (l.depthwise) {
@@ -1923,7 +1924,7 @@ bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hip
         return true;
     }
     c.kind = PK_CONV;
-    if (planes) c.out_sn = 4 * a.OHOW;
+    if (planes) c.out_sn = 4 * a.out_plane;
     c.nk = a.nk;
     const bool pair = (a.flags & CF_RES_GEMM) != 0;
     if (a.flags & CF_GELU) rows_kinds = true;
@@ -1956,7 +1957,7 @@ bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hip
         auto at = [&](int sn, int sh, int sw) { return static_cast<uint32_t>(n * sn + oh * sh + ow * sw); };
         pix[static_cast<size_t>(i)] = at(a.in_sn, a.in_sh * a.conv_sh, a.in_sw * a.conv_sw);
         pix[static_cast<size_t>(pitch + i)] = i < M ? at(a.out_sn, a.out_sh, a.out_sw) * (f32_out ? 4u : 1u) : static_cast<uint32_t>(kBeyond);
-        pix[static_cast<size_t>(2 * pitch + i)] = planes && i >= M ? static_cast<uint32_t>(kBeyond) : at(a.res_sn, a.res_sh, a.res_sw) * (f32_res ? 4u : 1u);
+        pix[static_cast<size_t>(2 * pitch + i)] = at(a.res_sn, a.res_sh, a.res_sw) * (f32_res ? 4u : 1u);
         pix[static_cast<size_t>(3 * pitch + i)] = pair ? at(a.in2_sn, a.in2_sh * a.conv2_sh, a.in2_sw * a.conv2_sw) : 0u;
     }
     c.pixels = keep(pix.data(), pix.size() * 4);

@@ -107,3 +107,57 @@ def test_a_result_is_in_its_tensor_as_well(hw, keep):
         assert np.array_equal(req.tensor(node).reshape(-1).view(np.uint32), seen[-1].view(np.uint32))
     assert plan.metric("SINGLE_LAUNCH_COUNTS") == "2 0"
     assert all(not np.array_equal(a, b) for a, b in zip(seen, seen[1:]))
+
+
+@pytest.mark.parametrize("single", ["NO", "256"])
+def test_a_tensor_that_is_held_shows_the_last_inference(single):
+    """the descriptor of a result's tensor, asked for once (before the first inference, or between two): the values of every
+    inference behind it, queued, waited for, or replayed from a captured graph"""
+    import ctypes
+    from dldt_amd._lib import check, lib
+    from dldt_amd.tensor import hipie_tensor
+    g = _graph(True, 1)
+    node = g.nodes[-1]["inputs"][0]
+    plan = g.compile(0, config={"HIP_TUNE": "NO", "HIP_THROUGHPUT_STREAMS": "1", "HIP_SINGLE_LAUNCH": single})
+    ins, outs = plan.create_request().device_buffers()
+
+    def held(req):
+        t = hipie_tensor()
+        check(lib().hipie_request_tensor(req._h, node, ctypes.byref(t)))
+        values = torch.empty(t.n * t.stride_n, dtype=torch.float32)
+
+        def shows():
+            torch.cuda.synchronize()
+            check(lib().hipie_memcpy(ctypes.c_void_p(values.data_ptr()), ctypes.c_void_p(t.data), ctypes.c_size_t(4 * values.numel()), 0))
+            v = torch.as_strided(values, (t.n, t.c, t.h, t.w), (t.stride_n, 1, t.stride_h, t.stride_w))
+            return torch.equal(v + 0.0, outs[0].cpu())
+        return shows
+
+    def feed(seed):
+        ins[0].uniform_(0, 2.55, generator=torch.Generator(device="cuda").manual_seed(seed))
+        torch.cuda.synchronize()
+
+    for asked in (0, 2):
+        req = plan.create_request()
+        shows = held(req) if asked == 0 else None
+        for turn, run in enumerate((req.infer_device, req.enqueue, req.infer_device, req.enqueue)):
+            if turn == asked and turn:
+                shows = held(req)
+                assert shows()
+            feed(turn)
+            run(ins, outs)
+            if turn >= asked:
+                assert shows(), (asked, turn)
+    req = plan.create_request()
+    stream = torch.cuda.ExternalStream(req.stream)
+    feed(7)
+    req.enqueue(ins, outs)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+        req.enqueue(ins, outs)
+    shows = held(req)
+    for turn in range(3):
+        feed(10 + turn)
+        graph.replay()
+        assert shows(), turn
