@@ -14,6 +14,7 @@
 #include <mutex>
 
 #include "convf.h"
+#include "entry_conv.h"
 #include "fq.h"
 #include "graph.h"
 #include "requant.h"
@@ -172,13 +173,16 @@ struct EntryStep : Step {
     int64_t channels = 0, levels = 0;
     std::vector<float> il, ih, ol, oh;
     hipie_fq* fq = nullptr;
+    bool inside_next = false;      // the convolution behind it does it in its launch
     ~EntryStep() override { hipie_fq_destroy(fq); }
+    int launches() const override { return inside_next ? 0 : 1; }
     void create(int device, const std::vector<TensorInfo>&) override {
         check_status(hipie_fq_create(device, channels, levels, il.data(), il.size(), ih.data(), ih.size(),
                                      ol.data(), ol.size(), oh.data(), oh.size(), &fq), name.c_str());
     }
     void run(uint8_t* arena, const std::vector<TensorInfo>& tensors, void* const* inputs, void* const*,
              hipStream_t s) const override {
+        if (inside_next) return;
         const hipie_tensor d = tensors[out].desc(arena);
         check_status(u8_in ? hipie_fq_run_q8_tensor_u8(fq, static_cast<const uint8_t*>(inputs[param_index]), &d, s)
                            : hipie_fq_run_q8_tensor(fq, static_cast<const float*>(inputs[param_index]), &d, s),
@@ -211,6 +215,16 @@ struct ConvStep : Step {
     // transposition and goes away in the single launch only
     bool writes_result = false, direct = false;
     float tuned_us = 0.f;          // per launch with every tuning lane busy, of the variant the tuner kept (0: not tuned)
+    // A graph input's FakeQuantize right in front of a `direct` layer: one launch for both where that is faster (entry_conv.hip).
+    // The levels between them are in their tensor either way
+    EntryStep* entry = nullptr;
+    std::shared_ptr<EntryConv> with_entry;         // null: the kernel does not take the two
+    int entry_mode = 1;                            // PlanConfig::fuse_convs
+    bool entry_fused = false;
+    void choose_entry(bool one_launch) {
+        entry_fused = one_launch && with_entry;
+        if (entry) entry->inside_next = entry_fused;
+    }
     ~ConvStep() override { hipie_conv_destroy(conv); }
     void fill_desc(const std::vector<TensorInfo>& tensors) {
         const TensorInfo& t = tensors[in];
@@ -255,6 +269,10 @@ struct ConvStep : Step {
              hipStream_t s) const override {
         const hipie_tensor i = tensors[in].desc(arena), o = tensors[out].desc(arena);
         hipie_tensor r{};
+        if (entry_fused) {
+            run_entry_conv(*with_entry, inputs[entry->param_index], i, outputs[result], s);
+            return;
+        }
         if (direct) {
             check_status(conv_run_planes(conv, i, o, outputs[result], s), name.c_str());
             return;
@@ -319,17 +337,18 @@ struct ConvStep : Step {
         return static_cast<double>(results) * epilogue_valu_ops(flags) + (shortcut && !fused ? shortcut->valu_ops() : 0.0);
     }
     bool deep = false;             // variant 24 with nine steps of weights in flight (hipie_conv_set_stages)
-    // kernel variant (hipie_conv_set_tile) + 32 for `deep`
+    // kernel variant (hipie_conv_set_tile) + 32 for `deep` + 64 for one launch with the FakeQuantize in front of it
     int variant() const override {
         int t = -1;
         if (conv) (void)hipie_conv_get_tile(conv, &t);
-        return t < 0 ? t : t + (deep ? 32 : 0);
+        return t < 0 ? t : t + (deep ? 32 : 0) + (entry_fused ? 64 : 0);
     }
     void set_variant(int v) override {
         if (!conv || v < 0) return;
         check_status(hipie_conv_set_tile(conv, v & 31), name.c_str());
         deep = (v & 32) != 0;
         check_status(hipie_conv_set_stages(conv, deep ? 8 : 0), name.c_str());
+        choose_entry((v & 64) != 0);
     }
     // Every variant computes the same integers, so the choice changes time only.  Variants a layer
     // cannot use are refused by hipie_conv_set_tile and skipped.
@@ -348,10 +367,14 @@ struct ConvStep : Step {
             else if (res_param >= 0) tr[l] = input_residual(to[l], lanes[l].inputs[res_param]);
         }
         const bool has_res = fused || res >= 0 || res_param >= 0;
+        bool entry_too = false;
         auto launch_all = [&](int times) {
             for (int w = 0; w < times; ++w)
                 for (size_t l = 0; l < nl; ++l)
-                    check_status(direct ? conv_run_planes(conv, ti[l], to[l], lanes[l].outputs[result], lanes[l].stream)
+                    if (entry_too) {
+                        entry->run(lanes[l].arena, tensors, lanes[l].inputs.data(), nullptr, lanes[l].stream);
+                        run(lanes[l].arena, tensors, lanes[l].inputs.data(), lanes[l].outputs.data(), lanes[l].stream);
+                    } else check_status(direct ? conv_run_planes(conv, ti[l], to[l], lanes[l].outputs[result], lanes[l].stream)
                                         : hipie_conv_run(conv, &ti[l], has_res ? &tr[l] : nullptr, &to[l], lanes[l].stream), name.c_str());
         };
         std::vector<hipEvent_t> e0(nl), e1(nl);
@@ -359,20 +382,7 @@ struct ConvStep : Step {
             HIPIE_CHECK_HIP(hipEventCreate(&e0[l]));
             HIPIE_CHECK_HIP(hipEventCreate(&e1[l]));
         }
-        int best = current;
-        float best_ms = 0.f, few_ms = -1.f;
-        const int candidates[] = {current, 0, 1, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17, 18, 19, 20, 21, 22, 23, 24, 24 + 32};
-        for (size_t c = 0; c < sizeof(candidates) / sizeof(candidates[0]); ++c) {
-            // (1 stands for 2 as well on a depthwise layer, whose third variant is the matrix-pipe form; the dense variant 2
-            // is a tile shape that no layer of a batch wants)
-            for (int alt = 0; alt < (desc.groups > 1 && candidates[c] == 1 ? 2 : 1); ++alt) {
-            const int tile = alt ? 2 : (candidates[c] & 31);
-            if (c > 0 && candidates[c] == current && !alt) continue;
-            if (hipie_conv_set_tile(conv, tile) != HIPIE_OK) continue;
-            int applied = -1;
-            check_status(hipie_conv_get_tile(conv, &applied), name.c_str());
-            if (applied != tile) continue;   // not available for this layer (kept its previous variant)
-            check_status(hipie_conv_set_stages(conv, (candidates[c] & 32) ? 8 : 0), name.c_str());
+        auto measure = [&] {
             launch_all(2);
             // the fastest of three rounds of five launches: a round disturbed by something else on the
             // device (another plan being compiled, a clock step) does not decide the choice
@@ -392,6 +402,23 @@ struct ConvStep : Step {
                     }
                 ms = round == 0 ? span : std::min(ms, span);
             }
+            return ms;
+        };
+        int best = current;
+        float best_ms = 0.f, few_ms = -1.f;
+        const int candidates[] = {current, 0, 1, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17, 18, 19, 20, 21, 22, 23, 24, 24 + 32};
+        for (size_t c = 0; c < sizeof(candidates) / sizeof(candidates[0]); ++c) {
+            // (1 stands for 2 as well on a depthwise layer, whose third variant is the matrix-pipe form; the dense variant 2
+            // is a tile shape that no layer of a batch wants)
+            for (int alt = 0; alt < (desc.groups > 1 && candidates[c] == 1 ? 2 : 1); ++alt) {
+            const int tile = alt ? 2 : (candidates[c] & 31);
+            if (c > 0 && candidates[c] == current && !alt) continue;
+            if (hipie_conv_set_tile(conv, tile) != HIPIE_OK) continue;
+            int applied = -1;
+            check_status(hipie_conv_get_tile(conv, &applied), name.c_str());
+            if (applied != tile) continue;   // not available for this layer (kept its previous variant)
+            check_status(hipie_conv_set_stages(conv, (candidates[c] & 32) ? 8 : 0), name.c_str());
+            const float ms = measure();
             // a variant has to beat the best so far by more than the timing noise of seven launches,
             // otherwise the choice (and the run-to-run spread of a whole network) follows the noise
             if ((c == 0 && !alt) || ms < 0.97f * best_ms) {
@@ -413,11 +440,24 @@ struct ConvStep : Step {
                 best_ms = few_ms;
             }
         }
+        set_variant(best);
+        float together = 0.f, apart = 0.f;
+        if (with_entry) {      // with the FakeQuantize in front of it, as one launch and as two
+            auto with = [&](bool one) {
+                choose_entry(one);
+                entry_too = true;
+                const float ms = measure();
+                entry_too = false;
+                return ms;
+            };
+            apart = with(false);
+            together = with(true);
+            choose_entry(entry_mode == 2 || together < 0.97f * apart);
+        }
         for (size_t l = 0; l < nl; ++l) {
             (void)hipEventDestroy(e0[l]);
             (void)hipEventDestroy(e1[l]);
         }
-        set_variant(best);
         tuned_us = best_ms * 200.f / static_cast<float>(nl);
         if (std::getenv("HIPIE_TUNE_LOG")) {
             uint32_t fl = 0;
@@ -425,6 +465,9 @@ struct ConvStep : Step {
             (void)hipie_conv_epilogue_flags(conv, &fl, &spec);
             std::fprintf(stderr, "hipie tune: %-28s variant %d (%.1f us per launch with %zu in flight; default %d) epilogue %#x%s\n",
                          name.c_str(), best, best_ms * 200.f / static_cast<float>(nl), nl, current, fl, spec ? "" : " GENERIC");
+            if (with_entry)
+                std::fprintf(stderr, "hipie tune: %-28s with the FakeQuantize in front of it one launch %.1f us, two %.1f us: %s\n", name.c_str(),
+                             together * 200.f / static_cast<float>(nl), apart * 200.f / static_cast<float>(nl), entry_fused ? "one" : "two");
         }
     }
 };
@@ -3481,6 +3524,22 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
             pair->create(device, plan->tensors);
             plan->steps[i] = std::move(pair);
             plan->steps.erase(plan->steps.begin() + static_cast<std::ptrdiff_t>(i) + 1);
+        }
+    // A graph input's FakeQuantize and the convolution behind it whose f32 values are the graph's result: two steps, of one launch
+    // where that is faster
+    if (cfg.fuse_convs != 0 && !cfg.keep_f32 && device >= 0)
+        for (size_t i = 0; i + 1 < plan->steps.size(); ++i) {
+            auto* e = dynamic_cast<EntryStep*>(plan->steps[i].get());
+            auto* c = dynamic_cast<ConvStep*>(plan->steps[i + 1].get());
+            if (!e || !c || !c->direct || c->in != e->out) continue;
+            const TensorInfo& mid = plan->tensors[e->out];
+            if (mid.alias >= 0 || !mid.fill_levels.empty()) continue;
+            c->with_entry = make_entry_conv(device, e->fq, e->u8_in, c->conv, mid.desc(nullptr), plan->tensors[c->out].desc(nullptr),
+                                            mid.dtype == HIPIE_U8B ? mid.fill_level - 128 : mid.fill_level);
+            if (!c->with_entry) continue;
+            c->entry = e;
+            c->entry_mode = cfg.fuse_convs;
+            c->choose_entry(cfg.fuse_convs == 2);
         }
     for (size_t i = 0; i < pl.values.size(); ++i)
         if (pl.values[i].kind == VK_TENSOR) {

@@ -1,0 +1,112 @@
+"""A graph input's FakeQuantize and the convolution behind it as one launch (csrc/entry_conv.hip) against the two, bit for bit: the
+values in the caller's buffer and the levels in the tensor between them."""
+import numpy as np
+import pytest
+import torch
+
+from dldt_amd import builders
+from dldt_amd.graph import Plan
+from dldt_amd.tensor import F32
+
+pytestmark = pytest.mark.gpu
+
+
+def _graph(n, c, h, w, oc, k=3, kind="u8", act="relu"):
+    """kind: the input's levels - u8, i8, u8 with a zero point, or u8 values as they are"""
+    rng = np.random.default_rng(n * c + h)
+    q = builders.QuantizedNet()
+    if kind == "bytes":
+        a = q.input("data", (n, c, h, w), 255.0, u8=True)
+    elif kind == "u8":
+        a = q.input("data", (n, c, h, w), 2.55)
+    else:
+        p = q.g.parameter("data", (n, c, h, w))
+        a = q.requantize(p, 1.9, signed=True) if kind == "i8" else q.asymmetric(p, -0.7, 1.9)
+    y = q.conv_f32(a, rng.standard_normal((oc, c, k, k), dtype=np.float32) * np.float32(0.1), rng.standard_normal(oc, dtype=np.float32), pads=(k // 2, k // 2), relu=act == "relu")
+    if act == "clamp":
+        y = q.g.clamp(y, -0.25, 0.5)
+    q.g.result(y, "out")
+    return q.g, a["node"]
+
+
+def _compile(g, fuse, **kw):
+    return g.compile(0, config=dict({"HIP_FUSE_CONVOLUTIONS": fuse, "HIP_TUNE": "NO", "HIP_SINGLE_LAUNCH": "NO"}, **kw))
+
+
+def _one(plan):
+    return int(plan.step_rt_info(0, "kernels")) == 0
+
+
+def _run(plan, node, x, offset=0):
+    req = plan.create_request()
+    ins, outs = req.device_buffers()
+    size = x.element_size()
+    feed = torch.zeros(x.numel() + 16, dtype=x.dtype, device="cuda")[offset:offset + x.numel()].view(x.shape)
+    feed.copy_(x)
+    place = torch.full((outs[0].numel() + 16,), float("nan"), device="cuda")
+    out = place[offset:offset + outs[0].numel()].view(outs[0].shape)
+    torch.cuda.synchronize()
+    assert feed.data_ptr() % (16 * size) == offset * size
+    req.enqueue([feed], [out])
+    torch.cuda.synchronize()
+    assert torch.isnan(place[:offset]).all() and torch.isnan(place[offset + out.numel():]).all()
+    return out.cpu().numpy().view(np.uint32), req.tensor(node)
+
+
+def _input(g, seed):
+    node = g.nodes[0]
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    if node["dtype"] != F32:
+        return torch.randint(0, 256, node["shape"], generator=gen, device="cuda", dtype=torch.uint8)
+    x = torch.randn(node["shape"], generator=gen, device="cuda") * 2
+    flat = x.view(-1)
+    for i, v in enumerate((float("nan"), float("inf"), -float("inf"), 0.0, -0.0, 1e-40, 3e38, -3e38)):
+        flat[i * 7 % flat.numel()::41] = v
+    return x
+
+
+# tiles of one row and of many, a last tile of fewer rows, pixels that end inside a fragment and a wave's chunk, channels that end
+# inside a quad, a pixel of four bytes, an odd and an even number of 16-byte pieces, output channels inside a tile of 32, several groups
+@pytest.mark.parametrize("n,c,h,w,oc", [(1, 1, 1, 2, 1), (1, 3, 7, 7, 8), (2, 4, 9, 31, 33), (1, 5, 33, 2, 31), (3, 17, 9, 65, 65), (2, 16, 5, 64, 32), (12, 72, 45, 45, 100),
+                                        (1, 64, 56, 56, 64), (2, 8, 107, 107, 301), (32, 256, 7, 7, 512), (1, 256, 112, 112, 9), (7, 30, 14, 512, 40), (5, 33, 1, 100, 130)])
+def test_one_launch_equals_two(n, c, h, w, oc):
+    g, node = _graph(n, c, h, w, oc)
+    one, two = _compile(g, "YES"), _compile(g, "NO")
+    assert _one(one) and not _one(two)
+    for seed, offset in ((1, 0), (2, 1)):                    # (buffers on a 4-byte boundary only)
+        x = _input(g, seed)
+        got, want = _run(one, node, x, offset), _run(two, node, x, offset)
+        assert np.array_equal(got[1], want[1]) and np.array_equal(got[0], want[0])
+
+
+@pytest.mark.parametrize("kind", ["u8", "i8", "zero point", "bytes"])
+@pytest.mark.parametrize("c,k,act", [(3, 3, "clamp"), (3, 7, "relu"), (20, 1, "none"), (20, 5, "clamp"), (40, 3, "none")])
+def test_kinds_of_levels_filters_and_activations(kind, c, k, act):
+    g, node = _graph(3, c, 13, 19, 37, k, kind, act)
+    one, two = _compile(g, "YES"), _compile(g, "NO")
+    assert _one(one) and not _one(two)
+    x = _input(g, 3)
+    got, want = _run(one, node, x), _run(two, node, x)
+    assert np.array_equal(got[1], want[1]) and np.array_equal(got[0], want[0])
+
+
+def test_what_the_kernel_does_not_take_runs_as_two():
+    g, node = _graph(1, 20, 4, 600, 8)                         # a row of more pixels than a workgroup's waves hold
+    assert not _one(_compile(g, "YES"))
+    assert not _one(_compile(_graph(2, 20, 9, 9, 8)[0], "YES", HIP_KEEP_F32="YES"))
+    assert not _one(_compile(_graph(2, 20, 9, 9, 8)[0], "AUTO"))   # (not measured)
+
+
+def test_the_choice_is_kept_in_files_and_exports(tmp_path):
+    g, node = _graph(2, 17, 9, 9, 65)
+    x = _input(g, 5)
+    want = _run(_compile(g, "NO"), node, x)
+    path = tmp_path / "choices"
+    tuned = _compile(g, "YES", HIP_TUNE="YES", HIP_TUNE_FILE=str(path))
+    again = _compile(g, "AUTO", HIP_TUNE="YES", HIP_TUNE_FILE=str(path))
+    loaded = Plan.load(tuned.export())
+    for plan in (tuned, again, loaded):
+        assert _one(plan) and plan.steps[1]["variant"] == tuned.steps[1]["variant"]
+        got = _run(plan, node, x)
+        assert np.array_equal(got[1], want[1]) and np.array_equal(got[0], want[0])
+    assert not _one(_compile(g, "NO", HIP_TUNE="YES", HIP_TUNE_FILE=str(path)))
