@@ -5,6 +5,7 @@ Every node is also recorded in ``Graph.nodes`` (plain dicts with numpy constants
 checker can evaluate the very same graph with reference kernels.
 """
 import ctypes
+import functools
 
 import numpy as np
 
@@ -296,6 +297,12 @@ class Plan:
         return Request(self, perf_count)
 
 
+@functools.lru_cache(maxsize=None)
+def _pointers(n):
+    """the C array type of n pointers"""
+    return ctypes.c_void_p * n
+
+
 class PinnedArray:
     """numpy array over page-locked host memory from hipie_host_alloc (`.array`); freed with the object"""
 
@@ -370,9 +377,7 @@ class Request:
         return ins, outs
 
     def _ptrs(self, ins, outs):
-        ip = (ctypes.c_void_p * len(ins))(*[t.data_ptr() for t in ins])
-        op = (ctypes.c_void_p * len(outs))(*[t.data_ptr() for t in outs])
-        return ip, op
+        return _pointers(len(ins))(*[t.data_ptr() for t in ins]), _pointers(len(outs))(*[t.data_ptr() for t in outs])
 
     def infer_device(self, ins, outs):
         ip, op = self._ptrs(ins, outs)

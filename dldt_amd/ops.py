@@ -19,8 +19,13 @@ def _fptr(a):
 
 
 def _stream():
+    """The current stream of the current device.  torch.cuda.current_stream() makes an object of it first: 2.9 us a call where the
+    handle alone takes 0.15, beside 3.6 for a kernel's launch."""
     import torch
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    try:
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
+    except AttributeError:
+        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
 def _dptr(t):
@@ -77,12 +82,11 @@ class FakeQuantize:
         n, hw = self._nhw(x)
         tdt = torch.int8 if dtype in ("i8", "u8b") else torch.uint8
         if layout == "nchw":
-            y = torch.empty(x.shape, dtype=tdt, device=x.device) if out is None else out
+            y = torch.empty_like(x, dtype=tdt) if out is None else out
             cs = 0
         else:
             cs = c_stride or -(-self.C // 16) * 16
-            y = torch.empty((n,) + tuple(x.shape[2:]) + (cs,), dtype=tdt, device=x.device) \
-                if out is None else out
+            y = x.new_empty((n, *x.shape[2:], cs), dtype=tdt) if out is None else out
         check(lib().hipie_fq_run_q8(self._h, _dptr(x), _dptr(y), ctypes.c_int64(n),
                                     ctypes.c_int64(hw), ctypes.c_int(_DT[dtype]),
                                     ctypes.c_int(NCHW if layout == "nchw" else NHWC),
