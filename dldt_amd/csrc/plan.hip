@@ -3103,6 +3103,7 @@ struct hipie_request {
     const ProgramForm* form = nullptr;
     const ProgramForm* ran = nullptr;        // the form of the last inference, if it was one (hipie_request_tensor)
     bool entered = false;                    // counted among the device's requests in flight
+    bool alone = false;                      // no other was when this one started, nor lately
     bool stream_taken = false;               // hipie_request_stream gave the stream out: its work is complete in stream order
     std::vector<void*> run_in, run_out, host_out;
     // Results whose tensors were looked at (hipie_request_tensor): from then on every inference fills these, so that a tensor
@@ -4259,6 +4260,7 @@ static int start_request(hipie_request* r, const void* const* inputs, void* cons
         r->entered = true;
         r->ran = nullptr;
         const int together = request_enters(p.device);
+        r->alone = together == 1;
         if (r->slot >= 0 && (awaited || (!device_memory && !r->stream_taken)) && buffers_fit_program(p, in.data(), out.data()))
             r->form = r->program->choose(together);
         if (r->form) {
@@ -4311,8 +4313,12 @@ int hipie_request_wait_for(hipie_request* r, int64_t timeout_ms) {
             } idle{r};
             do {
                 if (timeout_ms < 0) {
-                    // (a single launch into the caller's device buffers says itself when they are written: nothing follows it)
-                    if (!r->form || !r->host_out.empty() || r->looked_at() || !report_done(*r->program, r->slot)) HIPIE_CHECK_HIP(hipStreamSynchronize(r->stream));
+                    // A single launch into the caller's device buffers says itself when they are written: nothing follows it.  Beside
+                    // other requests it is waited for to its end: one that starts again the moment its results are there keeps its
+                    // place from the others for good (of three threads with 50 launches of 256 workgroups each, one made them all
+                    // and another none; 93, 97 and 15 of 100, 100 and 50 where they wait).
+                    const bool word = r->form && r->alone && r->host_out.empty() && !r->looked_at();
+                    if (!word || !report_done(*r->program, r->slot)) HIPIE_CHECK_HIP(hipStreamSynchronize(r->stream));
                     continue;
                 }
                 for (;;) {
