@@ -140,8 +140,17 @@ struct ProgBuilder {
         static_assert(sizeof(T) <= kProgramStepWords * 4 && sizeof(T) % 4 == 0, "step descriptor");
         std::array<int32_t, kProgramStepWords> w{};
         std::memcpy(w.data(), &s, sizeof(T));
-        steps.push_back(w);
+        push(w);
     }
+    void push(const std::array<int32_t, kProgramStepWords>& w) {
+        steps.push_back(w);
+        written = std::move(writing);
+        writing.clear();
+    }
+    // what the step that is built writes in the arena (or may: no less), and what the last one did
+    std::vector<std::pair<const uint8_t*, int64_t>> writing, written;
+    void writes(const void* p, int64_t bytes);
+    bool was_just_written(const void* p, const hipie_tensor& t) const;      // the tensor that begins at p
     // planes: the f32 results channel by channel at this address instead (conv_run_planes)
     bool conv(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out, void* planes = nullptr);
     // a dense layer and the depthwise 3 x 3 layer that is its only reader; `fill`: the stored byte of the padding between them

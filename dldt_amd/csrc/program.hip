@@ -63,6 +63,25 @@ constexpr uint32_t kGivenUp = 1u << 26;      // added to a counter that was not 
 
 __device__ __forceinline__ int lane_index() { return static_cast<int>(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u))); }
 
+// Everything that was asked of memory and LDS has come (or, of LDS only).  As instructions the compiler knows: behind a wait in inline
+// assembly it goes on counting what was in flight in front of it, and waits for all of it, the barrier's own addition included,
+// where a register of those loads is used again (0.5 us of a step's preparation).
+__device__ __forceinline__ void wait_memory() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070);      // vmcnt(0) lgkmcnt(0)
+    asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ void wait_lds() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+}
+// a barrier of the workgroup in front of which only LDS is waited for
+__device__ __forceinline__ void meet() {
+    wait_lds();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
 struct Ctx {
     int rank, n_wg, wg_shift;                // neighbouring ranks share an XCD; n_wg = 1 << wg_shift
     int tid, lane, wave;
@@ -95,10 +114,11 @@ struct Ctx {
     __device__ __forceinline__ void arrive(int next_step) {
         words = load_words(next_step, 0);
         words2 = load_words(next_step, 1);
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        wait_memory();
         __builtin_amdgcn_s_barrier();
         target += n_wg / 8;
-        if (tid == 0) (void)__hip_atomic_fetch_add(own, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // (not the wave that looks at the counters: its loads would come back behind the addition)
+        if (tid == kProgramThreads - 64) (void)__hip_atomic_fetch_add(own, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         dead = __builtin_amdgcn_readfirstlane(flag[0]) == 0;      // (of the wait before: its verdict is not waited for)
     }
     __device__ __forceinline__ void wait() {
@@ -120,9 +140,7 @@ struct Ctx {
             }
         }
         started = false;
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+        meet();
     }
     // Every workgroup has arrived behind the last step: the first one tells the host in the page-locked word that it looks at
     // (report_done).  All results were stored with device scope and acknowledged, so they are in memory.
@@ -287,7 +305,13 @@ __device__ __forceinline__ void first_weights(Ring<A, B>& g, const KSource& s, i
     for (int d = 0; d < Ring<A, B>::D; ++d) load_weights<A, B>(g, s, d, s.kk + d * s.ks, lane);
 }
 
-// acc += the wave's K steps; the first D steps' weights are already on their way (first_weights)
+template <int A, int B>
+__device__ __forceinline__ void first_pixels(Ring<A, B>& g, const KSource& s, const uint32_t (&off)[B], int lane) {
+#pragma unroll
+    for (int d = 0; d < Ring<A, B>::D; ++d) load_pixels<A, B>(g, s, off, d, s.kk + d * s.ks, lane);
+}
+
+// acc += the wave's K steps; the first D steps' operands are already on their way (first_weights, first_pixels)
 template <int A, int B>
 __device__ __forceinline__ void k_loop(Ring<A, B>& g, const KSource& s, const uint32_t (&off)[B], int lane, v4i (&acc)[A][B]) {
     constexpr int D = Ring<A, B>::D;
@@ -298,8 +322,6 @@ __device__ __forceinline__ void k_loop(Ring<A, B>& g, const KSource& s, const ui
             for (int b = 0; b < B; ++b) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(g.p[d][b], g.w[d][a], acc[a][b], 0, 0, 0);
     };
     int k = s.kk;
-#pragma unroll
-    for (int d = 0; d < D; ++d) load_pixels<A, B>(g, s, off, d, k + d * s.ks, lane);
     while (k + D * s.ks < s.nk) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
@@ -595,7 +617,11 @@ __device__ __forceinline__ void place_pixels(const uint32_t* pix, int M, int at,
 template <bool GELU, int A, int B, int R, bool PAIR>
 __device__ __forceinline__ void finish_column(const StepConstants& sc, const ChannelConstants<A>& k, const ChannelConstants<A>& k2, lds_v4i mine, lds_v4i mine2, int ks,
                                               int b, int r0, const Pixels<A>& q, int oc) {
-    auto total = [&](lds_v4i from, int32_t (&sum)[A][R]) {
+    auto total = [&](lds_v4i from, const int32_t (&corr)[A], int32_t (&sum)[A][R]) {
+#pragma unroll
+        for (int a = 0; a < A; ++a)
+#pragma unroll
+            for (int r = 0; r < R; ++r) sum[a][r] = corr[a];                     // a sum starts from the channel's integer correction
         const lds_i32 w = (lds_i32)(from + b * A * 64) + r0;
         for (int s = 0; s < ks; ++s)
 #pragma unroll
@@ -604,19 +630,19 @@ __device__ __forceinline__ void finish_column(const StepConstants& sc, const Cha
                 if constexpr (R == 4) {
                     const v4i t = *(lds_v4i)v;
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) sum[a][r] = s == 0 ? t[r] : sum[a][r] + t[r];
+                    for (int r = 0; r < 4; ++r) sum[a][r] += t[r];
                 } else {
 #pragma unroll
-                    for (int r = 0; r < R; ++r) sum[a][r] = s == 0 ? v[r] : sum[a][r] + v[r];
+                    for (int r = 0; r < R; ++r) sum[a][r] += v[r];
                 }
             }
     };
     int32_t sum[A][R];
     float rg[A][R] = {};
-    total(mine, sum);
+    total(mine, k.corr, sum);
     if constexpr (PAIR) {
         int32_t s2[A][R];
-        total(mine2, s2);
+        total(mine2, k2.corr, s2);
 #pragma unroll
         for (int a = 0; a < A; ++a)
 #pragma unroll
@@ -652,17 +678,18 @@ __device__ __forceinline__ void conv_tiles(Ctx& x, lds_ptr lds) {
     }
     const uint32_t tiles = static_cast<uint32_t>(PROG_FIELD(x.words, tiles));
     const int t0 = static_cast<int>((static_cast<uint32_t>(x.rank) * tiles) >> x.wg_shift), t1 = static_cast<int>((static_cast<uint32_t>(x.rank + 1) * tiles) >> x.wg_shift);
-    const StepConstants sc = step_constants<true>(x, x.words);
     const int M = PROG_FIELD(x.words, M);
     const uint32_t* pix = PROG_TABLE_OF(uint32_t, x.words, pixels);
     const lds_v4i part = (lds_v4i)lds + x.wave * (F * 64) + x.lane;
     const lds_v4i part2 = (lds_v4i)(lds + kPartBytes / 2) + x.wave * (F * 64) + x.lane;
     const lds_v4i mine = (lds_v4i)lds + sub * src.ks * (F * 64) + x.lane, mine2 = (lds_v4i)(lds + kPartBytes / 2) + sub * src.ks * (F * 64) + x.lane;
-    // The waves that share a tile's K share its chain as well: whole columns of pixels, or two of a quad's four pixels, or one.
-    // (The chain on one wave's eight values is 0.3 us of a step; the others of its tile would only wait for it.)
-    const int kk = src.kk, rows = B == 4 ? 4 : (4 * B) >> shift;      // (four columns and eight waves to a tile: choose_tile does not)
-    const int col0 = rows >= 4 ? kk & (B - 1) : (rows == 2 ? kk >> 1 : min(kk >> 2, B - 1)), r0 = rows >= 4 ? 0 : (rows == 2 ? 2 * (kk & 1) : kk & 3);
-    const bool finishes = rows >= 4 ? kk < B : kk < 4 * B;
+    // The waves that share a tile's K share its chain as well: whole columns of pixels, or one of a quad's four pixels.  (The chain on
+    // one wave's eight values is 0.3 us of a step; the others of its tile would only wait for it.  Two of the four pixels was a third
+    // form: 8 KB of the kernel.  Every form counts: steps whose code does not fit the 64 KB that a pair of units' instruction cache
+    // holds cost a ResNet-50 of batch 1 3 %, six times the misses, with a ring of its own for short K sums, for instance.)
+    const int kk = src.kk, rows = (4 * B) >> shift <= 1 ? 1 : 4;      // (four columns and eight waves to a tile: choose_tile does not)
+    const int col0 = rows == 4 ? kk & (B - 1) : min(kk >> 2, B - 1), r0 = rows == 4 ? 0 : kk & 3;
+    const bool finishes = rows == 4 ? kk < B : kk < 4 * B;
     bool first = true;
     int base = t0;
     do {
@@ -673,7 +700,11 @@ __device__ __forceinline__ void conv_tiles(Ctx& x, lds_ptr lds) {
         Ring<A, B> ring;
         uint32_t off[B], off2[B];
         Pixels<A> q;
-        const int lane16 = x.lane & 15, quad = x.lane >> 4;
+        int lane = x.lane;
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("" : "+v"(lane));       // (its functions are not kept in registers around the loop)
+#endif
+        const int lane16 = lane & 15, quad = lane >> 4;
         int ot, pt;
         fast_divmod(on ? tile : 0, PROG_FIELD(x.words, p_tiles), PROG_FIELD(x.words, inv_p_tiles), ot, pt);
         ot = __builtin_amdgcn_readfirstlane(ot);
@@ -681,24 +712,37 @@ __device__ __forceinline__ void conv_tiles(Ctx& x, lds_ptr lds) {
         const int mt = pt * (16 * B), oc = ot * (16 * A) + A * lane16;
         src.w = make_buffer(PROG_TABLE_OF(int8_t, x.words, wgt) + static_cast<int64_t>(ot) * src.nk * (A * 1024));
         if constexpr (PAIR) src2.w = make_buffer(PROG_TABLE_OF(int8_t, x.words, wgt2) + static_cast<int64_t>(ot) * src2.nk * (A * 1024));
+        // All that the step in front does not write is on its way before the wait: operands, constants, where the results go and, from
+        // an older step, the residual.  Loads come back in order and a branch hides from the compiler how many there were behind it:
+        // nothing that is loaded under a condition stands behind the pixels, which are the first to be waited for.
         if (on) {
 #pragma unroll
             for (int b = 0; b < B; ++b) off[b] = pix[mt + 16 * b + lane16];
-            const int pitch = PROG_FIELD(x.words, OCp) * 4;
+            if (finishes) place_pixels<A>(pix, M, mt + 16 * col0 + 4 * quad + r0, q);      // the first column this wave finishes
             if constexpr (PAIR) {
 #pragma unroll
                 for (int b = 0; b < B; ++b) off2[b] = pix[3 * M + mt + 16 * b + lane16];
-                first_weights<A, B>(ring, src2, x.lane);
-                const uint8_t* t2 = PROG_TABLE_OF(uint8_t, x.words, constants2) + oc * 4;
-                load_channels<A>(reinterpret_cast<const int32_t*>(t2), k2.corr);
-                load_channels<A>(reinterpret_cast<const float*>(t2 + pitch), k2.bias);
-                load_channels<A>(reinterpret_cast<const float*>(t2 + 2 * pitch), k2.scale);
-            } else {
-                first_weights<A, B>(ring, src, x.lane);
             }
-            if constexpr (kLate) load_channels<A>(reinterpret_cast<const int32_t*>(PROG_TABLE_OF(uint8_t, x.words, constants) + oc * 4), k.corr);
-            else load_constants<A>(sc.flags, PROG_TABLE_OF(uint8_t, x.words, constants), pitch, oc, k);
-            place_pixels<A>(pix, M, mt + 16 * col0 + 4 * quad + r0, q);      // the first column this wave finishes
+        }
+        if (on) {
+            if constexpr (PAIR) first_weights<A, B>(ring, src2, x.lane);
+            else first_weights<A, B>(ring, src, x.lane);
+            if (finishes) {
+                const int pitch = PROG_FIELD(x.words, OCp) * 4;
+                if constexpr (PAIR) {
+                    const uint8_t* t2 = PROG_TABLE_OF(uint8_t, x.words, constants2) + oc * 4;
+                    load_channels<A>(reinterpret_cast<const int32_t*>(t2), k2.corr);
+                    load_channels<A>(reinterpret_cast<const float*>(t2 + pitch), k2.bias);
+                    load_channels<A>(reinterpret_cast<const float*>(t2 + 2 * pitch), k2.scale);
+                }
+                if constexpr (!kLate) load_constants<A>(PROG_FIELD(x.words, flags), PROG_TABLE_OF(uint8_t, x.words, constants), pitch, oc, k);
+                StepConstants r{};
+                r.flags = PROG_FIELD(x.words, flags);
+                r.res = make_buffer(PROG_PLACE(x, res));
+                r.res_limit = PROG_FIELD(x.words, res_limit);
+                if (rows == 4) load_residual<A, 4>(r, oc, q);
+                    else load_residual<A, 1>(r, oc, q);
+            }
         }
         if (first) {
             if (!plain) {
@@ -708,14 +752,21 @@ __device__ __forceinline__ void conv_tiles(Ctx& x, lds_ptr lds) {
             x.wait();
             first = false;
         }
+        if (on) {
+            if constexpr (PAIR) first_pixels<A, B>(ring, src2, off2, x.lane);
+            else first_pixels<A, B>(ring, src, off, x.lane);
+        }
+        uint32_t words = x.words;
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("" : "+v"(words));      // (what only the end needs is read here, not in front of the loop)
+#endif
+        const StepConstants sc = step_constants<true>(x, words);
         v4i acc[A][B];
-        auto start = [&](const int32_t (&corr)[A]) {      // the sum starts from the channel's integer correction, once per tile
+        auto start = [&] {
 #pragma unroll
-            for (int a = 0; a < A; ++a) {
-                const int c0 = kk == 0 ? corr[a] : 0;
+            for (int a = 0; a < A; ++a)
 #pragma unroll
-                for (int b = 0; b < B; ++b) acc[a][b] = v4i{c0, c0, c0, c0};
-            }
+                for (int b = 0; b < B; ++b) acc[a][b] = v4i{0, 0, 0, 0};
         };
         auto put = [&](lds_v4i to) {
 #pragma unroll
@@ -725,28 +776,20 @@ __device__ __forceinline__ void conv_tiles(Ctx& x, lds_ptr lds) {
         };
         if (on) {
             if constexpr (PAIR) {
-                start(k2.corr);
+                start();
                 k_loop<A, B>(ring, src2, off2, x.lane, acc);
                 first_weights<A, B>(ring, src, x.lane);
+                first_pixels<A, B>(ring, src, off, x.lane);
                 put(part2);
             }
-            start(k.corr);
-            if (finishes) {
-                if (rows >= 4) load_residual<A, 4>(sc, oc, q);
-                else if (rows == 2) load_residual<A, 2>(sc, oc, q);
-                else load_residual<A, 1>(sc, oc, q);
-            }
+            start();
             k_loop<A, B>(ring, src, off, x.lane, acc);
-            if constexpr (kLate) load_constants<A>(sc.flags, PROG_TABLE_OF(uint8_t, x.words, constants), PROG_FIELD(x.words, OCp) * 4, oc, k);
+            if constexpr (kLate) load_constants<A>(sc.flags, PROG_TABLE_OF(uint8_t, words, constants), PROG_FIELD(words, OCp) * 4, oc, k);
             put(part);
         }
-        if (src.ks > 1) {
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-        }
+        if (src.ks > 1) meet();
         if (on && finishes) {
-            if (B == 4 || rows >= 4) {
+            if (B == 4 || rows == 4) {
                 for (int b = kk;;) {
                     finish_column<GELU, A, B, 4, PAIR>(sc, k, k2, mine, mine2, src.ks, b, 0, q, oc);
                     b += src.ks;
@@ -755,16 +798,11 @@ __device__ __forceinline__ void conv_tiles(Ctx& x, lds_ptr lds) {
                     load_residual<A, 4>(sc, oc, q);
                 }
             } else if constexpr (B < 4) {
-                if (rows == 2) finish_column<GELU, A, B, 2, PAIR>(sc, k, k2, mine, mine2, src.ks, col0, r0, q, oc);
-                else finish_column<GELU, A, B, 1, PAIR>(sc, k, k2, mine, mine2, src.ks, col0, r0, q, oc);
+                finish_column<GELU, A, B, 1, PAIR>(sc, k, k2, mine, mine2, src.ks, col0, r0, q, oc);
             }
         }
         base += per;
-        if (src.ks > 1 && base < t1) {
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-        }
+        if (src.ks > 1 && base < t1) meet();
     } while (base < t1);
 }
 
@@ -903,11 +941,6 @@ __device__ __forceinline__ void expand_depthwise(Ctx& x, lds_ptr lds) {
     }
     const uint32_t* pix = PROG_TABLE_OF(uint32_t, x.words, pixels);
     const int lane16 = x.lane & 15, quad = x.lane >> 4, c4 = x.tid & (4 * A - 1);
-    auto meet = [] {
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-    };
     int unit = t0;
     do {
         int ct, nb, n, band;
@@ -1376,11 +1409,6 @@ __device__ __forceinline__ void attention_units(const ProgAttention& s, Ctx& x, 
     const Buffer qb = make_buffer(x.place(s.q)), kb = make_buffer(x.place(s.k)), vb = make_buffer(x.place(s.v)), out = make_buffer(x.place(s.out));
     const float* mask = s.has_mask ? reinterpret_cast<const float*>(x.place(s.mask)) : nullptr;
     constexpr float kLog2e = 1.4426950408889634f;
-    auto meet = [] {
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-    };
     bool first = true;
     int u = x.rank;
     do {
@@ -1572,7 +1600,7 @@ __device__ __forceinline__ void attention_units(const ProgAttention& s, Ctx& x, 
 
 // ---- the program ------------------------------------------------------------------------------------------------------------
 // Three kernels, for networks over feature maps, for encoders, and for graphs with steps of both: every kind of step adds to the
-// registers of all others.  The 4 x 4 tiles ask for 250 and more vector registers, none is spilled to memory; 437, 422 and 696
+// registers of all others.  The 4 x 4 tiles ask for 250 and more vector registers, none is spilled to memory; 309, 286 and 541
 // scalar registers of the many step kinds are kept in lanes of vector registers.  The kernel with all kinds has no registers left for
 // 4 x 4 tiles (with them it spills); its convolutions take smaller ones (an encoder layer of 96 tokens beside a ResNet-50 of width
 // 16 at 64 x 64: 244 us, 467 by steps; beside a MobileNetV2 of 2 x 96 x 96 208 and 512).  A new step kind belongs into a kernel of its own where it
@@ -1729,9 +1757,9 @@ TileChoice choose_tile(int workgroups, int oc, int64_t pixels, int nk, int nk2, 
                 const double rate = std::max(waves * (a + b) * 11.4, std::max(1.0, waves / 4.0) * a * b * 14.6 + 2.7);
                 return std::max(n * rate, std::ceil(n / depth) * 431.0) + 1368.0;
             };
-            // a wave finishes whole columns of four pixels a lane, or part of one
-            const double rows = b == 4 ? 4.0 : std::min(4.0, std::max(1.0, 4.0 * b / ks)), columns = std::max(1.0, std::ceil(static_cast<double>(b) / ks));
-            const double writers = waves / ks * std::min(ks, b == 4 ? 4 : 4 * b);
+            // a wave finishes whole columns of four pixels a lane, or one of the four
+            const double rows = 4 * b <= ks ? 1.0 : 4.0, columns = std::max(1.0, std::ceil(static_cast<double>(b) / ks));
+            const double writers = waves / ks * std::min(ks, rows == 1.0 ? 4 * b : b);
             const double chain = (gelu ? 74.3 : 2.6) * rows * a + 376.0;
             const double epi = columns * (chain * std::max(5.8, writers) + rows * 10.6 * writers);
             const double meet = ks > 1 ? 354.0 + 67.6 * (waves * a * b / 8.0 + ks * a * columns * rows / 4.0) : 0.0;
@@ -1769,6 +1797,24 @@ ProgRef ProgBuilder::ref(const void* p) {
         off = v - io - (k << 40);
     }
     return {base, static_cast<uint32_t>(off), static_cast<uint32_t>(off >> 32)};
+}
+
+namespace {
+// the bytes from a tensor's first element to behind its last
+int64_t span_of(const hipie_tensor& t) {
+    const int64_t esize = t.dtype == HIPIE_F32 || t.dtype == HIPIE_I32 ? 4 : 1;
+    return ((t.n - 1) * t.stride_n + (t.h - 1) * t.stride_h + (t.w - 1) * t.stride_w + t.c) * esize;
+}
+}  // namespace
+
+void ProgBuilder::writes(const void* p, int64_t bytes) { writing.push_back({static_cast<const uint8_t*>(p), bytes}); }
+
+bool ProgBuilder::was_just_written(const void* p, const hipie_tensor& t) const {
+    const uint8_t* at = static_cast<const uint8_t*>(p);
+    const int64_t bytes = span_of(t);
+    for (const auto& w : written)
+        if (at < w.first + w.second && w.first < at + bytes) return true;
+    return false;
 }
 
 ProgPtr ProgBuilder::keep(const void* host, size_t bytes) {
@@ -1896,7 +1942,8 @@ bool ProgBuilder::expand_depthwise(const hipie_conv* first, const hipie_tensor& 
     std::array<int32_t, kProgramStepWords> w{};
     std::memcpy(w.data(), &c, sizeof c);
     std::memcpy(w.data() + kProgramStepWords / 2, &d, sizeof d);
-    steps.push_back(w);
+    writes(out.data, span_of(out));
+    push(w);
     return true;
 }
 
@@ -1920,10 +1967,18 @@ bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hip
         c.inv_c4 = 1.0f / static_cast<float>(c.c4);
         c.inv_quads = 1.0f / static_cast<float>(c.quads);
         c.inv_OH = 1.0f / static_cast<float>(c.OH);
+        writes(out.data, span_of(out));
         add(c);
         return true;
     }
     c.kind = PK_CONV;
+    // (a residual is loaded before the wait, so the step in front must not be the one that writes it: a step of no work goes between)
+    if (a.res != nullptr && !(a.flags & CF_RES_GEMM) && was_just_written(a.res, *residual)) {
+        ProgRows none{};
+        none.kind = PK_COPY;
+        none.in = none.out = ProgRef{0, 0, 0};
+        add(none);
+    }
     if (planes) c.out_sn = 4 * a.out_plane;
     c.nk = a.nk;
     const bool pair = (a.flags & CF_RES_GEMM) != 0;
@@ -1961,6 +2016,7 @@ bool ProgBuilder::conv(const hipie_conv* conv, const hipie_tensor& in, const hip
         pix[static_cast<size_t>(3 * pitch + i)] = pair ? at(a.in2_sn, a.in2_sh * a.conv2_sh, a.in2_sw * a.conv2_sw) : 0u;
     }
     c.pixels = keep(pix.data(), pix.size() * 4);
+    writes(out.data, span_of(out));
     add(c);
     return true;
 }
@@ -1995,6 +2051,7 @@ bool ProgBuilder::entry(const hipie_fq* fq, bool u8_in, const void* in, const hi
     e.in = ref(in);
     e.out = ref(out.data);
     e.tab = ptr(f.table);
+    writes(out.data, span_of(out));
     add(e);
     return true;
 }
@@ -2011,6 +2068,7 @@ bool ProgBuilder::pool(const PoolArgs& a, bool avg, bool rcp) {
     p.in = ref(a.in);
     p.out = ref(a.out);
     p.a = a;
+    writes(a.out, static_cast<int64_t>(a.M / a.OHOW) * 4 * a.out_sn);
     add(p);
     return true;
 }
@@ -2044,6 +2102,7 @@ bool ProgBuilder::embed(const float* table, int64_t vocab, int64_t hidden, const
     e.table = ptr(table);
     e.add0 = ptr(add0);
     e.add1 = ptr(add1);
+    writes(out, tokens * hidden * 4);
     add(e);
     return true;
 }
@@ -2066,6 +2125,8 @@ bool ProgBuilder::mvn(const void* in, void* out, void* outq, int64_t rows, int64
     m.beta = ptr(beta);
     if (outq) m.fq = make_requant(rq, "single-launch program");
     if (outq && !m.fq.rcp) return false;
+    if (out) writes(out, rows * axis * 4);
+    if (outq) writes(outq, rows * axis);
     add(m);
     return true;
 }
@@ -2115,6 +2176,7 @@ bool ProgBuilder::attention(const hipie_attention* att, const void* const (&qkv)
         }
     }
     if (best >= 1e30) return false;
+    writes(out, 4 * (batch_outer * oo + batch * so + proto.S * ldo));
     add(s);
     return true;
 }
@@ -2130,6 +2192,7 @@ bool ProgBuilder::fq_rows(const hipie_fq* fq, const void* in, void* out, int out
     r.p = f.first;
     r.lm1 = f.lm1;
     r.off = f.off;
+    writes(out, n);
     add(r);
     return true;
 }
@@ -2141,6 +2204,7 @@ bool ProgBuilder::copy(const void* in, void* out, int64_t bytes) {
     r.n = bytes;
     r.in = ref(in);
     r.out = ref(out);
+    writes(out, bytes);
     add(r);
     return true;
 }

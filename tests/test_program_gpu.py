@@ -96,6 +96,31 @@ def test_single_launch_equals_steps(name):
             assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
 
 
+@pytest.mark.parametrize("workgroups", ["64", "256"])
+@pytest.mark.parametrize("n,hw,c,signed", [(1, 5, 8, False), (1, 28, 72, True), (3, 14, 130, False), (4, 56, 64, False)])
+def test_a_residual_of_the_step_in_front_equals_steps(n, hw, c, signed, workgroups):
+    """a convolution asks for its residual before it waits for the step in front: here that one writes it, as bytes and as f32"""
+    rng = np.random.default_rng(hw)
+    net = builders.QuantizedNet()
+    g = net.g
+
+    def weights(k):
+        return (rng.standard_normal((c, c, k, k), dtype=np.float32) * np.float32(0.05)).astype(np.float32), \
+            (rng.standard_normal(c, dtype=np.float32) * np.float32(0.1)).astype(np.float32)
+
+    a = net.conv(net.input("data", (n, c, hw, hw), 2.0), *weights(3), out_high=2.0, pads=(1, 1), signed=signed)
+    y = g.add(net.conv_f32(a, *weights(1)), net.dequantize(a))
+    b = net.requantize(y, 2.0, signed=True)
+    z = g.add(net.conv_f32(b, *weights(1)), y)
+    g.result(z, "out")
+    steps, single = _compile(g, "NO"), _compile(g, workgroups)
+    assert single.config("HIP_SINGLE_LAUNCH") == workgroups
+    one, other = steps.create_request(), single.create_request()
+    for seed in range(3):
+        for x, v in zip(_infer(one, seed), _infer(other, seed)):
+            assert np.array_equal(x.view(np.uint8), v.view(np.uint8))
+
+
 @pytest.mark.parametrize("name", ["block_1x3x7", "block_3x64x14", "resnet_3_u8", "mobilenet_1x160", "encoder_3x96", "encoder_and_resnet"])
 def test_results_are_there_when_the_call_returns(name):
     """The call returns by the launch's own word, before its stream has drained: results are read on another stream at once, by a
