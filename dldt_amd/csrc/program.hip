@@ -1394,8 +1394,7 @@ __host__ __device__ constexpr int attention_exchange(int S, int split) {
     return k > ctx ? (k > e ? k : e) : (ctx > e ? ctx : e);
 }
 __host__ __device__ constexpr int attention_lds(int S, int split) { return 64 * (S + 16) + attention_exchange(S, split) + 4 * S + 8 * 32 * 4 + 8 * 64 * 4; }
-// LONG: the Softmax of rows longer than kPlainSoftmax.
-template <bool LONG, int PFORM>
+template <int PFORM>
 __device__ __forceinline__ void attention_units(const ProgAttention& s, Ctx& x, lds_ptr lds) {
     typedef __attribute__((address_space(3))) float* lds_f32;
     typedef float v4f __attribute__((ext_vector_type(4)));
@@ -1493,11 +1492,9 @@ __device__ __forceinline__ void attention_units(const ProgAttention& s, Ctx& x, 
             meet();
             for (int k = 0; k < split; ++k) m = fmaxf(m, sMax[(block * split + k) * 32 + l32]);
         }
-        // exponentials, and their sum: a lane's one behind the other (LONG: sums of four, and the tree over them of the stand-alone
-        // Softmax)
+        // exponentials, and their sum: a lane's one behind the other
         const float mL = -m * kLog2e;
         const lds_v4f sE = (lds_v4f)sK + block * nt * 4 * 64 + x.lane;   // [tile][group of four][64]
-        const lds_f32 sE4 = (lds_f32)sK + block * nt * 4 * 64 + x.lane;
         float sum = 0.f;
 #pragma unroll
         for (int j = 0; j < kMostTiles; ++j) {
@@ -1507,41 +1504,22 @@ __device__ __forceinline__ void attention_units(const ProgAttention& s, Ctx& x, 
             for (int g = 0; g < 4; ++g) {
 #pragma unroll
                 for (int r = 4 * g; r < 4 * g + 4; ++r) {
-                    v[j][r] = LONG ? expf(v[j][r] - m) : __builtin_amdgcn_exp2f(fmaf(v[j][r], kLog2e, mL));
-                    if (!LONG) sum += v[j][r];
+                    v[j][r] = __builtin_amdgcn_exp2f(fmaf(v[j][r], kLog2e, mL));
+                    sum += v[j][r];
                 }
-                if constexpr (LONG) sE4[(4 * t + g) * 64] = (v[j][4 * g] + v[j][4 * g + 1]) + (v[j][4 * g + 2] + v[j][4 * g + 3]);
-                else if (split > 1) sE[(4 * t + g) * 64] = v4f{v[j][4 * g], v[j][4 * g + 1], v[j][4 * g + 2], v[j][4 * g + 3]};
+                if (split > 1) sE[(4 * t + g) * 64] = v4f{v[j][4 * g], v[j][4 * g + 1], v[j][4 * g + 2], v[j][4 * g + 3]};
             }
         }
         if (split > 1) {
             meet();
             if (on && w == 0) {
-                if constexpr (LONG) {
-                    float p[8][4];
+                sum = 0.f;
+                for (int t = 0; t < nt; ++t)
 #pragma unroll
-                    for (int t = 0; t < 8; ++t)
-#pragma unroll
-                        for (int g = 0; g < 4; ++g) {
-                            p[t][g] = sE4[(4 * t + g) * 64];
-                            if (t + 8 < nt) p[t][g] += sE4[(4 * (t + 8) + g) * 64];
-                        }
-#pragma unroll
-                    for (int o = 4; o > 0; o >>= 1)
-#pragma unroll
-                        for (int t = 0; t < o; ++t)
-#pragma unroll
-                            for (int g = 0; g < 4; ++g) p[t][g] += p[t + o][g];
-                    sum = (p[0][0] + p[0][2]) + (p[0][1] + p[0][3]);
-                } else {
-                    sum = 0.f;
-                    for (int t = 0; t < nt; ++t)
-#pragma unroll
-                        for (int g = 0; g < 4; ++g) {
-                            const v4f e = sE[(4 * t + g) * 64];
-                            sum += e.x; sum += e.y; sum += e.z; sum += e.w;
-                        }
-                }
+                    for (int g = 0; g < 4; ++g) {
+                        const v4f e = sE[(4 * t + g) * 64];
+                        sum += e.x; sum += e.y; sum += e.z; sum += e.w;
+                    }
                 sSum[0] = sum;
             }
             meet();
@@ -1560,7 +1538,7 @@ __device__ __forceinline__ void attention_units(const ProgAttention& s, Ctx& x, 
             for (int g = 0; g < 4; ++g) {
                 float p[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) p[r] = LONG ? quotient(v[j][4 * g + r], sum, inv) : v[j][4 * g + r] * inv;
+                for (int r = 0; r < 4; ++r) p[r] = v[j][4 * g + r] * inv;
                 pf[g] = static_cast<int>(prob_levels4<true, PFORM>(a, p[0], p[1], p[2], p[3]));
             }
             // u8 probabilities q are stored as q - 128: the 128 that is missing from each, as twice 64
@@ -1598,9 +1576,209 @@ __device__ __forceinline__ void attention_units(const ProgAttention& s, Ctx& x, 
     } while (u < s.units);
 }
 
+// Softmax of rows longer than kPlainSoftmax: eight waves for 32 queries, up to two tiles of keys a wave.  A tile's keys are the operand
+// of one wave, so they come straight from memory, and its values go through LDS of the wave's own for their transposition: nothing
+// of either is waited for together.  A workgroup's units lie one behind the other, so that most of them find keys and values where
+// the unit before left them, and their queries are requested a unit ahead.  (With keys and values of a head in LDS for all waves,
+// requested by all of them for every unit, staging was 2.3 of a unit's 8.4 us at 512 keys, and the waves met six times, now three:
+// an encoder of 6 layers x 3 x 512 tokens took 592 us with 256 workgroups and 1387 with 64, and takes 563 and 1248.  At 128 keys, where
+// a workgroup has one unit and half of its waves a tile, staging by all eight is the faster: 7.0 us a step, 7.8 so.)
+__device__ __forceinline__ void attention_long(const ProgAttention& s, Ctx& x, lds_ptr lds) {
+    typedef __attribute__((address_space(3))) float* lds_f32;
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) v4f* lds_v4f;
+    constexpr int kTiles = 2, kPitch = 32 * kTiles + 16, kValues = 64 * kPitch + 32;      // of a wave: values, transposed
+    constexpr int kMaskAt = 8 * kValues, kMaxAt = kMaskAt + 8 * kTiles * 128, kSumAt = kMaxAt + 8 * 128, kCtxAt = kSumAt + 8 * 1024;
+    static_assert(kCtxAt + 64 * 1024 <= kPartBytes + kKoffBytes, "LDS");
+    const AttentionArgs& a = s.a;
+    const int S = s.S, nt = S / 32, w = x.wave;
+    const lds_ptr sVT = lds + w * kValues;                              // (every 16 rows 16 bytes on: no two of a wave's words in one bank)
+    const lds_f32 sMask = (lds_f32)(lds + kMaskAt) + w * 32 * kTiles, sMax = (lds_f32)(lds + kMaxAt);
+    const lds_v4i sCtx = (lds_v4i)(lds + kCtxAt);                       // [wave][8 groups of 4 registers][64]
+    const Buffer qb = make_buffer(x.place(s.q)), kb = make_buffer(x.place(s.k)), vb = make_buffer(x.place(s.v)), out = make_buffer(x.place(s.out));
+    const float* mask = s.has_mask ? reinterpret_cast<const float*>(x.place(s.mask)) : nullptr;
+    const uint32_t units = static_cast<uint32_t>(s.units);
+    int u = static_cast<int>((static_cast<uint32_t>(x.rank) * units) >> x.wg_shift);
+    const int end = static_cast<int>((static_cast<uint32_t>(x.rank + 1) * units) >> x.wg_shift);
+    v4i kf[kTiles][2], qf[2];
+    // (element, head, first query) of a unit: divisions, so they are done a unit ahead
+    auto place = [&](int unit, int& eh, int& n, int& hd, int& q0) {
+        eh = unit / s.parts;
+        n = eh / s.heads;
+        hd = eh - n * s.heads;
+        q0 = 32 * (unit - eh * s.parts);
+    };
+    int eh, n, hd, q0, have = -1;             // (have: whose keys and values are held)
+    place(min(u, s.units - 1), eh, n, hd, q0);
+    do {
+        int lane = x.lane;
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("" : "+v"(lane));       // (its functions are not kept in registers around the loop)
+#endif
+        const int l32 = lane & 31, h = lane >> 5;
+        auto load_queries = [&] {
+            const uint32_t row = static_cast<uint32_t>(n * a.oq + hd * a.sq) + static_cast<uint32_t>((q0 + l32) * a.ldq + 16 * h);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) qf[i] = shared16(qb, row + 32 * i);
+        };
+        const bool fresh = eh != have;
+        const uint32_t orow = static_cast<uint32_t>(n * a.oo + hd * a.so) + static_cast<uint32_t>((q0 + l32) * a.ldo);
+        const uint32_t krow = static_cast<uint32_t>(n * a.ok + hd * a.sk) + static_cast<uint32_t>(l32 * a.ldk + 16 * h);
+        const uint32_t vrow = static_cast<uint32_t>(n * a.ov + hd * a.sv) + static_cast<uint32_t>(8 * (lane >> 4) * a.ldv + 4 * (lane & 15));
+        float mk = 0.f;
+        if (fresh && mask) mk = mask[n * a.mask_outer + hd * a.mask_inner + min(32 * (w + 8 * h) + l32, S - 1)];
+        if (have < 0) {
+            x.wait();
+            if (u >= end) return;
+            load_queries();
+        }
+        have = eh;
+        // a tile's keys, and its values as 4 keys x 4 d: everything is requested before any of it is used
+        uint32_t vw[kTiles][2][4];
+        if (fresh) {
+#pragma unroll
+            for (int j = 0; j < kTiles; ++j) {
+                const int t = w + 8 * j;
+                if (t >= nt) continue;
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) kf[j][ks] = shared16(kb, krow + static_cast<uint32_t>(32 * t * a.ldk + 32 * ks));
+            }
+#pragma unroll
+            for (int j = 0; j < kTiles; ++j) {
+                const int t = w + 8 * j;
+                if (t >= nt) continue;
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        vw[j][i][q] = shared4(vb, vrow + static_cast<uint32_t>((32 * t + 4 * i + q) * a.ldv));
+            }
+            if (mask) sMask[32 * h + l32] = mk;
+        }
+        // the scores of this wave's tiles and their maximum
+        float v[kTiles][16];
+        float m = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < kTiles; ++j) {
+            const int t = w + 8 * j;
+            if (t >= nt) continue;
+            v16i acc = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[j][ks], qf[ks], acc, 0, 0, 0);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                v4f mg = {0.f, 0.f, 0.f, 0.f};
+                if (s.has_mask) mg = *(lds_v4f)(sMask + 32 * j + 8 * g + 4 * h);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float y = static_cast<float>(acc[4 * g + r]) * a.scale1;
+                    if (s.has_mask) y = y + mg[r];
+                    v[j][4 * g + r] = y;
+                    m = fmaxf(m, y);
+                }
+            }
+        }
+        if (u + 1 < end) {
+            place(u + 1, eh, n, hd, q0);
+            load_queries();
+        }
+        if (fresh) {
+#pragma unroll
+            for (int j = 0; j < kTiles; ++j) {
+                if (w + 8 * j >= nt) continue;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const uint32_t* y = vw[j][i];
+                    const uint32_t lo01 = __builtin_amdgcn_perm(y[1], y[0], 0x05010400u), hi01 = __builtin_amdgcn_perm(y[1], y[0], 0x07030602u);
+                    const uint32_t lo23 = __builtin_amdgcn_perm(y[3], y[2], 0x05010400u), hi23 = __builtin_amdgcn_perm(y[3], y[2], 0x07030602u);
+                    const uint32_t t[4] = {__builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
+                                           __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u)};
+                    const int d = 4 * (lane & 15);      // (keys in the order in which their scores leave the matrix unit)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) *(lds_i32)(sVT + (d + q) * kPitch + 16 * (d >> 4) + 32 * j + 16 * i + 4 * (lane >> 4)) = static_cast<int32_t>(t[q]);
+                }
+            }
+        }
+        m = fmaxf(m, __shfl_xor(m, 32, 64));
+        sMax[w * 32 + l32] = m;                     // (the same in both halves of the wave)
+        meet();
+#pragma unroll
+        for (int k = 0; k < 8; ++k) m = fmaxf(m, sMax[k * 32 + l32]);
+        // exponentials, their sums of four, and the tree over them of the stand-alone Softmax, whose first level, tiles t and t + 8, is
+        // within a wave
+        float e4[kTiles][4] = {};
+#pragma unroll
+        for (int j = 0; j < kTiles; ++j) {
+            if (w + 8 * j >= nt) continue;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+#pragma unroll
+                for (int r = 4 * g; r < 4 * g + 4; ++r) v[j][r] = expf(v[j][r] - m);
+                e4[j][g] = (v[j][4 * g] + v[j][4 * g + 1]) + (v[j][4 * g + 2] + v[j][4 * g + 3]);
+            }
+        }
+        const lds_v4f sSum = (lds_v4f)(lds + kSumAt) + lane;
+        v4f p8[8];
+        sSum[w * 64] = v4f{e4[0][0] + e4[1][0], e4[0][1] + e4[1][1], e4[0][2] + e4[1][2], e4[0][3] + e4[1][3]};
+        meet();
+#pragma unroll
+        for (int t = 0; t < 8; ++t) p8[t] = sSum[t * 64];
+#pragma unroll
+        for (int o = 4; o > 0; o >>= 1)
+#pragma unroll
+            for (int t = 0; t < o; ++t)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) p8[t][g] = p8[t][g] + p8[t + o][g];
+        float sum = (p8[0][0] + p8[0][2]) + (p8[0][1] + p8[0][3]);
+        sum += __shfl_xor(sum, 32, 64);
+        const float inv = 1.0f / sum;
+        // probabilities -> levels -> this wave's part of the second product
+        v16i ctx[2] = {{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}};
+#pragma unroll
+        for (int j = 0; j < kTiles; ++j) {
+            const int t = w + 8 * j;
+            if (t >= nt) continue;
+            v4i pf = {0, 0, 0, 0};
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                float p[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) p[r] = quotient(v[j][4 * g + r], sum, inv);
+                pf[g] = static_cast<int>(prob_levels4<true, 0>(a, p[0], p[1], p[2], p[3]));
+            }
+            // u8 probabilities q are stored as q - 128: the 128 that is missing from each, as twice 64
+            const int n64 = a.p_bias ? 0x40404040 : 0;
+            const v4i bias = {n64, n64, n64, n64};
+#pragma unroll
+            for (int db = 0; db < 2; ++db) {
+                const v4i vf = *(lds_v4i)(sVT + (32 * db + l32) * kPitch + 16 * (2 * db + (l32 >> 4)) + 32 * j + 16 * h);
+                ctx[db] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf, pf, ctx[db], 0, 0, 0);
+                if (a.p_bias) {
+                    ctx[db] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf, bias, ctx[db], 0, 0, 0);
+                    ctx[db] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf, bias, ctx[db], 0, 0, 0);
+                }
+            }
+        }
+        // the waves' integer sums meet; each finishes one of eight groups of four registers
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            sCtx[(w * 8 + i) * 64 + lane] = v4i{ctx[i >> 2][4 * (i & 3)], ctx[i >> 2][4 * (i & 3) + 1], ctx[i >> 2][4 * (i & 3) + 2], ctx[i >> 2][4 * (i & 3) + 3]};
+        meet();
+        v4i c = {0, 0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < 8; ++k) c += sCtx[(k * 8 + w) * 64 + lane];
+        const int d = 32 * (w >> 2) + 8 * (w & 3) + 4 * h;
+        const float4 o = make_float4(static_cast<float>(c.x) * a.scale2, static_cast<float>(c.y) * a.scale2, static_cast<float>(c.z) * a.scale2,
+                                     static_cast<float>(c.w) * a.scale2);
+        if (a.fq_o.levels) publish4(out, orow + d, levels4(a.fq_o, o));
+        else publish16f(out, 4u * (orow + d), o);
+        // (the next unit's maxima, sums and partial sums are written behind meetings that the readers of this one's have passed as well)
+    } while (++u < end);
+}
+
 // ---- the program ------------------------------------------------------------------------------------------------------------
 // Three kernels, for networks over feature maps, for encoders, and for graphs with steps of both: every kind of step adds to the
-// registers of all others.  The 4 x 4 tiles ask for 250 and more vector registers, none is spilled to memory; 309, 286 and 541
+// registers of all others.  The 4 x 4 tiles ask for 250 and more vector registers, none is spilled to memory; 309, 260 and 556
 // scalar registers of the many step kinds are kept in lanes of vector registers.  The kernel with all kinds has no registers left for
 // 4 x 4 tiles (with them it spills); its convolutions take smaller ones (an encoder layer of 96 tokens beside a ResNet-50 of width
 // 16 at 64 x 64: 244 us, 467 by steps; beside a MobileNetV2 of 2 x 96 x 96 208 and 512).  A new step kind belongs into a kernel of its own where it
@@ -1676,9 +1854,9 @@ __global__ __launch_bounds__(kProgramThreads, 1) void program_kernel(const ProgA
                 else if (kind == PK_MVN) mvn_rows(unpack<ProgMvn>(words), x);
                 else if (!MAPS || kind == PK_ATTENTION) {
                     const ProgAttention t = unpack<ProgAttention>(words);
-                    if (t.S > kPlainSoftmax) attention_units<true, 0>(t, x, lds);
-                    else if (t.pform == 2) attention_units<false, 2>(t, x, lds);
-                    else attention_units<false, 0>(t, x, lds);
+                    if (t.S > kPlainSoftmax) attention_long(t, x, lds);
+                    else if (t.pform == 2) attention_units<2>(t, x, lds);
+                    else attention_units<0>(t, x, lds);
                 }
             }
             if constexpr (!MAPS) break;
@@ -2165,7 +2343,7 @@ bool ProgBuilder::attention(const hipie_attention* att, const void* const (&qkv)
     for (int shift = 0; (1 << shift) <= kMostSplit; ++shift) {
         const int split = 1 << shift, blocks = std::min(kMostSplit / split, qt);
         const int64_t tiles = ceil_div(qt, split), parts = ceil_div(qt, kMostSplit / split), rounds = ceil_div(elements * parts, workgroups);
-        if (tiles > kMostTiles || attention_lds(proto.S, split) > kPlainAt) continue;
+        if (tiles > kMostTiles || attention_lds(proto.S, split) > kPartBytes + kKoffBytes || (proto.S > kPlainSoftmax && split < kMostSplit)) continue;
         const double waves = static_cast<double>(blocks * std::min(split, qt));
         const double t = static_cast<double>(rounds) * (5000.0 + 4.0 * proto.S + std::max(1.0, waves / 5.0) * static_cast<double>(tiles) * 2400.0);
         if (t < best) {

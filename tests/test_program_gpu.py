@@ -121,6 +121,33 @@ def test_a_residual_of_the_step_in_front_equals_steps(n, hw, c, signed, workgrou
             assert np.array_equal(x.view(np.uint8), v.view(np.uint8))
 
 
+@pytest.mark.parametrize("workgroups", ["64", "128", "256"])
+@pytest.mark.parametrize("batch,seq,masked", [(1, 448, False), (2, 448, True), (3, 512, True), (5, 448, True)])
+def test_long_rows_whose_workgroups_cross_heads_and_elements_equal_steps(batch, seq, masked, workgroups):
+    """keys, values and mask stay with a workgroup until its next unit is of another head or element: each has a mask of its own"""
+    g = builders.bert_encoder(layers=1, batch=batch, seq=seq, vocab=100, mask=masked)[0]
+    steps, single = _compile(g, "NO"), _compile(g, workgroups)
+    assert single.config("HIP_SINGLE_LAUNCH") == workgroups
+    results = []
+    for plan in (steps, single):
+        req = plan.create_request()
+        ins, outs = req.device_buffers()
+        _fill(ins, 7)
+        if masked:
+            keep = torch.arange(seq, device="cuda").view(1, 1, 1, seq) < torch.tensor([seq, 1, seq // 3, 33, seq - 1][:batch], device="cuda").view(batch, 1, 1, 1)
+            ins[1].copy_(torch.where(keep, 0.0, -10000.0))
+        torch.cuda.synchronize()
+        for _ in range(2):
+            for o in outs:
+                o.fill_(float("nan"))
+            torch.cuda.synchronize()
+            req.infer_device(ins, outs)
+            results.append([o.cpu().numpy() for o in outs])
+    for got in results[1:]:
+        for x, y in zip(results[0], got):
+            assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
+
+
 @pytest.mark.parametrize("name", ["block_1x3x7", "block_3x64x14", "resnet_3_u8", "mobilenet_1x160", "encoder_3x96", "encoder_and_resnet"])
 def test_results_are_there_when_the_call_returns(name):
     """The call returns by the launch's own word, before its stream has drained: results are read on another stream at once, by a
