@@ -22,7 +22,7 @@ struct AttentionArgs {
     int p_div2;                                       // ... verified against IEEE division on the device
     int p_sat;                                        // input_low of the probabilities' FakeQuantize is +0 and it has 256 levels
     int p_inside;                                     // ... or input_low <= 0 and input_high >= 1: a probability never leaves the interval
-    int qblocks;                                      // blocks of 128 queries per batch element
+    int qblocks;                                      // workgroups (128 queries, beyond kPlainSoftmax keys 64) per batch element
     int xcd_groups;                                   // 1: a one-dimensional grid that keeps the blocks of two neighbouring batch elements on one XCD
 #ifdef HIPIE_ATT_STAMPS
     long long* stamps;                                // probe builds only: cycle stamps per workgroup

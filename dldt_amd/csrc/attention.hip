@@ -19,19 +19,14 @@
 namespace hipie {
 namespace {
 
-// A lane holds S / 2 scores in registers: up to 384 keys two waves share a SIMD, up to 512 (192 more registers than the
-// accumulators and operands take) one has it to itself.  An instance per length: in steps of 32 keys to 384, of 64 beyond.
-// 3 x 12 heads x 512 keys with a mask: 28.6 us.  Each of the 576 waves has a SIMD to itself and issues 8700 vector
-// instructions (exp and quotient of 9.4 million scores), half of its cycles; the matrix pipe is busy for 3 %.  Kernels of their
-// own, with 38 MB of scores between them, take 75 us: the products 12.8 and 11.0, the mask's Add 28.4, the Softmax 14.6, the
-// transpose of V 7.9.
+// A lane holds S / 2 scores in registers, up to 384 keys: two waves share a SIMD.  An instance per length, in steps of 32 keys
+// (attention_long_kernel: in steps of 64 from there to 512).
 constexpr int kMaxSeq = 512;
 constexpr int kHeadDim = 64;
 
 template <int NT, bool DIV2, bool MASK, int PFORM>   // NT = S / 32 key tiles
-__global__ __launch_bounds__(256, NT * 32 <= kPlainSoftmax ? 2 : 1) void attention_kernel(const AttentionArgs a) {
+__global__ __launch_bounds__(256, 2) void attention_kernel(const AttentionArgs a) {
     constexpr int S = NT * 32;
-    constexpr bool kLong = S > kPlainSoftmax;
     constexpr int VT_LD = S + 16;                     // odd number of 16-byte groups per row: conflict-free
     __shared__ __attribute__((aligned(16))) int8_t sK[S * 64];       // [key][d], chunk c of row r in slot c ^ ((r >> 2) & 3)
     __shared__ __attribute__((aligned(16))) int8_t sVT[64 * VT_LD];  // [d][tile][half][j]: key 32 t + 8 (j / 4) + 4 half + j % 4
@@ -181,12 +176,11 @@ __global__ __launch_bounds__(256, NT * 32 <= kPlainSoftmax ? 2 : 1) void attenti
         }
     };
     // probabilities of a tile -> levels -> second product
-    auto finish_tile = [&](int t, const float (&e)[16], float sum, float inv) {
+    auto finish_tile = [&](int t, const float (&e)[16], float inv) {
         v4i pf;
-        auto prob = [&](int r) { return kLong ? quotient(e[r], sum, inv) : e[r] * inv; };
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const float4 p4 = make_float4(prob(4 * g), prob(4 * g + 1), prob(4 * g + 2), prob(4 * g + 3));
+            const float4 p4 = make_float4(e[4 * g] * inv, e[4 * g + 1] * inv, e[4 * g + 2] * inv, e[4 * g + 3] * inv);
             if (a.probs && q_ok)
                 *reinterpret_cast<float4*>(a.probs + dump_row + 32 * t + 8 * g + 4 * h) = p4;
             pf[g] = static_cast<int>(prob_levels4<DIV2, PFORM>(a, p4.x, p4.y, p4.z, p4.w));
@@ -217,41 +211,20 @@ __global__ __launch_bounds__(256, NT * 32 <= kPlainSoftmax ? 2 : 1) void attenti
     // reciprocal of the sum: within the tolerance the stand-alone kernel is held to.
     m = fmaxf(m, __shfl_xor(m, 32, 64));
     float s = 0.f;
-    if constexpr (kLong) {
-        // four keys, then the chunks of 8 tiles, then halves of the groups (tile bits 2, 1, 0, g bits 1, 0, h)
-        float part[8][4];
+    const float mL = -m * kLog2e;
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-#pragma unroll
-                for (int r = 4 * g; r < 4 * g + 4; ++r) x[t][r] = expf(x[t][r] - m);
-                const float e4 = (x[t][4 * g] + x[t][4 * g + 1]) + (x[t][4 * g + 2] + x[t][4 * g + 3]);
-                part[t % 8][g] = t < 8 ? e4 : part[t % 8][g] + e4;
-            }
-#pragma unroll
-        for (int o = 4; o > 0; o >>= 1)
-#pragma unroll
-            for (int t = 0; t < o; ++t)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) part[t][g] += part[t + o][g];
-        s = (part[0][0] + part[0][2]) + (part[0][1] + part[0][3]);
-    } else {
-        const float mL = -m * kLog2e;
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                x[t][r] = __builtin_amdgcn_exp2f(fmaf(x[t][r], kLog2e, mL));
-                s += x[t][r];
-            }
-    }
+        for (int r = 0; r < 16; ++r) {
+            x[t][r] = __builtin_amdgcn_exp2f(fmaf(x[t][r], kLog2e, mL));
+            s += x[t][r];
+        }
     s += __shfl_xor(s, 32, 64);
     const float inv = 1.0f / s;
     // probabilities -> i8 levels -> second product, one 32-key tile at a time
     init_ctx();
 #pragma unroll
-    for (int t = 0; t < NT; ++t) finish_tile(t, x[t], s, inv);
+    for (int t = 0; t < NT; ++t) finish_tile(t, x[t], inv);
 
     ATT_STAMP(5);
     // ---- context of query q_row: d = 32 db + 8 (r / 4) + 4 h + r % 4 --------------------------------
@@ -269,16 +242,198 @@ __global__ __launch_bounds__(256, NT * 32 <= kPlainSoftmax ? 2 : 1) void attenti
         }
 }
 
+// Rows longer than kPlainSoftmax, a multiple of 64 keys: 16 queries a wave, 64 a workgroup.  A lane holds a quarter of one query's
+// scores, so that two waves share a SIMD (with 32 queries and half of the scores a wave had it to itself) and twice as many
+// workgroups spread evenly.  Vector issue bounds it: exp and quotient of every score, half of the cycles of a lone wave.  us before / now,
+// with a mask: 12 heads x 512 keys 24.0 / 14.0, 36 x 512 24.7 / 19.9, 96 x 448 42.2 / 27.7, 384 x 512 138.5 / 99.5; an encoder of 4 layers x 8 x 448 tokens with
+// three requests in flight 338 / 315.  Kernels of their own for 36 x 512, with 38 MB of scores between them, take 75: the products 12.8
+// and 11.0, the mask's Add 28.4, the Softmax 14.6, the transpose of V 7.9.
+// Up to kPlainSoftmax keys it takes less as well where it has the device to itself (192 heads x 384: 28.9 / 24.6), but more beside others: the sum goes through
+// its keys one by one, which two lanes can only do one after the other, and K and V are staged by twice as many workgroups.  An encoder
+// of 12 layers x 16 x 384 tokens takes 2012 / 1955 alone and 1352 / 1372 with three requests in flight.
+// Lane group g = lane / 16 holds rows 4 g + r of every 16-row tile of the first product: keys in order, the last two levels of the
+// sum's tree are exchanges.  A group's four tiles in a row are 64 keys of the second product, in the order of V^T in LDS.
+template <int NI, bool DIV2, bool MASK, int PFORM>   // NI = S / 16 tiles of keys
+__global__ __launch_bounds__(256, 2) void attention_long_kernel(const AttentionArgs a) {
+    constexpr int S = NI * 16;
+    constexpr int VT_LD = S + 16;
+    __shared__ __attribute__((aligned(16))) int8_t sK[S * 64];       // [key][d], chunk c of row r in slot c ^ ((r >> 2) & 3)
+    __shared__ __attribute__((aligned(16))) int8_t sVT[64 * VT_LD];  // [d][four tiles][lane group][tile][r]
+    __shared__ __attribute__((aligned(16))) float sMask[MASK ? S : 4];
+    __shared__ __attribute__((aligned(16))) int32_t sVsum[64];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int l16 = lane & 15, grp = lane >> 4;
+    int qblk = blockIdx.x, b = blockIdx.y;
+    if (a.xcd_groups) {
+        const int id = blockIdx.x, per = 2 * a.qblocks, k = id >> 3, sub = k % per;
+        b = ((k / per) * 8 + (id & 7)) * 2 + sub / a.qblocks;
+        qblk = sub % a.qblocks;
+    }
+    const int bo = b / a.batch_inner, bi = b - bo * a.batch_inner;
+    const int8_t* qp = a.q + bo * a.oq + bi * a.sq;
+    const int8_t* kp = a.k + bo * a.ok + bi * a.sk;
+    const int8_t* vp = a.v + bo * a.ov + bi * a.sv;
+
+    constexpr int KI = (S * 4 + 255) / 256;
+    v4i kx[KI];
+    uint32_t vw[KI][4];
+#pragma unroll
+    for (int j = 0; j < KI; ++j) {
+        const int i = min(tid + j * 256, S * 4 - 1);
+        kx[j] = *reinterpret_cast<const v4i*>(kp + (i >> 2) * a.ldk + (i & 3) * 16);
+    }
+#pragma unroll
+    for (int j = 0; j < KI; ++j) {
+        const int i = min(tid + j * 256, S * 4 - 1);
+        const int d4 = i & 15, kq = i >> 4;            // 4 consecutive keys x 4 consecutive d
+#pragma unroll
+        for (int q = 0; q < 4; ++q) vw[j][q] = *reinterpret_cast<const uint32_t*>(vp + (4 * kq + q) * a.ldv + 4 * d4);
+    }
+    const int q_row = qblk * 64 + wave * 16 + l16;
+    const v4i qf = *reinterpret_cast<const v4i*>(qp + static_cast<int64_t>(q_row) * a.ldq + 16 * grp);
+    if (a.p_bias) {
+        if (tid < 64) sVsum[tid] = 0;
+        __syncthreads();
+    }
+#pragma unroll
+    for (int j = 0; j < KI; ++j) {
+        const int i = tid + j * 256;
+        if (i < S * 4) {
+            const int r = i >> 2, c = i & 3;
+            *reinterpret_cast<v4i*>(&sK[r * 64 + ((c ^ ((r >> 2) & 3)) * 16)]) = kx[j];
+        }
+    }
+    int32_t vsum[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < KI; ++j) {
+        const int i = tid + j * 256;
+        if (i >= S * 4) continue;
+        const int d4 = i & 15, kq = i >> 4;
+        const uint32_t* w = vw[j];
+        const uint32_t lo01 = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u);   // 4 x 4 bytes transposed, as above
+        const uint32_t hi01 = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u);
+        const uint32_t lo23 = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u);
+        const uint32_t hi23 = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
+        const uint32_t t[4] = {__builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
+                               __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u)};
+        const int col = (kq >> 4) * 64 + (kq & 3) * 16 + ((kq >> 2) & 3) * 4;       // tile kq / 4, lane group kq % 4
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            *reinterpret_cast<uint32_t*>(&sVT[(4 * d4 + e) * VT_LD + col]) = t[e];
+            vsum[e] = __builtin_amdgcn_sdot4(static_cast<int>(t[e]), 0x01010101, vsum[e], false);
+        }
+    }
+    if (a.p_bias) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) atomicAdd(&sVsum[4 * (tid & 15) + e], vsum[e]);
+    }
+    if constexpr (MASK) {
+        const float* mrow = a.mask + bo * a.mask_outer + bi * a.mask_inner;
+        for (int i = tid; i < S; i += 256) sMask[i] = mrow[i];
+    }
+    __syncthreads();
+
+    const int64_t dump_row = (static_cast<int64_t>(b) * a.S + q_row) * a.S;   // [batch][query][key]
+    const int slot = (grp ^ (l16 >> 2)) * 16;
+    float x[NI][4];
+    float m = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const v4i kf = *reinterpret_cast<const v4i*>(&sK[(16 * i + l16) * 64 + slot]);
+        const v4i acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf, qf, v4i{0, 0, 0, 0}, 0, 0, 0);
+        float mv[4] = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (MASK) {
+            const float4 mk = *reinterpret_cast<const float4*>(&sMask[16 * i + 4 * grp]);
+            mv[0] = mk.x; mv[1] = mk.y; mv[2] = mk.z; mv[3] = mk.w;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float y = static_cast<float>(acc[r]) * a.scale1;
+            if constexpr (MASK) y = y + mv[r];           // the mask Add between the Multiply and the Softmax
+            x[i][r] = y;
+            m = fmaxf(m, y);
+        }
+        if constexpr (MASK) if (i % 2 == 1) __builtin_amdgcn_sched_barrier(0);   // keep the mask reads next to their tile
+    }
+    if (a.scores) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) a.scores[dump_row + 16 * i + 4 * grp + r] = x[i][r];
+    }
+    m = fmaxf(m, __shfl_xor(m, 16, 64));
+    m = fmaxf(m, __shfl_xor(m, 32, 64));
+    // four keys, then the chunks of 256 keys, then halves of the groups (of 32 keys' eight groups of four: bits 1 and 0 of g, h; tile i
+    // has g = 2 (i % 2) + grp / 2 and h = grp % 2)
+    float part[8][2];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[i][r] = expf(x[i][r] - m);
+        const float e4 = (x[i][0] + x[i][1]) + (x[i][2] + x[i][3]);
+        const int t = i / 2;
+        part[t % 8][i % 2] = t < 8 ? e4 : part[t % 8][i % 2] + e4;
+    }
+#pragma unroll
+    for (int o = 4; o > 0; o >>= 1)
+#pragma unroll
+        for (int t = 0; t < o; ++t)
+#pragma unroll
+            for (int g = 0; g < 2; ++g) part[t][g] += part[t + o][g];
+    float s = part[0][0] + part[0][1];
+    s += __shfl_xor(s, 32, 64);
+    s += __shfl_xor(s, 16, 64);
+    const float inv = 1.0f / s;
+    v4i ctx[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+    if (a.p_bias) {                                      // register r of block db holds d = 16 db + 4 grp + r
+#pragma unroll
+        for (int db = 0; db < 4; ++db) {
+            const v4i sv = *reinterpret_cast<const v4i*>(&sVsum[16 * db + 4 * grp]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ctx[db][r] = sv[r] * a.p_bias;
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < NI / 4; ++c) {
+        v4i pf;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int i = 4 * c + k;
+            const float4 p4 = make_float4(quotient(x[i][0], s, inv), quotient(x[i][1], s, inv), quotient(x[i][2], s, inv), quotient(x[i][3], s, inv));
+            if (a.probs) *reinterpret_cast<float4*>(a.probs + dump_row + 16 * i + 4 * grp) = p4;
+            pf[k] = static_cast<int>(prob_levels4<DIV2, PFORM>(a, p4.x, p4.y, p4.z, p4.w));
+        }
+#pragma unroll
+        for (int db = 0; db < 4; ++db) {
+            const v4i vf = *reinterpret_cast<const v4i*>(&sVT[(16 * db + l16) * VT_LD + 64 * c + 16 * grp]);
+            ctx[db] = __builtin_amdgcn_mfma_i32_16x16x64_i8(vf, pf, ctx[db], 0, 0, 0);
+        }
+    }
+    const int64_t orow = bo * a.oo + bi * a.so + static_cast<int64_t>(q_row) * a.ldo;
+#pragma unroll
+    for (int db = 0; db < 4; ++db) {
+        const int d = 16 * db + 4 * grp;
+        const float4 o = make_float4(static_cast<float>(ctx[db][0]) * a.scale2, static_cast<float>(ctx[db][1]) * a.scale2,
+                                     static_cast<float>(ctx[db][2]) * a.scale2, static_cast<float>(ctx[db][3]) * a.scale2);
+        if (a.fq_o.levels) *reinterpret_cast<uint32_t*>(static_cast<int8_t*>(a.out) + orow + d) = requant4(a.fq_o, o);
+        else *reinterpret_cast<float4*>(static_cast<float*>(a.out) + orow + d) = o;
+    }
+}
+
 template <int NT>
 void launch(const AttentionArgs& a_in, int batches, hipStream_t s) {
     AttentionArgs a = a_in;
-    a.qblocks = static_cast<int>(ceil_div(a.S, 128));
+    a.qblocks = static_cast<int>(ceil_div(a.S, NT * 32 > kPlainSoftmax ? 64 : 128));
     a.xcd_groups = batches % 16 == 0 ? 1 : 0;         // pairs of batch elements, eight pairs at a time
     const dim3 grid = a.xcd_groups ? dim3(static_cast<uint32_t>(a.qblocks) * batches) : dim3(a.qblocks, static_cast<uint32_t>(batches));
     // (the forms without clamp: compiled for the usual division only)
     const int pform = !a.p_div2 ? 0 : (a.p_sat ? 2 : (a.p_inside ? 1 : 0));
     const int form = (a.mask ? 8 : 0) + (a.p_div2 ? 4 : 0) + pform;
-#define HIPIE_ATT_LAUNCH(D, M, P) hipLaunchKernelGGL((attention_kernel<NT, D, M, P>), grid, dim3(256), 0, s, a)
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, a); };
+#define HIPIE_ATT_LAUNCH(D, M, P)                                                       \
+    if constexpr (NT * 32 > kPlainSoftmax) go(attention_long_kernel<2 * NT, D, M, P>); \
+    else go(attention_kernel<NT, D, M, P>)
     switch (form) {
     case 0: HIPIE_ATT_LAUNCH(false, false, 0); break;
     case 4: HIPIE_ATT_LAUNCH(true, false, 0); break;

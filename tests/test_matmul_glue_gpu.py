@@ -398,6 +398,12 @@ def test_fused_attention_with_u8_probabilities(orc, S, masked):
     assert torch.equal(att.run(q, k, v, mask=md), ctx)
 
 
+@pytest.mark.parametrize("S,masked", [(448, True), (512, False)])
+def test_long_rows_with_u8_probabilities(orc, S, masked):
+    """beyond 384 keys another kernel: its sums of V, its mask, and the keys in the order of its second product"""
+    test_fused_attention_with_u8_probabilities(orc, S, masked)
+
+
 def test_nested_batches_inside_a_packed_tensor():
     """hipie_matmul_run_nested / hipie_transpose_bytes_nested address (sequence, head) batches inside one
     [tokens, 3 * hidden] tensor by pitch, inner and outer strides (the attention operands of an encoder without
