@@ -690,6 +690,12 @@ __device__ __forceinline__ void conv_tiles(Ctx& x, lds_ptr lds) {
     const int kk = src.kk, rows = (4 * B) >> shift <= 1 ? 1 : 4;      // (four columns and eight waves to a tile: choose_tile does not)
     const int col0 = rows == 4 ? kk & (B - 1) : min(kk >> 2, B - 1), r0 = rows == 4 ? 0 : kk & 3;
     const bool finishes = rows == 4 ? kk < B : kk < 4 * B;
+    // Gelu's chain is long and its largest tiles are few: five on eight waves with 3072 channels of 1536 tokens and 256 workgroups, two of
+    // them on one SIMD.  Where that takes fewer columns one behind the other every wave takes every eighth of the columns of all tiles:
+    // an encoder of 6 layers x 3 x 512 tokens 566 us without, 552 with it.  With all eight waves busy (64 workgroups) it does not, and
+    // would be slower (1243 and 1300: constants and places of another tile are fetched behind the product).  For the smaller tiles, as
+    // quarters of columns, the code cost 12 layers x 128 tokens 10 % and gave it nothing.
+    constexpr bool kSpreads = GELU && B == 4 && !PAIR;
     bool first = true;
     int base = t0;
     do {
@@ -710,15 +716,36 @@ __device__ __forceinline__ void conv_tiles(Ctx& x, lds_ptr lds) {
         ot = __builtin_amdgcn_readfirstlane(ot);
         pt = __builtin_amdgcn_readfirstlane(pt);
         const int mt = pt * (16 * B), oc = ot * (16 * A) + A * lane16;
+        bool spread = false, fin = on && finishes;
+        int fmt = mt, fot = ot, column = sub * B + kk, columns = (sub + 1) * B;      // (kSpreads) whose column comes next, the first that is not the wave's
+        auto take = [&] {
+            int fpt;
+            fast_divmod(base + column / B, PROG_FIELD(x.words, p_tiles), PROG_FIELD(x.words, inv_p_tiles), fot, fpt);
+            fot = __builtin_amdgcn_readfirstlane(fot);
+            fmt = __builtin_amdgcn_readfirstlane(fpt) * (16 * B);
+        };
+        if constexpr (kSpreads) {
+            const int all = min(per, t1 - base) * B;
+            spread = (PROG_FIELD(x.words, flags) & CF_GELU) && (all + 7) / 8 < (B + src.ks - 1) >> shift;
+            if (spread) {
+                column = x.wave;
+                columns = all;
+                fin = column < all;
+                if (fin) take();
+            }
+        }
         src.w = make_buffer(PROG_TABLE_OF(int8_t, x.words, wgt) + static_cast<int64_t>(ot) * src.nk * (A * 1024));
         if constexpr (PAIR) src2.w = make_buffer(PROG_TABLE_OF(int8_t, x.words, wgt2) + static_cast<int64_t>(ot) * src2.nk * (A * 1024));
         // All that the step in front does not write is on its way before the wait: operands, constants, where the results go and, from
         // an older step, the residual.  Loads come back in order and a branch hides from the compiler how many there were behind it:
         // nothing that is loaded under a condition stands behind the pixels, which are the first to be waited for.
+        if constexpr (kSpreads) {
+            if (fin) place_pixels<A>(pix, M, fmt + 16 * (column & (B - 1)) + 4 * quad, q);
+        }
         if (on) {
 #pragma unroll
             for (int b = 0; b < B; ++b) off[b] = pix[mt + 16 * b + lane16];
-            if (finishes) place_pixels<A>(pix, M, mt + 16 * col0 + 4 * quad + r0, q);      // the first column this wave finishes
+            if (!kSpreads && finishes) place_pixels<A>(pix, M, mt + 16 * col0 + 4 * quad + r0, q);      // the first column this wave finishes
             if constexpr (PAIR) {
 #pragma unroll
                 for (int b = 0; b < B; ++b) off2[b] = pix[3 * M + mt + 16 * b + lane16];
@@ -727,7 +754,7 @@ __device__ __forceinline__ void conv_tiles(Ctx& x, lds_ptr lds) {
         if (on) {
             if constexpr (PAIR) first_weights<A, B>(ring, src2, x.lane);
             else first_weights<A, B>(ring, src, x.lane);
-            if (finishes) {
+            if (!kSpreads && finishes) {
                 const int pitch = PROG_FIELD(x.words, OCp) * 4;
                 if constexpr (PAIR) {
                     const uint8_t* t2 = PROG_TABLE_OF(uint8_t, x.words, constants2) + oc * 4;
@@ -784,11 +811,31 @@ __device__ __forceinline__ void conv_tiles(Ctx& x, lds_ptr lds) {
             }
             start();
             k_loop<A, B>(ring, src, off, x.lane, acc);
-            if constexpr (kLate) load_constants<A>(sc.flags, PROG_TABLE_OF(uint8_t, words, constants), PROG_FIELD(words, OCp) * 4, oc, k);
-            put(part);
+            if constexpr (kLate && !kSpreads) load_constants<A>(sc.flags, PROG_TABLE_OF(uint8_t, words, constants), PROG_FIELD(words, OCp) * 4, oc, k);
+            if constexpr (!kSpreads) put(part);
         }
-        if (src.ks > 1) meet();
-        if (on && finishes) {
+        if constexpr (kSpreads) {
+            const int foc = fot * (16 * A) + A * lane16;
+            if (fin) {
+                load_constants<A>(sc.flags, PROG_TABLE_OF(uint8_t, words, constants), PROG_FIELD(words, OCp) * 4, foc, k);
+                load_residual<A, 4>(sc, foc, q);
+            }
+            if (on) put(part);
+        }
+        if (src.ks > 1 || spread) meet();
+        if constexpr (kSpreads) {
+            while (fin) {
+                const int foc = fot * (16 * A) + A * lane16;
+                finish_column<GELU, A, B, 4, PAIR>(sc, k, k2, (lds_v4i)lds + column / B * src.ks * (F * 64) + x.lane, mine2, src.ks, column & (B - 1), 0, q, foc);
+                column += spread ? 8 : src.ks;
+                if (column >= columns) break;
+                const int held = fot;
+                if (spread) take();
+                if (fot != held) load_constants<A>(sc.flags, PROG_TABLE_OF(uint8_t, words, constants), PROG_FIELD(words, OCp) * 4, fot * (16 * A) + A * lane16, k);
+                place_pixels<A>(pix, M, fmt + 16 * (column & (B - 1)) + 4 * quad, q);
+                load_residual<A, 4>(sc, fot * (16 * A) + A * lane16, q);
+            }
+        } else if (on && finishes) {
             if (B == 4 || rows == 4) {
                 for (int b = kk;;) {
                     finish_column<GELU, A, B, 4, PAIR>(sc, k, k2, mine, mine2, src.ks, b, 0, q, oc);
@@ -802,7 +849,7 @@ __device__ __forceinline__ void conv_tiles(Ctx& x, lds_ptr lds) {
             }
         }
         base += per;
-        if (src.ks > 1 && base < t1) meet();
+        if ((src.ks > 1 || spread) && base < t1) meet();
     } while (base < t1);
 }
 
@@ -1778,7 +1825,7 @@ __device__ __forceinline__ void attention_long(const ProgAttention& s, Ctx& x, l
 
 // ---- the program ------------------------------------------------------------------------------------------------------------
 // Three kernels, for networks over feature maps, for encoders, and for graphs with steps of both: every kind of step adds to the
-// registers of all others.  The 4 x 4 tiles ask for 250 and more vector registers, none is spilled to memory; 309, 260 and 556
+// registers of all others.  The 4 x 4 tiles ask for 250 and more vector registers, none is spilled to memory; 309, 278 and 556
 // scalar registers of the many step kinds are kept in lanes of vector registers.  The kernel with all kinds has no registers left for
 // 4 x 4 tiles (with them it spills); its convolutions take smaller ones (an encoder layer of 96 tokens beside a ResNet-50 of width
 // 16 at 64 x 64: 244 us, 467 by steps; beside a MobileNetV2 of 2 x 96 x 96 208 and 512).  A new step kind belongs into a kernel of its own where it
