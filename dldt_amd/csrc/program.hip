@@ -110,7 +110,7 @@ struct Ctx {
     // store in front, us with 64 / 128 / 256 workgroups: 1.3 / 1.5 / 1.6; by way of a root counter that the last of an XCD
     // adds to 2.1 / 2.3 / 2.6, all at one counter 1.5 / 2.3 / 4.1, a flag per workgroup that everybody reads 1.4 / 1.6 / 1.8.
     // (One way between two workgroups, store to sight, takes 0.5 - 0.6 us, the wait for a store 0.36.)  In the program a step without
-    // work, a copy of no bytes, takes 1.6 / 1.7 / 1.9 us; with the root counter and descriptors by scalar loads 3.6 / 4.1 / 4.2.
+    // work, a copy of no bytes, takes 1.5 / 1.6 / 1.8 us; with the root counter and descriptors by scalar loads 3.6 / 4.1 / 4.2.
     __device__ __forceinline__ void arrive(int next_step) {
         words = load_words(next_step, 0);
         words2 = load_words(next_step, 1);
@@ -1431,7 +1431,7 @@ __device__ __forceinline__ void copy_items(const ProgRows& s, const Ctx& x) {
 // and the waves meet for the maximum, for the sum and for the integer sums of the context.  What bounds a step is the chain of
 // exponentials and levels of one wave (1 us for a tile of 32 x 32), so the fewer tiles a wave has the better while there are
 // compute units: the step of one sequence of 128 tokens, 12 heads, barrier included, took 11.2 us with a wave for 32 queries, 48
-// waves in all, that multiplied the scores out three times, and takes 7.5 with four.  The sum keeps its order - a lane's keys one behind the
+// waves in all, that multiplied the scores out three times, and takes 7.2 with four.  The sum keeps its order - a lane's keys one behind the
 // other - so one wave adds the exponentials of all.  They take K's place in LDS, and the context's partial sums theirs.
 constexpr int kMostTiles = 4;                 // of a wave
 constexpr int kMostSplit = 8;
@@ -2538,7 +2538,7 @@ void request_leaves(int device) {
 // A lone request takes the form that was fastest alone.  Beside others it takes the smaller one, if units are left for it
 // (never more workgroups than compute units, so that all of them find a place), and else the steps, whose kernels share the
 // device.  ResNet-50, batch 1, us a request with 2 and 4 in flight: steps 251 and 167, 64 workgroups side by side 148 and 96
-// (alone: steps 492, 64 workgroups 284, 256 238).  With more than twice as many requests as find a place the ones by steps wait
+// (alone: steps 492, 64 workgroups 284, 256 227).  With more than twice as many requests as find a place the ones by steps wait
 // for the others: batch 3 with 128 workgroups, 4 in flight: 182, steps 182; 6 in flight: 221, steps 173 (batch 1 with 64
 // workgroups, 6 in flight: 113, steps 163).
 const ProgramForm* Program::choose(int together) {
