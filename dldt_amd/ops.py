@@ -82,7 +82,7 @@ class FakeQuantize:
         n, hw = self._nhw(x)
         tdt = torch.int8 if dtype in ("i8", "u8b") else torch.uint8
         if layout == "nchw":
-            y = torch.empty_like(x, dtype=tdt) if out is None else out
+            y = torch.empty_like(x, dtype=tdt, memory_format=torch.contiguous_format) if out is None else out
             cs = 0
         else:
             cs = c_stride or -(-self.C // 16) * 16

@@ -252,3 +252,19 @@ def test_many_small_images_are_not_slower_than_their_pixels_in_one_row(shape):
     many, one = micros(lambda: fq.run_q8(x, "u8b", "nhwc", cs, out=out)), micros(lambda: fq.run_q8(row, "u8b", "nhwc", cs, out=row_out))
     print("%s: %.1f us, one row %.1f" % (shape, many, one))
     assert many < 1.35 * one
+
+
+@pytest.mark.parametrize("shape", [(2, 1, 4, 6), (3, 7, 1, 1), (1, 5, 3, 2)])
+def test_levels_are_dense_in_order_whatever_strides_dimensions_of_one_have(shape):
+    import torch
+    from dldt_amd import FakeQuantize
+    x = torch.randn(shape, device="cuda")
+    if shape[0] > 1:
+        x = x.to(memory_format=torch.channels_last)              # (one channel or one pixel: contiguous both ways)
+    else:
+        x = x.as_strided(shape, (1, *x.stride()[1:]))
+    assert x.is_contiguous() and x.stride() != torch.empty(shape).stride()
+    fq = FakeQuantize(shape[1], 256, -3.0, 3.0, 0.0, 255.0)
+    y = fq.run_q8(x)
+    assert y.stride() == torch.empty(shape).stride()
+    assert torch.equal(y, fq.run_q8(x.clone(memory_format=torch.contiguous_format)))
