@@ -166,6 +166,12 @@ void check_status(int st, const char* what) {
     if (st != HIPIE_OK) fail(static_cast<hipie_status>(st), "%s: %s", what, hipie_last_error());
 }
 
+// whether two ranges of memory have a byte in common
+bool overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
+    const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
+    return p < q + static_cast<uintptr_t>(b_bytes) && q < p + static_cast<uintptr_t>(a_bytes);
+}
+
 // FakeQuantize on a graph input: f32 NCHW in the request's input buffer -> byte NHWC tensor
 struct EntryStep : Step {
     int param_index = 0, out = -1;
@@ -173,16 +179,22 @@ struct EntryStep : Step {
     int64_t channels = 0, levels = 0;
     std::vector<float> il, ih, ol, oh;
     hipie_fq* fq = nullptr;
-    bool inside_next = false;      // the convolution behind it does it in its launch
+    int into = -1;                 // the result that the convolution behind it stores in a launch that does both (-1: they are two)
+    int64_t reads = 0, stores = 0; // bytes of this step's input and of that result
+    // The launch that does both stores results while other workgroups have input to read: a caller's buffers that share a byte take
+    // the two, of which the first has read everything before the second begins
+    bool inside_next(void* const* inputs, void* const* outputs) const {
+        return into >= 0 && !overlap(inputs[param_index], reads, outputs[into], stores);
+    }
     ~EntryStep() override { hipie_fq_destroy(fq); }
-    int launches() const override { return inside_next ? 0 : 1; }
+    int launches() const override { return into >= 0 ? 0 : 1; }
     void create(int device, const std::vector<TensorInfo>&) override {
         check_status(hipie_fq_create(device, channels, levels, il.data(), il.size(), ih.data(), ih.size(),
                                      ol.data(), ol.size(), oh.data(), oh.size(), &fq), name.c_str());
     }
-    void run(uint8_t* arena, const std::vector<TensorInfo>& tensors, void* const* inputs, void* const*,
+    void run(uint8_t* arena, const std::vector<TensorInfo>& tensors, void* const* inputs, void* const* outputs,
              hipStream_t s) const override {
-        if (inside_next) return;
+        if (inside_next(inputs, outputs)) return;
         const hipie_tensor d = tensors[out].desc(arena);
         check_status(u8_in ? hipie_fq_run_q8_tensor_u8(fq, static_cast<const uint8_t*>(inputs[param_index]), &d, s)
                            : hipie_fq_run_q8_tensor(fq, static_cast<const float*>(inputs[param_index]), &d, s),
@@ -223,7 +235,7 @@ struct ConvStep : Step {
     bool entry_fused = false;
     void choose_entry(bool one_launch) {
         entry_fused = one_launch && with_entry;
-        if (entry) entry->inside_next = entry_fused;
+        if (entry) entry->into = entry_fused ? result : -1;
     }
     ~ConvStep() override { hipie_conv_destroy(conv); }
     void fill_desc(const std::vector<TensorInfo>& tensors) {
@@ -269,7 +281,7 @@ struct ConvStep : Step {
              hipStream_t s) const override {
         const hipie_tensor i = tensors[in].desc(arena), o = tensors[out].desc(arena);
         hipie_tensor r{};
-        if (entry_fused) {
+        if (entry_fused && entry->inside_next(inputs, outputs)) {
             run_entry_conv(*with_entry, inputs[entry->param_index], i, outputs[result], s);
             return;
         }
@@ -372,7 +384,7 @@ struct ConvStep : Step {
             for (int w = 0; w < times; ++w)
                 for (size_t l = 0; l < nl; ++l)
                     if (entry_too) {
-                        entry->run(lanes[l].arena, tensors, lanes[l].inputs.data(), nullptr, lanes[l].stream);
+                        entry->run(lanes[l].arena, tensors, lanes[l].inputs.data(), lanes[l].outputs.data(), lanes[l].stream);
                         run(lanes[l].arena, tensors, lanes[l].inputs.data(), lanes[l].outputs.data(), lanes[l].stream);
                     } else check_status(direct ? conv_run_planes(conv, ti[l], to[l], lanes[l].outputs[result], lanes[l].stream)
                                         : hipie_conv_run(conv, &ti[l], has_res ? &tr[l] : nullptr, &to[l], lanes[l].stream), name.c_str());
@@ -3539,6 +3551,8 @@ std::unique_ptr<hipie_plan> compile_plan(const hipie_graph* g, int device, const
                                             mid.dtype == HIPIE_U8B ? mid.fill_level - 128 : mid.fill_level);
             if (!c->with_entry) continue;
             c->entry = e;
+            e->reads = static_cast<int64_t>(mid.n) * mid.c * mid.h * mid.w * (e->u8_in ? 1 : 4);
+            e->stores = static_cast<int64_t>(mid.n) * plan->tensors[c->out].c * mid.h * mid.w * 4;      // (make_entry_conv: the same map)
             c->entry_mode = cfg.fuse_convs;
             c->choose_entry(cfg.fuse_convs == 2);
         }
@@ -4215,12 +4229,12 @@ int hipie_request_stream(hipie_request* r, void** stream) {
 // single launch was checked with stand-ins, on a 16-byte boundary and apart from each other.  Other buffers go by steps.
 static bool buffers_fit_program(const hipie_plan& p, void* const* in, void* const* out) {
     const size_t n_in = p.inputs.size(), n = n_in + p.outputs.size();
-    auto at = [&](size_t k) { return reinterpret_cast<uintptr_t>(k < n_in ? in[k] : out[k - n_in]); };
-    auto bytes = [&](size_t k) { return static_cast<uintptr_t>(k < n_in ? p.inputs[k].bytes : p.outputs[k - n_in].bytes); };
+    auto at = [&](size_t k) -> const void* { return k < n_in ? in[k] : out[k - n_in]; };
+    auto bytes = [&](size_t k) { return k < n_in ? p.inputs[k].bytes : p.outputs[k - n_in].bytes; };
     for (size_t k = 0; k < n; ++k) {
-        if (at(k) % 16 != 0) return false;
+        if (reinterpret_cast<uintptr_t>(at(k)) % 16 != 0) return false;
         for (size_t j = n_in; k >= n_in ? j < k : j < n; ++j)        // (inputs may lie on each other: they are only read)
-            if (at(k) < at(j) + bytes(j) && at(j) < at(k) + bytes(k)) return false;
+            if (overlap(at(k), bytes(k), at(j), bytes(j))) return false;
     }
     return true;
 }

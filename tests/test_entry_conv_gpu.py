@@ -110,3 +110,32 @@ def test_the_choice_is_kept_in_files_and_exports(tmp_path):
         got = _run(plan, node, x)
         assert np.array_equal(got[1], want[1]) and np.array_equal(got[0], want[0])
     assert not _one(_compile(g, "NO", HIP_TUNE="YES", HIP_TUNE_FILE=str(path)))
+
+
+# images of their own, rows that two workgroups share, several groups of channels over one patch, more workgroups than find a place
+@pytest.mark.parametrize("tuned", [False, True])
+@pytest.mark.parametrize("n,c,h,w,oc,kind", [(1, 64, 14, 14, 64, "u8"), (12, 72, 45, 45, 72, "u8"), (3, 17, 9, 65, 130, "zero point"), (32, 64, 28, 28, 512, "u8"),
+                                             (16, 96, 40, 40, 24, "bytes"), (32, 8, 112, 112, 48, "u8")])
+def test_an_output_on_its_input_is_the_result_of_two_launches(n, c, h, w, oc, kind, tuned):
+    """the FakeQuantize reads all of its input before the convolution stores anything where the two buffers share a byte"""
+    g, node = _graph(n, c, h, w, oc, kind=kind)
+    plan = _compile(g, "YES", HIP_TUNE="YES" if tuned else "NO")
+    assert _one(plan)
+    x = _input(g, 7)
+    want = _run(_compile(g, "NO"), node, x)
+    results = n * oc * h * w * 4
+    size = x.numel() * x.element_size()
+    # (whole, the output behind the input's start and in front of it, the last and the first of its bytes, side by side)
+    for at in (0, 4 * w, -4 * w, size - 4, 4 - results, size, -results):
+        start = max(0, -at)
+        place = torch.zeros(start + max(size, at + results) + 64, dtype=torch.uint8, device="cuda")
+        feed = place[start:start + size].view(x.dtype).view(x.shape)
+        out = place[start + at:start + at + results].view(torch.float32).view(n, oc, h, w)
+        req = plan.create_request()
+        for run in (req.enqueue, req.infer_device):
+            feed.copy_(x)
+            torch.cuda.synchronize()
+            run([feed], [out])
+            torch.cuda.synchronize()
+            got = out.cpu().numpy().view(np.uint32)
+            assert np.array_equal(got, want[0]) and np.array_equal(req.tensor(node), want[1]), (at, run.__name__)
