@@ -17,6 +17,7 @@
 #include <chrono>
 
 #include "div2.h"
+#include "step_barrier.h"
 
 struct hipie_fq;
 
@@ -33,8 +34,6 @@ constexpr int kLdsBytes = kPlainAt + kMaxPieces * 4;
 // waits for the same units) does not let go, and the steps need less than that beside it.
 constexpr uint32_t kRollCallTicks = 100000, kMaxRollCallTicks = 10000000;
 constexpr uint64_t kBarrierTicks = 200000000;
-// what a launch tells the host in its slot's word, 0 before it
-constexpr uint32_t kReportCancelled = 1, kReportLost = 2, kReportDone = 3;
 
 typedef __attribute__((address_space(3))) int8_t* lds_ptr;
 typedef __attribute__((address_space(3))) v4i* lds_v4i;
@@ -114,12 +113,19 @@ struct Ctx {
     __device__ __forceinline__ void arrive(int next_step) {
         words = load_words(next_step, 0);
         words2 = load_words(next_step, 1);
+        arrive_at(*this);
+    }
+    __device__ __forceinline__ int32_t verdict() const { return flag[0]; }      // of the wait before: 0 if it was given up
+    __device__ __forceinline__ bool lost(int32_t held) const { return __builtin_amdgcn_readfirstlane(held) == 0; }
+    __device__ __forceinline__ void lose() const { flag[0] = 0; }
+    __device__ __forceinline__ void settle() {
         wait_memory();
         __builtin_amdgcn_s_barrier();
         target += n_wg / 8;
+    }
+    __device__ __forceinline__ void count() const {
         // (not the wave that looks at the counters: its loads would come back behind the addition)
         if (tid == kProgramThreads - 64) (void)__hip_atomic_fetch_add(own, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        dead = __builtin_amdgcn_readfirstlane(flag[0]) == 0;      // (of the wait before: its verdict is not waited for)
     }
     __device__ __forceinline__ void wait() {
         if (wave == 0 && !started) {
@@ -131,10 +137,7 @@ struct Ctx {
                 if ((n & 255) != 0) continue;
                 if (t0 == 0) t0 = wall_clock64();
                 if (wall_clock64() - t0 > kBarrierTicks) {
-                    if (lane == 0) {
-                        tell(kReportLost);
-                        flag[0] = 0;
-                    }
+                    if (lane == 0) give_up(*this);
                     break;
                 }
             }
@@ -148,8 +151,9 @@ struct Ctx {
         if (rank != 0) return;
         lane = lane_index();
         wait();
-        if (wave == 0 && lane == 0 && flag[0] != 0) tell(kReportDone);
+        if (wave == 0 && lane == 0) report(*this);
     }
+    // (lane 0 of the first wave)
     __device__ __forceinline__ void tell(uint32_t what) const {
 #if defined(__HIP_DEVICE_COMPILE__)
         typedef uint32_t* Word;
@@ -2598,7 +2602,7 @@ bool report_done(const Program& p, int slot) {
 
 bool program_failed(const Program& p, int slot, uint32_t* control, hipStream_t s) {
     const uint32_t v = __atomic_load_n(p.report + 16 * slot, __ATOMIC_ACQUIRE);
-    if (v == 0 || v == kReportDone) return false;
+    if (v == kReportDone) return false;
     hipLaunchKernelGGL(clear_words, dim3(1), dim3(256), 0, s, control, static_cast<int>(kProgramControlBytes / 4));
     HIPIE_CHECK_HIP(hipGetLastError());
     return true;
