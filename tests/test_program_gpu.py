@@ -155,7 +155,10 @@ def test_results_are_there_when_the_call_returns(name):
     g = GRAPHS[name]()
     steps, single = _compile(g, "NO"), _compile(g, "64")
     want = [_infer(steps.create_request(), seed) for seed in range(4)]
-    other = torch.cuda.Stream()
+    # (a request's stream: the first torch.cuda.Stream() makes 32 that stay, and with them every later request's hardware queue is
+    # another one; test_requests_of_several_threads meets queues that two of its requests share)
+    aside = steps.create_request()
+    other = torch.cuda.ExternalStream(aside.stream)
     b = single.create_request()
     buffers = []
     for seed in range(4):
