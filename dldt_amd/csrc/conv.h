@@ -91,11 +91,16 @@ struct ConvLaunch {
     int kh, kw, dil_h, dil_w, pad_top, pad_left;
 };
 bool conv_launch_arguments(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out, ConvLaunch& l);
-// the same with the f32 results channel by channel, [N, C, H, W] dense at `planes`; `out` says their shape.  Layers that take it:
-// dense convolutions without a residual
+// where the variants that split K over workgroups (14 to 17) keep their partial sums: the stream's workspace, which the first such
+// launch makes and a captured one has to find; the device's array of fixed size; nowhere - variant 4, the same bits, runs instead
+enum class SplitScratch { workspace, fixed, none };
+// the same with the f32 results channel by channel, [N, C, H, W] dense at `planes`; `out` says their shape, and takes them as well
+// with `tensor_too`.  Layers that take it: dense convolutions without a residual
 bool conv_takes_planes(const hipie_conv* c, int64_t n, int64_t oh, int64_t ow);
-int conv_run_planes(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor& out, void* planes, hipStream_t s);
-void planes_arguments(ConvArgs& a, void* planes);
+int conv_run_planes(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor& out, void* planes, bool tensor_too, SplitScratch scratch, hipStream_t s);
+void planes_arguments(ConvArgs& a, void* planes, bool tensor_too = false);
+// hipie_conv_run where no launch on the stream may have made its workspace
+int conv_run_unsplit(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor& out, hipStream_t s);
 
 // a convolution of a short K and the depthwise 3 x 3 layer that alone reads it in one launch (expand_dw.hip); form 0: 32 channels a
 // workgroup, 1: the same in bands of half the height, 2: 48 channels, 3: 32 channels of several small images.

@@ -2264,13 +2264,13 @@ static int64_t fill_conv_args(const hipie_conv* c, const hipie_tensor* in, const
 }
 
 static int conv_run(const hipie_conv* c, const hipie_tensor* in, const hipie_tensor* residual,
-                    const hipie_tensor* out, void* stream, bool static_scratch_only, void* planes = nullptr) {
+                    const hipie_tensor* out, void* stream, SplitScratch scratch, void* planes = nullptr, bool tensor_too = false) {
     return guarded([&] {
         ConvArgs a;
         int32_t oh, ow;
         const int64_t M = fill_conv_args(c, in, residual, out, a, oh, ow);
         if (M == 0) return;
-        if (planes) planes_arguments(a, planes);
+        if (planes) planes_arguments(a, planes, tensor_too);
         const hipie_conv_desc& d = c->d;
         if (c->depthwise) {
             HIPIE_REQUIRE(in->stride_w >= d.ic && in->stride_w % 16 == 0, HIPIE_PARAMETER_MISMATCH,
@@ -2372,12 +2372,12 @@ static int conv_run(const hipie_conv* c, const hipie_tensor* in, const hipie_ten
         stages = stages >= 8 && max_stages >= 8 ? 8 : (stages >= 6 && max_stages >= 6 ? 6 : (stages >= 4 && max_stages >= 4 ? 4 : 3));
         // the K split pays where a launch has fewer tiles than the device has compute units; with many tiles
         // (more than 2048 workgroups, a 128 MB workspace) the plain pipelined kernel runs instead
-        if (tile >= 14 && tile <= 17 && static_cast<int64_t>(a.p_tiles) * a.t_tiles * split_parts(tile) > 2048) tile = 4;
+        if (tile >= 14 && tile <= 17 && (scratch == SplitScratch::none || static_cast<int64_t>(a.p_tiles) * a.t_tiles * split_parts(tile) > 2048)) tile = 4;
         std::unique_lock<std::mutex> workspace_lock;   // held across the launch below
         if (tile >= 14 && tile <= 17) {
             a.ksplit = split_parts(tile);
             const size_t tiles = static_cast<size_t>(a.p_tiles) * a.t_tiles;
-            if (static_scratch_only) {
+            if (scratch == SplitScratch::fixed) {
                 // the device's fixed array instead of an allocated workspace: nothing is allocated, larger launches are refused
                 HIPIE_REQUIRE(tiles * a.ksplit <= kStaticParts && tiles <= kStaticTiles, HIPIE_OUT_OF_BOUNDS,
                               "hipie_conv_run_static: %zu tiles x %d parts need %zu KB of partial sums, the static scratch holds %zu KB "
@@ -2433,7 +2433,7 @@ static int conv_run(const hipie_conv* c, const hipie_tensor* in, const hipie_ten
 
 int hipie_conv_run(const hipie_conv* c, const hipie_tensor* in, const hipie_tensor* residual,
                    const hipie_tensor* out, void* stream) {
-    return conv_run(c, in, residual, out, stream, false);
+    return conv_run(c, in, residual, out, stream, SplitScratch::workspace);
 }
 
 int hipie_conv_pair_fits(const hipie_conv* first, const hipie_conv* second, int32_t h, int32_t w, int* fits) {
@@ -2490,12 +2490,19 @@ int hipie_conv_run_pair(const hipie_conv* first, const hipie_conv* second, const
 
 int hipie_conv_run_static(const hipie_conv* c, const hipie_tensor* in, const hipie_tensor* residual,
                           const hipie_tensor* out, void* stream) {
-    return conv_run(c, in, residual, out, stream, true);
+    return conv_run(c, in, residual, out, stream, SplitScratch::fixed);
 }
 
 }  // extern "C"
 
-void hipie::planes_arguments(ConvArgs& a, void* planes) {
+void hipie::planes_arguments(ConvArgs& a, void* planes, bool tensor_too) {
+    if (tensor_too) {
+        a.res = a.out;
+        a.res_sn = a.out_sn;
+        a.res_sh = a.out_sh;
+        a.res_sw = a.out_sw;
+        a.flat_res = a.flat_out;
+    }
     a.out = planes;
     a.out_plane = a.OHOW;
     a.out_sn = a.OC * a.OHOW;
@@ -2508,8 +2515,12 @@ bool hipie::conv_takes_planes(const hipie_conv* c, int64_t n, int64_t oh, int64_
     return !c->depthwise && !c->fused && c->epi.out_dtype == HIPIE_F32 && !(c->epi.flags & CF_RES) && n * c->d.oc * oh * ow < (1ll << 31);
 }
 
-int hipie::conv_run_planes(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor& out, void* planes, hipStream_t s) {
-    return conv_run(c, &in, nullptr, &out, s, false, planes);
+int hipie::conv_run_planes(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor& out, void* planes, bool tensor_too, SplitScratch scratch, hipStream_t s) {
+    return conv_run(c, &in, nullptr, &out, s, scratch, planes, tensor_too);
+}
+
+int hipie::conv_run_unsplit(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor& out, hipStream_t s) {
+    return conv_run(c, &in, nullptr, &out, s, SplitScratch::none);
 }
 
 bool hipie::conv_launch_arguments(const hipie_conv* c, const hipie_tensor& in, const hipie_tensor* residual, const hipie_tensor& out, ConvLaunch& l) {

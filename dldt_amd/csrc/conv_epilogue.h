@@ -548,6 +548,15 @@ __device__ __forceinline__ void epilogue(const ConvArgs& a, const v16i (&acc)[2]
                 for (int j = 0; j < 4; ++j)
                     if (valid[pb] && oc_lane + 4 * e4 + j < a.OC) o[static_cast<int64_t>(oc_lane + 4 * e4 + j) * a.out_plane] = v[pb][j] + 0.f;
             }
+            if (a.res) {      // (uniform; into the layer's tensor as well: an inference that is captured, or whose tensor is looked at)
+#pragma unroll
+                for (int pb = 0; pb < 2; ++pb) {
+                    if (staged_out && pb != pass) continue;
+                    if (valid[pb] && oc_lane + 4 * e4 + 4 <= a.res_sw)
+                        *reinterpret_cast<float4*>(static_cast<float*>(const_cast<void*>(a.res)) + res_off[pb] + 4 * e4) =
+                            make_float4(v[pb][0], v[pb][1], v[pb][2], v[pb][3]);
+                }
+            }
         } else if (staged_out) {
             typedef float v4f __attribute__((ext_vector_type(4)));
             const int row = lane_id & 31, c = ((lane_id >> 5) * 8 + e4) ^ (row & 15);

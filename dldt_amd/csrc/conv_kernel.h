@@ -86,7 +86,7 @@ struct ConvArgs {
     const int8_t* in;     // element (n=0, h=0, w=0, c=0) of the input tensor
     const int8_t* wgt;    // packed [OCp][Kp]
     void* out;            // element (0,0,0,0) of the output tensor
-    const void* res;      // residual tensor or nullptr
+    const void* res;      // residual tensor or nullptr; of f32 results that are stored in planes (out_plane): where they go, channels innermost, as well
     const int32_t* koff;  // [Kp/16] byte offset of every 16-byte K piece relative to the window origin
     // per-channel tables, each [OCp]
     const int32_t* corr;  // 128 * sum_k w[oc][k] for U8B inputs (0 for I8)

@@ -86,8 +86,10 @@ __global__ __launch_bounds__(256) void conv_skinny_kernel(const ConvArgs a) {
         if (fl & CF_BIAS) v = v + a.bias[oc];
         if (fl & CF_SCALE) v = v * a.scale[oc];
         if (fl & CF_RELU) v = v > 0.f ? v : 0.f;
-        if (a.out_plane) static_cast<float*>(a.out)[off + static_cast<int64_t>(oc) * (a.out_plane - 1)] = v + 0.f;
-        else static_cast<float*>(a.out)[off] = v;
+        if (a.out_plane) {
+            static_cast<float*>(a.out)[off + static_cast<int64_t>(oc) * (a.out_plane - 1)] = v + 0.f;
+            if (a.res) static_cast<float*>(const_cast<void*>(a.res))[static_cast<int64_t>(c.n) * a.res_sn + c.oh * a.res_sh + c.ow * a.res_sw + oc] = v;
+        } else static_cast<float*>(a.out)[off] = v;
     }
 }
 

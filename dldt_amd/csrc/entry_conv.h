@@ -16,7 +16,8 @@ struct EntryConv;
 // byte of its padding
 std::shared_ptr<EntryConv> make_entry_conv(int device, const hipie_fq* fq, bool u8_in, const hipie_conv* conv, const hipie_tensor& mid, const hipie_tensor& out, int fill);
 // in: dense [N, C, H, W], f32 or u8 as made; the levels into `mid`, the values into `planes`, dense [N, OC, H, W], which has no byte
-// in common with `in`: values are stored while other workgroups still have input to read
-void run_entry_conv(const EntryConv& e, const void* in, const hipie_tensor& mid, void* planes, hipStream_t s);
+// in common with `in`: values are stored while other workgroups still have input to read.  With `out` the values go into that tensor
+// as well
+void run_entry_conv(const EntryConv& e, const void* in, const hipie_tensor& mid, const hipie_tensor* out, void* planes, hipStream_t s);
 
 }  // namespace hipie

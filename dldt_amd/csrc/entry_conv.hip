@@ -31,7 +31,7 @@ namespace hipie {
 namespace {
 
 constexpr int kThreads = 512, kWaves = kThreads / 64;
-constexpr int kMostFragments = 2;            // of 32 pixels that a wave multiplies (104 registers, two workgroups a compute unit; three take 140)
+constexpr int kMostFragments = 2;            // of 32 pixels that a wave multiplies (110 registers, two workgroups a compute unit; three take 140 and more)
 constexpr int kAhead = 4;                    // K steps of 32 bytes in a group: one is multiplied while the next one's weights come
 
 struct Args {
@@ -45,6 +45,9 @@ struct Args {
     const int32_t* corr;
     const float *bias, *scale;
     float* out;
+    float* tensor;                           // the values channels innermost as well, or nullptr
+    int64_t t_sn, t_sh;
+    int32_t t_sw;                            // its strides in elements: image, row, pixel
     int32_t C, H, W, HW, OC;
     int32_t kh, kw, pad_h, pad_w;
     int32_t R, row_tiles, tiles, per_xcd;    // rows of a tile, tiles of an image and of all, of an XCD
@@ -277,6 +280,15 @@ __global__ __launch_bounds__(kThreads, 4) void entry_conv_kernel(const Args a) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) r[i] = r[i] < a.clamp_lo ? a.clamp_lo : (r[i] > a.clamp_hi ? a.clamp_hi : r[i]);
             }
+            if (a.tensor) {
+                int y, xx;
+                fast_divmod(min(m, count - 1), a.W, a.inv_W, y, xx);
+                const int oc = (og * wo + o_wave) * 32 + 4 * h;
+                float* const t = a.tensor + n * a.t_sn + (y0 + y) * a.t_sh + static_cast<int64_t>(xx) * a.t_sw + oc;
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (m < count && oc + 8 * q + 4 <= a.t_sw) *reinterpret_cast<float4*>(t + 8 * q) = make_float4(r[4 * q], r[4 * q + 1], r[4 * q + 2], r[4 * q + 3]);
+            }
             // (offsets beyond the plane's records store nothing: pixels behind the tile, channels behind the last)
             uint32_t to = m < count ? 4u * (static_cast<uint32_t>(4 * h) * static_cast<uint32_t>(a.HW) + static_cast<uint32_t>(m)) : 0x80000000u;
 #pragma unroll
@@ -434,8 +446,14 @@ std::shared_ptr<EntryConv> make_entry_conv(int device, const hipie_fq* fq, bool 
     return e;
 }
 
-void run_entry_conv(const EntryConv& e, const void* in, const hipie_tensor& mid, void* planes, hipStream_t s) {
+void run_entry_conv(const EntryConv& e, const void* in, const hipie_tensor& mid, const hipie_tensor* out, void* planes, hipStream_t s) {
     Args a = e.a;
+    if (out) {
+        a.tensor = static_cast<float*>(out->data);
+        a.t_sn = out->stride_n;
+        a.t_sh = out->stride_h;
+        a.t_sw = static_cast<int32_t>(out->stride_w);
+    }
     a.x = in;
     a.levels = static_cast<uint8_t*>(mid.data);
     a.out = static_cast<float*>(planes);

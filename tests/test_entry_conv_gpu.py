@@ -139,3 +139,71 @@ def test_an_output_on_its_input_is_the_result_of_two_launches(n, c, h, w, oc, ki
             torch.cuda.synchronize()
             got = out.cpu().numpy().view(np.uint32)
             assert np.array_equal(got, want[0]) and np.array_equal(req.tensor(node), want[1]), (at, run.__name__)
+
+
+def _kernels(graph):
+    """how many nodes a captured graph has"""
+    import ctypes
+    (path,) = {line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line}
+    n = ctypes.c_size_t()
+    assert ctypes.CDLL(path).hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value
+
+
+# as one launch, as two with and without K split over workgroups (whose workspace an inference in front of the capture makes, where
+# it runs that layer); in place it is two either way
+@pytest.mark.parametrize("variant,in_place", [(64 + 4, False), (64 + 14, False), (64 + 15, True), (4, True), (14, False), (15, True), (22, False)])
+def test_a_captured_inference_stores_both_in_its_own_launches(tmp_path, variant, in_place):
+    g, node = _graph(3, 128, 9, 31, 128)
+    out_node = g.nodes[-1]["inputs"][0]
+    path = tmp_path / "choices"
+    path.write_text("0 -1\n1 %d\n2 -1\n" % variant)
+    plan = _compile(g, "AUTO", HIP_TUNE="YES", HIP_TUNE_FILE=str(path))
+    assert plan.steps[1]["variant"] == variant
+    want = [_run(_compile(g, "NO"), node, _input(g, seed)) for seed in range(4)]
+    req = plan.create_request()
+    ins, outs = req.device_buffers()
+    feed, out = ins[0], outs[0]
+    apart = torch.empty_like(out)
+    ins[0].copy_(_input(g, 0))
+    torch.cuda.synchronize()
+    req.enqueue([feed], [apart])                                   # (once before capturing, into another buffer)
+    torch.cuda.synchronize()
+    if in_place:
+        out = feed
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=torch.cuda.ExternalStream(req.stream), capture_error_mode="thread_local"):
+        req.enqueue([feed], [out])
+    assert _kernels(graph) == (1 if variant & 64 and not in_place else 2)
+    for seed in range(4):
+        feed.copy_(_input(g, seed))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out.cpu().numpy()
+        assert np.array_equal(got.view(np.uint32), want[seed][0])
+        assert np.array_equal((req.tensor(out_node) + np.float32(0)).view(np.uint32), want[seed][0]), seed
+        assert np.array_equal(req.tensor(node), want[seed][1])
+
+
+@pytest.mark.parametrize("n,c,h,w,oc", [(1, 3, 7, 7, 8), (2, 4, 9, 31, 33), (12, 72, 45, 45, 100), (5, 33, 1, 100, 130), (3, 20, 13, 21, 5)])
+@pytest.mark.parametrize("fuse", ["YES", "NO"])
+def test_an_inference_whose_tensor_is_looked_at_stores_both(n, c, h, w, oc, fuse):
+    g, node = _graph(n, c, h, w, oc, act="none")
+    out_node = g.nodes[-1]["inputs"][0]
+    plan = _compile(g, fuse)
+    keeps = _compile(g, "NO", HIP_KEEP_F32="YES")                  # (every value in its tensor, the result copied from there)
+    req, ref = plan.create_request(), keeps.create_request()
+    ins, outs = req.device_buffers()
+    for seed in range(3):
+        ins[0].copy_(_input(g, seed))
+        torch.cuda.synchronize()
+        ref.enqueue(ins, outs)
+        torch.cuda.synchronize()
+        want = outs[0].cpu().numpy().view(np.uint32)
+        outs[0].fill_(float("nan"))
+        torch.cuda.synchronize()
+        req.enqueue(ins, outs)
+        torch.cuda.synchronize()
+        assert np.array_equal(outs[0].cpu().numpy().view(np.uint32), want)
+        assert np.array_equal(req.tensor(out_node).view(np.uint32), ref.tensor(out_node).view(np.uint32))      # (also in the sign of zeros)
