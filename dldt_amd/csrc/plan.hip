@@ -3124,18 +3124,20 @@ struct hipie_request {
     uint32_t* control = nullptr;
     uint32_t launches[kProgramControlBlocks] = {};
     const ProgramForm* form = nullptr;
-    const ProgramForm* ran = nullptr;        // the form of the last inference, if it was one (hipie_request_tensor)
     bool entered = false;                    // counted among the device's requests in flight
     bool alone = false;                      // no other was when this one started, nor lately
     bool stream_taken = false;               // hipie_request_stream gave the stream out: its work is complete in stream order
     std::vector<void*> run_in, run_out, host_out;
-    // Results whose tensors were looked at (hipie_request_tensor): from then on every inference fills these, so that a tensor
-    // that is held goes on showing the last one's values
-    mutable std::mutex looked_lock;
-    mutable std::vector<const ConvStep*> looked;
+    // Held while an inference is queued, and by hipie_request_tensor, which any thread may call meanwhile: either the inference fills
+    // what was looked at, or the call finds it queued and fills that behind it.
+    mutable std::mutex queue_lock;
     bool inferred = false;
+    const ProgramForm* ran = nullptr;        // the form of the last inference, if it was one
+    // Results whose tensors were looked at: from then on every inference fills these, so that a tensor that is held goes on showing
+    // the last one's values.  (unfilled: looked at while the stream was captured, which cannot be filled then)
+    mutable std::vector<const ConvStep*> looked, unfilled;
     bool looked_at() const {
-        std::lock_guard<std::mutex> g(looked_lock);
+        std::lock_guard<std::mutex> g(queue_lock);
         return !looked.empty();
     }
     // the stream has drained
@@ -3178,14 +3180,13 @@ __global__ void fill_bytes(uint8_t* p, int64_t n, uint8_t v) {
 void enqueue(hipie_request* r, void* const* in, void* const* out) {
     const hipie_plan& p = *r->plan;
     uint8_t* arena = r->arena.as<uint8_t>();
+    std::lock_guard<std::mutex> g(r->queue_lock);
+    r->ran = nullptr;
     // Results whose tensors are stored too: those that were looked at, and all where the inference is captured and runs again where
     // the host does not see it.  (The layer's own launch stores both; us an inference in a graph of twenty, with a launch more for the
     // tensor / so: 12 x 72 x 45 x 45 to 100 channels 21.6 / 15.0, 8 x 128 x 56 x 56 to 128 27.8 / 18.0.)
-    std::vector<const ConvStep*> both;
-    if (!p.result_writers.empty()) {
-        std::lock_guard<std::mutex> g(r->looked_lock);
-        both = is_capturing(r->stream) ? p.result_writers : r->looked;
-    }
+    const bool captured = !p.result_writers.empty() && is_capturing(r->stream);
+    const auto& both = captured ? p.result_writers : r->looked;
     for (size_t i = 0; i < p.steps.size(); ++i) {
         if (r->perf) HIPIE_CHECK_HIP(hipEventRecord(r->events[i], r->stream));
         const auto w = std::find(both.begin(), both.end(), p.steps[i].get());
@@ -3194,6 +3195,7 @@ void enqueue(hipie_request* r, void* const* in, void* const* out) {
     }
     if (r->perf) HIPIE_CHECK_HIP(hipEventRecord(r->events[p.steps.size()], r->stream));
     r->inferred = true;
+    if (!captured) r->unfilled.clear();
 }
 
 // by the plan's single-launch form
@@ -3203,13 +3205,13 @@ void enqueue_program(hipie_request* r, void* const* in, void* const* out) {
     for (size_t i = 0; i < p.inputs.size(); ++i) io[i] = in[i];
     for (size_t i = 0; i < p.outputs.size(); ++i) io[p.inputs.size() + i] = out[i];
     const int block = r->form == r->program->lone.get() ? 0 : 1;
+    std::lock_guard<std::mutex> g(r->queue_lock);
+    r->ran = r->form;
     launch_program(*r->program, *r->form, r->arena.as<uint8_t>(), io, static_cast<int>(p.inputs.size() + p.outputs.size()),
                    r->control + block * (kProgramControlBytes / 4), r->launches[block]++, r->slot, r->stream);
-    {
-        std::lock_guard<std::mutex> g(r->looked_lock);
-        for (const ConvStep* w : r->looked) w->fill(r->arena.as<uint8_t>(), p.tensors, r->stream);
-    }
+    for (const ConvStep* w : r->looked) w->fill(r->arena.as<uint8_t>(), p.tensors, r->stream);
     r->inferred = true;
+    r->unfilled.clear();
 }
 
 // The stream has drained.  Where a single launch gave up (its workgroups did not come together) the inference is queued
@@ -3223,8 +3225,11 @@ bool run_again(hipie_request* r) {
     r->program->count(!failed);
     if (!failed) return false;
     r->launches[block] = 0;
-    r->ran = nullptr;
-    if (r->cancelled) return false;          // (nobody reads its outputs)
+    if (r->cancelled) {                      // (nobody reads its outputs)
+        std::lock_guard<std::mutex> g(r->queue_lock);
+        r->ran = nullptr;
+        return false;
+    }
     enqueue(r, r->run_in.data(), r->run_out.data());
     for (size_t i = 0; i < r->host_out.size(); ++i)
         HIPIE_CHECK_HIP(hipMemcpyAsync(r->host_out[i], r->run_out[i], static_cast<size_t>(p.outputs[i].bytes), hipMemcpyDeviceToHost, r->stream));
@@ -4278,7 +4283,6 @@ static int start_request(hipie_request* r, const void* const* inputs, void* cons
             out[i] = device_memory ? outputs[i] : r->out_dev[i].ptr;
         }
         r->entered = true;
-        r->ran = nullptr;
         const int together = request_enters(p.device);
         r->alone = together == 1;
         if (r->slot >= 0 && (awaited || (!device_memory && !r->stream_taken)) && buffers_fit_program(p, in.data(), out.data()))
@@ -4286,7 +4290,6 @@ static int start_request(hipie_request* r, const void* const* inputs, void* cons
         if (r->form) {
             enqueue_program(r, in.data(), out.data());
             if (device_memory) HIPIE_CHECK_HIP(hipEventRecord(r->behind, r->stream));
-            r->ran = r->form;
             r->run_in = in;
             r->run_out = out;
             r->host_out.clear();
@@ -4383,7 +4386,6 @@ int hipie_request_enqueue(hipie_request* r, const void* const* inputs, void* con
         DeviceGuard g(r->plan->device);
         std::vector<void*> in(r->plan->inputs.size());
         for (size_t i = 0; i < in.size(); ++i) in[i] = const_cast<void*>(inputs[i]);
-        r->ran = nullptr;
         enqueue(r, in.data(), outputs);
     });
 }
@@ -4423,20 +4425,28 @@ int hipie_request_tensor(const hipie_request* r, int node_id, hipie_tensor* t) {
             if (auto* pair = dynamic_cast<const PairStep*>(st.get()))
                 HIPIE_REQUIRE(!(pair->fused && pair->first->out == it->second), HIPIE_NOT_FOUND,
                               "hipie_request_tensor: node %d lives in LDS only (two convolutions run as one kernel)", node_id);
+        std::unique_lock<std::mutex> queue(r->queue_lock);
         if (r->ran)
             for (int tensor : r->ran->inside)
                 HIPIE_REQUIRE(tensor != it->second, HIPIE_NOT_FOUND, "hipie_request_tensor: node %d lives in LDS only (two layers are one step of the single launch)", node_id);
         for (const ConvStep* w : r->plan->result_writers) {
             if (w->out != it->second) continue;
-            {
-                std::lock_guard<std::mutex> g(r->looked_lock);
-                if (std::find(r->looked.begin(), r->looked.end(), w) == r->looked.end()) r->looked.push_back(w);
-            }
+            const auto late = std::find(r->unfilled.begin(), r->unfilled.end(), w);
+            const bool known = std::find(r->looked.begin(), r->looked.end(), w) != r->looked.end();
+            if (known && late == r->unfilled.end()) continue;            // (the inferences fill it)
+            if (!known) r->looked.push_back(w);
             if (!r->inferred || !(r->ran ? w->writes_result : w->direct)) continue;
             DeviceGuard g(r->device);
-            if (is_capturing(r->stream)) continue;       // (what is captured fills it)
+            if (is_capturing(r->stream)) {
+                if (late == r->unfilled.end()) r->unfilled.push_back(w);
+                continue;
+            }
             w->fill(r->arena.as<uint8_t>(), r->plan->tensors, r->stream);
-            if (!r->started) HIPIE_CHECK_HIP(hipStreamSynchronize(r->stream));      // (else the wait does)
+            if (late != r->unfilled.end()) r->unfilled.erase(late);
+            // (here, whoever waits for the inference: a single launch that is waited for by its word is over before this is)
+            queue.unlock();
+            HIPIE_CHECK_HIP(hipStreamSynchronize(r->stream));
+            break;
         }
         *t = r->plan->tensors[it->second].desc(r->arena.as<uint8_t>());
     });

@@ -598,8 +598,10 @@ int hipie_request_perf(hipie_request* request, int index, float* ms);
 /* the arena tensor holding the value of graph node `node_id` (inspection, parity tests).  HIPIE_NOT_FOUND where the last
  * inference left it in no tensor: a node fused into its reader, and a value between two layers that ran as one kernel or as one
  * step of a single launch.  With HIP_KEEP_F32 values in front of a depthwise layer are there.  An f32 result that its
- * convolution stores in the caller's buffer is computed into its tensor by this call, which waits for the request's stream
- * then, and by every later inference of the request */
+ * convolution stores in the caller's buffer alone is computed into its tensor by the first call that asks for it, which waits
+ * for the request's stream then, and stored there by every later inference of the request (a single launch is followed by the
+ * layer once more) and by every captured one.  While the stream is captured the call leaves the tensor as it is: the graph, the
+ * next inference or the next call fills it.  Any thread may call this while others start the request and wait for it */
 int hipie_request_tensor(const hipie_request* request, int node_id, hipie_tensor* tensor);
 
 /* ======================================================================================

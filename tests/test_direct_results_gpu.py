@@ -161,3 +161,93 @@ def test_a_tensor_that_is_held_shows_the_last_inference(single):
         feed(10 + turn)
         graph.replay()
         assert shows(), turn
+
+
+def _tensor(req, node):
+    import ctypes
+    from dldt_amd._lib import check, lib
+    from dldt_amd.tensor import hipie_tensor
+    t = hipie_tensor()
+    check(lib().hipie_request_tensor(req._h, node, ctypes.byref(t)))
+    return t
+
+
+def _image(t, n):
+    """image n of a dense f32 tensor's descriptor as [C, H, W], read at once: no other stream is waited for"""
+    import ctypes
+    from dldt_amd._lib import check, lib
+    values = torch.empty(t.stride_n, dtype=torch.float32)
+    check(lib().hipie_memcpy(ctypes.c_void_p(values.data_ptr()), ctypes.c_void_p(t.data + 4 * n * t.stride_n), ctypes.c_size_t(4 * t.stride_n), 0))
+    return torch.as_strided(values, (t.c, t.h, t.w), (1, t.stride_h, t.stride_w)) + 0.0
+
+
+def _block(n, c, hw, oc):
+    g = builders.conv_block(n=n, c=c, hw=hw, oc=oc)[0]
+    return g, g.nodes[-1]["inputs"][0]
+
+
+def test_the_call_that_asks_first_waits_for_an_inference_in_flight():
+    from dldt_amd._lib import check, lib
+    g, node = _block(32, 256, 56, 512)                              # (0.3 ms and more behind the call)
+    plan = g.compile(0, config={"HIP_TUNE": "NO", "HIP_SINGLE_LAUNCH": "NO"})
+    for seed in range(3):
+        req = plan.create_request()
+        ins, outs = req.device_buffers()
+        ins[0].uniform_(0, 2.55, generator=torch.Generator(device="cuda").manual_seed(seed))
+        torch.cuda.synchronize()
+        check(lib().hipie_request_start(req._h, *req._ptrs(ins, outs), 1))
+        seen = _image(_tensor(req, node), 31)
+        req.wait()
+        assert torch.equal(seen, outs[0][31].cpu())
+
+
+@pytest.mark.parametrize("single", ["NO", "64"])
+def test_a_tensor_asked_for_by_another_thread_shows_the_inference_beside_it(single):
+    """the call comes before, while or after the inference is queued and waited for; when both have returned the values are there"""
+    import threading
+    import time
+    g, node = _block(1, 64, 56, 64)
+    plan = g.compile(0, config={"HIP_TUNE": "NO", "HIP_THROUGHPUT_STREAMS": "1", "HIP_SINGLE_LAUNCH": single})
+    feed = [torch.rand((1, 64, 56, 56), generator=torch.Generator(device="cuda").manual_seed(k), device="cuda") * 2.55 for k in range(2)]
+    for turn in range(60):
+        req = plan.create_request()
+        _, outs = req.device_buffers()
+        torch.cuda.synchronize()
+        seen = []
+
+        def ask():
+            until = time.perf_counter() + turn * 1e-6
+            while time.perf_counter() < until:
+                pass
+            seen.append(_tensor(req, node))
+
+        other = threading.Thread(target=ask)
+        other.start()
+        for k in range(2):
+            req.infer_device([feed[k]], outs)
+        other.join()
+        assert torch.equal(_image(seen[0], 0), outs[0][0].cpu()), turn
+
+
+def test_a_tensor_asked_for_in_a_capture_shows_the_last_inference_behind_it():
+    g, node = _block(1, 64, 14, 70)
+    plan = g.compile(0, config={"HIP_TUNE": "NO", "HIP_SINGLE_LAUNCH": "NO"})
+    req = plan.create_request()
+    ins, outs = req.device_buffers()
+    later = [torch.empty_like(outs[0])]
+    ins[0].uniform_(0, 2.55)
+    torch.cuda.synchronize()
+    req.enqueue(ins, outs)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.ExternalStream(req.stream), capture_error_mode="thread_local"):
+        _tensor(req, node)
+        req.enqueue(ins, later)
+        _tensor(req, node)
+    assert torch.equal(_image(_tensor(req, node), 0), outs[0][0].cpu())      # (nothing of the graph has run)
+    for turn in range(3):
+        ins[0].uniform_(0, 2.55)
+        torch.cuda.synchronize()
+        (graph.replay if turn != 1 else lambda: req.enqueue(ins, later))()
+        torch.cuda.synchronize()
+        assert torch.equal(_image(_tensor(req, node), 0), later[0][0].cpu()), turn
