@@ -123,9 +123,9 @@ struct Ctx {
         __builtin_amdgcn_s_barrier();
         target += n_wg / 8;
     }
-    __device__ __forceinline__ void count() const {
+    __device__ __forceinline__ void count(bool held) const {
         // (not the wave that looks at the counters: its loads would come back behind the addition)
-        if (tid == kProgramThreads - 64) (void)__hip_atomic_fetch_add(own, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (held && tid == kProgramThreads - 64) (void)__hip_atomic_fetch_add(own, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __device__ __forceinline__ void wait() {
         if (wave == 0 && !started) {

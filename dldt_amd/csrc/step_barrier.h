@@ -23,8 +23,8 @@ template <class Workgroup>
 HIPIE_HD void arrive_at(Workgroup& w) {
     const int32_t held = w.verdict();        // (on its way while the stores are acknowledged)
     w.settle();
+    w.count(held != 0);                      // (by the lane that adds: the rest of the workgroup finds out beside the addition)
     w.dead = w.lost(held);
-    if (!w.dead) w.count();
 }
 
 // Behind the wait for everybody's last arrival, by the first workgroup.

@@ -42,7 +42,7 @@ struct Workgroup {
     bool lost(int32_t held) const { return held == 0; }
     void lose() { p.flag = 0; }
     void settle() {}
-    void count() { ++l.count; }
+    void count(bool held) { l.count += held; }
     void tell(uint32_t what) { l.word = static_cast<int8_t>(what); }
 };
 
@@ -51,7 +51,7 @@ long ends[2] = {0, 0}, wrong = 0, taken_back = 0, silent = 0, hasty = 0;
 
 void arrive(Workgroup& w) {
 #ifdef ADDS_BEFORE_IT_LOOKS
-    w.count();
+    w.count(true);
     w.dead = w.p.flag == 0;
 #else
     arrive_at(w);
