@@ -418,8 +418,8 @@ std::shared_ptr<EntryConv> make_entry_conv(int device, const hipie_fq* fq, bool 
     a.clamp_hi = c.clamp_hi;
     a.fill = (static_cast<uint32_t>(fill) & 0xffu) * 0x01010101u;
     a.inv_W = 1.0f / static_cast<float>(mid.w);
-    int units = 256;
-    if (device >= 0) HIPIE_CHECK_HIP(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device));
+    int units = 0;
+    HIPIE_CHECK_HIP(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device));
     const Shape s = choose_shape(a, mid.n, units);
     if (s.R == 0) return nullptr;
     a.R = s.R;
@@ -434,7 +434,6 @@ std::shared_ptr<EntryConv> make_entry_conv(int device, const hipie_fq* fq, bool 
     a.o_groups = static_cast<int32_t>(ceil_div(o_tiles, 1 << a.wo_shift));
     e->pf = s.pf;
     e->groups_y = s.gy;
-    if (device < 0) return e;
     DeviceGuard g(device);
     HIPIE_CHECK_HIP(hipFuncSetAttribute(kernel_of(*e), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     const int64_t pieces = o_tiles * a.steps * 64;

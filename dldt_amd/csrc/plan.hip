@@ -4185,7 +4185,7 @@ int hipie_request_create(const hipie_plan* p, int perf_count, hipie_request** ou
         if (p->program && !r->perf) {
             r->program = p->program;
             r->slot = r->program->take_slot();
-            HIPIE_CHECK_HIP(hipEventCreateWithFlags(&r->behind, hipEventDisableTiming));
+            if (r->slot >= 0) HIPIE_CHECK_HIP(hipEventCreateWithFlags(&r->behind, hipEventDisableTiming));
         }
         for (const auto& t : p->tensors) {
             if (t.alias >= 0) continue;
