@@ -50,6 +50,16 @@ __device__ __forceinline__ uint32_t prob_levels4(const AttentionArgs& a, float p
     return a.p_add ? add_bytes(w, a.p_add) : (w ^ a.p_xor);
 }
 
+// 4 x 4 byte transpose: t[e] = bytes e of p0 .. p3
+__device__ __forceinline__ void transpose_bytes(uint32_t p0, uint32_t p1, uint32_t p2, uint32_t p3, uint32_t (&t)[4]) {
+    const uint32_t lo01 = __builtin_amdgcn_perm(p1, p0, 0x05010400u), hi01 = __builtin_amdgcn_perm(p1, p0, 0x07030602u);      // p0.b0 p1.b0 p0.b1 p1.b1 ...
+    const uint32_t lo23 = __builtin_amdgcn_perm(p3, p2, 0x05010400u), hi23 = __builtin_amdgcn_perm(p3, p2, 0x07030602u);
+    t[0] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+    t[1] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+    t[2] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+    t[3] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+}
+
 // Rows longer than this have the Softmax of the stand-alone kernel bit for bit (softmax_rows_reg: exp(x - max), sums of
 // four keys, the chunks of 256 keys, then a tree over the groups of four), so that their levels do not depend on whether
 // the core is one kernel.  Up to it exp2 of one fused multiply-add, a serial sum and the reciprocal, within the same

@@ -103,14 +103,8 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const AttentionArgs a
         const int i = tid + j * 256;
         if (i >= S * 4) continue;
         const int d4 = i & 15, kq = i >> 4;
-        const uint32_t* w = vw[j];
-        // 4 x 4 byte transpose: t[e] = bytes e of w[0..3]
-        const uint32_t lo01 = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u);   // w0.b0 w1.b0 w0.b1 w1.b1
-        const uint32_t hi01 = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u);   // w0.b2 w1.b2 w0.b3 w1.b3
-        const uint32_t lo23 = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u);
-        const uint32_t hi23 = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
-        const uint32_t t[4] = {__builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
-                               __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u)};
+        uint32_t t[4];
+        transpose_bytes(vw[j][0], vw[j][1], vw[j][2], vw[j][3], t);
         const int key = 4 * kq, tile = key >> 5, in = key & 31;               // in = 8 a + 4 half
         const int col = tile * 32 + ((in >> 2) & 1) * 16 + (in >> 3) * 4;
 #pragma unroll
@@ -310,13 +304,8 @@ __global__ __launch_bounds__(256, 2) void attention_long_kernel(const AttentionA
         const int i = tid + j * 256;
         if (i >= S * 4) continue;
         const int d4 = i & 15, kq = i >> 4;
-        const uint32_t* w = vw[j];
-        const uint32_t lo01 = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u);   // 4 x 4 bytes transposed, as above
-        const uint32_t hi01 = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u);
-        const uint32_t lo23 = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u);
-        const uint32_t hi23 = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
-        const uint32_t t[4] = {__builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
-                               __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u)};
+        uint32_t t[4];
+        transpose_bytes(vw[j][0], vw[j][1], vw[j][2], vw[j][3], t);
         const int col = (kq >> 4) * 64 + (kq & 3) * 16 + ((kq >> 2) & 3) * 4;       // tile kq / 4, lane group kq % 4
 #pragma unroll
         for (int e = 0; e < 4; ++e) {

@@ -862,16 +862,6 @@ __device__ __forceinline__ void conv_tiles(Ctx& x, lds_ptr lds) {
 // v_dot4_i32_i8 as in dwconv.hip; consecutive lanes take consecutive channels.  G = 4 does the fewest operations per value,
 // G = 1 a quarter of the work per lane: where a step's values are no more than the launch's lanes at one pixel each, what a
 // lane does is what the step takes (ProgBuilder::conv).
-// 4 x 4 byte transpose: t[e] = bytes e of p0 .. p3
-__device__ __forceinline__ void transpose_bytes(uint32_t p0, uint32_t p1, uint32_t p2, uint32_t p3, uint32_t (&t)[4]) {
-    const uint32_t lo01 = __builtin_amdgcn_perm(p1, p0, 0x05010400u), hi01 = __builtin_amdgcn_perm(p1, p0, 0x07030602u);
-    const uint32_t lo23 = __builtin_amdgcn_perm(p3, p2, 0x05010400u), hi23 = __builtin_amdgcn_perm(p3, p2, 0x07030602u);
-    t[0] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
-    t[1] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
-    t[2] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
-    t[3] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
-}
-
 template <int STRIDE, int G>
 __device__ __forceinline__ void dw_items(Ctx& x) {
     constexpr int COLS = G == 1 ? 3 : 3 + 3 * STRIDE;
@@ -1473,7 +1463,7 @@ __device__ __forceinline__ void attention_units(const ProgAttention& s, Ctx& x, 
         first = false;
         if (u >= s.units) return;
         // K into LDS, V transposed into LDS: everything is requested before any of it is used
-        constexpr int kRounds = 4;              // S * 4 pieces of K, as many groups of 4 keys x 4 d of V, by 512 threads
+        constexpr int kRounds = kPlainSoftmax * 4 / kProgramThreads;      // S * 4 pieces of K, as many groups of 4 keys x 4 d of V, by 512 threads
         v4i kx[kRounds];
         uint32_t vw[kRounds][4];
 #pragma unroll
@@ -1502,11 +1492,8 @@ __device__ __forceinline__ void attention_units(const ProgAttention& s, Ctx& x, 
         for (int j = 0; j < kRounds; ++j) {
             if (j * kProgramThreads >= S * 4) continue;
             const int i = min(x.tid + j * kProgramThreads, S * 4 - 1), d4 = i & 15, kq = i >> 4;
-            const uint32_t* v = vw[j];
-            const uint32_t lo01 = __builtin_amdgcn_perm(v[1], v[0], 0x05010400u), hi01 = __builtin_amdgcn_perm(v[1], v[0], 0x07030602u);
-            const uint32_t lo23 = __builtin_amdgcn_perm(v[3], v[2], 0x05010400u), hi23 = __builtin_amdgcn_perm(v[3], v[2], 0x07030602u);
-            const uint32_t t[4] = {__builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
-                                   __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u)};
+            uint32_t t[4];
+            transpose_bytes(vw[j][0], vw[j][1], vw[j][2], vw[j][3], t);
             const int key = 4 * kq, tile = key >> 5, in = key & 31;
             const int col = tile * 32 + ((in >> 2) & 1) * 16 + (in >> 3) * 4;
 #pragma unroll
@@ -1739,11 +1726,8 @@ __device__ __forceinline__ void attention_long(const ProgAttention& s, Ctx& x, l
                 if (w + 8 * j >= nt) continue;
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
-                    const uint32_t* y = vw[j][i];
-                    const uint32_t lo01 = __builtin_amdgcn_perm(y[1], y[0], 0x05010400u), hi01 = __builtin_amdgcn_perm(y[1], y[0], 0x07030602u);
-                    const uint32_t lo23 = __builtin_amdgcn_perm(y[3], y[2], 0x05010400u), hi23 = __builtin_amdgcn_perm(y[3], y[2], 0x07030602u);
-                    const uint32_t t[4] = {__builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
-                                           __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u)};
+                    uint32_t t[4];
+                    transpose_bytes(vw[j][i][0], vw[j][i][1], vw[j][i][2], vw[j][i][3], t);
                     const int d = 4 * (lane & 15);      // (keys in the order in which their scores leave the matrix unit)
 #pragma unroll
                     for (int q = 0; q < 4; ++q) *(lds_i32)(sVT + (d + q) * kPitch + 16 * (d >> 4) + 32 * j + 16 * i + 4 * (lane >> 4)) = static_cast<int32_t>(t[q]);
@@ -2387,14 +2371,20 @@ bool ProgBuilder::attention(const hipie_attention* att, const void* const (&qkv)
     s.a.mask_outer = proto.S;
     // Waves per 32 queries, by the clocks of a workgroup's round: staging, and the chain of a wave's tiles (from five waves on two
     // share a SIMD).  Against the best of the four splits the choice costs an encoder of two layers 0 - 2 % of its time (1 to 4
-    // sequences of 32 to 512 keys, 64 and 256 workgroups; 6 % for 32 keys and 256, where one tile leaves nothing to share).
+    // sequences of 32 to 384 keys, 64 and 256 workgroups; 6 % for 32 keys and 256, where one tile leaves nothing to share).  Longer
+    // rows always take all eight (attention_long).
     const int qt = proto.S / 32;
     const int64_t elements = static_cast<int64_t>(batch_outer) * batch;
     double best = 1e30;
-    for (int shift = 0; (1 << shift) <= kMostSplit; ++shift) {
+    if (proto.S > kPlainSoftmax) {
+        best = 0.0;
+        s.split_shift = 3;
+        s.parts = qt;
+        s.units = static_cast<int32_t>(elements * qt);
+    } else for (int shift = 0; (1 << shift) <= kMostSplit; ++shift) {
         const int split = 1 << shift, blocks = std::min(kMostSplit / split, qt);
         const int64_t tiles = ceil_div(qt, split), parts = ceil_div(qt, kMostSplit / split), rounds = ceil_div(elements * parts, workgroups);
-        if (tiles > kMostTiles || attention_lds(proto.S, split) > kPartBytes + kKoffBytes || (proto.S > kPlainSoftmax && split < kMostSplit)) continue;
+        if (tiles > kMostTiles || attention_lds(proto.S, split) > kPartBytes + kKoffBytes) continue;
         const double waves = static_cast<double>(blocks * std::min(split, qt));
         const double t = static_cast<double>(rounds) * (5000.0 + 4.0 * proto.S + std::max(1.0, waves / 5.0) * static_cast<double>(tiles) * 2400.0);
         if (t < best) {
