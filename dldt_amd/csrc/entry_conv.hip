@@ -31,7 +31,7 @@ namespace hipie {
 namespace {
 
 constexpr int kThreads = 512, kWaves = kThreads / 64;
-constexpr int kMostFragments = 2;            // of 32 pixels that a wave multiplies (110 registers, two workgroups a compute unit; three take 140 and more)
+constexpr int kMostFragments = 2;            // of 32 pixels that a wave multiplies (104 registers, 110 with BOTH: two workgroups a compute unit; three fragments take 140)
 constexpr int kAhead = 4;                    // K steps of 32 bytes in a group: one is multiplied while the next one's weights come
 
 struct Args {
@@ -45,7 +45,7 @@ struct Args {
     const int32_t* corr;
     const float *bias, *scale;
     float* out;
-    float* tensor;                           // the values channels innermost as well, or nullptr
+    float* tensor;                           // (BOTH) the values channels innermost as well
     int64_t t_sn, t_sh;
     int32_t t_sw;                            // its strides in elements: image, row, pixel
     int32_t C, H, W, HW, OC;
@@ -70,8 +70,9 @@ __device__ __forceinline__ Buffer make_buffer(void* p, uint32_t) { return p; }
 __device__ __forceinline__ void store4(Buffer, uint32_t, float) {}
 #endif
 
-// PF: fragments of 32 pixels a wave multiplies; U8: bytes in; SMALL: pixels of four bytes (rows of taps contiguous, 4-byte aligned)
-template <int PF, bool U8, bool SMALL>
+// PF: fragments of 32 pixels a wave multiplies; U8: bytes in; SMALL: pixels of four bytes (rows of taps contiguous, 4-byte aligned);
+// BOTH: the values into a.tensor as well (its instructions beside the others' cost 12 x 72 x 45 x 45 to 100 1 %, taken or not)
+template <int PF, bool U8, bool SMALL, bool BOTH>
 __global__ __launch_bounds__(kThreads, 4) void entry_conv_kernel(const Args a) {
     extern __shared__ __attribute__((aligned(16))) int8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -280,7 +281,7 @@ __global__ __launch_bounds__(kThreads, 4) void entry_conv_kernel(const Args a) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) r[i] = r[i] < a.clamp_lo ? a.clamp_lo : (r[i] > a.clamp_hi ? a.clamp_hi : r[i]);
             }
-            if (a.tensor) {
+            if constexpr (BOTH) {
                 int y, xx;
                 fast_divmod(min(m, count - 1), a.W, a.inv_W, y, xx);
                 const int oc = (og * wo + o_wave) * 32 + 4 * h;
@@ -370,12 +371,15 @@ Shape choose_shape(const Args& a, int images, int units) {
     return best;
 }
 
-template <int PF>
+template <int PF, bool BOTH>
 const void* kernel_of(bool u8, bool small) {
-    if (u8) return small ? reinterpret_cast<const void*>(&entry_conv_kernel<PF, true, true>) : reinterpret_cast<const void*>(&entry_conv_kernel<PF, true, false>);
-    return small ? reinterpret_cast<const void*>(&entry_conv_kernel<PF, false, true>) : reinterpret_cast<const void*>(&entry_conv_kernel<PF, false, false>);
+    if (u8) return small ? reinterpret_cast<const void*>(&entry_conv_kernel<PF, true, true, BOTH>) : reinterpret_cast<const void*>(&entry_conv_kernel<PF, true, false, BOTH>);
+    return small ? reinterpret_cast<const void*>(&entry_conv_kernel<PF, false, true, BOTH>) : reinterpret_cast<const void*>(&entry_conv_kernel<PF, false, false, BOTH>);
 }
-const void* kernel_of(const EntryConv& e) { return e.pf == 1 ? kernel_of<1>(e.u8, e.small) : kernel_of<kMostFragments>(e.u8, e.small); }
+const void* kernel_of(const EntryConv& e, bool both) {
+    if (both) return e.pf == 1 ? kernel_of<1, true>(e.u8, e.small) : kernel_of<kMostFragments, true>(e.u8, e.small);
+    return e.pf == 1 ? kernel_of<1, false>(e.u8, e.small) : kernel_of<kMostFragments, false>(e.u8, e.small);
+}
 
 }  // namespace
 
@@ -435,7 +439,7 @@ std::shared_ptr<EntryConv> make_entry_conv(int device, const hipie_fq* fq, bool 
     e->pf = s.pf;
     e->groups_y = s.gy;
     DeviceGuard g(device);
-    HIPIE_CHECK_HIP(hipFuncSetAttribute(kernel_of(*e), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    for (bool both : {false, true}) HIPIE_CHECK_HIP(hipFuncSetAttribute(kernel_of(*e, both), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     const int64_t pieces = o_tiles * a.steps * 64;
     e->weights.alloc(device, static_cast<size_t>(pieces) * 16);
     hipLaunchKernelGGL(pack_entry_kernel, dim3(static_cast<uint32_t>(ceil_div(pieces, 256))), dim3(256), 0, nullptr, c.wgt, e->weights.as<int8_t>(), c.OCp, c.Kp, a.steps, pieces);
@@ -457,7 +461,7 @@ void run_entry_conv(const EntryConv& e, const void* in, const hipie_tensor& mid,
     a.levels = static_cast<uint8_t*>(mid.data);
     a.out = static_cast<float*>(planes);
     void* args[] = {&a};
-    HIPIE_CHECK_HIP(hipLaunchKernel(kernel_of(e), dim3(8u * static_cast<uint32_t>(a.per_xcd), static_cast<uint32_t>(e.groups_y)), dim3(kThreads), args, e.lds, s));
+    HIPIE_CHECK_HIP(hipLaunchKernel(kernel_of(e, out != nullptr), dim3(8u * static_cast<uint32_t>(a.per_xcd), static_cast<uint32_t>(e.groups_y)), dim3(kThreads), args, e.lds, s));
 }
 
 }  // namespace hipie
