@@ -1946,8 +1946,8 @@ __global__ void clear_words(uint32_t* p, int n) {
 // Tile shape of a convolution step, by the clocks its busiest compute unit takes.  The constants are fitted, not derived: to
 // the time of whole networks with one class of layers at a time in each of the shapes (ResNet-50, MobileNetV2, encoders and the
 // convolution block, at 64, 128 and 256 workgroups), so that the choice loses as little as possible against the best shape of
-// every class: summed over a network's classes, 167 in all, 0 - 8 % of its time, most of which is what the best of many noisy
-// medians lies too low.  Of the other shapes that were measured (1 x 2, 1 x 4, 2 x 4 of fragments) none is the best of a class by
+// every class: summed over a network's classes, 167 in all, 0 - 5 % of its time, most of which is what the best of many noisy
+// medians lies too low (the kernel as it is; the columns of Gelu that all waves share are not in the model).  Of the other shapes that were measured (1 x 2, 1 x 4, 2 x 4 of fragments) none is the best of a class by
 // more than the runs differ.
 // What the terms stand for: a load of 1 KB on a unit's path, a matrix instruction, a round trip to memory per filled ring, the
 // f32 chain per value, a store instruction, the partial sums of the waves that share a K in LDS.  Rounds are tiles a wave takes
@@ -2531,10 +2531,10 @@ void request_leaves(int device) {
 
 // A lone request takes the form that was fastest alone.  Beside others it takes the smaller one, if units are left for it
 // (never more workgroups than compute units, so that all of them find a place), and else the steps, whose kernels share the
-// device.  ResNet-50, batch 1, us a request with 2 and 4 in flight: steps 251 and 167, 64 workgroups side by side 148 and 96
-// (alone: steps 492, 64 workgroups 284, 256 227).  With more than twice as many requests as find a place the ones by steps wait
-// for the others: batch 3 with 128 workgroups, 4 in flight: 182, steps 182; 6 in flight: 221, steps 173 (batch 1 with 64
-// workgroups, 6 in flight: 113, steps 163).
+// device.  ResNet-50, batch 1, us a request with 2 and 4 in flight, two of the four on one hardware queue: steps 251 and 242, 64
+// workgroups side by side 144 and 136 (alone: steps 493, 64 workgroups 274, 256 222).  With more than twice as many requests as find
+// a place the ones by steps wait for the others: batch 3 with 128 workgroups, 4 in flight: 217, steps 254; 6 in flight: 242, steps
+// 174 (batch 1, 64 workgroups beside others, 6 in flight: 118, steps 163).
 const ProgramForm* Program::choose(int together) {
     const ProgramForm* f = together > 1 ? shared.get() : lone.get();
     if (!f || (lone != shared && together > 1 && together * f->workgroups > 2 * units)) return nullptr;

@@ -484,8 +484,9 @@ int hipie_compile(const hipie_graph* graph, int device, hipie_plan** plan);
  * depthwise 3 x 3 layer that alone reads its result, without HIP_KEEP_F32, in plans that are tuned and, measured or not, in a
  * single launch; the tensor between two layers run that way exists in LDS only and hipie_request_tensor gives
  * HIPIE_NOT_FOUND for it; and a graph input's FakeQuantize and the convolution behind it whose f32 values are the graph's
- * result, without HIP_KEEP_F32, in plans that are tuned, the levels between them stored as ever), HIP_SINGLE_LAUNCH (a request that is started and waited for runs as one persistent kernel:
- * AUTO = a plan for one stream, where the load-time measurement finds it faster, YES = wherever the plan has such a form,
+ * result, without HIP_KEEP_F32, with AUTO in plans that are tuned, the levels between them stored as ever, and as two in a
+ * call whose result shares a byte with its input), HIP_SINGLE_LAUNCH (a request that is started and waited for runs as one
+ * persistent kernel: AUTO = a plan for one stream, where the load-time measurement finds it faster, YES = wherever the plan has such a form,
  * in the fastest of its sizes, 64 / 128 / 256 = with that many workgroups, NO; beside other requests in flight the smallest
  * form that was no slower than the steps is used, as many at a time as the device has compute units for, and the steps
  * otherwise), NETWORK_NAME.  An unknown key gives HIPIE_NOT_FOUND, a value the key does not take
