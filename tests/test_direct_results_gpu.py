@@ -1,6 +1,6 @@
-"""A convolution whose f32 values are the graph's result stores them into the caller's [N, C, H, W] buffer itself, beside its own
-tensor: every kernel variant the layer has and the single launch, against the copy kernel behind the same convolution
-(HIP_KEEP_F32), bit for bit."""
+"""A convolution whose f32 values are the graph's result stores them into the caller's [N, C, H, W] buffer itself, and into its own
+tensor where somebody looks at that: every kernel variant the layer has and the single launch, against the copy kernel behind
+the same convolution (HIP_KEEP_F32), bit for bit."""
 import numpy as np
 import pytest
 import torch
@@ -70,6 +70,44 @@ def test_every_variant_stores_the_planes_that_the_copy_stores(tmp_path, n, c, hw
     req.infer_device(ins, outs)
     assert np.array_equal(outs[0].cpu().numpy().view(np.uint32), want[0])
     assert single.metric("SINGLE_LAUNCH_COUNTS") == "1 0"
+
+
+@pytest.mark.parametrize("n,c,hw,oc,k,more", [(1, 3, 7, 8, 3, []), (2, 17, 9, 65, 3, [14]), (3, 64, 14, 70, 3, LINES), (1, 64, 33, 129, 3, LINES),
+                                              (5, 128, 8, 3, 3, [6, 7, 16, 18, 19, 20, 21] + LINES), (2, 64, 5, 37, 1, [23]), (1, 3, 17, 9, 7, [13])])
+def test_every_variant_stores_the_tensor_beside_the_planes(tmp_path, n, c, hw, oc, k, more):
+    """... in the one launch, of a request whose tensor was asked for before its first inference"""
+    rng = np.random.default_rng(oc)
+    q = builders.QuantizedNet()
+    a = q.input("data", (n, c, hw, hw), 2.55)
+    node = q.conv_f32(a, rng.standard_normal((oc, c, k, k), dtype=np.float32) * np.float32(0.05), rng.standard_normal(oc, dtype=np.float32), pads=(k // 2, k // 2),
+                      strides=(2, 2) if k == 7 else (1, 1))
+    q.g.result(node, "out")
+    x = torch.rand((n, c, hw, hw), generator=torch.Generator(device="cuda").manual_seed(4), device="cuda") * 2.55
+    ref = q.g.compile(0, config={"HIP_KEEP_F32": "YES", "HIP_TUNE": "NO"}).create_request()
+    ins, outs = ref.device_buffers()
+    ins[0].copy_(x)
+    torch.cuda.synchronize()
+    ref.enqueue(ins, outs)
+    torch.cuda.synchronize()
+    want, planes, ran = ref.tensor(node).view(np.uint32), outs[0].cpu().numpy().view(np.uint32), []
+    for v in VARIANTS:
+        path = tmp_path / str(v)
+        path.write_text("0 -1\n1 %d\n2 -1\n" % v)
+        try:
+            plan = q.g.compile(0, config={"HIP_TUNE_FILE": str(path), "HIP_SINGLE_LAUNCH": "NO"})
+        except HipieError:
+            continue                                          # a variant this layer does not have
+        assert plan.steps[1]["variant"] == v and [int(plan.step_rt_info(i, "kernels")) for i in range(3)] == [1, 1, 0]
+        req = plan.create_request()
+        assert not req.tensor(node).any()
+        outs[0].fill_(float("nan"))
+        torch.cuda.synchronize()
+        req.enqueue(ins, outs)
+        torch.cuda.synchronize()
+        assert np.array_equal(outs[0].cpu().numpy().view(np.uint32), planes), v
+        assert np.array_equal(req.tensor(node).view(np.uint32), want), v
+        ran.append(v)
+    assert set(ran) >= set(ANY + more)
 
 
 @pytest.mark.parametrize("relu", [False, True])
