@@ -547,8 +547,8 @@ int64_t hipie_plan_arena_bytes(const hipie_plan* plan);
 int hipie_plan_num_steps(const hipie_plan* plan);
 int hipie_plan_step_info(const hipie_plan* plan, int index, char* name, size_t name_len, char* type,
                          size_t type_len, int64_t* macs, int64_t* bytes);
-/* the kernel variant a step runs (hipie_conv_set_tile numbering), -1 for a step without variants: part
- * of what GetExecGraphInfo reports per executed node (exec_graph_info.hpp:34-76, implementation type) */
+/* the kernel variant a step runs (hipie_conv_set_tile numbering; + 32: nine steps of weights in flight, + 64: in the launch
+ * of the FakeQuantize in front of it), -1 for a step without variants: part of what GetExecGraphInfo reports per executed node (exec_graph_info.hpp:34-76, implementation type) */
 int hipie_plan_step_variant(const hipie_plan* plan, int index, int* variant);
 /* the attributes GetExecGraphInfo attaches to every executed node (exec_graph_info.hpp:34-76), by their key there:
  * originalLayersNames (comma-separated graph nodes the step stands for), layerType, runtimePrecision (U8 / I8 for the
